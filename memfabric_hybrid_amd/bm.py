@@ -1,8 +1,9 @@
 """Python face of the BM copy API with the names of the reference's pybind
 module (``memfabric_hybrid.bm``: src/smem/csrc/python_wrapper/memfabric_hybrid/pymf_hybrid.cpp:151-175,
 584-638): ``initialize``, ``create``, ``BigMemory.copy_data`` / ``copy_data_batch``
-/ ``wait`` / ``peer_rank_ptr`` ...  Every call goes straight through ctypes to
-the C ABI; addresses are plain integers as in the reference.
+/ ``wait`` / ``peer_rank_ptr`` ...  Every call goes straight to the C ABI, the copies
+through an extension module of their own, the others through ctypes; addresses
+are plain integers as in the reference.
 """
 
 import ctypes
@@ -99,15 +100,12 @@ class BigMemory:
         return native.lib().smem_bm_unregister_user_mem(self._h, addr)
 
     def copy_data(self, src_ptr, dst_ptr, size, type, flags=0):  # noqa: A002 - the reference's argument name
-        params = native.SmemCopyParams(src_ptr, dst_ptr, size)
-        return native.lib().smem_bm_copy(self._h, ctypes.byref(params), int(type), flags)
+        return native.calls().copy(self._h, src_ptr, dst_ptr, size, type, flags)
 
     def copy_data_batch(self, src_addrs, dst_addrs, sizes, count, type, flags=0):  # noqa: A002
-        srcs = native.ptr_array(src_addrs[:count])
-        dsts = native.ptr_array(dst_addrs[:count])
-        lens = native.u64_array(sizes[:count])
-        params = native.BatchCopyParams(srcs, dsts, lens, count)
-        return native.lib().smem_bm_copy_batch(self._h, ctypes.byref(params), int(type), flags)
+        """The first `count` elements of three sequences of integers.  Arrays of 64-bit integers (numpy) are handed over
+        as they are."""
+        return native.calls().copy_batch(self._h, src_addrs, dst_addrs, sizes, count, type, flags)
 
     def wait(self):
         return native.lib().smem_bm_wait(self._h)

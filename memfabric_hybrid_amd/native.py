@@ -6,6 +6,8 @@ own init calls fail with their error codes.
 """
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -14,6 +16,7 @@ LIB_DIR = os.path.join(_HERE, "lib")
 DATAPLANE_PATH = os.path.join(LIB_DIR, "libmf_hip_dataplane.so")
 PLUGIN_PATH = os.path.join(LIB_DIR, "libmf_hybm_copy_extend.so")
 YARDSTICK_PATH = os.path.join(LIB_DIR, "libmf_hip_yardstick.so")
+CALLS_PATH = os.path.join(LIB_DIR, "_calls.so")
 
 # ---- enums (values pinned in include/mf_xcopy_types.h) ---------------------
 BM_OK = 0
@@ -299,6 +302,7 @@ _lock = threading.Lock()
 _lib = None
 _plugin = None
 _yardstick = None
+_calls = None
 
 
 # pace of the combine's read and write parts the library starts with (MB/s), for callers that switch it and back
@@ -348,6 +352,23 @@ def yardstick():
         return _yardstick
 
 
+def calls():
+    """The extension module behind the Python face: sequences of integers into the C API without a loop of the
+    interpreter's (csrc/python/calls.cpp).  Linked against the data-plane library, which is loaded first."""
+    global _calls
+    if _calls is None:
+        lib()
+        with _lock:
+            if _calls is None:
+                if not os.path.exists(CALLS_PATH):
+                    raise OSError(f"{CALLS_PATH} is missing: build it with `make -C memfabric_hybrid_amd/csrc`")
+                loader = importlib.machinery.ExtensionFileLoader("_calls", CALLS_PATH)
+                module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_calls", loader))
+                loader.exec_module(module)
+                _calls = module
+    return _calls
+
+
 def declared_symbols():
     return sorted(_SIGNATURES), sorted(_PLUGIN_SIGNATURES)
 
@@ -358,13 +379,11 @@ def last_error():
 
 def u64_array(values):
     arr = (ctypes.c_uint64 * len(values))()
-    for i, v in enumerate(values):
-        arr[i] = int(v)
+    calls().fill(arr, values)
     return arr
 
 
 def ptr_array(values):
     arr = (ctypes.c_void_p * len(values))()
-    for i, v in enumerate(values):
-        arr[i] = int(v)
+    calls().fill(arr, values)
     return arr

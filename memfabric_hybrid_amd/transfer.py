@@ -24,12 +24,6 @@ class TransDataOpType(IntEnum):
 _ROLES = {"Prefill": native.SMEM_TRANS_SENDER, "Decode": native.SMEM_TRANS_RECEIVER}
 
 
-def _arrays(buffers, peer_buffers, lengths):
-    if not (len(buffers) == len(peer_buffers) == len(lengths)) or len(buffers) > 0xFFFFFFFF:
-        return None
-    return native.ptr_array(buffers), native.ptr_array(peer_buffers), native.u64_array(lengths)
-
-
 class TransferEngine:
     TransferOpcode = TransferOpcode
     TransDataOpType = TransDataOpType
@@ -92,33 +86,22 @@ class TransferEngine:
         return self._lib.smem_trans_read_submit(self._handle, buffer, dest_session.encode(), peer_buffer, length,
                                                 stream, flags)
 
+    def _batch(self, dest_session, buffers, peer_buffers, lengths, flags, write, submit=False, stream=None):
+        # -1 before initialize() and for sequences of different lengths, else the library's code
+        return native.calls().transfer_batch(self._handle, write, dest_session, buffers, peer_buffers, lengths, submit, stream,
+                                             flags)
+
     def batch_transfer_sync_write(self, dest_session, buffers, peer_buffers, lengths, flags=0):
-        arrays = _arrays(buffers, peer_buffers, lengths) if self._handle else None
-        if arrays is None:
-            return -1
-        return self._lib.smem_trans_batch_write(self._handle, arrays[0], dest_session.encode(), arrays[1], arrays[2],
-                                                len(buffers), flags)
+        return self._batch(dest_session, buffers, peer_buffers, lengths, flags, True)
 
     def batch_transfer_sync_read(self, dest_session, buffers, peer_buffers, lengths, flags=0):
-        arrays = _arrays(buffers, peer_buffers, lengths) if self._handle else None
-        if arrays is None:
-            return -1
-        return self._lib.smem_trans_batch_read(self._handle, arrays[0], dest_session.encode(), arrays[1], arrays[2],
-                                               len(buffers), flags)
+        return self._batch(dest_session, buffers, peer_buffers, lengths, flags, False)
 
     def batch_transfer_async_write_submit(self, dest_session, buffers, peer_buffers, lengths, stream, flags=0):
-        arrays = _arrays(buffers, peer_buffers, lengths) if self._handle else None
-        if arrays is None:
-            return -1
-        return self._lib.smem_trans_batch_write_submit(self._handle, arrays[0], dest_session.encode(), arrays[1],
-                                                       arrays[2], len(buffers), stream, flags)
+        return self._batch(dest_session, buffers, peer_buffers, lengths, flags, True, True, stream)
 
     def batch_transfer_async_read_submit(self, dest_session, buffers, peer_buffers, lengths, stream, flags=0):
-        arrays = _arrays(buffers, peer_buffers, lengths) if self._handle else None
-        if arrays is None:
-            return -1
-        return self._lib.smem_trans_batch_read_submit(self._handle, arrays[0], dest_session.encode(), arrays[1],
-                                                      arrays[2], len(buffers), stream, flags)
+        return self._batch(dest_session, buffers, peer_buffers, lengths, flags, False, True, stream)
 
     def destroy(self):
         if self._handle:

@@ -1,0 +1,96 @@
+"""The extension module behind the Python face: integers of every kind of sequence arrive as the same 64-bit words."""
+
+import array
+import ctypes
+
+import numpy as np
+import pytest
+
+from memfabric_hybrid_amd import bm, native
+from memfabric_hybrid_amd.transfer import TransferEngine
+
+VALUES = [0, 1, (1 << 30) - 1, 1 << 30, (1 << 60) - 1, 1 << 60, (1 << 63) - 1]
+WIDE = VALUES + [1 << 63, (1 << 64) - 1]
+
+KINDS = {
+    "list": list, "tuple": tuple, "array": lambda v: array.array("Q", v),
+    "numpy_u64": lambda v: np.array(v, dtype=np.uint64),
+    "numpy_strided": lambda v: np.repeat(np.array(v, dtype=np.uint64), 2)[::2],
+    "numpy_big_endian": lambda v: np.array(v, dtype=">u8"),
+    "numpy_scalars": lambda v: list(np.array(v, dtype=np.uint64)),
+    "ctypes": lambda v: (ctypes.c_uint64 * len(v))(*v),
+    "numpy_i64": lambda v: np.array(v, dtype=np.uint64).astype(np.int64),
+    "numpy_object": lambda v: np.array(v, dtype=object),
+}
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("n", [0, 1, 2, len(WIDE)])
+def test_words_of_a_sequence(lib, kind, n):
+    assert list(native.u64_array(KINDS[kind](WIDE[:n]))) == WIDE[:n]
+    assert [p or 0 for p in native.ptr_array(KINDS[kind](WIDE[:n]))] == WIDE[:n]
+
+
+def test_words_are_taken_modulo_two_to_the_64(lib):
+    assert list(native.u64_array([-1, -(1 << 63), (1 << 64) + 5, True, 7.9, np.int32(-2)])) == \
+        [(1 << 64) - 1, 1 << 63, 5, 1, 7, (1 << 64) - 2]
+    assert list(native.u64_array(np.array([3, -3], dtype=np.int32))) == [3, (1 << 64) - 3]
+
+
+@pytest.mark.parametrize("bad, error", [(["x"], ValueError), ([None], TypeError), ([[1]], TypeError)])
+def test_elements_that_are_no_integers(lib, bad, error):
+    with pytest.raises(error):
+        native.u64_array(bad)
+    with pytest.raises(error):
+        bm.BigMemory(0x1000).copy_data_batch([1], bad, [1], 1, bm.BmCopyType.G2G)
+
+
+def test_a_list_that_changes_while_it_is_read(lib):
+    values = [1, 2, 3]
+
+    class Shrinks:
+        def __int__(self):
+            del values[1:]
+            return 1
+    values[0] = Shrinks()
+    with pytest.raises(RuntimeError):
+        native.calls().fill((ctypes.c_uint64 * 3)(), values)
+
+
+def test_codes_without_a_pool_or_a_session(lib):
+    pool = bm.BigMemory(None)
+    assert pool.copy_data(1, 2, 3, bm.BmCopyType.G2G) == native.SM_INVALID_PARAM
+    assert pool.copy_data_batch([1], [2], [3], 1, bm.BmCopyType.G2G) == native.SM_INVALID_PARAM
+    pool = bm.BigMemory(0x1000)
+    assert pool.copy_data_batch([1], [2], [3], 1, bm.BmCopyType.G2G) == native.SM_NOT_INITIALIZED
+    for count in (2, -1, 1 << 32):    # more than the sequences hold, or no count at all
+        assert pool.copy_data_batch([1], [2], [3], count, bm.BmCopyType.G2G) == native.SM_INVALID_PARAM
+    engine = TransferEngine()
+    assert engine.batch_transfer_sync_write("127.0.0.1:2000", [1], [2], [3]) == -1
+    engine._handle = 0x1000
+    assert engine.batch_transfer_sync_read("127.0.0.1:2000", [1], [2, 3], [3]) == -1
+    assert engine.batch_transfer_sync_read("127.0.0.1:2000", [1], [2], [3]) == native.SM_INVALID_PARAM
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["list", "tuple", "numpy_u64", "numpy_strided", "numpy_scalars"])
+@pytest.mark.parametrize("n", [1, 128, 129, 4000])
+def test_batch_copy_from_every_kind_of_sequence(lib, kind, n):
+    assert bm.initialize("tcp://127.0.0.1:0", 1, 0) == 0, native.last_error()
+    pool = bm.create(1, 0, 32 << 20)
+    try:
+        dev, rng = pool.peer_rank_ptr(0), np.random.default_rng(n)
+        before = rng.integers(0, 256, 32 << 20, dtype=np.uint8)
+        assert lib.mfrt_memcpy(dev, before.ctypes.data, before.nbytes) == 0
+        sizes = rng.integers(1, 2049, n)
+        source, target = rng.permutation(n) * 2048, (16 << 20) + rng.permutation(n) * 2048
+        words = [KINDS[kind]((a.astype(np.uint64) + np.uint64(b)).tolist()) for a, b in ((source, dev), (target, dev), (sizes, 0))]
+        assert pool.copy_data_batch(*words, n, bm.BmCopyType.G2G) == 0, native.last_error()
+        after = np.empty_like(before)
+        assert lib.mfrt_memcpy(after.ctypes.data, dev, after.nbytes) == 0
+        for s, d, size in zip(source, target, sizes):
+            before[d:d + size] = before[s:s + size]
+        assert np.array_equal(after, before)
+    finally:
+        pool.destroy()
+        bm.uninitialize()
