@@ -7,7 +7,8 @@
 //             (a stable counting sort of the flat (t,k) order by expert id)
 //   combine   y[t][h] = bf16_rne(fma(w[t][K-1], v[K-1], ... fma(w[t][0], v[0], 0)))
 //
-// Three launches for dispatch (two when the entries fill at most eight rank blocks), one for combine:
+// One launch for a dispatch of up to 4096 entries (MoeDispatchSmallKernel: every token ranks its own entries).
+// Three launches for a larger one (two when the entries fill at most eight rank blocks), one for combine:
 //   MoeHistKernel    per-block expert histograms (wave ballots + LDS); not launched for a few blocks,
 //                    which count one another's entries inside the rank kernel
 //   MoeRankKernel    cross-block scan, stable rank of every entry -> rowOf/srcOf, counts, offsets,
@@ -154,12 +155,11 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
     uint32_t myExpert[kRankRounds];
     uint32_t myRank[kRankRounds];
     uint32_t bad = 0;
-    // blockHist == nullptr: no histogram kernel ran before this launch.  A single block has all it needs in its own
-    // slice histograms and its own flag (a dispatch of up to 1024 entries: 128 tokens at top-8).  The blocks of a
-    // launch of a few count the entries of the other blocks themselves, each for itself: per expert, the entries of
-    // all other blocks and those of the blocks before it (plain counts, so LDS atomics give the same result every time).
+    // blockHist == nullptr: no histogram kernel ran before this launch.  Its few blocks count the entries of the other
+    // blocks themselves, each for itself: per expert, the entries of all other blocks and those of the blocks before it
+    // (plain counts, so LDS atomics give the same result every time).
     const bool tabled = blockHist != nullptr;
-    const bool counting = !tabled && gridDim.x > 1;
+    const bool counting = !tabled;
     const uint32_t steps = runOrder != nullptr ? kRankSlices / stepSlices : 0;
     uint32_t *others = cum + steps * experts;             // [2][experts], counting only
     for (uint32_t i = threadIdx.x; counting && i < 2 * experts; i += kRankThreads) {
@@ -554,6 +554,189 @@ __global__ __launch_bounds__(64) void MoePermuteTileKernel(const u32x4 *__restri
     }
 }
 
+// The whole dispatch of a small call in one launch: workgroup (token, part of the row) ranks the token's entries
+// itself, against all the others, and stores its part of the row to the K rows; the last workgroup counts the experts.
+// An entry's row is the number of entries that come before it by (expert, index), so every id is compared, as one
+// word with its index, with the words of the token's K entries, and a wave adds its lanes up by counting the bits of
+// the comparison.  Nothing is exchanged between workgroups.
+// What bounds it: the chain of a launch and of its memory round trips (kernel arguments; the ids and the row, side by side; the
+// stores), not bytes, as long as the comparisons stay few: with all parts they grow with tokens * entries.  Dispatch
+// alone, with the rank launch and the permute launch / in one: 16 tokens of 7168 elements at top-8 over 256 experts 12.0 / 4.3 us,
+// 64: 12.3 / 4.9, 128: 13.6 / 6.1, 256: 15.3 / 9.3, 512 (4096 entries): 19.6 / 16.0, 1024: 31.8 / 35.0; 2000 tokens of 1024
+// elements at top-2 12.1 / 7.1, 4096 at top-2 14.8 / 18.6.  So it ends at 4096 entries.  Plain stores leave the rows in
+// the caches, where the experts' kernel finds them (dispatch and combine in turn, 512 tokens: 27.9 us, 29.5 with nontemporal stores).
+constexpr uint32_t kSmallThreads = 256;
+constexpr uint32_t kSmallHold = 2;                      // 128-bit pieces of the row per lane: a part is 512 units at most
+constexpr uint32_t kSmallEntries = 4096;                // the largest such call
+constexpr uint32_t kSmallGroups = 256;                  // rows are cut until there are so many workgroups, one per CU
+constexpr uint32_t kSmallBatch = 4;                     // ids per lane requested together by the counting workgroup
+typedef int32_t i32x4a __attribute__((ext_vector_type(4), aligned(4)));
+static_assert(kSmallEntries <= 1u << 16 && kMaxExperts <= 1u << 16, "an entry's expert and index share a word");
+
+// (expert, index) in one word; an id out of range comes behind every entry.
+__device__ __forceinline__ uint32_t SmallKey(int32_t id, uint32_t index, uint32_t experts)
+{
+    return static_cast<uint32_t>(id) < experts ? static_cast<uint32_t>(id) << 16 | index : 0xFFFFFFFFu;
+}
+
+template <uint32_t kSlots>
+__global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(const u32x4 *__restrict__ x, const int32_t *__restrict__ topk,
+                                                                        uint32_t total, uint32_t topK, uint32_t experts,
+                                                                        uint32_t unitsPerRow, uint32_t parts, uint32_t perPart,
+                                                                        u32x4 *__restrict__ out, int32_t *__restrict__ counts,
+                                                                        int32_t *__restrict__ offsets, int32_t *__restrict__ rowOf,
+                                                                        int32_t *__restrict__ srcOf, uint32_t *__restrict__ status)
+{
+    __shared__ uint32_t lds[kMaxExperts + kSmallThreads / 64];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = threadIdx.x >> 6;
+    if (blockIdx.x == gridDim.x - 1) {
+        uint32_t *perWave = lds + kMaxExperts;
+        for (uint32_t e = threadIdx.x; e < kMaxExperts; e += kSmallThreads) {
+            lds[e] = 0;
+        }
+        __syncthreads();
+        uint32_t bad = 0;
+        for (uint32_t i0 = threadIdx.x; i0 < total; i0 += kSmallBatch * kSmallThreads) {
+            int32_t id[kSmallBatch];
+#pragma unroll
+            for (uint32_t q = 0; q < kSmallBatch; ++q) {
+                id[q] = i0 + q * kSmallThreads < total ? topk[i0 + q * kSmallThreads] : 0;
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < kSmallBatch; ++q) {
+                if (i0 + q * kSmallThreads < total) {
+                    if (static_cast<uint32_t>(id[q]) < experts) {
+                        atomicAdd(&lds[id[q]], 1u);     // plain counts: the same whatever the order
+                    } else {
+                        bad = 1;
+                    }
+                }
+            }
+        }
+        bad = __syncthreads_or(static_cast<int>(bad)) != 0 ? 1u : 0u;
+        constexpr uint32_t kPer = kMaxExperts / kSmallThreads;   // neighbouring experts per thread
+        uint32_t mine[kPer];
+        uint32_t incl = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < kPer; ++j) {
+            mine[j] = lds[threadIdx.x * kPer + j];
+            incl += mine[j];
+        }
+        const uint32_t sum = incl;
+#pragma unroll
+        for (uint32_t step = 1; step < 64; step <<= 1) {
+            const uint32_t up = __shfl_up(incl, step, 64);
+            incl += lane >= step ? up : 0u;
+        }
+        if (lane == 63) {
+            perWave[wave] = incl;
+        }
+        __syncthreads();
+        uint32_t run = incl - sum;
+        for (uint32_t w = 0; w < wave; ++w) {
+            run += perWave[w];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kPer; ++j) {
+            const uint32_t e = threadIdx.x * kPer + j;
+            if (e < experts) {
+                counts[e] = static_cast<int32_t>(mine[j]);
+                offsets[e] = static_cast<int32_t>(run);
+            }
+            run += mine[j];
+        }
+        if (threadIdx.x == 0) {
+            status[0] = bad;
+        }
+        return;
+    }
+    const uint32_t token = blockIdx.x / parts;
+    const uint32_t part = blockIdx.x - token * parts;
+    const uint32_t begin = part * perPart;
+    const uint32_t end = begin + perPart < unitsPerRow ? begin + perPart : unitsPerRow;
+    const MF_GLOBAL u32x4 *src = reinterpret_cast<const MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(x)) +
+                                 static_cast<uint64_t>(token) * unitsPerRow;
+    MF_GLOBAL u32x4 *dst = reinterpret_cast<MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(out));
+    u32x4 v[kSmallHold];
+#pragma unroll
+    for (uint32_t j = 0; j < kSmallHold; ++j) {
+        const uint32_t u = begin + j * kSmallThreads + threadIdx.x;
+        if (u < end) {
+            v[j] = src[u];
+        }
+    }
+    // An entry as one word, expert above index: what comes before the token's slots is what compares below their words.
+    // Every wave looks at a quarter of the ids, for all slots.
+    const uint32_t first = token * topK;
+    uint32_t own[kSlots];
+    uint32_t before[kSlots];
+#pragma unroll
+    for (uint32_t k = 0; k < kSlots; ++k) {
+        own[k] = k < topK ? SmallKey(topk[first + k], first + k, experts) : 0u;
+        before[k] = 0;
+    }
+    for (uint32_t c = wave * 256; c < total; c += 4 * kSmallThreads) {
+        const uint32_t at = c + lane * 4;
+        i32x4a id = {-1, -1, -1, -1};
+        if (at + 3 < total) {
+            id = *reinterpret_cast<const i32x4a *>(topk + at);
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < 3; ++i) {
+                if (at + i < total) {
+                    id[i] = topk[at + i];
+                }
+            }
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            const uint32_t key = SmallKey(id[i], at + i, experts);
+#pragma unroll
+            for (uint32_t k = 0; k < kSlots; ++k) {
+                before[k] += __popcll(__ballot(key < own[k]));
+            }
+        }
+    }
+    uint32_t mine = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kSlots; ++k) {
+        mine = lane == k ? before[k] : mine;
+    }
+    if (lane < kSlots) {
+        lds[kMaxTopK * (1 + wave) + lane] = mine;
+    }
+    __syncthreads();
+    if (threadIdx.x < topK) {
+        uint32_t row = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < kSmallThreads / 64; ++w) {
+            row += lds[kMaxTopK * (1 + w) + threadIdx.x];
+        }
+        lds[threadIdx.x] = static_cast<uint32_t>(topk[first + threadIdx.x]) < experts ? row : 0xFFFFFFFFu;
+    }
+    __syncthreads();
+    if (part == 0 && threadIdx.x < topK) {
+        const int32_t row = static_cast<int32_t>(lds[threadIdx.x]);
+        rowOf[first + threadIdx.x] = row;
+        if (srcOf != nullptr && row >= 0) {
+            srcOf[row] = static_cast<int32_t>(first + threadIdx.x);
+        }
+    }
+    for (uint32_t k = 0; k < topK; ++k) {
+        const uint32_t row = lds[k];
+        if (row != 0xFFFFFFFFu) {
+#pragma unroll
+            for (uint32_t j = 0; j < kSmallHold; ++j) {
+                const uint32_t u = begin + j * kSmallThreads + threadIdx.x;
+                if (u < end) {
+                    RowStore<0>(dst + static_cast<uint64_t>(row) * unitsPerRow + u, v[j]);
+                }
+            }
+        }
+    }
+}
+
 __device__ __forceinline__ float Bf16Lo(uint32_t w)
 {
     return __uint_as_float(w << 16);
@@ -827,6 +1010,31 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
     uint32_t *blockHist = blockBad + histStride;
     const size_t histLds = static_cast<size_t>(kRankSlices) * experts * sizeof(uint32_t);
     const uint32_t upr = hidden / 8;
+    if (total <= kSmallEntries) {   // where the line lies: see the kernel
+        const bool rows = x != nullptr && out != nullptr;
+        const uint32_t least = (upr + kSmallHold * kSmallThreads - 1) / (kSmallHold * kSmallThreads);
+        const uint32_t most = (upr + 63) / 64;
+        uint32_t parts = (kSmallGroups + tokens - 1) / tokens;
+        parts = parts < least ? least : parts > most ? most : parts;
+        const uint32_t perPart = rows ? ((upr + parts - 1) / parts + 7) / 8 * 8 : 0;   // whole cache lines
+        parts = rows ? (upr + perPart - 1) / perPart : 1;
+#define MF_DISPATCH_SMALL(SLOTS)                                                                                       \
+    hipLaunchKernelGGL(MoeDispatchSmallKernel<SLOTS>, dim3(tokens * parts + 1), dim3(kSmallThreads), 0, s,              \
+                       static_cast<const u32x4 *>(x), static_cast<const int32_t *>(topk), total, topK, experts, upr, parts, perPart, \
+                       static_cast<u32x4 *>(out), static_cast<int32_t *>(counts), static_cast<int32_t *>(offsets),      \
+                       static_cast<int32_t *>(rowOf), static_cast<int32_t *>(srcOf), status)
+        if (topK <= 2) {
+            MF_DISPATCH_SMALL(2);
+        } else if (topK <= 4) {
+            MF_DISPATCH_SMALL(4);
+        } else if (topK <= 8) {
+            MF_DISPATCH_SMALL(8);
+        } else {
+            MF_DISPATCH_SMALL(16);
+        }
+#undef MF_DISPATCH_SMALL
+        return static_cast<int>(hipGetLastError());
+    }
     // The output-ordered tile permute needs the token rows of one step (a block of kRankBlock entries, or a half, a
     // quarter ... down to one slice of 64 entries: stepEntries / topK tokens) to stay in an XCD's 4 MiB L2 while the
     // step's rows are written, and enough steps for the eight streams.  It wins on every shape of whole cache lines
@@ -837,8 +1045,7 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
     while (stepSlices > 1 && static_cast<uint64_t>(stepSlices * 64 / topK + 1) * hidden * 2 > 2200000ull) {
         stepSlices /= 2;
     }
-    // a small call is cut finer, so that every XCD gets steps to work on (256 / 512 tokens of 7168 elements at top-8:
-    // 24 / 28 us per dispatch, 34 / 35 us with the loop kernel, whose single wave per token writes its 112 KiB alone)
+    // a call of few blocks is cut finer, so that every XCD gets steps to work on
     while (stepSlices > 1 && static_cast<uint64_t>(blocks) * (kRankSlices / stepSlices) < 2 * kTileStreams) {
         stepSlices /= 2;
     }
@@ -851,20 +1058,18 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
                        hidden % 64 == 0 && static_cast<uint64_t>(stepEntries / topK + 1) * hidden * 2 <= 2200000ull &&
                        stepsPerBlock * experts <= 4096 && tileGrid <= 0x7FFFFFFFull;
     // Up to kCountingBlocks blocks rank without a histogram launch in front of them: every block counts the entries
-    // of the others itself.  129 / 256 / 512 / 1024 tokens of 7168 elements at top-8, 256 experts: 13.3 / 15.5 / 20.1 /
-    // 29.5 us per dispatch against 22.0 / 24.1 / 27.7 / 35.1 with the launch; 640 tokens over 512 experts 26 against 38.
+    // of the others itself.  1024 tokens of 7168 elements at top-8, 256 experts: 29.5 us per dispatch against 35.1 with the
+    // launch; 640 tokens over 512 experts 26 against 38.
     // At sixteen blocks the two are level (50.5 us), at thirty-two the counting costs 10 us; over 8 or 16 experts,
     // where the counts of a wave land on few LDS words, eight blocks are level (23.9 against 23.4 us) and sixteen
     // lose 4 us.
-    const bool counting = blocks > 1 && blocks <= kCountingBlocks;
+    const bool counting = blocks <= kCountingBlocks;
     const size_t rankLds = histLds + (experts + kRankThreads + kRankSlices + (tiles ? stepsPerBlock * experts : 0) +
                                       (counting ? 2 * experts : 0)) * sizeof(uint32_t);
     const uint64_t tableBytes = 256 + histStride * sizeof(uint32_t) + static_cast<uint64_t>(histStride) * experts * sizeof(uint32_t);
     int2 *runOrder = tiles ? reinterpret_cast<int2 *>(static_cast<char *>(workspace) + (tableBytes + 15) / 16 * 16) : nullptr;
-    if (blocks == 1 || counting) {
-        blockHist = nullptr;   // one block ranks from its own histograms: no launch in front of it (16 / 64 / 128 tokens of
-                               // 7168 elements at top-8: 12 / 12.5 / 14 us per dispatch; 22 / 23 / 24 us before, with the
-                               // histogram launch and the token-ordered permute); a few blocks count for themselves
+    if (counting) {
+        blockHist = nullptr;
     } else {
         hipLaunchKernelGGL(MoeHistKernel, dim3(blocks), dim3(kRankThreads), histLds, s, static_cast<const int32_t *>(topk),
                            total, experts, blockHist, histStride, blockBad);

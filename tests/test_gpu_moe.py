@@ -398,3 +398,33 @@ def test_full_size_local_share(gpu, oracle):
         y.free()
     finally:
         _free(bufs)
+
+
+@pytest.mark.parametrize("T,H,K,E", [
+    (1, 8, 1, 1), (1, 8, 16, 512), (255, 8, 1, 3), (257, 520, 1, 512), (64, 1032, 16, 512), (63, 4104, 4, 8), (171, 7168, 6, 256),
+    (4096, 16, 1, 2), (1365, 24, 3, 7), (512, 136, 8, 64), (256, 4096, 16, 16),    # 4095 and 4096 entries: the last in one launch
+    (4097, 16, 1, 2), (1366, 24, 3, 7), (513, 1024, 8, 64),                        # the first beyond
+])
+def test_dispatch_around_the_one_launch_form(gpu, oracle, T, H, K, E):
+    """Tails of the ids behind whole vectors and waves, parts of rows that end inside a lane's piece, every width of the
+    slot loop, ids out of range, and the permutation alone."""
+    x, topk, _ = _inputs(oracle, 0x5A + T, T, H, K, E)
+    late = topk.copy()
+    late[0, 0], late[T // 2, K - 1] = -1, E
+    for ids in (topk, late):
+        out_of_range = (ids < 0) | (ids >= E)
+        sent = np.where(out_of_range, E, ids).astype(np.int32)
+        exp_out, exp_counts, exp_offsets, exp_row, exp_src = _oracle_dispatch(oracle, x, sent, E + 1)
+        valid = T * K - int(out_of_range.sum())
+        for with_rows in (True, False):
+            bufs = _gpu_dispatch(gpu, x, ids, E, with_rows)
+            try:
+                assert _fetch(bufs["ws"], np.uint32, (1,))[0] == int(valid != T * K)
+                assert np.array_equal(_fetch(bufs["counts"], np.int32, (E,)), exp_counts[:E])
+                assert np.array_equal(_fetch(bufs["offsets"], np.int32, (E,)), exp_offsets[:E])
+                assert np.array_equal(_fetch(bufs["row_of"], np.int32, (T * K,)), np.where(out_of_range.reshape(-1), -1, exp_row))
+                assert np.array_equal(_fetch(bufs["src_of"], np.int32, (valid,)), exp_src[:valid])
+                if with_rows:
+                    assert np.array_equal(_fetch(bufs["out"], np.uint16, (valid, H)), exp_out[:valid])
+            finally:
+                _free(bufs)
