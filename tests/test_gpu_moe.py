@@ -428,3 +428,21 @@ def test_dispatch_around_the_one_launch_form(gpu, oracle, T, H, K, E):
                     assert np.array_equal(_fetch(bufs["out"], np.uint16, (valid, H)), exp_out[:valid])
             finally:
                 _free(bufs)
+
+
+@pytest.mark.parametrize("T,H,K,E", [
+    (4100, 10304, 2, 16),     # 84 MB of rows, the first to be read ahead of the permute; nine rank blocks, a last one of a few entries
+    (4090, 10304, 2, 16),     # eight blocks, which need no histogram launch
+    (14500, 8192, 1, 7),      # 238 MB: more than is read ahead
+])
+def test_rows_read_ahead_of_the_permute(gpu, oracle, T, H, K, E):
+    x = np.arange(T * H, dtype=np.uint32).astype(np.uint16).reshape(T, H) ^ (np.arange(T, dtype=np.uint16)[:, None] * 3)
+    topk = np.random.default_rng(T).integers(0, E, (T, K)).astype(np.int32)
+    bufs = _gpu_dispatch(gpu, x, topk, E)
+    try:
+        order = np.argsort(topk.reshape(-1), kind="stable")
+        assert np.array_equal(_fetch(bufs["src_of"], np.int32, (T * K,)), order)
+        assert np.array_equal(_fetch(bufs["counts"], np.int32, (E,)), np.bincount(topk.reshape(-1), minlength=E))
+        assert np.array_equal(_fetch(bufs["out"], np.uint16, (T * K, H)), x[order // K])
+    finally:
+        _free(bufs)
