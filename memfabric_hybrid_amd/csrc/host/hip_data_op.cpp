@@ -135,21 +135,11 @@ HipDataOp::Result HipDataOp::Run(void *const *src, void *const *dst, const uint6
 
     if (!srcPageable && !dstPageable) {
         static_assert(sizeof(void *) == sizeof(uint64_t), "64-bit addresses expected");
-        int ret = engine.Submit(reinterpret_cast<const uint64_t *>(src), reinterpret_cast<const uint64_t *>(dst), len, n,
-                                RouteOf(srcOnHost, dstOnHost), stream, nullptr, 0, unordered);
-        if (ret != BM_OK) {
-            return ret;
-        }
-        if (!async) {
-            uint64_t bytes = 0;
-            if (n <= 4096) {   // a long table is not worth adding up: such a batch waits on the stream
-                for (uint32_t i = 0; i < n; ++i) {
-                    bytes += len[i];
-                }
-            }
-            return engine.WaitStream(stream, bytes);
-        }
-        return BM_OK;
+        const auto *from = reinterpret_cast<const uint64_t *>(src);
+        const auto *to = reinterpret_cast<const uint64_t *>(dst);
+        const int route = RouteOf(srcOnHost, dstOnHost);
+        return async ? engine.Submit(from, to, len, n, route, stream, nullptr, 0, unordered)
+                     : engine.SubmitAndWait(from, to, len, n, route, stream);
     }
 
     // Host DRAM to host DRAM with a pageable side: both buffers are only a CPU

@@ -55,6 +55,7 @@ struct ThreadLease {
     bool adopted = false;           // taken over from a thread that ended: its queued kernels ran on streams unknown here
     uint64_t *doneWord = nullptr;   // pinned; a one-lane launch stores doneSeq there behind a blocking copy
     uint32_t doneSeq = 0;
+    void *doneCounter = nullptr;    // device memory, for launches that store the word themselves
     uint64_t pendingBytes = 0;      // bytes of the copies queued on `stream` since the thread last waited for it
     void *bounce = nullptr;
     uint64_t bounceBytes = 0;
@@ -105,6 +106,10 @@ struct ThreadLease {
         if (doneWord != nullptr) {
             (void)mfrt_free_host(doneWord);
             doneWord = nullptr;
+        }
+        if (doneCounter != nullptr) {
+            (void)mfrt_free_device(doneCounter);
+            doneCounter = nullptr;
         }
         for (uint32_t i = 0; i < XcopyEngine::kFanStreams; ++i) {
             if (fanEvent[i] != nullptr) {
@@ -1202,6 +1207,88 @@ int XcopyEngine::DrainThread()
     return WaitStream(t_ctx.lease->stream, t_ctx.lease->pendingBytes);
 }
 
+namespace {
+
+bool HasDoneWord(ThreadLease &lease)
+{
+    if (lease.doneWord == nullptr) {
+        lease.doneWord = static_cast<uint64_t *>(mfrt_alloc_host(64));
+        if (lease.doneWord != nullptr) {
+            *lease.doneWord = 0;
+            lease.doneSeq = 0;
+        }
+    }
+    return lease.doneWord != nullptr;
+}
+
+bool HasDoneCounter(ThreadLease &lease)
+{
+    if (lease.doneCounter == nullptr) {
+        lease.doneCounter = mfrt_alloc_device(64);
+        if (lease.doneCounter != nullptr && mfrt_memset(lease.doneCounter, 0, 64) != 0) {
+            (void)mfrt_free_device(lease.doneCounter);
+            lease.doneCounter = nullptr;
+        }
+    }
+    return lease.doneCounter != nullptr;
+}
+
+uint32_t NextDoneSeq(ThreadLease &lease)
+{
+    return ++lease.doneSeq == 0 ? ++lease.doneSeq : lease.doneSeq;   // 0 is the initial contents
+}
+
+// Polls the lease's word for `seq`; false when that takes longer than expected (or the GPU is busy with other work).
+bool PollDone(const ThreadLease &lease, uint32_t seq, uint32_t micros)
+{
+    const auto start = std::chrono::steady_clock::now();
+    for (uint32_t polls = 1;; ++polls) {
+        if (__atomic_load_n(lease.doneWord, __ATOMIC_ACQUIRE) == seq) {
+            return true;
+        }
+        if ((polls & 63u) == 0 && std::chrono::steady_clock::now() - start > std::chrono::microseconds(micros)) {
+            return false;
+        }
+    }
+}
+
+}  // namespace
+
+int XcopyEngine::SubmitAndWait(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, int route, void *stream)
+{
+    uint64_t bytes = 0;
+    if (n <= 4096) {   // a longer table is not worth adding up: such a batch waits on the stream
+        for (uint32_t i = 0; i < n; ++i) {
+            bytes += len[i];
+        }
+    }
+    // Up to here a launch that stores the word itself is the faster one (the kernel has the figures).
+    const uint64_t doneMax = route == MFRT_ROUTE_FROM_HOST ? kDoneFromHostBytes : kDoneBytes;
+    InlinePlan plan;
+    if (n <= kInlineSegs && bytes != 0 && bytes <= doneMax && Started() && mfrt_bind_thread() == 0 &&
+        BuildInlineDirect(src, dst, len, n, kDeepUnits, plan)) {
+        ThreadLease &lease = t_ctx.Lease();
+        if (HasDoneWord(lease) && HasDoneCounter(lease)) {
+            const uint32_t seq = NextDoneSeq(lease);
+            const int err = mfk_xcopy_done(&plan, route, lease.doneWord, seq, lease.doneCounter, stream);
+            if (err != 0) {
+                MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(err));
+            }
+            g_launches.fetch_add(1, std::memory_order_relaxed);
+            if (stream == lease.stream) {
+                lease.pendingBytes = 0;
+            }
+            const int waited = PollDone(lease, seq, kSpinMicros) ? 0 : mfrt_stream_sync(stream);
+            if (waited != 0) {
+                MF_FAIL(BM_ERROR, "copy failed on the GPU: " << mfrt_error_string(waited));
+            }
+            return BM_OK;
+        }
+    }
+    const int ret = Submit(src, dst, len, n, route, stream, nullptr, 0, false);
+    return ret != BM_OK ? ret : WaitStream(stream, bytes);
+}
+
 // A blocking call is a launch and a wait.  hipStreamSynchronize first has to put a marker with a
 // completion signal behind the kernel and then takes 7 us to see it fire, whatever the wait policy
 // of the device (measured: 16.1 us per blocking 9 MB batch with the default policy and with
@@ -1227,26 +1314,11 @@ int XcopyEngine::WaitStream(void *stream, uint64_t bytes)
     }
     if (bytes != 0 && bytes <= kSpinBytes) {
         ThreadLease &lease = t_ctx.Lease();
-        if (lease.doneWord == nullptr) {
-            lease.doneWord = static_cast<uint64_t *>(mfrt_alloc_host(64));
-            if (lease.doneWord != nullptr) {
-                *lease.doneWord = 0;
-                lease.doneSeq = 0;
-            }
-        }
-        if (lease.doneWord != nullptr) {
-            const uint32_t seq = ++lease.doneSeq == 0 ? ++lease.doneSeq : lease.doneSeq;   // 0 is the initial contents
-            if (mfk_xcopy_signal(lease.doneWord, seq, stream) == 0) {   // not counted by LaunchCount(): it moves no data
-                const auto start = std::chrono::steady_clock::now();
-                for (uint32_t polls = 1;; ++polls) {
-                    if (__atomic_load_n(lease.doneWord, __ATOMIC_ACQUIRE) == seq) {
-                        return BM_OK;
-                    }
-                    if ((polls & 63u) == 0 &&
-                        std::chrono::steady_clock::now() - start > std::chrono::microseconds(kSpinMicros)) {
-                        break;   // longer than expected (or the GPU is busy with other work): sleep on the stream instead
-                    }
-                }
+        if (HasDoneWord(lease)) {
+            const uint32_t seq = NextDoneSeq(lease);
+            // (the signal is not counted by LaunchCount(): it moves no data)
+            if (mfk_xcopy_signal(lease.doneWord, seq, stream) == 0 && PollDone(lease, seq, kSpinMicros)) {
+                return BM_OK;
             }
         }
     }

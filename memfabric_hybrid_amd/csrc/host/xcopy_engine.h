@@ -169,6 +169,11 @@ public:
     static constexpr uint64_t kSpinBytes = 256ull << 20;
     static constexpr uint32_t kSpinMicros = 200;
     int WaitStream(void *stream, uint64_t bytes);
+    // Submit() and WaitStream() of a blocking copy; one of up to kDoneBytes (from the host: kDoneFromHostBytes, beyond which
+    // written-through stores cost more than the launch they save) goes out as a launch that tells the host itself.
+    static constexpr uint64_t kDoneBytes = 1ull << 20;
+    static constexpr uint64_t kDoneFromHostBytes = 128ull << 10;
+    int SubmitAndWait(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, int route, void *stream);
     // Work that another part of the library has queued on `stream`: if it is the calling thread's own stream, the next
     // DrainThread() takes `bytes` into account when it chooses between polling and sleeping (~0: sleep).
     void NoteQueued(void *stream, uint64_t bytes);

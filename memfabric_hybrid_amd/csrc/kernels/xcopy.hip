@@ -77,9 +77,16 @@ __device__ __forceinline__ void StoreUnit(uint64_t addr, u32x4 v)
     }
 }
 
+template <int kStore>
 __device__ __forceinline__ void CopyByte(uint64_t src, uint64_t dst)
 {
-    *reinterpret_cast<GDstByte>(dst) = *reinterpret_cast<GSrcByte>(src);
+    GDstByte p = reinterpret_cast<GDstByte>(dst);
+    const uint8_t v = *reinterpret_cast<GSrcByte>(src);
+    if (kStore == kStoreThrough) {
+        asm volatile("global_store_byte %0, %1, off sc0 sc1 nt" : : "v"(p), "v"(static_cast<uint32_t>(v)) : "memory");
+    } else {
+        *p = v;
+    }
 }
 
 constexpr uint32_t kDepth = 4;                          // 128-bit loads in flight per lane
@@ -146,11 +153,11 @@ __device__ __forceinline__ void CopyChunk(uint64_t src, uint64_t dst, uint64_t l
         }
     }
     if (k == 0 && tid < g.head) {
-        CopyByte(src + tid, dst + tid);
+        CopyByte<kStore>(src + tid, dst + tid);
     }
     if (u0 + units >= g.body && tid < g.tail) {
         const uint64_t off = g.head + g.body * kUnitBytes + tid;
-        CopyByte(src + off, dst + off);
+        CopyByte<kStore>(src + off, dst + off);
     }
 }
 
@@ -167,7 +174,51 @@ __device__ __forceinline__ uint64_t ReadLane64(uint64_t v, uint32_t lane)
 // trip; the owner of a chunk is then found with two ballots and read out of
 // the owning lane.  (A scalar search would chain three dependent loads, each
 // a full L2 round trip, before the first byte of payload is requested.)
-//
+struct InlineChunk {
+    uint64_t src;
+    uint64_t dst;
+    uint32_t len;
+    uint32_t k;
+};
+
+struct InlineRows {
+    uint32_t f0, f1, l0, l1;
+    uint64_t s0, s1, d0, d1;
+
+    __device__ __forceinline__ explicit InlineRows(const InlinePlan &p)
+    {
+        const uint32_t lane = threadIdx.x & 63u;
+        f0 = p.first[lane];
+        f1 = p.first[lane + 64];
+        s0 = p.src[lane];
+        s1 = p.src[lane + 64];
+        d0 = p.dst[lane];
+        d1 = p.dst[lane + 64];
+        l0 = p.len[lane];
+        l1 = p.len[lane + 64];
+    }
+    // rows are ordered by prefix: the owner is the last row whose prefix is <= c
+    __device__ __forceinline__ InlineChunk Owner(uint32_t c) const
+    {
+        const uint32_t below = __popcll(__ballot(f0 <= c)) + __popcll(__ballot(f1 <= c));
+        const uint32_t s = below - 1;
+        const uint32_t row = s & 63u;
+        InlineChunk r;
+        if (s < 64) {
+            r.src = ReadLane64(s0, row);
+            r.dst = ReadLane64(d0, row);
+            r.len = __builtin_amdgcn_readlane(l0, row);
+            r.k = c - __builtin_amdgcn_readlane(f0, row);
+        } else {
+            r.src = ReadLane64(s1, row);
+            r.dst = ReadLane64(d1, row);
+            r.len = __builtin_amdgcn_readlane(l1, row);
+            r.k = c - __builtin_amdgcn_readlane(f1, row);
+        }
+        return r;
+    }
+};
+
 // kHold: every wave keeps its loaded data until `holdTicks` of the constant-rate clock after its own
 // start, which separates the read burst of the launch from its write burst (HoldNanosFor has the
 // rule); such a launch has one chunk per workgroup: of 4 KiB (kHoldShallow, four loads per lane) or, for
@@ -182,41 +233,15 @@ template <bool kNtLoad, int kStore, int kHold = kHoldNone>
 __global__ __launch_bounds__(kXcopyThreads) void XcopyInlineKernel(const InlinePlan p, uint32_t holdTicks)
 {
     const uint64_t t0 = kHold != kHoldNone ? wall_clock64() : 0;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t f0 = p.first[lane];
-    const uint32_t f1 = p.first[lane + 64];
-    const uint64_t s0 = p.src[lane];
-    const uint64_t s1 = p.src[lane + 64];
-    const uint64_t d0 = p.dst[lane];
-    const uint64_t d1 = p.dst[lane + 64];
-    const uint32_t l0 = p.len[lane];
-    const uint32_t l1 = p.len[lane + 64];
+    const InlineRows rows(p);
     const uint32_t nchunk = p.nchunk;
     const uint32_t units = p.units;
     // The host launches at most nchunk workgroups (and never this kernel for an empty plan), so
     // the first chunk needs no bound check and the table loads above are not held behind one.
     uint32_t c = blockIdx.x;
     do {
-        // rows are ordered by prefix: the owner is the last row whose prefix is <= c
-        const uint32_t below = __popcll(__ballot(f0 <= c)) + __popcll(__ballot(f1 <= c));
-        const uint32_t s = below - 1;
-        const uint32_t row = s & 63u;
-        uint64_t src;
-        uint64_t dst;
-        uint32_t len;
-        uint32_t first;
-        if (s < 64) {
-            src = ReadLane64(s0, row);
-            dst = ReadLane64(d0, row);
-            len = __builtin_amdgcn_readlane(l0, row);
-            first = __builtin_amdgcn_readlane(f0, row);
-        } else {
-            src = ReadLane64(s1, row);
-            dst = ReadLane64(d1, row);
-            len = __builtin_amdgcn_readlane(l1, row);
-            first = __builtin_amdgcn_readlane(f1, row);
-        }
-        CopyChunkHeld<kNtLoad, kStore, kHold>(src, dst, len, c - first, units, t0, holdTicks);
+        const InlineChunk r = rows.Owner(c);
+        CopyChunkHeld<kNtLoad, kStore, kHold>(r.src, r.dst, r.len, r.k, units, t0, holdTicks);
         c += gridDim.x;
     } while (c < nchunk);
 }
@@ -310,11 +335,11 @@ __device__ __forceinline__ void CopyChunkHeld(uint64_t src, uint64_t dst, uint64
         }
     }
     if (k == 0 && tid < g.head) {
-        CopyByte(src + tid, dst + tid);
+        CopyByte<kStore>(src + tid, dst + tid);
     }
     if (u0 + kWindowUnits >= g.body && tid < g.tail) {
         const uint64_t off = g.head + g.body * kUnitBytes + tid;
-        CopyByte(src + off, dst + off);
+        CopyByte<kStore>(src + off, dst + off);
     }
 }
 
@@ -323,38 +348,13 @@ __device__ __forceinline__ void CopyChunkHeld(uint64_t src, uint64_t dst, uint64
 template <bool kNtLoad, int kStore>
 __global__ __launch_bounds__(64) void XcopyWindowKernel(const InlinePlan p, uint32_t period, uint32_t seq)
 {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t f0 = p.first[lane];
-    const uint32_t f1 = p.first[lane + 64];
-    const uint64_t s0 = p.src[lane];
-    const uint64_t s1 = p.src[lane + 64];
-    const uint64_t d0 = p.dst[lane];
-    const uint64_t d1 = p.dst[lane + 64];
-    const uint32_t l0 = p.len[lane];
-    const uint32_t l1 = p.len[lane + 64];
+    const InlineRows rows(p);
     const uint32_t nchunk = p.nchunk;
     const uint32_t half = period / 2;
     uint64_t slot = AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * half / gridDim.x;
     for (uint32_t c = blockIdx.x; c < nchunk; c += gridDim.x) {
-        const uint32_t below = __popcll(__ballot(f0 <= c)) + __popcll(__ballot(f1 <= c));
-        const uint32_t s = below - 1;
-        const uint32_t row = s & 63u;
-        uint64_t src;
-        uint64_t dst;
-        uint32_t len;
-        uint32_t first;
-        if (s < 64) {
-            src = ReadLane64(s0, row);
-            dst = ReadLane64(d0, row);
-            len = __builtin_amdgcn_readlane(l0, row);
-            first = __builtin_amdgcn_readlane(f0, row);
-        } else {
-            src = ReadLane64(s1, row);
-            dst = ReadLane64(d1, row);
-            len = __builtin_amdgcn_readlane(l1, row);
-            first = __builtin_amdgcn_readlane(f1, row);
-        }
-        CopyChunkWindowed<kNtLoad, kStore>(src, dst, len, c - first, slot, half);
+        const InlineChunk r = rows.Owner(c);
+        CopyChunkWindowed<kNtLoad, kStore>(r.src, r.dst, r.len, r.k, slot, half);
         slot += period;
     }
 }
@@ -387,6 +387,55 @@ __global__ void XcopySignalKernel(uint64_t *mask, uint32_t maskValue)
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         __hip_atomic_store(mask, static_cast<uint64_t>(maskValue), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
+}
+
+// A short blocking copy that says itself when it is done.  It is bound by the chain of launch, kernel and the word's way to the host;
+// a signal launch behind the copy adds a launch to the host's side and a launch boundary to the GPU's.  Blocking calls with the
+// signal launch / with this kernel: 16 KiB in HBM 10.5 / 8.4 us, 1 MiB 10.7 / 9.5, 122 blocks of 8 KiB 11.9 / 10.6, 32 x 4 KiB to the
+// host 12.2 / 11.0.  Workgroups of 16 KiB (four 128-bit accesses per lane of four waves): every workgroup beyond the first
+// costs an atomic on one word, so 4 KiB ones lose at 1 MiB (11.6) and the form as a whole at 4 MiB (11.0 / 11.5); 64 KiB in one
+// workgroup of sixteen waves gain nothing in HBM (8.9 / 8.9) and lose over the link (from the host 12.5 / 10.6).
+constexpr uint32_t kDoneMaxChunks = 4096;
+struct DoneMark {
+    uint64_t *word;         // pinned host memory, polled by the caller
+    uint32_t *counter;      // device memory, 0 between launches
+    uint32_t value;
+};
+
+// Every store of the launch is written through (kStoreThrough), so it has reached memory once vmcnt says so, and the last
+// workgroup to count itself done may tell the host without waiting for the end of the kernel.
+__device__ __forceinline__ void MarkDone(const DoneMark &mark)
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x != 0) {
+        return;
+    }
+    if (gridDim.x > 1) {
+        if (__hip_atomic_fetch_add(mark.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1) {
+            return;
+        }
+        __hip_atomic_store(mark.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    __hip_atomic_store(mark.word, static_cast<uint64_t>(mark.value), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+template <bool kNtLoad>
+__global__ __launch_bounds__(kXcopyThreads) void XcopySingleDoneKernel(uint64_t src, uint64_t dst, uint32_t len, uint32_t units,
+                                                                       DoneMark mark)
+{
+    CopyChunk<kNtLoad, kStoreThrough>(src, dst, len, blockIdx.x, units);
+    MarkDone(mark);
+}
+
+template <bool kNtLoad>
+__global__ __launch_bounds__(kXcopyThreads) void XcopyInlineDoneKernel(const InlinePlan p, DoneMark mark)
+{
+    const InlineRows rows(p);
+    const InlineChunk r = rows.Owner(blockIdx.x);
+    CopyChunk<kNtLoad, kStoreThrough>(r.src, r.dst, r.len, r.k, p.units);
+    MarkDone(mark);
 }
 
 // The table form: any number of segments, {src, dst, len} triples in memory.  A wave finds the owner of its
@@ -1034,6 +1083,33 @@ extern "C" int mfk_xcopy_inline(const void *inlinePlan, int route, uint32_t grid
     return err != 0 ? err : mf::Signal(mask, maskValue, s);
 }
 
+extern "C" int mfk_xcopy_done(const void *inlinePlan, int route, void *word, uint32_t value, void *counter, void *stream)
+{
+    using namespace mf;
+    const InlinePlan &plan = *static_cast<const InlinePlan *>(inlinePlan);
+    const bool single = plan.first[1] == kNoChunk;
+    const uint32_t lanes = (plan.units / kDepth + 63) / 64 * 64;     // a chunk in one step of kDepth accesses per lane
+    if (plan.nchunk == 0 || plan.nchunk > kDoneMaxChunks || lanes == 0 || lanes > kXcopyThreads) {
+        return static_cast<int>(hipErrorInvalidValue);
+    }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    DoneMark mark{static_cast<uint64_t *>(word), static_cast<uint32_t *>(counter), value};
+    uint64_t src = plan.src[0];
+    uint64_t dst = plan.dst[0];
+    uint32_t len = plan.len[0];
+    uint32_t units = plan.units;
+    void *singleArgs[] = {&src, &dst, &len, &units, &mark};
+    void *args[] = {const_cast<InlinePlan *>(&plan), &mark};
+    const bool nt = PolicyOf(route).ntLoad;
+    const void *kernel = nt ? reinterpret_cast<const void *>(&XcopyInlineDoneKernel<true>)
+                            : reinterpret_cast<const void *>(&XcopyInlineDoneKernel<false>);
+    if (single) {
+        kernel = nt ? reinterpret_cast<const void *>(&XcopySingleDoneKernel<true>)
+                    : reinterpret_cast<const void *>(&XcopySingleDoneKernel<false>);
+    }
+    return static_cast<int>(hipLaunchKernel(kernel, dim3(plan.nchunk), dim3(lanes), single ? singleArgs : args, 0, s));
+}
+
 extern "C" uint32_t mfk_xcopy_window_units(void)
 {
     return mf::kWindowUnits;
@@ -1138,6 +1214,7 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
     none.nseg = 1;
     none.units = kXcopyThreads;
     none.groupShift = kGroupShiftMin;
+    // (the copies that store a word of their own are never captured: a blocking call cannot be)
     for (int route = MFRT_ROUTE_HBM; route <= MFRT_ROUTE_FROM_HOST; ++route) {
         (void)WithPolicy(PolicyOf(route), [&](auto ntLoad, auto store) {
             constexpr bool kNt = decltype(ntLoad)::value;

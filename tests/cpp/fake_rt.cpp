@@ -284,6 +284,10 @@ int mfk_xcopy_inline(const void *inlinePlan, int, uint32_t, void *mask, uint32_t
     return 0;
 }
 
+int mfk_xcopy_done(const void *inlinePlan, int route, void *word, uint32_t value, void *counter, void *stream)
+{
+    return counter == nullptr ? -1 : mfk_xcopy_inline(inlinePlan, route, 0, word, value, stream, 0, 0);
+}
 int mfk_xcopy_windows_available(void) { return 1; }
 int mfk_xcopy_prelaunch(void *) { return 0; }
 // The calibration "measures" what the test has put here (all zero: nothing measured, the defaults stay).
