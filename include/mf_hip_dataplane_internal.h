@@ -43,7 +43,7 @@ int32_t mf_bm_copy_batch_replay_threads(smem_bm_t handle, smem_batch_copy_params
 /* Launch-shape knobs.  units: 16-byte units per workgroup chunk (0 = choose
  * per batch); wgPerCu: grid cap in workgroups per CU on HBM routes (0 = the
  * default: one workgroup per chunk, no cap); wgPerCuLink: workgroups per CU
- * on host-link routes (0 = the default, 1). */
+ * on host-link routes (0 = the default, 64 for the whole chip). */
 int32_t mf_xcopy_tune(uint32_t units, uint32_t wgPerCu, uint32_t wgPerCuLink);
 /* Stores held back.  A batch of 960 to 6144 chunks of 4 KiB between HBM addresses (4 to 25 MB in up
  * to 128 segments) is copied 7 to 20 % faster when every wave waits with its stores until the loads of

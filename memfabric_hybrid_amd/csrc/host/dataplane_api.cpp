@@ -152,7 +152,7 @@ MF_EXPORT int32_t mf_xcopy_tune(uint32_t units, uint32_t wgPerCu, uint32_t wgPer
     XcopyTuning &t = XcopyEngine::Instance().Tuning();
     t.unitsOverride = units;
     t.wgPerCu = wgPerCu;                               // 0: no cap, one workgroup per chunk
-    t.wgPerCuLink = wgPerCuLink == 0 ? 1 : wgPerCuLink;
+    t.wgPerCuLink = wgPerCuLink;
     return BM_OK;
 }
 

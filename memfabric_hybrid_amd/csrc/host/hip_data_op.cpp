@@ -13,22 +13,19 @@
 namespace mf {
 namespace {
 
-constexpr uint32_t kRounds = 16;                       // slots of the staging ring
-constexpr uint64_t kRoundBytes = 2ull << 20;           // bytes per slot: ~70 us of CPU memcpy against ~40 us on the link
-constexpr uint64_t kBounceBytes = kRounds * kRoundBytes;
-constexpr uint32_t kAhead = 2;                        // launches queued beyond the slot being emptied (device to pageable memory)
-static_assert(kRounds <= XcopyEngine::kBounceEvents, "one event per staging slot");
+// The staging ring.  A round is a launch, which has a start and an end in which the link is not full (8 MiB move at 55.4 GB/s, 2 MiB at
+// 51.9), so rounds are as long as the ring allows; the first of a copy to the GPU and the last of one from it are short, because
+// the other side waits for them.
+constexpr uint32_t kSlots = 4;
+constexpr uint64_t kRoundBytes = 8ull << 20;           // bytes per slot, the most one round moves
+constexpr uint64_t kRoundMinBytes = 512ull << 10;
+constexpr uint64_t kBounceBytes = kSlots * kRoundBytes;
+constexpr uint32_t kAhead = 2;                         // launches queued beyond the slot being emptied (device to pageable memory)
 
 // Caller memory the GPU cannot address (ordinary pageable host memory) goes through a pinned
 // staging area.  The reference allocates and frees a device buffer per segment for these
 // directions (src/hybm/csrc/data_operation/host/hybm_data_op_sdma.cpp:171-221); here one pinned
 // area per thread, owned by the engine, is filled by the CPU and scattered by one launch.
-
-struct Piece {
-    uint64_t src;
-    uint64_t dst;
-    uint64_t len;
-};
 
 bool AnyPageable(void *const *ptrs, uint32_t n)
 {
@@ -38,6 +35,204 @@ bool AnyPageable(void *const *ptrs, uint32_t n)
         }
     }
     return false;
+}
+
+// Walks the bytes of a batch in rounds.
+class RoundCursor {
+public:
+    RoundCursor(void *const *src, void *const *dst, const uint64_t *len, uint32_t n) : src_(src), dst_(dst), len_(len), n_(n)
+    {
+        for (uint32_t i = 0; i < n; ++i) {
+            left_ += len[i];
+        }
+        Skip();
+    }
+    uint64_t Left() const
+    {
+        return left_;
+    }
+    // The next pieces, at most `bytes` with every piece on a 64-byte boundary of the slot; place(src, dst, len, offset in the slot).
+    template <class Place>
+    void Next(uint64_t bytes, Place place)
+    {
+        uint64_t used = 0;
+        while (i_ < n_ && used < bytes) {
+            const uint64_t rest = len_[i_] - at_;
+            const uint64_t take = rest < bytes - used ? rest : bytes - used;
+            if (take < rest && take < kSliver && used != 0) {
+                break;   // too little of a segment to be worth a piece of its own
+            }
+            place(reinterpret_cast<uint64_t>(src_[i_]) + at_, reinterpret_cast<uint64_t>(dst_[i_]) + at_, take, used);
+            used += (take + 63) & ~63ull;
+            at_ += take;
+            left_ -= take;
+            Skip();
+        }
+    }
+
+private:
+    static constexpr uint64_t kSliver = 4096;
+    void Skip()   // finished and empty segments
+    {
+        while (i_ < n_ && at_ == len_[i_]) {
+            ++i_;
+            at_ = 0;
+        }
+    }
+    void *const *src_;
+    void *const *dst_;
+    const uint64_t *len_;
+    uint32_t n_;
+    uint32_t i_ = 0;
+    uint64_t at_ = 0;
+    uint64_t left_ = 0;
+};
+
+// The launches of one staged copy.  Whatever way it ends, nothing of it is in flight afterwards: its slots are free.
+class StagedLaunches {
+public:
+    explicit StagedLaunches(void *stream) : stream_(stream) {}
+    ~StagedLaunches()
+    {
+        (void)Finish();
+    }
+    int Launch(const std::vector<uint64_t> &src, const std::vector<uint64_t> &dst, const std::vector<uint64_t> &len, int route)
+    {
+        const int ret = XcopyEngine::Instance().SubmitTicket(src.data(), dst.data(), len.data(), static_cast<uint32_t>(len.size()), route,
+                                                             stream_, tickets_[count_ % kSlots]);
+        count_ += ret == BM_OK ? 1 : 0;
+        return ret;
+    }
+    // Waits for launch `index`, one of the last kSlots.
+    int Wait(uint32_t index)
+    {
+        waited_ = index + 1 > waited_ ? index + 1 : waited_;
+        return XcopyEngine::Instance().WaitTicket(tickets_[index % kSlots], stream_);
+    }
+    int Finish()
+    {
+        return waited_ < count_ ? Wait(count_ - 1) : BM_OK;
+    }
+    uint32_t Count() const
+    {
+        return count_;
+    }
+
+private:
+    void *stream_;
+    uint32_t count_ = 0;
+    uint32_t waited_ = 0;
+    uint32_t tickets_[kSlots] = {};
+};
+
+uint64_t RoundBytes(uint64_t wanted)
+{
+    return wanted < kRoundMinBytes ? kRoundMinBytes : wanted > kRoundBytes ? kRoundBytes : wanted & ~63ull;
+}
+
+// Pageable memory to the GPU: the CPU fills a slot while the launches of the slots before it run.  Rounds grow from
+// kRoundMinBytes, so that the link does not wait for the first slot longer than it has to.
+int StageIn(void *const *src, void *const *dst, const uint64_t *len, uint32_t n, void *stream)
+{
+    XcopyEngine &engine = XcopyEngine::Instance();
+    const auto bounce = reinterpret_cast<uint64_t>(engine.ThreadBounce(kBounceBytes));
+    if (bounce == 0) {
+        MF_FAIL(BM_MALLOC_FAILED, "pinned staging allocation failed");
+    }
+    RoundCursor cursor(src, dst, len, n);
+    StagedLaunches launches(stream);
+    std::vector<uint64_t> a, b, l;
+    std::vector<HostCopyHelper::Task> tasks;   // the CPU copies of one round
+    const uint64_t total = cursor.Left();
+    while (cursor.Left() != 0) {
+        const uint32_t round = launches.Count();
+        if (round >= kSlots) {
+            const int ret = launches.Wait(round - kSlots);   // the slot's last reader
+            if (ret != BM_OK) {
+                return ret;
+            }
+        }
+        a.clear();
+        b.clear();
+        l.clear();
+        tasks.clear();
+        const uint64_t slot = bounce + round % kSlots * kRoundBytes;
+        cursor.Next(RoundBytes(total - cursor.Left()), [&](uint64_t from, uint64_t to, uint64_t bytes, uint64_t at) {
+            tasks.push_back(HostCopyHelper::Task{reinterpret_cast<void *>(slot + at), reinterpret_cast<const void *>(from), bytes});
+            a.push_back(slot + at);
+            b.push_back(to);
+            l.push_back(bytes);
+        });
+        HostCopyHelper::Instance().CopySet(tasks.data(), tasks.size());
+        if (round == 0 && cursor.Left() == 0) {
+            return engine.SubmitAndWait(a.data(), b.data(), l.data(), static_cast<uint32_t>(l.size()), MFRT_ROUTE_FROM_HOST, stream);
+        }
+        const int ret = launches.Launch(a, b, l, MFRT_ROUTE_FROM_HOST);
+        if (ret != BM_OK) {
+            return ret;
+        }
+    }
+    return launches.Finish();   // the caller's memory has been consumed before; the copy itself is done as well
+}
+
+// The GPU to pageable memory: the CPU empties a slot while the launches that fill the next ones run.  Rounds shrink to
+// kRoundMinBytes at the end, so that the CPU is not left with a whole slot when the link is done.
+int StageOut(void *const *src, void *const *dst, const uint64_t *len, uint32_t n, void *stream)
+{
+    XcopyEngine &engine = XcopyEngine::Instance();
+    const auto bounce = reinterpret_cast<uint64_t>(engine.ThreadBounce(kBounceBytes));
+    if (bounce == 0) {
+        MF_FAIL(BM_MALLOC_FAILED, "pinned staging allocation failed");
+    }
+    RoundCursor cursor(src, dst, len, n);
+    StagedLaunches launches(stream);
+    std::vector<uint64_t> a, b, l;
+    std::vector<HostCopyHelper::Task> tasks[kSlots];   // the CPU copies of the rounds in flight
+    uint32_t emptied = 0;
+    auto empty = [&]() -> int {
+        const int ret = launches.Wait(emptied);
+        if (ret == BM_OK) {
+            HostCopyHelper::Instance().CopySet(tasks[emptied % kSlots].data(), tasks[emptied % kSlots].size());
+            ++emptied;
+        }
+        return ret;
+    };
+    while (cursor.Left() != 0) {
+        const uint32_t round = launches.Count();
+        a.clear();
+        b.clear();
+        l.clear();
+        tasks[round % kSlots].clear();
+        const uint64_t slot = bounce + round % kSlots * kRoundBytes;
+        cursor.Next(RoundBytes(cursor.Left() / 2), [&](uint64_t from, uint64_t to, uint64_t bytes, uint64_t at) {
+            tasks[round % kSlots].push_back(
+                HostCopyHelper::Task{reinterpret_cast<void *>(to), reinterpret_cast<const void *>(slot + at), bytes});
+            a.push_back(from);
+            b.push_back(slot + at);
+            l.push_back(bytes);
+        });
+        if (round == 0 && cursor.Left() == 0) {
+            const int ret = engine.SubmitAndWait(a.data(), b.data(), l.data(), static_cast<uint32_t>(l.size()), MFRT_ROUTE_TO_HOST, stream);
+            if (ret == BM_OK) {
+                HostCopyHelper::Instance().CopySet(tasks[0].data(), tasks[0].size());
+            }
+            return ret;
+        }
+        int ret = launches.Launch(a, b, l, MFRT_ROUTE_TO_HOST);
+        if (ret == BM_OK && round - emptied >= kAhead) {
+            ret = empty();
+        }
+        if (ret != BM_OK) {
+            return ret;
+        }
+    }
+    while (emptied < launches.Count()) {
+        const int ret = empty();
+        if (ret != BM_OK) {
+            return ret;
+        }
+    }
+    return BM_OK;
 }
 
 int RouteOf(bool srcOnHost, bool dstOnHost)
@@ -164,151 +359,7 @@ HipDataOp::Result HipDataOp::Run(void *const *src, void *const *dst, const uint6
         return BM_OK;
     }
 
-    uint8_t *bounce = static_cast<uint8_t *>(engine.ThreadBounce(kBounceBytes));
-    if (bounce == nullptr) {
-        MF_FAIL(BM_MALLOC_FAILED, "pinned staging allocation failed");
-    }
-    // The staging area is a ring of kRounds slots.  The CPU side (memcpy between caller memory and
-    // a slot) and the GPU side (one fused launch per slot) overlap: towards the GPU the CPU fills
-    // slot r+1 while the launch of slot r runs, away from it the CPU empties slot r-1 while the
-    // launch that fills slot r runs.  An event per slot says when its launch has finished.
-    // 512 KiB rounds were tried for small batches: slower (more launches).  Large transfers take
-    // slots of twice the size: the launch and the event of a round cost the host about 10 us.
-    uint64_t totalBytes = 0;
-    for (uint32_t i = 0; i < n; ++i) {
-        totalBytes += len[i];
-    }
-    const uint64_t roundBytes = totalBytes >= (64ull << 20) ? 2 * kRoundBytes : kRoundBytes;
-    const uint32_t ringSlots = static_cast<uint32_t>(kBounceBytes / roundBytes);
-    std::vector<Piece> pieces;
-    pieces.reserve(n);
-    for (uint32_t i = 0; i < n; ++i) {
-        uint64_t s = reinterpret_cast<uint64_t>(src[i]);
-        uint64_t d = reinterpret_cast<uint64_t>(dst[i]);
-        uint64_t left = len[i];
-        while (left > 0) {
-            const uint64_t take = left > roundBytes ? roundBytes : left;
-            pieces.push_back(Piece{s, d, take});
-            s += take;
-            d += take;
-            left -= take;
-        }
-    }
-    HostCopyHelper &copier = HostCopyHelper::Instance();   // large pieces are copied by two cores
-    struct Round {
-        size_t begin = 0;
-        size_t end = 0;
-        std::vector<uint64_t> staged;   // slot address of every piece of the round
-    };
-    Round rounds[kRounds];
-    std::vector<uint64_t> a;
-    std::vector<uint64_t> b;
-    std::vector<uint64_t> l;
-    std::vector<HostCopyHelper::Task> tasks;   // the CPU copies of one round
-    auto drain = [&](Round &round, uint32_t slot) -> int {   // GPU -> caller: wait for the slot's launch, empty it
-        if (round.begin == round.end) {
-            return BM_OK;
-        }
-        int err = mfrt_event_sync(engine.ThreadBounceEvent(slot));
-        if (err != 0) {
-            MF_FAIL(BM_ERROR, "copy failed on the GPU: " << mfrt_error_string(err));
-        }
-        tasks.clear();
-        for (size_t i = round.begin; i < round.end; ++i) {
-            tasks.push_back(HostCopyHelper::Task{reinterpret_cast<void *>(pieces[i].dst),
-                                                 reinterpret_cast<const void *>(round.staged[i - round.begin]), pieces[i].len});
-        }
-        copier.CopySet(tasks.data(), tasks.size());
-        round.begin = round.end = 0;
-        return BM_OK;
-    };
-    const int route = srcPageable ? MFRT_ROUTE_FROM_HOST : MFRT_ROUTE_TO_HOST;
-    size_t at = 0;
-    uint32_t r = 0;
-    for (; at < pieces.size(); ++r) {
-        const uint32_t slot = r % ringSlots;
-        Round &round = rounds[slot];
-        void *event = engine.ThreadBounceEvent(slot);
-        if (event == nullptr) {
-            MF_FAIL(BM_ERROR, "event creation failed");
-        }
-        if (r >= ringSlots) {   // the slot's previous launch must be over before the slot is reused
-            if (dstPageable) {
-                int ret = drain(round, slot);
-                if (ret != BM_OK) {
-                    return ret;
-                }
-            } else {
-                int err = mfrt_event_sync(event);
-                if (err != 0) {
-                    MF_FAIL(BM_ERROR, "copy failed on the GPU: " << mfrt_error_string(err));
-                }
-            }
-        }
-        a.clear();
-        b.clear();
-        l.clear();
-        tasks.clear();
-        round.staged.clear();
-        round.begin = at;
-        uint64_t used = 0;
-        const uint64_t base = reinterpret_cast<uint64_t>(bounce) + static_cast<uint64_t>(slot) * roundBytes;
-        while (at < pieces.size()) {
-            const uint64_t padded = (pieces[at].len + 63) & ~63ull;  // keep staged pieces 64-byte aligned
-            if (used + padded > roundBytes) {
-                break;
-            }
-            const uint64_t where = base + used;
-            if (srcPageable) {
-                tasks.push_back(HostCopyHelper::Task{reinterpret_cast<void *>(where), reinterpret_cast<const void *>(pieces[at].src),
-                                                     pieces[at].len});
-                a.push_back(where);
-                b.push_back(pieces[at].dst);
-            } else {
-                a.push_back(pieces[at].src);
-                b.push_back(where);
-                round.staged.push_back(where);
-            }
-            l.push_back(pieces[at].len);
-            used += padded;
-            ++at;
-        }
-        round.end = at;
-        if (srcPageable) {
-            copier.CopySet(tasks.data(), tasks.size());
-        }
-        int ret = engine.Submit(a.data(), b.data(), l.data(), static_cast<uint32_t>(l.size()), route, stream, nullptr, 0);
-        if (ret != BM_OK) {
-            return ret;
-        }
-        int err = mfrt_event_record(event, stream);
-        if (err != 0) {
-            MF_FAIL(BM_ERROR, "event record failed: " << mfrt_error_string(err));
-        }
-        // Two launches stay queued while an older slot is emptied: with only one, the next launch is
-        // submitted just as the running one ends, and any delay leaves the GPU idle.
-        if (dstPageable && r >= kAhead) {
-            ret = drain(rounds[(r - kAhead) % ringSlots], (r - kAhead) % ringSlots);
-            if (ret != BM_OK) {
-                return ret;
-            }
-        }
-    }
-    if (dstPageable) {
-        for (uint32_t k = 0; k < ringSlots; ++k) {   // what is still staged, oldest first
-            const uint32_t slot = (r + k) % ringSlots;
-            int ret = drain(rounds[slot], slot);
-            if (ret != BM_OK) {
-                return ret;
-            }
-        }
-    } else {
-        int err = mfrt_stream_sync(stream);   // caller memory has been consumed; the copy itself is done as well
-        if (err != 0) {
-            MF_FAIL(BM_ERROR, "copy failed on the GPU: " << mfrt_error_string(err));
-        }
-    }
-    return BM_OK;
+    return srcPageable ? StageIn(src, dst, len, n, stream) : StageOut(src, dst, len, n, stream);
 }
 
 }  // namespace mf

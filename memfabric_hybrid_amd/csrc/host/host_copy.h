@@ -41,7 +41,7 @@ public:
     void CopySet(const Task *tasks, size_t count);
 
     static constexpr size_t kSplitMin = 512u << 10;
-    static constexpr uint32_t kWorkers = 2;
+    static constexpr uint32_t kWorkers = 3;
 
     uint64_t SharedCopies() const   // sets the helpers took part in (for tests)
     {

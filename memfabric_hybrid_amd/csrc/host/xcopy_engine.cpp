@@ -59,7 +59,6 @@ struct ThreadLease {
     uint64_t pendingBytes = 0;      // bytes of the copies queued on `stream` since the thread last waited for it
     void *bounce = nullptr;
     uint64_t bounceBytes = 0;
-    void *bounceEvents[XcopyEngine::kBounceEvents] = {};
     // unordered batches handed to the submit threads: fanDirty bit w = submitter w holds batches of this thread that the
     // thread's stream has not been made to wait for, the last of them under ticket fanTicket[w]
     void *fanEvent[XcopyEngine::kFanStreams] = {};
@@ -118,12 +117,6 @@ struct ThreadLease {
             }
         }
         fanDirty = 0;
-        for (void *&event : bounceEvents) {
-            if (event != nullptr) {
-                (void)mfrt_event_destroy(event);
-                event = nullptr;
-            }
-        }
     }
 };
 
@@ -671,16 +664,22 @@ int EnsureDevice(StagingSlot &slot, uint64_t bytes)
     return BM_OK;
 }
 
+constexpr uint32_t kLinkGroups = 64;
+
 uint32_t GridFor(uint64_t nchunk, uint32_t cuCount, int route, const XcopyTuning &tuning)
 {
     // HBM routes: one workgroup per chunk unless a cap is set.  Measured on 128 MiB ... 4 GiB copies:
     // letting the hardware dispatcher hand out the chunks one by one sustains 6.0-6.2 TB/s, a
     // grid capped at 16 workgroups per CU that strides over the chunks 5.3-5.7 TB/s (its static
-    // assignment leaves a tail).  Link routes: one workgroup per CU, more only adds contention.
+    // assignment leaves a tail).  Link routes: kLinkGroups for the whole chip.  They keep 256 KiB in flight, more than the link's
+    // rate times its round trip, from the host; what is in flight beyond that queues in front of the link and lowers its rate.
+    // Back to back, from the host 256 workgroups on 8 KiB / 64 on 4 KiB: 1 / 2 / 4 / 8 / 64 MiB 23.8 / 44.6 / 81.2 / 154.6 / 1178 us
+    // against 22.6 / 41.3 / 77.9 / 151.0 / 1173; to the host, both on 4 KiB: 22.1 / 41.1 / 77.8 / 151.2 / 1179 against 20.9 / 39.7 /
+    // 76.5 / 149.9 / 1178.
     const bool link = route == MFRT_ROUTE_TO_HOST || route == MFRT_ROUTE_FROM_HOST;
-    const uint32_t perCu = link ? (tuning.wgPerCuLink == 0 ? 1 : tuning.wgPerCuLink) : tuning.wgPerCu;
+    const uint32_t perCu = link ? tuning.wgPerCuLink : tuning.wgPerCu;
     const uint64_t limit = (1ull << 24) - 1;   // grid size in lanes must stay below 2^32 with up to 256 lanes per workgroup
-    uint64_t cap = perCu == 0 ? limit : static_cast<uint64_t>(cuCount == 0 ? 256 : cuCount) * perCu;
+    uint64_t cap = perCu != 0 ? static_cast<uint64_t>(cuCount == 0 ? 256 : cuCount) * perCu : link ? kLinkGroups : limit;
     if (cap > limit) {
         cap = limit;
     }
@@ -752,12 +751,12 @@ uint32_t ChooseUnits(uint64_t totalBytes, uint32_t cuCount, int route, const Xco
     // 1 GiB copy (6.4 against 6.25 TB/s).  4 KiB also divides the usual power-of-two block sizes, so
     // no workgroup runs a ragged tile.
     if (route == MFRT_ROUTE_TO_HOST || route == MFRT_ROUTE_FROM_HOST) {
-        // The host link, not the GPU, is the bound: one four-wave workgroup per CU with small chunks
-        // keeps the link busy without flooding it (measured: 56 GB/s out, 55 GB/s in on a Gen5 x16 link).
+        // See GridFor for the workgroups.  From the host one access per lane for short copies (512 KiB 19.8 us, 20.6 with two), two
+        // beyond (122 blocks, 9 MB: 162.9, 165.4 with one), four for the longest, which take any.
         if (totalBytes > (256ull << 20)) {
             return 4 * kXcopyThreads;
         }
-        return route == MFRT_ROUTE_TO_HOST ? kXcopyThreads : 2 * kXcopyThreads;
+        return route == MFRT_ROUTE_TO_HOST || totalBytes <= (2ull << 20) ? kXcopyThreads : 2 * kXcopyThreads;
     }
     (void)totalBytes;
     return tuning.minUnits;
@@ -1183,18 +1182,6 @@ void *XcopyEngine::ThreadBounce(uint64_t bytes)
     return lease.bounce;
 }
 
-void *XcopyEngine::ThreadBounceEvent(uint32_t index)
-{
-    if (index >= kBounceEvents) {
-        return nullptr;
-    }
-    ThreadLease &lease = t_ctx.Lease();
-    if (lease.bounceEvents[index] == nullptr && mfrt_bind_thread() == 0) {
-        lease.bounceEvents[index] = mfrt_event_create();
-    }
-    return lease.bounceEvents[index];
-}
-
 int XcopyEngine::DrainThread()
 {
     if (!Started()) {
@@ -1238,21 +1225,103 @@ uint32_t NextDoneSeq(ThreadLease &lease)
     return ++lease.doneSeq == 0 ? ++lease.doneSeq : lease.doneSeq;   // 0 is the initial contents
 }
 
-// Polls the lease's word for `seq`; false when that takes longer than expected (or the GPU is busy with other work).
-bool PollDone(const ThreadLease &lease, uint32_t seq, uint32_t micros)
+// What the route needs at the least for `bytes`: a link route 58 GB/s, HBM 7.4 TB/s of reads and writes.
+uint64_t LeastMicros(uint64_t bytes, int route)
+{
+    return route == MFRT_ROUTE_HBM ? bytes / 3700000u : bytes / 58000u;
+}
+
+// Polls the lease's word until it has come to `seq`, for at most kSpinMicros more than `least`; false when that takes longer
+// than expected (or the GPU is busy with other work).  A thread with a millisecond and more ahead of it sleeps for most of it.
+bool PollDone(const ThreadLease &lease, uint32_t seq, uint64_t least)
 {
     const auto start = std::chrono::steady_clock::now();
+    if (least > 1000) {
+        std::this_thread::sleep_for(std::chrono::microseconds(least * 9 / 10 - 100));   // a sleep may last 50 us longer
+    }
+    const auto most = std::chrono::microseconds(least + XcopyEngine::kSpinMicros);
     for (uint32_t polls = 1;; ++polls) {
-        if (__atomic_load_n(lease.doneWord, __ATOMIC_ACQUIRE) == seq) {
+        const auto seen = static_cast<uint32_t>(__atomic_load_n(lease.doneWord, __ATOMIC_ACQUIRE));
+        if (static_cast<int32_t>(seen - seq) >= 0) {
             return true;
         }
-        if ((polls & 63u) == 0 && std::chrono::steady_clock::now() - start > std::chrono::microseconds(micros)) {
+        if ((polls & 63u) == 0 && std::chrono::steady_clock::now() - start > most) {
             return false;
         }
     }
 }
 
 }  // namespace
+
+int XcopyEngine::LaunchDone(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t bytes, int route,
+                            void *stream, uint32_t &ticket)
+{
+    // To the host a copy has few workgroups whatever its size, and each costs the launch one atomic at its end.  In HBM one of
+    // up to kDoneBytes has few enough (the kernel has the figures).  From the host written-through stores cost more than the
+    // launch they save beyond kDoneFromHostBytes (1 MiB 33.1 us, 30.2 with a signal launch; 256 KiB 14.2 either way).
+    constexpr uint64_t kDoneBytes = 1ull << 20;
+    constexpr uint64_t kDoneFromHostBytes = 128ull << 10;
+    const uint64_t most = route == MFRT_ROUTE_TO_HOST ? ~0ull : route == MFRT_ROUTE_HBM ? kDoneBytes : kDoneFromHostBytes;
+    InlinePlan plan;
+    if (n > kInlineSegs || bytes == 0 || bytes > most || tuning_.unitsOverride != 0 || !Started() || mfrt_bind_thread() != 0 ||
+        !BuildInlineDirect(src, dst, len, n, kDeepUnits, plan)) {
+        return kNotLaunched;
+    }
+    ThreadLease &lease = t_ctx.Lease();
+    if (!HasDoneWord(lease) || !HasDoneCounter(lease)) {
+        return kNotLaunched;
+    }
+    ticket = NextDoneSeq(lease);
+    const uint32_t grid = GridFor(plan.nchunk, mfrt_cu_count(), route, tuning_);
+    const int err = mfk_xcopy_done(&plan, route, grid, lease.doneWord, ticket, lease.doneCounter, stream);
+    if (err != 0) {
+        MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(err));
+    }
+    g_launches.fetch_add(1, std::memory_order_relaxed);
+    NotePending(stream, bytes);
+    return BM_OK;
+}
+
+int XcopyEngine::SubmitTicket(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, int route, void *stream,
+                              uint32_t &ticket)
+{
+    uint64_t bytes = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        bytes += len[i];
+    }
+    int ret = LaunchDone(src, dst, len, n, bytes, route, stream, ticket);
+    if (ret != kNotLaunched) {
+        return ret;
+    }
+    ret = Submit(src, dst, len, n, route, stream, nullptr, 0);
+    if (ret != BM_OK) {
+        return ret;
+    }
+    ThreadLease &lease = t_ctx.Lease();
+    if (!HasDoneWord(lease)) {
+        MF_FAIL(BM_MALLOC_FAILED, "the thread's pinned word could not be allocated");
+    }
+    ticket = NextDoneSeq(lease);
+    const int err = mfk_xcopy_signal(lease.doneWord, ticket, stream);
+    if (err != 0) {
+        MF_FAIL(BM_ERROR, "signal launch failed: " << mfrt_error_string(err));
+    }
+    return BM_OK;
+}
+
+int XcopyEngine::WaitTicket(uint32_t ticket, void *stream)
+{
+    ThreadLease &lease = t_ctx.Lease();
+    const uint64_t queued = stream == lease.stream ? lease.pendingBytes : 0;
+    const int err = PollDone(lease, ticket, 4 * kSpinMicros) ? 0 : mfrt_stream_sync(stream);
+    if (err != 0) {
+        MF_FAIL(BM_ERROR, "copy failed on the GPU: " << mfrt_error_string(err));
+    }
+    if (ticket == lease.doneSeq && queued != 0) {
+        lease.pendingBytes = 0;     // the thread's latest: nothing else is queued on its stream
+    }
+    return BM_OK;
+}
 
 int XcopyEngine::SubmitAndWait(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, int route, void *stream)
 {
@@ -1262,31 +1331,24 @@ int XcopyEngine::SubmitAndWait(const uint64_t *src, const uint64_t *dst, const u
             bytes += len[i];
         }
     }
-    // Up to here a launch that stores the word itself is the faster one (the kernel has the figures).
-    const uint64_t doneMax = route == MFRT_ROUTE_FROM_HOST ? kDoneFromHostBytes : kDoneBytes;
-    InlinePlan plan;
-    if (n <= kInlineSegs && bytes != 0 && bytes <= doneMax && Started() && mfrt_bind_thread() == 0 &&
-        BuildInlineDirect(src, dst, len, n, kDeepUnits, plan)) {
-        ThreadLease &lease = t_ctx.Lease();
-        if (HasDoneWord(lease) && HasDoneCounter(lease)) {
-            const uint32_t seq = NextDoneSeq(lease);
-            const int err = mfk_xcopy_done(&plan, route, lease.doneWord, seq, lease.doneCounter, stream);
-            if (err != 0) {
-                MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(err));
-            }
-            g_launches.fetch_add(1, std::memory_order_relaxed);
-            if (stream == lease.stream) {
-                lease.pendingBytes = 0;
-            }
-            const int waited = PollDone(lease, seq, kSpinMicros) ? 0 : mfrt_stream_sync(stream);
-            if (waited != 0) {
-                MF_FAIL(BM_ERROR, "copy failed on the GPU: " << mfrt_error_string(waited));
-            }
-            return BM_OK;
-        }
+    uint32_t ticket = 0;
+    int ret = LaunchDone(src, dst, len, n, bytes, route, stream, ticket);
+    if (ret == kNotLaunched) {
+        ret = Submit(src, dst, len, n, route, stream, nullptr, 0, false);
+        return ret != BM_OK ? ret : WaitStream(stream, bytes, route);
     }
-    const int ret = Submit(src, dst, len, n, route, stream, nullptr, 0, false);
-    return ret != BM_OK ? ret : WaitStream(stream, bytes);
+    if (ret != BM_OK) {
+        return ret;
+    }
+    ThreadLease &lease = t_ctx.Lease();
+    if (stream == lease.stream) {
+        lease.pendingBytes = 0;
+    }
+    const int err = PollDone(lease, ticket, LeastMicros(bytes, route)) ? 0 : mfrt_stream_sync(stream);
+    if (err != 0) {
+        MF_FAIL(BM_ERROR, "copy failed on the GPU: " << mfrt_error_string(err));
+    }
+    return BM_OK;
 }
 
 // A blocking call is a launch and a wait.  hipStreamSynchronize first has to put a marker with a
@@ -1299,7 +1361,7 @@ int XcopyEngine::SubmitAndWait(const uint64_t *src, const uint64_t *dst, const u
 // the copy kernel has ended, so it carries the same guarantee as the stream wait: the copy's
 // end-of-kernel release has made its stores visible to the device, and stores to host memory were
 // issued, in order, before the word's.
-int XcopyEngine::WaitStream(void *stream, uint64_t bytes)
+int XcopyEngine::WaitStream(void *stream, uint64_t bytes, int route)
 {
     if (t_ctx.HasLiveLease() && stream == t_ctx.lease->stream) {
         const uint64_t queued = t_ctx.lease->pendingBytes;
@@ -1317,7 +1379,7 @@ int XcopyEngine::WaitStream(void *stream, uint64_t bytes)
         if (HasDoneWord(lease)) {
             const uint32_t seq = NextDoneSeq(lease);
             // (the signal is not counted by LaunchCount(): it moves no data)
-            if (mfk_xcopy_signal(lease.doneWord, seq, stream) == 0 && PollDone(lease, seq, kSpinMicros)) {
+            if (mfk_xcopy_signal(lease.doneWord, seq, stream) == 0 && PollDone(lease, seq, LeastMicros(bytes, route))) {
                 return BM_OK;
             }
         }
@@ -1673,6 +1735,11 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
             return BM_OK;
         }
         units = ChooseUnits(total, cu, route, tuning_);
+        if (route == MFRT_ROUTE_TO_HOST && tuning_.unitsOverride == 0) {
+            // Four accesses per lane, whose loads from HBM are in flight together: with one the walk over a table's chunks is too
+            // slow for the link (K and V blocks of four requests 638 us, 669 with one; 256 workgroups with one 639).
+            units = kDeepUnits;
+        }
         deepTable = DeepHoldApplies(total, n, route, unordered);
         // Many short segments: a chunk size that holds the longest of them gives every segment exactly
         // one chunk, which is the equal-count form below (no prefix, no search, no upload): 16 384
@@ -1741,7 +1808,10 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
     // it runs beside the caller's earlier copies, was measured for these batches too: the extra launch costs the
     // stream 2 us whether it overlaps or not, more than the fetch from HBM saves: 36 MB of K and V blocks 20.5
     // against 18.4 us per call.)
-    if (pattern.period != 0) {
+    // Over the link a few workgroups walk all the chunks, and a descriptor fetch across the link it saturates would be in every
+    // one of their steps: those tables are uploaded (K and V blocks of four requests to the host: 638 us, 681 from the slot and
+    // on 4 KiB chunks).
+    if (pattern.period != 0 && route == MFRT_ROUTE_HBM) {
         const uint32_t hold = HoldForTable(static_cast<uint32_t>(nchunk), grid, units, route, unordered, true);
         table.triples = triples;
         table.pattern = pattern;
@@ -1753,10 +1823,15 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         // launched without a barrier: the slot's device half is free (AcquireSlot has waited for its last
         // reader), so it may run while the caller's earlier copies still do; the table launch behind it waits
         // for both.
+        // A pattern needs the triples only.
         uint32_t *group = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(slot->host) + tripleBytes + prefixBytes);
-        table.groupShift = BuildGroupMap(first, count, group, groupCapacity);
-        const uint64_t usedBytes =
-            RoundUp(tripleBytes + prefixBytes + 4ull * (GroupCount(nchunk, table.groupShift) + 1), kUnitBytes);
+        uint64_t usedBytes = RoundUp(24ull * count, kUnitBytes);
+        if (pattern.period != 0) {
+            table.pattern = pattern;
+        } else {
+            table.groupShift = BuildGroupMap(first, count, group, groupCapacity);
+            usedBytes = RoundUp(tripleBytes + prefixBytes + 4ull * (GroupCount(nchunk, table.groupShift) + 1), kUnitBytes);
+        }
         ret = EnsureDevice(*slot, slotBytes);
         if (ret != BM_OK) {
             return ret;

@@ -44,7 +44,7 @@ void NormalizeSegments(const uint64_t *src, const uint64_t *dst, const uint64_t 
 struct XcopyTuning {
     uint32_t unitsOverride = 0;  // 16-byte units per chunk, 0 = choose from batch size
     uint32_t wgPerCu = 0;        // HBM routes: grid cap in workgroups per CU, 0 = one workgroup per chunk
-    uint32_t wgPerCuLink = 1;    // routes bound by the host link: workgroups per CU
+    uint32_t wgPerCuLink = 0;    // routes bound by the host link: workgroups per CU; 0: kLinkGroups for the whole chip
     uint32_t minUnits = kXcopyThreads;   // 4 KiB: the chunk of HBM routes
     int32_t holdNanos = -1;      // stores held back in inline launches: -1 = HoldNanosFor's rule (+ holdDeltaNanos), 0 = never, else that long
     int32_t holdDeltaNanos = 0;  // added to the rule's wait: what the calibration at start found best on this GPU
@@ -157,23 +157,21 @@ public:
     // Pinned, device-mapped staging memory of the calling thread, at least `bytes` long; it lives
     // until Stop().  NULL when it cannot be allocated.
     void *ThreadBounce(uint64_t bytes);
-    // One of the calling thread's events for slots of that staging memory (index < kBounceEvents).
-    static constexpr uint32_t kBounceEvents = 16;
-    void *ThreadBounceEvent(uint32_t index);
     // Wait for everything this thread enqueued on its own stream.
     int DrainThread();
     // Wait for everything queued on `stream` so far: what a blocking copy does after its launch.
-    // Work expected to be short (`bytes` moved, 0 = unknown) is awaited by polling a word in pinned
-    // memory that a one-lane launch behind the copy stores, for at most kSpinMicros; anything else,
+    // Work of known size (`bytes` moved, 0 = unknown) is awaited by polling a word in pinned memory that a one-lane
+    // launch behind the copy stores, for at most kSpinMicros more than the route needs for it; anything else,
     // and a poll that runs out of time, waits on the stream.
     static constexpr uint64_t kSpinBytes = 256ull << 20;
     static constexpr uint32_t kSpinMicros = 200;
-    int WaitStream(void *stream, uint64_t bytes);
-    // Submit() and WaitStream() of a blocking copy; one of up to kDoneBytes (from the host: kDoneFromHostBytes, beyond which
-    // written-through stores cost more than the launch they save) goes out as a launch that tells the host itself.
-    static constexpr uint64_t kDoneBytes = 1ull << 20;
-    static constexpr uint64_t kDoneFromHostBytes = 128ull << 10;
+    int WaitStream(void *stream, uint64_t bytes, int route = 0 /* MFRT_ROUTE_HBM */);
+    // Submit() and WaitStream() of a blocking copy.
     int SubmitAndWait(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, int route, void *stream);
+    // The two halves for a thread that has several copies on their way on one stream: `ticket` says what WaitTicket() waits
+    // for, everything queued on `stream` up to that copy.
+    int SubmitTicket(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, int route, void *stream, uint32_t &ticket);
+    int WaitTicket(uint32_t ticket, void *stream);
     // Work that another part of the library has queued on `stream`: if it is the calling thread's own stream, the next
     // DrainThread() takes `bytes` into account when it chooses between polling and sleeping (~0: sleep).
     void NoteQueued(void *stream, uint64_t bytes);
@@ -206,6 +204,10 @@ private:
     uint32_t HoldForTable(uint32_t nchunk, uint32_t grid, uint32_t units, int route, bool unordered, bool pinned) const;
     // Whether a batch of `bytes` in n segments is planned in chunks of kDeepUnits units, to hold the stores of 16 KiB per wave.
     bool DeepHoldApplies(uint64_t bytes, uint32_t n, int route, bool unordered) const;
+    // A launch that stores the thread's word itself, where that is the faster form: kNotLaunched where it is not.
+    static constexpr int kNotLaunched = 1;
+    int LaunchDone(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t bytes, int route, void *stream,
+                   uint32_t &ticket);
     int SubmitInPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t total, int route,
                        void *stream, void *mask, uint32_t maskValue);
     int SubmitOne(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, int route, void *stream,

@@ -395,7 +395,6 @@ __global__ void XcopySignalKernel(uint64_t *mask, uint32_t maskValue)
 // host 12.2 / 11.0.  Workgroups of 16 KiB (four 128-bit accesses per lane of four waves): every workgroup beyond the first
 // costs an atomic on one word, so 4 KiB ones lose at 1 MiB (11.6) and the form as a whole at 4 MiB (11.0 / 11.5); 64 KiB in one
 // workgroup of sixteen waves gain nothing in HBM (8.9 / 8.9) and lose over the link (from the host 12.5 / 10.6).
-constexpr uint32_t kDoneMaxChunks = 4096;
 struct DoneMark {
     uint64_t *word;         // pinned host memory, polled by the caller
     uint32_t *counter;      // device memory, 0 between launches
@@ -422,10 +421,12 @@ __device__ __forceinline__ void MarkDone(const DoneMark &mark)
 }
 
 template <bool kNtLoad>
-__global__ __launch_bounds__(kXcopyThreads) void XcopySingleDoneKernel(uint64_t src, uint64_t dst, uint32_t len, uint32_t units,
-                                                                       DoneMark mark)
+__global__ __launch_bounds__(kXcopyThreads) void XcopySingleDoneKernel(uint64_t src, uint64_t dst, uint32_t len, uint32_t nchunk,
+                                                                       uint32_t units, DoneMark mark)
 {
-    CopyChunk<kNtLoad, kStoreThrough>(src, dst, len, blockIdx.x, units);
+    for (uint32_t c = blockIdx.x; c < nchunk; c += gridDim.x) {
+        CopyChunk<kNtLoad, kStoreThrough>(src, dst, len, c, units);
+    }
     MarkDone(mark);
 }
 
@@ -433,8 +434,14 @@ template <bool kNtLoad>
 __global__ __launch_bounds__(kXcopyThreads) void XcopyInlineDoneKernel(const InlinePlan p, DoneMark mark)
 {
     const InlineRows rows(p);
-    const InlineChunk r = rows.Owner(blockIdx.x);
-    CopyChunk<kNtLoad, kStoreThrough>(r.src, r.dst, r.len, r.k, p.units);
+    const uint32_t nchunk = p.nchunk;
+    const uint32_t units = p.units;
+    uint32_t c = blockIdx.x;
+    do {
+        const InlineChunk r = rows.Owner(c);
+        CopyChunk<kNtLoad, kStoreThrough>(r.src, r.dst, r.len, r.k, units);
+        c += gridDim.x;
+    } while (c < nchunk);
     MarkDone(mark);
 }
 
@@ -1083,23 +1090,24 @@ extern "C" int mfk_xcopy_inline(const void *inlinePlan, int route, uint32_t grid
     return err != 0 ? err : mf::Signal(mask, maskValue, s);
 }
 
-extern "C" int mfk_xcopy_done(const void *inlinePlan, int route, void *word, uint32_t value, void *counter, void *stream)
+extern "C" int mfk_xcopy_done(const void *inlinePlan, int route, uint32_t grid, void *word, uint32_t value, void *counter, void *stream)
 {
     using namespace mf;
     const InlinePlan &plan = *static_cast<const InlinePlan *>(inlinePlan);
-    const bool single = plan.first[1] == kNoChunk;
-    const uint32_t lanes = (plan.units / kDepth + 63) / 64 * 64;     // a chunk in one step of kDepth accesses per lane
-    if (plan.nchunk == 0 || plan.nchunk > kDoneMaxChunks || lanes == 0 || lanes > kXcopyThreads) {
+    if (plan.nchunk == 0 || grid == 0) {
         return static_cast<int>(hipErrorInvalidValue);
     }
+    grid = grid < plan.nchunk ? grid : plan.nchunk;
     hipStream_t s = static_cast<hipStream_t>(stream);
     DoneMark mark{static_cast<uint64_t *>(word), static_cast<uint32_t *>(counter), value};
     uint64_t src = plan.src[0];
     uint64_t dst = plan.dst[0];
     uint32_t len = plan.len[0];
+    uint32_t nchunk = plan.nchunk;
     uint32_t units = plan.units;
-    void *singleArgs[] = {&src, &dst, &len, &units, &mark};
+    void *singleArgs[] = {&src, &dst, &len, &nchunk, &units, &mark};
     void *args[] = {const_cast<InlinePlan *>(&plan), &mark};
+    const bool single = plan.first[1] == kNoChunk;
     const bool nt = PolicyOf(route).ntLoad;
     const void *kernel = nt ? reinterpret_cast<const void *>(&XcopyInlineDoneKernel<true>)
                             : reinterpret_cast<const void *>(&XcopyInlineDoneKernel<false>);
@@ -1107,7 +1115,7 @@ extern "C" int mfk_xcopy_done(const void *inlinePlan, int route, void *word, uin
         kernel = nt ? reinterpret_cast<const void *>(&XcopySingleDoneKernel<true>)
                     : reinterpret_cast<const void *>(&XcopySingleDoneKernel<false>);
     }
-    return static_cast<int>(hipLaunchKernel(kernel, dim3(plan.nchunk), dim3(lanes), single ? singleArgs : args, 0, s));
+    return static_cast<int>(hipLaunchKernel(kernel, dim3(grid), dim3(LanesFor(plan.units, route)), single ? singleArgs : args, 0, s));
 }
 
 extern "C" uint32_t mfk_xcopy_window_units(void)

@@ -80,10 +80,10 @@ int mfrt_memcpy_async(void *dst, const void *src, uint64_t bytes, void *stream);
  * mfk_xcopy_window_units() units (16 KiB, copied by single waves with sixteen loads per lane in flight). */
 int mfk_xcopy_inline(const void *inlinePlan, int route, uint32_t grid, void *mask, uint32_t maskValue, void *stream,
                      int anyOrder, uint32_t holdNanos);
-/* A short copy, one workgroup per chunk, that stores `value` into `word` (pinned host memory) itself once every byte it moved
- * is in memory, without a launch behind it.  Chunks of 16 KiB at most.  `counter` is a word
- * of device memory, 0 before the launch and 0 again when `word` has been stored: one launch at a time may use it. */
-int mfk_xcopy_done(const void *inlinePlan, int route, void *word, uint32_t value, void *counter, void *stream);
+/* A copy by `grid` workgroups, few or short-lived ones, that stores `value` into `word` (pinned host memory) itself once every
+ * byte it moved is in memory, without a launch behind it.  `counter` is a word of device memory, 0 before the launch and 0
+ * again when `word` has been stored: launches that share it follow one another on a stream. */
+int mfk_xcopy_done(const void *inlinePlan, int route, uint32_t grid, void *word, uint32_t value, void *counter, void *stream);
 /* HBM to HBM copies of hundreds of MiB: the plan's chunks are mfk_xcopy_window_units() units (16 KiB), copied by up to
  * mfk_xcopy_window_waves() single-wave workgroups that alternate, chip-wide and by the clock, between a read half and a
  * write half of a period cut for `windowMBps` MB/s of HBM traffic (see XcopyWindowKernel). */

@@ -284,7 +284,7 @@ int mfk_xcopy_inline(const void *inlinePlan, int, uint32_t, void *mask, uint32_t
     return 0;
 }
 
-int mfk_xcopy_done(const void *inlinePlan, int route, void *word, uint32_t value, void *counter, void *stream)
+int mfk_xcopy_done(const void *inlinePlan, int route, uint32_t, void *word, uint32_t value, void *counter, void *stream)
 {
     return counter == nullptr ? -1 : mfk_xcopy_inline(inlinePlan, route, 0, word, value, stream, 0, 0);
 }

@@ -67,3 +67,43 @@ def test_batches_one_behind_the_other(lib, pool, route, count, most):
                 image[to][d:d + n] = image[frm][s:s + n]
     for addr, data in image.items():
         assert np.array_equal(_read(lib, addr, ROOM), data)
+
+
+HALF_MIB = 512 << 10
+
+
+@pytest.mark.parametrize("way", ["load", "save"])
+@pytest.mark.parametrize("sizes", [
+    [HALF_MIB], [HALF_MIB + 1], [2 * HALF_MIB - 1], [3 * HALF_MIB + 4097, 0, 5],      # one round, its edge, the first of several
+    [1000] * 700, [4000, 0, 60001] * 40,                                              # more segments in a round than a launch takes as arguments
+    [HALF_MIB - 100, 300, 70000, HALF_MIB],                                           # a segment that would leave a sliver in a round
+    [(37 << 20) + 13], [(9 << 20) + 1, 3, (31 << 20) + 70],                           # more rounds than there are slots
+], ids=lambda s: f"{len(s)}x{s[0]}")
+def test_staged_copies_of_pageable_memory(lib, pool, way, sizes):
+    """Ordinary host memory through the staging ring: rounds that grow or shrink, cut inside segments, reuse their slots."""
+    room = sum(sizes) + 64 * len(sizes) + 4096
+    big = bm.create(2, 0, (room + (2 << 20)) // (2 << 20) * (2 << 20))
+    try:
+        dev = big.peer_rank_ptr(0)
+        rng = np.random.default_rng(len(sizes))
+        inside = np.cumsum([0] + [n + int(rng.integers(1, 64)) for n in sizes[:-1]])
+        flat = rng.integers(0, 256, sum(sizes), dtype=np.uint8)
+        outside = flat.ctypes.data + np.cumsum([0] + sizes[:-1])
+        image = rng.integers(0, 256, room, dtype=np.uint8)
+        assert lib.mfrt_memcpy(dev, image.ctypes.data, room) == 0
+        source, target = (outside, dev + inside) if way == "load" else (dev + inside, outside)
+        kind = bm.BmCopyType.H2G if way == "load" else bm.BmCopyType.G2H
+        before = flat.copy()
+        for _ in range(2):
+            assert big.copy_data_batch(source.tolist(), target.tolist(), sizes, len(sizes), kind) == 0, native.last_error()
+        at = 0
+        for offset, n in zip(inside, sizes):
+            if way == "load":
+                image[offset:offset + n] = before[at:at + n]
+            else:
+                before[at:at + n] = image[offset:offset + n]
+            at += n
+        assert np.array_equal(flat, before)
+        assert np.array_equal(_read(lib, dev, room), image)
+    finally:
+        big.destroy()
