@@ -32,6 +32,7 @@ struct StagingSlot {
     enum State : uint8_t { kFree, kQueued, kGuarded };
     void *host = nullptr;
     void *dev = nullptr;
+    void *rest = nullptr;       // RestList of device-resident tables, in device memory
     uint64_t capacity = 0;      // of host
     uint64_t devCapacity = 0;
     void *event = nullptr;
@@ -88,6 +89,9 @@ struct ThreadLease {
             }
             if (slot.dev != nullptr) {
                 (void)mfrt_free_device(slot.dev);
+            }
+            if (slot.rest != nullptr) {
+                (void)mfrt_free_device(slot.rest);
             }
             slot = StagingSlot{};
         }
@@ -664,6 +668,26 @@ int EnsureDevice(StagingSlot &slot, uint64_t bytes)
     return BM_OK;
 }
 
+int EnsureRestList(StagingSlot &slot)
+{
+    if (slot.rest != nullptr) {
+        return BM_OK;
+    }
+    slot.rest = mfrt_alloc_device(RestListBytes(kRestCapacity));
+    if (slot.rest == nullptr) {
+        MF_FAIL(BM_MALLOC_FAILED, "list of " << kRestCapacity << " pieces could not be allocated in HBM");
+    }
+    // cleared once, on a stream of the engine: the caller's may be recording
+    void *own = XcopyEngine::Instance().ThreadStream();
+    const int err = own == nullptr ? -1 : mfk_xcopy_signal(slot.rest, 0, own);   // one 64-bit word, both counts
+    if (err != 0 || mfrt_stream_sync(own) != 0) {
+        (void)mfrt_free_device(slot.rest);
+        slot.rest = nullptr;
+        MF_FAIL(BM_ERROR, "list of pieces could not be cleared: " << mfrt_error_string(err));
+    }
+    return BM_OK;
+}
+
 constexpr uint32_t kLinkGroups = 64;
 
 uint32_t GridFor(uint64_t nchunk, uint32_t cuCount, int route, const XcopyTuning &tuning)
@@ -687,19 +711,21 @@ uint32_t GridFor(uint64_t nchunk, uint32_t cuCount, int route, const XcopyTuning
     return grid == 0 ? 1u : static_cast<uint32_t>(grid);
 }
 
-// Grid of a table launch whose chunk count only the GPU knows: workgroups walk the chunks with the grid as their
-// stride, surplus workgroups leave at once.  Eight workgroups per segment (pages of 32 KiB have eight chunks)
-// between 32 and 4096 per CU: measured on 262 144 pages of 32 KiB, 256 / 512 / 1024 / 2048 / 4096 per CU take
-// 3.27 / 3.21 / 3.15 / 3.09 / 3.06 ms (one workgroup per chunk, which needs the count: 3.05 ms), while on 4096 pages
-// 512 per CU cost 14 us in workgroups that find nothing to do (69 against 55 us).
+// Grid of the launch that copies a table only the GPU can read.  Workgroups walk the items of the table with the grid as their
+// stride, surplus workgroups leave at once, at 0.4 ns each.  Four per segment between 16 and 1024 per CU: 16 080 pages of 8 KiB
+// (two chunks) take 53 / 58 / 71 us with two / four / eight per segment, 4096 pages of 32 KiB (eight chunks) 49.8 / 47.1 / 48.5.
 uint32_t DeviceTableGrid(uint32_t nseg, uint32_t cuCount, int route, const XcopyTuning &tuning)
 {
     const uint64_t cus = cuCount == 0 ? 256 : cuCount;
-    uint64_t want = tuning.deviceTableWgPerCu != 0 ? cus * tuning.deviceTableWgPerCu : 8ull * nseg;
-    if (tuning.deviceTableWgPerCu == 0) {
-        want = want < 32 * cus ? 32 * cus : (want > 4096 * cus ? 4096 * cus : want);
-    }
-    return GridFor(want, cuCount, route, tuning);
+    uint64_t want = 4ull * nseg;
+    want = want < 16 * cus ? 16 * cus : want > 1024 * cus ? 1024 * cus : want;
+    return GridFor(tuning.deviceTableWgPerCu != 0 ? cus * tuning.deviceTableWgPerCu : want, cuCount, route, tuning);
+}
+
+// Grid of the launch behind it, which usually finds nothing to do: four per CU keep enough loads in flight when it does.
+uint32_t DeviceTableRestGrid(uint32_t cuCount, int route, const XcopyTuning &tuning)
+{
+    return GridFor(4ull * (cuCount == 0 ? 256 : cuCount), cuCount, route, tuning);
 }
 
 }  // namespace
@@ -1886,31 +1912,24 @@ int XcopyEngine::SubmitDeviceTable(const void *triples, uint32_t n, int route, v
         int err = mfk_xcopy_inline(&empty, route, 1, mask, maskValue, stream, 0, 0);
         return err == 0 ? BM_OK : BM_ERROR;
     }
-    // Prefix, group map and pattern are computed on the GPU; their slot is only ever touched by kernels of this stream.
+    // The list of long segments' pieces belongs to a slot: the next call of another stream gets another one.
     ThreadCtx &ctx = t_ctx;
     StagingSlot *slot = nullptr;
-    const uint32_t groupCapacity = GroupCapacityFor(n);
-    const uint64_t scratchBytes = RoundUp(4ull * mfk_xcopy_plan_scratch_words(n, groupCapacity), kUnitBytes);
     ThreadLease &lease = ctx.Lease();
     int ret = AcquireSlot(lease, 0, stream, slot);
     if (ret == BM_OK) {
-        ret = EnsureDevice(*slot, scratchBytes);
+        ret = EnsureRestList(*slot);
     }
     if (ret != BM_OK) {
         return ret;
     }
     const uint32_t cu = mfrt_cu_count();
     const uint32_t units = ChooseUnits(0, cu, route, tuning_);   // sizes are only known on the GPU
-    TablePlan table;
-    int err = mfk_xcopy_plan(triples, n, units, slot->dev, groupCapacity, &table, stream);
+    const int err = mfk_xcopy_direct(triples, n, units, route, DeviceTableGrid(n, cu, route, tuning_), DeviceTableRestGrid(cu, route, tuning_),
+                                     slot->rest, kRestCapacity, mask, maskValue, stream);
     if (err != 0) {
-        MF_FAIL(BM_ERROR, "xcopy plan launch failed: " << mfrt_error_string(err));
-    }
-    const uint32_t grid = DeviceTableGrid(n, cu, route, tuning_);
-    err = mfk_xcopy_table(&table, route, grid, mask, maskValue, stream, 0);
-    if (err != 0) {
-        (void)MarkQueued(lease, slot, stream, true);   // the plan launch writes the slot
-        MF_FAIL(BM_ERROR, "xcopy table launch failed: " << mfrt_error_string(err));
+        (void)MarkQueued(lease, slot, stream, true);   // the first launch writes the list
+        MF_FAIL(BM_ERROR, "xcopy launch of a device table failed: " << mfrt_error_string(err));
     }
     g_launches.fetch_add(2, std::memory_order_relaxed);
     NotePending(stream, ~0ull);   // sizes unknown here: the next wait sleeps on the stream
@@ -1935,8 +1954,8 @@ int XcopyEngine::SubmitDeviceTableStatic(const void *triples, uint32_t n, int ro
     }
     const uint32_t cu = mfrt_cu_count();
     const uint32_t units = ChooseUnits(0, cu, route, tuning_);   // sizes are only known on the GPU
-    const uint32_t grid = DeviceTableGrid(n, cu, route, tuning_);
-    const int err = mfk_xcopy_table_static(triples, n, units, route, grid, stream);
+    const int err = mfk_xcopy_table_static(triples, n, units, route, DeviceTableGrid(n, cu, route, tuning_),
+                                           DeviceTableRestGrid(cu, route, tuning_), stream);
     if (err != 0) {
         MF_FAIL(BM_ERROR, "static-scratch table launch failed (" << err << ")");
     }

@@ -54,7 +54,7 @@ struct XcopyTuning {
     bool deepHold = true;        // batches of 24 to 64 MiB hold the stores of 16 KiB per wave
     int32_t holdPinnedExtraNanos = 1600;   // added to the rule for table launches, whose descriptors come from pinned host memory: a link round trip before the loads
     bool stageUnordered = true;  // the upload of a ragged table's descriptors is launched without a barrier
-    uint32_t deviceTableWgPerCu = 0;   // grid of a device-resident table in workgroups per CU, 0 = eight per segment between 32 and 4096 per CU
+    uint32_t deviceTableWgPerCu = 0;   // grid of a device-resident table in workgroups per CU, 0 = four per segment between 16 and 1024 per CU
     uint32_t windowMBps = 6800000;   // HBM copies of kWindowRectMinBytes and more alternate between read and write windows cut for this rate; 0 = never
     uint32_t windowAlignedMBps = 7100000;   // the same for launches of segments that all start at multiples of kWindowAlignBytes in source and destination, which hold more; 0 = the rate above
     uint32_t windowLongMBps = 7400000;      // and for those of them whose segments are kWindowLongSegmentBytes and longer on average, which hold more still; 0 = the rate above

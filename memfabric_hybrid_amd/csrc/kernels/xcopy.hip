@@ -510,27 +510,14 @@ __device__ __forceinline__ uint64_t Uniform(uint64_t v)
     return (static_cast<uint64_t>(Uniform(static_cast<uint32_t>(v >> 32))) << 32) | Uniform(static_cast<uint32_t>(v));
 }
 
-// kHeader: chunk count, group shift and pattern come from the header the device-side planner left in
-// device memory (the host knows none of them) instead of the kernel arguments.
 // kHold: as for the inline kernel, for launches of one chunk per workgroup (the host knows the chunk count).
-template <bool kNtLoad, int kStore, bool kHeader, int kHold = kHoldNone>
+template <bool kNtLoad, int kStore, int kHold = kHoldNone>
 __global__ __launch_bounds__(kXcopyThreads) void XcopyTableKernel(const TablePlan plan, uint32_t holdTicks)
 {
     const uint64_t t0 = kHold != kHoldNone ? wall_clock64() : 0;
-    uint32_t nchunk = plan.nchunk;
-    uint32_t shift = plan.groupShift;
-    ChunkPattern pattern = plan.pattern;
-    if (kHeader) {
-        const TableHeader *__restrict__ header = plan.header;
-        nchunk = Uniform(header->nchunk);
-        shift = Uniform(header->groupShift);
-        pattern.period = Uniform(header->pattern.period);
-        pattern.chunksPerPeriod = Uniform(header->pattern.chunksPerPeriod);
-#pragma unroll
-        for (uint32_t i = 0; i <= kMaxPeriod; ++i) {
-            pattern.start[i] = Uniform(header->pattern.start[i]);
-        }
-    }
+    const uint32_t nchunk = plan.nchunk;
+    const uint32_t shift = plan.groupShift;
+    const ChunkPattern pattern = plan.pattern;
     uint32_t c = blockIdx.x;
     if (c >= nchunk) {
         return;
@@ -570,30 +557,14 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyTableKernel(const TablePla
         }
     }
     const uint32_t lane = threadIdx.x & 63u;
-    // A workgroup that walks several chunks of a table it looks up through the map (the host did not know the chunk
-    // count when it sized the grid) takes a run of consecutive chunks: their owners lie in the same few segments,
-    // whose prefix entries and triples the lookup then finds in cache (16 384 ragged segments, four chunks per
-    // workgroup: 907 against 963 us with the grid as the stride).  Under a pattern, where the lookup is a division,
-    // the stride stays: all workgroups then write one contiguous span per round.
-    uint32_t step = gridDim.x;
-    uint32_t stop = nchunk;
-    if (kHeader) {
-        const uint32_t per = (nchunk + gridDim.x - 1) / gridDim.x;
-        c = blockIdx.x * per;
-        step = 1;
-        stop = c + per < nchunk ? c + per : nchunk;
-        if (c >= stop) {
-            return;
-        }
-    }
     // even lanes fetch the map entry of the chunk's group, odd lanes the one behind it
     uint32_t bounds = plan.group[(c >> shift) + (lane & 1u)];
     for (;;) {
         const uint32_t lo = __builtin_amdgcn_readlane(bounds, 0);
         const uint32_t hiEx = __builtin_amdgcn_readlane(bounds, 1) + 1;
         const ChunkRef r = OwnerOf(plan.triples, plan.first, lo, hiEx, c, lane);
-        const uint32_t next = c + step;
-        const bool more = next < stop;
+        const uint32_t next = c + gridDim.x;
+        const bool more = next < nchunk;
         if (more) {
             bounds = plan.group[(next >> shift) + (lane & 1u)];
         }
@@ -605,273 +576,109 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyTableKernel(const TablePla
     }
 }
 
-// Device-side planner for a table the host cannot read: chunk prefix, group map and, where the chunk
-// counts repeat with a short period, the pattern that lets the table kernel do without both.
-__device__ __forceinline__ uint32_t ChunksOf(const uint64_t *__restrict__ triples, uint32_t i, uint32_t units)
+// A table that only the GPU can read, copied as xcopy_plan.h says: item (segment, part), parts in a row.  The launch is sized from
+// the segment count alone, so a workgroup walks the items with the grid as its stride; it fetches the next item's triple before
+// it copies the current item.  What bounds it is HBM; a launch in front of it that planned the table (chunk prefix, owner map,
+// repeating pattern) took 8 us, after which the copy was no faster: 4096 pages of 32 KiB scattered 60.0 / 52.8 us with the
+// planner / so, 16 080 pages of 8 KiB 76.7 / 57.9, 100 pages 10.0 / 7.1, 2000 ragged segments of up to 70 KB 41.5 / 36.5, 16 384 of up to
+// 262 KB 940 / 897, one of 1 GiB among 4096 short ones 459 / 411.
+template <bool kNtLoad, int kStore>
+__global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_t *__restrict__ triples, uint32_t nseg, uint32_t units,
+                                                                   RestList *__restrict__ rest, uint32_t capacity)
 {
-    return static_cast<uint32_t>(SegmentChunks(triples[3ull * i + 1], triples[3ull * i + 2], units));
-}
-
-__device__ __forceinline__ uint32_t WaveInclusiveSum(uint32_t v, uint32_t lane)
-{
+    const uint32_t sample = (threadIdx.x & 63u) < kDirectSample && (threadIdx.x & 63u) < nseg ? threadIdx.x & 63u : 0;
+    const uint64_t sampled = SegmentChunks(triples[3ull * sample + 1], triples[3ull * sample + 2], units);
+    uint32_t parts = 1;
 #pragma unroll
-    for (uint32_t d = 1; d < 64; d <<= 1) {
-        const uint32_t o = __shfl_up(v, d, 64);
-        v += lane >= d ? o : 0u;
+    for (uint32_t i = 0; i < kDirectSample; ++i) {
+        const uint32_t chunks = __builtin_amdgcn_readlane(sampled < kDirectMaxParts ? static_cast<uint32_t>(sampled) : kDirectMaxParts, i);
+        parts = chunks > parts ? chunks : parts;
     }
-    return v;
-}
-
-__device__ __forceinline__ uint32_t WaveSum(uint32_t v)
-{
-#pragma unroll
-    for (uint32_t d = 32; d != 0; d >>= 1) {
-        v += __shfl_xor(v, d, 64);
+    uint32_t seg = blockIdx.x / parts;
+    uint32_t part = blockIdx.x - seg * parts;
+    if (seg >= nseg) {
+        return;
     }
-    return v;
-}
-
-__device__ __forceinline__ uint32_t WaveAnd(uint32_t v)
-{
-#pragma unroll
-    for (uint32_t d = 32; d != 0; d >>= 1) {
-        v &= __shfl_xor(v, d, 64);
-    }
-    return v;
-}
-
-constexpr uint32_t kPlanWaves = kPlanThreads / 64;
-constexpr uint32_t kAllPeriods = ((1u << kMaxPeriod) - 1) << 1;     // bit p: the counts repeat with period p
-
-// First of two launches for tables beyond kPlanSingleBlockSegs segments: every workgroup sums the chunk
-// counts of its kPlanThreads segments and notes which periods they contradict.
-__global__ __launch_bounds__(kPlanThreads) void XcopyPlanSumsKernel(const uint64_t *__restrict__ triples, uint32_t nseg, uint32_t units,
-                                                                    uint32_t *__restrict__ scratch, uint32_t groupCapacity)
-{
-    __shared__ uint32_t counts[kMaxPeriod + kPlanThreads];
-    __shared__ uint32_t waveSum[kPlanWaves];
-    __shared__ uint32_t waveAlive[kPlanWaves];
-    const ScratchLayout at = ScratchLayoutFor(nseg, groupCapacity);
-    const uint32_t tid = threadIdx.x;
-    const uint32_t seg0 = blockIdx.x * kPlanThreads;
-    const uint32_t i = seg0 + tid;
-    const uint32_t mine = i < nseg ? ChunksOf(triples, i, units) : 0u;
-    counts[kMaxPeriod + tid] = mine;
-    if (tid < kMaxPeriod) {
-        counts[tid] = seg0 + tid >= kMaxPeriod ? ChunksOf(triples, seg0 + tid - kMaxPeriod, units) : 0u;
-    }
-    __syncthreads();
-    uint32_t alive = kAllPeriods;
-    if (i < nseg) {
-#pragma unroll
-        for (uint32_t p = 1; p <= kMaxPeriod; ++p) {
-            if (i >= p && counts[kMaxPeriod + tid - p] != mine) {
-                alive &= ~(1u << p);
-            }
+    const uint32_t segStep = gridDim.x / parts;
+    const uint32_t partStep = gridDim.x - segStep * parts;
+    const uint64_t own = static_cast<uint64_t>(parts) * kDirectRounds;     // chunks of a segment that are copied here
+    uint64_t src = triples[3ull * seg];
+    uint64_t dst = triples[3ull * seg + 1];
+    uint64_t len = triples[3ull * seg + 2];
+    for (;;) {
+        const uint32_t carry = part + partStep >= parts ? 1 : 0;
+        const uint64_t next = static_cast<uint64_t>(seg) + segStep + carry;
+        const bool more = next < nseg;
+        const uint64_t *t = triples + 3 * (more ? next : seg);             // requested now, needed after the copy
+        const uint64_t nsrc = t[0];
+        const uint64_t ndst = t[1];
+        const uint64_t nlen = t[2];
+        const uint64_t chunks = SegmentChunks(dst, len, units);
+        for (uint64_t c = part; c < chunks && c < own; c += parts) {
+            CopyChunk<kNtLoad, kStore>(src, dst, len, c, units);
         }
-    }
-    const uint32_t sum = WaveSum(mine);
-    const uint32_t all = WaveAnd(alive);
-    if ((tid & 63u) == 0) {
-        waveSum[tid >> 6] = sum;
-        waveAlive[tid >> 6] = all;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        uint32_t s = 0;
-        uint32_t a = kAllPeriods;
-        for (uint32_t w = 0; w < kPlanWaves; ++w) {
-            s += waveSum[w];
-            a &= waveAlive[w];
-        }
-        scratch[at.blockSum + blockIdx.x] = s;
-        scratch[at.blockAlive + blockIdx.x] = a;
-    }
-}
-
-// The planner proper.  Thread t takes kEach consecutive segments.  One workgroup and one launch for up to
-// kPlanSingleBlockSegs segments (kEach = 1, 2, 4 or 8); beyond, one workgroup per kPlanThreads segments
-// (kEach = 1) behind XcopyPlanSumsKernel, which has left the sums and the periods of all workgroups.
-template <uint32_t kEach>
-__global__ __launch_bounds__(kPlanThreads) void XcopyPlanKernel(const uint64_t *__restrict__ triples, uint32_t nseg, uint32_t units,
-                                                                uint32_t *__restrict__ scratch, uint32_t groupCapacity)
-{
-    __shared__ uint32_t counts[kMaxPeriod + kEach * kPlanThreads];
-    __shared__ uint32_t waveTotal[kPlanWaves];      // inclusive sums of the waves, then their exclusive prefix
-    __shared__ uint32_t reduced[2 * kPlanWaves + 4];
-    const ScratchLayout at = ScratchLayoutFor(nseg, groupCapacity);
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u;
-    const uint32_t wave = tid >> 6;
-    const bool alone = gridDim.x == 1;
-    const uint32_t i0 = (blockIdx.x * kPlanThreads + tid) * kEach;
-
-    uint32_t mine[kEach];
-    uint32_t sum = 0;
-#pragma unroll
-    for (uint32_t q = 0; q < kEach; ++q) {
-        mine[q] = i0 + q < nseg ? ChunksOf(triples, i0 + q, units) : 0u;
-        sum += mine[q];
-        if (alone) {
-            counts[kMaxPeriod + tid * kEach + q] = mine[q];
-        }
-    }
-    if (alone && tid < kMaxPeriod) {
-        counts[tid] = 0;
-    }
-    const uint32_t incl = WaveInclusiveSum(sum, lane);
-    if (lane == 63) {
-        waveTotal[wave] = incl;
-    }
-    __syncthreads();
-
-    uint32_t aliveMine = kAllPeriods;
-    if (alone) {
-        // the eight counts in front of this thread's segments, then its own, checked against every period
-        uint32_t window[kMaxPeriod + kEach];
-#pragma unroll
-        for (uint32_t w = 0; w < kMaxPeriod; ++w) {
-            window[w] = counts[tid * kEach + w];
-        }
-#pragma unroll
-        for (uint32_t q = 0; q < kEach; ++q) {
-            window[kMaxPeriod + q] = mine[q];
-        }
-#pragma unroll
-        for (uint32_t q = 0; q < kEach; ++q) {
-#pragma unroll
-            for (uint32_t p = 1; p <= kMaxPeriod; ++p) {
-                if (i0 + q < nseg && i0 + q >= p && window[kMaxPeriod + q - p] != mine[q]) {
-                    aliveMine &= ~(1u << p);
+        if (part == 0 && chunks > own) {
+            const uint64_t at = SegmentGeometry(dst, len).head + own * units * kUnitBytes;
+            const uint64_t left = len - at;
+            const uint64_t each = RestPieceBytesFor(left);
+            const uint32_t count = static_cast<uint32_t>((left + each - 1) / each);
+            __shared__ uint32_t first;
+            if (threadIdx.x == 0) {
+                // a full list takes no more, so that the count stays far from its end
+                first = __hip_atomic_load(&rest->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (first < capacity) {
+                    first = __hip_atomic_fetch_add(&rest->count, count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
             }
+            __syncthreads();
+            const uint32_t room = first < capacity ? capacity - first : 0;
+            for (uint32_t i = threadIdx.x; i < count && i < room; i += blockDim.x) {
+                const uint64_t from = i * each;
+                rest->piece[first + i] = RestPiece{src + at + from, dst + at + from, left - from < each ? left - from : each};
+            }
+            if (count > room) {                                            // a list of thousands of long segments: the others go on here
+                const uint64_t from = at + room * each;
+                const uint64_t over = SegmentChunks(dst + from, len - from, units);
+                for (uint64_t c = 0; c < over; ++c) {
+                    CopyChunk<kNtLoad, kStore>(src + from, dst + from, len - from, c, units);
+                }
+            }
+            __syncthreads();                                               // `first` is free again
         }
+        if (!more) {
+            return;
+        }
+        seg = static_cast<uint32_t>(next);
+        part = part + partStep - (carry != 0 ? parts : 0);
+        src = Uniform(nsrc);
+        dst = Uniform(ndst);
+        len = Uniform(nlen);
     }
-    const uint32_t aliveWave = WaveAnd(aliveMine);
-    // wave 0: exclusive prefix over the wave totals and their sum
-    if (wave == 0) {
-        const uint32_t own = lane < kPlanWaves ? waveTotal[lane] : 0u;
-        const uint32_t scan = WaveInclusiveSum(own, lane);
-        if (lane < kPlanWaves) {
-            waveTotal[lane] = scan - own;
-        }
-        if (lane == 63) {
-            reduced[2 * kPlanWaves] = scan;          // chunks of this workgroup's segments
-        }
+}
+
+// The pieces XcopyDirectKernel has listed; usually none (1.6 us then).  The last workgroup leaves the list empty.
+template <bool kNtLoad, int kStore>
+__global__ __launch_bounds__(kXcopyThreads) void XcopyRestKernel(RestList *rest, uint32_t capacity, uint32_t units)
+{
+    const uint32_t listed = Uniform(__hip_atomic_load(&rest->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    if (listed == 0) {
+        return;
     }
-    if (lane == 0) {
-        reduced[wave] = aliveWave;
+    const uint32_t count = listed < capacity ? listed : capacity;
+    for (uint32_t p = blockIdx.x; p < count; p += gridDim.x) {
+        const RestPiece r = rest->piece[p];
+        const uint64_t src = Uniform(r.src);
+        const uint64_t dst = Uniform(r.dst);
+        const uint64_t len = Uniform(r.len);
+        const uint64_t chunks = SegmentChunks(dst, len, units);
+        for (uint64_t c = 0; c < chunks; ++c) {
+            CopyChunk<kNtLoad, kStore>(src, dst, len, c, units);
+        }
     }
     __syncthreads();
-
-    // chunks in front of this workgroup, chunks of the whole table, periods still alive
-    uint32_t base = 0;
-    uint32_t total = reduced[2 * kPlanWaves];
-    uint32_t alive = kAllPeriods;
-    if (alone) {
-        for (uint32_t w = 0; w < kPlanWaves; ++w) {
-            alive &= reduced[w];
-        }
-    } else {
-        uint32_t front = 0;
-        uint32_t whole = 0;
-        uint32_t bits = kAllPeriods;
-        for (uint32_t b = tid; b < gridDim.x; b += kPlanThreads) {
-            const uint32_t blockSum = scratch[at.blockSum + b];
-            whole += blockSum;
-            front += b < blockIdx.x ? blockSum : 0u;
-            bits &= scratch[at.blockAlive + b];
-        }
-        front = WaveSum(front);
-        whole = WaveSum(whole);
-        bits = WaveAnd(bits);
-        __syncthreads();                               // every thread has read reduced[] above
-        if (lane == 0) {
-            reduced[wave] = front;
-            reduced[kPlanWaves + wave] = whole;
-            counts[wave] = bits;
-        }
-        __syncthreads();
-        total = 0;
-        for (uint32_t w = 0; w < kPlanWaves; ++w) {
-            base += reduced[w];
-            total += reduced[kPlanWaves + w];
-            alive &= counts[w];
-        }
-    }
-
-    const uint32_t shift = GroupShiftFor(total, at.groupCapacity);
-    const uint32_t ngroups = GroupCount(total, shift);
-    uint32_t *first = scratch + at.first;
-    uint32_t *group = scratch + at.group;
-    uint32_t f = base + waveTotal[wave] + incl - sum;
-#pragma unroll
-    for (uint32_t q = 0; q < kEach; ++q) {
-        const uint32_t i = i0 + q;
-        const bool live = i < nseg;
-        if (live) {
-            first[i] = f;
-            if (i == nseg - 1) {
-                first[nseg] = f + mine[q];
-            }
-        }
-        // map entries of the groups whose first chunk this segment owns; the segment that owns the last chunk also closes the map
-        uint32_t gLo = 1;
-        uint32_t gHi = 0;
-        if (live && mine[q] != 0) {
-            gLo = static_cast<uint32_t>((static_cast<uint64_t>(f) + (1ull << shift) - 1) >> shift);
-            gHi = (f + mine[q] - 1) >> shift;
-            if (f + mine[q] == total) {
-                group[ngroups] = i;
-            }
-        }
-        const bool some = gLo <= gHi;
-        const bool many = some && gHi - gLo >= 4;
-        if (some && !many) {
-            for (uint32_t g = gLo; g <= gHi; ++g) {
-                group[g] = i;
-            }
-        }
-        // a segment of many groups is written by its whole wave
-        uint64_t todo = __ballot(many);
-        while (todo != 0) {
-            const uint32_t from = static_cast<uint32_t>(__builtin_ctzll(todo));
-            todo &= todo - 1;
-            const uint32_t lo = __builtin_amdgcn_readlane(gLo, from);
-            const uint32_t hi = __builtin_amdgcn_readlane(gHi, from);
-            const uint32_t owner = __builtin_amdgcn_readlane(i, from);
-            for (uint64_t g = static_cast<uint64_t>(lo) + lane; g <= hi; g += 64) {
-                group[g] = owner;
-            }
-        }
-        f += mine[q];
-    }
-
-    if (blockIdx.x == 0 && tid == 0) {
-        TableHeader *header = reinterpret_cast<TableHeader *>(scratch);
-        header->nchunk = total;
-        header->groupShift = shift;
-        header->reserved[0] = 0;
-        header->reserved[1] = 0;
-        ChunkPattern pattern{};
-        if (alive != 0 && total != 0) {
-            // the shortest period never exceeds the segment count: period nseg is never contradicted
-            const uint32_t period = static_cast<uint32_t>(__builtin_ctz(alive));
-            uint32_t run = 0;
-            for (uint32_t q = 0; q < period; ++q) {
-                pattern.start[q] = run;
-                run += ChunksOf(triples, q, units);
-            }
-            pattern.start[period] = run;
-            if (run != 0) {
-                pattern.period = period;
-                pattern.chunksPerPeriod = run;
-            } else {
-                pattern = ChunkPattern{};
-            }
-        }
-        header->pattern = pattern;
-        header->pad = 0;
+    if (threadIdx.x == 0 && __hip_atomic_fetch_add(&rest->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+        __hip_atomic_store(&rest->done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&rest->count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -1011,50 +818,36 @@ int LaunchWindowed(const InlinePlan &plan, uint32_t grid, uint32_t windowMBps, h
 template <bool kNtLoad, int kStore>
 int LaunchTable(const TablePlan &plan, uint32_t grid, uint32_t lanes, hipStream_t stream, uint32_t holdNanos)
 {
-    if (plan.header != nullptr) {
-        hipLaunchKernelGGL((XcopyTableKernel<kNtLoad, kStore, true>), dim3(grid), dim3(lanes), 0, stream, plan, 0u);
-        return static_cast<int>(hipGetLastError());
-    }
     const bool deep = plan.units == kWindowUnits && holdNanos != 0;
     if (deep) {
         lanes = 64;
     }
     const uint32_t ticks = grid == plan.nchunk && lanes == 64 ? HoldTicks(holdNanos) : 0;
     if (ticks != 0 && deep) {
-        hipLaunchKernelGGL((XcopyTableKernel<kNtLoad, kStore, false, kHoldDeep>), dim3(grid), dim3(lanes), 0, stream, plan, ticks);
+        hipLaunchKernelGGL((XcopyTableKernel<kNtLoad, kStore, kHoldDeep>), dim3(grid), dim3(lanes), 0, stream, plan, ticks);
     } else if (ticks != 0) {
-        hipLaunchKernelGGL((XcopyTableKernel<kNtLoad, kStore, false, kHoldShallow>), dim3(grid), dim3(lanes), 0, stream, plan, ticks);
+        hipLaunchKernelGGL((XcopyTableKernel<kNtLoad, kStore, kHoldShallow>), dim3(grid), dim3(lanes), 0, stream, plan, ticks);
     } else {
-        hipLaunchKernelGGL((XcopyTableKernel<kNtLoad, kStore, false>), dim3(grid), dim3(lanes), 0, stream, plan, 0u);
+        hipLaunchKernelGGL((XcopyTableKernel<kNtLoad, kStore>), dim3(grid), dim3(lanes), 0, stream, plan, 0u);
     }
     return static_cast<int>(hipGetLastError());
 }
 
-// The planner's one or two launches for a table of nseg segments in device memory.
-int LaunchPlanner(const uint64_t *triples, uint32_t nseg, uint32_t units, uint32_t *scratch, uint32_t groupCapacity,
-                  hipStream_t stream)
+template <bool kNtLoad, int kStore>
+int LaunchDirect(const uint64_t *triples, uint32_t nseg, uint32_t units, uint32_t grid, uint32_t restGrid, uint32_t lanes, RestList *rest,
+                 uint32_t capacity, hipStream_t stream)
 {
-    const uint32_t blocks = PlanBlocks(nseg);
-    if (blocks > 1) {
-        hipLaunchKernelGGL(XcopyPlanSumsKernel, dim3(blocks), dim3(kPlanThreads), 0, stream, triples, nseg, units, scratch,
-                           groupCapacity);
-        const hipError_t err = hipGetLastError();
-        if (err != hipSuccess) {
-            return static_cast<int>(err);
-        }
+    hipLaunchKernelGGL((XcopyDirectKernel<kNtLoad, kStore>), dim3(grid), dim3(lanes), 0, stream, triples, nseg, units, rest, capacity);
+    hipError_t err = hipGetLastError();
+    if (err != hipSuccess) {
+        return static_cast<int>(err);
     }
-    const uint32_t tiles = blocks > 1 ? 1u : (nseg + kPlanThreads - 1) / kPlanThreads;   // segments per thread
-    if (tiles <= 1) {
-        hipLaunchKernelGGL(XcopyPlanKernel<1>, dim3(blocks), dim3(kPlanThreads), 0, stream, triples, nseg, units, scratch, groupCapacity);
-    } else if (tiles <= 2) {
-        hipLaunchKernelGGL(XcopyPlanKernel<2>, dim3(1), dim3(kPlanThreads), 0, stream, triples, nseg, units, scratch, groupCapacity);
-    } else if (tiles <= 4) {
-        hipLaunchKernelGGL(XcopyPlanKernel<4>, dim3(1), dim3(kPlanThreads), 0, stream, triples, nseg, units, scratch, groupCapacity);
-    } else {
-        hipLaunchKernelGGL(XcopyPlanKernel<kPlanTiles>, dim3(1), dim3(kPlanThreads), 0, stream, triples, nseg, units, scratch,
-                           groupCapacity);
+    hipLaunchKernelGGL((XcopyRestKernel<kNtLoad, kStore>), dim3(restGrid), dim3(lanes), 0, stream, rest, capacity, units);
+    err = hipGetLastError();
+    if (err != hipSuccess) {   // what the first launch has listed must not be taken for the next call's
+        hipLaunchKernelGGL(XcopySignalKernel, dim3(1), dim3(64), 0, stream, reinterpret_cast<uint64_t *>(rest), 0u);
     }
-    return static_cast<int>(hipGetLastError());
+    return static_cast<int>(err);
 }
 
 int Signal(void *mask, uint32_t maskValue, hipStream_t stream)
@@ -1161,16 +954,12 @@ extern "C" int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, 
     if (plan.nseg == 0 || grid == 0 || plan.triples == nullptr) {
         return -1;
     }
-    if (plan.header == nullptr) {
-        if (pat.period == 0 && (plan.first == nullptr || plan.group == nullptr || plan.groupShift < mf::kGroupShiftMin ||
-                                plan.groupShift > 31)) {
-            return -1;
-        }
-        if (pat.period != 0 && (pat.period > mf::kMaxPeriod || pat.chunksPerPeriod == 0 || pat.start[0] != 0 ||
-                                pat.start[pat.period] != pat.chunksPerPeriod || mf::PatternChunks(pat, plan.nseg) != plan.nchunk)) {
-            return -1;
-        }
-    } else if (plan.first == nullptr || plan.group == nullptr) {
+    if (pat.period == 0 && (plan.first == nullptr || plan.group == nullptr || plan.groupShift < mf::kGroupShiftMin ||
+                            plan.groupShift > 31)) {
+        return -1;
+    }
+    if (pat.period != 0 && (pat.period > mf::kMaxPeriod || pat.chunksPerPeriod == 0 || pat.start[0] != 0 ||
+                            pat.start[pat.period] != pat.chunksPerPeriod || mf::PatternChunks(pat, plan.nseg) != plan.nchunk)) {
         return -1;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -1181,30 +970,21 @@ extern "C" int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, 
     return err != 0 ? err : mf::Signal(mask, maskValue, s);
 }
 
-extern "C" uint64_t mfk_xcopy_plan_scratch_words(uint32_t nseg, uint32_t groupCapacity)
+// rest: a RestList with room for `capacity` pieces, its counts 0.
+extern "C" int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *rest,
+                                uint32_t capacity, void *mask, uint32_t maskValue, void *stream)
 {
-    return mf::ScratchLayoutFor(nseg, groupCapacity).words;
-}
-
-// scratch: mfk_xcopy_plan_scratch_words(nseg, groupCapacity) words of device memory.  *tablePlan receives the plan for
-// mfk_xcopy_table that reads what the planner leaves there.
-extern "C" int mfk_xcopy_plan(const void *triples, uint32_t nseg, uint32_t units, void *scratch, uint32_t groupCapacity,
-                              void *tablePlan, void *stream)
-{
-    if (nseg == 0 || scratch == nullptr || groupCapacity < 2 || tablePlan == nullptr) {
+    using namespace mf;
+    if (nseg == 0 || grid == 0 || restGrid == 0 || rest == nullptr || capacity == 0) {
         return -1;
     }
-    uint32_t *words = static_cast<uint32_t *>(scratch);
-    const mf::ScratchLayout at = mf::ScratchLayoutFor(nseg, groupCapacity);
-    mf::TablePlan &plan = *static_cast<mf::TablePlan *>(tablePlan);
-    plan = mf::TablePlan{};
-    plan.triples = static_cast<const uint64_t *>(triples);
-    plan.first = words + at.first;
-    plan.group = words + at.group;
-    plan.header = reinterpret_cast<const mf::TableHeader *>(words);
-    plan.nseg = nseg;
-    plan.units = units;
-    return mf::LaunchPlanner(plan.triples, nseg, units, words, groupCapacity, static_cast<hipStream_t>(stream));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int err = WithPolicy(PolicyOf(route), [&](auto ntLoad, auto store) {
+        return LaunchDirect<decltype(ntLoad)::value, decltype(store)::value>(static_cast<const uint64_t *>(triples), nseg, units, grid, restGrid,
+                                                                             LanesFor(units, route), static_cast<RestList *>(rest),
+                                                                             capacity, s);
+    });
+    return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
 // Every copy kernel once, on plans that hold nothing, so that a caller who captures a stream later finds the code of
@@ -1229,14 +1009,14 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
             constexpr int kSt = decltype(store)::value;
             hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, empty, 0u);
             hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 0u);
-            hipLaunchKernelGGL((XcopyTableKernel<kNt, kSt, false, kHoldNone>), dim3(1), dim3(64), 0, s, none, 0u);
+            hipLaunchKernelGGL((XcopyTableKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, none, 0u);
             if (route == MFRT_ROUTE_HBM) {
                 hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, empty, 1u);
                 hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, empty, 1u);
                 hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 1u);
                 hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kWindowUnits, 1u);
-                hipLaunchKernelGGL((XcopyTableKernel<kNt, kSt, false, kHoldShallow>), dim3(1), dim3(64), 0, s, none, 1u);
-                hipLaunchKernelGGL((XcopyTableKernel<kNt, kSt, false, kHoldDeep>), dim3(1), dim3(64), 0, s, none, 1u);
+                hipLaunchKernelGGL((XcopyTableKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, none, 1u);
+                hipLaunchKernelGGL((XcopyTableKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, none, 1u);
                 hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
             }
             return 0;
@@ -1375,14 +1155,11 @@ extern "C" int mfk_xcopy_calibrate(void *stream, const uint32_t *holdNanos, cons
 }
 
 #ifndef MF_RT_HIDDEN   // the plugin library has no entry point that needs it
-// Scratch of the entry point that allocates nothing (mfk_xcopy_table_static): header, chunk prefix,
-// the planner's partial sums and the group map, written by the planner and read by XcopyTableKernel of the
-// same call.  One copy per GPU, held until the process ends.  In host code the array's name is only a
-// handle for hipGetSymbolAddress: kernels get the address that call returned for the current device,
-// never the name.
-constexpr uint32_t kStaticGroupCapacity = MFK_STATIC_TABLE_SEGMENTS;
-constexpr uint64_t kStaticScratchWords = mf::ScratchLayoutFor(MFK_STATIC_TABLE_SEGMENTS, kStaticGroupCapacity).words;
-static __device__ __align__(256) uint32_t scratch[kStaticScratchWords];
+// List of the entry point that allocates nothing (mfk_xcopy_table_static).  One copy per GPU, zero when its code is loaded and
+// held until the process ends.  In host code the array's name is only a handle for hipGetSymbolAddress: kernels get the
+// address that call returned for the current device, never the name.
+constexpr uint32_t kStaticRestCapacity = 10240;
+static __device__ __align__(256) uint32_t scratch[mf::RestListBytes(kStaticRestCapacity) / 4];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -1416,30 +1193,18 @@ extern "C" int mfk_xcopy_static_setup(void)
         g_staticDone[dev] = nullptr;   // calls then go unguarded, as documented for callers that overlap them
         (void)hipGetLastError();
     }
-    // The kernels of the device-table path once, on a table of no segments whose header lands in the array (what
-    // mfk_xcopy_prelaunch cannot do without device memory): a caller may then capture its very first call.
+    // The kernels of the device-table path once, on a table of no segments (what mfk_xcopy_prelaunch cannot do without device
+    // memory): a caller may then capture its very first call.
     {
         using namespace mf;
         uint32_t *words = g_scratchOf[dev];
+        RestList *rest = reinterpret_cast<RestList *>(words);
         const uint64_t *none = reinterpret_cast<const uint64_t *>(words);
-        hipLaunchKernelGGL(XcopySignalKernel, dim3(1), dim3(64), 0, nullptr, reinterpret_cast<uint64_t *>(words + 2), 0u);   // the header's spare words
-        hipLaunchKernelGGL(XcopyPlanSumsKernel, dim3(1), dim3(kPlanThreads), 0, nullptr, none, 0u, kXcopyThreads, words, kStaticGroupCapacity);
-        hipLaunchKernelGGL(XcopyPlanKernel<1>, dim3(1), dim3(kPlanThreads), 0, nullptr, none, 0u, kXcopyThreads, words, kStaticGroupCapacity);
-        hipLaunchKernelGGL(XcopyPlanKernel<2>, dim3(1), dim3(kPlanThreads), 0, nullptr, none, 0u, kXcopyThreads, words, kStaticGroupCapacity);
-        hipLaunchKernelGGL(XcopyPlanKernel<4>, dim3(1), dim3(kPlanThreads), 0, nullptr, none, 0u, kXcopyThreads, words, kStaticGroupCapacity);
-        hipLaunchKernelGGL(XcopyPlanKernel<8>, dim3(1), dim3(kPlanThreads), 0, nullptr, none, 0u, kXcopyThreads, words, kStaticGroupCapacity);
-        const ScratchLayout at = ScratchLayoutFor(0, kStaticGroupCapacity);
-        TablePlan plan{};
-        plan.triples = none;
-        plan.first = words + at.first;
-        plan.group = words + at.group;
-        plan.header = reinterpret_cast<const TableHeader *>(words);   // the planner launches above left nchunk = 0 there
-        plan.units = kXcopyThreads;
+        hipLaunchKernelGGL(XcopySignalKernel, dim3(1), dim3(64), 0, nullptr, reinterpret_cast<uint64_t *>(rest->reserved), 0u);
         for (int route = MFRT_ROUTE_HBM; route <= MFRT_ROUTE_FROM_HOST; ++route) {
             (void)WithPolicy(PolicyOf(route), [&](auto ntLoad, auto store) {
-                hipLaunchKernelGGL((XcopyTableKernel<decltype(ntLoad)::value, decltype(store)::value, true>), dim3(1), dim3(64), 0,
-                                   nullptr, plan, 0u);
-                return 0;
+                return LaunchDirect<decltype(ntLoad)::value, decltype(store)::value>(none, 0, kXcopyThreads, 1, 1, 64, rest,
+                                                                                     kStaticRestCapacity, nullptr);
             });
         }
         err = hipGetLastError();
@@ -1453,7 +1218,7 @@ extern "C" int mfk_xcopy_static_setup(void)
     return 0;
 }
 
-extern "C" int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid,
+extern "C" int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid,
                                       void *stream)
 {
     if (nseg == 0 || nseg > MFK_STATIC_TABLE_SEGMENTS || grid == 0) {
@@ -1471,12 +1236,7 @@ extern "C" int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32
     if (guarded && g_staticUsed[dev] && g_staticLast[dev] != s && hipStreamWaitEvent(s, g_staticDone[dev], 0) != hipSuccess) {
         return static_cast<int>(hipGetLastError());
     }
-    // the planner writes every word the table kernel reads: nothing has to start at zero
-    mf::TablePlan plan;
-    int err = mfk_xcopy_plan(triples, nseg, units, g_scratchOf[dev], kStaticGroupCapacity, &plan, stream);
-    if (err == 0) {
-        err = mfk_xcopy_table(&plan, route, grid, nullptr, 0, stream, 0);
-    }
+    const int err = mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, g_scratchOf[dev], kStaticRestCapacity, nullptr, 0, stream);
     if (guarded && hipEventRecord(g_staticDone[dev], s) == hipSuccess) {
         g_staticLast[dev] = s;
         g_staticUsed[dev] = true;

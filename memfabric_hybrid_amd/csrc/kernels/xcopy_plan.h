@@ -231,46 +231,38 @@ inline uint32_t BuildGroupMap(const uint32_t *first, uint32_t nseg, uint32_t *gr
     return shift;
 }
 
-// What the device-side planner leaves for the table kernel of the same call (64 bytes).
-struct TableHeader {
-    uint32_t nchunk;
-    uint32_t groupShift;
-    uint32_t reserved[2];
-    ChunkPattern pattern;               // period != 0: owner by division, prefix and group map are not read
-    uint32_t pad;
+// A table that only the GPU can read, copied without a plan.  Its launch takes `parts` items per segment, part j of a segment
+// copying the chunks j, j + parts, ... of it: right for every table, whatever `parts` is, and evenly spread where `parts` is near
+// the chunk count of the usual segment.  That is taken from the first kDirectSample segments, by every wave for itself.
+// A part copies kDirectRounds chunks at most; what a segment holds beyond parts * kDirectRounds chunks is cut into pieces and
+// listed for a second launch, so that no wave is left with a long segment.
+constexpr uint32_t kDirectSample = 8;
+constexpr uint32_t kDirectMaxParts = 64;
+constexpr uint32_t kDirectRounds = 4;
+constexpr uint64_t kRestPieceBytes = 64ull << 10;     // the least
+constexpr uint32_t kRestMaxPieces = 4096;             // of one segment
+
+struct RestPiece {
+    uint64_t src;
+    uint64_t dst;
+    uint64_t len;
 };
-static_assert(sizeof(TableHeader) == 64, "the planner's scratch layout counts on a 64-byte header");
-
-// Segments one workgroup of the device-side planner takes, and its lanes.
-constexpr uint32_t kPlanThreads = 1024;
-constexpr uint32_t kPlanTiles = 8;                          // a workgroup walks up to this many tiles of kPlanThreads segments
-constexpr uint32_t kPlanSingleBlockSegs = kPlanThreads * kPlanTiles;   // up to here one workgroup plans the whole table in one launch
-
-// Words of device scratch the planner and the table kernel of a device-resident table share:
-// header | first[nseg + 1] | blockSum[blocks] | blockAlive[blocks] | group[groupCapacity].
-MF_HD constexpr inline uint32_t PlanBlocks(uint32_t nseg)
+struct RestList {                                     // both counts are 0 between calls
+    uint32_t count;                                   // pieces listed, beyond the capacity too
+    uint32_t done;                                    // workgroups of the second launch that are done with it
+    uint32_t reserved[14];
+    RestPiece piece[1];                               // as many as the list has room for
+};
+static_assert(sizeof(RestList) == 64 + sizeof(RestPiece), "pieces start on a cache line");
+constexpr uint32_t kRestCapacity = 65536;              // 1.5 MiB
+constexpr uint64_t RestListBytes(uint32_t capacity)
 {
-    return nseg <= kPlanSingleBlockSegs ? 1u : (nseg + kPlanThreads - 1) / kPlanThreads;
+    return sizeof(RestList) + static_cast<uint64_t>(capacity - 1) * sizeof(RestPiece);
 }
-struct ScratchLayout {
-    uint32_t first;                     // word offsets
-    uint32_t blockSum;
-    uint32_t blockAlive;
-    uint32_t group;
-    uint32_t groupCapacity;             // entries
-    uint64_t words;
-};
-MF_HD constexpr inline ScratchLayout ScratchLayoutFor(uint32_t nseg, uint32_t groupCapacity)
+MF_HD inline uint64_t RestPieceBytesFor(uint64_t left)
 {
-    ScratchLayout l{};
-    const uint32_t blocks = PlanBlocks(nseg);
-    l.first = sizeof(TableHeader) / 4;
-    l.blockSum = l.first + nseg + 1;
-    l.blockAlive = l.blockSum + blocks;
-    l.group = (l.blockAlive + blocks + 3u) & ~3u;
-    l.groupCapacity = groupCapacity;
-    l.words = static_cast<uint64_t>(l.group) + groupCapacity;
-    return l;
+    const uint64_t each = (left + kRestMaxPieces - 1) / kRestMaxPieces;
+    return (each + kRestPieceBytes - 1) / kRestPieceBytes * kRestPieceBytes;
 }
 
 // A table-driven launch: triples, prefix and group map live in device memory (under a pattern the
@@ -279,7 +271,6 @@ struct TablePlan {
     const uint64_t *triples;            // {src,dst,len} * nseg
     const uint32_t *first;              // nseg + 1 entries, first[nseg] == nchunk
     const uint32_t *group;              // GroupCount(nchunk, groupShift) + 1 entries
-    const TableHeader *header;          // not NULL: nchunk, groupShift and pattern are read from there
     uint32_t nseg;
     uint32_t nchunk;
     uint32_t groupShift;

@@ -92,8 +92,7 @@ uint32_t mfk_xcopy_window_units(void);
 uint32_t mfk_xcopy_window_waves(void);
 int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream);
 /* tablePlan: a mf::TablePlan (kernels/xcopy_plan.h).  Under a pattern its triples may live in pinned host
- * memory and neither prefix nor group map is read; with a header (left by mfk_xcopy_plan on the same stream)
- * chunk count, group shift and pattern are read from device memory and `grid` workgroups walk the chunks.
+ * memory and neither prefix nor group map is read.
  * holdNanos: as for mfk_xcopy_inline, for a launch of one chunk per workgroup between HBM addresses. */
 int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, void *mask, uint32_t maskValue, void *stream,
                     uint32_t holdNanos);
@@ -106,20 +105,18 @@ int mfk_xcopy_calibrate(void *stream, const uint32_t *holdNanos, const uint32_t 
 /* One lane stores `value` (as a 64-bit word, released at system scope) into `word` once everything queued on
  * `stream` before it has finished. */
 int mfk_xcopy_signal(void *word, uint32_t value, void *stream);
-/* Device-side planner for a triple table in device memory: one launch (two beyond 8192 segments) that leaves
- * header, chunk prefix and group map in `scratch` (mfk_xcopy_plan_scratch_words(nseg, groupCapacity) 32-bit words of
- * device memory; groupCapacity: entries of room for the group map, the more the finer) and fills *tablePlan
- * (a mf::TablePlan) for the mfk_xcopy_table call behind it on the same stream. */
-uint64_t mfk_xcopy_plan_scratch_words(uint32_t nseg, uint32_t groupCapacity);
-int mfk_xcopy_plan(const void *triples, uint32_t nseg, uint32_t units, void *scratch, uint32_t groupCapacity, void *tablePlan,
-                   void *stream);
-/* The table form with the planner's scratch in a statically allocated device array instead of memory the
- * engine allocates: no allocation anywhere, at most MFK_STATIC_TABLE_SEGMENTS segments, one call at a
- * time per GPU.  mfk_xcopy_static_setup looks the array's address up for the current device (once per
- * device, at start-up); mfk_xcopy_table_static returns -2 when that has not happened. */
+/* A triple table in device memory, copied without a plan (kernels/xcopy_plan.h says how): `grid` workgroups walk its segments,
+ * `restGrid` those of the second launch the pieces of long segments that the first has listed in `rest`, a mf::RestList in
+ * device memory with room for `capacity` pieces whose counts are 0 before and after.  One call at a time may use a list. */
+int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *rest,
+                     uint32_t capacity, void *mask, uint32_t maskValue, void *stream);
+/* The same with the list in a statically allocated device array instead of memory the engine allocates: no allocation
+ * anywhere, at most MFK_STATIC_TABLE_SEGMENTS segments, one call at a time per GPU.  mfk_xcopy_static_setup looks the
+ * array's address up for the current device (once per device, at start-up); mfk_xcopy_table_static returns -2 when that has
+ * not happened. */
 #define MFK_STATIC_TABLE_SEGMENTS 32768u
 int mfk_xcopy_static_setup(void);
-int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, void *stream);
+int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *stream);
 
 /* ---- MoE launchers (kernels/moe.hip) ---------------------------------------- */
 uint64_t mfk_moe_workspace_bytes(uint32_t tokens, uint32_t topK, uint32_t experts);

@@ -313,8 +313,7 @@ int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, 
     return mfk_xcopy_inline(inlinePlan, 0, p.nchunk, mask, maskValue, stream, 0, 0);
 }
 
-// As the kernel: chunk count, group shift and pattern out of the header when there is one; the owner of a
-// chunk by division under a pattern, else from the two group-map entries around it and the prefix between
+// As the kernel: the owner of a chunk by division under a pattern, else from the two group-map entries around it and the prefix between
 // them.  A map whose entries do not bracket the owner fails the launch.
 int mfk_xcopy_table(const void *tablePlan, int, uint32_t grid, void *mask, uint32_t maskValue, void *, uint32_t holdNanos)
 {
@@ -322,17 +321,13 @@ int mfk_xcopy_table(const void *tablePlan, int, uint32_t grid, void *mask, uint3
     const mf::TablePlan &plan = *static_cast<const mf::TablePlan *>(tablePlan);
     const uint64_t *t = plan.triples;
     const uint32_t *f = plan.first;
-    uint32_t total = plan.nchunk;
-    uint32_t shift = plan.groupShift;
-    mf::ChunkPattern pat = plan.pattern;
+    const uint32_t total = plan.nchunk;
+    const uint32_t shift = plan.groupShift;
+    const mf::ChunkPattern pat = plan.pattern;
     if (plan.nseg == 0 || grid == 0 || t == nullptr) {
         return -1;
     }
-    if (plan.header != nullptr) {
-        total = plan.header->nchunk;
-        shift = plan.header->groupShift;
-        pat = plan.header->pattern;
-    } else if (pat.period != 0 && (pat.period > mf::kMaxPeriod || mf::PatternChunks(pat, plan.nseg) != total)) {
+    if (pat.period != 0 && (pat.period > mf::kMaxPeriod || mf::PatternChunks(pat, plan.nseg) != total)) {
         return -1;
     }
     if (pat.period == 0 && (f == nullptr || plan.group == nullptr || shift < mf::kGroupShiftMin || shift > 31)) {
@@ -376,67 +371,62 @@ int mfk_xcopy_table(const void *tablePlan, int, uint32_t grid, void *mask, uint3
     return 0;
 }
 
-uint64_t mfk_xcopy_plan_scratch_words(uint32_t nseg, uint32_t groupCapacity)
+// The direct copy of a device-resident table restated: the parts of every segment, and the pieces of long ones out of a list
+// that a small capacity makes run over.
+int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int, uint32_t grid, uint32_t restGrid, void *rest,
+                     uint32_t capacity, void *mask, uint32_t maskValue, void *)
 {
-    return mf::ScratchLayoutFor(nseg, groupCapacity).words;
-}
-
-// The device-side planner restated: same scratch layout, same header, prefix, group map and pattern rule.
-int mfk_xcopy_plan(const void *triples, uint32_t nseg, uint32_t units, void *scratch, uint32_t groupCapacity, void *tablePlan,
-                   void *)
-{
-    if (nseg == 0 || scratch == nullptr || groupCapacity < 2 || tablePlan == nullptr) {
+    mf::RestList *list = static_cast<mf::RestList *>(rest);
+    if (nseg == 0 || grid == 0 || restGrid == 0 || list == nullptr || capacity == 0 || list->count != 0 || list->done != 0) {
         return -1;
     }
-    const uint64_t *t = static_cast<const uint64_t *>(triples);
-    uint32_t *words = static_cast<uint32_t *>(scratch);
-    const mf::ScratchLayout at = mf::ScratchLayoutFor(nseg, groupCapacity);
-    uint32_t *f = words + at.first;
-    uint32_t run = 0;
-    uint32_t alive = 0x1FEu;
-    std::vector<uint32_t> counts(nseg);
-    for (uint32_t i = 0; i < nseg; ++i) {
-        f[i] = run;
-        counts[i] = static_cast<uint32_t>(mf::SegmentChunks(t[3 * i + 1], t[3 * i + 2], units));
-        for (uint32_t p = 1; p <= mf::kMaxPeriod; ++p) {
-            if (i >= p && counts[i - p] != counts[i]) {
-                alive &= ~(1u << p);
-            }
-        }
-        run += counts[i];
-    }
-    f[nseg] = run;
-    mf::TableHeader *header = reinterpret_cast<mf::TableHeader *>(words);
-    *header = mf::TableHeader{};
-    header->nchunk = run;
-    header->groupShift = mf::GroupShiftFor(run, groupCapacity);
-    if (run != 0) {
-        header->groupShift = mf::BuildGroupMap(f, nseg, words + at.group, groupCapacity);
-    }
-    if (alive != 0 && run != 0) {
-        const uint32_t period = static_cast<uint32_t>(__builtin_ctz(alive));
-        uint32_t sum = 0;
-        for (uint32_t q = 0; q < period; ++q) {
-            header->pattern.start[q] = sum;
-            sum += counts[q];
-        }
-        header->pattern.start[period] = sum;
-        if (sum != 0) {
-            header->pattern.period = period;
-            header->pattern.chunksPerPeriod = sum;
-        } else {
-            header->pattern = mf::ChunkPattern{};
-        }
-    }
-    mf::TablePlan &plan = *static_cast<mf::TablePlan *>(tablePlan);
-    plan = mf::TablePlan{};
-    plan.triples = t;
-    plan.first = f;
-    plan.group = words + at.group;
-    plan.header = header;
-    plan.nseg = nseg;
-    plan.units = units;
     ++g_launches;
+    const uint64_t *t = static_cast<const uint64_t *>(triples);
+    uint64_t parts = 1;
+    for (uint32_t i = 0; i < mf::kDirectSample && i < nseg; ++i) {
+        const uint64_t chunks = mf::SegmentChunks(t[3 * i + 1], t[3 * i + 2], units);
+        parts = chunks > parts ? (chunks < mf::kDirectMaxParts ? chunks : mf::kDirectMaxParts) : parts;
+    }
+    const uint32_t room = capacity < 5 ? capacity : 5;
+    for (uint64_t item = 0; item < nseg * parts; ++item) {
+        const uint64_t seg = item / parts;
+        const uint64_t part = item % parts;
+        const uint64_t src = t[3 * seg];
+        const uint64_t dst = t[3 * seg + 1];
+        const uint64_t len = t[3 * seg + 2];
+        const uint64_t chunks = mf::SegmentChunks(dst, len, units);
+        const uint64_t own = parts * mf::kDirectRounds;
+        for (uint64_t c = part; c < chunks && c < own; c += parts) {
+            RunChunk(src, dst, len, c, units);
+        }
+        if (part != 0 || chunks <= own) {
+            continue;
+        }
+        const uint64_t at = mf::SegmentGeometry(dst, len).head + own * units * mf::kUnitBytes;
+        const uint64_t each = mf::RestPieceBytesFor(len - at);
+        for (uint64_t from = at; from < len; from += each, ++list->count) {
+            if (list->count < room) {
+                list->piece[list->count] = mf::RestPiece{src + from, dst + from, len - from < each ? len - from : each};
+                continue;
+            }
+            for (uint64_t c = 0; c < mf::SegmentChunks(dst + from, len - from, units); ++c) {
+                RunChunk(src + from, dst + from, len - from, c, units);
+            }
+            list->count = room;
+            break;
+        }
+    }
+    ++g_launches;
+    for (uint32_t p = 0; p < list->count && p < room; ++p) {
+        const mf::RestPiece &r = list->piece[p];
+        for (uint64_t c = 0; c < mf::SegmentChunks(r.dst, r.len, units); ++c) {
+            RunChunk(r.src, r.dst, r.len, c, units);
+        }
+    }
+    list->count = 0;
+    if (mask != nullptr) {
+        *static_cast<uint64_t *>(mask) = maskValue;
+    }
     return 0;
 }
 
@@ -453,15 +443,13 @@ int mfk_xcopy_signal(void *word, uint32_t value, void *)
     return 0;
 }
 int mfk_xcopy_static_setup(void) { return 0; }
-int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, void *stream)
+int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *stream)
 {
-    static std::vector<uint32_t> scratch(mf::ScratchLayoutFor(MFK_STATIC_TABLE_SEGMENTS, MFK_STATIC_TABLE_SEGMENTS).words);
+    static std::vector<uint64_t> list(mf::RestListBytes(16) / 8, 0);
     if (nseg == 0 || nseg > MFK_STATIC_TABLE_SEGMENTS) {
         return -1;
     }
-    mf::TablePlan plan;
-    int err = mfk_xcopy_plan(triples, nseg, units, scratch.data(), MFK_STATIC_TABLE_SEGMENTS, &plan, stream);
-    return err != 0 ? err : mfk_xcopy_table(&plan, route, grid, nullptr, 0, stream, 0);
+    return mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, list.data(), 16, nullptr, 0, stream);
 }
 
 static uint32_t g_lastRectMates = 0;
