@@ -1017,6 +1017,48 @@ uint64_t BuildTableDirect(const uint64_t *src, const uint64_t *dst, const uint64
     return run;
 }
 
+// The pieces of a batch (xcopy_plan.h), empty segments dropped and neighbours that continue each other merged, straight into the
+// staging slot.  `out` has room for PieceBound() of them; returns their number.
+uint32_t BuildPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t units, Piece *out)
+{
+    const uint64_t most = static_cast<uint64_t>(units) * kUnitBytes;
+    const uint32_t shift = static_cast<uint32_t>(__builtin_ctzll(most));
+    Piece *p = out;
+    for (uint32_t i = 0; i < n;) {
+        const uint64_t s = src[i];
+        const uint64_t d = dst[i];
+        uint64_t l = len[i];
+        ++i;
+        if (l == 0) {
+            continue;
+        }
+        for (; i < n && (len[i] == 0 || (s + l == src[i] && d + l == dst[i])); ++i) {
+            l += len[i];
+        }
+        // pieces of equal length between multiples of kPieceAlign, counted from the one at or below the first byte
+        const uint64_t skip = d & (kPieceAlign - 1);
+        const uint64_t span = skip + l;
+        if (span <= most) {
+            *p++ = MakePiece(s, d, static_cast<uint32_t>(l));
+            continue;
+        }
+        const uint64_t parts = (span + most - 1) >> shift;
+        const uint64_t each = ((span + parts - 1) / parts + kPieceAlign - 1) & ~static_cast<uint64_t>(kPieceAlign - 1);
+        uint64_t from = 0;
+        for (uint64_t to = each - skip; from < l; to += each) {
+            const uint64_t end = to < l ? to : l;
+            *p++ = MakePiece(s + from, d + from, static_cast<uint32_t>(end - from));
+            from = end;
+        }
+    }
+    return static_cast<uint32_t>(p - out);
+}
+
+uint64_t PieceBound(uint64_t bytes, uint32_t n, uint32_t units)
+{
+    return n + (bytes + static_cast<uint64_t>(n) * (kPieceAlign - 1)) / (static_cast<uint64_t>(units) * kUnitBytes);
+}
+
 void ChooseCalibration(const float *batchMicros, const float *copyMicros, uint32_t defaultWindowMBps, uint32_t defaultAlignedMBps,
                        uint32_t defaultLongMBps, XcopyCalibration &out)
 {
@@ -1466,18 +1508,18 @@ uint32_t XcopyEngine::HoldFor(const InlinePlan &plan, uint32_t grid, int route, 
     return with > 0 ? static_cast<uint32_t>(with) : 0;
 }
 
-// Hold of a table launch.  Under a pattern (pinned) its waves fetch their descriptors across the host link and issue
-// their loads that much later than those of a launch whose descriptors are kernel arguments; without one they find them
-// through the group map in device memory, two dependent loads.
-uint32_t XcopyEngine::HoldForTable(uint32_t nchunk, uint32_t grid, uint32_t units, int route, bool unordered, bool pinned) const
+// Hold of a launch of pieces, as that of a table of `count` chunks whose waves fetch their descriptors across the host link and
+// issue their loads that much later than those of a launch whose descriptors are kernel arguments.  (The launcher takes off
+// what pieces wait less: PieceHoldNanos.)
+uint32_t XcopyEngine::HoldForPieces(uint32_t count, uint32_t units, bool unordered) const
 {
-    if (route != MFRT_ROUTE_HBM || unordered || tuning_.holdNanos == 0) {
+    if (unordered || tuning_.holdNanos == 0) {
         return 0;
     }
-    if ((nchunk > kHoldSharedMaxChunks || units == kDeepUnits) && g_leasesOut.load(std::memory_order_relaxed) > 1) {
+    if ((count > kHoldSharedMaxChunks || units == kDeepUnits) && g_leasesOut.load(std::memory_order_relaxed) > 1) {
         return 0;
     }
-    const uint32_t rule = HoldNanosFor(nchunk, grid, units, false);
+    const uint32_t rule = HoldNanosFor(count, count, units, false);
     if (rule == 0) {
         return 0;
     }
@@ -1487,15 +1529,7 @@ uint32_t XcopyEngine::HoldForTable(uint32_t nchunk, uint32_t grid, uint32_t unit
     if (tuning_.holdCalibratedOff) {
         return 0;
     }
-    // The 16 KiB form wants its wait another 800 ns longer than the link round trip explains (sixteen loads per lane take
-    // longer to leave than four): K and V blocks of 3 / 4 / 5 / 6 requests, 27 to 54 MB, with 1600 / 2000 / 2400 / 2800 ns on
-    // top of the rule: 13.3 / 12.7 / 13.0 / 13.4 us, 17.2 / 16.5 / 16.1 / 16.4, 20.3 / 19.8 / 19.1 / 19.3, 24.3 / 23.8 / 23.5 / 23.5;
-    // two requests on 4 KiB chunks 9.3 / 9.7 / 10.1 / 10.5 (and 9.3 with 1200).
-    // Ragged tables, whose descriptors were uploaded: 36 / 40 / 58 MB on 16 KiB chunks 18.4 / 20.0 / 26.2 us with 500 ns on top
-    // of the rule (19.0 / 20.5 / 27.0 with none, 18.7 / 20.4 / 26.0 with 1000) against 20.5 / 22.6 / 28.7 us not held; 12 / 13 /
-    // 20 / 19 MB on 4 KiB chunks 10.9 / 11.6 / 13.8 / 13.9 us with 800 ns against 11.3 / 12.3 / 14.8 / 14.7 (6 MB: 9.3 either way).
-    const int32_t extra = pinned ? tuning_.holdPinnedExtraNanos + (units == kDeepUnits ? kHoldPinnedDeepExtraNanos : 0)
-                                 : (units == kDeepUnits ? kHoldLookupDeepExtraNanos : kHoldLookupExtraNanos);
+    const int32_t extra = tuning_.holdPinnedExtraNanos + (units == kDeepUnits ? kHoldPinnedDeepExtraNanos : 0);
     const int64_t with = static_cast<int64_t>(rule) + extra + tuning_.holdDeltaNanos;
     return with > 0 ? static_cast<uint32_t>(with) : 0;
 }
@@ -1721,9 +1755,8 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         return BM_OK;
     }
 
-    // Table form: {triples, prefix} are built in a pinned slot; the general form moves them to HBM
-    // with a copy launch and searches them there.  The slot is sized for n segments; merging can only make the table shorter.
-    bool deepTable = false;
+    // Beyond the kernel arguments descriptors are built in a pinned slot, which is sized for n segments; merging can only make
+    // them fewer.
     {
         uint64_t total = 0;
         uint64_t longest = 0;
@@ -1738,9 +1771,9 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         // then takes the form with read and write windows: the few extra launches cost microseconds, the windows
         // gain 8 % (896 segments, 8.5 GB: 2.55 ms in seven launches against 2.78 ms in one).  Segments on cache lines
         // are worth it from 1 MiB each, 128 MiB a launch (1024 x 1 MiB 327 against 361 us, 1024 x 2 MiB 658 against
-        // 753 to 772 us, 512 x 3 MiB 458 against 588 us; 1024 x 512 KiB, 64 MiB a launch, the same either way).  The table form
-        // itself was measured under windows three times, with the prefix search it once had, with the division and
-        // group map it has now, and with full periods at rates from 6.0 to 7.1 TB/s, and is left without them: 262 144
+        // 753 to 772 us, 512 x 3 MiB 458 against 588 us; 1024 x 512 KiB, 64 MiB a launch, the same either way).  Tables
+        // themselves were measured under windows three times, with a search of the whole prefix, with the division and
+        // group map, and with full periods at rates from 6.0 to 7.1 TB/s, and are left without them: 262 144
         // pages of 32 KiB at random places lose 7 to 12 % (3.23 to 3.45 against 3.04 ms; the third time 2.93 to 3.38
         // against 2.89 to 3.06), 4096 pages take 58 to 60 instead of 46.5 to 49 us, 16 384 ragged segments lose 3 %, and
         // the 896 long segments in one windowed table launch are no faster than in seven launches of the kernel-argument form.
@@ -1761,16 +1794,20 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
             return BM_OK;
         }
         units = ChooseUnits(total, cu, route, tuning_);
+        if (route == MFRT_ROUTE_HBM) {
+            const int ret = SubmitPieces(src, dst, len, n, total, units, stream, mask, maskValue, unordered);
+            if (ret != kNotLaunched) {
+                return ret;
+            }
+        }
         if (route == MFRT_ROUTE_TO_HOST && tuning_.unitsOverride == 0) {
             // Four accesses per lane, whose loads from HBM are in flight together: with one the walk over a table's chunks is too
             // slow for the link (K and V blocks of four requests 638 us, 669 with one; 256 workgroups with one 639).
             units = kDeepUnits;
         }
-        deepTable = DeepHoldApplies(total, n, route, unordered);
         // Many short segments: a chunk size that holds the longest of them gives every segment exactly
-        // one chunk, which is the equal-count form below (no prefix, no search, no upload): 16 384
-        // segments of 2-14 KB take 62 us instead of 74 us.
-        if (tuning_.unitsOverride == 0 && longest != 0 && !deepTable) {
+        // one chunk, which is the equal-count form below (no prefix, no search).
+        if (tuning_.unitsOverride == 0 && longest != 0) {
             for (uint32_t u = units; u <= 4 * kXcopyThreads; u *= 2) {
                 if (longest <= static_cast<uint64_t>(u) * kUnitBytes - kUnitBytes) {
                     units = u;
@@ -1797,18 +1834,7 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
     uint32_t *first = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(slot->host) + tripleBytes);
     uint32_t count = 0;
     ChunkPattern pattern;
-    uint64_t nchunk = 0;
-    if (deepTable) {
-        nchunk = BuildTableDirect(src, dst, len, n, kDeepUnits, triples, first, count, &pattern);
-        if (HoldNanosFor(static_cast<uint32_t>(nchunk < kNoChunk ? nchunk : 0), static_cast<uint32_t>(nchunk), kDeepUnits, false) != 0) {
-            units = kDeepUnits;
-        } else {
-            deepTable = false;   // ragged enough to exceed the waves that hold: the usual chunks
-        }
-    }
-    if (!deepTable) {
-        nchunk = BuildTableDirect(src, dst, len, n, units, triples, first, count, &pattern);
-    }
+    const uint64_t nchunk = BuildTableDirect(src, dst, len, n, units, triples, first, count, &pattern);
     if (nchunk >= kNoChunk) {
         MF_FAIL(BM_INVALID_PARAM, "batch too large for one launch: " << nchunk << " chunks");
     }
@@ -1828,20 +1854,14 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
     int err = 0;
     // Chunk counts that repeat (pages of one size, K and V blocks in turn): a workgroup finds its descriptor by
     // a division and a few comparisons, so the only thing it needs from the table is that one descriptor, which it
-    // can read straight out of the pinned slot.  No upload launch, nothing serial in front of the copy (a 4096-page
-    // gather on an idle stream: 50 us instead of 55); the 64 bytes per workgroup that cross the host link stay
-    // below 2 % of the payload rate.  (Uploading the table by a launch of its own that carries no barrier, so that
-    // it runs beside the caller's earlier copies, was measured for these batches too: the extra launch costs the
-    // stream 2 us whether it overlaps or not, more than the fetch from HBM saves: 36 MB of K and V blocks 20.5
-    // against 18.4 us per call.)
+    // can read straight out of the pinned slot.  No upload launch, nothing serial in front of the copy.
     // Over the link a few workgroups walk all the chunks, and a descriptor fetch across the link it saturates would be in every
     // one of their steps: those tables are uploaded (K and V blocks of four requests to the host: 638 us, 681 from the slot and
     // on 4 KiB chunks).
     if (pattern.period != 0 && route == MFRT_ROUTE_HBM) {
-        const uint32_t hold = HoldForTable(static_cast<uint32_t>(nchunk), grid, units, route, unordered, true);
         table.triples = triples;
         table.pattern = pattern;
-        err = mfk_xcopy_table(&table, route, grid, mask, maskValue, stream, hold);
+        err = mfk_xcopy_table(&table, route, grid, mask, maskValue, stream);
         g_launches.fetch_add(1, std::memory_order_relaxed);
     } else {
         // Ragged segments: prefix and group map go to HBM with the triples (with them in host memory every
@@ -1877,8 +1897,7 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         table.triples = reinterpret_cast<const uint64_t *>(devBase);
         table.first = reinterpret_cast<const uint32_t *>(devBase + tripleBytes);
         table.group = reinterpret_cast<const uint32_t *>(devBase + tripleBytes + prefixBytes);
-        err = mfk_xcopy_table(&table, route, grid, mask, maskValue, stream,
-                              HoldForTable(static_cast<uint32_t>(nchunk), grid, units, route, unordered, false));
+        err = mfk_xcopy_table(&table, route, grid, mask, maskValue, stream);
         g_launches.fetch_add(2, std::memory_order_relaxed);
     }
     if (err != 0) {
@@ -1887,6 +1906,53 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         MF_FAIL(BM_ERROR, "xcopy table launch failed: " << mfrt_error_string(err));
     }
     NotePending(stream, queuedBytes);
+    return MarkQueued(lease, slot, stream, false);
+}
+
+// A batch between HBM addresses in one launch of pieces; kNotLaunched where their list would outgrow the batch.
+int XcopyEngine::SubmitPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t total, uint32_t units,
+                              void *stream, void *mask, uint32_t maskValue, bool unordered)
+{
+    const uint64_t mean = total / n;
+    if (tuning_.unitsOverride != 0) {
+        units = units <= kXcopyThreads ? kXcopyThreads : units <= 2 * kXcopyThreads ? 2 * kXcopyThreads : kDeepUnits;
+    } else if (DeepHoldApplies(total, n, MFRT_ROUTE_HBM, unordered)) {
+        units = kDeepUnits;
+        // ragged enough to exceed the waves that hold: not held
+    } else if (total > kDeepMinBytes) {
+        // Up to 24 MiB waves of 4 KiB are resident together and hold their stores.  Beyond, what the usual segment fills: each
+        // workgroup twice the size halves the descriptors the host writes and the link carries, but lanes without a unit cost
+        // (16 080 pages of 8 KiB 45.2 / 46.1 / 47.0 us with one, two and four waves; 4096 of 32 KiB 45.8 / 46.8 / 46.4).
+        units = mean <= 6144 ? kXcopyThreads : mean <= 12288 ? 2 * kXcopyThreads : kDeepUnits;
+    } else {
+        units = kXcopyThreads;
+    }
+    // A few segments of gigabytes would make a list of millions of pieces, megabytes that take the host longer to write than a chunk
+    // prefix takes the GPU to read.
+    const uint64_t bound = PieceBound(total, n, units);
+    if (bound > std::max<uint64_t>(kPieceListMin, 2ull * n) || bound > kPieceMaxCount) {
+        return kNotLaunched;
+    }
+    ThreadLease &lease = t_ctx.Lease();
+    StagingSlot *slot = nullptr;
+    const int ret = AcquireSlot(lease, bound * sizeof(Piece), stream, slot);
+    if (ret != BM_OK) {
+        return ret;
+    }
+    Piece *pieces = static_cast<Piece *>(slot->host);
+    const uint32_t count = BuildPieces(src, dst, len, n, units, pieces);
+    if (count == 0) {   // nothing but empty segments
+        InlinePlan empty;
+        SegList none;
+        (void)BuildInlinePlan(none, kXcopyThreads, empty);
+        return mfk_xcopy_inline(&empty, MFRT_ROUTE_HBM, 1, mask, maskValue, stream, 0, 0) == 0 ? BM_OK : BM_ERROR;
+    }
+    const int err = mfk_xcopy_pieces(pieces, count, total, units, mask, maskValue, stream, HoldForPieces(count, units, unordered));
+    if (err != 0) {
+        MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(err));
+    }
+    g_launches.fetch_add(1, std::memory_order_relaxed);
+    NotePending(stream, total);
     return MarkQueued(lease, slot, stream, false);
 }
 

@@ -41,6 +41,13 @@ struct SegList {
 void NormalizeSegments(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t pieceLimit,
                        SegList &out);
 
+// On top of HoldNanosFor's rule where the waves of a launch have to look their descriptors up outside the kernel arguments, a
+// round trip across the host link before their loads, and the same on 16 KiB chunks: sixteen loads per lane take longer to leave.
+constexpr int32_t kHoldLookupExtraNanos = 1600;
+constexpr int32_t kHoldLookupDeepExtraNanos = 2000;
+constexpr int32_t kHoldPinnedDeepExtraNanos = kHoldLookupDeepExtraNanos - kHoldLookupExtraNanos;
+constexpr uint64_t kPieceListMin = 1ull << 18;     // pieces that any batch may be cut into, 4 MiB of descriptors
+
 struct XcopyTuning {
     uint32_t unitsOverride = 0;  // 16-byte units per chunk, 0 = choose from batch size
     uint32_t wgPerCu = 0;        // HBM routes: grid cap in workgroups per CU, 0 = one workgroup per chunk
@@ -52,7 +59,7 @@ struct XcopyTuning {
     uint32_t unorderedStreams = 0;   // unordered batches are launched by this many submit threads of the library's, a stream each (0, 1: by the caller on its own stream)
     bool holdOnSideStreams = false;  // launches of the submit threads overlap on purpose: their stores are not held
     bool deepHold = true;        // batches of 24 to 64 MiB hold the stores of 16 KiB per wave
-    int32_t holdPinnedExtraNanos = 1600;   // added to the rule for table launches, whose descriptors come from pinned host memory: a link round trip before the loads
+    int32_t holdPinnedExtraNanos = kHoldLookupExtraNanos;   // added to the rule for launches of more than kInlineSegs segments
     bool stageUnordered = true;  // the upload of a ragged table's descriptors is launched without a barrier
     uint32_t deviceTableWgPerCu = 0;   // grid of a device-resident table in workgroups per CU, 0 = four per segment between 16 and 1024 per CU
     uint32_t windowMBps = 6800000;   // HBM copies of kWindowRectMinBytes and more alternate between read and write windows cut for this rate; 0 = never
@@ -72,9 +79,6 @@ constexpr uint64_t kWindowMinBytes = 128ull << 20;
 constexpr uint64_t kWindowRectMinBytes = 512ull << 20;
 constexpr uint64_t kWindowPieceBytes = 512ull << 20;          // launches into which long segments are cut
 constexpr uint64_t kWindowLongSegmentBytes = 64ull << 20;     // launches whose segments average this much go out in pieces of kWindowPieceBytes and more
-constexpr int32_t kHoldLookupExtraNanos = 800;                // on top of the rule where a table launch finds its descriptors through the group map
-constexpr int32_t kHoldLookupDeepExtraNanos = 500;            // the same on 16 KiB chunks
-constexpr int32_t kHoldPinnedDeepExtraNanos = 800;            // on top of holdPinnedExtraNanos where a table launch works on 16 KiB chunks
 constexpr uint64_t kWindowAlignBytes = 128;                   // a cache line: segments that start on one are read and written in whole lines by every wave
 constexpr uint64_t kWindowSliceMinSegmentBytes = 4ull << 20;   // tables of segments this long on average are cut into windowed launches
 constexpr uint64_t kWindowSliceMinAlignedSegmentBytes = 1ull << 20;   // the same for segments on cache lines: kInlineSegs of them reach kWindowMinBytes
@@ -201,13 +205,15 @@ private:
     XcopyEngine() = default;
 
     uint32_t HoldFor(const InlinePlan &plan, uint32_t grid, int route, bool unordered) const;
-    uint32_t HoldForTable(uint32_t nchunk, uint32_t grid, uint32_t units, int route, bool unordered, bool pinned) const;
+    uint32_t HoldForPieces(uint32_t count, uint32_t units, bool unordered) const;
     // Whether a batch of `bytes` in n segments is planned in chunks of kDeepUnits units, to hold the stores of 16 KiB per wave.
     bool DeepHoldApplies(uint64_t bytes, uint32_t n, int route, bool unordered) const;
     // A launch that stores the thread's word itself, where that is the faster form: kNotLaunched where it is not.
     static constexpr int kNotLaunched = 1;
     int LaunchDone(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t bytes, int route, void *stream,
                    uint32_t &ticket);
+    int SubmitPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t total, uint32_t units,
+                     void *stream, void *mask, uint32_t maskValue, bool unordered);
     int SubmitInPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t total, int route,
                        void *stream, void *mask, uint32_t maskValue);
     int SubmitOne(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, int route, void *stream,

@@ -61,6 +61,11 @@ __device__ __forceinline__ u32x4 LoadUnit(uint64_t addr)
     return *p;
 }
 
+__device__ __forceinline__ u32x4 LoadAligned(uint64_t addr)
+{
+    return __builtin_nontemporal_load(reinterpret_cast<const MF_GLOBAL u32x4 *>(addr));
+}
+
 // kStoreStream: nontemporal hint, the line may still linger dirty in L2 until the end of the kernel.
 // kStoreThrough: nontemporal and written through at system scope, so that the write-back of the
 // destination overlaps the copy instead of trailing it.
@@ -510,11 +515,9 @@ __device__ __forceinline__ uint64_t Uniform(uint64_t v)
     return (static_cast<uint64_t>(Uniform(static_cast<uint32_t>(v >> 32))) << 32) | Uniform(static_cast<uint32_t>(v));
 }
 
-// kHold: as for the inline kernel, for launches of one chunk per workgroup (the host knows the chunk count).
-template <bool kNtLoad, int kStore, int kHold = kHoldNone>
-__global__ __launch_bounds__(kXcopyThreads) void XcopyTableKernel(const TablePlan plan, uint32_t holdTicks)
+template <bool kNtLoad, int kStore>
+__global__ __launch_bounds__(kXcopyThreads) void XcopyTableKernel(const TablePlan plan)
 {
-    const uint64_t t0 = kHold != kHoldNone ? wall_clock64() : 0;
     const uint32_t nchunk = plan.nchunk;
     const uint32_t shift = plan.groupShift;
     const ChunkPattern pattern = plan.pattern;
@@ -545,7 +548,7 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyTableKernel(const TablePla
                 ndst = t[1];
                 nlen = t[2];
             }
-            CopyChunkHeld<kNtLoad, kStore, kHold>(src, dst, len, k, units, t0, holdTicks);
+            CopyChunk<kNtLoad, kStore>(src, dst, len, k, units);
             if (!more) {
                 return;
             }
@@ -568,11 +571,135 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyTableKernel(const TablePla
         if (more) {
             bounds = plan.group[(next >> shift) + (lane & 1u)];
         }
-        CopyChunkHeld<kNtLoad, kStore, kHold>(r.src, r.dst, r.len, r.k, units, t0, holdTicks);
+        CopyChunk<kNtLoad, kStore>(r.src, r.dst, r.len, r.k, units);
         if (!more) {
             return;
         }
         c = next;
+    }
+}
+
+// The unit of the source that the next lane holds; lane 63 gets `wrap`.
+__device__ __forceinline__ uint32_t NextLane(uint32_t v, uint32_t wrap)
+{
+    const uint32_t next = __builtin_amdgcn_update_dpp(0u, v, 0x130, 0xf, 0xf, true);   // wave_shl:1
+    return (threadIdx.x & 63u) == 63u ? wrap : next;
+}
+
+// Sixteen bytes from byte 4 * kWords + bytes of the pair (a, b) on.
+template <uint32_t kWords>
+__device__ __forceinline__ u32x4 Straddle(u32x4 a, u32x4 b, uint32_t bytes)
+{
+    const uint32_t w[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    u32x4 r;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        r[i] = __builtin_amdgcn_alignbyte(w[i + kWords + 1], w[i + kWords], bytes);
+    }
+    return r;
+}
+
+// Pieces of up to kLanes * kUnits units (xcopy_plan.h), one per workgroup.  HBM is the bound; what the form saves is everything in
+// front of the first load: descriptors are fetched in one step from the host's memory, where a table with a chunk prefix and
+// an owner map had to be moved to HBM by a launch of its own first, and no wave looks anything up.
+// A source that differs from its destination modulo 16 is read in whole aligned units, each lane taking what it lacks from the
+// next lane's: loads that straddle units cost twice the cache accesses (4.9 MB of ragged segments 4.7 / 3.9 us, 69 MB 30.4 / 29.2).
+// Such a load reads up to 15 bytes beside the piece, of units that hold some of its bytes.
+// Shapes, measured on the kernel alone: single waves of 4 KiB as long as those are resident together, for their held stores;
+// single waves of 16 KiB, held, beyond; and without hold four waves of 16 KiB, or as many as the usual segment fills: 4096 pages of 32 KiB
+// gathered 45.8 / 49.4 / 46.4 us with 4 KiB waves / 16 KiB waves / four waves, scattered 49.9 / 51.4 / 49.2, and a quarter of the
+// descriptors for the host to write.
+template <uint32_t kLanes, uint32_t kUnits, bool kHold>
+__global__ __launch_bounds__(kLanes) void XcopyPieceKernel(const Piece *__restrict__ pieces, uint32_t count, uint32_t holdTicks)
+{
+    const uint64_t t0 = kHold ? wall_clock64() : 0;
+    const uint32_t at = PieceOf(blockIdx.x);
+    if (at >= count) {
+        return;
+    }
+    const Piece p = pieces[at];
+    const uint64_t srcWord = Uniform(p.src);
+    const uint64_t dstWord = Uniform(p.dst);
+    const uint64_t src = srcWord & kPieceAddress;
+    const uint64_t dst = dstWord & kPieceAddress;
+    const SegGeom g = SegmentGeometry(dst, PieceLength(srcWord, dstWord));
+    const uint32_t body = static_cast<uint32_t>(g.body);
+    const uint64_t s = src + g.head;
+    const uint64_t d = dst + g.head;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t apart = static_cast<uint32_t>(s) & (kUnitBytes - 1);
+    u32x4 v[kUnits];
+    if (apart == 0 && body == kLanes * kUnits) {
+#pragma unroll
+        for (uint32_t j = 0; j < kUnits; ++j) {
+            v[j] = LoadAligned(s + (j * kLanes + tid) * kUnitBytes);
+        }
+        if (kHold) {
+            HoldStores(t0, holdTicks);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kUnits; ++j) {
+            StoreUnit<kStoreStream>(d + (j * kLanes + tid) * kUnitBytes, v[j]);
+        }
+    } else if (apart == 0) {
+#pragma unroll
+        for (uint32_t j = 0; j < kUnits; ++j) {
+            if (j * kLanes + tid < body) {
+                v[j] = LoadAligned(s + (j * kLanes + tid) * kUnitBytes);
+            }
+        }
+        if (kHold) {
+            HoldStores(t0, holdTicks);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kUnits; ++j) {
+            if (j * kLanes + tid < body) {
+                StoreUnit<kStoreStream>(d + (j * kLanes + tid) * kUnitBytes, v[j]);
+            }
+        }
+    } else if (body != 0) {
+        // units 0 ... body of the aligned source; a wave has consecutive ones, so that the next unit is the next lane's
+        const uint64_t a = s - apart;
+        const uint32_t u0 = (tid >> 6) * kUnits * 64;
+        const uint32_t u = u0 + (tid & 63u);
+#pragma unroll
+        for (uint32_t j = 0; j < kUnits; ++j) {
+            if (u + j * 64 <= body) {
+                v[j] = LoadAligned(a + (u + j * 64) * kUnitBytes);
+            }
+        }
+        const uint32_t behind = u0 + kUnits * 64 < body ? u0 + kUnits * 64 : body;      // what lane 63 of the last unit lacks
+        const u32x4 last = LoadAligned(a + behind * kUnitBytes);
+        if (kHold) {
+            HoldStores(t0, holdTicks);
+        }
+        auto store = [&](auto words) {
+#pragma unroll
+            for (uint32_t j = 0; j < kUnits; ++j) {
+                u32x4 next;
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) {
+                    next[i] = NextLane(v[j][i], Uniform(j + 1 < kUnits ? v[j + 1 < kUnits ? j + 1 : 0][i] : last[i]));
+                }
+                const u32x4 r = Straddle<decltype(words)::value>(v[j], next, apart & 3u);
+                if (u + j * 64 < body) {
+                    StoreUnit<kStoreStream>(d + (u + j * 64) * kUnitBytes, r);
+                }
+            }
+        };
+        switch (apart >> 2) {
+            case 0: store(std::integral_constant<uint32_t, 0>()); break;
+            case 1: store(std::integral_constant<uint32_t, 1>()); break;
+            case 2: store(std::integral_constant<uint32_t, 2>()); break;
+            default: store(std::integral_constant<uint32_t, 3>()); break;
+        }
+    }
+    if (tid < g.head) {
+        CopyByte<kStoreStream>(src + tid, dst + tid);
+    }
+    if (tid < g.tail) {
+        const uint64_t off = g.head + g.body * kUnitBytes + tid;
+        CopyByte<kStoreStream>(src + off, dst + off);
     }
 }
 
@@ -815,22 +942,11 @@ int LaunchWindowed(const InlinePlan &plan, uint32_t grid, uint32_t windowMBps, h
     return static_cast<int>(hipGetLastError());
 }
 
-template <bool kNtLoad, int kStore>
-int LaunchTable(const TablePlan &plan, uint32_t grid, uint32_t lanes, hipStream_t stream, uint32_t holdNanos)
+template <uint32_t kLanes, uint32_t kUnits, bool kHold>
+void LaunchPieces(const Piece *pieces, uint32_t count, uint32_t ticks, hipStream_t stream)
 {
-    const bool deep = plan.units == kWindowUnits && holdNanos != 0;
-    if (deep) {
-        lanes = 64;
-    }
-    const uint32_t ticks = grid == plan.nchunk && lanes == 64 ? HoldTicks(holdNanos) : 0;
-    if (ticks != 0 && deep) {
-        hipLaunchKernelGGL((XcopyTableKernel<kNtLoad, kStore, kHoldDeep>), dim3(grid), dim3(lanes), 0, stream, plan, ticks);
-    } else if (ticks != 0) {
-        hipLaunchKernelGGL((XcopyTableKernel<kNtLoad, kStore, kHoldShallow>), dim3(grid), dim3(lanes), 0, stream, plan, ticks);
-    } else {
-        hipLaunchKernelGGL((XcopyTableKernel<kNtLoad, kStore>), dim3(grid), dim3(lanes), 0, stream, plan, 0u);
-    }
-    return static_cast<int>(hipGetLastError());
+    const uint32_t grid = (count + kPieceGroup - 1) / kPieceGroup * kPieceGroup;
+    hipLaunchKernelGGL((XcopyPieceKernel<kLanes, kUnits, kHold>), dim3(grid), dim3(kLanes), 0, stream, pieces, count, ticks);
 }
 
 template <bool kNtLoad, int kStore>
@@ -946,8 +1062,34 @@ extern "C" int mfk_xcopy_signal(void *word, uint32_t value, void *stream)
     return mf::Signal(word, value, static_cast<hipStream_t>(stream));
 }
 
-extern "C" int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, void *mask, uint32_t maskValue, void *stream,
-                               uint32_t holdNanos)
+// pieces: `count` mf::Piece of together `bytes` bytes, none longer than `units` units and the bytes beside them; holdNanos: what a
+// table of as many chunks would wait.
+extern "C" int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, void *mask, uint32_t maskValue,
+                                void *stream, uint32_t holdNanos)
+{
+    using namespace mf;
+    if (pieces == nullptr || count == 0 || count > kPieceMaxCount || (units != 256 && units != 512 && units != 1024)) {
+        return -1;
+    }
+    const Piece *p = static_cast<const Piece *>(pieces);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const uint32_t ticks = units != 512 ? HoldTicks(PieceHoldNanos(holdNanos, count, bytes, units)) : 0;
+    if (units == 256 && ticks != 0) {
+        LaunchPieces<64, 4, true>(p, count, ticks, s);
+    } else if (units == 256) {
+        LaunchPieces<64, 4, false>(p, count, 0, s);
+    } else if (units == 512) {
+        LaunchPieces<128, 4, false>(p, count, 0, s);
+    } else if (ticks != 0) {
+        LaunchPieces<64, 16, true>(p, count, ticks, s);
+    } else {
+        LaunchPieces<256, 4, false>(p, count, 0, s);
+    }
+    const int err = static_cast<int>(hipGetLastError());
+    return err != 0 ? err : Signal(mask, maskValue, s);
+}
+
+extern "C" int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, void *mask, uint32_t maskValue, void *stream)
 {
     const mf::TablePlan &plan = *static_cast<const mf::TablePlan *>(tablePlan);
     const mf::ChunkPattern &pat = plan.pattern;
@@ -964,8 +1106,9 @@ extern "C" int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, 
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int err = mf::WithPolicy(mf::PolicyOf(route), [&](auto ntLoad, auto store) {
-        return mf::LaunchTable<decltype(ntLoad)::value, decltype(store)::value>(plan, grid, mf::LanesFor(plan.units, route), s,
-                                                                                route == MFRT_ROUTE_HBM ? holdNanos : 0u);
+        hipLaunchKernelGGL((mf::XcopyTableKernel<decltype(ntLoad)::value, decltype(store)::value>), dim3(grid),
+                           dim3(mf::LanesFor(plan.units, route)), 0, s, plan);
+        return static_cast<int>(hipGetLastError());
     });
     return err != 0 ? err : mf::Signal(mask, maskValue, s);
 }
@@ -1009,14 +1152,17 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
             constexpr int kSt = decltype(store)::value;
             hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, empty, 0u);
             hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 0u);
-            hipLaunchKernelGGL((XcopyTableKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, none, 0u);
+            hipLaunchKernelGGL((XcopyTableKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, none);
             if (route == MFRT_ROUTE_HBM) {
                 hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, empty, 1u);
                 hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, empty, 1u);
                 hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 1u);
                 hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kWindowUnits, 1u);
-                hipLaunchKernelGGL((XcopyTableKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, none, 1u);
-                hipLaunchKernelGGL((XcopyTableKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, none, 1u);
+                hipLaunchKernelGGL((XcopyPieceKernel<64, 4, false>), dim3(1), dim3(64), 0, s, nullptr, 0u, 0u);
+                hipLaunchKernelGGL((XcopyPieceKernel<64, 4, true>), dim3(1), dim3(64), 0, s, nullptr, 0u, 0u);
+                hipLaunchKernelGGL((XcopyPieceKernel<64, 16, true>), dim3(1), dim3(64), 0, s, nullptr, 0u, 0u);
+                hipLaunchKernelGGL((XcopyPieceKernel<128, 4, false>), dim3(1), dim3(128), 0, s, nullptr, 0u, 0u);
+                hipLaunchKernelGGL((XcopyPieceKernel<256, 4, false>), dim3(1), dim3(256), 0, s, nullptr, 0u, 0u);
                 hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
             }
             return 0;

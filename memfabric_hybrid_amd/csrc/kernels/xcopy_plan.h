@@ -123,6 +123,20 @@ inline uint32_t HoldNanosFor(uint32_t nchunk, uint32_t grid, uint32_t units, boo
     return 640 + kHoldKneeChunks * 6 / 10 + (nchunk - kHoldKneeChunks) * 33 / 100;
 }
 
+// What a launch of `count` pieces waits of the time a table of as many chunks would.  Its descriptors arrive eight to a line, and
+// kPieceLeadNanos sooner than three words per wave did; and ragged pieces are not full, so that the reads are over sooner: by
+// the rate of the rule above for the bytes that are not there.  Best waits beyond HoldNanosFor(count): K and V blocks of 10 / 18 /
+// 24 MB +400 / 200 / 400 ns, 27 / 36 / 45 / 54 / 63 MB on 16 KiB +400 / 800 / 800 / 1200 / 1000; ragged segments of 14 / 21 MB 0, 31 / 41 /
+// 52 MB -800 / -800 / -1200, where the bytes that are not there make 1000 / 1300 / 1700.
+constexpr uint32_t kPieceLeadNanos = 1400;
+inline uint32_t PieceHoldNanos(uint32_t holdNanos, uint32_t count, uint64_t bytes, uint32_t units)
+{
+    const uint64_t full = static_cast<uint64_t>(count) * units * kUnitBytes;
+    const uint64_t missing = full > bytes ? (full - bytes) / kUnitBytes : 0;                 // units
+    const uint64_t less = kPieceLeadNanos + missing * (units == kDeepUnits ? 215 : 180) / (100ull * kDeepUnits);
+    return holdNanos > less ? static_cast<uint32_t>(holdNanos - less) : 0;
+}
+
 // The start of a windowed launch's first period travels between its waves as the low kEpochClockBits bits of a
 // clock value (2^40 ticks of 10 ns: three hours) under a sequence number; NearClock restores the full value: the
 // one with those low bits that is nearest to `now`.
@@ -229,6 +243,36 @@ inline uint32_t BuildGroupMap(const uint32_t *first, uint32_t nseg, uint32_t *gr
     }
     group[ngroups] = last;
     return shift;
+}
+
+// A batch of more than kInlineSegs segments between HBM addresses, cut up by the host: one piece, one workgroup, one step.
+// A piece is 16 bytes in pinned host memory, addresses of 56 bits and a length of 16 in the bytes above them.  Inside a segment
+// pieces end where the destination reaches a multiple of kPieceAlign, so that no two workgroups write one cache line; all but
+// the last are of one length.
+constexpr uint32_t kPieceAlign = 128;
+constexpr uint32_t kPieceGroup = 64;
+constexpr uint32_t kPieceMaxCount = 1u << 23;      // below 2^32 lanes in a launch
+struct Piece {
+    uint64_t src;
+    uint64_t dst;
+};
+static_assert(sizeof(Piece) == 16, "eight pieces make a line");
+constexpr uint64_t kPieceAddress = (1ull << 56) - 1;
+MF_HD inline Piece MakePiece(uint64_t src, uint64_t dst, uint32_t len)
+{
+    return Piece{(src & kPieceAddress) | static_cast<uint64_t>(len & 0xFFu) << 56, (dst & kPieceAddress) | static_cast<uint64_t>(len >> 8) << 56};
+}
+MF_HD inline uint32_t PieceLength(uint64_t src, uint64_t dst)
+{
+    return static_cast<uint32_t>(src >> 56) | static_cast<uint32_t>(dst >> 56) << 8;
+}
+// Which piece a workgroup copies.  Consecutive workgroups go to the eight XCDs in turn, and an XCD fetches descriptors over the
+// host link by lines of eight: the eight of a line go to one XCD, which is then the only one to fetch it (4096 pages of 32 KiB in
+// pieces of 4 KiB: 45.8 us, 101 with the pieces dealt out in their order), and 64 workgroups still copy 64 consecutive pieces
+// (with an eighth of the whole list for each XCD: 51.6).
+MF_HD inline uint32_t PieceOf(uint32_t workgroup)
+{
+    return (workgroup & ~(kPieceGroup - 1)) | (workgroup & 7u) << 3 | (workgroup >> 3 & 7u);
 }
 
 // A table that only the GPU can read, copied without a plan.  Its launch takes `parts` items per segment, part j of a segment

@@ -92,10 +92,12 @@ uint32_t mfk_xcopy_window_units(void);
 uint32_t mfk_xcopy_window_waves(void);
 int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream);
 /* tablePlan: a mf::TablePlan (kernels/xcopy_plan.h).  Under a pattern its triples may live in pinned host
- * memory and neither prefix nor group map is read.
- * holdNanos: as for mfk_xcopy_inline, for a launch of one chunk per workgroup between HBM addresses. */
-int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, void *mask, uint32_t maskValue, void *stream,
-                    uint32_t holdNanos);
+ * memory and neither prefix nor group map is read. */
+int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, void *mask, uint32_t maskValue, void *stream);
+/* HBM to HBM: `count` mf::Piece (kernels/xcopy_plan.h) in pinned host memory, of together `bytes` bytes and up to `units` (256, 512
+ * or 1024) units each.  holdNanos: as for mfk_xcopy_inline; it is what a table of as many chunks would wait. */
+int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, void *mask, uint32_t maskValue, void *stream,
+                     uint32_t holdNanos);
 /* Launches every copy kernel once on empty plans (a kernel's first launch is not capturable into a HIP graph). */
 int mfk_xcopy_prelaunch(void *stream);
 /* Times the calibration workloads on `stream` with HIP events, in 1 GiB of device memory it allocates and frees:

@@ -315,9 +315,8 @@ int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, 
 
 // As the kernel: the owner of a chunk by division under a pattern, else from the two group-map entries around it and the prefix between
 // them.  A map whose entries do not bracket the owner fails the launch.
-int mfk_xcopy_table(const void *tablePlan, int, uint32_t grid, void *mask, uint32_t maskValue, void *, uint32_t holdNanos)
+int mfk_xcopy_table(const void *tablePlan, int, uint32_t grid, void *mask, uint32_t maskValue, void *)
 {
-    g_lastTableHold = holdNanos;
     const mf::TablePlan &plan = *static_cast<const mf::TablePlan *>(tablePlan);
     const uint64_t *t = plan.triples;
     const uint32_t *f = plan.first;
@@ -364,6 +363,48 @@ int mfk_xcopy_table(const void *tablePlan, int, uint32_t grid, void *mask, uint3
             ++s;
         }
         RunChunk(t[3 * s], t[3 * s + 1], t[3 * s + 2], c - f[s], plan.units);
+    }
+    if (mask != nullptr) {
+        *static_cast<uint64_t *>(mask) = maskValue;
+    }
+    return 0;
+}
+
+// The pieces in the order of the kernel's workgroups.  One that is longer than its workgroup or reaches past the end of the list
+// fails the launch.
+int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, void *mask, uint32_t maskValue, void *,
+                     uint32_t holdNanos)
+{
+    g_lastTableHold = holdNanos;
+    if (pieces == nullptr || count == 0 || (units != 256 && units != 512 && units != 1024)) {
+        return -1;
+    }
+    if (g_failLaunches > 0) {
+        --g_failLaunches;
+        return 719;
+    }
+    ++g_launches;
+    const mf::Piece *p = static_cast<const mf::Piece *>(pieces);
+    TrackTable(p, sizeof(mf::Piece) * count);
+    uint64_t moved = 0;
+    for (uint32_t w = 0; w < (count + 63) / 64 * 64; ++w) {
+        const uint32_t at = mf::PieceOf(w);
+        if (at >= count) {
+            continue;
+        }
+        const uint64_t src = p[at].src & mf::kPieceAddress;
+        const uint64_t dst = p[at].dst & mf::kPieceAddress;
+        const uint32_t len = mf::PieceLength(p[at].src, p[at].dst);
+        if (len == 0 || mf::SegmentGeometry(dst, len).body > units) {
+            return 720;
+        }
+        moved += len;
+        if (!g_skipCopies) {
+            RunChunk(src, dst, len, 0, units);
+        }
+    }
+    if (moved != bytes) {
+        return 721;
     }
     if (mask != nullptr) {
         *static_cast<uint64_t *>(mask) = maskValue;

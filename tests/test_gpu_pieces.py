@@ -1,0 +1,64 @@
+"""Batches of more than 128 segments between HBM addresses: every way a source and a destination can differ modulo 16, lengths at
+the edges of the pieces they are cut into, and sizes that take each of the launch's shapes, with stores held and not."""
+import numpy as np
+import pytest
+
+from memfabric_hybrid_amd import native
+from tests import gpu_util
+from tests.test_gpu_xcopy import _random_bytes
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [1, 15, 16, 17, 31, 33, 4079, 4080, 4096, 4097, 4111, 8192, 8193, 16383, 16384, 16385, 16399, 0, 0, 65537]
+
+
+@pytest.fixture(scope="module")
+def gpu(lib):
+    assert lib.hybm_init(0, 0) == 0, native.last_error()
+    yield lib
+    lib.hybm_uninit()
+
+
+def _lengths(kind, rng):
+    if kind == "every shift":                                    # 256 pairs of source and destination bytes, one wave each
+        return np.concatenate([rng.integers(1, 4000, 256), np.tile(EDGES, 16)])
+    if kind == "held 4 KiB":                                     # 6 MB and more: stores held
+        return np.concatenate([rng.integers(1, 70000, 200), EDGES])
+    if kind == "held 16 KiB":                                    # 24 to 64 MiB of long segments
+        return np.concatenate([rng.integers(1, 200000, 400), EDGES])
+    if kind == "one wave":                                       # beyond 24 MiB the usual segment decides
+        return np.concatenate([rng.integers(1, 9000, 7000), EDGES])
+    if kind == "two waves":
+        return np.concatenate([rng.integers(1, 20000, 3000), EDGES])
+    return np.concatenate([rng.integers(1, 90000, 2000), EDGES])   # "four waves"
+
+
+@pytest.mark.parametrize("kind", ["every shift", "held 4 KiB", "held 16 KiB", "one wave", "two waves", "four waves"])
+@pytest.mark.parametrize("odd", [True, False])
+def test_batch_in_pieces(gpu, oracle, kind, odd):
+    rng = np.random.default_rng(len(kind) + odd)
+    lens = _lengths(kind, rng).astype(np.uint64)
+    n = len(lens)
+    steps = (lens + np.uint64(159)) // np.uint64(128) * np.uint64(128)
+    at = np.concatenate(([0], np.cumsum(steps)[:-1])).astype(np.uint64)
+    size = int(steps.sum()) + 128
+    pairs = np.arange(n, dtype=np.uint64)
+    src = at + (pairs % np.uint64(16) if odd else np.uint64(0))
+    dst = at + (pairs // np.uint64(16) % np.uint64(16) if odd else np.uint64(0))
+    order = rng.permutation(n)
+    src, dst, lens = src[order], dst[order], lens[order]
+    source = _random_bytes(oracle, size, 3)
+    before = _random_bytes(oracle, size, 4)
+    a, b = gpu_util.DeviceBuffer(gpu, size), gpu_util.DeviceBuffer(gpu, size)
+    try:
+        a.upload(source)
+        b.upload(before)
+        launches = gpu.mf_xcopy_launch_count()
+        gpu_util.xcopy(gpu, a.ptr + src, b.ptr + dst, lens, native.ROUTE_HBM)
+        assert gpu.mf_xcopy_launch_count() - launches == 1
+        got = b.download()
+    finally:
+        a.free()
+        b.free()
+    gpu_util.oracle_batch(oracle, source, before, src, dst, lens)
+    assert np.array_equal(got, before)
