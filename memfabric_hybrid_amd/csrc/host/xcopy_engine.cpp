@@ -568,8 +568,20 @@ int SealQueued(ThreadLease &ctx)
 
 // The kernels just launched on `stream` read `slot`.  Only launches on the lease's own stream wait
 // for a shared event: a caller's stream may be gone by the time the next launch comes.
-int MarkQueued(ThreadLease &ctx, StagingSlot *slot, void *stream, bool sealNow)
+// The event a launch on `stream` should complete for its slot: launches on a caller's stream are guarded one by one, since nothing
+// says how long the stream lives; those on the thread's own stream several at a time, by an event recorded behind them.
+void *EventOfLaunch(const ThreadLease &ctx, const StagingSlot &slot, const void *stream)
 {
+    return stream != ctx.stream ? slot.event : nullptr;
+}
+
+int MarkQueued(ThreadLease &ctx, StagingSlot *slot, void *stream, bool sealNow, bool attached = false)
+{
+    if (attached) {   // its launch completes the slot's event
+        slot->state = StagingSlot::kGuarded;
+        slot->guard = slot;
+        return BM_OK;
+    }
     sealNow = sealNow || stream != ctx.stream;
     slot->state = StagingSlot::kQueued;
     slot->guard = nullptr;
@@ -1947,13 +1959,16 @@ int XcopyEngine::SubmitPieces(const uint64_t *src, const uint64_t *dst, const ui
         (void)BuildInlinePlan(none, kXcopyThreads, empty);
         return mfk_xcopy_inline(&empty, MFRT_ROUTE_HBM, 1, mask, maskValue, stream, 0, 0) == 0 ? BM_OK : BM_ERROR;
     }
-    const int err = mfk_xcopy_pieces(pieces, count, total, units, mask, maskValue, stream, HoldForPieces(count, units, unordered));
+    int attached = 0;
+    const int err = mfk_xcopy_pieces(pieces, count, total, units, mask, maskValue, stream, HoldForPieces(count, units, unordered),
+                                     EventOfLaunch(lease, *slot, stream), &attached);
     if (err != 0) {
+        (void)MarkQueued(lease, slot, stream, true);   // the launch may have gone out with only the word behind it failing
         MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(err));
     }
     g_launches.fetch_add(1, std::memory_order_relaxed);
     NotePending(stream, total);
-    return MarkQueued(lease, slot, stream, false);
+    return MarkQueued(lease, slot, stream, false, attached != 0);
 }
 
 int XcopyEngine::SubmitDeviceTable(const void *triples, uint32_t n, int route, void *stream, void *mask,
@@ -1991,15 +2006,16 @@ int XcopyEngine::SubmitDeviceTable(const void *triples, uint32_t n, int route, v
     }
     const uint32_t cu = mfrt_cu_count();
     const uint32_t units = ChooseUnits(0, cu, route, tuning_);   // sizes are only known on the GPU
+    int attached = 0;
     const int err = mfk_xcopy_direct(triples, n, units, route, DeviceTableGrid(n, cu, route, tuning_), DeviceTableRestGrid(cu, route, tuning_),
-                                     slot->rest, kRestCapacity, mask, maskValue, stream);
+                                     slot->rest, kRestCapacity, mask, maskValue, stream, EventOfLaunch(lease, *slot, stream), &attached);
     if (err != 0) {
         (void)MarkQueued(lease, slot, stream, true);   // the first launch writes the list
         MF_FAIL(BM_ERROR, "xcopy launch of a device table failed: " << mfrt_error_string(err));
     }
     g_launches.fetch_add(2, std::memory_order_relaxed);
     NotePending(stream, ~0ull);   // sizes unknown here: the next wait sleeps on the stream
-    return MarkQueued(lease, slot, stream, false);
+    return MarkQueued(lease, slot, stream, false, attached != 0);
 }
 
 #ifndef MF_RT_HIDDEN

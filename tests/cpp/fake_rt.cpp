@@ -372,8 +372,8 @@ int mfk_xcopy_table(const void *tablePlan, int, uint32_t grid, void *mask, uint3
 
 // The pieces in the order of the kernel's workgroups.  One that is longer than its workgroup or reaches past the end of the list
 // fails the launch.
-int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, void *mask, uint32_t maskValue, void *,
-                     uint32_t holdNanos)
+int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, void *mask, uint32_t maskValue,
+                     void *stream, uint32_t holdNanos, void *event, int *attached)
 {
     g_lastTableHold = holdNanos;
     if (pieces == nullptr || count == 0 || (units != 256 && units != 512 && units != 1024)) {
@@ -406,6 +406,7 @@ int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_
     if (moved != bytes) {
         return 721;
     }
+    *attached = event != nullptr && mfrt_event_record(event, stream) == 0 ? 1 : 0;
     if (mask != nullptr) {
         *static_cast<uint64_t *>(mask) = maskValue;
     }
@@ -415,8 +416,9 @@ int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_
 // The direct copy of a device-resident table restated: the parts of every segment, and the pieces of long ones out of a list
 // that a small capacity makes run over.
 int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int, uint32_t grid, uint32_t restGrid, void *rest,
-                     uint32_t capacity, void *mask, uint32_t maskValue, void *)
+                     uint32_t capacity, void *mask, uint32_t maskValue, void *stream, void *event, int *attached)
 {
+    *attached = event != nullptr && mfrt_event_record(event, stream) == 0 ? 1 : 0;
     mf::RestList *list = static_cast<mf::RestList *>(rest);
     if (nseg == 0 || grid == 0 || restGrid == 0 || list == nullptr || capacity == 0 || list->count != 0 || list->done != 0) {
         return -1;
@@ -490,7 +492,8 @@ int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, i
     if (nseg == 0 || nseg > MFK_STATIC_TABLE_SEGMENTS) {
         return -1;
     }
-    return mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, list.data(), 16, nullptr, 0, stream);
+    int attached = 0;
+    return mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, list.data(), 16, nullptr, 0, stream, nullptr, &attached);
 }
 
 static uint32_t g_lastRectMates = 0;
