@@ -624,14 +624,14 @@ template <uint32_t kSlots>
 __global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(const u32x4 *__restrict__ x, const int32_t *__restrict__ topk,
                                                                         uint32_t total, uint32_t topK, uint32_t experts,
                                                                         uint32_t unitsPerRow, uint32_t parts, uint32_t perPart,
-                                                                        u32x4 *__restrict__ out, int32_t *__restrict__ counts,
+                                                                        uint32_t groups, u32x4 *__restrict__ out, int32_t *__restrict__ counts,
                                                                         int32_t *__restrict__ offsets, int32_t *__restrict__ rowOf,
                                                                         int32_t *__restrict__ srcOf, uint32_t *__restrict__ status)
 {
     __shared__ uint32_t lds[kMaxExperts + kSmallThreads / 64];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = threadIdx.x >> 6;
-    if (blockIdx.x == gridDim.x - 1) {
+    if (blockIdx.x == groups - 1) {
         uint32_t *perWave = lds + kMaxExperts;
         for (uint32_t e = threadIdx.x; e < kMaxExperts; e += kSmallThreads) {
             lds[e] = 0;
@@ -1062,7 +1062,7 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
 #define MF_DISPATCH_SMALL(SLOTS)                                                                                       \
     hipLaunchKernelGGL(MoeDispatchSmallKernel<SLOTS>, dim3(tokens * parts + 1), dim3(kSmallThreads), 0, s,              \
                        static_cast<const u32x4 *>(x), static_cast<const int32_t *>(topk), total, topK, experts, upr, parts, perPart, \
-                       static_cast<u32x4 *>(out), static_cast<int32_t *>(counts), static_cast<int32_t *>(offsets),      \
+                       tokens * parts + 1, static_cast<u32x4 *>(out), static_cast<int32_t *>(counts), static_cast<int32_t *>(offsets),      \
                        static_cast<int32_t *>(rowOf), static_cast<int32_t *>(srcOf), status)
         if (topK <= 2) {
             MF_DISPATCH_SMALL(2);

@@ -106,11 +106,11 @@ __device__ __forceinline__ void HoldStores(uint64_t t0, uint32_t ticks)
     }
 }
 
-// Copy chunk k of one segment.  All arguments are wave-uniform.  kHold: the stores of the first step wait
+// Copy chunk k of one segment.  All arguments are wave-uniform.  lanes: 64, 128 or 256, the launcher's choice.  kHold: the stores of the first step wait
 // for HoldStores(t0, ticks).
 template <bool kNtLoad, int kStore, bool kHold = false>
 __device__ __forceinline__ void CopyChunk(uint64_t src, uint64_t dst, uint64_t len, uint64_t k, uint32_t units, uint64_t t0 = 0,
-                                          uint32_t ticks = 0)
+                                          uint32_t ticks = 0, uint32_t lanes = blockDim.x)
 {
     const SegGeom g = SegmentGeometry(dst, len);
     const uint64_t u0 = k * units;
@@ -119,7 +119,6 @@ __device__ __forceinline__ void CopyChunk(uint64_t src, uint64_t dst, uint64_t l
     const uint64_t s = src + g.head + u0 * kUnitBytes;
     const uint64_t d = dst + g.head + u0 * kUnitBytes;
     const uint32_t tid = threadIdx.x;
-    const uint32_t lanes = blockDim.x;                  // 64, 128 or 256: the launcher's choice
     const uint32_t kTile = kDepth * lanes;              // units one workgroup moves per step
 
     uint32_t i = 0;
@@ -232,7 +231,7 @@ enum HoldMode : int { kHoldNone = 0, kHoldShallow = 1, kHoldDeep = 2 };
 
 template <bool kNtLoad, int kStore, int kHold>
 __device__ __forceinline__ void CopyChunkHeld(uint64_t src, uint64_t dst, uint64_t len, uint64_t k, uint32_t units, uint64_t t0,
-                                              uint32_t ticks);
+                                              uint32_t ticks, uint32_t lanes = blockDim.x);
 
 template <bool kNtLoad, int kStore, int kHold = kHoldNone>
 __global__ __launch_bounds__(kXcopyThreads) void XcopyInlineKernel(const InlinePlan p, uint32_t holdTicks)
@@ -300,10 +299,10 @@ __device__ __forceinline__ void CopyChunkWindowed(uint64_t src, uint64_t dst, ui
 // body are skipped lane by lane, head and tail bytes travel as in CopyChunk.
 template <bool kNtLoad, int kStore, int kHold>
 __device__ __forceinline__ void CopyChunkHeld(uint64_t src, uint64_t dst, uint64_t len, uint64_t k, uint32_t units, uint64_t t0,
-                                              uint32_t ticks)
+                                              uint32_t ticks, uint32_t lanes)
 {
     if (kHold != kHoldDeep) {
-        CopyChunk<kNtLoad, kStore, kHold == kHoldShallow>(src, dst, len, k, units, t0, ticks);
+        CopyChunk<kNtLoad, kStore, kHold == kHoldShallow>(src, dst, len, k, units, t0, ticks, lanes);
         return;
     }
     const SegGeom g = SegmentGeometry(dst, len);
@@ -371,12 +370,12 @@ __global__ __launch_bounds__(64) void XcopyWindowKernel(const InlinePlan p, uint
 constexpr uint32_t kSingleMaxChunks = 49152;
 template <bool kNtLoad, int kStore, int kHold = kHoldNone>
 __global__ __launch_bounds__(kXcopyThreads) void XcopySingleKernel(uint64_t src, uint64_t dst, uint32_t len, uint32_t nchunk,
-                                                                   uint32_t units, uint32_t holdTicks)
+                                                                   uint32_t units, uint32_t holdTicks, uint32_t lanes)
 {
     const uint64_t t0 = kHold != kHoldNone ? wall_clock64() : 0;
     uint32_t c = blockIdx.x;
     do {
-        CopyChunkHeld<kNtLoad, kStore, kHold>(src, dst, len, c, units, t0, holdTicks);
+        CopyChunkHeld<kNtLoad, kStore, kHold>(src, dst, len, c, units, t0, holdTicks, lanes);
         c += gridDim.x;
     } while (c < nchunk);
 }
@@ -404,6 +403,7 @@ struct DoneMark {
     uint64_t *word;         // pinned host memory, polled by the caller
     uint32_t *counter;      // device memory, 0 between launches
     uint32_t value;
+    uint32_t groups;        // of the launch
 };
 
 // Every store of the launch is written through (kStoreThrough), so it has reached memory once vmcnt says so, and the last
@@ -415,8 +415,8 @@ __device__ __forceinline__ void MarkDone(const DoneMark &mark)
     if (threadIdx.x != 0) {
         return;
     }
-    if (gridDim.x > 1) {
-        if (__hip_atomic_fetch_add(mark.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1) {
+    if (mark.groups > 1) {
+        if (__hip_atomic_fetch_add(mark.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != mark.groups - 1) {
             return;
         }
         __hip_atomic_store(mark.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -425,14 +425,16 @@ __device__ __forceinline__ void MarkDone(const DoneMark &mark)
     __hip_atomic_store(mark.word, static_cast<uint64_t>(mark.value), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// (Arguments one by one: the 56 bytes are in scalar registers when a wave starts, those of a struct are memory it has to read.)
 template <bool kNtLoad>
 __global__ __launch_bounds__(kXcopyThreads) void XcopySingleDoneKernel(uint64_t src, uint64_t dst, uint32_t len, uint32_t nchunk,
-                                                                       uint32_t units, DoneMark mark)
+                                                                       uint32_t units, uint32_t lanes, uint64_t *word, uint32_t *counter,
+                                                                       uint32_t value, uint32_t groups)
 {
-    for (uint32_t c = blockIdx.x; c < nchunk; c += gridDim.x) {
-        CopyChunk<kNtLoad, kStoreThrough>(src, dst, len, c, units);
+    for (uint32_t c = blockIdx.x; c < nchunk; c += groups) {
+        CopyChunk<kNtLoad, kStoreThrough>(src, dst, len, c, units, 0, 0, lanes);
     }
-    MarkDone(mark);
+    MarkDone(DoneMark{word, counter, value, groups});
 }
 
 template <bool kNtLoad>
@@ -445,7 +447,7 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyInlineDoneKernel(const Inl
     do {
         const InlineChunk r = rows.Owner(c);
         CopyChunk<kNtLoad, kStoreThrough>(r.src, r.dst, r.len, r.k, units);
-        c += gridDim.x;
+        c += mark.groups;
     } while (c < nchunk);
     MarkDone(mark);
 }
@@ -900,16 +902,16 @@ int LaunchInline(const InlinePlan &plan, uint32_t grid, uint32_t lanes, hipStrea
     if (plan.first[1] == kNoChunk && plan.nchunk <= kSingleMaxChunks) {
         if (anyOrder) {
             hipExtLaunchKernelGGL((XcopySingleKernel<kNtLoad, kStore>), dim3(grid), dim3(lanes), 0, stream, nullptr, nullptr, flags,
-                                  plan.src[0], plan.dst[0], plan.len[0], plan.nchunk, plan.units, 0u);
+                                  plan.src[0], plan.dst[0], plan.len[0], plan.nchunk, plan.units, 0u, lanes);
         } else if (ticks != 0 && deep) {
             hipLaunchKernelGGL((XcopySingleKernel<kNtLoad, kStore, kHoldDeep>), dim3(grid), dim3(lanes), 0, stream, plan.src[0],
-                               plan.dst[0], plan.len[0], plan.nchunk, plan.units, ticks);
+                               plan.dst[0], plan.len[0], plan.nchunk, plan.units, ticks, lanes);
         } else if (ticks != 0) {
             hipLaunchKernelGGL((XcopySingleKernel<kNtLoad, kStore, kHoldShallow>), dim3(grid), dim3(lanes), 0, stream, plan.src[0],
-                               plan.dst[0], plan.len[0], plan.nchunk, plan.units, ticks);
+                               plan.dst[0], plan.len[0], plan.nchunk, plan.units, ticks, lanes);
         } else {
             hipLaunchKernelGGL((XcopySingleKernel<kNtLoad, kStore>), dim3(grid), dim3(lanes), 0, stream, plan.src[0], plan.dst[0],
-                               plan.len[0], plan.nchunk, plan.units, 0u);
+                               plan.len[0], plan.nchunk, plan.units, 0u, lanes);
         }
         return static_cast<int>(hipGetLastError());
     }
@@ -1028,13 +1030,14 @@ extern "C" int mfk_xcopy_done(const void *inlinePlan, int route, uint32_t grid, 
     }
     grid = grid < plan.nchunk ? grid : plan.nchunk;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    DoneMark mark{static_cast<uint64_t *>(word), static_cast<uint32_t *>(counter), value};
+    DoneMark mark{static_cast<uint64_t *>(word), static_cast<uint32_t *>(counter), value, grid};
     uint64_t src = plan.src[0];
     uint64_t dst = plan.dst[0];
     uint32_t len = plan.len[0];
     uint32_t nchunk = plan.nchunk;
     uint32_t units = plan.units;
-    void *singleArgs[] = {&src, &dst, &len, &nchunk, &units, &mark};
+    uint32_t lanes = LanesFor(plan.units, route);
+    void *singleArgs[] = {&src, &dst, &len, &nchunk, &units, &lanes, &mark.word, &mark.counter, &mark.value, &mark.groups};
     void *args[] = {const_cast<InlinePlan *>(&plan), &mark};
     const bool single = plan.first[1] == kNoChunk;
     const bool nt = PolicyOf(route).ntLoad;
@@ -1044,7 +1047,7 @@ extern "C" int mfk_xcopy_done(const void *inlinePlan, int route, uint32_t grid, 
         kernel = nt ? reinterpret_cast<const void *>(&XcopySingleDoneKernel<true>)
                     : reinterpret_cast<const void *>(&XcopySingleDoneKernel<false>);
     }
-    return static_cast<int>(hipLaunchKernel(kernel, dim3(grid), dim3(LanesFor(plan.units, route)), single ? singleArgs : args, 0, s));
+    return static_cast<int>(hipLaunchKernel(kernel, dim3(grid), dim3(lanes), single ? singleArgs : args, 0, s));
 }
 
 extern "C" uint32_t mfk_xcopy_window_units(void)
@@ -1175,13 +1178,13 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
             constexpr bool kNt = decltype(ntLoad)::value;
             constexpr int kSt = decltype(store)::value;
             hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, empty, 0u);
-            hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 0u);
+            hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 0u, 64u);
             hipLaunchKernelGGL((XcopyTableKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, none);
             if (route == MFRT_ROUTE_HBM) {
                 hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, empty, 1u);
                 hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, empty, 1u);
-                hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 1u);
-                hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kWindowUnits, 1u);
+                hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 1u, 64u);
+                hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kWindowUnits, 1u, 64u);
                 hipLaunchKernelGGL((XcopyPieceKernel<64, 4, false>), dim3(1), dim3(64), 0, s, nullptr, 0u, 0u);
                 hipLaunchKernelGGL((XcopyPieceKernel<64, 4, true>), dim3(1), dim3(64), 0, s, nullptr, 0u, 0u);
                 hipLaunchKernelGGL((XcopyPieceKernel<64, 16, true>), dim3(1), dim3(64), 0, s, nullptr, 0u, 0u);
