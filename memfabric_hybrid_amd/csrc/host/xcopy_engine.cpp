@@ -1703,9 +1703,9 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         oversized = total > 0xFFFFFFFFull;
         units = ChooseUnits(total, cu, route, tuning_);
         // Large HBM copies of one submitter: 16 KiB chunks for the kernel that alternates between read and write windows.
-        // Not where a source and its destination differ modulo 16: the kernels align their 128-bit units on the destination,
-        // the loads then straddle units, cost twice the issue slots, and the waves keep no schedule at any rate that pays
-        // (100 segments of 10 MB: 5.35 TB/s in windows cut for 6.8, 5.26 for 7.4, 5.51 to 5.56 without windows).
+        // Not where a source and its destination differ modulo 16: the loads that straddle units cost twice the issue slots,
+        // and the waves keep no schedule at any rate that pays (100 segments of 10 MB: 5.35 TB/s in windows cut for 6.8, 5.26
+        // for 7.4, 5.51 to 5.56 without windows).
         const bool aligned = (addressBits & (kWindowAlignBytes - 1)) == 0;
         windowed = !unordered && (apartBits & (kUnitBytes - 1)) == 0 && WindowsApply(total, route, kWindowMinBytes);
         // Segments that all start on cache lines, in source and destination, hold a higher rate.  Back to back at 6.8 / 7.1 /
@@ -1734,6 +1734,14 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
             units = mfk_xcopy_window_units();
         }
         const bool deep = !windowed && DeepHoldApplies(total, n, route, unordered);
+        if (deep && (apartBits & (kUnitBytes - 1)) != 0) {
+            // as pieces: sixteen loads per lane of aligned units and what shifts them, with the table of the kernel arguments, take
+            // more registers than sixteen waves per CU have (42 MB 17.5 us with straddling loads)
+            const int ret = SubmitPieces(src, dst, len, n, total, kDeepUnits, stream, mask, maskValue, unordered);
+            if (ret != kNotLaunched) {
+                return ret;
+            }
+        }
         inlined = BuildInlineDirect(src, dst, len, n, deep ? kDeepUnits : units, plan);
         if (inlined && deep && HoldNanosFor(plan.nchunk, plan.nchunk, kDeepUnits, false) == 0) {
             inlined = BuildInlineDirect(src, dst, len, n, units, plan);   // ragged enough to exceed the waves that hold: the usual chunks

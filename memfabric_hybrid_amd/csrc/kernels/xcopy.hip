@@ -94,6 +94,71 @@ __device__ __forceinline__ void CopyByte(uint64_t src, uint64_t dst)
     }
 }
 
+// The unit of the source that the next lane holds; lane 63 gets `wrap`.
+__device__ __forceinline__ uint32_t NextLane(uint32_t v, uint32_t wrap)
+{
+    const uint32_t next = __builtin_amdgcn_update_dpp(0u, v, 0x130, 0xf, 0xf, true);   // wave_shl:1
+    return (threadIdx.x & 63u) == 63u ? wrap : next;
+}
+
+// Sixteen bytes from byte 4 * kWords + bytes of the pair (a, b) on.
+template <uint32_t kWords>
+__device__ __forceinline__ u32x4 Straddle(u32x4 a, u32x4 b, uint32_t bytes)
+{
+    const uint32_t w[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    u32x4 r;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        r[i] = __builtin_amdgcn_alignbyte(w[i + kWords + 1], w[i + kWords], bytes);
+    }
+    return r;
+}
+
+// A source that differs from its destination modulo 16, read in whole aligned units: loads that straddle units cost twice the cache
+// accesses (4.9 MB of ragged segments 4.7 / 3.9 us, 69 MB 30.4 / 29.2).  A wave takes kUnits * 64 consecutive ones from u0 on, of
+// those 0 ... end that hold any of the bytes, so that what a lane lacks is in the next lane's unit; `last` is what lane 63 of
+// its last unit lacks.  Up to 15 bytes beside the source are read, of units that hold some of its bytes.
+template <uint32_t kUnits>
+__device__ __forceinline__ void LoadApart(u32x4 (&v)[kUnits], u32x4 &last, uint64_t aligned, uint32_t u0, uint32_t end)
+{
+    const uint32_t u = u0 + (threadIdx.x & 63u);
+#pragma unroll
+    for (uint32_t j = 0; j < kUnits; ++j) {
+        if (u + j * 64 <= end) {
+            v[j] = LoadAligned(aligned + (u + j * 64) * kUnitBytes);
+        }
+    }
+    const uint32_t behind = u0 + kUnits * 64 < end ? u0 + kUnits * 64 : end;
+    last = LoadAligned(aligned + behind * kUnitBytes);
+}
+
+template <int kStore, uint32_t kUnits>
+__device__ __forceinline__ void StoreApart(const u32x4 (&v)[kUnits], u32x4 last, uint64_t dst, uint32_t u0, uint32_t end, uint32_t apart)
+{
+    const uint32_t u = u0 + (threadIdx.x & 63u);
+    auto store = [&](auto words) {
+#pragma unroll
+        for (uint32_t j = 0; j < kUnits; ++j) {
+            u32x4 next;
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                const uint32_t wrap = j + 1 < kUnits ? v[j + 1 < kUnits ? j + 1 : 0][i] : last[i];
+                next[i] = NextLane(v[j][i], __builtin_amdgcn_readfirstlane(wrap));
+            }
+            const u32x4 r = Straddle<decltype(words)::value>(v[j], next, apart & 3u);
+            if (u + j * 64 < end) {
+                StoreUnit<kStore>(dst + (u + j * 64) * kUnitBytes, r);
+            }
+        }
+    };
+    switch (apart >> 2) {
+        case 0: store(std::integral_constant<uint32_t, 0>()); break;
+        case 1: store(std::integral_constant<uint32_t, 1>()); break;
+        case 2: store(std::integral_constant<uint32_t, 2>()); break;
+        default: store(std::integral_constant<uint32_t, 3>()); break;
+    }
+}
+
 constexpr uint32_t kDepth = 4;                          // 128-bit loads in flight per lane
 
 // Wait until `ticks` of the constant-rate clock have passed since t0, after the loads have landed (so
@@ -122,6 +187,19 @@ __device__ __forceinline__ void CopyChunk(uint64_t src, uint64_t dst, uint64_t l
     const uint32_t kTile = kDepth * lanes;              // units one workgroup moves per step
 
     uint32_t i = 0;
+    const uint32_t apart = static_cast<uint32_t>(s) & (kUnitBytes - 1);
+    if (kStore == kStoreStream && apart != 0) {
+        for (; i < n; i += kTile) {
+            u32x4 v[kDepth];
+            u32x4 last;
+            const uint32_t u = i + (tid >> 6) * kDepth * 64;
+            LoadApart(v, last, s - apart, u, n);
+            if (kHold && i == 0) {
+                HoldStores(t0, ticks);
+            }
+            StoreApart<kStore>(v, last, d, u, n, apart);
+        }
+    }
     for (; i + kTile <= n; i += kTile) {
         u32x4 v[kDepth];
 #pragma unroll
@@ -581,32 +659,9 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyTableKernel(const TablePla
     }
 }
 
-// The unit of the source that the next lane holds; lane 63 gets `wrap`.
-__device__ __forceinline__ uint32_t NextLane(uint32_t v, uint32_t wrap)
-{
-    const uint32_t next = __builtin_amdgcn_update_dpp(0u, v, 0x130, 0xf, 0xf, true);   // wave_shl:1
-    return (threadIdx.x & 63u) == 63u ? wrap : next;
-}
-
-// Sixteen bytes from byte 4 * kWords + bytes of the pair (a, b) on.
-template <uint32_t kWords>
-__device__ __forceinline__ u32x4 Straddle(u32x4 a, u32x4 b, uint32_t bytes)
-{
-    const uint32_t w[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-    u32x4 r;
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-        r[i] = __builtin_amdgcn_alignbyte(w[i + kWords + 1], w[i + kWords], bytes);
-    }
-    return r;
-}
-
 // Pieces of up to kLanes * kUnits units (xcopy_plan.h), one per workgroup.  HBM is the bound; what the form saves is everything in
 // front of the first load: descriptors are fetched in one step from the host's memory, where a table with a chunk prefix and
 // an owner map had to be moved to HBM by a launch of its own first, and no wave looks anything up.
-// A source that differs from its destination modulo 16 is read in whole aligned units, each lane taking what it lacks from the
-// next lane's: loads that straddle units cost twice the cache accesses (4.9 MB of ragged segments 4.7 / 3.9 us, 69 MB 30.4 / 29.2).
-// Such a load reads up to 15 bytes beside the piece, of units that hold some of its bytes.
 // Shapes, measured on the kernel alone: single waves of 4 KiB as long as those are resident together, for their held stores;
 // single waves of 16 KiB, held, beyond; and without hold four waves of 16 KiB, or as many as the usual segment fills: 4096 pages of 32 KiB
 // gathered 45.8 / 49.4 / 46.4 us with 4 KiB waves / 16 KiB waves / four waves, scattered 49.9 / 51.4 / 49.2, and a quarter of the
@@ -660,41 +715,13 @@ __global__ __launch_bounds__(kLanes) void XcopyPieceKernel(const Piece *__restri
             }
         }
     } else if (body != 0) {
-        // units 0 ... body of the aligned source; a wave has consecutive ones, so that the next unit is the next lane's
-        const uint64_t a = s - apart;
+        u32x4 last;
         const uint32_t u0 = (tid >> 6) * kUnits * 64;
-        const uint32_t u = u0 + (tid & 63u);
-#pragma unroll
-        for (uint32_t j = 0; j < kUnits; ++j) {
-            if (u + j * 64 <= body) {
-                v[j] = LoadAligned(a + (u + j * 64) * kUnitBytes);
-            }
-        }
-        const uint32_t behind = u0 + kUnits * 64 < body ? u0 + kUnits * 64 : body;      // what lane 63 of the last unit lacks
-        const u32x4 last = LoadAligned(a + behind * kUnitBytes);
+        LoadApart(v, last, s - apart, u0, body);
         if (kHold) {
             HoldStores(t0, holdTicks);
         }
-        auto store = [&](auto words) {
-#pragma unroll
-            for (uint32_t j = 0; j < kUnits; ++j) {
-                u32x4 next;
-#pragma unroll
-                for (uint32_t i = 0; i < 4; ++i) {
-                    next[i] = NextLane(v[j][i], Uniform(j + 1 < kUnits ? v[j + 1 < kUnits ? j + 1 : 0][i] : last[i]));
-                }
-                const u32x4 r = Straddle<decltype(words)::value>(v[j], next, apart & 3u);
-                if (u + j * 64 < body) {
-                    StoreUnit<kStoreStream>(d + (u + j * 64) * kUnitBytes, r);
-                }
-            }
-        };
-        switch (apart >> 2) {
-            case 0: store(std::integral_constant<uint32_t, 0>()); break;
-            case 1: store(std::integral_constant<uint32_t, 1>()); break;
-            case 2: store(std::integral_constant<uint32_t, 2>()); break;
-            default: store(std::integral_constant<uint32_t, 3>()); break;
-        }
+        StoreApart<kStoreStream>(v, last, d, u0, body, apart);
     }
     if (tid < g.head) {
         CopyByte<kStoreStream>(src + tid, dst + tid);
