@@ -3,8 +3,8 @@
 // descriptor lookup, the loads and the stores of a batch add, and what the product kernels need, each as
 // the period per launch of dependent launches on one stream.  A batch holds the blocks of `requests`
 // requests (122 segments of 128 KiB and 16 KiB in turn per request, 8 994 816 bytes): one request is the
-// form whose descriptors travel in the kernel-argument block, several requests take the table form, whose
-// descriptors are fetched from pinned host memory (what the library does for such a batch) or from HBM.
+// form whose descriptors travel in the kernel-argument block, several requests take the form of pieces cut by the
+// host, whose descriptors are fetched from pinned host memory; beside it the table form, from pinned memory or HBM.
 // Every kernel is first run from the host loop (period by HIP events; cheap kernels are bound by the host
 // there) and then replayed from a HIP graph of the same launches, where the host does not set the pace.
 //
@@ -151,8 +151,10 @@ struct Batch {
     TablePlan pinned;                   // triples in pinned host memory, owner by pattern
     TablePlan hbm;                      // triples in HBM, owner by pattern
     TablePlan grouped;                  // triples, prefix and group map in HBM, no pattern
-    TablePlan deepPinned;               // chunks of 16 KiB (what the library takes for 24 to 64 MiB), triples in pinned memory
-    TablePlan deepHbm;                  // the same with the triples in HBM
+    const Piece *pieces;                // of 4 KiB, in pinned host memory: as many as nchunk
+    const Piece *deepPieces;            // of 16 KiB (what the library takes for 24 to 64 MiB)
+    uint32_t ndeep;
+    uint64_t bytes;
     uint32_t nchunk;
 };
 
@@ -242,10 +244,13 @@ std::vector<Batch> MakeBatches(char *pool, uint64_t poolBytes, int count, uint32
     const uint32_t ngroups = GroupCount(nchunk, kGroupShiftMin);
     const uint64_t tableWords64 = 3ull * nseg;                                     // triples
     const uint64_t tableBytes = (tableWords64 * 8 + 4ull * (nseg + 1) + 4ull * (ngroups + 1) + 255) & ~255ull;
+    const uint32_t ndeep = nseg / 2 * 9;                                           // 128 KiB: eight pieces of 16 KiB, 16 KiB: one
+    Piece *pieces = nullptr;
     char *hostTables = nullptr;
     char *devTables = nullptr;
     MF_CHECK(hipHostMalloc(&hostTables, tableBytes * count, hipHostMallocDefault));
     MF_CHECK(hipMalloc(&devTables, tableBytes * count));
+    MF_CHECK(hipHostMalloc(&pieces, sizeof(Piece) * (nchunk + ndeep) * count, hipHostMallocDefault));
     std::vector<Batch> batches(count);
     for (int b = 0; b < count; ++b) {
         std::vector<uint32_t> pick;
@@ -312,16 +317,20 @@ std::vector<Batch> MakeBatches(char *pool, uint64_t poolBytes, int count, uint32
         const char *dev = devTables + b * tableBytes;
         plan.triples = reinterpret_cast<const uint64_t *>(dev);
         batch.hbm = plan;
-        {
-            TablePlan deep = batch.pinned;
-            deep.units = kDeepUnits;
-            deep.pattern.chunksPerPeriod = 9;      // 128 KiB: eight chunks of 16 KiB, 16 KiB: one
-            deep.pattern.start[1] = 8;
-            deep.pattern.start[2] = 9;
-            deep.nchunk = nseg / 2 * 9;
-            batch.deepPinned = deep;
-            deep.triples = reinterpret_cast<const uint64_t *>(dev);
-            batch.deepHbm = deep;
+        batch.pieces = pieces;
+        batch.bytes = 0;
+        for (uint32_t i = 0; i < nseg; ++i) {
+            for (uint64_t off = 0; off < triples[3 * i + 2]; off += 4096) {
+                *pieces++ = MakePiece(triples[3 * i] + off, triples[3 * i + 1] + off, 4096);
+            }
+            batch.bytes += triples[3 * i + 2];
+        }
+        batch.deepPieces = pieces;
+        batch.ndeep = ndeep;
+        for (uint32_t i = 0; i < nseg; ++i) {
+            for (uint64_t off = 0; off < triples[3 * i + 2]; off += 16384) {
+                *pieces++ = MakePiece(triples[3 * i] + off, triples[3 * i + 1] + off, 16384);
+            }
         }
         plan.pattern = ChunkPattern{};
         plan.first = reinterpret_cast<const uint32_t *>(dev + tableWords64 * 8);
@@ -358,24 +367,32 @@ void LaunchInlineProduct(const InlinePlan &plan, hipStream_t s, bool held, bool 
         hipExtLaunchKernelGGL((XcopyInlineKernel<true, kStoreStream>), dim3(plan.nchunk), dim3(64), 0, s, nullptr, nullptr,
                               hipExtAnyOrderLaunch, plan, 0u);
     } else if (ticks != 0) {
-        hipLaunchKernelGGL((XcopyInlineKernel<true, kStoreStream, true>), dim3(plan.nchunk), dim3(64), 0, s, plan, ticks);
+        hipLaunchKernelGGL((XcopyInlineKernel<true, kStoreStream, kHoldShallow>), dim3(plan.nchunk), dim3(64), 0, s, plan, ticks);
     } else {
         hipLaunchKernelGGL((XcopyInlineKernel<true, kStoreStream>), dim3(plan.nchunk), dim3(64), 0, s, plan, 0u);
     }
 }
 
-// What the library launches for a batch of 24 to 64 MiB: 16 KiB per wave, sixteen loads per lane, stores held back
-// (2.4 us longer where every workgroup first fetches its descriptor over the link).
-void LaunchTableDeep(const TablePlan &plan, hipStream_t s, bool pinned)
+// What the library launches for more than kInlineSegs segments: up to 24 MiB in waves of 4 KiB, up to 64 MiB in waves of 16 KiB,
+// stores held back by the rule of the kernel-argument form and what the engine adds for descriptors behind the link.
+void LaunchPiecesProduct(const Batch &b, hipStream_t s)
 {
-    const uint32_t nanos = HoldNanosFor(plan.nchunk, plan.nchunk, plan.units, false);
-    const uint32_t ticks = HoldTicks(nanos != 0 && pinned ? nanos + 2400 : nanos);
-    hipLaunchKernelGGL((XcopyTableKernel<true, kStoreStream, false, kHoldDeep>), dim3(plan.nchunk), dim3(64), 0, s, plan, ticks);
+    const bool deep = b.bytes > kDeepMinBytes && b.bytes <= kDeepMaxBytes;
+    const uint32_t units = b.bytes > kDeepMinBytes ? kDeepUnits : kXcopyThreads;
+    const uint32_t count = units == kDeepUnits ? b.ndeep : b.nchunk;
+    const uint32_t rule = HoldNanosFor(count, count, units, false);
+    int attached = 0;
+    const int err = mfk_xcopy_pieces(units == kDeepUnits ? b.deepPieces : b.pieces, count, b.bytes, units, nullptr, 0, s,
+                                     rule != 0 ? rule + (deep ? kHoldLookupDeepExtraNanos : kHoldLookupExtraNanos) : 0, nullptr, &attached);
+    if (err != 0) {
+        std::fprintf(stderr, "mfk_xcopy_pieces failed: %d\n", err);
+        std::exit(1);
+    }
 }
 
 void LaunchTableProduct(const TablePlan &plan, hipStream_t s)
 {
-    hipLaunchKernelGGL((XcopyTableKernel<true, kStoreStream, false>), dim3(plan.nchunk), dim3(64), 0, s, plan, 0u);
+    hipLaunchKernelGGL((XcopyTableKernel<true, kStoreStream>), dim3(plan.nchunk), dim3(64), 0, s, plan);
 }
 
 void Measure(uint32_t requests, char *pool, uint64_t poolBytes, hipStream_t s)
@@ -401,14 +418,11 @@ void Measure(uint32_t requests, char *pool, uint64_t poolBytes, hipStream_t s)
         rows.push_back({"hbm_descriptor_and_loads", [](const Batch &b, hipStream_t st) { LaunchTablePhase<2>(b.hbm, st); }, true});
         rows.push_back({"hbm_descriptor_and_stores", [](const Batch &b, hipStream_t st) { LaunchTablePhase<3>(b.hbm, st); }, true});
         rows.push_back({"pinned_descriptor_and_loads", [](const Batch &b, hipStream_t st) { LaunchTablePhase<2>(b.pinned, st); }, true});
-        rows.push_back({"product_table_kernel_pinned_descriptors",
+        rows.push_back({"table_kernel_pinned_descriptors",
                         [](const Batch &b, hipStream_t st) { LaunchTableProduct(b.pinned, st); }, true});
-        rows.push_back({"product_table_kernel_hbm_descriptors", [](const Batch &b, hipStream_t st) { LaunchTableProduct(b.hbm, st); }, true});
-        rows.push_back({"product_table_kernel_group_map", [](const Batch &b, hipStream_t st) { LaunchTableProduct(b.grouped, st); }, true});
-        rows.push_back({"product_table_kernel_16KiB_chunks_held_pinned_descriptors",
-                        [](const Batch &b, hipStream_t st) { LaunchTableDeep(b.deepPinned, st, true); }, true});
-        rows.push_back({"product_table_kernel_16KiB_chunks_held_hbm_descriptors",
-                        [](const Batch &b, hipStream_t st) { LaunchTableDeep(b.deepHbm, st, false); }, true});
+        rows.push_back({"table_kernel_hbm_descriptors", [](const Batch &b, hipStream_t st) { LaunchTableProduct(b.hbm, st); }, true});
+        rows.push_back({"table_kernel_group_map", [](const Batch &b, hipStream_t st) { LaunchTableProduct(b.grouped, st); }, true});
+        rows.push_back({"product_pieces_pinned_descriptors", [](const Batch &b, hipStream_t st) { LaunchPiecesProduct(b, st); }, true});
         rows.push_back({"inline_launches_first_ordered_rest_any_order", [](const Batch &b, hipStream_t st) {
                             for (size_t i = 0; i < b.slices.size(); ++i) {
                                 LaunchInlineProduct(b.slices[i], st, false, i != 0);

@@ -41,10 +41,6 @@ struct SegList {
 void NormalizeSegments(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t pieceLimit,
                        SegList &out);
 
-// On top of HoldNanosFor's rule where the waves of a launch have to look their descriptors up outside the kernel arguments, a
-// round trip across the host link before their loads, and the same on 16 KiB chunks: sixteen loads per lane take longer to leave.
-constexpr int32_t kHoldLookupExtraNanos = 1600;
-constexpr int32_t kHoldLookupDeepExtraNanos = 2000;
 constexpr int32_t kHoldPinnedDeepExtraNanos = kHoldLookupDeepExtraNanos - kHoldLookupExtraNanos;
 constexpr uint64_t kPieceListMin = 1ull << 18;     // pieces that any batch may be cut into, 4 MiB of descriptors
 

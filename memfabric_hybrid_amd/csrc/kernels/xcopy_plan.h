@@ -123,6 +123,11 @@ inline uint32_t HoldNanosFor(uint32_t nchunk, uint32_t grid, uint32_t units, boo
     return 640 + kHoldKneeChunks * 6 / 10 + (nchunk - kHoldKneeChunks) * 33 / 100;
 }
 
+// On top of HoldNanosFor's rule where the waves of a launch have to look their descriptors up outside the kernel arguments, a
+// round trip across the host link before their loads, and the same on 16 KiB chunks: sixteen loads per lane take longer to leave.
+constexpr int32_t kHoldLookupExtraNanos = 1600;
+constexpr int32_t kHoldLookupDeepExtraNanos = 2000;
+
 // What a launch of `count` pieces waits of the time a table of as many chunks would.  Its descriptors arrive eight to a line, and
 // kPieceLeadNanos sooner than three words per wave did; and ragged pieces are not full, so that the reads are over sooner: by
 // the rate of the rule above for the bytes that are not there.  Best waits beyond HoldNanosFor(count): K and V blocks of 10 / 18 /
