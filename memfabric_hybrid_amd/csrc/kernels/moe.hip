@@ -788,15 +788,75 @@ __device__ __forceinline__ float Bf16Hi(uint32_t w)
     return __uint_as_float(w & 0xFFFF0000u);
 }
 
-// round to nearest even; NaN stays a quiet NaN
-__device__ __forceinline__ uint32_t ToBf16(float f)
+// Two results in one word, each rounded to nearest even; NaN stays a quiet NaN, subnormal numbers stay what they are: one
+// v_cvt_pk_bf16_f32, which gives what the eight integer operations per value that it replaces gave, for all 2^32 inputs.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t ToBf16Pair(float lo, float hi)
 {
-    const uint32_t w = __float_as_uint(f);
-    if ((w & 0x7FFFFFFFu) > 0x7F800000u) {
-        return (w >> 16) | 0x0040u;
-    }
-    return (w + 0x7FFFu + ((w >> 16) & 1u)) >> 16;
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
+
+// The columns [begin, end) of one token.  kAllLive: every slot has a row, which is the usual case and needs no
+// branch per slot.
+template <uint32_t kTopK, uint32_t kThreads, bool kNtLoad, uint32_t kBatch, bool kAllLive, uint32_t kSlots = kTopK != 0 ? kTopK : kMaxTopK>
+__device__ __forceinline__ void CombineColumns(const MF_GLOBAL u32x4 *in, MF_GLOBAL u32x4 *dst, const uint64_t (&rowBase)[kSlots],
+                                               const float (&w)[kSlots], uint32_t live, uint32_t begin, uint32_t end)
+{
+    // kBatch column positions per lane are requested together (kBatch * K loads in flight per lane)
+    // before any of them is consumed.
+    for (uint32_t u0 = begin + threadIdx.x; u0 < end; u0 += kBatch * kThreads) {
+        u32x4 v[kBatch][kSlots];
+#pragma unroll
+        for (uint32_t b = 0; b < kBatch; ++b) {
+            const uint32_t u = u0 + b * kThreads;
+#pragma unroll
+            for (uint32_t k = 0; k < kSlots; ++k) {
+                if ((kAllLive || ((live >> k) & 1u) != 0) && u < end) {
+                    v[b][k] = kNtLoad ? __builtin_nontemporal_load(in + rowBase[k] + u) : in[rowBase[k] + u];
+                }
+            }
+        }
+#pragma unroll
+        for (uint32_t b = 0; b < kBatch; ++b) {
+            const uint32_t u = u0 + b * kThreads;
+            if (u >= end) {
+                break;
+            }
+            float acc[8];
+#pragma unroll
+            for (uint32_t i = 0; i < 8; ++i) {
+                acc[i] = 0.0f;
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < kSlots; ++k) {
+                if (kAllLive || ((live >> k) & 1u) != 0) {
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; ++i) {
+                        acc[2 * i] = __builtin_fmaf(w[k], Bf16Lo(v[b][k][i]), acc[2 * i]);
+                        acc[2 * i + 1] = __builtin_fmaf(w[k], Bf16Hi(v[b][k][i]), acc[2 * i + 1]);
+                    }
+                }
+            }
+            u32x4 o;
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                o[i] = ToBf16Pair(acc[2 * i], acc[2 * i + 1]);
+            }
+            __builtin_nontemporal_store(o, dst + u);
+        }
+    }
+}
+
+// Calls whose dispatch is one launch and whose buffers, this much together, stay in the last-level cache (256 MiB, used by others
+// too) find the rows there: plain loads, and one column position per lane, so that twice as many waves each do half as much.
+// What bounds those calls is the chain of one wave; before, a test per slot stood between any two loads and each result took
+// sixteen integer operations to round, code that is fetched anew in every launch.  Dispatch and combine in turn, of 7168
+// elements at top-8 (before / all slots tested at once and the rounding in one instruction / this): 16 tokens 11.0 / 8.2 / 7.1 us,
+// 64 12.4 / 10.4 / 10.1, 256 16.2 / 15.9 / 14.7, 512 26.2 / 30.5 / 25.2; combine alone 64 tokens 5.7 / 3.7 / 3.1.  Beyond, plain loads
+// lose: 2048 tokens at top-2, 117 MB, 27.5 us without and 30.1 with them, 1000 at top-8 52.8 and 61.2.  Larger calls gain from the shorter
+// code alone: 1500 tokens 76.8 -> 74.3 us.
+constexpr uint64_t kCombineCachedBytes = 80ull << 20;
 
 template <uint32_t kTopK, uint32_t kThreads, bool kNtLoad, uint32_t kBatch = 1>
 __global__ __launch_bounds__(kThreads) void MoeCombineKernel(const u32x4 *__restrict__ rowsIn,
@@ -832,48 +892,10 @@ __global__ __launch_bounds__(kThreads) void MoeCombineKernel(const u32x4 *__rest
     const MF_GLOBAL u32x4 *in = reinterpret_cast<const MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(rowsIn));
     MF_GLOBAL u32x4 *dst = reinterpret_cast<MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(y)) +
                            static_cast<uint64_t>(token) * unitsPerRow;
-    // kBatch column positions per lane are requested together (kBatch * K loads in flight per lane)
-    // before any of them is consumed.
-    for (uint32_t u0 = begin + threadIdx.x; u0 < end; u0 += kBatch * kThreads) {
-        u32x4 v[kBatch][kSlots];
-#pragma unroll
-        for (uint32_t b = 0; b < kBatch; ++b) {
-            const uint32_t u = u0 + b * kThreads;
-#pragma unroll
-            for (uint32_t k = 0; k < kSlots; ++k) {
-                if (((live >> k) & 1u) != 0 && u < end) {
-                    v[b][k] = kNtLoad ? __builtin_nontemporal_load(in + rowBase[k] + u) : in[rowBase[k] + u];
-                }
-            }
-        }
-#pragma unroll
-        for (uint32_t b = 0; b < kBatch; ++b) {
-            const uint32_t u = u0 + b * kThreads;
-            if (u >= end) {
-                break;
-            }
-            float acc[8];
-#pragma unroll
-            for (uint32_t i = 0; i < 8; ++i) {
-                acc[i] = 0.0f;
-            }
-#pragma unroll
-            for (uint32_t k = 0; k < kSlots; ++k) {
-                if (((live >> k) & 1u) != 0) {
-#pragma unroll
-                    for (uint32_t i = 0; i < 4; ++i) {
-                        acc[2 * i] = __builtin_fmaf(w[k], Bf16Lo(v[b][k][i]), acc[2 * i]);
-                        acc[2 * i + 1] = __builtin_fmaf(w[k], Bf16Hi(v[b][k][i]), acc[2 * i + 1]);
-                    }
-                }
-            }
-            u32x4 o;
-#pragma unroll
-            for (uint32_t i = 0; i < 4; ++i) {
-                o[i] = ToBf16(acc[2 * i]) | (ToBf16(acc[2 * i + 1]) << 16);
-            }
-            __builtin_nontemporal_store(o, dst + u);
-        }
+    if (kTopK != 0 && live == (1u << nk) - 1u) {
+        CombineColumns<kTopK, kThreads, kNtLoad, kBatch, true>(in, dst, rowBase, w, live, begin, end);
+    } else {
+        CombineColumns<kTopK, kThreads, kNtLoad, kBatch, false>(in, dst, rowBase, w, live, begin, end);
     }
 }
 
@@ -977,7 +999,7 @@ __global__ __launch_bounds__(64) void MoeCombineWindowKernel(const u32x4 *__rest
                     }
 #pragma unroll
                     for (uint32_t i = 0; i < 4; ++i) {
-                        o[j][b][i] = ToBf16(acc[2 * i]) | (ToBf16(acc[2 * i + 1]) << 16);
+                        o[j][b][i] = ToBf16Pair(acc[2 * i], acc[2 * i + 1]);
                     }
                 }
             }
@@ -1164,7 +1186,23 @@ extern "C" int mfk_moe_combine(const void *rows, const void *rowOf, const void *
     const float *w = static_cast<const float *>(weights);
     u32x4 *o = static_cast<u32x4 *>(y);
     const uint32_t upr = hidden / 8;
-    if (upr >= 256 && (topK == 2 || topK == 4 || topK == 6 || topK == 8)) {
+    const uint64_t traffic = static_cast<uint64_t>(tokens) * (topK + 2) * upr * 16;   // the rows, the tokens they came from, the result
+    const bool fanIn = topK == 2 || topK == 4 || topK == 6 || topK == 8;
+    if (upr >= 256 && fanIn && static_cast<uint64_t>(tokens) * topK <= kSmallEntries && traffic <= kCombineCachedBytes) {
+        // One column position per lane and plain loads: where the line lies, see kCombineCachedBytes.
+        const uint32_t parts = (upr + 63) / 64;
+#define MF_COMBINE_CACHED(K) hipLaunchKernelGGL((MoeCombineKernel<K, 64, false>), dim3(tokens * parts), dim3(64), 0, s, in, ro, w, topK, upr, parts, o)
+        if (topK == 2) {
+            MF_COMBINE_CACHED(2);
+        } else if (topK == 4) {
+            MF_COMBINE_CACHED(4);
+        } else if (topK == 6) {
+            MF_COMBINE_CACHED(6);
+        } else {
+            MF_COMBINE_CACHED(8);
+        }
+#undef MF_COMBINE_CACHED
+    } else if (upr >= 256 && fanIn) {
         // Wide rows: single-wave workgroups, each on a 128-unit slice of the row with two column positions per
         // lane in flight (2 x topK loads), the fastest shape measured on 7168-element rows at top-8 (178 us; one
         // four-wave workgroup per token 188 us; plain instead of nontemporal loads 194 us).  Compiled for the common
@@ -1210,10 +1248,21 @@ extern "C" int mfk_moe_combine(const void *rows, const void *rowOf, const void *
         }
 #undef MF_COMBINE_SLICES
 #undef MF_COMBINE_WINDOWS
-    } else if (topK == 8) {
-        hipLaunchKernelGGL((MoeCombineKernel<8, 256, true>), dim3(tokens), dim3(256), 0, s, in, ro, w, topK, upr, 1u, o);
     } else {
-        hipLaunchKernelGGL((MoeCombineKernel<0, 256, true>), dim3(tokens), dim3(256), 0, s, in, ro, w, topK, upr, 1u, o);
+        // Narrow rows: one four-wave workgroup per token, compiled for the common fan-ins too, whose loads are then in flight together.
+#define MF_COMBINE_TOKEN(K) hipLaunchKernelGGL((MoeCombineKernel<K, 256, true>), dim3(tokens), dim3(256), 0, s, in, ro, w, topK, upr, 1u, o)
+        if (topK == 2) {
+            MF_COMBINE_TOKEN(2);
+        } else if (topK == 4) {
+            MF_COMBINE_TOKEN(4);
+        } else if (topK == 6) {
+            MF_COMBINE_TOKEN(6);
+        } else if (topK == 8) {
+            MF_COMBINE_TOKEN(8);
+        } else {
+            MF_COMBINE_TOKEN(0);
+        }
+#undef MF_COMBINE_TOKEN
     }
     return static_cast<int>(hipGetLastError());
 }

@@ -446,3 +446,40 @@ def test_rows_read_ahead_of_the_permute(gpu, oracle, T, H, K, E):
         assert np.array_equal(_fetch(bufs["out"], np.uint16, (T * K, H)), x[order // K])
     finally:
         _free(bufs)
+
+
+@pytest.mark.parametrize("T,H,K", [
+    (1, 7168, 8), (3, 2048, 2), (33, 2056, 4),           # few entries: one column position per lane, rows of 256 and 257 units
+    (512, 2048, 8), (513, 2048, 8),                      # the last call of 4096 entries and one beyond
+    (682, 2064, 6),                                      # 4092 entries
+    (1700, 4096, 2), (2048, 7168, 2),                    # 56 MB, and 117 MB at 4096 entries
+    (9, 2040, 6), (40, 8, 2), (300, 1992, 4), (77, 512, 2), (21, 1536, 8),   # narrow rows: one workgroup per token
+])
+def test_combine_of_any_values(gpu, oracle, T, H, K):
+    """Rows of all bit patterns (infinities, NaN, subnormal numbers) and weights down to 1e-38, tokens with and without
+    slots that have no row: the oracle's bits, and NaN where it has NaN (which NaN is the hardware's matter)."""
+    rng = np.random.default_rng(T * K + H)
+    rows = rng.integers(0, 1 << 16, (T * K, H), dtype=np.uint16)
+    plain = rng.random((T * K, H)) < 0.98                # most are ordinary, so that most results are
+    rows[plain] = rows[plain] & 0x80FF | 0x3F00
+    row_of = rng.permutation(T * K).astype(np.int32).reshape(T, K)
+    row_of[rng.random((T, K)) < 0.05] = -1
+    w = rng.random((T, K), dtype=np.float32)
+    w[::3] *= np.float32(1e-38)
+    expected = np.zeros((T, H), dtype=np.uint16)
+    row_of = np.ascontiguousarray(row_of)
+    oracle.orc_moe_combine(np_ptr(rows), np_ptr(row_of), np_ptr(w), T, H, K, np_ptr(expected))
+    bufs = [_dev(gpu, a) for a in (rows, row_of, w)]
+    y = gpu_util.DeviceBuffer(gpu, T * H * 2)
+    try:
+        y.fill(0xEE)
+        assert gpu.mf_moe_combine(*[b.ptr for b in bufs], T, H, K, y.ptr, None) == 0, native.last_error()
+        assert gpu.mfrt_device_sync() == 0
+        got = _fetch(y, np.uint16, (T, H))
+        nan = (expected & 0x7FFF) > 0x7F80
+        assert np.array_equal((got & 0x7FFF) > 0x7F80, nan)
+        assert np.array_equal(got[~nan], expected[~nan])
+        assert np.any((expected & 0x7F80) == 0)          # subnormal results are among them
+    finally:
+        for b in bufs + [y]:
+            b.free()
