@@ -8,7 +8,7 @@
 //   combine   y[t][h] = bf16_rne(fma(w[t][K-1], v[K-1], ... fma(w[t][0], v[0], 0)))
 //
 // One launch for a dispatch of up to 4096 entries (MoeDispatchSmallKernel: every token ranks its own entries).
-// Three launches for a larger one (two when the entries fill at most eight rank blocks), one for combine:
+// Three launches for a larger one (two when the entries fill few rank blocks), one for combine:
 //   MoeHistKernel    per-block expert histograms (wave ballots + LDS); not launched for a few blocks,
 //                    which count one another's entries inside the rank kernel
 //   MoeRankKernel    cross-block scan, stable rank of every entry -> rowOf/srcOf, counts, offsets,
@@ -39,17 +39,23 @@
 namespace mf {
 namespace {
 
-constexpr uint32_t kRankThreads = 256;                 // 4 waves
-constexpr uint32_t kRankRounds = 4;                    // entries per lane
+// A rank launch is a chain of steps that each wait (ids, ballots, LDS tables, scans), so a block has a wave per slice: with four
+// waves of four slices each 1024 / 2048 tokens of 1024 elements at top-8 took 14.5 / 18.5 us per dispatch, so 12.4 / 15.3, 4096 of 7168
+// 92.5 / 90.4.
+constexpr uint32_t kRankThreads = 1024;                // 16 waves
+constexpr uint32_t kRankRounds = 1;                    // entries per lane
 constexpr uint32_t kRankBlock = kRankThreads * kRankRounds;  // 1024 entries per workgroup
 constexpr uint32_t kRankSlices = kRankBlock / 64;      // 16 wave-sized slices, in entry order
 constexpr uint32_t kMaxExperts = 512;
 constexpr uint32_t kRowThreads = 256;
 constexpr uint32_t kMaxTopK = 16;
-constexpr uint32_t kCountingBlocks = 8;                 // launches of up to this many rank blocks need no histogram kernel
+constexpr uint32_t kCountingBlocks = 24;                // launches of up to this many rank blocks need no histogram kernel
+constexpr uint32_t kCountingBatch = 8;                  // ... whose ids they request together
+static_assert(kCountingBlocks * kRankBlock < 1u << 16, "counts of half a word");
 constexpr uint32_t kHistPad = 32;                      // rows of the [expert][block] table are padded to this many blocks
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef int32_t i32x4a __attribute__((ext_vector_type(4), aligned(4)));
 #define MF_GLOBAL __attribute__((address_space(1)))
 
 // Lanes of the wave whose expert id equals mine (among lanes with valid == true).
@@ -70,7 +76,7 @@ __device__ __forceinline__ uint32_t BitsFor(uint32_t experts)
 }
 
 // Slice s of a block holds entries [block*1024 + s*64, +64), lane = offset in the slice.
-// Wave w of the workgroup handles slices w, w+4, w+8, w+12.
+// Wave w of the workgroup handles slice w.
 // hist[s][e] = number of entries of slice s routed to expert e.
 __device__ __forceinline__ void SliceHistograms(const int32_t *__restrict__ topk, uint32_t total, uint32_t experts,
                                                 uint32_t blockBase, uint32_t *hist /* [kRankSlices][experts] in LDS */,
@@ -114,7 +120,8 @@ __device__ __forceinline__ void SliceHistograms(const int32_t *__restrict__ topk
 // leaves them in the last-level cache (256 MiB, in front of HBM) for the permute: it then streams its stores without
 // the eleventh part of reads from HBM between them.  8192 tokens of 7168 elements at top-8, rows not in that cache before: dispatch
 // 191 against 218 us; 16 384 tokens 375 against 413.  Rows that are there already gain nothing from it: dispatch and combine of the same
-// 117 MB 352 against 350 us with 128 workgroups (dispatch alone 184 against 178), 356 with 1024, which read no faster (191 and 189 us).
+// 117 MB 352 against 350 us (dispatch alone 184 against 178).  128 workgroups of sixteen waves: with 64 / 32 of them dispatch takes 203 / 239 us,
+// with 128 of four waves 195, with 128 of sixteen 189.
 // Rows below kWarmMinBytes are the likelier to be there (94 us for 58 MB in turn with two others, 97 with this); beyond
 // kWarmMaxBytes the first rows would be gone again before their turn.
 constexpr uint64_t kWarmMinBytes = 80ull << 20;
@@ -202,32 +209,27 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
     const bool tabled = blockHist != nullptr;
     const bool counting = !tabled;
     const uint32_t steps = runOrder != nullptr ? kRankSlices / stepSlices : 0;
-    uint32_t *others = cum + steps * experts;             // [2][experts], counting only
-    for (uint32_t i = threadIdx.x; counting && i < 2 * experts; i += kRankThreads) {
+    uint32_t *others = cum + steps * experts;             // [experts], counting only
+    for (uint32_t i = threadIdx.x; counting && i < experts; i += kRankThreads) {
         others[i] = 0;
     }
     SliceHistograms(topk, total, experts, blockIdx.x * kRankBlock, hist, myExpert, myRank, &bad);
     if (counting) {
-        const uint32_t blockBase = blockIdx.x * kRankBlock;
-        for (uint32_t start = 0; start < total; start += kRankBlock) {
-            if (start == blockBase) {
-                continue;
-            }
-            int32_t id[kRankRounds];
+        // One word per expert, entries of the blocks before this one above entries of all others (kCountingBlocks * kRankBlock
+        // fit 16 bits).  The ids of eight blocks are requested before the first is counted: with a round trip per block, 1024 tokens
+        // took 15.9 us per dispatch, so 14.5.
+        for (uint32_t from = 0; from < blocks; from += kCountingBatch) {
+            int32_t id[kCountingBatch];
 #pragma unroll
-            for (uint32_t q = 0; q < kRankRounds; ++q) {
-                const uint32_t idx = start + q * kRankThreads + threadIdx.x;
-                id[q] = idx < total ? topk[idx] : 0;
+            for (uint32_t q = 0; q < kCountingBatch; ++q) {
+                const uint32_t at = (from + q) * kRankBlock + threadIdx.x;
+                id[q] = at < total ? topk[at] : 0;
             }
 #pragma unroll
-            for (uint32_t q = 0; q < kRankRounds; ++q) {
-                const uint32_t idx = start + q * kRankThreads + threadIdx.x;
-                if (idx < total) {
-                    if (id[q] >= 0 && static_cast<uint32_t>(id[q]) < experts) {
-                        atomicAdd(&others[id[q]], 1u);
-                        if (start < blockBase) {
-                            atomicAdd(&others[experts + id[q]], 1u);
-                        }
+            for (uint32_t q = 0; q < kCountingBatch; ++q) {
+                if (from + q != blockIdx.x && (from + q) * kRankBlock + threadIdx.x < total) {
+                    if (static_cast<uint32_t>(id[q]) < experts) {
+                        atomicAdd(&others[id[q]], from + q < blockIdx.x ? 0x10001u : 1u);
                     } else {
                         bad = 1;
                     }
@@ -247,16 +249,16 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
         }
     }
     // totals and "entries of earlier blocks" per expert
-    uint32_t tot[kMaxExperts / kRankThreads];
-    uint32_t before[kMaxExperts / kRankThreads];
+    uint32_t tot[(kMaxExperts + kRankThreads - 1) / kRankThreads];
+    uint32_t before[(kMaxExperts + kRankThreads - 1) / kRankThreads];
     uint32_t mine = 0;
 #pragma unroll
-    for (uint32_t j = 0; j < kMaxExperts / kRankThreads; ++j) {
+    for (uint32_t j = 0; j < (kMaxExperts + kRankThreads - 1) / kRankThreads; ++j) {
         // thread t owns the contiguous experts t*per .. t*per+per-1 so that a scan over threads is a scan over experts
         tot[j] = 0;
         before[j] = 0;
     }
-    const uint32_t per = (experts + kRankThreads - 1) / kRankThreads;  // 1 or 2
+    const uint32_t per = (experts + kRankThreads - 1) / kRankThreads;
     for (uint32_t j = 0; j < per; ++j) {
         const uint32_t x = threadIdx.x * per + j;
         if (x < experts) {
@@ -264,12 +266,13 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
             const uint32_t *rowHist = blockHist + static_cast<uint64_t>(x) * histStride;
             uint32_t t = 0;
             uint32_t b = 0;
-            for (uint32_t sl = 0; !tabled && sl < kRankSlices; ++sl) {
-                t += hist[sl * experts + x];
-            }
             if (counting) {
-                t += others[x];
-                b = others[experts + x];
+#pragma unroll
+                for (uint32_t sl = 0; sl < kRankSlices; ++sl) {
+                    t += hist[sl * experts + x];
+                }
+                t += others[x] & 0xFFFFu;
+                b = others[x] >> 16;
             }
             // kHistPad blocks per step, all their loads requested before the first is used (with one load per step the
             // loop waited a round trip per four blocks)
@@ -293,7 +296,7 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
             mine += t;
         }
     }
-    // exclusive scan of `mine` over the 256 threads: shuffles inside each wave, LDS across the four waves
+    // exclusive scan of `mine` over the threads: shuffles inside each wave, LDS across the waves
     uint32_t incl = mine;
 #pragma unroll
     for (uint32_t step = 1; step < 64; step <<= 1) {
@@ -328,10 +331,15 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
     for (uint32_t x = threadIdx.x; x < experts; x += kRankThreads) {
         uint32_t acc = base[x];
         uint32_t stepStart = acc;
+        uint32_t v[kRankSlices];                          // all read before the first is replaced
+#pragma unroll
         for (uint32_t s = 0; s < kRankSlices; ++s) {
-            const uint32_t v = hist[s * experts + x];
+            v[s] = hist[s * experts + x];
+        }
+#pragma unroll
+        for (uint32_t s = 0; s < kRankSlices; ++s) {
             hist[s * experts + x] = acc;
-            acc += v;
+            acc += v[s];
             if (steps != 0 && (s + 1) % stepSlices == 0) {
                 cum[(s / stepSlices) * experts + x] = acc - stepStart;
                 stepStart = acc;
@@ -611,7 +619,6 @@ constexpr uint32_t kSmallHold = 2;                      // 128-bit pieces of the
 constexpr uint32_t kSmallEntries = 4096;                // the largest such call
 constexpr uint32_t kSmallGroups = 256;                  // rows are cut until there are so many workgroups, one per CU
 constexpr uint32_t kSmallBatch = 4;                     // ids per lane requested together by the counting workgroup
-typedef int32_t i32x4a __attribute__((ext_vector_type(4), aligned(4)));
 static_assert(kSmallEntries <= 1u << 16 && kMaxExperts <= 1u << 16, "an entry's expert and index share a word");
 
 // (expert, index) in one word; an id out of range comes behind every entry.
@@ -1121,14 +1128,13 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
                        hidden % 64 == 0 && static_cast<uint64_t>(stepEntries / topK + 1) * hidden * 2 <= 2200000ull &&
                        stepsPerBlock * experts <= 4096 && tileGrid <= 0x7FFFFFFFull;
     // Up to kCountingBlocks blocks rank without a histogram launch in front of them: every block counts the entries
-    // of the others itself.  1024 tokens of 7168 elements at top-8, 256 experts: 29.5 us per dispatch against 35.1 with the
-    // launch; 640 tokens over 512 experts 26 against 38.
-    // At sixteen blocks the two are level (50.5 us), at thirty-two the counting costs 10 us; over 8 or 16 experts,
-    // where the counts of a wave land on few LDS words, eight blocks are level (23.9 against 23.4 us) and sixteen
-    // lose 4 us.
-    const bool counting = blocks <= kCountingBlocks;
+    // of the others itself.  Dispatch of rows of 1024 elements, with the launch / so: 2200 tokens at top-8 over 256 experts (18 blocks)
+    // 20.1 / 17.6 us, 3000 (24) 19.7 / 18.3, 4096 (32) 22.2 / 22.0 (of 7168 elements 90.3 / 90.6).  The counts of a wave land on few LDS
+    // words when the experts are few: over 64, 12 blocks 15.7 / 13.8, 16 34.5 / 34.0, 24 63.6 / 63.9 (longer rows); over 8, 16 blocks
+    // 19.7 / 20.2.
+    const bool counting = blocks <= (experts >= 128 ? kCountingBlocks : experts >= 64 ? 16u : 8u);
     const size_t rankLds = histLds + (experts + kRankThreads + kRankSlices + (tiles ? stepsPerBlock * experts : 0) +
-                                      (counting ? 2 * experts : 0)) * sizeof(uint32_t);
+                                      (counting ? experts : 0)) * sizeof(uint32_t);
     const uint64_t tableBytes = 256 + histStride * sizeof(uint32_t) + static_cast<uint64_t>(histStride) * experts * sizeof(uint32_t);
     int2 *runOrder = tiles ? reinterpret_cast<int2 *>(static_cast<char *>(workspace) + (tableBytes + 15) / 16 * 16) : nullptr;
     const uint64_t rowBytes = static_cast<uint64_t>(upr) * 16;

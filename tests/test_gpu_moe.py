@@ -483,3 +483,14 @@ def test_combine_of_any_values(gpu, oracle, T, H, K):
     finally:
         for b in bufs + [y]:
             b.free()
+
+
+@pytest.mark.parametrize("T,K,E", [
+    (3072, 8, 256), (3073, 8, 256),     # 24 blocks that count, 25 with a histogram launch
+    (4097, 4, 128), (1229, 7, 130),     # 17 blocks, the last of 4 entries; 9 blocks
+    (2048, 8, 64), (2049, 8, 64),       # fewer experts: up to 16 blocks
+    (1024, 8, 63), (1025, 8, 63),       # fewer yet: up to 8
+    (3000, 8, 512), (9000, 1, 200),     # the widest table; one entry per token
+])
+def test_more_blocks_that_count_one_anothers_entries(gpu, oracle, T, K, E):
+    test_few_blocks_that_count_one_anothers_entries(gpu, oracle, T, K, E)
