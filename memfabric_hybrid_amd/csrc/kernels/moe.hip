@@ -717,6 +717,7 @@ __global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(const u3
     // An entry as one word, expert above index: what comes before the token's slots is what compares below their words.
     // Every wave looks at a quarter of the ids, for all slots.
     const uint32_t first = token * topK;
+    const int32_t idOfLane = threadIdx.x < topK ? topk[first + threadIdx.x] : -1;
     uint32_t own[kSlots];
     uint32_t before[kSlots];
 #pragma unroll
@@ -761,7 +762,7 @@ __global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(const u3
         for (uint32_t w = 0; w < kSmallThreads / 64; ++w) {
             row += lds[kMaxTopK * (1 + w) + threadIdx.x];
         }
-        lds[threadIdx.x] = static_cast<uint32_t>(topk[first + threadIdx.x]) < experts ? row : 0xFFFFFFFFu;
+        lds[threadIdx.x] = static_cast<uint32_t>(idOfLane) < experts ? row : 0xFFFFFFFFu;
     }
     __syncthreads();
     if (part == 0 && threadIdx.x < topK) {
