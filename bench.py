@@ -589,7 +589,7 @@ def extras_paged(lib):
         assert p and lib.mfrt_memcpy(p, t.ctypes.data, t.nbytes) == 0
         return p
 
-    # the same gather with its {src, dst, len} table resident in device memory (the plugin ABI's other legal form): planned on the GPU
+    # the same gather with its {src, dst, len} table resident in device memory (the plugin ABI's other legal form)
     ids = workloads.page_ids(0xC3, pool_bytes // page, count)
     tab = device_table(pool + ids * page, buf + np.arange(count, dtype=np.uint64) * page, np.full(count, page))
     us, _ = timer.run(lambda: lib.mf_xcopy_device_table(tab, count, native.ROUTE_HBM, None), 40, warm=10)
@@ -641,9 +641,8 @@ def extras_paged(lib):
         lib.mfrt_device_sync()
         lib.mfrt_free_device(tab)
         lib.mfrt_free_device(big)
-    table_path["note"] = ("device_table_*: mf_xcopy_device_table, the table planned on the GPU (chunk prefix, group map, and the repeating chunk "
-                          "counts of equal pages found there) in one launch up to 8192 segments, two beyond, in front of the copy launch; "
-                          "ragged_16384: mf_xcopy_batch from host arrays (descriptors, prefix and group map uploaded by a launch of its own) "
+    table_path["note"] = ("device_table_*: mf_xcopy_device_table, the table copied without a plan and a second launch for what long segments hold "
+                          "beyond their share; ragged_16384: mf_xcopy_batch from host arrays (cut into pieces by the host) "
                           "and the same table resident in device memory")
     res["table_path"] = table_path
     lib.mfrt_free_device(pool)
