@@ -107,3 +107,16 @@ def test_staged_copies_of_pageable_memory(lib, pool, way, sizes):
         assert np.array_equal(_read(lib, dev, room), image)
     finally:
         big.destroy()
+
+
+LEAST_ROUND = 576 << 10
+
+
+@pytest.mark.parametrize("way", ["load", "save"])
+@pytest.mark.parametrize("sizes", [
+    [LEAST_ROUND], [LEAST_ROUND + 1], [3 * LEAST_ROUND // 2], [3 * LEAST_ROUND // 2 + 1],   # one round, as much as one takes, the first of two
+    [5 * LEAST_ROUND // 2, 1], [130001] * 7, [LEAST_ROUND - 1, 1, 2 * LEAST_ROUND],         # the second's end, padded parts
+    [1] * 9000, [(8 << 20) + 64, (4 << 20) - 1],                                            # padding alone, the longest rounds
+], ids=lambda s: f"{len(s)}x{s[0]}")
+def test_staged_copies_at_the_edges_of_rounds(lib, pool, way, sizes):
+    test_staged_copies_of_pageable_memory(lib, pool, way, sizes)
