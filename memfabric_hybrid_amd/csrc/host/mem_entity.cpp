@@ -5,6 +5,8 @@
 #include <immintrin.h>
 #endif
 #include <cstring>
+#include <memory>
+#include <new>
 #include <thread>
 
 #include "../rt/mf_rt.h"
@@ -586,7 +588,7 @@ uint32_t MemEntity::FirstOutside(void *const *ptrs, const uint64_t *lengths, uin
     return n;
 }
 
-void MemEntity::LocateAddrAndRank(void *&src, void *&dest, uint64_t length, std::pair<uint32_t, uint32_t> &ranks) const
+std::pair<uint32_t, uint32_t> MemEntity::RanksOf(const void *src, const void *dest, uint64_t length) const
 {
     auto owner = [&](uint64_t a) -> uint32_t {
         bool inside = false;
@@ -596,13 +598,28 @@ void MemEntity::LocateAddrAndRank(void *&src, void *&dest, uint64_t length, std:
         }
         return device_.RankByStride(a, length, options_.rankId, inside);
     };
-    ranks.first = owner(reinterpret_cast<uint64_t>(src));
-    src = reinterpret_cast<void *>(Mask48(reinterpret_cast<uint64_t>(src)));
-    ranks.second = owner(reinterpret_cast<uint64_t>(dest));
-    dest = reinterpret_cast<void *>(Mask48(reinterpret_cast<uint64_t>(dest)));
+    return {owner(reinterpret_cast<uint64_t>(src)), owner(reinterpret_cast<uint64_t>(dest))};
 }
 
-int MemEntity::CopyData(hybm_copy_params &params, hybm_data_copy_direction direction, void *stream, uint32_t flags)
+namespace {
+
+void *PlainAddress(const void *p)
+{
+    return reinterpret_cast<void *>(Mask48(reinterpret_cast<uint64_t>(p)));
+}
+
+bool AnyTagged(void *const *a, void *const *b, uint32_t n)
+{
+    uint64_t bits = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        bits |= reinterpret_cast<uint64_t>(a[i]) | reinterpret_cast<uint64_t>(b[i]);
+    }
+    return bits != Mask48(bits);
+}
+
+}  // namespace
+
+int MemEntity::CopyData(const hybm_copy_params &params, hybm_data_copy_direction direction, void *stream, uint32_t flags)
 {
     if (!initialized_) {
         return BM_NOT_INITIALIZED;
@@ -613,17 +630,17 @@ int MemEntity::CopyData(hybm_copy_params &params, hybm_data_copy_direction direc
     if (mfrt_bind_thread() != 0) {
         return BM_ERROR;
     }
-    std::pair<uint32_t, uint32_t> ranks;
-    LocateAddrAndRank(params.src, params.dest, params.dataSize, ranks);
+    const std::pair<uint32_t, uint32_t> ranks = RanksOf(params.src, params.dest, params.dataSize);
     ExtOptions options{};
     options.flags = flags;
     options.stream = stream;
     options.srcRankId = ranks.first;
     options.destRankId = ranks.second;
-    return dataOperator_->DataCopy(params, direction, options);
+    hybm_copy_params plain{PlainAddress(params.src), PlainAddress(params.dest), params.dataSize};
+    return dataOperator_->DataCopy(plain, direction, options);
 }
 
-int MemEntity::BatchCopyData(hybm_batch_copy_params &params, hybm_data_copy_direction direction, void *stream,
+int MemEntity::BatchCopyData(const hybm_batch_copy_params &params, hybm_data_copy_direction direction, void *stream,
                              uint32_t flags)
 {
     if (!initialized_) {
@@ -640,22 +657,29 @@ int MemEntity::BatchCopyData(hybm_batch_copy_params &params, hybm_data_copy_dire
     options.flags = flags;
     options.srcRankId = options_.rankId;
     options.destRankId = options_.rankId;
-    if (options_.rankCount > 1) {
-        for (uint32_t i = 0; i < params.batchSize; ++i) {
-            std::pair<uint32_t, uint32_t> ranks;
-            LocateAddrAndRank(params.sources[i], params.destinations[i], params.dataSizes[i], ranks);
-            options.groupMap[ranks].push_back(i);
-        }
-    } else {
-        // One rank: every element belongs to the pair (rank, rank).  The
-        // addresses are still normalised in place as callers may rely on it.
-        for (uint32_t i = 0; i < params.batchSize; ++i) {
-            params.sources[i] = reinterpret_cast<void *>(Mask48(reinterpret_cast<uint64_t>(params.sources[i])));
-            params.destinations[i] =
-                reinterpret_cast<void *>(Mask48(reinterpret_cast<uint64_t>(params.destinations[i])));
+    const uint32_t n = params.batchSize;
+    if (options_.rankCount > 1) {   // with one rank every element belongs to the pair (rank, rank)
+        for (uint32_t i = 0; i < n; ++i) {
+            options.groupMap[RanksOf(params.sources[i], params.destinations[i], params.dataSizes[i])].push_back(i);
         }
     }
-    return dataOperator_->BatchDataCopy(params, direction, options);
+    hybm_batch_copy_params plain = params;
+    if (!AnyTagged(params.sources, params.destinations, n)) {
+        return dataOperator_->BatchDataCopy(plain, direction, options);
+    }
+    // Addresses with bits above the lower 48 lose them in a copy of the arrays: the caller's may be read-only, or in use by
+    // another thread.
+    std::unique_ptr<void *[]> addresses(new (std::nothrow) void *[2ull * n]);
+    if (addresses == nullptr) {
+        MF_FAIL(BM_MALLOC_FAILED, "no memory for the addresses of " << n << " elements");
+    }
+    plain.sources = addresses.get();
+    plain.destinations = addresses.get() + n;
+    for (uint32_t i = 0; i < n; ++i) {
+        plain.sources[i] = PlainAddress(params.sources[i]);
+        plain.destinations[i] = PlainAddress(params.destinations[i]);
+    }
+    return dataOperator_->BatchDataCopy(plain, direction, options);
 }
 
 int MemEntity::Wait()

@@ -81,10 +81,11 @@ public:
     // The same test for every element of a batch in one pass; the index of the first element that
     // is null or leaves the entity, n when all are inside.
     uint32_t FirstOutside(void *const *ptrs, const uint64_t *lengths, uint32_t n) const;
-    void LocateAddrAndRank(void *&src, void *&dest, uint64_t length, std::pair<uint32_t, uint32_t> &ranks) const;
+    std::pair<uint32_t, uint32_t> RanksOf(const void *src, const void *dest, uint64_t length) const;
 
-    int CopyData(hybm_copy_params &params, hybm_data_copy_direction direction, void *stream, uint32_t flags);
-    int BatchCopyData(hybm_batch_copy_params &params, hybm_data_copy_direction direction, void *stream, uint32_t flags);
+    // Neither writes to what the caller has passed.
+    int CopyData(const hybm_copy_params &params, hybm_data_copy_direction direction, void *stream, uint32_t flags);
+    int BatchCopyData(const hybm_batch_copy_params &params, hybm_data_copy_direction direction, void *stream, uint32_t flags);
     int Wait();
 
     const hybm_options &Options() const

@@ -3,8 +3,8 @@
 //
 // What it replaces: a ctypes array filled element by element costs 40 to 60 ns an element (a 122-segment batch
 // 15 us of interpreter before a 4.4 us copy, 4096 pages in numpy arrays 700 us before a 50 us copy).  Here an int
-// of a list is read where it lies (about 1 ns), and an array of 64-bit integers is handed to the library as it is.
-// The interpreter lock is released for the call itself, as ctypes does; while it is, an array that was handed over must
+// of a list is read where it lies (about 1 ns), and an array of 64-bit integers, which may be read-only, is handed to the
+// library as it is: the library only reads it.  The interpreter lock is released for the call itself, as ctypes does; while it is, an array that was handed over must
 // not be written to by another thread (the rule of the C API's own arrays).
 //
 // The words of the sequences of one call live in a per-thread workspace that is kept between calls up to

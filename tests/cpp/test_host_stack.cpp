@@ -13,6 +13,7 @@
 #include <vector>
 
 #include <sched.h>
+#include <sys/mman.h>
 
 #include "../../include/mf_hip_dataplane_internal.h"
 #include "../../include/mf_xcopy_api.h"
@@ -336,6 +337,47 @@ static void TestCApi()
 // (test/ut/testcase/smem/smem_trans_test.cpp:145-168 create, :170-219 register, :1016-1098 batch
 // write); the data cases follow its two-object write / read tests (:272-373, :655-779) with both
 // objects in this process.
+// The arrays of a batch belong to the caller: they may lie in read-only memory, and addresses that carry bits above the
+// lower 48 (local memory only; pool addresses are checked as they are) lose them on the way, not in the arrays.
+static void TestBatchArraysAreOnlyRead()
+{
+    const uint64_t pool = 8ull << 20;
+    smem_bm_config_t cfg;
+    CHECK(smem_bm_config_init(&cfg) == SM_OK);
+    CHECK(smem_bm_init("tcp://127.0.0.1:1", 1, 0, &cfg) == SM_OK);
+    smem_bm_t bm = smem_bm_create(2, 1, SMEMB_DATA_OP_SDMA, pool, pool, 0);
+    CHECK(bm != nullptr && smem_bm_join(bm, 0) == SM_OK);
+    uint8_t *dev = static_cast<uint8_t *>(smem_bm_ptr_by_mem_type(bm, SMEM_MEM_TYPE_DEVICE, 0));
+    std::vector<uint8_t> local(4u << 20);
+    Fill(local, 11);
+    constexpr uint64_t kTag = 0x5A5Aull << 48;
+    for (uint32_t n : {1u, 128u, 129u, 1000u}) {
+        for (uint64_t tag : {static_cast<uint64_t>(0), kTag}) {
+            const size_t bytes = (24ull * n + 4095) / 4096 * 4096;
+            auto *words = static_cast<uint64_t *>(mmap(nullptr, bytes, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0));
+            CHECK(words != MAP_FAILED);
+            for (uint32_t i = 0; i < n; ++i) {
+                words[i] = (reinterpret_cast<uint64_t>(local.data()) + 4000ull * i) | (i % 3 == 0 ? tag : 0);
+                words[n + i] = reinterpret_cast<uint64_t>(dev) + 4096ull * i;
+                words[2 * n + i] = 3999;
+            }
+            CHECK(mprotect(words, bytes, PROT_READ) == 0);
+            std::memset(dev, 0, pool);
+            auto **from = reinterpret_cast<void **>(words);
+            smem_batch_copy_params bp{from, from + n, words + 2 * n, n};
+            CHECK(smem_bm_copy_batch(bm, &bp, SMEMB_COPY_H2G, 0) == SM_OK);
+            bool same = true;
+            for (uint32_t i = 0; i < n; ++i) {
+                same = same && std::memcmp(dev + 4096ull * i, local.data() + 4000ull * i, 3999) == 0 && dev[4096ull * i + 3999] == 0;
+            }
+            CHECK(same);
+            munmap(words, bytes);
+        }
+    }
+    smem_bm_destroy(bm);
+    smem_bm_uninit(0);
+}
+
 // Launch cost per CPU and the pinning built on it: every CPU of the thread's set is measured, the set is put back,
 // and the pinned set is a part of it.
 static void TestHostLaunchCosts()
@@ -1680,6 +1722,7 @@ int main()
     setenv("MF_HIP_GVA_WINDOW", "malloc", 1);
     TestCApi();                                  // device window: one ordinary allocation
     unsetenv("MF_HIP_GVA_WINDOW");
+    TestBatchArraysAreOnlyRead();
     TestTrans();
     TestLeases();
     TestMappedWindow();

@@ -94,3 +94,30 @@ def test_batch_copy_from_every_kind_of_sequence(lib, kind, n):
     finally:
         pool.destroy()
         bm.uninitialize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 128, 129, 4000])
+def test_arrays_of_a_batch_are_only_read(lib, tmp_path, n):
+    """Addresses in a read-only map of a file and in a bytes object, some with bits above the lower 48."""
+    assert bm.initialize("tcp://127.0.0.1:0", 1, 0) == 0, native.last_error()
+    pool = bm.create(1, 0, 32 << 20)
+    try:
+        dev = pool.peer_rank_ptr(0)
+        local = np.random.default_rng(n).integers(0, 256, (n, 2048), dtype=np.uint8)
+        source = np.uint64(local.ctypes.data) + np.arange(n, dtype=np.uint64) * np.uint64(2048)
+        source[::3] |= np.uint64(0x5A5A << 48)
+        target = np.uint64(dev) + np.arange(n, dtype=np.uint64) * np.uint64(4096)
+        target.tofile(tmp_path / "targets")
+        for sources in (memoryview(source.tobytes()).cast("Q"), source):
+            kept = bytes(sources)
+            assert lib.mfrt_memset(dev, 0, 32 << 20) == 0
+            targets = np.memmap(tmp_path / "targets", dtype=np.uint64, mode="r")
+            assert pool.copy_data_batch(sources, targets, np.full(n, 2047), n, bm.BmCopyType.H2G) == 0, native.last_error()
+            after = np.empty((n, 4096), dtype=np.uint8)
+            assert lib.mfrt_memcpy(after.ctypes.data, dev, after.nbytes) == 0
+            assert np.array_equal(after[:, :2047], local[:, :2047]) and not after[:, 2047:].any()
+            assert bytes(sources) == kept
+    finally:
+        pool.destroy()
+        bm.uninitialize()
