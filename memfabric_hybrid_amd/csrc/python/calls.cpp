@@ -7,8 +7,8 @@
 // library as it is: the library only reads it.  The interpreter lock is released for the call itself, as ctypes does; while it is, an array that was handed over must
 // not be written to by another thread (the rule of the C API's own arrays).
 //
-// The words of the sequences of one call live in a per-thread workspace that is kept between calls up to
-// kKeptWords and given back when the thread ends.  The module is linked against libmf_hip_dataplane.so.
+// The words of the sequences of one call live in a workspace that the thread keeps between calls, up to kKeptWords, until it ends.
+// A call takes it out of the thread's hands: an element's __int__ may make a batch call of its own.  The module is linked against libmf_hip_dataplane.so.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #if PY_VERSION_HEX < 0x030C0000
@@ -19,6 +19,7 @@
 #include <cstring>
 #include <memory>
 #include <new>
+#include <utility>
 
 #include "../../../include/mf_xcopy_api.h"
 
@@ -31,25 +32,17 @@ struct Workspace {
     std::unique_ptr<uint64_t[]> words;
     size_t capacity = 0;
 
-    uint64_t *Take(size_t n)
+    uint64_t *Room(size_t n)
     {
         if (n > capacity) {
             words.reset();
-            capacity = 0;
             words.reset(new (std::nothrow) uint64_t[n]);
             capacity = words ? n : 0;
         }
         return words.get();
     }
-    void Trim()
-    {
-        if (capacity > kKeptWords) {
-            words.reset();
-            capacity = 0;
-        }
-    }
 };
-thread_local Workspace t_workspace;
+thread_local Workspace t_workspace;   // what the thread's last call has left; empty while a call uses it
 
 inline uint64_t WordOfInt(PyObject *o)   // an int, modulo 2^64
 {
@@ -205,13 +198,18 @@ private:
     size_t count_ = 0;
 };
 
-// The three sequences of a batch.  Close() (or the destructor) gives an outsized workspace back.
+// The three sequences of a batch.
 class Batch {
 public:
+    Batch() : workspace_(std::exchange(t_workspace, Workspace{})) {}
     ~Batch()
     {
-        t_workspace.Trim();
+        if (workspace_.capacity <= kKeptWords && workspace_.capacity > t_workspace.capacity) {
+            t_workspace = std::move(workspace_);
+        }
     }
+    Batch(const Batch &) = delete;
+    Batch &operator=(const Batch &) = delete;
     bool Open(PyObject *a, PyObject *b, PyObject *c)
     {
         return words_[0].Open(a) && words_[1].Open(b) && words_[2].Open(c);
@@ -226,7 +224,7 @@ public:
         for (const Words &w : words_) {
             needed += w.NeedsRoom() ? n : 0;
         }
-        uint64_t *room = t_workspace.Take(needed);
+        uint64_t *room = workspace_.Room(needed);
         if (room == nullptr) {
             PyErr_NoMemory();
             return false;
@@ -254,6 +252,7 @@ public:
     }
 
 private:
+    Workspace workspace_;
     Words words_[3];
     const uint64_t *at_[3] = {};
 };

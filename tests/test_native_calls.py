@@ -2,6 +2,9 @@
 
 import array
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -55,6 +58,29 @@ def test_a_list_that_changes_while_it_is_read(lib):
     values[0] = Shrinks()
     with pytest.raises(RuntimeError):
         native.calls().fill((ctypes.c_uint64 * 3)(), values)
+
+
+NESTED = """
+from memfabric_hybrid_amd import bm
+pool = bm.BigMemory(0x1000)
+class Nests:
+    def __int__(self):
+        pool.copy_data_batch([7] * {inner}, [7] * {inner}, [7] * {inner}, {inner}, bm.BmCopyType.G2G)
+        return 1
+words = [1] * {outer}
+words[{outer} // 2] = Nests()
+for _ in range(3):
+    print(pool.copy_data_batch(words, [2] * {outer}, [3] * {outer}, {outer}, bm.BmCopyType.G2G))
+"""
+
+
+@pytest.mark.parametrize("outer, inner", [(60000, 400000), (400000, 60000), (1000, 2000), (2000, 1000)])
+def test_a_batch_call_inside_a_batch_call(lib, outer, inner):
+    """The inner call outgrows, or leaves alone, the words the outer one is filling; in a process of its own."""
+    done = subprocess.run([sys.executable, "-c", NESTED.format(outer=outer, inner=inner)], capture_output=True, text=True,
+                          cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), timeout=120)
+    assert done.returncode == 0, done.stderr[-2000:]
+    assert done.stdout.split() == [str(native.SM_NOT_INITIALIZED)] * 3
 
 
 def test_codes_without_a_pool_or_a_session(lib):
@@ -118,6 +144,42 @@ def test_arrays_of_a_batch_are_only_read(lib, tmp_path, n):
             assert lib.mfrt_memcpy(after.ctypes.data, dev, after.nbytes) == 0
             assert np.array_equal(after[:, :2047], local[:, :2047]) and not after[:, 2047:].any()
             assert bytes(sources) == kept
+    finally:
+        pool.destroy()
+        bm.uninitialize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("outer, inner", [(300, 200), (300, 3000)])
+def test_a_batch_call_inside_a_batch_call_copies_both(lib, outer, inner):
+    assert bm.initialize("tcp://127.0.0.1:0", 1, 0) == 0, native.last_error()
+    pool = bm.create(1, 0, 32 << 20)
+    try:
+        dev = pool.peer_rank_ptr(0)
+        before = np.random.default_rng(outer + inner).integers(0, 256, 32 << 20, dtype=np.uint8)
+        assert lib.mfrt_memcpy(dev, before.ctypes.data, before.nbytes) == 0
+        after = before.copy()
+
+        def words(n, source, target):
+            for i in range(n):
+                after[target + 1024 * i:target + 1024 * i + 1000] = before[source + 1024 * i:source + 1024 * i + 1000]
+            return [dev + source + 1024 * i for i in range(n)], [dev + target + 1024 * i for i in range(n)], [1000] * n
+
+        nested = words(inner, 4 << 20, 16 << 20)
+        sources, targets, sizes = words(outer, 0, 24 << 20)
+
+        class Nests:
+            def __init__(self, value):
+                self.value = value
+
+            def __int__(self):
+                assert pool.copy_data_batch(*nested, inner, bm.BmCopyType.G2G) == 0, native.last_error()
+                return self.value
+        sources[outer // 2] = Nests(sources[outer // 2])
+        assert pool.copy_data_batch(sources, targets, sizes, outer, bm.BmCopyType.G2G) == 0, native.last_error()
+        got = np.empty_like(before)
+        assert lib.mfrt_memcpy(got.ctypes.data, dev, got.nbytes) == 0
+        assert np.array_equal(got, after)
     finally:
         pool.destroy()
         bm.uninitialize()
