@@ -9,6 +9,8 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import sys
+import sysconfig
 import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -16,7 +18,8 @@ LIB_DIR = os.path.join(_HERE, "lib")
 DATAPLANE_PATH = os.path.join(LIB_DIR, "libmf_hip_dataplane.so")
 PLUGIN_PATH = os.path.join(LIB_DIR, "libmf_hybm_copy_extend.so")
 YARDSTICK_PATH = os.path.join(LIB_DIR, "libmf_hip_yardstick.so")
-CALLS_PATH = os.path.join(LIB_DIR, "_calls.so")
+# an extension module reads the interpreter's objects: one per interpreter version, told apart by the file's name
+CALLS_PATH = os.path.join(LIB_DIR, "_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 # ---- enums (values pinned in include/mf_xcopy_types.h) ---------------------
 BM_OK = 0
@@ -361,7 +364,8 @@ def calls():
         with _lock:
             if _calls is None:
                 if not os.path.exists(CALLS_PATH):
-                    raise OSError(f"{CALLS_PATH} is missing: build it with `make -C memfabric_hybrid_amd/csrc`")
+                    raise OSError(f"{CALLS_PATH} is missing: build it for this interpreter with `make -C memfabric_hybrid_amd/csrc "
+                                  f"PYTHON={sys.executable}`")
                 loader = importlib.machinery.ExtensionFileLoader("_calls", CALLS_PATH)
                 module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_calls", loader))
                 loader.exec_module(module)

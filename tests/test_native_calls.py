@@ -3,6 +3,7 @@
 import array
 import ctypes
 import os
+import shutil
 import subprocess
 import sys
 
@@ -58,6 +59,21 @@ def test_a_list_that_changes_while_it_is_read(lib):
     values[0] = Shrinks()
     with pytest.raises(RuntimeError):
         native.calls().fill((ctypes.c_uint64 * 3)(), values)
+
+
+def test_a_module_built_for_another_interpreter_is_not_loaded(lib, tmp_path):
+    """The module reads the layout of the interpreter's integers: a file without this interpreter's tag stays unused."""
+    package = os.path.dirname(native.__file__)
+    there = tmp_path / "memfabric_hybrid_amd"
+    (there / "lib").mkdir(parents=True)
+    for name in ("__init__.py", "native.py"):
+        shutil.copy(os.path.join(package, name), there / name)
+    shutil.copy(native.DATAPLANE_PATH, there / "lib")
+    for name in ("_calls.so", "_calls.cpython-39-x86_64-linux-gnu.so"):
+        shutil.copy(native.CALLS_PATH, there / "lib" / name)
+    program = "from memfabric_hybrid_amd import native\ntry:\n    native.calls()\nexcept OSError as e:\n    print('refused', e)\n"
+    done = subprocess.run([sys.executable, "-c", program], capture_output=True, text=True, cwd=tmp_path, timeout=120)
+    assert done.returncode == 0 and done.stdout.startswith("refused"), (done.stdout, done.stderr[-2000:])
 
 
 NESTED = """
