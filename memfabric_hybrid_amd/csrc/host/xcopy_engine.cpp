@@ -57,6 +57,8 @@ struct ThreadLease {
     uint64_t *doneWord = nullptr;   // pinned; a one-lane launch stores doneSeq there behind a blocking copy
     uint32_t doneSeq = 0;
     void *doneCounter = nullptr;    // device memory, for launches that store the word themselves
+    void *graphRests = nullptr;     // kSlots RestLists for the device-table calls that become nodes of a graph: not those plain calls use
+    uint32_t graphCursor = 0;
     uint64_t pendingBytes = 0;      // bytes of the copies queued on `stream` since the thread last waited for it
     void *bounce = nullptr;
     uint64_t bounceBytes = 0;
@@ -113,6 +115,10 @@ struct ThreadLease {
         if (doneCounter != nullptr) {
             (void)mfrt_free_device(doneCounter);
             doneCounter = nullptr;
+        }
+        if (graphRests != nullptr) {
+            (void)mfrt_free_device(graphRests);
+            graphRests = nullptr;
         }
         for (uint32_t i = 0; i < XcopyEngine::kFanStreams; ++i) {
             if (fanEvent[i] != nullptr) {
@@ -566,8 +572,6 @@ int SealQueued(ThreadLease &ctx)
     return BM_OK;
 }
 
-// The kernels just launched on `stream` read `slot`.  Only launches on the lease's own stream wait
-// for a shared event: a caller's stream may be gone by the time the next launch comes.
 // The event a launch on `stream` should complete for its slot: launches on a caller's stream are guarded one by one, since nothing
 // says how long the stream lives; those on the thread's own stream several at a time, by an event recorded behind them.
 void *EventOfLaunch(const ThreadLease &ctx, const StagingSlot &slot, const void *stream)
@@ -575,6 +579,8 @@ void *EventOfLaunch(const ThreadLease &ctx, const StagingSlot &slot, const void 
     return stream != ctx.stream ? slot.event : nullptr;
 }
 
+// The kernels just launched on `stream` read `slot`.  Only launches on the lease's own stream wait
+// for a shared event: a caller's stream may be gone by the time the next launch comes.
 int MarkQueued(ThreadLease &ctx, StagingSlot *slot, void *stream, bool sealNow, bool attached = false)
 {
     if (attached) {   // its launch completes the slot's event
@@ -591,7 +597,9 @@ int MarkQueued(ThreadLease &ctx, StagingSlot *slot, void *stream, bool sealNow, 
     return sealNow || ctx.queued >= kGuardEvery ? SealQueued(ctx) : BM_OK;
 }
 
-// The next slot of the ring, free to be rewritten, with at least `bytes` of pinned host memory.
+// The next slot of the ring, free to be rewritten, with at least `bytes` of pinned host memory.  Not for launches that become nodes
+// of a graph: a replay would read what a later call has left in the slot, memory may not be allocated while a stream records, and
+// an event recorded there is none that anybody could wait for.
 int AcquireSlot(ThreadLease &ctx, uint64_t bytes, void *stream, StagingSlot *&out)
 {
     if (ctx.adopted) {
@@ -680,21 +688,29 @@ int EnsureDevice(StagingSlot &slot, uint64_t bytes)
     return BM_OK;
 }
 
-int EnsureRestList(StagingSlot &slot)
+void *RestListAt(void *lists, uint32_t i)
 {
-    if (slot.rest != nullptr) {
+    return static_cast<uint8_t *>(lists) + i * RoundUp(RestListBytes(kRestCapacity), 256);
+}
+
+int EnsureRestLists(void *&lists, uint32_t count)
+{
+    if (lists != nullptr) {
         return BM_OK;
     }
-    slot.rest = mfrt_alloc_device(RestListBytes(kRestCapacity));
-    if (slot.rest == nullptr) {
+    lists = mfrt_alloc_device(count * RoundUp(RestListBytes(kRestCapacity), 256));
+    if (lists == nullptr) {
         MF_FAIL(BM_MALLOC_FAILED, "list of " << kRestCapacity << " pieces could not be allocated in HBM");
     }
     // cleared once, on a stream of the engine: the caller's may be recording
     void *own = XcopyEngine::Instance().ThreadStream();
-    const int err = own == nullptr ? -1 : mfk_xcopy_signal(slot.rest, 0, own);   // one 64-bit word, both counts
+    int err = own == nullptr ? -1 : 0;
+    for (uint32_t i = 0; i < count && err == 0; ++i) {
+        err = mfk_xcopy_signal(RestListAt(lists, i), 0, own);   // one 64-bit word, both counts
+    }
     if (err != 0 || mfrt_stream_sync(own) != 0) {
-        (void)mfrt_free_device(slot.rest);
-        slot.rest = nullptr;
+        (void)mfrt_free_device(lists);
+        lists = nullptr;
         MF_FAIL(BM_ERROR, "list of pieces could not be cleared: " << mfrt_error_string(err));
     }
     return BM_OK;
@@ -1734,7 +1750,7 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
             units = mfk_xcopy_window_units();
         }
         const bool deep = !windowed && DeepHoldApplies(total, n, route, unordered);
-        if (deep && (apartBits & (kUnitBytes - 1)) != 0) {
+        if (deep && (apartBits & (kUnitBytes - 1)) != 0 && mfrt_stream_capturing(stream) == 0) {
             // as pieces: sixteen loads per lane of aligned units and what shifts them, with the table of the kernel arguments, take
             // more registers than sixteen waves per CU have (42 MB 17.5 us with straddling loads)
             const int ret = SubmitPieces(src, dst, len, n, total, kDeepUnits, stream, mask, maskValue, unordered);
@@ -1776,7 +1792,10 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
     }
 
     // Beyond the kernel arguments descriptors are built in a pinned slot, which is sized for n segments; merging can only make
-    // them fewer.
+    // them fewer.  A graph has no use for a slot.
+    if (mfrt_stream_capturing(stream) != 0) {
+        return SubmitRecorded(src, dst, len, n, route, stream, mask, maskValue);
+    }
     {
         uint64_t total = 0;
         uint64_t longest = 0;
@@ -1929,6 +1948,26 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
     return MarkQueued(lease, slot, stream, false);
 }
 
+// A batch that becomes part of a graph: launches of kInlineSegs segments, whose descriptors are copied into the graph with their
+// arguments.  (Every run fits the kernel arguments: it has at most kInlineSegs segments of at most kInlinePiece once merged and cut.)
+int XcopyEngine::SubmitRecorded(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, int route, void *stream,
+                                void *mask, uint32_t maskValue)
+{
+    SegList segs;
+    NormalizeSegments(src, dst, len, n, kInlinePiece, segs);
+    uint32_t at = 0;
+    do {
+        const uint32_t m = segs.Size() - at < kInlineSegs ? segs.Size() - at : kInlineSegs;
+        const int ret = SubmitOne(segs.src.data() + at, segs.dst.data() + at, segs.len.data() + at, m, route, stream,
+                                  at + m == segs.Size() ? mask : nullptr, maskValue, false, false);
+        if (ret != BM_OK) {
+            return ret;
+        }
+        at += m;
+    } while (at < segs.Size());
+    return BM_OK;
+}
+
 // A batch between HBM addresses in one launch of pieces; kNotLaunched where their list would outgrow the batch.
 int XcopyEngine::SubmitPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t total, uint32_t units,
                               void *stream, void *mask, uint32_t maskValue, bool unordered)
@@ -1967,16 +2006,15 @@ int XcopyEngine::SubmitPieces(const uint64_t *src, const uint64_t *dst, const ui
         (void)BuildInlinePlan(none, kXcopyThreads, empty);
         return mfk_xcopy_inline(&empty, MFRT_ROUTE_HBM, 1, mask, maskValue, stream, 0, 0) == 0 ? BM_OK : BM_ERROR;
     }
-    int attached = 0;
-    const int err = mfk_xcopy_pieces(pieces, count, total, units, mask, maskValue, stream, HoldForPieces(count, units, unordered),
-                                     EventOfLaunch(lease, *slot, stream), &attached);
+    void *event = EventOfLaunch(lease, *slot, stream);
+    const int err = mfk_xcopy_pieces(pieces, count, total, units, mask, maskValue, stream, HoldForPieces(count, units, unordered), event);
     if (err != 0) {
         (void)MarkQueued(lease, slot, stream, true);   // the launch may have gone out with only the word behind it failing
         MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(err));
     }
     g_launches.fetch_add(1, std::memory_order_relaxed);
     NotePending(stream, total);
-    return MarkQueued(lease, slot, stream, false, attached != 0);
+    return MarkQueued(lease, slot, stream, false, event != nullptr);
 }
 
 int XcopyEngine::SubmitDeviceTable(const void *triples, uint32_t n, int route, void *stream, void *mask,
@@ -2001,29 +2039,35 @@ int XcopyEngine::SubmitDeviceTable(const void *triples, uint32_t n, int route, v
         int err = mfk_xcopy_inline(&empty, route, 1, mask, maskValue, stream, 0, 0);
         return err == 0 ? BM_OK : BM_ERROR;
     }
-    // The list of long segments' pieces belongs to a slot: the next call of another stream gets another one.
+    // The list of long segments' pieces belongs to a slot: the next call of another stream gets another one.  Calls that become
+    // nodes of a graph have lists of their own, made by the thread's first call: a graph may be replayed beside plain calls.
     ThreadCtx &ctx = t_ctx;
     StagingSlot *slot = nullptr;
     ThreadLease &lease = ctx.Lease();
-    int ret = AcquireSlot(lease, 0, stream, slot);
-    if (ret == BM_OK) {
-        ret = EnsureRestList(*slot);
+    const bool recorded = mfrt_stream_capturing(stream) != 0;
+    int ret = EnsureRestLists(lease.graphRests, kSlots);
+    if (ret == BM_OK && !recorded) {
+        ret = AcquireSlot(lease, 0, stream, slot);
+        ret = ret == BM_OK ? EnsureRestLists(slot->rest, 1) : ret;
     }
     if (ret != BM_OK) {
         return ret;
     }
+    void *list = recorded ? RestListAt(lease.graphRests, lease.graphCursor++ % kSlots) : slot->rest;
+    void *event = recorded ? nullptr : EventOfLaunch(lease, *slot, stream);
     const uint32_t cu = mfrt_cu_count();
     const uint32_t units = ChooseUnits(0, cu, route, tuning_);   // sizes are only known on the GPU
-    int attached = 0;
     const int err = mfk_xcopy_direct(triples, n, units, route, DeviceTableGrid(n, cu, route, tuning_), DeviceTableRestGrid(cu, route, tuning_),
-                                     slot->rest, kRestCapacity, mask, maskValue, stream, EventOfLaunch(lease, *slot, stream), &attached);
+                                     list, kRestCapacity, mask, maskValue, stream, event);
     if (err != 0) {
-        (void)MarkQueued(lease, slot, stream, true);   // the first launch writes the list
+        if (!recorded) {
+            (void)MarkQueued(lease, slot, stream, true);   // the first launch writes the list
+        }
         MF_FAIL(BM_ERROR, "xcopy launch of a device table failed: " << mfrt_error_string(err));
     }
     g_launches.fetch_add(2, std::memory_order_relaxed);
     NotePending(stream, ~0ull);   // sizes unknown here: the next wait sleeps on the stream
-    return MarkQueued(lease, slot, stream, false, attached != 0);
+    return recorded ? BM_OK : MarkQueued(lease, slot, stream, false, event != nullptr);
 }
 
 #ifndef MF_RT_HIDDEN

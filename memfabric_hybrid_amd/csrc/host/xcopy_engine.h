@@ -210,6 +210,8 @@ private:
                    uint32_t &ticket);
     int SubmitPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t total, uint32_t units,
                      void *stream, void *mask, uint32_t maskValue, bool unordered);
+    int SubmitRecorded(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, int route, void *stream, void *mask,
+                       uint32_t maskValue);
     int SubmitInPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t total, int route,
                        void *stream, void *mask, uint32_t maskValue);
     int SubmitOne(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, int route, void *stream,

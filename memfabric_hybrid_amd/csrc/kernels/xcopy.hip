@@ -983,14 +983,6 @@ void LaunchWithEvent(Kernel kernel, uint32_t grid, uint32_t lanes, hipStream_t s
     }
 }
 
-// The event, unless the stream is recording a graph, where launches cannot carry one.
-hipEvent_t Attachable(void *event, hipStream_t stream)
-{
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const bool free = event != nullptr && hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
-    return free ? static_cast<hipEvent_t>(event) : nullptr;
-}
-
 template <uint32_t kLanes, uint32_t kUnits, bool kHold>
 void LaunchPieces(const Piece *pieces, uint32_t count, uint32_t ticks, hipStream_t stream, hipEvent_t event)
 {
@@ -1115,7 +1107,7 @@ extern "C" int mfk_xcopy_signal(void *word, uint32_t value, void *stream)
 // pieces: `count` mf::Piece of together `bytes` bytes, none longer than `units` units and the bytes beside them; holdNanos: what a
 // table of as many chunks would wait.
 extern "C" int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, void *mask, uint32_t maskValue,
-                                void *stream, uint32_t holdNanos, void *event, int *attached)
+                                void *stream, uint32_t holdNanos, void *event)
 {
     using namespace mf;
     if (pieces == nullptr || count == 0 || count > kPieceMaxCount || (units != 256 && units != 512 && units != 1024)) {
@@ -1124,8 +1116,7 @@ extern "C" int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t byt
     const Piece *p = static_cast<const Piece *>(pieces);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const uint32_t ticks = units != 512 ? HoldTicks(PieceHoldNanos(holdNanos, count, bytes, units)) : 0;
-    const hipEvent_t end = Attachable(event, s);
-    *attached = end != nullptr ? 1 : 0;
+    const hipEvent_t end = static_cast<hipEvent_t>(event);
     if (units == 256 && ticks != 0) {
         LaunchPieces<64, 4, true>(p, count, ticks, s, end);
     } else if (units == 256) {
@@ -1167,19 +1158,17 @@ extern "C" int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, 
 
 // rest: a RestList with room for `capacity` pieces, its counts 0.
 extern "C" int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *rest,
-                                uint32_t capacity, void *mask, uint32_t maskValue, void *stream, void *event, int *attached)
+                                uint32_t capacity, void *mask, uint32_t maskValue, void *stream, void *event)
 {
     using namespace mf;
     if (nseg == 0 || grid == 0 || restGrid == 0 || rest == nullptr || capacity == 0) {
         return -1;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const hipEvent_t end = Attachable(event, s);
-    *attached = end != nullptr ? 1 : 0;
     const int err = WithPolicy(PolicyOf(route), [&](auto ntLoad, auto store) {
         return LaunchDirect<decltype(ntLoad)::value, decltype(store)::value>(static_cast<const uint64_t *>(triples), nseg, units, grid, restGrid,
                                                                              LanesFor(units, route), static_cast<RestList *>(rest),
-                                                                             capacity, s, end);
+                                                                             capacity, s, static_cast<hipEvent_t>(event));
     });
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
@@ -1436,9 +1425,8 @@ extern "C" int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32
     if (guarded && g_staticUsed[dev] && g_staticLast[dev] != s && hipStreamWaitEvent(s, g_staticDone[dev], 0) != hipSuccess) {
         return static_cast<int>(hipGetLastError());
     }
-    int attached = 0;
     const int err = mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, g_scratchOf[dev], kStaticRestCapacity, nullptr, 0, stream,
-                                     nullptr, &attached);
+                                     nullptr);
     if (guarded && hipEventRecord(g_staticDone[dev], s) == hipSuccess) {
         g_staticLast[dev] = s;
         g_staticUsed[dev] = true;

@@ -55,6 +55,7 @@ int mfrt_window_last_error(void);                       /* failed step (1 create
 void *mfrt_stream_create(void);
 int mfrt_stream_destroy(void *stream);
 int mfrt_stream_sync(void *stream);
+int mfrt_stream_capturing(void *stream);                /* 1: launches on the stream become nodes of a HIP graph */
 int mfrt_device_sync(void);
 
 void *mfrt_event_create(void);
@@ -96,9 +97,9 @@ int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, 
 int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, void *mask, uint32_t maskValue, void *stream);
 /* HBM to HBM: `count` mf::Piece (kernels/xcopy_plan.h) in pinned host memory, of together `bytes` bytes and up to `units` (256, 512
  * or 1024) units each.  holdNanos: as for mfk_xcopy_inline; it is what a table of as many chunks would wait.
- * event (may be NULL): completes with the launch if *attached is 1 afterwards; it is not where the stream records a graph. */
+ * event (may be NULL): completes with the launch.  The stream must not be one that records a graph, whose launches cannot carry one. */
 int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, void *mask, uint32_t maskValue, void *stream,
-                     uint32_t holdNanos, void *event, int *attached);
+                     uint32_t holdNanos, void *event);
 /* Launches every copy kernel once on empty plans (a kernel's first launch is not capturable into a HIP graph). */
 int mfk_xcopy_prelaunch(void *stream);
 /* Times the calibration workloads on `stream` with HIP events, in 1 GiB of device memory it allocates and frees:
@@ -111,9 +112,9 @@ int mfk_xcopy_signal(void *word, uint32_t value, void *stream);
 /* A triple table in device memory, copied without a plan (kernels/xcopy_plan.h says how): `grid` workgroups walk its segments,
  * `restGrid` those of the second launch the pieces of long segments that the first has listed in `rest`, a mf::RestList in
  * device memory with room for `capacity` pieces whose counts are 0 before and after.  One call at a time may use a list.
- * event, attached: as for mfk_xcopy_pieces. */
+ * event: as for mfk_xcopy_pieces; NULL on a stream that records a graph. */
 int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *rest,
-                     uint32_t capacity, void *mask, uint32_t maskValue, void *stream, void *event, int *attached);
+                     uint32_t capacity, void *mask, uint32_t maskValue, void *stream, void *event);
 /* The same with the list in a statically allocated device array instead of memory the engine allocates: no allocation
  * anywhere, at most MFK_STATIC_TABLE_SEGMENTS segments, one call at a time per GPU.  mfk_xcopy_static_setup looks the
  * array's address up for the current device (once per device, at start-up); mfk_xcopy_table_static returns -2 when that has

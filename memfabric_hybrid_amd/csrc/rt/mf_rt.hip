@@ -276,6 +276,16 @@ extern "C" int mfrt_stream_sync(void *stream)
     return Code(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
 }
 
+extern "C" int mfrt_stream_capturing(void *stream)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return 1;   // the null stream while another one records: what a graph may hold is right in any case
+    }
+    return status != hipStreamCaptureStatusNone ? 1 : 0;
+}
+
 extern "C" int mfrt_device_sync(void)
 {
     return Code(hipDeviceSynchronize());

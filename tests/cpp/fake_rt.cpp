@@ -33,8 +33,19 @@ uint64_t g_groupMapErrors = 0;
 uint32_t g_lastTableHold = 0;    // holdNanos of the latest table launch
 std::atomic<uint64_t> g_streamsMade{0};   // streams made since mfrt_init
 
+// The stream that records a graph, and what a graph cannot hold or replay that was done while it did: allocations, events recorded
+// on it, launches whose descriptors lie in memory of the host's.
+void *g_capturing = nullptr;
+uint64_t g_captureErrors = 0;
+void NoteRecorded(const void *stream)
+{
+    g_captureErrors += g_capturing != nullptr && stream == g_capturing ? 1 : 0;
+}
+const void *g_lastRestList = nullptr;
+
 void *Track(uint64_t bytes, int kind)
 {
+    NoteRecorded(g_capturing);
     void *p = nullptr;
     if (posix_memalign(&p, 4096, bytes == 0 ? 4096 : bytes) != 0) {
         return nullptr;
@@ -127,6 +138,9 @@ static void Guard(const char *what)
         std::abort();
     }
 }
+void fake_rt_capture(void *stream) { g_capturing = stream; }
+uint64_t fake_rt_capture_errors(void) { return g_captureErrors; }
+const void *fake_rt_last_rest_list(void) { return g_lastRestList; }
 uint64_t fake_rt_launches(void) { return g_launches; }
 uint32_t fake_rt_last_hold(void) { return g_lastHold; }
 uint32_t fake_rt_last_window(void) { const uint32_t w = g_lastWindow; g_lastWindow = 0; return w; }
@@ -235,11 +249,13 @@ uint64_t fake_rt_in_flight(void)
 
 extern "C" void fake_rt_count_stream_sync(void);
 int mfrt_stream_sync(void *) { Guard("mfrt_stream_sync"); Retire(~0ull); fake_rt_count_stream_sync(); return 0; }
+int mfrt_stream_capturing(void *stream) { return g_capturing != nullptr && stream == g_capturing ? 1 : 0; }
 int mfrt_device_sync(void) { Guard("mfrt_device_sync"); Retire(~0ull); return 0; }
 void *mfrt_event_create(void) { return calloc(1, 8); }
 int mfrt_event_destroy(void *e) { Guard("mfrt_event_destroy"); free(e); return 0; }
-int mfrt_event_record(void *e, void *)
+int mfrt_event_record(void *e, void *stream)
 {
+    NoteRecorded(stream);
     std::lock_guard<std::mutex> guard(g_flightLock);
     *static_cast<uint64_t *>(e) = g_flightSeq;
     return 0;
@@ -315,8 +331,9 @@ int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, 
 
 // As the kernel: the owner of a chunk by division under a pattern, else from the two group-map entries around it and the prefix between
 // them.  A map whose entries do not bracket the owner fails the launch.
-int mfk_xcopy_table(const void *tablePlan, int, uint32_t grid, void *mask, uint32_t maskValue, void *)
+int mfk_xcopy_table(const void *tablePlan, int, uint32_t grid, void *mask, uint32_t maskValue, void *stream)
 {
+    NoteRecorded(stream);
     const mf::TablePlan &plan = *static_cast<const mf::TablePlan *>(tablePlan);
     const uint64_t *t = plan.triples;
     const uint32_t *f = plan.first;
@@ -373,8 +390,9 @@ int mfk_xcopy_table(const void *tablePlan, int, uint32_t grid, void *mask, uint3
 // The pieces in the order of the kernel's workgroups.  One that is longer than its workgroup or reaches past the end of the list
 // fails the launch.
 int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, void *mask, uint32_t maskValue,
-                     void *stream, uint32_t holdNanos, void *event, int *attached)
+                     void *stream, uint32_t holdNanos, void *event)
 {
+    NoteRecorded(stream);
     g_lastTableHold = holdNanos;
     if (pieces == nullptr || count == 0 || (units != 256 && units != 512 && units != 1024)) {
         return -1;
@@ -406,7 +424,9 @@ int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_
     if (moved != bytes) {
         return 721;
     }
-    *attached = event != nullptr && mfrt_event_record(event, stream) == 0 ? 1 : 0;
+    if (event != nullptr) {
+        (void)mfrt_event_record(event, stream);
+    }
     if (mask != nullptr) {
         *static_cast<uint64_t *>(mask) = maskValue;
     }
@@ -416,9 +436,12 @@ int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_
 // The direct copy of a device-resident table restated: the parts of every segment, and the pieces of long ones out of a list
 // that a small capacity makes run over.
 int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int, uint32_t grid, uint32_t restGrid, void *rest,
-                     uint32_t capacity, void *mask, uint32_t maskValue, void *stream, void *event, int *attached)
+                     uint32_t capacity, void *mask, uint32_t maskValue, void *stream, void *event)
 {
-    *attached = event != nullptr && mfrt_event_record(event, stream) == 0 ? 1 : 0;
+    if (event != nullptr) {
+        (void)mfrt_event_record(event, stream);
+    }
+    g_lastRestList = rest;
     mf::RestList *list = static_cast<mf::RestList *>(rest);
     if (nseg == 0 || grid == 0 || restGrid == 0 || list == nullptr || capacity == 0 || list->count != 0 || list->done != 0) {
         return -1;
@@ -492,8 +515,7 @@ int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, i
     if (nseg == 0 || nseg > MFK_STATIC_TABLE_SEGMENTS) {
         return -1;
     }
-    int attached = 0;
-    return mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, list.data(), 16, nullptr, 0, stream, nullptr, &attached);
+    return mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, list.data(), 16, nullptr, 0, stream, nullptr);
 }
 
 static uint32_t g_lastRectMates = 0;

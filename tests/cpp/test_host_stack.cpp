@@ -43,6 +43,9 @@ extern "C" uint32_t fake_rt_last_table_shift(void);
 extern "C" uint32_t fake_rt_last_table_hold(void);
 extern "C" uint64_t fake_rt_group_map_errors(void);
 extern "C" uint64_t fake_rt_in_flight(void);
+extern "C" void fake_rt_capture(void *stream);
+extern "C" uint64_t fake_rt_capture_errors(void);
+extern "C" const void *fake_rt_last_rest_list(void);
 
 using namespace mf;
 using ock::mf::DataOperatorPtr;
@@ -1293,6 +1296,75 @@ static void TestSlotRing()
     hybm_uninit();
 }
 
+// Calls on a stream that records a graph: nothing they launch may read host memory that a later call rewrites, nothing may be
+// allocated and no event recorded; and plain calls afterwards find their slots as they left them.
+static void TestRecordedCalls()
+{
+    CHECK(hybm_init(0, 0) == BM_OK);
+    const uint64_t bytes = 96ull << 20;
+    auto *a = static_cast<uint8_t *>(mfrt_alloc_device(bytes));
+    auto *b = static_cast<uint8_t *>(mfrt_alloc_device(bytes));
+    auto *table = static_cast<uint64_t *>(mfrt_alloc_device(24 * 4096));
+    CHECK(a != nullptr && b != nullptr && table != nullptr);
+    std::vector<uint8_t> ref(bytes);
+    Fill(ref, 31);
+    std::memcpy(a, ref.data(), bytes);
+    void *stream = mfrt_stream_create();
+    const struct {
+        uint32_t n;
+        uint64_t len;
+        uint32_t apart;
+        bool ragged;
+    } cases[] = {{3, 10u << 20, 5, false}, {128, 300000, 3, true}, {129, 4096, 0, false}, {300, 70000, 7, true}, {1000, 5000, 0, true}, {4000, 77, 1, true}};
+    for (const auto &c : cases) {
+        std::vector<uint64_t> s(c.n), d(c.n), l(c.n);
+        for (uint32_t i = 0; i < c.n; ++i) {
+            s[i] = reinterpret_cast<uint64_t>(a) + i * c.len + c.apart;
+            d[i] = reinterpret_cast<uint64_t>(b) + i * c.len;
+            l[i] = c.ragged ? c.len - (i * 37) % (c.len / 2) - 1 : c.len;
+            table[3 * i] = s[i];
+            table[3 * i + 1] = d[i];
+            table[3 * i + 2] = l[i];
+        }
+        for (int route : {MF_ROUTE_HBM, MF_ROUTE_TO_HOST, MF_ROUTE_FROM_HOST}) {
+            for (int form = 0; form < 2; ++form) {
+                auto call = [&] {
+                    return form == 0 ? mf_xcopy_batch(s.data(), d.data(), l.data(), c.n, route, stream)
+                                     : mf_xcopy_device_table(table, c.n, route, stream);
+                };
+                CHECK(call() == BM_OK);
+                const void *plainList = fake_rt_last_rest_list();
+                std::memset(b, 0, bytes);
+                const uint64_t errors = fake_rt_capture_errors();
+                fake_rt_capture(stream);
+                const void *list = nullptr;
+                for (int k = 0; k < 9; ++k) {      // more than the ring has slots
+                    CHECK(call() == BM_OK);
+                    CHECK(form == 0 || fake_rt_last_rest_list() != (k == 0 ? plainList : list));   // side by side in a graph
+                    list = fake_rt_last_rest_list();
+                }
+                fake_rt_capture(nullptr);
+                CHECK(fake_rt_capture_errors() == errors);
+                bool same = true;
+                for (uint32_t i = 0; i < c.n; ++i) {
+                    same = same && std::memcmp(reinterpret_cast<void *>(d[i]), reinterpret_cast<void *>(s[i]), l[i]) == 0;
+                }
+                CHECK(same);
+                for (int k = 0; k < 9; ++k) {
+                    CHECK(call() == BM_OK);
+                    CHECK(form == 0 || fake_rt_last_rest_list() != list);
+                }
+            }
+        }
+    }
+    CHECK(mfrt_device_sync() == 0);
+    mfrt_stream_destroy(stream);
+    mfrt_free_device(a);
+    mfrt_free_device(b);
+    mfrt_free_device(table);
+    hybm_uninit();
+}
+
 // The two-symbol plugin over the same engine: the completion word of a table the CPU can read is
 // stored before the call returns; a failed launch leaves the word alone and is counted.
 static void TestPlugin()
@@ -1718,6 +1790,7 @@ int main()
     TestPlanners();
     TestHostCopy();
     TestSlotRing();
+    TestRecordedCalls();
     TestCApi();                                  // device window: reserved address space, HBM mapped in
     setenv("MF_HIP_GVA_WINDOW", "malloc", 1);
     TestCApi();                                  // device window: one ordinary allocation
