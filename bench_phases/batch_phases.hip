@@ -381,9 +381,8 @@ void LaunchPiecesProduct(const Batch &b, hipStream_t s)
     const uint32_t units = b.bytes > kDeepMinBytes ? kDeepUnits : kXcopyThreads;
     const uint32_t count = units == kDeepUnits ? b.ndeep : b.nchunk;
     const uint32_t rule = HoldNanosFor(count, count, units, false);
-    int attached = 0;
     const int err = mfk_xcopy_pieces(units == kDeepUnits ? b.deepPieces : b.pieces, count, b.bytes, units, nullptr, 0, s,
-                                     rule != 0 ? rule + (deep ? kHoldLookupDeepExtraNanos : kHoldLookupExtraNanos) : 0, nullptr, &attached);
+                                     rule != 0 ? rule + (deep ? kHoldLookupDeepExtraNanos : kHoldLookupExtraNanos) : 0, nullptr);
     if (err != 0) {
         std::fprintf(stderr, "mfk_xcopy_pieces failed: %d\n", err);
         std::exit(1);
