@@ -1538,8 +1538,8 @@ uint32_t XcopyEngine::HoldFor(const InlinePlan &plan, uint32_t grid, int route, 
 
 // Hold of a launch of pieces, as that of a table of `count` chunks whose waves fetch their descriptors across the host link and
 // issue their loads that much later than those of a launch whose descriptors are kernel arguments.  (The launcher takes off
-// what pieces wait less: PieceHoldNanos.)
-uint32_t XcopyEngine::HoldForPieces(uint32_t count, uint32_t units, bool unordered) const
+// what pieces wait less, PieceLessNanos, so a wait set by hand, which is meant as it is, gets that on top.)
+uint32_t XcopyEngine::HoldForPieces(uint32_t count, uint64_t bytes, uint32_t units, bool unordered) const
 {
     if (unordered || tuning_.holdNanos == 0) {
         return 0;
@@ -1552,7 +1552,7 @@ uint32_t XcopyEngine::HoldForPieces(uint32_t count, uint32_t units, bool unorder
         return 0;
     }
     if (tuning_.holdNanos > 0) {
-        return static_cast<uint32_t>(tuning_.holdNanos);
+        return static_cast<uint32_t>(tuning_.holdNanos) + PieceLessNanos(count, bytes, units);
     }
     if (tuning_.holdCalibratedOff) {
         return 0;
@@ -2007,7 +2007,7 @@ int XcopyEngine::SubmitPieces(const uint64_t *src, const uint64_t *dst, const ui
         return mfk_xcopy_inline(&empty, MFRT_ROUTE_HBM, 1, mask, maskValue, stream, 0, 0) == 0 ? BM_OK : BM_ERROR;
     }
     void *event = EventOfLaunch(lease, *slot, stream);
-    const int err = mfk_xcopy_pieces(pieces, count, total, units, mask, maskValue, stream, HoldForPieces(count, units, unordered), event);
+    const int err = mfk_xcopy_pieces(pieces, count, total, units, mask, maskValue, stream, HoldForPieces(count, total, units, unordered), event);
     if (err != 0) {
         (void)MarkQueued(lease, slot, stream, true);   // the launch may have gone out with only the word behind it failing
         MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(err));

@@ -201,7 +201,7 @@ private:
     XcopyEngine() = default;
 
     uint32_t HoldFor(const InlinePlan &plan, uint32_t grid, int route, bool unordered) const;
-    uint32_t HoldForPieces(uint32_t count, uint32_t units, bool unordered) const;
+    uint32_t HoldForPieces(uint32_t count, uint64_t bytes, uint32_t units, bool unordered) const;
     // Whether a batch of `bytes` in n segments is planned in chunks of kDeepUnits units, to hold the stores of 16 KiB per wave.
     bool DeepHoldApplies(uint64_t bytes, uint32_t n, int route, bool unordered) const;
     // A launch that stores the thread's word itself, where that is the faster form: kNotLaunched where it is not.

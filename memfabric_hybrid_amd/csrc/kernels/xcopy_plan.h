@@ -134,12 +134,16 @@ constexpr int32_t kHoldLookupDeepExtraNanos = 2000;
 // 24 MB +400 / 200 / 400 ns, 27 / 36 / 45 / 54 / 63 MB on 16 KiB +400 / 800 / 800 / 1200 / 1000; ragged segments of 14 / 21 MB 0, 31 / 41 /
 // 52 MB -800 / -800 / -1200, where the bytes that are not there make 1000 / 1300 / 1700.
 constexpr uint32_t kPieceLeadNanos = 1400;
-inline uint32_t PieceHoldNanos(uint32_t holdNanos, uint32_t count, uint64_t bytes, uint32_t units)
+inline uint32_t PieceLessNanos(uint32_t count, uint64_t bytes, uint32_t units)
 {
     const uint64_t full = static_cast<uint64_t>(count) * units * kUnitBytes;
     const uint64_t missing = full > bytes ? (full - bytes) / kUnitBytes : 0;                 // units
-    const uint64_t less = kPieceLeadNanos + missing * (units == kDeepUnits ? 215 : 180) / (100ull * kDeepUnits);
-    return holdNanos > less ? static_cast<uint32_t>(holdNanos - less) : 0;
+    return static_cast<uint32_t>(kPieceLeadNanos + missing * (units == kDeepUnits ? 215 : 180) / (100ull * kDeepUnits));
+}
+inline uint32_t PieceHoldNanos(uint32_t holdNanos, uint32_t count, uint64_t bytes, uint32_t units)
+{
+    const uint32_t less = PieceLessNanos(count, bytes, units);
+    return holdNanos > less ? holdNanos - less : 0;
 }
 
 // The start of a windowed launch's first period travels between its waves as the low kEpochClockBits bits of a

@@ -30,6 +30,7 @@ std::atomic<uint64_t> g_chunksRun{0};
 bool g_skipCopies = false;       // launches count and check their plans but move nothing (tables of segments no test can back with memory)
 uint32_t g_lastTableShift = 0;   // group shift of the latest table launch that used a group map, 0 under a pattern
 uint64_t g_groupMapErrors = 0;
+uint32_t g_lastPieceWait = 0;    // what the waves of the latest launch of pieces wait
 uint32_t g_lastTableHold = 0;    // holdNanos of the latest table launch
 std::atomic<uint64_t> g_streamsMade{0};   // streams made since mfrt_init
 
@@ -151,6 +152,7 @@ uint64_t fake_rt_chunks(void) { return g_chunksRun; }
 void fake_rt_skip_copies(int on) { g_skipCopies = on != 0; }
 uint32_t fake_rt_last_table_shift(void) { return g_lastTableShift; }
 uint64_t fake_rt_group_map_errors(void) { return g_groupMapErrors; }
+uint32_t fake_rt_last_piece_wait(void) { return g_lastPieceWait; }
 uint32_t fake_rt_last_table_hold(void) { return g_lastTableHold; }
 
 int mfrt_init(int device)
@@ -394,6 +396,7 @@ int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_
 {
     NoteRecorded(stream);
     g_lastTableHold = holdNanos;
+    g_lastPieceWait = mf::PieceHoldNanos(holdNanos, count, bytes, units);
     if (pieces == nullptr || count == 0 || (units != 256 && units != 512 && units != 1024)) {
         return -1;
     }

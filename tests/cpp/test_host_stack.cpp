@@ -41,6 +41,7 @@ extern "C" void fake_rt_set_calibration(const float *us);
 extern "C" const uint32_t *fake_rt_calibration_holds(void);
 extern "C" uint32_t fake_rt_last_table_shift(void);
 extern "C" uint32_t fake_rt_last_table_hold(void);
+extern "C" uint32_t fake_rt_last_piece_wait(void);
 extern "C" uint64_t fake_rt_group_map_errors(void);
 extern "C" uint64_t fake_rt_in_flight(void);
 extern "C" void fake_rt_capture(void *stream);
@@ -1575,6 +1576,15 @@ static void TestHeldStores()
         CHECK(rule != 0 && fake_rt_last_table_hold() == rule + kHoldLookupExtraNanos);
         rule = submit(600, true);                           // ragged, some 40 MB
         CHECK(rule != 0 && fake_rt_last_table_hold() == rule + kHoldLookupDeepExtraNanos);
+        // a wait set by hand is what the waves wait, whatever the pieces are like
+        for (int32_t nanos : {700, 3000}) {
+            CHECK(mf_xcopy_hold_stores(nanos) == BM_OK);
+            for (uint32_t n : {244u, 300u, 488u, 600u}) {
+                (void)submit(n, n == 300 || n == 600);
+                CHECK(fake_rt_last_piece_wait() == static_cast<uint32_t>(nanos));
+            }
+        }
+        CHECK(mf_xcopy_hold_stores(-1) == BM_OK);
     }
     hybm_uninit();
 }
