@@ -49,7 +49,7 @@ int32_t mf_xcopy_tune(uint32_t units, uint32_t wgPerCu, uint32_t wgPerCuLink);
  * to 128 segments) is copied 7 to 20 % faster when every wave waits with its stores until the loads of
  * the whole launch are out, so that HBM sees a burst of reads and then a burst of writes instead of both
  * mixed.  nanos: -1 = the library's rule for how long a wave waits after its start (the default),
- * 0 = never wait, otherwise that many ns for every launch the rule would pick.  Other launches, and
+ * 0 = never wait, otherwise that many ns for every launch the rule would pick, also of more than 128 segments.  Other launches, and
  * batches submitted with MF_COPY_UNORDERED_FLAG, never wait. */
 int32_t mf_xcopy_hold_stores(int32_t nanos);
 /* Read and write windows.  A batch of up to 128 segments and 512 MiB or more between HBM addresses is copied
@@ -101,15 +101,15 @@ uint32_t mf_xcopy_stream_queues(uint32_t *queues, uint32_t capacity);
 /* Table launches.  stageUnordered: 1 (default) launches the upload of a ragged table's descriptors without a
  * barrier, so that it runs while the caller's earlier copies still do; 0 orders it behind them.
  * deviceTableWgPerCu: workgroups per CU of the launch that copies a table in device memory, whose chunk
- * count only the GPU knows (0 = the default: eight workgroups per segment, between 32 and 4096 per CU); each walks
- * the chunks with the grid as its stride. */
+ * count only the GPU knows (0 = the default: four workgroups per segment, between 16 and 1024 per CU); each walks
+ * the parts of the segments with the grid as its stride. */
 int32_t mf_xcopy_tune_table(uint32_t stageUnordered, uint32_t deviceTableWgPerCu);
 /* Held stores beyond the kernel-argument form.  deepHold: 1 (default) lets batches of 24 to 64 MiB whose segments
  * average 32 KiB and more be copied in 16 KiB chunks, one single wave each with sixteen loads per lane in flight,
  * stores held like those of the smaller batches; 0 keeps them on 4 KiB chunks that store at once.
  * pinnedExtraNanos: added to the wait of launches of more than 128 segments, whose descriptors come out of pinned
  * host memory rather than out of the kernel arguments (default 1600: a wave's loads start a link round trip later;
- * launches on 16 KiB chunks wait 800 ns more than that).
+ * launches on 16 KiB chunks wait 400 ns more than that; of the sum they take off what their pieces save).
  * holdOnSideStreams: 1 lets batches launched by the submit threads (mf_xcopy_unordered_streams) hold their stores too;
  * 0 (default): they overlap one another on purpose and store at once. */
 int32_t mf_xcopy_tune_hold(uint32_t deepHold, int32_t pinnedExtraNanos, uint32_t holdOnSideStreams);
