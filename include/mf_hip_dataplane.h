@@ -73,8 +73,8 @@ int32_t mf_xcopy_device_table(const void *triples, uint32_t n, int32_t route, vo
 
 /* No counterpart in the reference.  mf_xcopy_device_table for callers that cannot allocate: code
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  What the first launch
- * leaves for the second (a list of the pieces of long segments) lives in a statically allocated device
- * array (240 KiB per GPU, held until the process ends) instead of memory the library allocates on
+ * leaves for the second (a list of long segments) lives in a statically allocated device
+ * array (1 MiB per GPU, held until the process ends) instead of memory the library allocates on
  * demand, and the call creates no stream, event or staging either: `stream` is used as given (NULL is
  * the null stream).
  * Limits: n <= MF_XCOPY_STATIC_TABLE_MAX segments (BM_INVALID_PARAM beyond); every call on one GPU

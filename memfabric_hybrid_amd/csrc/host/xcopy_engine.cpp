@@ -688,30 +688,34 @@ int EnsureDevice(StagingSlot &slot, uint64_t bytes)
     return BM_OK;
 }
 
-void *RestListAt(void *lists, uint32_t i)
+RestList *RestListAt(void *lists, uint32_t i, uint32_t capacity)
 {
-    return static_cast<uint8_t *>(lists) + i * RoundUp(RestListBytes(kRestCapacity), 256);
+    return reinterpret_cast<RestList *>(static_cast<uint8_t *>(lists) + i * RoundUp(RestListBytes(capacity), 256));
 }
 
-int EnsureRestLists(void *&lists, uint32_t count)
+int EnsureRestLists(void *&lists, uint32_t count, uint32_t capacity)
 {
     if (lists != nullptr) {
         return BM_OK;
     }
-    lists = mfrt_alloc_device(count * RoundUp(RestListBytes(kRestCapacity), 256));
+    lists = mfrt_alloc_device(count * RoundUp(RestListBytes(capacity), 256));
     if (lists == nullptr) {
-        MF_FAIL(BM_MALLOC_FAILED, "list of " << kRestCapacity << " pieces could not be allocated in HBM");
+        MF_FAIL(BM_MALLOC_FAILED, "lists of " << capacity << " segments could not be allocated in HBM");
     }
     // cleared once, on a stream of the engine: the caller's may be recording
     void *own = XcopyEngine::Instance().ThreadStream();
     int err = own == nullptr ? -1 : 0;
     for (uint32_t i = 0; i < count && err == 0; ++i) {
-        err = mfk_xcopy_signal(RestListAt(lists, i), 0, own);   // one 64-bit word, both counts
+        RestList *list = RestListAt(lists, i, capacity);
+        err = mfk_xcopy_signal(&list->taken, 0, own);
+        for (uint32_t g = 0; g <= kRestGroups && err == 0; ++g) {
+            err = mfk_xcopy_signal(&list->done[g].count, 0, own);
+        }
     }
     if (err != 0 || mfrt_stream_sync(own) != 0) {
         (void)mfrt_free_device(lists);
         lists = nullptr;
-        MF_FAIL(BM_ERROR, "list of pieces could not be cleared: " << mfrt_error_string(err));
+        MF_FAIL(BM_ERROR, "lists of segments could not be cleared: " << mfrt_error_string(err));
     }
     return BM_OK;
 }
@@ -750,10 +754,10 @@ uint32_t DeviceTableGrid(uint32_t nseg, uint32_t cuCount, int route, const Xcopy
     return GridFor(tuning.deviceTableWgPerCu != 0 ? cus * tuning.deviceTableWgPerCu : want, cuCount, route, tuning);
 }
 
-// Grid of the launch behind it, which usually finds nothing to do: four per CU keep enough loads in flight when it does.
+// Grid of the launch behind it, which usually finds nothing to do (the kernel has the figures).
 uint32_t DeviceTableRestGrid(uint32_t cuCount, int route, const XcopyTuning &tuning)
 {
-    return GridFor(4ull * (cuCount == 0 ? 256 : cuCount), cuCount, route, tuning);
+    return GridFor(2ull * (cuCount == 0 ? 256 : cuCount), cuCount, route, tuning);
 }
 
 }  // namespace
@@ -2039,33 +2043,41 @@ int XcopyEngine::SubmitDeviceTable(const void *triples, uint32_t n, int route, v
         int err = mfk_xcopy_inline(&empty, route, 1, mask, maskValue, stream, 0, 0);
         return err == 0 ? BM_OK : BM_ERROR;
     }
-    // The list of long segments' pieces belongs to a slot: the next call of another stream gets another one.  Calls that become
+    // The list of long segments belongs to a slot: the next call of another stream gets another one.  Calls that become
     // nodes of a graph have lists of their own, made by the thread's first call: a graph may be replayed beside plain calls.
     ThreadCtx &ctx = t_ctx;
     StagingSlot *slot = nullptr;
     ThreadLease &lease = ctx.Lease();
     const bool recorded = mfrt_stream_capturing(stream) != 0;
-    int ret = EnsureRestLists(lease.graphRests, kSlots);
+    int ret = EnsureRestLists(lease.graphRests, kSlots, kRestGraphCapacity);
     if (ret == BM_OK && !recorded) {
         ret = AcquireSlot(lease, 0, stream, slot);
-        ret = ret == BM_OK ? EnsureRestLists(slot->rest, 1) : ret;
+        ret = ret == BM_OK ? EnsureRestLists(slot->rest, 1, kRestCapacity) : ret;
     }
     if (ret != BM_OK) {
         return ret;
     }
-    void *list = recorded ? RestListAt(lease.graphRests, lease.graphCursor++ % kSlots) : slot->rest;
+    void *list = recorded ? RestListAt(lease.graphRests, lease.graphCursor++ % kSlots, kRestGraphCapacity) : slot->rest;
     void *event = recorded ? nullptr : EventOfLaunch(lease, *slot, stream);
     const uint32_t cu = mfrt_cu_count();
     const uint32_t units = ChooseUnits(0, cu, route, tuning_);   // sizes are only known on the GPU
-    const int err = mfk_xcopy_direct(triples, n, units, route, DeviceTableGrid(n, cu, route, tuning_), DeviceTableRestGrid(cu, route, tuning_),
-                                     list, kRestCapacity, mask, maskValue, stream, event);
+    const uint32_t capacity = recorded ? kRestGraphCapacity : kRestCapacity;
+    int err = 0;
+    for (uint32_t at = 0; at < n && err == 0; ) {
+        const uint32_t m = n - at < capacity ? n - at : capacity;
+        const bool last = m == n - at;
+        err = mfk_xcopy_direct(static_cast<const uint64_t *>(triples) + 3ull * at, m, units, route, DeviceTableGrid(m, cu, route, tuning_),
+                               DeviceTableRestGrid(cu, route, tuning_), list, capacity, last ? mask : nullptr, maskValue, stream,
+                               last ? event : nullptr);
+        g_launches.fetch_add(err == 0 ? 2 : 0, std::memory_order_relaxed);
+        at += m;
+    }
     if (err != 0) {
         if (!recorded) {
             (void)MarkQueued(lease, slot, stream, true);   // the first launch writes the list
         }
         MF_FAIL(BM_ERROR, "xcopy launch of a device table failed: " << mfrt_error_string(err));
     }
-    g_launches.fetch_add(2, std::memory_order_relaxed);
     NotePending(stream, ~0ull);   // sizes unknown here: the next wait sleeps on the stream
     return recorded ? BM_OK : MarkQueued(lease, slot, stream, false, event != nullptr);
 }

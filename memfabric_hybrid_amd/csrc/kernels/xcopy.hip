@@ -737,7 +737,8 @@ __global__ __launch_bounds__(kLanes) void XcopyPieceKernel(const Piece *__restri
 // it copies the current item.  What bounds it is HBM; a launch in front of it that planned the table (chunk prefix, owner map,
 // repeating pattern) took 8 us, after which the copy was no faster: 4096 pages of 32 KiB scattered 60.0 / 52.8 us with the
 // planner / so, 16 080 pages of 8 KiB 76.7 / 57.9, 100 pages 10.0 / 7.1, 2000 ragged segments of up to 70 KB 41.5 / 36.5, 16 384 of up to
-// 262 KB 940 / 897, one of 1 GiB among 4096 short ones 459 / 411.
+// 262 KB 940 / 897.  (The triples of 64 items at a time, one per lane, so that empty items cost no wait: more registers than eight
+// waves per SIMD have, 10 to 60 % slower on short tables; two triples ahead instead of one: no faster, 16 384 segments of 2 to 14 KB 4 % slower.)
 template <bool kNtLoad, int kStore>
 __global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_t *__restrict__ triples, uint32_t nseg, uint32_t units,
                                                                    RestList *__restrict__ rest, uint32_t capacity)
@@ -775,31 +776,13 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_
         }
         if (part == 0 && chunks > own) {
             const uint64_t at = SegmentGeometry(dst, len).head + own * units * kUnitBytes;
-            const uint64_t left = len - at;
-            const uint64_t each = RestPieceBytesFor(left);
-            const uint32_t count = static_cast<uint32_t>((left + each - 1) / each);
-            __shared__ uint32_t first;
             if (threadIdx.x == 0) {
-                // a full list takes no more, so that the count stays far from its end
-                first = __hip_atomic_load(&rest->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (first < capacity) {
-                    first = __hip_atomic_fetch_add(&rest->count, count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint64_t taken = __hip_atomic_fetch_add(&rest->taken, kRestEntry + RestPieces(len - at), __ATOMIC_RELAXED,
+                                                              __HIP_MEMORY_SCOPE_AGENT);
+                if (taken / kRestEntry < capacity) {   // which nseg is not more than: calls that share a list against the rules stay inside it
+                    rest->entry[taken / kRestEntry] = RestSegment{taken % kRestEntry, src + at, dst + at, len - at};
                 }
             }
-            __syncthreads();
-            const uint32_t room = first < capacity ? capacity - first : 0;
-            for (uint32_t i = threadIdx.x; i < count && i < room; i += blockDim.x) {
-                const uint64_t from = i * each;
-                rest->piece[first + i] = RestPiece{src + at + from, dst + at + from, left - from < each ? left - from : each};
-            }
-            if (count > room) {                                            // a list of thousands of long segments: the others go on here
-                const uint64_t from = at + room * each;
-                const uint64_t over = SegmentChunks(dst + from, len - from, units);
-                for (uint64_t c = 0; c < over; ++c) {
-                    CopyChunk<kNtLoad, kStore>(src + from, dst + from, len - from, c, units);
-                }
-            }
-            __syncthreads();                                               // `first` is free again
         }
         if (!more) {
             return;
@@ -812,29 +795,108 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_
     }
 }
 
-// The pieces XcopyDirectKernel has listed; usually none (1.6 us then).  The last workgroup leaves the list empty.
-template <bool kNtLoad, int kStore>
-__global__ __launch_bounds__(kXcopyThreads) void XcopyRestKernel(RestList *rest, uint32_t capacity, uint32_t units)
+// The segments of a list that a wave is at, one per lane, so that the owner of a piece is found without a load.
+struct RestRows {
+    uint64_t first = ~0ull;     // of the lane's segment
+    uint64_t src = 0;
+    uint64_t dst = 0;
+    uint64_t len = 0;
+    uint64_t end;               // pieces of the segments up to these, ~0 when they are the last
+
+    __device__ __forceinline__ RestRows(const RestList *rest, uint32_t lo, uint32_t count)
+    {
+        const uint32_t i = lo + (threadIdx.x & 63u);
+        if (i < count) {
+            const RestSegment r = rest->entry[i];
+            first = r.first;
+            src = r.src;
+            dst = r.dst;
+            len = r.len;
+        }
+        end = lo + 64 < count ? Uniform(rest->entry[lo + 64].first) : ~0ull;
+    }
+};
+
+// The last segment of [lo, count) whose `first` is <= p; that of lo is.
+__device__ __forceinline__ uint32_t RestOwner(const RestList *rest, uint32_t lo, uint32_t count, uint64_t p)
 {
-    const uint32_t listed = Uniform(__hip_atomic_load(&rest->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    if (listed == 0) {
+    const uint32_t lane = threadIdx.x & 63u;
+    while (count - lo > 1) {
+        const uint32_t step = (count - lo + 63u) >> 6;
+        const uint32_t probe = lo + lane * step;
+        const uint32_t hits = __popcll(__ballot(probe < count && rest->entry[probe < count ? probe : lo].first <= p));
+        lo += hits > 1 ? (hits - 1) * step : 0;
+        count = count - lo < step ? count : lo + step;
+    }
+    return lo;
+}
+
+// Whether this is the last of `all` calls on a counter, which it leaves at 0.
+__device__ __forceinline__ bool CountsLast(uint64_t *counter, uint64_t all)
+{
+    if (__hip_atomic_fetch_add(counter, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != all - 1) {
+        return false;
+    }
+    __hip_atomic_store(counter, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
+
+// The segments XcopyDirectKernel has listed; usually none.  The last workgroup leaves the list empty.  HBM is the bound; two workgroups
+// of eight waves per CU, sixteen of them on neighbouring chunks of one MiB, is the shape that loses on no kind of table.  By where the
+// allocator has put a pool a copy runs in one of two modes; us in the slower / faster one, with the planner that listed chunks, with a
+// list of pieces (room for sixteen segments of 256 MiB, what came after was copied by one wave each) and so:
+//   1 GiB among 4096 short segments   434 / 408    421 / 390         411 / 389
+//   one of 1 GiB                      410 / 396    409 / 383         398 / 376
+//   16 x 256 MiB                     1742 / 1414  1578 / 1487       1660 / 1419
+//   32 x 512 MiB                     7100 / 5774  145768 / 145898   6815 / 5711
+//   300 x 32 MiB at odd addresses    4244 / 3556  58363 / 58413     4244 / 3496
+// Half the lanes: aligned segments 0 to 5 % faster in the slower mode, odd ones 3 to 11 % slower; twice the workgroups: 1 to 5 % slower.
+// Neighbouring waves on neighbouring pieces of 64 KiB instead: 1 GiB 421 / 401.  Every workgroup that counts itself done on one word costs
+// 35 to 70 ns at the end (1024 of them: 256 MiB 146 us, on sixteen words 112), hence the groups.
+template <bool kNtLoad, int kStore>
+__global__ __launch_bounds__(kRestLanes) void XcopyRestKernel(RestList *rest, uint32_t capacity, uint32_t units)
+{
+    const uint64_t taken = Uniform(__hip_atomic_load(&rest->taken, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    if (taken == 0) {
         return;
     }
-    const uint32_t count = listed < capacity ? listed : capacity;
-    for (uint32_t p = blockIdx.x; p < count; p += gridDim.x) {
-        const RestPiece r = rest->piece[p];
-        const uint64_t src = Uniform(r.src);
-        const uint64_t dst = Uniform(r.dst);
-        const uint64_t len = Uniform(r.len);
-        const uint64_t chunks = SegmentChunks(dst, len, units);
-        for (uint64_t c = 0; c < chunks; ++c) {
-            CopyChunk<kNtLoad, kStore>(src, dst, len, c, units);
+    const uint32_t count = taken / kRestEntry < capacity ? static_cast<uint32_t>(taken / kRestEntry) : capacity;
+    const uint64_t pieces = taken % kRestEntry;
+    uint32_t lo = 0;
+    RestRows rows(rest, lo, count);
+    for (uint64_t p = blockIdx.x; p < pieces; p += gridDim.x) {
+        if (p >= rows.end) {
+            lo = RestOwner(rest, lo + 64, count, p);
+            rows = RestRows(rest, lo, count);
+        }
+        const uint32_t row = __popcll(__ballot(rows.first <= p)) - 1;
+        const uint64_t src = ReadLane64(rows.src, row);
+        const uint64_t dst = ReadLane64(rows.dst, row);
+        const uint64_t len = ReadLane64(rows.len, row);
+        const uint64_t mine = p - ReadLane64(rows.first, row);
+        const uint64_t all = RestPieces(len);
+        if (mine >= all) {
+            continue;       // not with a list of one call's
+        }
+        // pieces side by side share a stretch of the segment chunk by chunk
+        const uint64_t stretch = mine / kRestShare * kRestShare;
+        const uint32_t share = all - stretch < kRestShare ? static_cast<uint32_t>(all - stretch) : kRestShare;
+        const uint64_t from = stretch * kRestPieceBytes;
+        const uint64_t bytes = len - from < share * kRestPieceBytes ? len - from : share * kRestPieceBytes;
+        const uint64_t chunks = SegmentChunks(dst + from, bytes, units);
+        for (uint64_t c = mine - stretch; c < chunks; c += share) {
+            CopyChunk<kNtLoad, kStore>(src + from, dst + from, bytes, c, units);
         }
     }
     __syncthreads();
-    if (threadIdx.x == 0 && __hip_atomic_fetch_add(&rest->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
-        __hip_atomic_store(&rest->done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&rest->count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x != 0) {
+        return;
+    }
+    const uint32_t group = blockIdx.x % kRestGroups;
+    const uint32_t groups = gridDim.x < kRestGroups ? gridDim.x : kRestGroups;
+    if (CountsLast(&rest->done[group].count, (gridDim.x - group + kRestGroups - 1) / kRestGroups) &&
+        CountsLast(&rest->done[kRestGroups].count, groups)) {
+        __hip_atomic_store(&rest->taken, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -999,10 +1061,12 @@ int LaunchDirect(const uint64_t *triples, uint32_t nseg, uint32_t units, uint32_
     if (err != hipSuccess) {
         return static_cast<int>(err);
     }
-    LaunchWithEvent(XcopyRestKernel<kNtLoad, kStore>, restGrid, lanes, stream, event, rest, capacity, units);
+    const bool link = kStore != kStoreStream;
+    LaunchWithEvent(XcopyRestKernel<kNtLoad, kStore>, restGrid, link ? lanes : kRestLanes, stream, event, rest, capacity,
+                    link ? units : kDepth * kRestLanes);
     err = hipGetLastError();
     if (err != hipSuccess) {   // what the first launch has listed must not be taken for the next call's
-        hipLaunchKernelGGL(XcopySignalKernel, dim3(1), dim3(64), 0, stream, reinterpret_cast<uint64_t *>(rest), 0u);
+        hipLaunchKernelGGL(XcopySignalKernel, dim3(1), dim3(64), 0, stream, &rest->taken, 0u);
     }
     return static_cast<int>(err);
 }
@@ -1156,12 +1220,12 @@ extern "C" int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, 
     return err != 0 ? err : mf::Signal(mask, maskValue, s);
 }
 
-// rest: a RestList with room for `capacity` pieces, its counts 0.
+// rest: a RestList with room for `capacity` segments, its counts 0.
 extern "C" int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *rest,
                                 uint32_t capacity, void *mask, uint32_t maskValue, void *stream, void *event)
 {
     using namespace mf;
-    if (nseg == 0 || grid == 0 || restGrid == 0 || rest == nullptr || capacity == 0) {
+    if (nseg == 0 || nseg > capacity || grid == 0 || restGrid == 0 || rest == nullptr) {
         return -1;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -1344,10 +1408,10 @@ extern "C" int mfk_xcopy_calibrate(void *stream, const uint32_t *holdNanos, cons
 }
 
 #ifndef MF_RT_HIDDEN   // the plugin library has no entry point that needs it
-// List of the entry point that allocates nothing (mfk_xcopy_table_static).  One copy per GPU, zero when its code is loaded and
+// List of the entry point that allocates nothing (mfk_xcopy_table_static), with room for every segment of the longest table.  One copy per GPU, zero when its code is loaded and
 // held until the process ends.  In host code the array's name is only a handle for hipGetSymbolAddress: kernels get the
 // address that call returned for the current device, never the name.
-constexpr uint32_t kStaticRestCapacity = 10240;
+constexpr uint32_t kStaticRestCapacity = MFK_STATIC_TABLE_SEGMENTS;
 static __device__ __align__(256) uint32_t scratch[mf::RestListBytes(kStaticRestCapacity) / 4];
 
 namespace {
@@ -1389,7 +1453,7 @@ extern "C" int mfk_xcopy_static_setup(void)
         uint32_t *words = g_scratchOf[dev];
         RestList *rest = reinterpret_cast<RestList *>(words);
         const uint64_t *none = reinterpret_cast<const uint64_t *>(words);
-        hipLaunchKernelGGL(XcopySignalKernel, dim3(1), dim3(64), 0, nullptr, reinterpret_cast<uint64_t *>(rest->reserved), 0u);
+        hipLaunchKernelGGL(XcopySignalKernel, dim3(1), dim3(64), 0, nullptr, rest->reserved, 0u);
         for (int route = MFRT_ROUTE_HBM; route <= MFRT_ROUTE_FROM_HOST; ++route) {
             (void)WithPolicy(PolicyOf(route), [&](auto ntLoad, auto store) {
                 return LaunchDirect<decltype(ntLoad)::value, decltype(store)::value>(none, 0, kXcopyThreads, 1, 1, 64, rest,

@@ -287,35 +287,44 @@ MF_HD inline uint32_t PieceOf(uint32_t workgroup)
 // A table that only the GPU can read, copied without a plan.  Its launch takes `parts` items per segment, part j of a segment
 // copying the chunks j, j + parts, ... of it: right for every table, whatever `parts` is, and evenly spread where `parts` is near
 // the chunk count of the usual segment.  That is taken from the first kDirectSample segments, by every wave for itself.
-// A part copies kDirectRounds chunks at most; what a segment holds beyond parts * kDirectRounds chunks is cut into pieces and
-// listed for a second launch, so that no wave is left with a long segment.
+// A part copies kDirectRounds chunks at most; a segment that holds more than parts * kDirectRounds chunks is listed for a second
+// launch, which cuts what is left of the listed segments into pieces, so that no wave is left with a long segment.
 constexpr uint32_t kDirectSample = 8;
 constexpr uint32_t kDirectMaxParts = 64;
 constexpr uint32_t kDirectRounds = 4;
-constexpr uint64_t kRestPieceBytes = 64ull << 10;     // the least
-constexpr uint32_t kRestMaxPieces = 4096;             // of one segment
+constexpr uint64_t kRestPieceBytes = 64ull << 10;
+constexpr uint32_t kRestShare = 16;                   // pieces side by side whose workgroups take their chunks in turn
+constexpr uint32_t kRestLanes = 512;                  // of a workgroup of the second launch between HBM addresses
 
-struct RestPiece {
+struct RestSegment {                                  // what is left of a long segment
+    uint64_t first;                                   // pieces of those listed before
     uint64_t src;
     uint64_t dst;
     uint64_t len;
 };
-struct RestList {                                     // both counts are 0 between calls
-    uint32_t count;                                   // pieces listed, beyond the capacity too
-    uint32_t done;                                    // workgroups of the second launch that are done with it
-    uint32_t reserved[14];
-    RestPiece piece[1];                               // as many as the list has room for
+struct RestCount {                                    // on a line of its own
+    uint64_t count;
+    uint64_t reserved[15];
 };
-static_assert(sizeof(RestList) == 64 + sizeof(RestPiece), "pieces start on a cache line");
-constexpr uint32_t kRestCapacity = 65536;              // 1.5 MiB
+constexpr uint32_t kRestGroups = 16;
+// One entry a segment, however long: a list with room for a table's segments holds what any table of them leaves.  All counts are 0
+// between calls.  `taken` counts entries and pieces in one word, which makes `first` ascend with the entries.
+struct RestList {
+    uint64_t taken;                                   // entries * kRestEntry + pieces
+    uint64_t reserved[15];
+    RestCount done[kRestGroups + 1];                  // workgroups of the second launch that are done with it, by group, and groups
+    RestSegment entry[1];                             // as many as the list has room for
+};
+constexpr uint64_t kRestEntry = 1ull << 40;           // pieces of 64 KiB: 2^56 bytes
+constexpr uint32_t kRestCapacity = 65536;             // 2 MiB; a longer table goes in several pairs of launches
+constexpr uint32_t kRestGraphCapacity = 16384;        // of the lists for calls recorded into a graph
 constexpr uint64_t RestListBytes(uint32_t capacity)
 {
-    return sizeof(RestList) + static_cast<uint64_t>(capacity - 1) * sizeof(RestPiece);
+    return sizeof(RestList) + static_cast<uint64_t>(capacity - 1) * sizeof(RestSegment);
 }
-MF_HD inline uint64_t RestPieceBytesFor(uint64_t left)
+MF_HD inline uint64_t RestPieces(uint64_t left)
 {
-    const uint64_t each = (left + kRestMaxPieces - 1) / kRestMaxPieces;
-    return (each + kRestPieceBytes - 1) / kRestPieceBytes * kRestPieceBytes;
+    return (left + kRestPieceBytes - 1) / kRestPieceBytes;
 }
 
 // A table-driven launch: triples, prefix and group map live in device memory (under a pattern the

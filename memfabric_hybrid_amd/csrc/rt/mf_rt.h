@@ -110,8 +110,8 @@ int mfk_xcopy_calibrate(void *stream, const uint32_t *holdNanos, const uint32_t 
  * `stream` before it has finished. */
 int mfk_xcopy_signal(void *word, uint32_t value, void *stream);
 /* A triple table in device memory, copied without a plan (kernels/xcopy_plan.h says how): `grid` workgroups walk its segments,
- * `restGrid` those of the second launch the pieces of long segments that the first has listed in `rest`, a mf::RestList in
- * device memory with room for `capacity` pieces whose counts are 0 before and after.  One call at a time may use a list.
+ * `restGrid` those of the second launch what is left of the long segments that the first has listed in `rest`, a mf::RestList in
+ * device memory with room for `capacity` segments whose counts are 0 before and after.  One call at a time may use a list.
  * event: as for mfk_xcopy_pieces; NULL on a stream that records a graph. */
 int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *rest,
                      uint32_t capacity, void *mask, uint32_t maskValue, void *stream, void *event);

@@ -436,8 +436,8 @@ int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_
     return 0;
 }
 
-// The direct copy of a device-resident table restated: the parts of every segment, and the pieces of long ones out of a list
-// that a small capacity makes run over.
+// The direct copy of a device-resident table restated: the parts of every segment, and the pieces of what long ones have left out
+// of a list.
 int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int, uint32_t grid, uint32_t restGrid, void *rest,
                      uint32_t capacity, void *mask, uint32_t maskValue, void *stream, void *event)
 {
@@ -446,7 +446,7 @@ int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int, ui
     }
     g_lastRestList = rest;
     mf::RestList *list = static_cast<mf::RestList *>(rest);
-    if (nseg == 0 || grid == 0 || restGrid == 0 || list == nullptr || capacity == 0 || list->count != 0 || list->done != 0) {
+    if (nseg == 0 || nseg > capacity || grid == 0 || restGrid == 0 || list == nullptr || list->taken != 0 || list->done[0].count != 0) {
         return -1;
     }
     ++g_launches;
@@ -456,7 +456,7 @@ int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int, ui
         const uint64_t chunks = mf::SegmentChunks(t[3 * i + 1], t[3 * i + 2], units);
         parts = chunks > parts ? (chunks < mf::kDirectMaxParts ? chunks : mf::kDirectMaxParts) : parts;
     }
-    const uint32_t room = capacity < 5 ? capacity : 5;
+    const uint64_t own = parts * mf::kDirectRounds;
     for (uint64_t item = 0; item < nseg * parts; ++item) {
         const uint64_t seg = item / parts;
         const uint64_t part = item % parts;
@@ -464,7 +464,6 @@ int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int, ui
         const uint64_t dst = t[3 * seg + 1];
         const uint64_t len = t[3 * seg + 2];
         const uint64_t chunks = mf::SegmentChunks(dst, len, units);
-        const uint64_t own = parts * mf::kDirectRounds;
         for (uint64_t c = part; c < chunks && c < own; c += parts) {
             RunChunk(src, dst, len, c, units);
         }
@@ -472,27 +471,25 @@ int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int, ui
             continue;
         }
         const uint64_t at = mf::SegmentGeometry(dst, len).head + own * units * mf::kUnitBytes;
-        const uint64_t each = mf::RestPieceBytesFor(len - at);
-        for (uint64_t from = at; from < len; from += each, ++list->count) {
-            if (list->count < room) {
-                list->piece[list->count] = mf::RestPiece{src + from, dst + from, len - from < each ? len - from : each};
-                continue;
-            }
-            for (uint64_t c = 0; c < mf::SegmentChunks(dst + from, len - from, units); ++c) {
-                RunChunk(src + from, dst + from, len - from, c, units);
-            }
-            list->count = room;
-            break;
-        }
+        const uint64_t before = list->taken;
+        list->taken += mf::kRestEntry + mf::RestPieces(len - at);
+        list->entry[before / mf::kRestEntry] = mf::RestSegment{before % mf::kRestEntry, src + at, dst + at, len - at};
     }
     ++g_launches;
-    for (uint32_t p = 0; p < list->count && p < room; ++p) {
-        const mf::RestPiece &r = list->piece[p];
-        for (uint64_t c = 0; c < mf::SegmentChunks(r.dst, r.len, units); ++c) {
-            RunChunk(r.src, r.dst, r.len, c, units);
+    const uint64_t pieces = list->taken % mf::kRestEntry;
+    uint32_t e = 0;
+    for (uint64_t p = 0; p < pieces; ++p) {
+        while (e + 1 < list->taken / mf::kRestEntry && list->entry[e + 1].first <= p) {
+            ++e;
+        }
+        const mf::RestSegment &r = list->entry[e];
+        const uint64_t from = (p - r.first) * mf::kRestPieceBytes;
+        const uint64_t len = r.len - from < mf::kRestPieceBytes ? r.len - from : mf::kRestPieceBytes;
+        for (uint64_t c = 0; c < mf::SegmentChunks(r.dst + from, len, units); ++c) {
+            RunChunk(r.src + from, r.dst + from, len, c, units);
         }
     }
-    list->count = 0;
+    list->taken = 0;
     if (mask != nullptr) {
         *static_cast<uint64_t *>(mask) = maskValue;
     }
@@ -514,11 +511,11 @@ int mfk_xcopy_signal(void *word, uint32_t value, void *)
 int mfk_xcopy_static_setup(void) { return 0; }
 int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *stream)
 {
-    static std::vector<uint64_t> list(mf::RestListBytes(16) / 8, 0);
+    static std::vector<uint64_t> list(mf::RestListBytes(MFK_STATIC_TABLE_SEGMENTS) / 8, 0);
     if (nseg == 0 || nseg > MFK_STATIC_TABLE_SEGMENTS) {
         return -1;
     }
-    return mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, list.data(), 16, nullptr, 0, stream, nullptr);
+    return mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, list.data(), MFK_STATIC_TABLE_SEGMENTS, nullptr, 0, stream, nullptr);
 }
 
 static uint32_t g_lastRectMates = 0;

@@ -1358,6 +1358,31 @@ static void TestRecordedCalls()
             }
         }
     }
+    // a table beyond a list's room goes in pairs of launches; with long segments in each
+    for (bool recorded : {false, true}) {
+        const uint32_t n = (recorded ? kRestGraphCapacity : kRestCapacity) + 100;
+        std::vector<uint64_t> rows(3ull * n);
+        uint64_t at = 0;
+        for (uint32_t i = 0; i < n; ++i) {
+            rows[3 * i] = reinterpret_cast<uint64_t>(a) + at + 3;
+            rows[3 * i + 1] = reinterpret_cast<uint64_t>(b) + at;
+            rows[3 * i + 2] = i % 1000 == 999 || i + 50 == n ? 150000 : i % 700;
+            at += rows[3 * i + 2] + 1;
+        }
+        CHECK(at < bytes);
+        std::memset(b, 0, bytes);
+        const uint64_t before = fake_rt_launches();
+        fake_rt_capture(recorded ? stream : nullptr);
+        CHECK(mf_xcopy_device_table(rows.data(), n, MF_ROUTE_HBM, stream) == BM_OK);
+        fake_rt_capture(nullptr);
+        CHECK(fake_rt_launches() - before == 4);
+        bool same = true;
+        for (uint32_t i = 0; i < n; ++i) {
+            const auto *to = reinterpret_cast<const uint8_t *>(rows[3 * i + 1]);
+            same = same && std::memcmp(to, reinterpret_cast<void *>(rows[3 * i]), rows[3 * i + 2]) == 0 && to[rows[3 * i + 2]] == 0;
+        }
+        CHECK(same);
+    }
     CHECK(mfrt_device_sync() == 0);
     mfrt_stream_destroy(stream);
     mfrt_free_device(a);

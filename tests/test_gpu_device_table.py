@@ -1,6 +1,6 @@
 """Tables in device memory whose segments are unlike the first ones, which decide how a table is shared out: lengths on both
-sides of what a segment's own workgroups copy and of a listed piece, and lists that run over; on every route, and twice in a row,
-so that a list left behind by the first call shows."""
+sides of what a segment's own workgroups copy and of a listed piece, long lists, tables beyond a list; on every route, and twice in
+a row, so that a list left behind by the first call shows."""
 import numpy as np
 import pytest
 
@@ -42,13 +42,15 @@ def _lengths(kind):
         return [0, 5 << 20, 33]
     if kind == "one":
         return [9 << 20]
-    return [5] * 8 + [OWN + 16 + i % 32 for i in range(11000)]   # "list": more pieces than the static list has room for
+    if kind == "pairs of launches":                              # more segments than a list has room for, long ones in each part
+        return [i * 7 % 300 for i in range(65000)] + [OWN + PIECE + 5] * 900 + [i * 7 % 300 for i in range(300)]
+    return [5] * 8 + [OWN + 16 + i % 32 for i in range(11000)]   # "list": more long segments than a wave has lanes
 
 
 @pytest.mark.parametrize("kind,route,static", [
     ("short first", native.ROUTE_HBM, False), ("long first", native.ROUTE_HBM, False), ("few", native.ROUTE_HBM, False),
     ("one", native.ROUTE_HBM, False), ("short first", native.ROUTE_TO_HOST, False), ("long first", native.ROUTE_FROM_HOST, False),
-    ("long first", native.ROUTE_HBM, True), ("list", native.ROUTE_HBM, True),
+    ("long first", native.ROUTE_HBM, True), ("list", native.ROUTE_HBM, True), ("pairs of launches", native.ROUTE_HBM, False),
 ])
 def test_table_unlike_its_first_segments(gpu, oracle, kind, route, static):
     lens = np.array(_lengths(kind), dtype=np.uint64)
@@ -78,3 +80,25 @@ def test_table_unlike_its_first_segments(gpu, oracle, kind, route, static):
         a.free()
         b.free()
         table.free()
+
+
+@pytest.mark.parametrize("count,size,static", [(3, (256 << 20) + 48, True), (20, (260 << 20) + 16, False), (20, (130 << 20) + 3, True)])
+def test_table_of_a_few_very_long_segments(gpu, count, size, static):
+    """Gigabytes in a few segments, compared on the GPU."""
+    torch = pytest.importorskip("torch")
+    step = (size + 4095) // 4096 * 4096
+    source = torch.randint(-2**63, 2**63 - 1, (count * step // 8,), dtype=torch.int64, device="cuda").view(torch.uint8)
+    target = torch.zeros_like(source)
+    at = np.arange(count, dtype=np.uint64) * np.uint64(step)
+    rows = np.stack([source.data_ptr() + at, target.data_ptr() + at[::-1], np.full(count, size, dtype=np.uint64)], axis=1).astype(np.uint64)
+    table = torch.from_numpy(rows.view(np.int64)).cuda()
+    torch.cuda.synchronize()
+    entry = gpu.mf_xcopy_device_table_static if static else gpu.mf_xcopy_device_table
+    for _ in range(2):
+        target.zero_()
+        torch.cuda.synchronize()
+        assert entry(table.data_ptr(), count, native.ROUTE_HBM, None) == 0, native.last_error()
+        assert gpu.mfrt_device_sync() == 0
+        got = target.view(count, step).flip(0)
+        assert torch.equal(got[:, :size], source.view(count, step)[:, :size])
+        assert not got[:, size:].any()

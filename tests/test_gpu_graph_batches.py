@@ -32,6 +32,8 @@ def _batch(kind, seed):
         lens = np.full(129, 8192)
     elif kind == "300 ragged":
         lens = rng.integers(0, 150000, 300)
+    elif kind == "20000 short":                              # a table beyond one of the lists for recorded calls
+        lens = np.concatenate([rng.integers(0, 800, 19000), rng.integers(16385, 17000, 1000)])
     elif kind == "4000 short":
         lens = rng.integers(0, 3000, 4000)
     else:                                                    # a table: one segment far beyond the others
@@ -48,13 +50,14 @@ def _batch(kind, seed):
 
 
 @pytest.mark.parametrize("form, kind", [("batch", "few, apart modulo 16"), ("batch", "128 ragged, apart"), ("batch", "129 pages"),
-                                        ("batch", "300 ragged"), ("batch", "4000 short"), ("table", "300 ragged"), ("table", "one long")])
+                                        ("batch", "300 ragged"), ("batch", "4000 short"), ("table", "300 ragged"), ("table", "one long"),
+                                        ("table", "20000 short")])
 def test_captured_and_replayed_between_plain_calls(gpu, oracle, form, kind):
     torch = pytest.importorskip("torch")
     assert torch.cuda.is_available()
     pool = gpu_util.DeviceBuffer(gpu, POOL)
     other = gpu_util.DeviceBuffer(gpu, POOL)
-    table = gpu_util.DeviceBuffer(gpu, 24 * 4096)
+    table = gpu_util.DeviceBuffer(gpu, 24 * 20000)
     stream = torch.cuda.Stream()
     raw = stream.cuda_stream
     src, dst, lens = _batch(kind, 1)
