@@ -42,6 +42,8 @@ def _lengths(kind):
         return [0, 5 << 20, 33]
     if kind == "one":
         return [9 << 20]
+    if kind == "turns":                                          # ragged, and a grid (6000) that is a multiple of the 16 parts
+        return [16 * CHUNK - 3] + [i * 7919 % (16 * CHUNK) for i in range(1498)] + [7 * OWN * 16 + 5]
     if kind == "pairs of launches":                              # more segments than a list has room for, long ones in each part
         return [i * 7 % 300 for i in range(65000)] + [OWN + PIECE + 5] * 900 + [i * 7 % 300 for i in range(300)]
     return [5] * 8 + [OWN + 16 + i % 32 for i in range(11000)]   # "list": more long segments than a wave has lanes
@@ -51,6 +53,7 @@ def _lengths(kind):
     ("short first", native.ROUTE_HBM, False), ("long first", native.ROUTE_HBM, False), ("few", native.ROUTE_HBM, False),
     ("one", native.ROUTE_HBM, False), ("short first", native.ROUTE_TO_HOST, False), ("long first", native.ROUTE_FROM_HOST, False),
     ("long first", native.ROUTE_HBM, True), ("list", native.ROUTE_HBM, True), ("pairs of launches", native.ROUTE_HBM, False),
+    ("turns", native.ROUTE_HBM, False), ("turns", native.ROUTE_TO_HOST, False),
 ])
 def test_table_unlike_its_first_segments(gpu, oracle, kind, route, static):
     lens = np.array(_lengths(kind), dtype=np.uint64)
