@@ -104,7 +104,7 @@ class BigMemory:
 
     def copy_data_batch(self, src_addrs, dst_addrs, sizes, count, type, flags=0):  # noqa: A002
         """The first `count` elements of three sequences of integers.  Arrays of 64-bit integers (numpy) are handed over
-        as they are."""
+        as they are; they may be read-only, and must not be written to by another thread before the call returns."""
         return native.calls().copy_batch(self._h, src_addrs, dst_addrs, sizes, count, type, flags)
 
     def wait(self):

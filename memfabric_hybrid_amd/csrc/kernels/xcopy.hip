@@ -959,7 +959,7 @@ int WithPolicy(const Policy &policy, Launch launch)
 uint32_t LanesFor(uint32_t units, int route)
 {
     if (route == MFRT_ROUTE_TO_HOST || route == MFRT_ROUTE_FROM_HOST) {
-        return kXcopyThreads;   // link routes were tuned with four-wave workgroups, one per CU
+        return kXcopyThreads;   // link routes were tuned with four-wave workgroups, few of them (GridFor)
     }
     const uint32_t lanes = units / kDepth;
     return lanes <= 64 ? 64u : (lanes <= 128 ? 128u : kXcopyThreads);

@@ -247,7 +247,7 @@ def test_pinned_host_routes(gpu, oracle):
 
 
 def _device_table_case(kind, count, rng, pool):
-    """(src, dst, lens) offsets of one table for the device-side planner."""
+    """(src, dst, lens) offsets of one table in device memory."""
     half = pool // 2
     if kind == "ragged":
         return workloads.ragged_batch(count * 3 + 1, pool, count, max_len=min(9000, half // count - 64))
@@ -285,9 +285,9 @@ def _device_table_case(kind, count, rng, pool):
     ("gaps", 6000), ("gaps", 30000), ("empty", 3000), ("long", 400), ("long", 12000),
 ])
 def test_device_resident_table(gpu, oracle, kind, count):
-    """A {src, dst, len} table the host cannot read is planned on the GPU: by one workgroup up to 8192 segments (1, 2, 4 or
-    8 tiles of 1024), by one workgroup per 1024 segments beyond; chunk counts that repeat are found there and take the
-    launch without a prefix, the rest the group map, whose groups empty segments and long segments stretch."""
+    """A {src, dst, len} table the host cannot read is copied without a plan: every segment in as many parts as the longest of the
+    first eight has chunks, walked by a grid sized from the segment count; what long segments hold beyond goes through a list to
+    a second launch.  Pages, segments of other lengths than the first ones, empty ones, and tables shorter and longer than the grid."""
     pool = 96 * MIB
     rng = np.random.default_rng(count + len(kind))
     src, dst, lens = _device_table_case(kind, count, rng, pool)

@@ -107,7 +107,7 @@ def test_static_entry_point_captured_in_a_graph_and_replayed(gpu, oracle):
         for count, seed, kind in ((9000, 91, "ragged"), (700, 92, "pages")):
             if kind == "ragged":
                 src, dst, lens = workloads.ragged_batch(seed, POOL, count, max_len=3000)
-            else:   # equal pages: the planner finds the repeating chunk counts, the copy takes the form without a prefix
+            else:   # equal pages: every item of the table has something to copy
                 rng = np.random.default_rng(seed)
                 src = rng.permutation(count).astype(np.uint64) * np.uint64(32768)
                 dst = np.uint64(POOL // 2) + rng.permutation(count).astype(np.uint64) * np.uint64(32768)
