@@ -736,13 +736,16 @@ __global__ __launch_bounds__(kLanes) void XcopyPieceKernel(const Piece *__restri
 // the segment count alone, so a workgroup walks the items with the grid as its stride; it fetches the next item's triple before
 // it copies the current item.  What bounds it is HBM; a launch in front of it that planned the table (chunk prefix, owner map,
 // repeating pattern) took 8 us, after which the copy was no faster: 4096 pages of 32 KiB scattered 60.0 / 52.8 us with the
-// planner / so, 16 080 pages of 8 KiB 76.7 / 57.9, 100 pages 10.0 / 7.1.  In a ragged table part numbers turn from segment to
-// segment: the grid is often a multiple of the parts, and a workgroup that met the same part of every segment found something to
-// copy in all of them, or in none.  In the slower / faster mode that a pool's place decides, us with the planner, without the turn and
-// so: 2000 segments of up to 70 KB in 48 GiB 45.4 / 40.4, 50.5 / 46.3, 42.5 / 37.3; 16 384 of up to 262 KB 949 / 777, 969 / 775, 963 / 767.
-// Pages keep their order, which is 1 % faster (scatter 55.6 / 56.2).  (The triples of 64 items at a time, one per lane, so that empty items
-// cost no wait: more registers than eight waves per SIMD have, 10 to 60 % slower on short tables; two triples ahead instead of
-// one: no faster, 16 384 segments of 2 to 14 KB 4 % slower.)
+// planner / so, 16 080 pages of 8 KiB 76.7 / 57.9, 100 pages 10.0 / 7.1.
+// A ragged table has an odd number of parts: workgroups go to the eight XCDs in turn, and with an even number the first parts,
+// which every segment has, went to some and the last, which few have, to others.  In the slower / faster of the two modes that
+// the place of a pool decides, us with the planner, with an even number and so: 16 384 segments of 2 to 14 KB 87.1 / 77.5, 79.4 / 74.1,
+// 66 / 57.5; 4000 K and V blocks 139.4 / 138.1, 160 / 160, 135.5 / 135.5; 2000 of up to 70 KB 43.4 / 38.7, 40.2 / 35.4, 39.3 / 34.6 and spread over
+// 48 GiB 45.4 / 40.4, 50.5 / 46.3, 41.4 / 36.5.  16 384 of up to 262 KB are none the faster for it: 949 / 778, 967 / 774, 967 / 773.
+// Not taken: eight workgroups per segment, 1 to 7 % faster where segments have dozens of chunks, 16 080 pages of 8 KiB 24 % slower;
+// part numbers that turn from segment to segment, pages 1 % slower; the triples of 64 items at a time, one per lane, so that
+// empty items cost no wait, more registers than eight waves per SIMD have, 10 to 60 % slower on short tables; two triples ahead
+// instead of one, 16 384 segments of 2 to 14 KB 4 % slower.
 template <bool kNtLoad, int kStore>
 __global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_t *__restrict__ triples, uint32_t nseg, uint32_t units,
                                                                    RestList *__restrict__ rest, uint32_t capacity)
@@ -757,6 +760,7 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_
         parts = chunks > parts ? chunks : parts;
         least = chunks < least ? chunks : least;
     }
+    parts |= least == parts ? 0u : 1u;      // odd in a ragged table: every XCD gets each of them in turn
     uint32_t seg = blockIdx.x / parts;
     uint32_t part = blockIdx.x - seg * parts;
     if (seg >= nseg) {
@@ -764,9 +768,6 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_
     }
     const uint32_t segStep = gridDim.x / parts;
     const uint32_t partStep = gridDim.x - segStep * parts;
-    const uint32_t turns = least == parts ? 1 : parts;
-    const uint32_t turnStep = segStep % turns;
-    uint32_t turn = seg % turns;                                           // added to the part, modulo the parts
     const uint64_t own = static_cast<uint64_t>(parts) * kDirectRounds;     // chunks of a segment that are copied here
     uint64_t src = triples[3ull * seg];
     uint64_t dst = triples[3ull * seg + 1];
@@ -780,8 +781,7 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_
         const uint64_t ndst = t[1];
         const uint64_t nlen = t[2];
         const uint64_t chunks = SegmentChunks(dst, len, units);
-        const uint32_t mine = part + turn < parts ? part + turn : part + turn - parts;
-        for (uint64_t c = mine; c < chunks && c < own; c += parts) {
+        for (uint64_t c = part; c < chunks && c < own; c += parts) {
             CopyChunk<kNtLoad, kStore>(src, dst, len, c, units);
         }
         if (part == 0 && chunks > own) {
@@ -799,8 +799,6 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_
         }
         seg = static_cast<uint32_t>(next);
         part = part + partStep - (carry != 0 ? parts : 0);
-        turn += turnStep + carry;
-        turn -= turn >= turns ? turns : 0;
         src = Uniform(nsrc);
         dst = Uniform(ndst);
         len = Uniform(nlen);

@@ -42,7 +42,7 @@ def _lengths(kind):
         return [0, 5 << 20, 33]
     if kind == "one":
         return [9 << 20]
-    if kind == "turns":                                          # ragged, and a grid (6000) that is a multiple of the 16 parts
+    if kind == "turns":                                          # ragged, an even number of chunks at the most: one part more
         return [16 * CHUNK - 3] + [i * 7919 % (16 * CHUNK) for i in range(1498)] + [7 * OWN * 16 + 5]
     if kind == "pairs of launches":                              # more segments than a list has room for, long ones in each part
         return [i * 7 % 300 for i in range(65000)] + [OWN + PIECE + 5] * 900 + [i * 7 % 300 for i in range(300)]
