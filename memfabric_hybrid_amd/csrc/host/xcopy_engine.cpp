@@ -688,9 +688,9 @@ int EnsureDevice(StagingSlot &slot, uint64_t bytes)
     return BM_OK;
 }
 
-RestList *RestListAt(void *lists, uint32_t i, uint32_t capacity)
+uint64_t RestListStride(uint32_t capacity)
 {
-    return reinterpret_cast<RestList *>(static_cast<uint8_t *>(lists) + i * RoundUp(RestListBytes(capacity), 256));
+    return RoundUp(RestListBytes(capacity), 256);
 }
 
 int EnsureRestLists(void *&lists, uint32_t count, uint32_t capacity)
@@ -698,20 +698,13 @@ int EnsureRestLists(void *&lists, uint32_t count, uint32_t capacity)
     if (lists != nullptr) {
         return BM_OK;
     }
-    lists = mfrt_alloc_device(count * RoundUp(RestListBytes(capacity), 256));
+    lists = mfrt_alloc_device(count * RestListStride(capacity));
     if (lists == nullptr) {
         MF_FAIL(BM_MALLOC_FAILED, "lists of " << capacity << " segments could not be allocated in HBM");
     }
     // cleared once, on a stream of the engine: the caller's may be recording
     void *own = XcopyEngine::Instance().ThreadStream();
-    int err = own == nullptr ? -1 : 0;
-    for (uint32_t i = 0; i < count && err == 0; ++i) {
-        RestList *list = RestListAt(lists, i, capacity);
-        err = mfk_xcopy_signal(&list->taken, 0, own);
-        for (uint32_t g = 0; g <= kRestGroups && err == 0; ++g) {
-            err = mfk_xcopy_signal(&list->done[g].count, 0, own);
-        }
-    }
+    const int err = own == nullptr ? -1 : mfk_xcopy_clear_lists(lists, count, RestListStride(capacity), own);
     if (err != 0 || mfrt_stream_sync(own) != 0) {
         (void)mfrt_free_device(lists);
         lists = nullptr;
@@ -2057,7 +2050,8 @@ int XcopyEngine::SubmitDeviceTable(const void *triples, uint32_t n, int route, v
     if (ret != BM_OK) {
         return ret;
     }
-    void *list = recorded ? RestListAt(lease.graphRests, lease.graphCursor++ % kSlots, kRestGraphCapacity) : slot->rest;
+    void *list = recorded ? static_cast<uint8_t *>(lease.graphRests) + lease.graphCursor++ % kSlots * RestListStride(kRestGraphCapacity)
+                          : slot->rest;
     void *event = recorded ? nullptr : EventOfLaunch(lease, *slot, stream);
     const uint32_t cu = mfrt_cu_count();
     const uint32_t units = ChooseUnits(0, cu, route, tuning_);   // sizes are only known on the GPU

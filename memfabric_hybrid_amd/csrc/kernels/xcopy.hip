@@ -910,6 +910,15 @@ __global__ __launch_bounds__(kRestLanes) void XcopyRestKernel(RestList *rest, ui
     }
 }
 
+// The heads of lists that are new, one a workgroup.
+__global__ void XcopyClearListsKernel(uint8_t *lists, uint64_t stride)
+{
+    uint64_t *head = reinterpret_cast<uint64_t *>(lists + blockIdx.x * stride);
+    for (uint32_t i = threadIdx.x; i < kRestHeadBytes / 8; i += blockDim.x) {
+        head[i] = 0;
+    }
+}
+
 Policy PolicyOf(int route)
 {
     switch (route) {
@@ -1247,6 +1256,14 @@ extern "C" int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t uni
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
+// Makes `count` lists `stride` bytes apart empty.
+extern "C" int mfk_xcopy_clear_lists(void *lists, uint32_t count, uint64_t stride, void *stream)
+{
+    using namespace mf;
+    hipLaunchKernelGGL(XcopyClearListsKernel, dim3(count), dim3(64), 0, static_cast<hipStream_t>(stream), static_cast<uint8_t *>(lists), stride);
+    return static_cast<int>(hipGetLastError());
+}
+
 // Every copy kernel once, on plans that hold nothing, so that a caller who captures a stream later finds the code of
 // this file loaded and every kernel known to the runtime (a kernel's first launch is not capturable).
 extern "C" int mfk_xcopy_prelaunch(void *stream)
@@ -1464,6 +1481,7 @@ extern "C" int mfk_xcopy_static_setup(void)
         RestList *rest = reinterpret_cast<RestList *>(words);
         const uint64_t *none = reinterpret_cast<const uint64_t *>(words);
         hipLaunchKernelGGL(XcopySignalKernel, dim3(1), dim3(64), 0, nullptr, rest->reserved, 0u);
+        hipLaunchKernelGGL(XcopyClearListsKernel, dim3(1), dim3(64), 0, nullptr, reinterpret_cast<uint8_t *>(rest), 0ull);
         for (int route = MFRT_ROUTE_HBM; route <= MFRT_ROUTE_FROM_HOST; ++route) {
             (void)WithPolicy(PolicyOf(route), [&](auto ntLoad, auto store) {
                 return LaunchDirect<decltype(ntLoad)::value, decltype(store)::value>(none, 0, kXcopyThreads, 1, 1, 64, rest,

@@ -315,6 +315,7 @@ struct RestList {
     RestCount done[kRestGroups + 1];                  // workgroups of the second launch that are done with it, by group, and groups
     RestSegment entry[1];                             // as many as the list has room for
 };
+constexpr uint64_t kRestHeadBytes = sizeof(RestList) - sizeof(RestSegment);
 constexpr uint64_t kRestEntry = 1ull << 40;           // pieces of 64 KiB: 2^56 bytes
 constexpr uint32_t kRestCapacity = 65536;             // 2 MiB; a longer table goes in several pairs of launches
 constexpr uint32_t kRestGraphCapacity = 16384;        // of the lists for calls recorded into a graph

@@ -115,6 +115,8 @@ int mfk_xcopy_signal(void *word, uint32_t value, void *stream);
  * event: as for mfk_xcopy_pieces; NULL on a stream that records a graph. */
 int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *rest,
                      uint32_t capacity, void *mask, uint32_t maskValue, void *stream, void *event);
+/* Makes `count` mf::RestList in device memory, `stride` bytes apart, empty. */
+int mfk_xcopy_clear_lists(void *lists, uint32_t count, uint64_t stride, void *stream);
 /* The same with the list in a statically allocated device array instead of memory the engine allocates: no allocation
  * anywhere, at most MFK_STATIC_TABLE_SEGMENTS segments, one call at a time per GPU.  mfk_xcopy_static_setup looks the
  * array's address up for the current device (once per device, at start-up); mfk_xcopy_table_static returns -2 when that has

@@ -508,6 +508,13 @@ int mfk_xcopy_signal(void *word, uint32_t value, void *)
     __atomic_store_n(static_cast<uint64_t *>(word), static_cast<uint64_t>(value), __ATOMIC_RELEASE);
     return 0;
 }
+int mfk_xcopy_clear_lists(void *lists, uint32_t count, uint64_t stride, void *)
+{
+    for (uint32_t i = 0; i < count; ++i) {
+        std::memset(static_cast<uint8_t *>(lists) + i * stride, 0, mf::kRestHeadBytes);
+    }
+    return 0;
+}
 int mfk_xcopy_static_setup(void) { return 0; }
 int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *stream)
 {
