@@ -152,7 +152,7 @@ struct Batch {
     TablePlan hbm;                      // triples in HBM, owner by pattern
     TablePlan grouped;                  // triples, prefix and group map in HBM, no pattern
     const Piece *pieces;                // of 4 KiB, in pinned host memory: as many as nchunk
-    const Piece *deepPieces;            // of 16 KiB (what the library takes for 24 to 64 MiB)
+    const Piece *deepPieces;            // of 16 KiB (what the library takes for 4 to 64 MiB)
     uint32_t ndeep;
     uint64_t bytes;
     uint32_t nchunk;
@@ -373,15 +373,16 @@ void LaunchInlineProduct(const InlinePlan &plan, hipStream_t s, bool held, bool 
     }
 }
 
-// What the library launches for more than kInlineSegs segments: up to 24 MiB in waves of 4 KiB, up to 64 MiB in waves of 16 KiB,
-// stores held back by the rule of the kernel-argument form and what the engine adds for descriptors behind the link.
+// What the library launches for more than kInlineSegs segments of up to 64 MiB: waves of 16 KiB, stores held back by the rule of the
+// kernel-argument form, up to 24 MiB for as many chunks of 4 KiB, and what the engine adds for descriptors behind the link.
 void LaunchPiecesProduct(const Batch &b, hipStream_t s)
 {
     const bool deep = b.bytes > kDeepMinBytes && b.bytes <= kDeepMaxBytes;
-    const uint32_t units = b.bytes > kDeepMinBytes ? kDeepUnits : kXcopyThreads;
-    const uint32_t count = units == kDeepUnits ? b.ndeep : b.nchunk;
-    const uint32_t rule = HoldNanosFor(count, count, units, false);
-    const int err = mfk_xcopy_pieces(units == kDeepUnits ? b.deepPieces : b.pieces, count, b.bytes, units, nullptr, 0, s,
+    const uint32_t units = kDeepUnits;
+    const uint32_t count = b.ndeep;
+    const uint32_t chunks = b.nchunk < kHoldMaxChunks ? b.nchunk : kHoldMaxChunks;
+    const uint32_t rule = b.bytes <= kDeepMinBytes ? HoldNanosFor(chunks, chunks, kXcopyThreads, false) : HoldNanosFor(count, count, units, false);
+    const int err = mfk_xcopy_pieces(b.deepPieces, count, b.bytes, units, nullptr, 0, s,
                                      rule != 0 ? rule + (deep ? kHoldLookupDeepExtraNanos : kHoldLookupExtraNanos) : 0, nullptr);
     if (err != 0) {
         std::fprintf(stderr, "mfk_xcopy_pieces failed: %d\n", err);

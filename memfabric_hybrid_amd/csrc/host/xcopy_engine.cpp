@@ -1533,30 +1533,103 @@ uint32_t XcopyEngine::HoldFor(const InlinePlan &plan, uint32_t grid, int route, 
     return with > 0 ? static_cast<uint32_t>(with) : 0;
 }
 
-// Hold of a launch of pieces, as that of a table of `count` chunks whose waves fetch their descriptors across the host link and
-// issue their loads that much later than those of a launch whose descriptors are kernel arguments.  (The launcher takes off
-// what pieces wait less, PieceLessNanos, so a wait set by hand, which is meant as it is, gets that on top.)
-uint32_t XcopyEngine::HoldForPieces(uint32_t count, uint64_t bytes, uint32_t units, bool unordered) const
+BatchStats StatsOf(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n)
+{
+    BatchStats st;
+    for (uint32_t i = 0; i < n; ++i) {
+        st.total += len[i];
+        st.longest = len[i] > st.longest ? len[i] : st.longest;
+        st.addressBits |= src[i] | dst[i];
+        st.lengthBits |= len[i];
+    }
+    return st;
+}
+
+bool WrittenInOrder(const uint64_t *dst, const uint64_t *len, uint32_t n)
+{
+    const uint32_t seen = n < 256 ? n : 256;
+    uint32_t following = 0;
+    for (uint32_t i = 1; i < seen; ++i) {
+        following += dst[i - 1] + len[i - 1] == dst[i] ? 1 : 0;
+    }
+    return following >= seen / 2;
+}
+
+// Hold of a launch of pieces, as that of a table of as many chunks whose waves fetch their descriptors across the host link and
+// issue their loads that much later than those of a launch whose descriptors are kernel arguments; of a batch of up to
+// kDeepMinBytes, of its chunks of 4 KiB, whatever its pieces.  (The launcher takes off what pieces wait less, PieceLessNanos, so a
+// wait set by hand, which is meant as it is, gets that on top.)
+uint32_t XcopyEngine::HoldForPieces(const BatchStats &stats, uint32_t n, uint32_t count, uint32_t units, bool unordered) const
 {
     if (unordered || tuning_.holdNanos == 0) {
         return 0;
     }
-    if ((count > kHoldSharedMaxChunks || units == kDeepUnits) && g_leasesOut.load(std::memory_order_relaxed) > 1) {
+    if ((count > kHoldSharedMaxChunks || units != kXcopyThreads) && g_leasesOut.load(std::memory_order_relaxed) > 1) {
         return 0;
     }
-    const uint32_t rule = HoldNanosFor(count, count, units, false);
+    const bool byChunks = stats.total <= kDeepMinBytes && units != kXcopyThreads && count <= kDeepMaxChunks;
+    constexpr uint64_t kChunkBytes = static_cast<uint64_t>(kXcopyThreads) * kUnitBytes;
+    const uint64_t allChunks = (stats.total + kChunkBytes - 1) / kChunkBytes + (stats.lengthBits % kChunkBytes != 0 ? n / 2 : 0);
+    const uint32_t chunks = static_cast<uint32_t>(std::min<uint64_t>(allChunks, kHoldMaxChunks));
+    // pieces of 8 KiB, two waves of four loads per lane, wait as those of 16 KiB for the same bytes
+    const uint32_t rule = byChunks ? HoldNanosFor(chunks, chunks, kXcopyThreads, false)
+                          : units != kDeepUnits / 2 ? HoldNanosFor(count, count, units, false)
+                          : count <= kDeepMaxChunks ? HoldNanosFor(count / 2, count / 2, kDeepUnits, false)
+                                                    : 0;
     if (rule == 0) {
         return 0;
     }
     if (tuning_.holdNanos > 0) {
-        return static_cast<uint32_t>(tuning_.holdNanos) + PieceLessNanos(count, bytes, units);
+        return static_cast<uint32_t>(tuning_.holdNanos) + PieceLessNanos(count, stats.total, units);
     }
     if (tuning_.holdCalibratedOff) {
         return 0;
     }
-    const int32_t extra = tuning_.holdPinnedExtraNanos + (units == kDeepUnits ? kHoldPinnedDeepExtraNanos : 0);
+    const int32_t extra = tuning_.holdPinnedExtraNanos + (!byChunks && units != kXcopyThreads ? kHoldPinnedDeepExtraNanos : 0);
     const int64_t with = static_cast<int64_t>(rule) + extra + tuning_.holdDeltaNanos;
     return with > 0 ? static_cast<uint32_t>(with) : 0;
+}
+
+// Units of the pieces of a batch.  Waves that are resident together hold their stores, and from kPieceLongMinBytes on the longer
+// pieces are the better shape for that (see there) as long as 4096 of them hold the batch: one wave of 16 KiB, or two of 4 KiB
+// where no segment has more than 8 KiB (4096 pages of 8 KiB 12.0 us, 14.5 without hold, 12.9 in waves of 16 KiB).  Beyond, what the
+// usual segment fills: each workgroup twice the size halves the descriptors the host writes and the link carries, but lanes
+// without a unit cost (16 080 pages of 8 KiB 45.2 / 46.1 / 47.0 us with one, two and four waves; 4096 of 32 KiB 45.8 / 46.8 / 46.4).
+// Threads with streams of their own hold nothing but 4 KiB pieces (HoldFor).
+uint32_t XcopyEngine::PieceUnits(const BatchStats &stats, uint32_t n, bool unordered) const
+{
+    const uint64_t mean = stats.total / n;
+    const bool holds = !unordered && tuning_.holdNanos != 0 && tuning_.deepHold && g_leasesOut.load(std::memory_order_relaxed) <= 1;
+    constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kDeepUnits) * kUnitBytes;
+    const uint64_t deepPieces = n + (stats.longest + kPieceAlign <= kDeepBytes ? 0 : stats.total / kDeepBytes);   // at the most
+    if (holds && stats.total > kPieceLongMinBytes && stats.total <= kDeepMaxBytes && stats.longest > kXcopyThreads * kUnitBytes &&
+        deepPieces <= kDeepMaxChunks) {
+        return mean > 6144 && stats.longest <= kDeepUnits / 2 * kUnitBytes ? kDeepUnits / 2 : kDeepUnits;
+    }
+    if (stats.total <= kDeepMinBytes) {
+        return kXcopyThreads;
+    }
+    return mean <= 6144 ? kXcopyThreads : mean <= 12288 ? kDeepUnits / 2 : kDeepUnits;
+}
+
+// Of 6.0 TB/s, which blocks at random places hold; of 6.4 for long ones that are written one behind the other, which leaves the
+// rows of HBM open (short ones hold that in some places of the pool only, and gain nothing at 6.0: 16 384 pages of 32 KiB gathered 182 us
+// without windows, 171 to 194 at 6.4, 181 at 6.0; the kernel has the other figures).  Pieces that are much less than full gain
+// nothing; segments between cache lines keep the launch without windows, as they do in launches of kInlineSegs segments up to
+// kWindowSliceMinSegmentBytes.
+uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t count, uint32_t units,
+                                      bool unordered) const
+{
+    constexpr uint64_t kLongBytes = 64ull << 10;
+    const bool full = stats.total >= static_cast<uint64_t>(count) * (kDeepUnits * kUnitBytes) / 100 * 85;
+    if (unordered || units != kDeepUnits || !full || (stats.addressBits & (kWindowAlignBytes - 1)) != 0 ||
+        !WindowsApply(stats.total, MFRT_ROUTE_HBM, kPieceWindowMinBytes)) {
+        return 0;
+    }
+    if (WrittenInOrder(dst, len, n)) {
+        return stats.total / n >= kLongBytes ? tuning_.windowMBps / 17 * 16 : 0;
+    }
+    return tuning_.windowMBps / 17 * 15;
 }
 
 bool XcopyEngine::DeepHoldApplies(uint64_t bytes, uint32_t n, int route, bool unordered) const
@@ -1750,7 +1823,7 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         if (deep && (apartBits & (kUnitBytes - 1)) != 0 && mfrt_stream_capturing(stream) == 0) {
             // as pieces: sixteen loads per lane of aligned units and what shifts them, with the table of the kernel arguments, take
             // more registers than sixteen waves per CU have (42 MB 17.5 us with straddling loads)
-            const int ret = SubmitPieces(src, dst, len, n, total, kDeepUnits, stream, mask, maskValue, unordered);
+            const int ret = SubmitPieces(src, dst, len, n, StatsOf(src, dst, len, n), kDeepUnits, stream, mask, maskValue, unordered);
             if (ret != kNotLaunched) {
                 return ret;
             }
@@ -1794,14 +1867,8 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         return SubmitRecorded(src, dst, len, n, route, stream, mask, maskValue);
     }
     {
-        uint64_t total = 0;
-        uint64_t longest = 0;
-        uint64_t addressBits = 0;
-        for (uint32_t i = 0; i < n; ++i) {
-            total += len[i];
-            longest = len[i] > longest ? len[i] : longest;
-            addressBits |= src[i] | dst[i];
-        }
+        const BatchStats stats = StatsOf(src, dst, len, n);
+        const uint64_t total = stats.total;
         queuedBytes = total;
         // A table of long segments between HBM addresses is cut into launches of kInlineSegs segments, each of which
         // then takes the form with read and write windows: the few extra launches cost microseconds, the windows
@@ -1815,7 +1882,7 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         // the 896 long segments in one windowed table launch are no faster than in seven launches of the kernel-argument form.
         if (maySlice && n > kInlineSegs && route == MFRT_ROUTE_HBM && !unordered && tuning_.windowMBps != 0 && windowsAvailable_ &&
             tuning_.unitsOverride == 0 &&
-            total / n >= ((addressBits & (kWindowAlignBytes - 1)) == 0 && tuning_.windowAlignedMBps != 0 ? kWindowSliceMinAlignedSegmentBytes
+            total / n >= ((stats.addressBits & (kWindowAlignBytes - 1)) == 0 && tuning_.windowAlignedMBps != 0 ? kWindowSliceMinAlignedSegmentBytes
                                                                                                          : kWindowSliceMinSegmentBytes) &&
             g_leasesOut.load(std::memory_order_relaxed) <= 1) {
             for (uint32_t at = 0; at < n; at += kInlineSegs) {
@@ -1831,7 +1898,7 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         }
         units = ChooseUnits(total, cu, route, tuning_);
         if (route == MFRT_ROUTE_HBM) {
-            const int ret = SubmitPieces(src, dst, len, n, total, units, stream, mask, maskValue, unordered);
+            const int ret = SubmitPieces(src, dst, len, n, stats, units, stream, mask, maskValue, unordered);
             if (ret != kNotLaunched) {
                 return ret;
             }
@@ -1843,9 +1910,9 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         }
         // Many short segments: a chunk size that holds the longest of them gives every segment exactly
         // one chunk, which is the equal-count form below (no prefix, no search).
-        if (tuning_.unitsOverride == 0 && longest != 0) {
+        if (tuning_.unitsOverride == 0 && stats.longest != 0) {
             for (uint32_t u = units; u <= 4 * kXcopyThreads; u *= 2) {
-                if (longest <= static_cast<uint64_t>(u) * kUnitBytes - kUnitBytes) {
+                if (stats.longest <= static_cast<uint64_t>(u) * kUnitBytes - kUnitBytes) {
                     units = u;
                     break;
                 }
@@ -1966,22 +2033,14 @@ int XcopyEngine::SubmitRecorded(const uint64_t *src, const uint64_t *dst, const 
 }
 
 // A batch between HBM addresses in one launch of pieces; kNotLaunched where their list would outgrow the batch.
-int XcopyEngine::SubmitPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t total, uint32_t units,
+int XcopyEngine::SubmitPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, const BatchStats &stats, uint32_t units,
                               void *stream, void *mask, uint32_t maskValue, bool unordered)
 {
-    const uint64_t mean = total / n;
+    const uint64_t total = stats.total;
     if (tuning_.unitsOverride != 0) {
         units = units <= kXcopyThreads ? kXcopyThreads : units <= 2 * kXcopyThreads ? 2 * kXcopyThreads : kDeepUnits;
-    } else if (DeepHoldApplies(total, n, MFRT_ROUTE_HBM, unordered)) {
-        units = kDeepUnits;
-        // ragged enough to exceed the waves that hold: not held
-    } else if (total > kDeepMinBytes) {
-        // Up to 24 MiB waves of 4 KiB are resident together and hold their stores.  Beyond, what the usual segment fills: each
-        // workgroup twice the size halves the descriptors the host writes and the link carries, but lanes without a unit cost
-        // (16 080 pages of 8 KiB 45.2 / 46.1 / 47.0 us with one, two and four waves; 4096 of 32 KiB 45.8 / 46.8 / 46.4).
-        units = mean <= 6144 ? kXcopyThreads : mean <= 12288 ? 2 * kXcopyThreads : kDeepUnits;
     } else {
-        units = kXcopyThreads;
+        units = DeepHoldApplies(total, n, MFRT_ROUTE_HBM, unordered) ? kDeepUnits : PieceUnits(stats, n, unordered);
     }
     // A few segments of gigabytes would make a list of millions of pieces, megabytes that take the host longer to write than a chunk
     // prefix takes the GPU to read.
@@ -2004,7 +2063,9 @@ int XcopyEngine::SubmitPieces(const uint64_t *src, const uint64_t *dst, const ui
         return mfk_xcopy_inline(&empty, MFRT_ROUTE_HBM, 1, mask, maskValue, stream, 0, 0) == 0 ? BM_OK : BM_ERROR;
     }
     void *event = EventOfLaunch(lease, *slot, stream);
-    const int err = mfk_xcopy_pieces(pieces, count, total, units, mask, maskValue, stream, HoldForPieces(count, total, units, unordered), event);
+    const uint32_t rate = PieceWindowRate(stats, dst, len, n, count, units, unordered);
+    const int err = rate != 0 ? mfk_xcopy_pieces_windowed(pieces, count, total, rate, mask, maskValue, stream, event)
+                              : mfk_xcopy_pieces(pieces, count, total, units, mask, maskValue, stream, HoldForPieces(stats, n, count, units, unordered), event);
     if (err != 0) {
         (void)MarkQueued(lease, slot, stream, true);   // the launch may have gone out with only the word behind it failing
         MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(err));

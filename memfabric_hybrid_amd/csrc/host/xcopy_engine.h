@@ -42,6 +42,25 @@ void NormalizeSegments(const uint64_t *src, const uint64_t *dst, const uint64_t 
                        SegList &out);
 
 constexpr int32_t kHoldPinnedDeepExtraNanos = kHoldLookupDeepExtraNanos - kHoldLookupExtraNanos;
+// What the shape of a launch of pieces is chosen by, from one pass over a batch.
+struct BatchStats {
+    uint64_t total = 0;
+    uint64_t longest = 0;
+    uint64_t addressBits = 0;       // low bits that any address has set
+    uint64_t lengthBits = 0;        // and any length
+};
+BatchStats StatsOf(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n);
+// Whether most of the first segments of a batch are written one behind the other.
+bool WrittenInOrder(const uint64_t *dst, const uint64_t *len, uint32_t n);
+
+// A batch of this much and more is cut into pieces of 8 and 16 KiB.  Shorter ones keep 4 KiB, which more CUs share: 150 pages of 8 KiB
+// 2.8 us, 4.0 in waves of 16 KiB; 200 pages of 32 KiB 4.4 / 4.6.  From there on the longer pieces are as fast and a quarter of the
+// descriptors for the host to write, which had bounded those batches: a call of 500 pages of 32 KiB took 10.6 us, the launch 6.6 on
+// 4 KiB and 7.0 on 16; uneven segments gain on the GPU too (1000 of 5000 bytes 5.9 / 5.2, 500 of 40 000 9.5 / 8.9).
+constexpr uint64_t kPieceLongMinBytes = 4ull << 20;
+// Pieces in windows: below, too few periods pay for the halves of the first and the last one in which the chip only reads or only
+// writes (72 MB of K and V blocks 28.7 us without windows and 28.3 with them, 82 MB of pages 29.6 / 29.0, 90 MB of blocks 35.7 / 32.8).
+constexpr uint64_t kPieceWindowMinBytes = 80ull << 20;
 constexpr uint64_t kPieceListMin = 1ull << 18;     // pieces that any batch may be cut into, 4 MiB of descriptors
 
 struct XcopyTuning {
@@ -201,14 +220,18 @@ private:
     XcopyEngine() = default;
 
     uint32_t HoldFor(const InlinePlan &plan, uint32_t grid, int route, bool unordered) const;
-    uint32_t HoldForPieces(uint32_t count, uint64_t bytes, uint32_t units, bool unordered) const;
+    uint32_t HoldForPieces(const BatchStats &stats, uint32_t n, uint32_t count, uint32_t units, bool unordered) const;
+    uint32_t PieceUnits(const BatchStats &stats, uint32_t n, bool unordered) const;
+    // Rate of the windows a list of `count` pieces of `units` units is copied in, 0: in none.
+    uint32_t PieceWindowRate(const BatchStats &stats, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t count, uint32_t units,
+                             bool unordered) const;
     // Whether a batch of `bytes` in n segments is planned in chunks of kDeepUnits units, to hold the stores of 16 KiB per wave.
     bool DeepHoldApplies(uint64_t bytes, uint32_t n, int route, bool unordered) const;
     // A launch that stores the thread's word itself, where that is the faster form: kNotLaunched where it is not.
     static constexpr int kNotLaunched = 1;
     int LaunchDone(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t bytes, int route, void *stream,
                    uint32_t &ticket);
-    int SubmitPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t total, uint32_t units,
+    int SubmitPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, const BatchStats &stats, uint32_t units,
                      void *stream, void *mask, uint32_t maskValue, bool unordered);
     int SubmitRecorded(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, int route, void *stream, void *mask,
                        uint32_t maskValue);

@@ -732,6 +732,77 @@ __global__ __launch_bounds__(kLanes) void XcopyPieceKernel(const Piece *__restri
     }
 }
 
+// Pieces of kWindowUnits units in read and write windows, as XcopyWindowKernel walks chunks; every piece of the list begins on a
+// cache line in source and destination.  A wave requests its next piece's descriptor before it copies the current piece.
+// Bound: HBM, whose rows a random place opens for 256 bytes a channel, so the rate that holds is lower than that of long segments.
+// Back to back, us without windows / in windows cut for 6.0 / 6.4 / 6.8 TB/s: 4096 pages of 32 KiB gathered 46.9 / 47.1 / 44.7 / 48.1,
+// scattered 50.6 / 47.5 / 48.4 / 51.0, 12 000 scattered 146 / 137 / 148 / 152, 4096 of 64 KiB scattered 97.0 / 91.9 / 86.9 / 88.8,
+// K and V blocks of 128 and 16 KiB, 90 MB 35.7 / 32.8 / 36.4 / 37.0 and 144 MB 55.8 / 51.0 / 56.2 / 57.3, 1500 segments of 120 000 bytes
+// 70.2 / 63.6 / 68.8 / 71.7.  Pieces that are four fifths full gain nothing (8192 x 40 000 130 / 128 / 133 / 133), ragged ones at odd
+// addresses lose (4000 of up to 131 072 bytes 106 / 108 / 110 / 111).
+// (A schedule that stretches when sampled waves fall behind it was tried: it overshoots, 20 to 50 % slower than none.)
+// What a lane past the end of its piece loads is the last unit: a load under a condition would leave the registers of the
+// loop's last round alive in the others and take more of them than sixteen waves per CU have.
+__global__ __launch_bounds__(64) void XcopyPieceWindowKernel(const Piece *__restrict__ pieces, uint32_t count, uint32_t period, uint32_t seq)
+{
+    uint32_t at = PieceOf(blockIdx.x);
+    if (at >= count) {
+        return;
+    }
+    Piece next = pieces[at];
+    const uint32_t half = period / 2;
+    uint64_t slot = AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * half / gridDim.x;
+    for (;;) {
+        uint32_t tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));       // offsets are computed in each round instead of held through all of them
+        const uint64_t srcWord = Uniform(next.src);
+        const uint64_t dstWord = Uniform(next.dst);
+        const bool more = count - at > gridDim.x;
+        next = pieces[more ? at + gridDim.x : at];
+        const uint64_t src = srcWord & kPieceAddress;
+        const uint64_t dst = dstWord & kPieceAddress;
+        const uint32_t length = PieceLength(srcWord, dstWord);
+        const uint32_t body = length / kUnitBytes;
+        u32x4 v[kWindowDepth];
+        WaitForClock(slot);
+        if (body == kWindowUnits) {
+#pragma unroll
+            for (uint32_t j = 0; j < kWindowDepth; ++j) {
+                v[j] = LoadAligned(src + (j * 64 + tid) * kUnitBytes);
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            WaitForClock(slot + half);
+#pragma unroll
+            for (uint32_t j = 0; j < kWindowDepth; ++j) {
+                StoreUnit<kStoreStream>(dst + (j * 64 + tid) * kUnitBytes, v[j]);
+            }
+        } else if (body != 0) {
+#pragma unroll
+            for (uint32_t j = 0; j < kWindowDepth; ++j) {
+                const uint32_t u = j * 64 + tid < body ? j * 64 + tid : body - 1;
+                v[j] = LoadAligned(src + u * kUnitBytes);
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            WaitForClock(slot + half);
+#pragma unroll
+            for (uint32_t j = 0; j < kWindowDepth; ++j) {
+                if (j * 64 + tid < body) {
+                    StoreUnit<kStoreStream>(dst + (j * 64 + tid) * kUnitBytes, v[j]);
+                }
+            }
+        }
+        if (tid < length % kUnitBytes) {
+            const uint64_t off = body * kUnitBytes + tid;
+            CopyByte<kStoreStream>(src + off, dst + off);
+        }
+        if (!more) {
+            return;
+        }
+        at += gridDim.x;
+        slot += period;
+    }
+}
+
 // A table that only the GPU can read, copied as xcopy_plan.h says: item (segment, part), parts in a row.  The launch is sized from
 // the segment count alone, so a workgroup walks the items with the grid as its stride; it fetches the next item's triple before
 // it copies the current item.  What bounds it is HBM; a launch in front of it that planned the table (chunk prefix, owner map,
@@ -1198,12 +1269,14 @@ extern "C" int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t byt
     }
     const Piece *p = static_cast<const Piece *>(pieces);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const uint32_t ticks = units != 512 ? HoldTicks(PieceHoldNanos(holdNanos, count, bytes, units)) : 0;
+    const uint32_t ticks = HoldTicks(PieceHoldNanos(holdNanos, count, bytes, units));
     const hipEvent_t end = static_cast<hipEvent_t>(event);
     if (units == 256 && ticks != 0) {
         LaunchPieces<64, 4, true>(p, count, ticks, s, end);
     } else if (units == 256) {
         LaunchPieces<64, 4, false>(p, count, 0, s, end);
+    } else if (units == 512 && ticks != 0) {
+        LaunchPieces<128, 4, true>(p, count, ticks, s, end);
     } else if (units == 512) {
         LaunchPieces<128, 4, false>(p, count, 0, s, end);
     } else if (ticks != 0) {
@@ -1211,6 +1284,27 @@ extern "C" int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t byt
     } else {
         LaunchPieces<256, 4, false>(p, count, 0, s, end);
     }
+    const int err = static_cast<int>(hipGetLastError());
+    return err != 0 ? err : Signal(mask, maskValue, s);
+}
+
+// The same pieces, of up to kWindowUnits units, in windows cut for windowMBps.
+extern "C" int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t windowMBps, void *mask, uint32_t maskValue,
+                                         void *stream, void *event)
+{
+    using namespace mf;
+    if (pieces == nullptr || count == 0 || count > kPieceMaxCount) {
+        return -1;
+    }
+    // whole groups of pieces, evenly over the rounds; the last group of the list may be short
+    const uint32_t grid = (WindowGrid(count, kWindowWaves) + kPieceGroup - 1) / kPieceGroup * kPieceGroup;
+    const uint32_t ticks = WindowPeriodTicks(2 * bytes * grid / (count > grid ? count : grid), windowMBps);
+    if (ticks == 0) {
+        return static_cast<int>(hipErrorInvalidValue);
+    }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    LaunchWithEvent(XcopyPieceWindowKernel, grid, 64, s, static_cast<hipEvent_t>(event), static_cast<const Piece *>(pieces), count, ticks,
+                    NextWindowSeq());
     const int err = static_cast<int>(hipGetLastError());
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
@@ -1296,7 +1390,9 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
                 hipLaunchKernelGGL((XcopyPieceKernel<64, 4, true>), dim3(1), dim3(64), 0, s, nullptr, 0u, 0u);
                 hipLaunchKernelGGL((XcopyPieceKernel<64, 16, true>), dim3(1), dim3(64), 0, s, nullptr, 0u, 0u);
                 hipLaunchKernelGGL((XcopyPieceKernel<128, 4, false>), dim3(1), dim3(128), 0, s, nullptr, 0u, 0u);
+                hipLaunchKernelGGL((XcopyPieceKernel<128, 4, true>), dim3(1), dim3(128), 0, s, nullptr, 0u, 0u);
                 hipLaunchKernelGGL((XcopyPieceKernel<256, 4, false>), dim3(1), dim3(256), 0, s, nullptr, 0u, 0u);
+                hipLaunchKernelGGL(XcopyPieceWindowKernel, dim3(1), dim3(64), 0, s, nullptr, 0u, 64u, NextWindowSeq());
                 hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
             }
             return 0;

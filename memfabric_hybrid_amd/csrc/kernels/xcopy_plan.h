@@ -133,12 +133,18 @@ constexpr int32_t kHoldLookupDeepExtraNanos = 2000;
 // the rate of the rule above for the bytes that are not there.  Best waits beyond HoldNanosFor(count): K and V blocks of 10 / 18 /
 // 24 MB +400 / 200 / 400 ns, 27 / 36 / 45 / 54 / 63 MB on 16 KiB +400 / 800 / 800 / 1200 / 1000; ragged segments of 14 / 21 MB 0, 31 / 41 /
 // 52 MB -800 / -800 / -1200, where the bytes that are not there make 1000 / 1300 / 1700.
+// Pieces of 8 and 16 KiB of a batch of up to kDeepMinBytes wait as its chunks of 4 KiB would, but for the knee of that rule: best
+// waits beyond it with K and V blocks of 18 / 20 / 22 MB 0 / 40 / 250 ns, 23 MB of pages 300, on 8 KiB 8 / 16 / 25 MB of pages 200 / -100 / 300.
 constexpr uint32_t kPieceLeadNanos = 1400;
+constexpr uint64_t kPieceKneeBytes = 18000000;
 inline uint32_t PieceLessNanos(uint32_t count, uint64_t bytes, uint32_t units)
 {
+    if (units != kXcopyThreads && bytes <= kDeepMinBytes) {
+        return kPieceLeadNanos - (bytes > kPieceKneeBytes ? static_cast<uint32_t>((bytes - kPieceKneeBytes) * 7 / 100000) : 0);
+    }
     const uint64_t full = static_cast<uint64_t>(count) * units * kUnitBytes;
     const uint64_t missing = full > bytes ? (full - bytes) / kUnitBytes : 0;                 // units
-    return static_cast<uint32_t>(kPieceLeadNanos + missing * (units == kDeepUnits ? 215 : 180) / (100ull * kDeepUnits));
+    return static_cast<uint32_t>(kPieceLeadNanos + missing * (units != kXcopyThreads ? 215 : 180) / (100ull * kDeepUnits));
 }
 inline uint32_t PieceHoldNanos(uint32_t holdNanos, uint32_t count, uint64_t bytes, uint32_t units)
 {

@@ -100,6 +100,10 @@ int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, void *mask,
  * event (may be NULL): completes with the launch.  The stream must not be one that records a graph, whose launches cannot carry one. */
 int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, void *mask, uint32_t maskValue, void *stream,
                      uint32_t holdNanos, void *event);
+/* The same pieces, of up to mfk_xcopy_window_units() units, which all begin on cache lines in source and destination, in read and
+ * write windows cut for `windowMBps` MB/s of HBM traffic. */
+int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t windowMBps, void *mask, uint32_t maskValue,
+                              void *stream, void *event);
 /* Launches every copy kernel once on empty plans (a kernel's first launch is not capturable into a HIP graph). */
 int mfk_xcopy_prelaunch(void *stream);
 /* Times the calibration workloads on `stream` with HIP events, in 1 GiB of device memory it allocates and frees:

@@ -436,6 +436,20 @@ int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_
     return 0;
 }
 
+// The same in windows: the rate is noted, and a piece that begins between cache lines fails the launch.
+int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t windowMBps, void *mask, uint32_t maskValue,
+                              void *stream, void *event)
+{
+    const mf::Piece *p = static_cast<const mf::Piece *>(pieces);
+    for (uint32_t i = 0; p != nullptr && i < count; ++i) {
+        if (((p[i].src | p[i].dst) & 127u) != 0) {
+            return 722;
+        }
+    }
+    g_lastWindow = windowMBps;
+    return windowMBps == 0 ? -1 : mfk_xcopy_pieces(pieces, count, bytes, 1024, mask, maskValue, stream, 0, event);
+}
+
 // The direct copy of a device-resident table restated: the parts of every segment, and the pieces of what long ones have left out
 // of a list.
 int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int, uint32_t grid, uint32_t restGrid, void *rest,

@@ -28,12 +28,19 @@ def _lengths(kind, rng):
         return np.concatenate([rng.integers(1, 200000, 400), EDGES])
     if kind == "one wave":                                       # beyond 24 MiB the usual segment decides
         return np.concatenate([rng.integers(1, 9000, 7000), EDGES])
+    if kind == "held 8 KiB":                                     # no segment longer, 4096 pieces at the most
+        return np.concatenate([rng.integers(7000, 8065, 2900), [1, 0, 8064, 8065, 17, 4096]])
+    if kind == "windows":                                        # nearly full pieces, 80 MiB and more; a round and a fraction of 4096
+        return np.concatenate([rng.integers(111000, 131000, 760), EDGES])
+    if kind == "windows, three rounds":
+        return np.concatenate([np.full(8193, 16384), [16384 + 15, 16383, 1, 0]])
     if kind == "two waves":
         return np.concatenate([rng.integers(1, 20000, 3000), EDGES])
     return np.concatenate([rng.integers(1, 90000, 2000), EDGES])   # "four waves"
 
 
-@pytest.mark.parametrize("kind", ["every shift", "held 4 KiB", "held 16 KiB", "one wave", "two waves", "four waves"])
+@pytest.mark.parametrize("kind", ["every shift", "held 4 KiB", "held 16 KiB", "held 8 KiB", "one wave", "two waves", "four waves", "windows",
+                                  "windows, three rounds"])
 @pytest.mark.parametrize("odd", [True, False])
 def test_batch_in_pieces(gpu, oracle, kind, odd):
     rng = np.random.default_rng(len(kind) + odd)
