@@ -1632,6 +1632,17 @@ uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *d
     return tuning_.windowMBps / 17 * 15;
 }
 
+// A wave has its descriptor after two loads from HBM (kTableHoldNanos), and then waits as one of a launch of pieces does.
+void XcopyEngine::TablePaceFor(uint32_t &holdNanos, uint32_t &holdMoreNanos, uint32_t &windowMBps) const
+{
+    const bool alone = g_leasesOut.load(std::memory_order_relaxed) <= 1;
+    const bool rule = tuning_.holdNanos < 0 && !tuning_.holdCalibratedOff;
+    const int32_t base = tuning_.holdNanos > 0 ? tuning_.holdNanos : kTableHoldNanos + tuning_.holdDeltaNanos;
+    holdNanos = alone && tuning_.deepHold && (rule || tuning_.holdNanos > 0) && base > 0 ? static_cast<uint32_t>(base) : 0;
+    holdMoreNanos = holdNanos != 0 && rule ? kTableHoldMoreNanos : 0;
+    windowMBps = WindowsApply(kDeepMaxBytes, MFRT_ROUTE_HBM, kDeepMaxBytes) ? tuning_.windowMBps / 17 * 15 : 0;
+}
+
 bool XcopyEngine::DeepHoldApplies(uint64_t bytes, uint32_t n, int route, bool unordered) const
 {
     return route == MFRT_ROUTE_HBM && !unordered && tuning_.holdNanos != 0 && tuning_.unitsOverride == 0 && tuning_.deepHold &&
@@ -2096,6 +2107,22 @@ int XcopyEngine::SubmitDeviceTable(const void *triples, uint32_t n, int route, v
         (void)BuildInlinePlan(none, kXcopyThreads, empty);
         int err = mfk_xcopy_inline(&empty, route, 1, mask, maskValue, stream, 0, 0);
         return err == 0 ? BM_OK : BM_ERROR;
+    }
+    // Up to kPlannedSegments segments one launch plans and copies.  Where it may not pace itself for the whole chip, because other
+    // threads submit too, only the shorter ones.
+    uint32_t hold = 0;
+    uint32_t holdMore = 0;
+    uint32_t windows = 0;
+    TablePaceFor(hold, holdMore, windows);
+    if (route == MFRT_ROUTE_HBM && tuning_.unitsOverride == 0 && tuning_.deviceTableWgPerCu == 0 &&
+        n <= (windows != 0 ? kPlannedSegments : 64 * kPlannedShortRun)) {
+        const int err = mfk_xcopy_planned(triples, n, hold, holdMore, windows, mask, maskValue, stream);
+        if (err != 0) {
+            MF_FAIL(BM_ERROR, "xcopy launch of a device table failed: " << mfrt_error_string(err));
+        }
+        g_launches.fetch_add(1, std::memory_order_relaxed);
+        NotePending(stream, ~0ull);   // sizes unknown here: the next wait sleeps on the stream
+        return BM_OK;
     }
     // The list of long segments belongs to a slot: the next call of another stream gets another one.  Calls that become
     // nodes of a graph have lists of their own, made by the thread's first call: a graph may be replayed beside plain calls.

@@ -133,9 +133,10 @@ __device__ __forceinline__ void LoadApart(u32x4 (&v)[kUnits], u32x4 &last, uint6
 }
 
 template <int kStore, uint32_t kUnits>
-__device__ __forceinline__ void StoreApart(const u32x4 (&v)[kUnits], u32x4 last, uint64_t dst, uint32_t u0, uint32_t end, uint32_t apart)
+__device__ __forceinline__ void StoreApart(const u32x4 (&v)[kUnits], u32x4 last, uint64_t dst, uint32_t u0, uint32_t end, uint32_t apart,
+                                           uint32_t lane = threadIdx.x & 63u)
 {
-    const uint32_t u = u0 + (threadIdx.x & 63u);
+    const uint32_t u = u0 + lane;
     auto store = [&](auto words) {
 #pragma unroll
         for (uint32_t j = 0; j < kUnits; ++j) {
@@ -175,7 +176,7 @@ __device__ __forceinline__ void HoldStores(uint64_t t0, uint32_t ticks)
 // for HoldStores(t0, ticks).
 template <bool kNtLoad, int kStore, bool kHold = false>
 __device__ __forceinline__ void CopyChunk(uint64_t src, uint64_t dst, uint64_t len, uint64_t k, uint32_t units, uint64_t t0 = 0,
-                                          uint32_t ticks = 0, uint32_t lanes = blockDim.x)
+                                          uint32_t ticks = 0, uint32_t lanes = blockDim.x, uint32_t tid = threadIdx.x)
 {
     const SegGeom g = SegmentGeometry(dst, len);
     const uint64_t u0 = k * units;
@@ -183,7 +184,6 @@ __device__ __forceinline__ void CopyChunk(uint64_t src, uint64_t dst, uint64_t l
     const uint32_t n = left < units ? static_cast<uint32_t>(left) : units;
     const uint64_t s = src + g.head + u0 * kUnitBytes;
     const uint64_t d = dst + g.head + u0 * kUnitBytes;
-    const uint32_t tid = threadIdx.x;
     const uint32_t kTile = kDepth * lanes;              // units one workgroup moves per step
 
     uint32_t i = 0;
@@ -876,6 +876,332 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_
     }
 }
 
+// How a launch of a device table paces itself; 0: not.
+struct TablePace {
+    uint32_t holdTicks;         // of the clock, what a wave waits before it stores, where all waves of the launch are resident together,
+    uint32_t holdMoreTicks;     // and what more per 64 MiB of the table
+    uint32_t windowTicks;       // period in which 64 MiB pass at the rate of random blocks
+    uint32_t seq;               // of AgreedStart
+};
+
+// The sum of the lanes up to and with this one.
+__device__ __forceinline__ uint32_t LanesUpTo(uint32_t v)
+{
+    v += __builtin_amdgcn_update_dpp(0u, v, 0x111, 0xf, 0xf, false);       // row_shr:1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0u, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0u, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0u, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0u, v, 0x142, 0xa, 0xf, false);       // row_bcast:15 into the rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0u, v, 0x143, 0xc, 0xf, false);       // row_bcast:31 into the rows 2 and 3
+    return v;
+}
+
+// The last of n ascending words that is not above c; the first is 0.
+__device__ __forceinline__ uint32_t LastUpTo(const uint32_t *first, uint32_t n, uint32_t c)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t lo = 0;
+    while (n > 1) {
+        const uint32_t step = (n + 63u) >> 6;
+        const uint32_t probe = lane * step;
+        const uint32_t at = (__popcll(__ballot(probe < n && first[lo + (probe < n ? probe : 0)] <= c)) - 1) * step;
+        lo += at;
+        n = n - at < step ? n - at : step;
+    }
+    return lo;
+}
+
+// Chunk k of kWindowUnits units of a segment, whatever its addresses, by one wave with sixteen loads per lane in flight: loads from
+// `loadAt` on the clock, stores from `storeAt` on, and `meanwhile` while the loads are on their way.  What a lane past the end of the
+// chunk loads is the last unit (XcopyPieceWindowKernel says why).
+template <class F>
+__device__ __forceinline__ void CopyDeepChunk(uint64_t src, uint64_t dst, uint64_t len, uint32_t k, uint64_t loadAt, uint64_t storeAt,
+                                              F meanwhile)
+{
+    uint32_t tid = threadIdx.x & 63u;
+    asm volatile("" : "+v"(tid));
+    const SegGeom g = SegmentGeometry(dst, len);
+    const uint64_t u0 = static_cast<uint64_t>(k) * kWindowUnits;
+    const uint64_t left = g.body > u0 ? g.body - u0 : 0;
+    const uint32_t n = left < kWindowUnits ? static_cast<uint32_t>(left) : kWindowUnits;
+    const uint64_t s = src + g.head + u0 * kUnitBytes;
+    const uint64_t d = dst + g.head + u0 * kUnitBytes;
+    const uint32_t apart = static_cast<uint32_t>(s) & (kUnitBytes - 1);
+    if (n != 0) {
+        const uint64_t from = s - apart;
+        const uint32_t most = apart != 0 ? n : n - 1;
+        u32x4 v[kWindowDepth];
+        WaitForClock(loadAt);
+#pragma unroll
+        for (uint32_t j = 0; j < kWindowDepth; ++j) {
+            const uint32_t u = j * 64 + tid < most ? j * 64 + tid : most;
+            v[j] = LoadAligned(from + u * kUnitBytes);
+        }
+        const u32x4 last = LoadAligned(from + most * kUnitBytes);
+        meanwhile();
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(tid) : : "memory");     // offsets are computed again, not held
+        WaitForClock(storeAt);
+        if (apart == 0) {
+#pragma unroll
+            for (uint32_t j = 0; j < kWindowDepth; ++j) {
+                if (j * 64 + tid < n) {
+                    StoreUnit<kStoreStream>(d + (j * 64 + tid) * kUnitBytes, v[j]);
+                }
+            }
+        } else {
+            StoreApart<kStoreStream>(v, last, d, 0, n, apart, tid);
+        }
+    } else {
+        meanwhile();
+    }
+    // (the last chunk of a segment may have been counted without its head, and hold nothing)
+    if (k == 0 && tid < g.head) {
+        CopyByte<kStoreStream>(src + tid, dst + tid);
+    }
+    if ((u0 < g.body || k == 0) && u0 + kWindowUnits >= g.body && tid < g.tail) {
+        const uint64_t off = g.head + g.body * kUnitBytes + tid;
+        CopyByte<kStoreStream>(src + off, dst + off);
+    }
+}
+
+// Four chunks of 4 KiB, of up to four segments, as one of 16 KiB; all begin on units and hold one at least.
+struct QuadChunk {
+    uint64_t src;
+    uint64_t dst;
+    uint32_t n;         // units
+};
+__device__ __forceinline__ void CopyQuad(const QuadChunk (&q)[4], uint64_t loadAt, uint64_t storeAt)
+{
+    uint32_t tid = threadIdx.x & 63u;
+    asm volatile("" : "+v"(tid));
+    u32x4 v[kWindowDepth];
+    WaitForClock(loadAt);
+#pragma unroll
+    for (uint32_t j = 0; j < kWindowDepth; ++j) {
+        const QuadChunk &c = q[j / kDepth];
+        const uint32_t u = j % kDepth * 64 + tid;
+        v[j] = LoadAligned(c.src + (u < c.n ? u : c.n - 1) * kUnitBytes);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(tid) : : "memory");
+    WaitForClock(storeAt);
+#pragma unroll
+    for (uint32_t j = 0; j < kWindowDepth; ++j) {
+        const QuadChunk &c = q[j / kDepth];
+        const uint32_t u = j % kDepth * 64 + tid;
+        if (u < c.n) {
+            StoreUnit<kStoreStream>(c.dst + u * kUnitBytes, v[j]);
+        }
+    }
+}
+
+// Chunk k of 4 KiB of a segment, by one wave of a workgroup.
+__device__ __forceinline__ void CopyCountedChunk(uint64_t src, uint64_t dst, uint64_t len, uint32_t k, uint32_t lane)
+{
+    if (k < SegmentChunks(dst, len, kXcopyThreads)) {      // it may have been counted without the segment's head, and hold nothing
+        CopyChunk<true, kStoreStream, false>(src, dst, len, k, kXcopyThreads, 0, 0, 64, lane);
+    }
+}
+
+// Chunk c of a table whose chunk prefix is `first`.
+__device__ __forceinline__ ChunkRef PlannedOwner(const uint64_t *__restrict__ triples, const uint32_t *first, uint32_t nseg, uint32_t c)
+{
+    const uint32_t seg = Uniform(LastUpTo(first, nseg, c));
+    const uint64_t *t = triples + 3ull * seg;
+    ChunkRef r;
+    r.src = Uniform(t[0]);
+    r.dst = Uniform(t[1]);
+    r.len = Uniform(t[2]);
+    r.k = c - Uniform(first[seg]);
+    return r;
+}
+
+// The chunks c to c + 3, of 4 KiB; false unless all four are there, begin on units and end with one.
+__device__ __forceinline__ bool PlannedQuad(const uint64_t *__restrict__ triples, const uint32_t *first, uint32_t nseg, uint32_t c,
+                                            uint32_t nchunk, QuadChunk (&q)[4])
+{
+    if (nchunk - c < 4) {
+        return false;
+    }
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t seg0 = Uniform(LastUpTo(first, nseg, c));
+    const uint32_t near = seg0 + lane < nseg ? first[seg0 + lane] : 0xFFFFFFFFu;      // of this segment and those behind it
+    bool whole = true;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+        const uint32_t row = __popcll(__ballot(near <= c + j)) - 1;
+        whole = whole && row < 63;          // more than 60 empty ones between two
+        const uint64_t *t = triples + 3ull * (seg0 + row);
+        const uint64_t src = Uniform(t[0]);
+        const uint64_t dst = Uniform(t[1]);
+        const uint64_t len = Uniform(t[2]);
+        const uint64_t at = static_cast<uint64_t>(c + j - __builtin_amdgcn_readlane(near, row)) * kXcopyThreads * kUnitBytes;
+        q[j].src = src + at;
+        q[j].dst = dst + at;
+        q[j].n = len - at < kXcopyThreads * kUnitBytes ? static_cast<uint32_t>(len - at) / kUnitBytes : kXcopyThreads;
+        whole = whole && ((src | dst | len) & (kUnitBytes - 1)) == 0;
+    }
+    return whole;
+}
+
+// A table that only the GPU can read, of up to kPlannedSegments segments between HBM addresses, in one launch of kWindowWaves waves:
+// every workgroup reads the lengths of all of it and has their chunk prefix in LDS after two sums over its lanes.  So it knows what a
+// host that could read the table would: the total, which chooses the form, and the owner of every chunk.  No list of long segments,
+// no second launch, no event.  Bound: the chain of launch, lengths, prefix, descriptor and first load (4 us) for short tables, HBM for
+// long ones.  With the two launches of XcopyDirectKernel / so, us: 64 pages of 8 KiB 9.2 / 4.6, 1000 9.7 / 6.1, 4096 17.2 / 15.2; 500 of
+// 32 KiB 11.6 / 8.0, 2000 29.8 / 24.9, 4096 scattered 55.7 / 50.6; 1952 K and V blocks 65.4 / 53.9; 1000 / 4000 ragged segments of up to
+// 70 000 bytes 24.0 / 16.6, 71.2 / 65.6; 300 of 2 MB 240 / 206.  Longer tables cost each workgroup more lanes' worth of lengths: with
+// kPlannedRun 16, 8000 pages of 8 KiB 28.3 / 30.9, 16 384 ragged of 14 000 bytes 60.3 / 68.9, and that much more code made all others
+// 1 to 3 us slower.  Looking four chunks ahead of a quad up while it loads: registers spill, 8000 pages of 8 KiB 33.3.
+template <uint32_t kWaves, uint32_t kRun>
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void XcopyPlannedKernel(const uint64_t *__restrict__ triples, uint32_t nseg, TablePace pace)
+{
+    extern __shared__ uint32_t words[];                     // PlannedLds()
+    if (nseg == 0) {
+        return;
+    }
+    const uint64_t t0 = wall_clock64();
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = threadIdx.x >> 6;
+    uint32_t *sums = words;                                 // [3][kWaves]
+    uint32_t *first = words + 3 * kWaves;                   // [nseg + 1]: chunks of 4 KiB of each segment, then the prefix of its chunks
+    const uint32_t run = (nseg + 64 * kWaves - 1) / (64 * kWaves);
+    const uint64_t *t = triples + 3ull * (lane < nseg ? lane : 0);
+    const uint32_t bits = static_cast<uint32_t>(t[0] | t[1]);      // of the first 64 segments, the same for every wave
+    uint64_t len[kRun];
+#pragma unroll
+    for (uint32_t r = 0; r < kRun; ++r) {
+        const uint32_t seg = r * 64 * kWaves + threadIdx.x;
+        len[r] = r < run ? triples[3ull * (seg < nseg ? seg : 0) + 2] : 0;
+    }
+    uint64_t size = 0;          // of 256 bytes
+#pragma unroll
+    for (uint32_t r = 0; r < kRun; ++r) {
+        const uint32_t seg = r * 64 * kWaves + threadIdx.x;
+        if (r < run && seg < nseg) {
+            first[seg] = static_cast<uint32_t>((len[r] + 4095) >> 12);
+            size += len[r] >> 8;
+        }
+    }
+    __syncthreads();
+    uint32_t count[kRun];
+    uint32_t shallow = 0;       // chunks of 4 KiB,
+    uint32_t deep = 0;          // of 16 KiB
+#pragma unroll
+    for (uint32_t r = 0; r < kRun; ++r) {
+        const uint32_t seg = threadIdx.x * run + r;
+        count[r] = r < run && seg < nseg ? first[seg] : 0;
+        shallow += count[r];
+        deep += (count[r] + 3) / 4;
+    }
+    const uint32_t shallowUpTo = LanesUpTo(shallow);
+    const uint32_t deepUpTo = LanesUpTo(deep);
+    // in 4 KiB, from lanes of up to 512 MiB
+    uint32_t total = __builtin_amdgcn_readlane(LanesUpTo(static_cast<uint32_t>(size < 1u << 21 ? size : 1u << 21)), 63) / 16;
+    uint32_t shallowAll = __builtin_amdgcn_readlane(shallowUpTo, 63);
+    uint32_t deepAll = __builtin_amdgcn_readlane(deepUpTo, 63);
+    uint32_t shallowBase = 0;
+    uint32_t deepBase = 0;
+    if (kWaves > 1) {
+        if (lane == 0) {
+            sums[wave] = shallowAll;
+            sums[kWaves + wave] = deepAll;
+            sums[2 * kWaves + wave] = total;
+        }
+        __syncthreads();
+        const uint32_t at = lane < kWaves ? lane : 0;
+        const uint32_t a = LanesUpTo(lane < kWaves ? sums[at] : 0);
+        const uint32_t b = LanesUpTo(lane < kWaves ? sums[kWaves + at] : 0);
+        total = __builtin_amdgcn_readlane(LanesUpTo(lane < kWaves ? sums[2 * kWaves + at] : 0), 63);
+        shallowBase = wave == 0 ? 0 : __builtin_amdgcn_readlane(a, wave == 0 ? 0 : wave - 1);
+        deepBase = wave == 0 ? 0 : __builtin_amdgcn_readlane(b, wave == 0 ? 0 : wave - 1);
+        shallowAll = __builtin_amdgcn_readlane(a, 63);
+        deepAll = __builtin_amdgcn_readlane(b, 63);
+    }
+    // The form: short tables a chunk of 4 KiB per wave; others 16 KiB, of one segment where those are nearly full or where a source and
+    // its destination may differ modulo 16, else of up to four.
+    const bool aligned = __ballot(bits % kUnitBytes != 0) == 0;
+    const bool full = static_cast<uint64_t>(total) * 100 >= static_cast<uint64_t>(deepAll) * (4 * kPlannedFullPercent);
+    const bool large = total > kPlannedShallowChunks;
+    const bool quads = large && aligned && !full;
+    const bool byDeep = large && !quads;
+    uint32_t before = byDeep ? deepBase + deepUpTo - deep : shallowBase + shallowUpTo - shallow;
+#pragma unroll
+    for (uint32_t r = 0; r < kRun; ++r) {
+        const uint32_t seg = threadIdx.x * run + r;
+        if (r < run && seg < nseg) {
+            first[seg] = before;
+            before += byDeep ? (count[r] + 3) / 4 : count[r];
+        }
+    }
+    const uint32_t nchunk = byDeep ? deepAll : shallowAll;
+    if (threadIdx.x == 0) {
+        first[nseg] = nchunk;
+    }
+    __syncthreads();
+
+    const uint32_t grid = gridDim.x * kWaves;
+    const uint32_t items = quads ? (nchunk + 3) / 4 : nchunk;
+    const bool held = large && items <= grid && total <= kPlannedHeldChunks;
+    const bool paced = large && total > kPlannedHeldChunks && aligned && pace.windowTicks != 0 &&
+                       static_cast<uint64_t>(total) * 100 >= static_cast<uint64_t>(items) * (4 * kPlannedFullPercent);
+    const uint32_t rounds = (items + grid - 1) / grid;
+    const uint32_t waves = paced ? (items + rounds - 1) / rounds : grid;
+    uint32_t item = wave * gridDim.x + blockIdx.x;          // neighbouring ones on neighbouring XCDs
+    if (item >= items || item >= waves) {
+        return;
+    }
+    constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kWindowUnits) * kUnitBytes;
+    const uint32_t period = static_cast<uint32_t>(pace.windowTicks * (waves * kDeepBytes) >> 26);
+    const uint32_t hold = pace.holdTicks + static_cast<uint32_t>(static_cast<uint64_t>(pace.holdMoreTicks) * total >> 14);
+    uint64_t loadAt = paced ? AgreedStart(pace.seq) + static_cast<uint64_t>(item) * (period / 2) / waves : 0;
+    uint64_t storeAt = paced ? loadAt + period / 2 : held && pace.holdTicks != 0 ? t0 + hold : 0;
+    const uint32_t step = paced ? period : 0;
+    if (byDeep) {
+        // the next chunk's owner is looked up while the loads of this one are on their way
+        ChunkRef r = PlannedOwner(triples, first, nseg, item);
+        for (;;) {
+            const bool more = items - item > waves;
+            ChunkRef next = r;
+            CopyDeepChunk(r.src, r.dst, r.len, r.k, loadAt, storeAt, [&] {
+                if (more) {
+                    next = PlannedOwner(triples, first, nseg, item + waves);
+                }
+            });
+            if (!more) {
+                return;
+            }
+            r = next;
+            item += waves;
+            loadAt += step;
+            storeAt += step;
+        }
+    }
+    if (quads) {
+        for (; item < items; item += waves) {
+            QuadChunk q[4];
+            if (PlannedQuad(triples, first, nseg, item * 4, nchunk, q)) {
+                CopyQuad(q, loadAt, storeAt);
+            } else {
+                WaitForClock(storeAt);
+                const uint32_t end = item * 4 + 4 < nchunk ? item * 4 + 4 : nchunk;
+#pragma unroll 1
+                for (uint32_t c = item * 4; c < end; ++c) {
+                    const ChunkRef r = PlannedOwner(triples, first, nseg, c);
+                    CopyCountedChunk(r.src, r.dst, r.len, r.k, lane);
+                }
+            }
+            loadAt += step;
+            storeAt += step;
+        }
+        return;
+    }
+    for (; item < items; item += waves) {
+        const ChunkRef r = PlannedOwner(triples, first, nseg, item);
+        CopyCountedChunk(r.src, r.dst, r.len, r.k, lane);
+    }
+}
+
 // The segments of a list that a wave is at, one per lane, so that the owner of a piece is found without a load.
 struct RestRows {
     uint64_t first = ~0ull;     // of the lane's segment
@@ -1350,6 +1676,26 @@ extern "C" int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t uni
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
+extern "C" int mfk_xcopy_planned(const void *triples, uint32_t nseg, uint32_t holdNanos, uint32_t holdMoreNanos, uint32_t windowMBps, void *mask,
+                                 uint32_t maskValue, void *stream)
+{
+    using namespace mf;
+    if (triples == nullptr || nseg == 0 || nseg > kPlannedSegments) {
+        return -1;
+    }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const uint64_t *t = static_cast<const uint64_t *>(triples);
+    const TablePace pace{HoldTicks(holdNanos), HoldTicks(holdMoreNanos), WindowPeriodTicks(2ull << 26, windowMBps), NextWindowSeq()};
+    if (nseg <= 64 * kPlannedShortRun) {
+        hipLaunchKernelGGL((XcopyPlannedKernel<1, kPlannedShortRun>), dim3(kWindowWaves), dim3(64), PlannedLds(1, nseg), s, t, nseg, pace);
+    } else {
+        hipLaunchKernelGGL((XcopyPlannedKernel<kPlannedWaves, kPlannedRun>), dim3(kWindowWaves / kPlannedWaves), dim3(64 * kPlannedWaves),
+                           PlannedLds(kPlannedWaves, nseg), s, t, nseg, pace);
+    }
+    const int err = static_cast<int>(hipGetLastError());
+    return err != 0 ? err : Signal(mask, maskValue, s);
+}
+
 // Makes `count` lists `stride` bytes apart empty.
 extern "C" int mfk_xcopy_clear_lists(void *lists, uint32_t count, uint64_t stride, void *stream)
 {
@@ -1393,6 +1739,8 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
                 hipLaunchKernelGGL((XcopyPieceKernel<128, 4, true>), dim3(1), dim3(128), 0, s, nullptr, 0u, 0u);
                 hipLaunchKernelGGL((XcopyPieceKernel<256, 4, false>), dim3(1), dim3(256), 0, s, nullptr, 0u, 0u);
                 hipLaunchKernelGGL(XcopyPieceWindowKernel, dim3(1), dim3(64), 0, s, nullptr, 0u, 64u, NextWindowSeq());
+                hipLaunchKernelGGL((XcopyPlannedKernel<1, kPlannedShortRun>), dim3(1), dim3(64), 64, s, nullptr, 0u, TablePace{});
+                hipLaunchKernelGGL((XcopyPlannedKernel<kPlannedWaves, kPlannedRun>), dim3(1), dim3(64 * kPlannedWaves), 64, s, nullptr, 0u, TablePace{});
                 hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
             }
             return 0;

@@ -302,6 +302,23 @@ constexpr uint64_t kRestPieceBytes = 64ull << 10;
 constexpr uint32_t kRestShare = 16;                   // pieces side by side whose workgroups take their chunks in turn
 constexpr uint32_t kRestLanes = 512;                  // of a workgroup of the second launch between HBM addresses
 
+// A table of up to kPlannedSegments segments between HBM addresses is planned by every workgroup of its one launch for itself: one
+// wave, or sixteen for more than 512 segments, whose lanes take a run of them each.  Up to kPlannedShallowChunks chunks of 4 KiB it is
+// cut into those, else into 16 KiB, whose stores are held up to kPlannedHeldChunks of 4 KiB.
+constexpr uint32_t kPlannedShortRun = 8;
+constexpr uint32_t kPlannedWaves = 16;
+constexpr uint32_t kPlannedRun = 4;
+constexpr uint32_t kPlannedSegments = 64 * kPlannedWaves * kPlannedRun;
+constexpr uint32_t kPlannedFullPercent = 85;          // pieces of 16 KiB that are less full gain nothing from windows
+constexpr uint32_t kPlannedShallowChunks = 1024;
+constexpr uint32_t kPlannedHeldChunks = 16384;
+constexpr uint32_t PlannedLds(uint32_t waves, uint32_t nseg)          // bytes: the prefix, and three sums of each wave
+{
+    return (nseg + 1 + 3 * waves) * 4;
+}
+constexpr int32_t kTableHoldNanos = 2000;             // held stores of device tables: the wait,
+constexpr uint32_t kTableHoldMoreNanos = 8800;        // and what more for 64 MiB
+
 struct RestSegment {                                  // what is left of a long segment
     uint64_t first;                                   // pieces of those listed before
     uint64_t src;

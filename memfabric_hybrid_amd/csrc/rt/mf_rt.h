@@ -119,6 +119,11 @@ int mfk_xcopy_signal(void *word, uint32_t value, void *stream);
  * event: as for mfk_xcopy_pieces; NULL on a stream that records a graph. */
 int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *rest,
                      uint32_t capacity, void *mask, uint32_t maskValue, void *stream, void *event);
+/* A triple table in device memory of up to kPlannedSegments (kernels/xcopy_plan.h) segments between HBM addresses, in one launch that
+ * reads and plans it.  Waves that are resident together hold their stores for holdNanos and holdMoreNanos per 64 MiB; what is more goes
+ * in read and write windows cut for `windowMBps`.  0: not held, no windows. */
+int mfk_xcopy_planned(const void *triples, uint32_t nseg, uint32_t holdNanos, uint32_t holdMoreNanos, uint32_t windowMBps, void *mask,
+                      uint32_t maskValue, void *stream);
 /* Makes `count` mf::RestList in device memory, `stride` bytes apart, empty. */
 int mfk_xcopy_clear_lists(void *lists, uint32_t count, uint64_t stride, void *stream);
 /* The same with the list in a statically allocated device array instead of memory the engine allocates: no allocation

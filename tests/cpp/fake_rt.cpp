@@ -510,6 +510,28 @@ int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int, ui
     return 0;
 }
 
+// One launch without a list: as far as the users of lists go, one that no other call has.
+int mfk_xcopy_planned(const void *triples, uint32_t nseg, uint32_t, uint32_t, uint32_t, void *mask, uint32_t maskValue, void *)
+{
+    static uint8_t none[4096];
+    static uint32_t turn = 0;
+    g_lastRestList = &none[++turn % 4096];
+    if (triples == nullptr || nseg == 0 || nseg > mf::kPlannedSegments) {
+        return -1;
+    }
+    ++g_launches;
+    const uint64_t *t = static_cast<const uint64_t *>(triples);
+    for (uint32_t i = 0; i < nseg; ++i) {
+        for (uint64_t c = 0; c < mf::SegmentChunks(t[3 * i + 1], t[3 * i + 2], 1024); ++c) {
+            RunChunk(t[3 * i], t[3 * i + 1], t[3 * i + 2], c, 1024);
+        }
+    }
+    if (mask != nullptr) {
+        *static_cast<uint64_t *>(mask) = maskValue;
+    }
+    return 0;
+}
+
 static uint64_t g_signals = 0;
 static uint64_t g_streamSyncs = 0;
 extern "C" uint64_t fake_rt_signals() { return g_signals; }

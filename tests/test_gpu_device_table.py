@@ -105,3 +105,54 @@ def test_table_of_a_few_very_long_segments(gpu, count, size, static):
         got = target.view(count, step).flip(0)
         assert torch.equal(got[:, :size], source.view(count, step)[:, :size])
         assert not got[:, size:].any()
+
+
+# Tables of up to 4096 segments, which their launch plans itself: one wave or sixteen per plan on either side of 512 segments, and the
+# forms: chunks of 4 KiB, of 16 KiB held and beyond 64 MiB in windows or not, and four chunks of 4 KiB of up to four segments.
+PLANNED = {
+    "one wave, short": (512, lambda rng, n: rng.integers(0, 7000, n), 16),
+    "one wave, held": (511, lambda rng, n: rng.integers(1, 60000, n), 16),
+    "one wave, held, on lines": (300, lambda rng, n: np.full(n, 65536), 0),
+    "one wave, windows": (512, lambda rng, n: np.full(n, 163840), 0),
+    "one wave, one long": (64, lambda rng, n: np.where(np.arange(n) == 40, 80 << 20, 100), 16),
+    "sixteen, short": (4096, lambda rng, n: rng.integers(0, 1500, n), 16),
+    "sixteen, held": (513, lambda rng, n: rng.integers(1, 90000, n), 16),
+    "sixteen, held, head": (1025, lambda rng, n: np.full(n, 16384), 16),
+    "sixteen, quads": (2048, lambda rng, n: rng.integers(0, 1200, n) * 16, 0),
+    "sixteen, quads, odd lengths": (4095, lambda rng, n: np.where(np.arange(n) % 50 == 7, rng.integers(1, 9000, n), 8192), 0),
+    "sixteen, quads after many empty": (3000, lambda rng, n: np.where(np.arange(n) % 200 < 70, 0, 5008), 0),
+    "sixteen, windows": (4096, lambda rng, n: np.full(n, 32768), 0),
+    "sixteen, more than held, between units": (3001, lambda rng, n: rng.integers(1, 70000, n), 16),
+    "sixteen, more than held, not full": (2500, lambda rng, n: rng.integers(1, 4000, n) * 16, 0),
+    "beyond": (4097, lambda rng, n: rng.integers(1, 9000, n), 16),
+}
+
+
+@pytest.mark.parametrize("kind", PLANNED)
+def test_tables_that_their_launch_plans(gpu, kind):
+    torch = pytest.importorskip("torch")
+    count, lengths, odd = PLANNED[kind]
+    rng = np.random.default_rng(len(kind))
+    lens = lengths(rng, count).astype(np.int64)
+    steps = (lens + 191) // 128 * 128
+    order = rng.permutation(count)
+    at = np.cumsum(steps) - steps
+    place = np.empty(count, dtype=np.int64)
+    place[order] = np.cumsum(steps[order]) - steps[order]
+    if odd:
+        at, place = at + rng.integers(0, odd, count), place + rng.integers(0, odd, count)
+    size = int(steps.sum()) + 4096
+    source = torch.randint(0, 256, (size,), dtype=torch.uint8, device="cuda")
+    before = torch.randint(0, 256, (size,), dtype=torch.uint8, device="cuda")
+    target = before.clone()
+    rows = np.stack([source.data_ptr() + at, target.data_ptr() + place, lens], axis=1)
+    table = torch.from_numpy(rows).cuda()
+    torch.cuda.synchronize()
+    launches = gpu.mf_xcopy_launch_count()
+    assert gpu.mf_xcopy_device_table(table.data_ptr(), count, native.ROUTE_HBM, None) == 0, native.last_error()
+    assert gpu.mfrt_device_sync() == 0
+    assert gpu.mf_xcopy_launch_count() - launches == (1 if count <= 4096 else 2)
+    expect, data = before.cpu().numpy(), source.cpu().numpy()
+    for s, d, l in zip(at, place, lens):
+        expect[d:d + l] = data[s:s + l]
+    assert np.array_equal(target.cpu().numpy(), expect)
