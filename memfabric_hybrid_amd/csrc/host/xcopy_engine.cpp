@@ -1049,6 +1049,8 @@ uint32_t BuildPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *l
     const uint64_t most = static_cast<uint64_t>(units) * kUnitBytes;
     const uint32_t shift = static_cast<uint32_t>(__builtin_ctzll(most));
     Piece *p = out;
+    uint64_t lastSpan = 0;
+    uint64_t each = 0;
     for (uint32_t i = 0; i < n;) {
         const uint64_t s = src[i];
         const uint64_t d = dst[i];
@@ -1067,14 +1069,24 @@ uint32_t BuildPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *l
             *p++ = MakePiece(s, d, static_cast<uint32_t>(l));
             continue;
         }
-        const uint64_t parts = (span + most - 1) >> shift;
-        const uint64_t each = ((span + parts - 1) / parts + kPieceAlign - 1) & ~static_cast<uint64_t>(kPieceAlign - 1);
-        uint64_t from = 0;
-        for (uint64_t to = each - skip; from < l; to += each) {
-            const uint64_t end = to < l ? to : l;
-            *p++ = MakePiece(s + from, d + from, static_cast<uint32_t>(end - from));
-            from = end;
+        if (span != lastSpan) {     // a division a segment of another size
+            lastSpan = span;
+            const uint64_t parts = (span + most - 1) >> shift;
+            const uint64_t lines = (span + kPieceAlign - 1) / kPieceAlign;
+            each = kPieceAlign * (lines >> 31 == 0 ? (static_cast<uint32_t>(lines) + static_cast<uint32_t>(parts) - 1) / static_cast<uint32_t>(parts)
+                                                   : (lines + parts - 1) / parts);
         }
+        *p++ = MakePiece(s, d, static_cast<uint32_t>(each - skip));
+        const Piece length = MakePiece(0, 0, static_cast<uint32_t>(each));
+        uint64_t left = l - (each - skip);
+        uint64_t from = (s + (each - skip)) & kPieceAddress;
+        uint64_t to = (d + (each - skip)) & kPieceAddress;
+        for (; left > each; left -= each) {
+            *p++ = Piece{from | length.src, to | length.dst};
+            from += each;
+            to += each;
+        }
+        *p++ = MakePiece(from, to, static_cast<uint32_t>(left));
     }
     return static_cast<uint32_t>(p - out);
 }
@@ -1419,15 +1431,13 @@ int XcopyEngine::WaitTicket(uint32_t ticket, void *stream)
 int XcopyEngine::SubmitAndWait(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, int route, void *stream)
 {
     uint64_t bytes = 0;
-    if (n <= 4096) {   // a longer table is not worth adding up: such a batch waits on the stream
-        for (uint32_t i = 0; i < n; ++i) {
-            bytes += len[i];
-        }
+    for (uint32_t i = 0; i < n; ++i) {
+        bytes += len[i];
     }
     uint32_t ticket = 0;
     int ret = LaunchDone(src, dst, len, n, bytes, route, stream, ticket);
     if (ret == kNotLaunched) {
-        ret = Submit(src, dst, len, n, route, stream, nullptr, 0, false);
+        ret = SubmitInSlices(src, dst, len, n, bytes, route, stream);
         return ret != BM_OK ? ret : WaitStream(stream, bytes, route);
     }
     if (ret != BM_OK) {
@@ -1440,6 +1450,35 @@ int XcopyEngine::SubmitAndWait(const uint64_t *src, const uint64_t *dst, const u
     const int err = PollDone(lease, ticket, LeastMicros(bytes, route)) ? 0 : mfrt_stream_sync(stream);
     if (err != 0) {
         MF_FAIL(BM_ERROR, "copy failed on the GPU: " << mfrt_error_string(err));
+    }
+    return BM_OK;
+}
+
+// The GPU of a caller that waits has nothing to do while the host plans, so a long batch whose planning takes a while goes in two or
+// three launches, the first of them a quarter or an eighth of it: the GPU then needs longer for each than the host for the next.
+// Not below kDeepMaxBytes: a launch more costs the host 3 us, and short launches leave the GPU idle at their ends (2000 ragged segments
+// of up to 40 000 bytes, 40 MB, 48 us in one launch and 59 in four).
+int XcopyEngine::SubmitInSlices(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t bytes, int route,
+                                void *stream)
+{
+    const uint64_t planNanos = 3ull * n + bytes / 16384;        // segments, and pieces of 16 KiB
+    const bool sliced = route == MFRT_ROUTE_HBM && n > 4 * kInlineSegs && planNanos >= kSliceMinNanos && bytes >= kDeepMaxBytes &&
+                        tuning_.unitsOverride == 0 && bytes / n < kWindowSliceMinAlignedSegmentBytes;
+    const bool three = bytes >= 3 * kDeepMaxBytes;
+    const uint32_t ends[3] = {sliced ? (three ? n / 8 : n / 4) : 0, sliced && three ? n / 8 * 3 : 0, n};
+    uint32_t at = 0;
+    for (uint32_t end : ends) {
+        if (end <= at && end != n) {
+            continue;
+        }
+        const int ret = Submit(src + at, dst + at, len + at, end - at, route, stream, nullptr, 0, false);
+        if (ret != BM_OK) {
+            if (at != 0) {
+                (void)mfrt_stream_sync(stream);     // what has gone out is not left running behind a call that failed
+            }
+            return ret;
+        }
+        at = end;
     }
     return BM_OK;
 }

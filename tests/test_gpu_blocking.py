@@ -120,3 +120,34 @@ LEAST_ROUND = 576 << 10
 ], ids=lambda s: f"{len(s)}x{s[0]}")
 def test_staged_copies_at_the_edges_of_rounds(lib, pool, way, sizes):
     test_staged_copies_of_pageable_memory(lib, pool, way, sizes)
+
+
+@pytest.mark.parametrize("count, most, launches", [(513, 131072, 1), (1400, 65536, 2), (1601, 131072, 3)])
+def test_long_batch_in_launches_that_planning_overlaps(lib, pool, count, most, launches):
+    """Every byte is there when the call returns, whichever of its launches moved it."""
+    rng = np.random.default_rng(count)
+    lens = rng.integers(most * 15 // 16, most, count) // 16 * 16 - rng.integers(0, 2, count)
+    steps = (lens + 127) // 128 * 128
+    order = rng.permutation(count)
+    at = np.cumsum(steps) - steps
+    place = np.empty(count, dtype=np.int64)
+    place[order] = np.cumsum(steps[order]) - steps[order]
+    size = int(steps.sum())
+    room = (size + (2 << 20) - 1) // (2 << 20) * (2 << 20)
+    other = bm.create(2, 0, 2 * room)
+    try:
+        source = other.peer_rank_ptr(0, bm.BmMemType.DEVICE)
+        data = rng.integers(0, 256, size, dtype=np.uint8)
+        assert lib.mfrt_memcpy(source, data.ctypes.data, size) == 0
+        assert lib.mfrt_memset(source + room, 0, room) == 0
+        before = lib.mf_xcopy_launch_count()
+        assert other.copy_data_batch((source + at).tolist(), (source + room + place).tolist(), lens.tolist(), count,
+                                     bm.BmCopyType.G2G) == 0, native.last_error()
+        assert lib.mf_xcopy_launch_count() - before == launches
+        got = _read(lib, source + room, size)
+    finally:
+        other.destroy()
+    expect = np.zeros(size, dtype=np.uint8)
+    for s, d, n in zip(at, place, lens):
+        expect[d:d + n] = data[s:s + n]
+    assert np.array_equal(got, expect)
