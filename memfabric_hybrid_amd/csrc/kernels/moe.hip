@@ -7,7 +7,8 @@
 //             (a stable counting sort of the flat (t,k) order by expert id)
 //   combine   y[t][h] = bf16_rne(fma(w[t][K-1], v[K-1], ... fma(w[t][0], v[0], 0)))
 //
-// One launch for a dispatch of up to 4096 entries (MoeDispatchSmallKernel: every token ranks its own entries).
+// One launch for a small dispatch (MoeDispatchSmallKernel, up to 4096 entries: every token ranks its own entries) and for one whose
+// rows fit the last-level cache (MoeDispatchCountKernel, up to 49152 entries: every workgroup counts all entries).
 // Three launches for a larger one (two when the entries fill few rank blocks), one for combine:
 //   MoeHistKernel    per-block expert histograms (wave ballots + LDS); not launched for a few blocks,
 //                    which count one another's entries inside the rank kernel
@@ -612,11 +613,14 @@ __global__ __launch_bounds__(64) void MoePermuteTileKernel(const u32x4 *__restri
 // stores), not bytes, as long as the comparisons stay few: with all parts they grow with tokens * entries.  Dispatch
 // alone, with the rank launch and the permute launch / in one: 16 tokens of 7168 elements at top-8 over 256 experts 12.0 / 4.3 us,
 // 64: 12.3 / 4.9, 128: 13.6 / 6.1, 256: 15.3 / 9.3, 512 (4096 entries): 19.6 / 16.0, 1024: 31.8 / 35.0; 2000 tokens of 1024
-// elements at top-2 12.1 / 7.1, 4096 at top-2 14.8 / 18.6.  So it ends at 4096 entries.  Plain stores leave the rows in
+// elements at top-2 12.1 / 7.1, 4096 at top-2 14.8 / 18.6.  It ends where counting is the quicker (MoeDispatchCountKernel): at 4096 entries, and
+// at 16384 comparisons per part (2048 elements, dispatch and combine: 256 tokens at top-8 11.6 here and 12.0 there, 300 12.6 and 11.1;
+// 1000 at top-4 12.5 and 12.3).  Plain stores leave the rows in
 // the caches, where the experts' kernel finds them (dispatch and combine in turn, 512 tokens: 27.9 us, 29.5 with nontemporal stores).
 constexpr uint32_t kSmallThreads = 256;
 constexpr uint32_t kSmallHold = 2;                      // 128-bit pieces of the row per lane: a part is 512 units at most
 constexpr uint32_t kSmallEntries = 4096;                // the largest such call
+constexpr uint32_t kSmallCompares = 16384;              // entries times slots: what a part of a token compares
 constexpr uint32_t kSmallGroups = 256;                  // rows are cut until there are so many workgroups, one per CU
 constexpr uint32_t kSmallBatch = 4;                     // ids per lane requested together by the counting workgroup
 static_assert(kSmallEntries <= 1u << 16 && kMaxExperts <= 1u << 16, "an entry's expert and index share a word");
@@ -786,6 +790,240 @@ __global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(const u3
     }
 }
 
+// A dispatch in one launch whose entries are too many to compare with one another: a workgroup per CU takes neighbouring tokens,
+// counts all ids for itself, in LDS, an id before its own entries in the upper half of the word too, and so knows where its
+// own entries of every expert begin without a word from the others.  Their ranks inside the workgroup come from ballots, slice by slice.
+// The rows wait in registers meanwhile, and every wave stores its pieces of 64 units K-fold.
+// What bounds it: up to about 8000 entries of 2048 elements the chain of a launch (ids, counts, scan, rows, stores), beyond
+// its stores.  Two launches and what lies between them went, as did the second read of the index tables.  Dispatch / dispatch and
+// combine in turn, with the rank launch and the permute in front of this / with it, us: 700 tokens of 2048 elements at top-8 over 256 experts
+// 13.1, 19.6 / 8.6, 13.9; 1500 17.3, 28.4 / 12.7, 21.8; 3000 26.4, 46.3 / 23.1, 38.5; 1500 of 5120 at top-6 over 128 28.3, 47.5 /
+// 21.1, 35.5; 4000 of 2048 at top-2 over 8 16.3, 26.3 / 10.9, 18.4; and with every token against every entry in front of it:
+// 400 of 2048 at top-8 8.6, 13.4 / 6.6, 10.7; 512 of 7168 15.4, 25.9 / 13.0, 23.4.
+// A thread per id and 1024 of them: two workgroups of 512 threads took 0.1 to 1 us more, one 1 us more.
+// Counts that fall on the same word wait for each other, so an expert has several words, side by side, the fewer experts the more,
+// and a lane adds to its own: 16 us with four of them over 8 experts, where 64 take 7.
+constexpr uint32_t kCountThreads = 1024;
+constexpr uint32_t kCountWaves = kCountThreads / 64;
+constexpr uint32_t kCountBatch = 4;                     // 128-bit loads of ids per lane in flight
+constexpr uint32_t kCountEntries = 48u << 10;           // the largest such call: every workgroup counts all of them
+constexpr uint32_t kCountLeastGroups = 128;             // so that a workgroup's own entries are fewer than its threads
+static_assert(kCountEntries < 1u << 16, "counts of half a word");
+static_assert(kCountEntries / kCountLeastGroups + kMaxTopK <= kCountThreads && kMaxExperts <= kCountThreads, "one per thread");
+
+__host__ __device__ constexpr uint32_t CountCopiesLog(uint32_t experts)
+{
+    return experts <= 16 ? 6 : experts <= 64 ? 4 : 2;
+}
+
+// [experts][copies] counts, [experts] first rows, a sum per wave, the rows of the own entries, [slices][experts] of those
+constexpr uint32_t CountLdsWords(uint32_t experts, uint32_t ownMost)
+{
+    return (experts << CountCopiesLog(experts)) + experts + kCountWaves + ownMost + (ownMost + 63) / 64 * experts;
+}
+
+// The lines lie where the token rows and the stored rows together, in bytes, change what a store should do.
+// Up to kCountQuickBytes nontemporal stores: they are on their way at once, where plain ones wait in an XCD's L2 for the end of
+// the launch (dispatch and combine in turn, 400 tokens of 2048 elements at top-8: 10.7 us, 11.4 with plain ones).  Beyond, plain
+// stores leave the rows in the last-level cache, where the next kernel finds them (1000 of 5120 at top-8: 31.2, 35.5 with
+// nontemporal ones; 1500 of 2048 21.8, 23.6).  From kCountNearBytes on nontemporal loads and twice as many of them ahead keep the token rows
+// from taking turns with them (2400 of 7168 at top-2: dispatch 19.4, 25.9 without; before kCountNearBytes the longer code
+// costs 0.5).  Calls of few slots read most: from kCountDeepBytes on plain stores cost them more than the next kernel
+// gains (4096 of 7168 at top-2, dispatch / both: nontemporal 28.6 / 57.4, plain 36.5 / 56.0).
+// What does not fit the last-level cache (256 MiB) goes to the tiles: 8192 of 2048 at top-8 57 us, 61 to 63 with this.  Below that
+// the tiles may be the quicker dispatch, but not the quicker pair: 2000 of 7168 at top-8 47.0 / 91.1, with this 51.1 / 80.0; 1500 37.5 / 70.6
+// and 39.1 / 61.3.  Rows that are not whole cache lines are always stored plainly: two waves share a line.
+constexpr uint64_t kCountQuickBytes = 24ull << 20;
+constexpr uint64_t kCountNearBytes = 96ull << 20;
+constexpr uint64_t kCountDeepBytes = 150ull << 20;
+constexpr uint64_t kCountBytes = 256ull << 20;
+
+template <bool kNt>
+__device__ __forceinline__ u32x4 RowLoad(const MF_GLOBAL u32x4 *p)
+{
+    return kNt ? __builtin_nontemporal_load(p) : *p;
+}
+
+template <uint32_t kAhead, int kMode, bool kNtLoad>
+__global__ __launch_bounds__(kCountThreads) void MoeDispatchCountKernel(const u32x4 *__restrict__ x, const int32_t *__restrict__ topk,
+                                                                        uint32_t total, uint32_t topK, uint32_t experts,
+                                                                        uint32_t unitsPerRow, uint32_t perGroup, u32x4 *__restrict__ out,
+                                                                        int32_t *__restrict__ counts, int32_t *__restrict__ offsets,
+                                                                        int32_t *__restrict__ rowOf, int32_t *__restrict__ srcOf,
+                                                                        uint32_t *__restrict__ status)
+{
+    extern __shared__ uint32_t lds[];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t copiesLog = CountCopiesLog(experts);
+    const uint32_t ownMost = perGroup * topK;
+    const uint32_t slices = (ownMost + 63) / 64;
+    uint32_t *count = lds;
+    uint32_t *base = count + (experts << copiesLog);
+    uint32_t *scan = base + experts;
+    uint32_t *rows = scan + kCountWaves;
+    uint32_t *hist = rows + ownMost;
+    const uint32_t begin = blockIdx.x * ownMost;
+    const uint32_t end = begin + ownMost < total ? begin + ownMost : total;
+    // the ids before the rows: everything waits for them.  The last vector ends with the last id.
+    i32x4a id[kCountBatch];
+#pragma unroll
+    for (uint32_t q = 0; q < kCountBatch; ++q) {
+        const uint32_t at = (q * kCountThreads + threadIdx.x) * 4;
+        id[q] = *reinterpret_cast<const i32x4a *>(topk + (at + 3 < total ? at : total - 4));
+    }
+    const uint32_t own = begin + threadIdx.x;
+    const int32_t ownId = own < end ? topk[own] : -1;
+    const uint32_t tokens = (end - begin) / topK;
+    const uint32_t parts = (unitsPerRow + 63) / 64;     // pieces of 64 units
+    const uint32_t items = x != nullptr ? tokens * parts : 0;
+    const MF_GLOBAL u32x4 *src = reinterpret_cast<const MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(x)) +
+                                 static_cast<uint64_t>(blockIdx.x) * perGroup * unitsPerRow;
+    MF_GLOBAL u32x4 *dst = reinterpret_cast<MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(out));
+    u32x4 v[kAhead];
+#pragma unroll
+    for (uint32_t j = 0; j < kAhead; ++j) {
+        const uint32_t item = wave + j * kCountWaves;
+        if (item < items) {
+            const uint32_t token = item / parts;
+            const uint32_t u = (item - token * parts) * 64 + lane;
+            if (u < unitsPerRow) {
+                v[j] = RowLoad<kNtLoad>(src + static_cast<uint64_t>(token) * unitsPerRow + u);
+            }
+        }
+    }
+    for (uint32_t i = threadIdx.x; i < experts << copiesLog; i += kCountThreads) {
+        count[i] = 0;
+    }
+    for (uint32_t i = threadIdx.x; i < slices * experts; i += kCountThreads) {
+        hist[i] = 0;
+    }
+    __syncthreads();
+    uint32_t bad = 0;
+    uint32_t *counting = count + (lane & ((1u << copiesLog) - 1u));
+    for (uint32_t from = 0; from < total; from += kCountBatch * kCountThreads * 4) {
+#pragma unroll
+        for (uint32_t q = 0; q < kCountBatch; ++q) {
+            if (from + q * kCountThreads * 4 >= total) {
+                break;
+            }
+            const uint32_t at = from + (q * kCountThreads + threadIdx.x) * 4;
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                const uint32_t index = at + 3 < total ? at + i : total - 4 + i;
+                if (index >= at) {
+                    const uint32_t e = static_cast<uint32_t>(id[q][i]);
+                    if (e < experts) {
+                        atomicAdd(&counting[e << copiesLog], index < begin ? 0x10001u : 1u);   // plain counts: the same whatever the order
+                    } else {
+                        bad = 1;
+                    }
+                }
+            }
+        }
+        if (from + kCountBatch * kCountThreads * 4 < total) {
+#pragma unroll
+            for (uint32_t q = 0; q < kCountBatch; ++q) {
+                const uint32_t at = from + ((kCountBatch + q) * kCountThreads + threadIdx.x) * 4;
+                id[q] = *reinterpret_cast<const i32x4a *>(topk + (at + 3 < total ? at : total - 4));
+            }
+        }
+    }
+    uint32_t rank = 0;
+    const bool valid = static_cast<uint32_t>(ownId) < experts;
+    if (wave < slices) {
+        const uint64_t peers = PeersOf(static_cast<uint32_t>(ownId), valid, BitsFor(experts));
+        const uint64_t below = peers & ((1ull << lane) - 1ull);
+        rank = __popcll(below);
+        if (valid && below == 0) {
+            hist[wave * experts + static_cast<uint32_t>(ownId)] = __popcll(peers);
+        }
+    }
+    bad = __syncthreads_or(static_cast<int>(bad)) != 0 ? 1u : 0u;
+    uint32_t all = 0;
+    uint32_t before = 0;
+    if (threadIdx.x < experts) {
+        for (uint32_t c = 0; c < 1u << copiesLog; c += 4) {
+            const u32x4 w = *reinterpret_cast<const u32x4 *>(&count[(threadIdx.x << copiesLog) + c]);
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                all += w[i] & 0xFFFFu;
+                before += w[i] >> 16;
+            }
+        }
+    }
+    uint32_t incl = all;
+#pragma unroll
+    for (uint32_t step = 1; step < 64; step <<= 1) {
+        const uint32_t up = __shfl_up(incl, step, 64);
+        incl += lane >= step ? up : 0u;
+    }
+    if (lane == 63) {
+        scan[wave] = incl;                              // experts of a wave: the sums in front of theirs are added by who asks
+    }
+    if (threadIdx.x < experts) {
+        base[threadIdx.x] = incl - all + before;
+    }
+    __syncthreads();
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < experts) {
+            uint32_t run = incl - all;
+            for (uint32_t w = 0; w < wave; ++w) {
+                run += scan[w];
+            }
+            counts[threadIdx.x] = static_cast<int32_t>(all);
+            offsets[threadIdx.x] = static_cast<int32_t>(run);
+        }
+        if (threadIdx.x == 0) {
+            status[0] = bad;
+        }
+    }
+    if (own < end) {
+        uint32_t row = 0xFFFFFFFFu;
+        if (valid) {
+            const uint32_t e = static_cast<uint32_t>(ownId);
+            row = base[e] + rank;
+            for (uint32_t w = 0; w < e >> 6; ++w) {
+                row += scan[w];
+            }
+            for (uint32_t s = 0; s < wave; ++s) {
+                row += hist[s * experts + e];
+            }
+            if (srcOf != nullptr) {
+                srcOf[row] = static_cast<int32_t>(own);
+            }
+        }
+        rows[threadIdx.x] = row;
+        rowOf[own] = static_cast<int32_t>(row);
+    }
+    __syncthreads();
+    // the next piece is requested into the registers of the one that was stored
+    for (uint32_t first = wave; first < items; first += kAhead * kCountWaves) {
+#pragma unroll
+        for (uint32_t j = 0; j < kAhead; ++j) {
+            const uint32_t item = first + j * kCountWaves;
+            if (item < items) {
+                const uint32_t token = item / parts;
+                const uint32_t u = (item - token * parts) * 64 + lane;
+                for (uint32_t k = 0; k < topK; ++k) {
+                    const uint32_t row = __builtin_amdgcn_readfirstlane(rows[token * topK + k]);
+                    if (row != 0xFFFFFFFFu && u < unitsPerRow) {
+                        RowStore<kMode>(dst + static_cast<uint64_t>(row) * unitsPerRow + u, v[j]);
+                    }
+                }
+                const uint32_t next = item + kAhead * kCountWaves;
+                if (next < items) {
+                    const uint32_t nextToken = next / parts;
+                    const uint32_t nextU = (next - nextToken * parts) * 64 + lane;
+                    if (nextU < unitsPerRow) {
+                        v[j] = RowLoad<kNtLoad>(src + static_cast<uint64_t>(nextToken) * unitsPerRow + nextU);
+                    }
+                }
+            }
+        }
+    }
+}
+
 __device__ __forceinline__ float Bf16Lo(uint32_t w)
 {
     return __uint_as_float(w << 16);
@@ -865,6 +1103,7 @@ __device__ __forceinline__ void CombineColumns(const MF_GLOBAL u32x4 *in, MF_GLO
 // lose: 2048 tokens at top-2, 117 MB, 27.5 us without and 30.1 with them, 1000 at top-8 52.8 and 61.2.  Larger calls gain from the shorter
 // code alone: 1500 tokens 76.8 -> 74.3 us.
 constexpr uint64_t kCombineCachedBytes = 80ull << 20;
+constexpr uint32_t kCombineCachedEntries = 4096;        // measured with rows that were stored past the caches; rows in them change nothing (29 shapes)
 
 template <uint32_t kTopK, uint32_t kThreads, bool kNtLoad, uint32_t kBatch = 1>
 __global__ __launch_bounds__(kThreads) void MoeCombineKernel(const u32x4 *__restrict__ rowsIn,
@@ -1081,8 +1320,8 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
     uint32_t *blockHist = blockBad + histStride;
     const size_t histLds = static_cast<size_t>(kRankSlices) * experts * sizeof(uint32_t);
     const uint32_t upr = hidden / 8;
-    if (total <= kSmallEntries) {   // where the line lies: see the kernel
-        const bool rows = x != nullptr && out != nullptr;
+    const bool rows = x != nullptr && out != nullptr && hidden != 0;
+    if (total <= kSmallEntries && total * topK <= kSmallCompares) {   // where the lines lie: see the kernel
         const uint32_t least = (upr + kSmallHold * kSmallThreads - 1) / (kSmallHold * kSmallThreads);
         const uint32_t most = (upr + 63) / 64;
         uint32_t parts = (kSmallGroups + tokens - 1) / tokens;
@@ -1104,6 +1343,28 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
             MF_DISPATCH_SMALL(16);
         }
 #undef MF_DISPATCH_SMALL
+        return static_cast<int>(hipGetLastError());
+    }
+    const uint64_t moved = rows ? (static_cast<uint64_t>(tokens) + total) * upr * 16 : 0;
+    if (total <= kCountEntries && moved <= kCountBytes) {   // where the lines lie: see those
+        const uint32_t cus = static_cast<uint32_t>(mfrt_cu_count() > 0 ? mfrt_cu_count() : 256);
+        const uint32_t most = cus < kCountLeastGroups ? kCountLeastGroups : cus;
+        const uint32_t perGroup = (tokens + most - 1) / most;
+        const uint32_t lds = CountLdsWords(experts, perGroup * topK) * sizeof(uint32_t);
+#define MF_DISPATCH_COUNT(AHEAD, MODE, NT)                                                                             \
+    hipLaunchKernelGGL((MoeDispatchCountKernel<AHEAD, MODE, NT>), dim3((tokens + perGroup - 1) / perGroup),             \
+                       dim3(kCountThreads), lds, s, rows ? static_cast<const u32x4 *>(x) : nullptr, static_cast<const int32_t *>(topk), total, topK, \
+                       experts, upr, perGroup, static_cast<u32x4 *>(out), static_cast<int32_t *>(counts), static_cast<int32_t *>(offsets), \
+                       static_cast<int32_t *>(rowOf), static_cast<int32_t *>(srcOf), status)
+        const bool lines = hidden % 64 == 0;
+        if (lines && (moved <= kCountQuickBytes || (topK <= 4 && moved > kCountDeepBytes))) {
+            MF_DISPATCH_COUNT(4, 1, false);
+        } else if (moved <= kCountNearBytes) {
+            MF_DISPATCH_COUNT(4, 0, false);
+        } else {
+            MF_DISPATCH_COUNT(8, 0, true);
+        }
+#undef MF_DISPATCH_COUNT
         return static_cast<int>(hipGetLastError());
     }
     // The output-ordered tile permute needs the token rows of one step (a block of kRankBlock entries, or a half, a
@@ -1132,7 +1393,7 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
     // of the others itself.  Dispatch of rows of 1024 elements, with the launch / so: 2200 tokens at top-8 over 256 experts (18 blocks)
     // 20.1 / 17.6 us, 3000 (24) 19.7 / 18.3, 4096 (32) 22.2 / 22.0 (of 7168 elements 90.3 / 90.6).  The counts of a wave land on few LDS
     // words when the experts are few: over 64, 12 blocks 15.7 / 13.8, 16 34.5 / 34.0, 24 63.6 / 63.9 (longer rows); over 8, 16 blocks
-    // 19.7 / 20.2.
+    // 19.7 / 20.2.  (The short ones of these have one launch by now.)
     const bool counting = blocks <= (experts >= 128 ? kCountingBlocks : experts >= 64 ? 16u : 8u);
     const size_t rankLds = histLds + (experts + kRankThreads + kRankSlices + (tiles ? stepsPerBlock * experts : 0) +
                                       (counting ? experts : 0)) * sizeof(uint32_t);
@@ -1195,7 +1456,7 @@ extern "C" int mfk_moe_combine(const void *rows, const void *rowOf, const void *
     const uint32_t upr = hidden / 8;
     const uint64_t traffic = static_cast<uint64_t>(tokens) * (topK + 2) * upr * 16;   // the rows, the tokens they came from, the result
     const bool fanIn = topK == 2 || topK == 4 || topK == 6 || topK == 8;
-    if (upr >= 256 && fanIn && static_cast<uint64_t>(tokens) * topK <= kSmallEntries && traffic <= kCombineCachedBytes) {
+    if (upr >= 256 && fanIn && static_cast<uint64_t>(tokens) * topK <= kCombineCachedEntries && traffic <= kCombineCachedBytes) {
         // One column position per lane and plain loads: where the line lies, see kCombineCachedBytes.
         const uint32_t parts = (upr + 63) / 64;
 #define MF_COMBINE_CACHED(K) hipLaunchKernelGGL((MoeCombineKernel<K, 64, false>), dim3(tokens * parts), dim3(64), 0, s, in, ro, w, topK, upr, parts, o)

@@ -448,6 +448,39 @@ def test_rows_read_ahead_of_the_permute(gpu, oracle, T, H, K, E):
         _free(bufs)
 
 
+@pytest.mark.parametrize("T,H,K,E", [
+    (256, 72, 8, 256), (257, 72, 8, 256), (1025, 8, 16, 512),       # the last call whose tokens look at one another, the first that counts
+    (1171, 24, 7, 65), (3073, 16, 3, 1), (2201, 1032, 2, 16),       # ids that end inside a vector; one expert; rows that end inside a wave
+    (49152, 8, 1, 17), (49153, 8, 1, 17), (6145, 520, 8, 64),       # the last call that counts, and the first beyond
+    (700, 5120, 8, 256), (703, 5128, 8, 256), (1000, 7168, 8, 128), (4100, 7168, 2, 8),   # each form of its stores
+    (2674, 7168, 6, 256), (2675, 7168, 6, 256), (6200, 4104, 8, 16),                      # 255.9 and 256.2 MiB of rows; tokens that waves walk
+])
+def test_dispatch_that_counts_in_one_launch(gpu, T, H, K, E):
+    """Against a stable sort; some ids out of range, whose entries get no row."""
+    rng = np.random.default_rng(T + K)
+    x = np.arange(T * H, dtype=np.uint32).astype(np.uint16).reshape(T, H) ^ (np.arange(T, dtype=np.uint32) * 3).astype(np.uint16)[:, None]
+    topk = rng.integers(0, E, (T, K)).astype(np.int32)
+    late = topk.copy()
+    late.reshape(-1)[[1, T * K // 2, T * K - 1]] = [-1, E, 0x7FFFFFFF]
+    for ids, with_rows in ((topk, True), (late, True), (late, False)):
+        flat = np.where((ids < 0) | (ids >= E), E, ids).reshape(-1)
+        order = np.argsort(flat, kind="stable")[:int((flat < E).sum())]
+        row_of = np.full(T * K, -1, dtype=np.int32)
+        row_of[order] = np.arange(len(order), dtype=np.int32)
+        counts = np.bincount(flat, minlength=E + 1)[:E]
+        bufs = _gpu_dispatch(gpu, x, ids, E, with_rows)
+        try:
+            assert _fetch(bufs["ws"], np.uint32, (1,))[0] == int(len(order) != T * K)
+            assert np.array_equal(_fetch(bufs["counts"], np.int32, (E,)), counts)
+            assert np.array_equal(_fetch(bufs["offsets"], np.int32, (E,)), np.cumsum(counts) - counts)
+            assert np.array_equal(_fetch(bufs["row_of"], np.int32, (T * K,)), row_of)
+            assert np.array_equal(_fetch(bufs["src_of"], np.int32, (len(order),)), order)
+            if with_rows:
+                assert np.array_equal(_fetch(bufs["out"], np.uint16, (len(order), H)), x[order // K])
+        finally:
+            _free(bufs)
+
+
 @pytest.mark.parametrize("T,H,K", [
     (1, 7168, 8), (3, 2048, 2), (33, 2056, 4),           # few entries: one column position per lane, rows of 256 and 257 units
     (512, 2048, 8), (513, 2048, 8),                      # the last call of 4096 entries and one beyond
