@@ -35,6 +35,7 @@
 #include <atomic>
 
 #include "../rt/mf_rt.h"
+#include "launch.h"
 #include "window_clock.h"
 
 namespace mf {
@@ -58,6 +59,13 @@ constexpr uint32_t kHistPad = 32;                      // rows of the [expert][b
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef int32_t i32x4a __attribute__((ext_vector_type(4), aligned(4)));
 #define MF_GLOBAL __attribute__((address_space(1)))
+
+// Buffers of kernels that short calls launch arrive as addresses: the runtime looks every pointer argument up (launch.h).
+template <typename T>
+__device__ __forceinline__ T *Buffer(uint64_t address)
+{
+    return (T *)reinterpret_cast<MF_GLOBAL T *>(address);
+}
 
 // Lanes of the wave whose expert id equals mine (among lanes with valid == true).
 __device__ __forceinline__ uint64_t PeersOf(uint32_t expert, bool valid, uint32_t bits)
@@ -632,20 +640,28 @@ __device__ __forceinline__ uint32_t SmallKey(int32_t id, uint32_t index, uint32_
 }
 
 template <uint32_t kSlots>
-__global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(const u32x4 *__restrict__ x, const int32_t *__restrict__ topk,
-                                                                        uint32_t total, uint32_t topK, uint32_t experts,
-                                                                        uint32_t unitsPerRow, uint32_t parts, uint32_t perPart,
-                                                                        uint32_t groups, u32x4 *__restrict__ out, int32_t *__restrict__ counts,
-                                                                        int32_t *__restrict__ offsets, int32_t *__restrict__ rowOf,
-                                                                        int32_t *__restrict__ srcOf, uint32_t *__restrict__ status)
+__global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(uint64_t x, uint64_t topkAt, uint32_t total, uint32_t topK,
+                                                                        uint32_t experts, uint32_t unitsPerRow, uint32_t parts,
+                                                                        uint32_t perPart, uint32_t groups, uint64_t out,
+                                                                        uint64_t countsAt, uint64_t offsetsAt, uint64_t rowOfAt,
+                                                                        uint64_t srcOfAt, uint64_t statusAt)
 {
+    const int32_t *const topk = Buffer<const int32_t>(topkAt);
+    int32_t *const counts = Buffer<int32_t>(countsAt);
+    int32_t *const offsets = Buffer<int32_t>(offsetsAt);
+    int32_t *const rowOf = Buffer<int32_t>(rowOfAt);
+    int32_t *const srcOf = Buffer<int32_t>(srcOfAt);
     __shared__ uint32_t lds[kMaxExperts + kSmallThreads / 64];
+    __shared__ uint32_t anyBad;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = threadIdx.x >> 6;
     if (blockIdx.x == groups - 1) {
         uint32_t *perWave = lds + kMaxExperts;
         for (uint32_t e = threadIdx.x; e < kMaxExperts; e += kSmallThreads) {
             lds[e] = 0;
+        }
+        if (threadIdx.x == 0) {
+            anyBad = 0;
         }
         __syncthreads();
         uint32_t bad = 0;
@@ -666,7 +682,10 @@ __global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(const u3
                 }
             }
         }
-        bad = __syncthreads_or(static_cast<int>(bad)) != 0 ? 1u : 0u;
+        if (bad != 0) {
+            anyBad = 1;
+        }
+        __syncthreads();
         constexpr uint32_t kPer = kMaxExperts / kSmallThreads;   // neighbouring experts per thread
         uint32_t mine[kPer];
         uint32_t incl = 0;
@@ -699,7 +718,7 @@ __global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(const u3
             run += mine[j];
         }
         if (threadIdx.x == 0) {
-            status[0] = bad;
+            *Buffer<uint32_t>(statusAt) = anyBad;
         }
         return;
     }
@@ -707,9 +726,9 @@ __global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(const u3
     const uint32_t part = blockIdx.x - token * parts;
     const uint32_t begin = part * perPart;
     const uint32_t end = begin + perPart < unitsPerRow ? begin + perPart : unitsPerRow;
-    const MF_GLOBAL u32x4 *src = reinterpret_cast<const MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(x)) +
+    const MF_GLOBAL u32x4 *src = reinterpret_cast<const MF_GLOBAL u32x4 *>(x) +
                                  static_cast<uint64_t>(token) * unitsPerRow;
-    MF_GLOBAL u32x4 *dst = reinterpret_cast<MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(out));
+    MF_GLOBAL u32x4 *dst = reinterpret_cast<MF_GLOBAL u32x4 *>(out);
     u32x4 v[kSmallHold];
 #pragma unroll
     for (uint32_t j = 0; j < kSmallHold; ++j) {
@@ -772,7 +791,7 @@ __global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(const u3
     if (part == 0 && threadIdx.x < topK) {
         const int32_t row = static_cast<int32_t>(lds[threadIdx.x]);
         rowOf[first + threadIdx.x] = row;
-        if (srcOf != nullptr && row >= 0) {
+        if (srcOfAt != 0 && row >= 0) {
             srcOf[row] = static_cast<int32_t>(first + threadIdx.x);
         }
     }
@@ -816,10 +835,10 @@ __host__ __device__ constexpr uint32_t CountCopiesLog(uint32_t experts)
     return experts <= 16 ? 6 : experts <= 64 ? 4 : 2;
 }
 
-// [experts][copies] counts, [experts] first rows, a sum per wave, the rows of the own entries, [slices][experts] of those
+// [experts][copies] counts, [experts] first rows, a sum per wave, whether an id is out of range, the rows of the own entries, [slices][experts] of those
 constexpr uint32_t CountLdsWords(uint32_t experts, uint32_t ownMost)
 {
-    return (experts << CountCopiesLog(experts)) + experts + kCountWaves + ownMost + (ownMost + 63) / 64 * experts;
+    return (experts << CountCopiesLog(experts)) + experts + kCountWaves + 1 + ownMost + (ownMost + 63) / 64 * experts;
 }
 
 // The lines lie where the token rows and the stored rows together, in bytes, change what a store should do.
@@ -845,13 +864,16 @@ __device__ __forceinline__ u32x4 RowLoad(const MF_GLOBAL u32x4 *p)
 }
 
 template <uint32_t kAhead, int kMode, bool kNtLoad>
-__global__ __launch_bounds__(kCountThreads) void MoeDispatchCountKernel(const u32x4 *__restrict__ x, const int32_t *__restrict__ topk,
-                                                                        uint32_t total, uint32_t topK, uint32_t experts,
-                                                                        uint32_t unitsPerRow, uint32_t perGroup, u32x4 *__restrict__ out,
-                                                                        int32_t *__restrict__ counts, int32_t *__restrict__ offsets,
-                                                                        int32_t *__restrict__ rowOf, int32_t *__restrict__ srcOf,
-                                                                        uint32_t *__restrict__ status)
+__global__ __launch_bounds__(kCountThreads) void MoeDispatchCountKernel(uint64_t x, uint64_t topkAt, uint32_t total, uint32_t topK,
+                                                                        uint32_t experts, uint32_t unitsPerRow, uint32_t perGroup,
+                                                                        uint64_t out, uint64_t countsAt, uint64_t offsetsAt,
+                                                                        uint64_t rowOfAt, uint64_t srcOfAt, uint64_t statusAt)
 {
+    const int32_t *const topk = Buffer<const int32_t>(topkAt);
+    int32_t *const counts = Buffer<int32_t>(countsAt);
+    int32_t *const offsets = Buffer<int32_t>(offsetsAt);
+    int32_t *const rowOf = Buffer<int32_t>(rowOfAt);
+    int32_t *const srcOf = Buffer<int32_t>(srcOfAt);
     extern __shared__ uint32_t lds[];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = threadIdx.x >> 6;
@@ -861,7 +883,8 @@ __global__ __launch_bounds__(kCountThreads) void MoeDispatchCountKernel(const u3
     uint32_t *count = lds;
     uint32_t *base = count + (experts << copiesLog);
     uint32_t *scan = base + experts;
-    uint32_t *rows = scan + kCountWaves;
+    uint32_t *rows = scan + kCountWaves + 1;
+    uint32_t *anyBad = scan + kCountWaves;
     uint32_t *hist = rows + ownMost;
     const uint32_t begin = blockIdx.x * ownMost;
     const uint32_t end = begin + ownMost < total ? begin + ownMost : total;
@@ -876,10 +899,10 @@ __global__ __launch_bounds__(kCountThreads) void MoeDispatchCountKernel(const u3
     const int32_t ownId = own < end ? topk[own] : -1;
     const uint32_t tokens = (end - begin) / topK;
     const uint32_t parts = (unitsPerRow + 63) / 64;     // pieces of 64 units
-    const uint32_t items = x != nullptr ? tokens * parts : 0;
-    const MF_GLOBAL u32x4 *src = reinterpret_cast<const MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(x)) +
+    const uint32_t items = x != 0 ? tokens * parts : 0;
+    const MF_GLOBAL u32x4 *src = reinterpret_cast<const MF_GLOBAL u32x4 *>(x) +
                                  static_cast<uint64_t>(blockIdx.x) * perGroup * unitsPerRow;
-    MF_GLOBAL u32x4 *dst = reinterpret_cast<MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(out));
+    MF_GLOBAL u32x4 *dst = reinterpret_cast<MF_GLOBAL u32x4 *>(out);
     u32x4 v[kAhead];
 #pragma unroll
     for (uint32_t j = 0; j < kAhead; ++j) {
@@ -897,6 +920,9 @@ __global__ __launch_bounds__(kCountThreads) void MoeDispatchCountKernel(const u3
     }
     for (uint32_t i = threadIdx.x; i < slices * experts; i += kCountThreads) {
         hist[i] = 0;
+    }
+    if (threadIdx.x == 0) {
+        *anyBad = 0;
     }
     __syncthreads();
     uint32_t bad = 0;
@@ -939,7 +965,10 @@ __global__ __launch_bounds__(kCountThreads) void MoeDispatchCountKernel(const u3
             hist[wave * experts + static_cast<uint32_t>(ownId)] = __popcll(peers);
         }
     }
-    bad = __syncthreads_or(static_cast<int>(bad)) != 0 ? 1u : 0u;
+    if (bad != 0) {
+        *anyBad = 1;
+    }
+    __syncthreads();
     uint32_t all = 0;
     uint32_t before = 0;
     if (threadIdx.x < experts) {
@@ -975,7 +1004,7 @@ __global__ __launch_bounds__(kCountThreads) void MoeDispatchCountKernel(const u3
             offsets[threadIdx.x] = static_cast<int32_t>(run);
         }
         if (threadIdx.x == 0) {
-            status[0] = bad;
+            *Buffer<uint32_t>(statusAt) = *anyBad;
         }
     }
     if (own < end) {
@@ -989,7 +1018,7 @@ __global__ __launch_bounds__(kCountThreads) void MoeDispatchCountKernel(const u3
             for (uint32_t s = 0; s < wave; ++s) {
                 row += hist[s * experts + e];
             }
-            if (srcOf != nullptr) {
+            if (srcOfAt != 0) {
                 srcOf[row] = static_cast<int32_t>(own);
             }
         }
@@ -1106,11 +1135,11 @@ constexpr uint64_t kCombineCachedBytes = 80ull << 20;
 constexpr uint32_t kCombineCachedEntries = 4096;        // measured with rows that were stored past the caches; rows in them change nothing (29 shapes)
 
 template <uint32_t kTopK, uint32_t kThreads, bool kNtLoad, uint32_t kBatch = 1>
-__global__ __launch_bounds__(kThreads) void MoeCombineKernel(const u32x4 *__restrict__ rowsIn,
-                                                             const int32_t *__restrict__ rowOf,
-                                                             const float *__restrict__ weights, uint32_t topK,
-                                                             uint32_t unitsPerRow, uint32_t parts, u32x4 *__restrict__ y)
+__global__ __launch_bounds__(kThreads) void MoeCombineKernel(uint64_t rowsIn, uint64_t rowOfAt, uint64_t weightsAt, uint32_t topK,
+                                                             uint32_t unitsPerRow, uint32_t parts, uint64_t y)
 {
+    const int32_t *const rowOf = Buffer<const int32_t>(rowOfAt);
+    const float *const weights = Buffer<const float>(weightsAt);
     const uint32_t token = blockIdx.x / parts;
     const uint32_t part = blockIdx.x - token * parts;
     const uint32_t perPart = (unitsPerRow + parts - 1) / parts;
@@ -1136,8 +1165,8 @@ __global__ __launch_bounds__(kThreads) void MoeCombineKernel(const u32x4 *__rest
             w[k] = 0.0f;
         }
     }
-    const MF_GLOBAL u32x4 *in = reinterpret_cast<const MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(rowsIn));
-    MF_GLOBAL u32x4 *dst = reinterpret_cast<MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(y)) +
+    const MF_GLOBAL u32x4 *in = reinterpret_cast<const MF_GLOBAL u32x4 *>(rowsIn);
+    MF_GLOBAL u32x4 *dst = reinterpret_cast<MF_GLOBAL u32x4 *>(y) +
                            static_cast<uint64_t>(token) * unitsPerRow;
     if (kTopK != 0 && live == (1u << nk) - 1u) {
         CombineColumns<kTopK, kThreads, kNtLoad, kBatch, true>(in, dst, rowBase, w, live, begin, end);
@@ -1291,6 +1320,11 @@ std::atomic<uint32_t> g_combineWriteMBps{6200000};
 }  // namespace
 }  // namespace mf
 
+static uint64_t At(const void *buffer)
+{
+    return reinterpret_cast<uint64_t>(buffer);
+}
+
 extern "C" uint64_t mfk_moe_workspace_bytes(uint32_t tokens, uint32_t topK, uint32_t experts)
 {
     const uint64_t total = static_cast<uint64_t>(tokens) * topK;
@@ -1329,10 +1363,8 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
         const uint32_t perPart = rows ? ((upr + parts - 1) / parts + 7) / 8 * 8 : 0;   // whole cache lines
         parts = rows ? (upr + perPart - 1) / perPart : 1;
 #define MF_DISPATCH_SMALL(SLOTS)                                                                                       \
-    hipLaunchKernelGGL(MoeDispatchSmallKernel<SLOTS>, dim3(tokens * parts + 1), dim3(kSmallThreads), 0, s,              \
-                       static_cast<const u32x4 *>(x), static_cast<const int32_t *>(topk), total, topK, experts, upr, parts, perPart, \
-                       tokens * parts + 1, static_cast<u32x4 *>(out), static_cast<int32_t *>(counts), static_cast<int32_t *>(offsets),      \
-                       static_cast<int32_t *>(rowOf), static_cast<int32_t *>(srcOf), status)
+    return Launch(MoeDispatchSmallKernel<SLOTS>, tokens * parts + 1, kSmallThreads, 0, s, At(x), At(topk), total, topK, experts, upr, parts, \
+                  perPart, tokens * parts + 1, At(out), At(counts), At(offsets), At(rowOf), At(srcOf), At(workspace))
         if (topK <= 2) {
             MF_DISPATCH_SMALL(2);
         } else if (topK <= 4) {
@@ -1343,7 +1375,6 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
             MF_DISPATCH_SMALL(16);
         }
 #undef MF_DISPATCH_SMALL
-        return static_cast<int>(hipGetLastError());
     }
     const uint64_t moved = rows ? (static_cast<uint64_t>(tokens) + total) * upr * 16 : 0;
     if (total <= kCountEntries && moved <= kCountBytes) {   // where the lines lie: see those
@@ -1352,10 +1383,8 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
         const uint32_t perGroup = (tokens + most - 1) / most;
         const uint32_t lds = CountLdsWords(experts, perGroup * topK) * sizeof(uint32_t);
 #define MF_DISPATCH_COUNT(AHEAD, MODE, NT)                                                                             \
-    hipLaunchKernelGGL((MoeDispatchCountKernel<AHEAD, MODE, NT>), dim3((tokens + perGroup - 1) / perGroup),             \
-                       dim3(kCountThreads), lds, s, rows ? static_cast<const u32x4 *>(x) : nullptr, static_cast<const int32_t *>(topk), total, topK, \
-                       experts, upr, perGroup, static_cast<u32x4 *>(out), static_cast<int32_t *>(counts), static_cast<int32_t *>(offsets), \
-                       static_cast<int32_t *>(rowOf), static_cast<int32_t *>(srcOf), status)
+    return Launch(MoeDispatchCountKernel<AHEAD, MODE, NT>, (tokens + perGroup - 1) / perGroup, kCountThreads, lds, s, rows ? At(x) : 0, \
+                  At(topk), total, topK, experts, upr, perGroup, At(out), At(counts), At(offsets), At(rowOf), At(srcOf), At(workspace))
         const bool lines = hidden % 64 == 0;
         if (lines && (moved <= kCountQuickBytes || (topK <= 4 && moved > kCountDeepBytes))) {
             MF_DISPATCH_COUNT(4, 1, false);
@@ -1365,7 +1394,6 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
             MF_DISPATCH_COUNT(8, 0, true);
         }
 #undef MF_DISPATCH_COUNT
-        return static_cast<int>(hipGetLastError());
     }
     // The output-ordered tile permute needs the token rows of one step (a block of kRankBlock entries, or a half, a
     // quarter ... down to one slice of 64 entries: stepEntries / topK tokens) to stay in an XCD's 4 MiB L2 while the
@@ -1459,7 +1487,7 @@ extern "C" int mfk_moe_combine(const void *rows, const void *rowOf, const void *
     if (upr >= 256 && fanIn && static_cast<uint64_t>(tokens) * topK <= kCombineCachedEntries && traffic <= kCombineCachedBytes) {
         // One column position per lane and plain loads: where the line lies, see kCombineCachedBytes.
         const uint32_t parts = (upr + 63) / 64;
-#define MF_COMBINE_CACHED(K) hipLaunchKernelGGL((MoeCombineKernel<K, 64, false>), dim3(tokens * parts), dim3(64), 0, s, in, ro, w, topK, upr, parts, o)
+#define MF_COMBINE_CACHED(K) return Launch(MoeCombineKernel<K, 64, false, 1>, tokens * parts, 64, 0, s, At(rows), At(rowOf), At(weights), topK, upr, parts, At(y))
         if (topK == 2) {
             MF_COMBINE_CACHED(2);
         } else if (topK == 4) {
@@ -1493,11 +1521,11 @@ extern "C" int mfk_moe_combine(const void *rows, const void *rowOf, const void *
         // and top-2 loses (16 384 x 4096: 79 against 66 us): their read parts are too short for the switch to pay.
         const bool windows = paced != 0 && topK >= 6 && items >= static_cast<uint64_t>(waves) * kCombineMinItemsPerWave &&
                              items < 0x40000000ull && readTicks != 0 && writeTicks != 0;
-        const dim3 grid(windows ? waves : tokens * parts);
+        const uint32_t grid = windows ? waves : tokens * parts;
 #define MF_COMBINE_SLICES(K)                                                                                           \
-    hipLaunchKernelGGL((MoeCombineKernel<K, 64, true, 2>), grid, dim3(64), 0, s, in, ro, w, topK, upr, parts, o)
+    return Launch(MoeCombineKernel<K, 64, true, 2>, grid, 64, 0, s, At(rows), At(rowOf), At(weights), topK, upr, parts, At(y))
 #define MF_COMBINE_WINDOWS(K)                                                                                          \
-    hipLaunchKernelGGL((MoeCombineWindowKernel<kCombineItems, K>), grid, dim3(64), 0, s, in, ro, w, upr, parts,        \
+    hipLaunchKernelGGL((MoeCombineWindowKernel<kCombineItems, K>), dim3(grid), dim3(64), 0, s, in, ro, w, upr, parts,        \
                        static_cast<uint32_t>(items), o, readTicks, writeTicks, NextWindowSeq())
         if (topK == 2) {
             MF_COMBINE_SLICES(2);
@@ -1518,7 +1546,7 @@ extern "C" int mfk_moe_combine(const void *rows, const void *rowOf, const void *
 #undef MF_COMBINE_WINDOWS
     } else {
         // Narrow rows: one four-wave workgroup per token, compiled for the common fan-ins too, whose loads are then in flight together.
-#define MF_COMBINE_TOKEN(K) hipLaunchKernelGGL((MoeCombineKernel<K, 256, true>), dim3(tokens), dim3(256), 0, s, in, ro, w, topK, upr, 1u, o)
+#define MF_COMBINE_TOKEN(K) return Launch(MoeCombineKernel<K, 256, true, 1>, tokens, 256, 0, s, At(rows), At(rowOf), At(weights), topK, upr, 1u, At(y))
         if (topK == 2) {
             MF_COMBINE_TOKEN(2);
         } else if (topK == 4) {
