@@ -151,8 +151,7 @@ struct Batch {
     TablePlan pinned;                   // triples in pinned host memory, owner by pattern
     TablePlan hbm;                      // triples in HBM, owner by pattern
     TablePlan grouped;                  // triples, prefix and group map in HBM, no pattern
-    const Piece *pieces;                // of 4 KiB, in pinned host memory: as many as nchunk
-    const Piece *deepPieces;            // of 16 KiB (what the library takes for 4 to 64 MiB)
+    const Piece *deepPieces;            // of 16 KiB (what the library takes for 4 to 64 MiB), in pinned host memory
     uint32_t ndeep;
     uint64_t bytes;
     uint32_t nchunk;
@@ -250,7 +249,7 @@ std::vector<Batch> MakeBatches(char *pool, uint64_t poolBytes, int count, uint32
     char *devTables = nullptr;
     MF_CHECK(hipHostMalloc(&hostTables, tableBytes * count, hipHostMallocDefault));
     MF_CHECK(hipMalloc(&devTables, tableBytes * count));
-    MF_CHECK(hipHostMalloc(&pieces, sizeof(Piece) * (nchunk + ndeep) * count, hipHostMallocDefault));
+    MF_CHECK(hipHostMalloc(&pieces, sizeof(Piece) * ndeep * count, hipHostMallocDefault));
     std::vector<Batch> batches(count);
     for (int b = 0; b < count; ++b) {
         std::vector<uint32_t> pick;
@@ -317,12 +316,8 @@ std::vector<Batch> MakeBatches(char *pool, uint64_t poolBytes, int count, uint32
         const char *dev = devTables + b * tableBytes;
         plan.triples = reinterpret_cast<const uint64_t *>(dev);
         batch.hbm = plan;
-        batch.pieces = pieces;
         batch.bytes = 0;
         for (uint32_t i = 0; i < nseg; ++i) {
-            for (uint64_t off = 0; off < triples[3 * i + 2]; off += 4096) {
-                *pieces++ = MakePiece(triples[3 * i] + off, triples[3 * i + 1] + off, 4096);
-            }
             batch.bytes += triples[3 * i + 2];
         }
         batch.deepPieces = pieces;

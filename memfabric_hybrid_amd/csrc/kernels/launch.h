@@ -15,6 +15,18 @@
 namespace mf {
 namespace {
 
+// A buffer as such kernels get it, and what they make of it.
+inline uint64_t At(const volatile void *buffer)
+{
+    return reinterpret_cast<uint64_t>(buffer);
+}
+
+template <typename T>
+__device__ __forceinline__ T *Buffer(uint64_t address)
+{
+    return (T *)reinterpret_cast<__attribute__((address_space(1))) T *>(address);
+}
+
 // What <<<>>> does without the launch configuration that it pushes and pops around the same call (0.15 us).  `args` are converted to the types
 // of the kernel's parameters.
 template <typename... Params, typename... Args>

@@ -60,13 +60,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef int32_t i32x4a __attribute__((ext_vector_type(4), aligned(4)));
 #define MF_GLOBAL __attribute__((address_space(1)))
 
-// Buffers of kernels that short calls launch arrive as addresses: the runtime looks every pointer argument up (launch.h).
-template <typename T>
-__device__ __forceinline__ T *Buffer(uint64_t address)
-{
-    return (T *)reinterpret_cast<MF_GLOBAL T *>(address);
-}
-
 // Lanes of the wave whose expert id equals mine (among lanes with valid == true).
 __device__ __forceinline__ uint64_t PeersOf(uint32_t expert, bool valid, uint32_t bits)
 {
@@ -1319,11 +1312,6 @@ std::atomic<uint32_t> g_combineWriteMBps{6200000};
 
 }  // namespace
 }  // namespace mf
-
-static uint64_t At(const void *buffer)
-{
-    return reinterpret_cast<uint64_t>(buffer);
-}
 
 extern "C" uint64_t mfk_moe_workspace_bytes(uint32_t tokens, uint32_t topK, uint32_t experts)
 {

@@ -25,6 +25,7 @@
 #include <cstdlib>
 
 #include "xcopy_plan.h"
+#include "launch.h"
 #include "window_clock.h"
 #include "../rt/mf_rt.h"
 
@@ -448,13 +449,13 @@ __global__ __launch_bounds__(64) void XcopyWindowKernel(const InlinePlan p, uint
 constexpr uint32_t kSingleMaxChunks = 49152;
 template <bool kNtLoad, int kStore, int kHold = kHoldNone>
 __global__ __launch_bounds__(kXcopyThreads) void XcopySingleKernel(uint64_t src, uint64_t dst, uint32_t len, uint32_t nchunk,
-                                                                   uint32_t units, uint32_t holdTicks, uint32_t lanes)
+                                                                   uint32_t units, uint32_t holdTicks, uint32_t lanes, uint32_t groups)
 {
     const uint64_t t0 = kHold != kHoldNone ? wall_clock64() : 0;
     uint32_t c = blockIdx.x;
     do {
         CopyChunkHeld<kNtLoad, kStore, kHold>(src, dst, len, c, units, t0, holdTicks, lanes);
-        c += gridDim.x;
+        c += groups;
     } while (c < nchunk);
 }
 
@@ -464,10 +465,10 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopySingleKernel(uint64_t src,
 // for the whole grid.  (Signalling from inside the copy kernel needs a system-scope release in
 // every workgroup before it may count itself done, an L2 write-back each: 77 us instead of 5.5 us
 // for an 9 MB batch.)  An empty batch gets the word alone.
-__global__ void XcopySignalKernel(uint64_t *mask, uint32_t maskValue)
+__global__ void XcopySignalKernel(uint64_t mask, uint32_t maskValue)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
-        __hip_atomic_store(mask, static_cast<uint64_t>(maskValue), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(Buffer<uint64_t>(mask), static_cast<uint64_t>(maskValue), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -506,13 +507,13 @@ __device__ __forceinline__ void MarkDone(const DoneMark &mark)
 // (Arguments one by one: the 56 bytes are in scalar registers when a wave starts, those of a struct are memory it has to read.)
 template <bool kNtLoad>
 __global__ __launch_bounds__(kXcopyThreads) void XcopySingleDoneKernel(uint64_t src, uint64_t dst, uint32_t len, uint32_t nchunk,
-                                                                       uint32_t units, uint32_t lanes, uint64_t *word, uint32_t *counter,
+                                                                       uint32_t units, uint32_t lanes, uint64_t word, uint64_t counter,
                                                                        uint32_t value, uint32_t groups)
 {
     for (uint32_t c = blockIdx.x; c < nchunk; c += groups) {
         CopyChunk<kNtLoad, kStoreThrough>(src, dst, len, c, units, 0, 0, lanes);
     }
-    MarkDone(DoneMark{word, counter, value, groups});
+    MarkDone(DoneMark{Buffer<uint64_t>(word), Buffer<uint32_t>(counter), value, groups});
 }
 
 template <bool kNtLoad>
@@ -667,8 +668,9 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyTableKernel(const TablePla
 // gathered 45.8 / 49.4 / 46.4 us with 4 KiB waves / 16 KiB waves / four waves, scattered 49.9 / 51.4 / 49.2, and a quarter of the
 // descriptors for the host to write.
 template <uint32_t kLanes, uint32_t kUnits, bool kHold>
-__global__ __launch_bounds__(kLanes) void XcopyPieceKernel(const Piece *__restrict__ pieces, uint32_t count, uint32_t holdTicks)
+__global__ __launch_bounds__(kLanes) void XcopyPieceKernel(uint64_t list, uint32_t count, uint32_t holdTicks)
 {
+    const Piece *const pieces = Buffer<const Piece>(list);
     const uint64_t t0 = kHold ? wall_clock64() : 0;
     const uint32_t at = PieceOf(blockIdx.x);
     if (at >= count) {
@@ -743,22 +745,23 @@ __global__ __launch_bounds__(kLanes) void XcopyPieceKernel(const Piece *__restri
 // (A schedule that stretches when sampled waves fall behind it was tried: it overshoots, 20 to 50 % slower than none.)
 // What a lane past the end of its piece loads is the last unit: a load under a condition would leave the registers of the
 // loop's last round alive in the others and take more of them than sixteen waves per CU have.
-__global__ __launch_bounds__(64) void XcopyPieceWindowKernel(const Piece *__restrict__ pieces, uint32_t count, uint32_t period, uint32_t seq)
+__global__ __launch_bounds__(64) void XcopyPieceWindowKernel(uint64_t list, uint32_t count, uint32_t period, uint32_t seq, uint32_t groups)
 {
+    const Piece *const pieces = Buffer<const Piece>(list);
     uint32_t at = PieceOf(blockIdx.x);
     if (at >= count) {
         return;
     }
     Piece next = pieces[at];
     const uint32_t half = period / 2;
-    uint64_t slot = AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * half / gridDim.x;
+    uint64_t slot = AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * half / groups;
     for (;;) {
         uint32_t tid = threadIdx.x;
         asm volatile("" : "+v"(tid));       // offsets are computed in each round instead of held through all of them
         const uint64_t srcWord = Uniform(next.src);
         const uint64_t dstWord = Uniform(next.dst);
-        const bool more = count - at > gridDim.x;
-        next = pieces[more ? at + gridDim.x : at];
+        const bool more = count - at > groups;
+        next = pieces[more ? at + groups : at];
         const uint64_t src = srcWord & kPieceAddress;
         const uint64_t dst = dstWord & kPieceAddress;
         const uint32_t length = PieceLength(srcWord, dstWord);
@@ -798,7 +801,7 @@ __global__ __launch_bounds__(64) void XcopyPieceWindowKernel(const Piece *__rest
         if (!more) {
             return;
         }
-        at += gridDim.x;
+        at += groups;
         slot += period;
     }
 }
@@ -1054,8 +1057,10 @@ __device__ __forceinline__ bool PlannedQuad(const uint64_t *__restrict__ triples
 // 1 to 3 us slower.  Looking four chunks ahead of a quad up while it loads: registers spill, 8000 pages of 8 KiB 33.3.
 template <uint32_t kWaves, uint32_t kRun>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(4, 4)))
-void XcopyPlannedKernel(const uint64_t *__restrict__ triples, uint32_t nseg, TablePace pace)
+void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
 {
+    constexpr uint32_t kGroups = kWindowWaves / kWaves;     // the launch's workgroups
+    const uint64_t *const triples = Buffer<const uint64_t>(table);
     extern __shared__ uint32_t words[];                     // PlannedLds()
     if (nseg == 0) {
         return;
@@ -1140,14 +1145,14 @@ void XcopyPlannedKernel(const uint64_t *__restrict__ triples, uint32_t nseg, Tab
     }
     __syncthreads();
 
-    const uint32_t grid = gridDim.x * kWaves;
+    constexpr uint32_t grid = kWindowWaves;
     const uint32_t items = quads ? (nchunk + 3) / 4 : nchunk;
     const bool held = large && items <= grid && total <= kPlannedHeldChunks;
     const bool paced = large && total > kPlannedHeldChunks && aligned && pace.windowTicks != 0 &&
                        static_cast<uint64_t>(total) * 100 >= static_cast<uint64_t>(items) * (4 * kPlannedFullPercent);
     const uint32_t rounds = (items + grid - 1) / grid;
     const uint32_t waves = paced ? (items + rounds - 1) / rounds : grid;
-    uint32_t item = wave * gridDim.x + blockIdx.x;          // neighbouring ones on neighbouring XCDs
+    uint32_t item = wave * kGroups + blockIdx.x;          // neighbouring ones on neighbouring XCDs
     if (item >= items || item >= waves) {
         return;
     }
@@ -1407,18 +1412,13 @@ int LaunchInline(const InlinePlan &plan, uint32_t grid, uint32_t lanes, hipStrea
     if (plan.first[1] == kNoChunk && plan.nchunk <= kSingleMaxChunks) {
         if (anyOrder) {
             hipExtLaunchKernelGGL((XcopySingleKernel<kNtLoad, kStore>), dim3(grid), dim3(lanes), 0, stream, nullptr, nullptr, flags,
-                                  plan.src[0], plan.dst[0], plan.len[0], plan.nchunk, plan.units, 0u, lanes);
-        } else if (ticks != 0 && deep) {
-            hipLaunchKernelGGL((XcopySingleKernel<kNtLoad, kStore, kHoldDeep>), dim3(grid), dim3(lanes), 0, stream, plan.src[0],
-                               plan.dst[0], plan.len[0], plan.nchunk, plan.units, ticks, lanes);
-        } else if (ticks != 0) {
-            hipLaunchKernelGGL((XcopySingleKernel<kNtLoad, kStore, kHoldShallow>), dim3(grid), dim3(lanes), 0, stream, plan.src[0],
-                               plan.dst[0], plan.len[0], plan.nchunk, plan.units, ticks, lanes);
-        } else {
-            hipLaunchKernelGGL((XcopySingleKernel<kNtLoad, kStore>), dim3(grid), dim3(lanes), 0, stream, plan.src[0], plan.dst[0],
-                               plan.len[0], plan.nchunk, plan.units, 0u, lanes);
+                                  plan.src[0], plan.dst[0], plan.len[0], plan.nchunk, plan.units, 0u, lanes, grid);
+            return static_cast<int>(hipGetLastError());
         }
-        return static_cast<int>(hipGetLastError());
+        const auto kernel = ticks == 0 ? XcopySingleKernel<kNtLoad, kStore, kHoldNone>
+                            : deep     ? XcopySingleKernel<kNtLoad, kStore, kHoldDeep>
+                                       : XcopySingleKernel<kNtLoad, kStore, kHoldShallow>;
+        return Launch(kernel, grid, lanes, 0, stream, plan.src[0], plan.dst[0], plan.len[0], plan.nchunk, plan.units, ticks, lanes, grid);
     }
     // The ordered launches go through hipLaunchKernel with an argument array: the triple-chevron form pushes and pops a
     // launch configuration around the same call, 0.15 us of host time per launch with this 3 KiB argument block.
@@ -1451,21 +1451,21 @@ int LaunchWindowed(const InlinePlan &plan, uint32_t grid, uint32_t windowMBps, h
 
 // A launch whose own end is what `event` (may be null) stands for: an event recorded behind a launch is a packet of its own, 2.8 us
 // of the stream's time (launches of 10 us with an event each 13.8 us, so 11.0, without 11.0).
-template <typename Kernel, typename... Args>
-void LaunchWithEvent(Kernel kernel, uint32_t grid, uint32_t lanes, hipStream_t stream, hipEvent_t event, Args... args)
+template <typename... Params, typename... Args>
+int LaunchWithEvent(void (*kernel)(Params...), uint32_t grid, uint32_t lanes, hipStream_t stream, hipEvent_t event, Args... args)
 {
-    if (event != nullptr) {
-        hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(lanes), 0, stream, nullptr, event, 0, args...);
-    } else {
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(lanes), 0, stream, args...);
+    if (event == nullptr) {
+        return Launch(kernel, grid, lanes, 0, stream, args...);
     }
+    hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(lanes), 0, stream, nullptr, event, 0, args...);
+    return static_cast<int>(hipGetLastError());
 }
 
 template <uint32_t kLanes, uint32_t kUnits, bool kHold>
-void LaunchPieces(const Piece *pieces, uint32_t count, uint32_t ticks, hipStream_t stream, hipEvent_t event)
+int LaunchPieces(const void *pieces, uint32_t count, uint32_t ticks, hipStream_t stream, hipEvent_t event)
 {
     const uint32_t grid = (count + kPieceGroup - 1) / kPieceGroup * kPieceGroup;
-    LaunchWithEvent(XcopyPieceKernel<kLanes, kUnits, kHold>, grid, kLanes, stream, event, pieces, count, ticks);
+    return LaunchWithEvent(XcopyPieceKernel<kLanes, kUnits, kHold>, grid, kLanes, stream, event, At(pieces), count, ticks);
 }
 
 template <bool kNtLoad, int kStore>
@@ -1478,11 +1478,10 @@ int LaunchDirect(const uint64_t *triples, uint32_t nseg, uint32_t units, uint32_
         return static_cast<int>(err);
     }
     const bool link = kStore != kStoreStream;
-    LaunchWithEvent(XcopyRestKernel<kNtLoad, kStore>, restGrid, link ? lanes : kRestLanes, stream, event, rest, capacity,
-                    link ? units : kDepth * kRestLanes);
-    err = hipGetLastError();
+    err = static_cast<hipError_t>(LaunchWithEvent(XcopyRestKernel<kNtLoad, kStore>, restGrid, link ? lanes : kRestLanes, stream, event, rest,
+                                                  capacity, link ? units : kDepth * kRestLanes));
     if (err != hipSuccess) {   // what the first launch has listed must not be taken for the next call's
-        hipLaunchKernelGGL(XcopySignalKernel, dim3(1), dim3(64), 0, stream, &rest->taken, 0u);
+        (void)Launch(XcopySignalKernel, 1, 64, 0, stream, At(&rest->taken), 0u);
     }
     return static_cast<int>(err);
 }
@@ -1492,8 +1491,7 @@ int Signal(void *mask, uint32_t maskValue, hipStream_t stream)
     if (mask == nullptr) {
         return 0;
     }
-    hipLaunchKernelGGL(XcopySignalKernel, dim3(1), dim3(64), 0, stream, static_cast<uint64_t *>(mask), maskValue);
-    return static_cast<int>(hipGetLastError());
+    return Launch(XcopySignalKernel, 1, 64, 0, stream, At(mask), maskValue);
 }
 
 }  // namespace
@@ -1593,24 +1591,23 @@ extern "C" int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t byt
     if (pieces == nullptr || count == 0 || count > kPieceMaxCount || (units != 256 && units != 512 && units != 1024)) {
         return -1;
     }
-    const Piece *p = static_cast<const Piece *>(pieces);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const uint32_t ticks = HoldTicks(PieceHoldNanos(holdNanos, count, bytes, units));
     const hipEvent_t end = static_cast<hipEvent_t>(event);
+    int err;
     if (units == 256 && ticks != 0) {
-        LaunchPieces<64, 4, true>(p, count, ticks, s, end);
+        err = LaunchPieces<64, 4, true>(pieces, count, ticks, s, end);
     } else if (units == 256) {
-        LaunchPieces<64, 4, false>(p, count, 0, s, end);
+        err = LaunchPieces<64, 4, false>(pieces, count, 0, s, end);
     } else if (units == 512 && ticks != 0) {
-        LaunchPieces<128, 4, true>(p, count, ticks, s, end);
+        err = LaunchPieces<128, 4, true>(pieces, count, ticks, s, end);
     } else if (units == 512) {
-        LaunchPieces<128, 4, false>(p, count, 0, s, end);
+        err = LaunchPieces<128, 4, false>(pieces, count, 0, s, end);
     } else if (ticks != 0) {
-        LaunchPieces<64, 16, true>(p, count, ticks, s, end);
+        err = LaunchPieces<64, 16, true>(pieces, count, ticks, s, end);
     } else {
-        LaunchPieces<256, 4, false>(p, count, 0, s, end);
+        err = LaunchPieces<256, 4, false>(pieces, count, 0, s, end);
     }
-    const int err = static_cast<int>(hipGetLastError());
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
@@ -1629,9 +1626,8 @@ extern "C" int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uin
         return static_cast<int>(hipErrorInvalidValue);
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    LaunchWithEvent(XcopyPieceWindowKernel, grid, 64, s, static_cast<hipEvent_t>(event), static_cast<const Piece *>(pieces), count, ticks,
-                    NextWindowSeq());
-    const int err = static_cast<int>(hipGetLastError());
+    const int err = LaunchWithEvent(XcopyPieceWindowKernel, grid, 64, s, static_cast<hipEvent_t>(event), At(pieces), count, ticks,
+                                    NextWindowSeq(), grid);
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
@@ -1684,15 +1680,11 @@ extern "C" int mfk_xcopy_planned(const void *triples, uint32_t nseg, uint32_t ho
         return -1;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const uint64_t *t = static_cast<const uint64_t *>(triples);
     const TablePace pace{HoldTicks(holdNanos), HoldTicks(holdMoreNanos), WindowPeriodTicks(2ull << 26, windowMBps), NextWindowSeq()};
-    if (nseg <= 64 * kPlannedShortRun) {
-        hipLaunchKernelGGL((XcopyPlannedKernel<1, kPlannedShortRun>), dim3(kWindowWaves), dim3(64), PlannedLds(1, nseg), s, t, nseg, pace);
-    } else {
-        hipLaunchKernelGGL((XcopyPlannedKernel<kPlannedWaves, kPlannedRun>), dim3(kWindowWaves / kPlannedWaves), dim3(64 * kPlannedWaves),
-                           PlannedLds(kPlannedWaves, nseg), s, t, nseg, pace);
-    }
-    const int err = static_cast<int>(hipGetLastError());
+    const int err = nseg <= 64 * kPlannedShortRun
+                        ? Launch(XcopyPlannedKernel<1, kPlannedShortRun>, kWindowWaves, 64, PlannedLds(1, nseg), s, At(triples), nseg, pace)
+                        : Launch(XcopyPlannedKernel<kPlannedWaves, kPlannedRun>, kWindowWaves / kPlannedWaves, 64 * kPlannedWaves,
+                                 PlannedLds(kPlannedWaves, nseg), s, At(triples), nseg, pace);
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
@@ -1725,22 +1717,22 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
             constexpr bool kNt = decltype(ntLoad)::value;
             constexpr int kSt = decltype(store)::value;
             hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, empty, 0u);
-            hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 0u, 64u);
+            hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 0u, 64u, 1u);
             hipLaunchKernelGGL((XcopyTableKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, none);
             if (route == MFRT_ROUTE_HBM) {
                 hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, empty, 1u);
                 hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, empty, 1u);
-                hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 1u, 64u);
-                hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kWindowUnits, 1u, 64u);
-                hipLaunchKernelGGL((XcopyPieceKernel<64, 4, false>), dim3(1), dim3(64), 0, s, nullptr, 0u, 0u);
-                hipLaunchKernelGGL((XcopyPieceKernel<64, 4, true>), dim3(1), dim3(64), 0, s, nullptr, 0u, 0u);
-                hipLaunchKernelGGL((XcopyPieceKernel<64, 16, true>), dim3(1), dim3(64), 0, s, nullptr, 0u, 0u);
-                hipLaunchKernelGGL((XcopyPieceKernel<128, 4, false>), dim3(1), dim3(128), 0, s, nullptr, 0u, 0u);
-                hipLaunchKernelGGL((XcopyPieceKernel<128, 4, true>), dim3(1), dim3(128), 0, s, nullptr, 0u, 0u);
-                hipLaunchKernelGGL((XcopyPieceKernel<256, 4, false>), dim3(1), dim3(256), 0, s, nullptr, 0u, 0u);
-                hipLaunchKernelGGL(XcopyPieceWindowKernel, dim3(1), dim3(64), 0, s, nullptr, 0u, 64u, NextWindowSeq());
-                hipLaunchKernelGGL((XcopyPlannedKernel<1, kPlannedShortRun>), dim3(1), dim3(64), 64, s, nullptr, 0u, TablePace{});
-                hipLaunchKernelGGL((XcopyPlannedKernel<kPlannedWaves, kPlannedRun>), dim3(1), dim3(64 * kPlannedWaves), 64, s, nullptr, 0u, TablePace{});
+                hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 1u, 64u, 1u);
+                hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kWindowUnits, 1u, 64u, 1u);
+                (void)Launch(XcopyPieceKernel<64, 4, false>, 1, 64, 0, s, 0, 0u, 0u);
+                (void)Launch(XcopyPieceKernel<64, 4, true>, 1, 64, 0, s, 0, 0u, 0u);
+                (void)Launch(XcopyPieceKernel<64, 16, true>, 1, 64, 0, s, 0, 0u, 0u);
+                (void)Launch(XcopyPieceKernel<128, 4, false>, 1, 128, 0, s, 0, 0u, 0u);
+                (void)Launch(XcopyPieceKernel<128, 4, true>, 1, 128, 0, s, 0, 0u, 0u);
+                (void)Launch(XcopyPieceKernel<256, 4, false>, 1, 256, 0, s, 0, 0u, 0u);
+                (void)Launch(XcopyPieceWindowKernel, 1, 64, 0, s, 0, 0u, 64u, NextWindowSeq(), 1u);
+                (void)Launch(XcopyPlannedKernel<1, kPlannedShortRun>, 1, 64, 64, s, 0, 0u, TablePace{});
+                (void)Launch(XcopyPlannedKernel<kPlannedWaves, kPlannedRun>, 1, 64 * kPlannedWaves, 64, s, 0, 0u, TablePace{});
                 hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
             }
             return 0;
@@ -1924,7 +1916,7 @@ extern "C" int mfk_xcopy_static_setup(void)
         uint32_t *words = g_scratchOf[dev];
         RestList *rest = reinterpret_cast<RestList *>(words);
         const uint64_t *none = reinterpret_cast<const uint64_t *>(words);
-        hipLaunchKernelGGL(XcopySignalKernel, dim3(1), dim3(64), 0, nullptr, rest->reserved, 0u);
+        (void)Launch(XcopySignalKernel, 1, 64, 0, nullptr, At(rest->reserved), 0u);
         hipLaunchKernelGGL(XcopyClearListsKernel, dim3(1), dim3(64), 0, nullptr, reinterpret_cast<uint8_t *>(rest), 0ull);
         for (int route = MFRT_ROUTE_HBM; route <= MFRT_ROUTE_FROM_HOST; ++route) {
             (void)WithPolicy(PolicyOf(route), [&](auto ntLoad, auto store) {
