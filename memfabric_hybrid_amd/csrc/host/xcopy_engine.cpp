@@ -1316,8 +1316,8 @@ bool HasDoneWord(ThreadLease &lease)
 bool HasDoneCounter(ThreadLease &lease)
 {
     if (lease.doneCounter == nullptr) {
-        lease.doneCounter = mfrt_alloc_device(64);
-        if (lease.doneCounter != nullptr && mfrt_memset(lease.doneCounter, 0, 64) != 0) {
+        lease.doneCounter = mfrt_alloc_device(kDoneCounterBytes);
+        if (lease.doneCounter != nullptr && mfrt_memset(lease.doneCounter, 0, kDoneCounterBytes) != 0) {
             (void)mfrt_free_device(lease.doneCounter);
             lease.doneCounter = nullptr;
         }
@@ -1361,12 +1361,18 @@ bool PollDone(const ThreadLease &lease, uint32_t seq, uint64_t least)
 int XcopyEngine::LaunchDone(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t bytes, int route,
                             void *stream, uint32_t &ticket)
 {
-    // To the host a copy has few workgroups whatever its size, and each costs the launch one atomic at its end.  In HBM one of
-    // up to kDoneBytes has few enough (the kernel has the figures).  From the host written-through stores cost more than the
+    // To the host a copy has few workgroups whatever its size, and each costs the launch one atomic at its end.  In HBM they are worth
+    // it (a launch less for the host, a launch boundary less for the GPU) up to the bytes that held stores gain more with:
+    // 2 / 4 / 8 MiB 11.4 / 11.5 / 11.9 us with a signal launch, 9.5 / 9.6 / 10.8 so, 16 MiB 13.9 / 14.6; K and V blocks of 1.8 / 3.7 MB 11.5 /
+    // 12.0 and 10.3 / 10.8, of 8 MB 12.1 and 12.8.  From the host written-through stores cost more than the
     // launch they save beyond kDoneFromHostBytes (1 MiB 33.1 us, 30.2 with a signal launch; 256 KiB 14.2 either way).
-    constexpr uint64_t kDoneBytes = 1ull << 20;
+    constexpr uint64_t kDoneBytes = 4ull << 20;
+    constexpr uint64_t kDoneSingleBytes = 8ull << 20;
     constexpr uint64_t kDoneFromHostBytes = 128ull << 10;
-    const uint64_t most = route == MFRT_ROUTE_TO_HOST ? ~0ull : route == MFRT_ROUTE_HBM ? kDoneBytes : kDoneFromHostBytes;
+    const uint64_t most = route == MFRT_ROUTE_TO_HOST ? ~0ull
+                          : route != MFRT_ROUTE_HBM   ? kDoneFromHostBytes
+                          : n == 1                    ? kDoneSingleBytes
+                                                      : kDoneBytes;
     InlinePlan plan;
     if (n > kInlineSegs || bytes == 0 || bytes > most || tuning_.unitsOverride != 0 || !Started() || mfrt_bind_thread() != 0 ||
         !BuildInlineDirect(src, dst, len, n, kDeepUnits, plan)) {

@@ -474,16 +474,23 @@ __global__ void XcopySignalKernel(uint64_t mask, uint32_t maskValue)
 
 // A short blocking copy that says itself when it is done.  It is bound by the chain of launch, kernel and the word's way to the host;
 // a signal launch behind the copy adds a launch to the host's side and a launch boundary to the GPU's.  Blocking calls with the
-// signal launch / with this kernel: 16 KiB in HBM 10.5 / 8.4 us, 1 MiB 10.7 / 9.5, 122 blocks of 8 KiB 11.9 / 10.6, 32 x 4 KiB to the
+// signal launch / with this kernel: 16 KiB in HBM 10.5 / 8.4 us, 2 MiB 11.4 / 9.5, 122 blocks of 8 KiB 11.9 / 10.6, 32 x 4 KiB to the
 // host 12.2 / 11.0.  Workgroups of 16 KiB (four 128-bit accesses per lane of four waves): every workgroup beyond the first
-// costs an atomic on one word, so 4 KiB ones lose at 1 MiB (11.6) and the form as a whole at 4 MiB (11.0 / 11.5); 64 KiB in one
-// workgroup of sixteen waves gain nothing in HBM (8.9 / 8.9) and lose over the link (from the host 12.5 / 10.6).
+// costs an atomic, and those on one word wait for each other, so many workgroups count in two steps (4 MiB: 11.5 with all on one
+// word, as much as the signal launch, so 9.6); 64 KiB in one workgroup of sixteen waves gain nothing in HBM (8.9 / 8.9) and lose
+// over the link (from the host 12.5 / 10.6).
 struct DoneMark {
     uint64_t *word;         // pinned host memory, polled by the caller
-    uint32_t *counter;      // device memory, 0 between launches
+    uint32_t *counter;      // device memory of kDoneCounterBytes, 0 between launches
     uint32_t value;
     uint32_t groups;        // of the launch
 };
+
+// Counts the caller in; true for the last of `expect`, which leaves the counter at 0.
+__device__ __forceinline__ bool LastIn(uint32_t *counter, uint32_t expect)
+{
+    return atomicInc(counter, expect - 1) == expect - 1;
+}
 
 // Every store of the launch is written through (kStoreThrough), so it has reached memory once vmcnt says so, and the last
 // workgroup to count itself done may tell the host without waiting for the end of the kernel.
@@ -494,12 +501,16 @@ __device__ __forceinline__ void MarkDone(const DoneMark &mark)
     if (threadIdx.x != 0) {
         return;
     }
-    if (mark.groups > 1) {
-        if (__hip_atomic_fetch_add(mark.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != mark.groups - 1) {
+    uint32_t expect = mark.groups;
+    if (expect > kDoneFewGroups) {
+        const uint32_t sub = blockIdx.x % kDoneCounters;
+        if (!LastIn(mark.counter + (1 + sub) * kDoneCounterWords, (expect + kDoneCounters - 1 - sub) / kDoneCounters)) {
             return;
         }
-        __hip_atomic_store(mark.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        expect = kDoneCounters;
+    }
+    if (expect > 1 && !LastIn(mark.counter, expect)) {
+        return;
     }
     __hip_atomic_store(mark.word, static_cast<uint64_t>(mark.value), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }

@@ -123,6 +123,13 @@ inline uint32_t HoldNanosFor(uint32_t nchunk, uint32_t grid, uint32_t units, boo
     return 640 + kHoldKneeChunks * 6 / 10 + (nchunk - kHoldKneeChunks) * 33 / 100;
 }
 
+// Counters of the workgroups of a launch that says itself when it is done: one, and beyond kDoneFewGroups workgroups
+// kDoneCounters more, on lines of their own, in front of it.
+constexpr uint32_t kDoneFewGroups = 64;
+constexpr uint32_t kDoneCounters = 32;
+constexpr uint32_t kDoneCounterWords = 32;
+constexpr uint64_t kDoneCounterBytes = (1 + kDoneCounters) * kDoneCounterWords * sizeof(uint32_t);
+
 // On top of HoldNanosFor's rule where the waves of a launch have to look their descriptors up outside the kernel arguments, a
 // round trip across the host link before their loads, and the same on 16 KiB chunks: sixteen loads per lane take longer to leave.
 constexpr int32_t kHoldLookupExtraNanos = 1600;

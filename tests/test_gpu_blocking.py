@@ -1,5 +1,7 @@
 """Short blocking copies, which report their own end: what they moved is where it belongs when the call returns."""
 
+import threading
+
 import numpy as np
 import pytest
 
@@ -151,3 +153,46 @@ def test_long_batch_in_launches_that_planning_overlaps(lib, pool, count, most, l
     for s, d, n in zip(at, place, lens):
         expect[d:d + n] = data[s:s + n]
     assert np.array_equal(got, expect)
+
+
+@pytest.mark.parametrize("threads", [1, 3])
+def test_copies_whose_workgroups_count_in_two_steps(lib, pool, threads):
+    """65 workgroups and more, in turn with fewer, and batches, each thread with counters of its own: 1 MiB and 16 bytes, the last
+    sizes that report their own end and the first beyond."""
+    mib = 1 << 20
+    room = 9 * mib
+    handle = bm.create(2, 0, 2 * room * threads)
+    dev = handle.peer_rank_ptr(0, bm.BmMemType.DEVICE)
+    failures = []
+
+    def work(t):
+        try:
+            rng = np.random.default_rng(t)
+            source, target = dev + 2 * room * t, dev + 2 * room * t + room
+            data = rng.integers(0, 256, room, dtype=np.uint8)
+            assert lib.mfrt_memcpy(source, data.ctypes.data, room) == 0
+            for size in [mib, mib + 16, 4 * mib, 33, 8 * mib, 8 * mib + 1, 2 * mib - 5, mib + 1] * 2:
+                s, d = int(rng.integers(0, 200)), int(rng.integers(0, 200))
+                assert lib.mfrt_memset(target, 0xA5, size + 512) == 0
+                assert handle.copy_data(source + s, target + d, size, bm.BmCopyType.G2G) == 0, native.last_error()
+                got = _read(lib, target, size + 512)
+                assert np.array_equal(got[d:d + size], data[s:s + size]) and np.all(got[d + size:] == 0xA5), (size, s, d)
+            for count, each in [(128, 32768), (100, 41000), (2, 2 * mib), (2, 2 * mib + 8), (64, 16385)]:
+                assert lib.mfrt_memset(target, 0xA5, room) == 0
+                at = rng.permutation(count) * (each + 7)
+                to = rng.permutation(count) * (each + 9)
+                assert handle.copy_data_batch(source + at, target + to, np.full(count, each), count, bm.BmCopyType.G2G) == 0, native.last_error()
+                want = np.full(room, 0xA5, dtype=np.uint8)
+                for a, b in zip(at, to):
+                    want[b:b + each] = data[a:a + each]
+                assert np.array_equal(_read(lib, target, room), want), (count, each)
+        except Exception as e:  # noqa: BLE001 - reported by the test's own thread
+            failures.append(repr(e))
+
+    workers = [threading.Thread(target=work, args=(t,)) for t in range(threads)]
+    for w in workers:
+        w.start()
+    for w in workers:
+        w.join()
+    handle.destroy()
+    assert not failures, failures
