@@ -1366,13 +1366,12 @@ int XcopyEngine::LaunchDone(const uint64_t *src, const uint64_t *dst, const uint
     // 2 / 4 / 8 MiB 11.4 / 11.5 / 11.9 us with a signal launch, 9.5 / 9.6 / 10.8 so, 16 MiB 13.9 / 14.6; K and V blocks of 1.8 / 3.7 MB 11.5 /
     // 12.0 and 10.3 / 10.8, of 8 MB 12.1 and 12.8.  From the host written-through stores cost more than the
     // launch they save beyond kDoneFromHostBytes (1 MiB 33.1 us, 30.2 with a signal launch; 256 KiB 14.2 either way).
-    constexpr uint64_t kDoneBytes = 4ull << 20;
     constexpr uint64_t kDoneSingleBytes = 8ull << 20;
     constexpr uint64_t kDoneFromHostBytes = 128ull << 10;
     const uint64_t most = route == MFRT_ROUTE_TO_HOST ? ~0ull
                           : route != MFRT_ROUTE_HBM   ? kDoneFromHostBytes
                           : n == 1                    ? kDoneSingleBytes
-                                                      : kDoneBytes;
+                                                      : kDonePiecesBytes;
     InlinePlan plan;
     if (n > kInlineSegs || bytes == 0 || bytes > most || tuning_.unitsOverride != 0 || !Started() || mfrt_bind_thread() != 0 ||
         !BuildInlineDirect(src, dst, len, n, kDeepUnits, plan)) {
@@ -1385,6 +1384,31 @@ int XcopyEngine::LaunchDone(const uint64_t *src, const uint64_t *dst, const uint
     ticket = NextDoneSeq(lease);
     const uint32_t grid = GridFor(plan.nchunk, mfrt_cu_count(), route, tuning_);
     const int err = mfk_xcopy_done(&plan, route, grid, lease.doneWord, ticket, lease.doneCounter, stream);
+    if (err != 0) {
+        MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(err));
+    }
+    g_launches.fetch_add(1, std::memory_order_relaxed);
+    NotePending(stream, bytes);
+    return BM_OK;
+}
+
+// A batch of pieces that reports its own end.  Its slot is free again when it has, so no event guards it.
+int XcopyEngine::LaunchPiecesDone(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t bytes, int route,
+                                  void *stream, uint32_t &ticket)
+{
+    const uint64_t bound = PieceBound(bytes, n, kXcopyThreads);
+    if (route != MFRT_ROUTE_HBM || bytes == 0 || bytes > kDonePiecesBytes || n > kDonePiecesSegments || tuning_.unitsOverride != 0 || !Started() ||
+        mfrt_bind_thread() != 0 || mfrt_stream_capturing(stream) != 0) {
+        return kNotLaunched;
+    }
+    ThreadLease &lease = t_ctx.Lease();
+    StagingSlot *slot = nullptr;
+    if (lease.fanDirty != 0 || !HasDoneWord(lease) || !HasDoneCounter(lease) || AcquireSlot(lease, bound * sizeof(Piece), stream, slot) != BM_OK) {
+        return kNotLaunched;
+    }
+    const uint32_t count = BuildPieces(src, dst, len, n, kXcopyThreads, static_cast<Piece *>(slot->host));
+    ticket = NextDoneSeq(lease);
+    const int err = mfk_xcopy_pieces_done(slot->host, count, lease.doneWord, ticket, lease.doneCounter, stream);
     if (err != 0) {
         MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(err));
     }
@@ -1441,7 +1465,8 @@ int XcopyEngine::SubmitAndWait(const uint64_t *src, const uint64_t *dst, const u
         bytes += len[i];
     }
     uint32_t ticket = 0;
-    int ret = LaunchDone(src, dst, len, n, bytes, route, stream, ticket);
+    int ret = n <= kInlineSegs ? LaunchDone(src, dst, len, n, bytes, route, stream, ticket)
+                               : LaunchPiecesDone(src, dst, len, n, bytes, route, stream, ticket);
     if (ret == kNotLaunched) {
         ret = SubmitInSlices(src, dst, len, n, bytes, route, stream);
         return ret != BM_OK ? ret : WaitStream(stream, bytes, route);

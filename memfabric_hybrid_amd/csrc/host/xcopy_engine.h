@@ -61,6 +61,8 @@ constexpr uint64_t kPieceLongMinBytes = 4ull << 20;
 // Pieces in windows: below, too few periods pay for the halves of the first and the last one in which the chip only reads or only
 // writes (72 MB of K and V blocks 28.7 us without windows and 28.3 with them, 82 MB of pages 29.6 / 29.0, 90 MB of blocks 35.7 / 32.8).
 constexpr uint64_t kPieceWindowMinBytes = 80ull << 20;
+constexpr uint64_t kDonePiecesBytes = 4ull << 20; // blocking batches up to here report their own end,
+constexpr uint32_t kDonePiecesSegments = 2048;    // and up to so many segments: every piece counts itself done
 constexpr uint64_t kSliceMinNanos = 6000;         // planning that a blocking batch is not sliced for
 constexpr uint64_t kPieceListMin = 1ull << 18;     // pieces that any batch may be cut into, 4 MiB of descriptors
 
@@ -234,6 +236,8 @@ private:
     static constexpr int kNotLaunched = 1;
     int LaunchDone(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t bytes, int route, void *stream,
                    uint32_t &ticket);
+    int LaunchPiecesDone(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t bytes, int route, void *stream,
+                         uint32_t &ticket);
     int SubmitPieces(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, const BatchStats &stats, uint32_t units,
                      void *stream, void *mask, uint32_t maskValue, bool unordered);
     int SubmitInSlices(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint64_t bytes, int route, void *stream);

@@ -494,7 +494,7 @@ __device__ __forceinline__ bool LastIn(uint32_t *counter, uint32_t expect)
 
 // Every store of the launch is written through (kStoreThrough), so it has reached memory once vmcnt says so, and the last
 // workgroup to count itself done may tell the host without waiting for the end of the kernel.
-__device__ __forceinline__ void MarkDone(const DoneMark &mark)
+__device__ __forceinline__ void MarkDone(const DoneMark &mark, uint32_t group = blockIdx.x)
 {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -503,7 +503,7 @@ __device__ __forceinline__ void MarkDone(const DoneMark &mark)
     }
     uint32_t expect = mark.groups;
     if (expect > kDoneFewGroups) {
-        const uint32_t sub = blockIdx.x % kDoneCounters;
+        const uint32_t sub = group % kDoneCounters;
         if (!LastIn(mark.counter + (1 + sub) * kDoneCounterWords, (expect + kDoneCounters - 1 - sub) / kDoneCounters)) {
             return;
         }
@@ -678,16 +678,9 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyTableKernel(const TablePla
 // single waves of 16 KiB, held, beyond; and without hold four waves of 16 KiB, or as many as the usual segment fills: 4096 pages of 32 KiB
 // gathered 45.8 / 49.4 / 46.4 us with 4 KiB waves / 16 KiB waves / four waves, scattered 49.9 / 51.4 / 49.2, and a quarter of the
 // descriptors for the host to write.
-template <uint32_t kLanes, uint32_t kUnits, bool kHold>
-__global__ __launch_bounds__(kLanes) void XcopyPieceKernel(uint64_t list, uint32_t count, uint32_t holdTicks)
+template <uint32_t kLanes, uint32_t kUnits, bool kHold, int kStore>
+__device__ __forceinline__ void CopyPiece(const Piece &p, uint64_t t0, uint32_t holdTicks)
 {
-    const Piece *const pieces = Buffer<const Piece>(list);
-    const uint64_t t0 = kHold ? wall_clock64() : 0;
-    const uint32_t at = PieceOf(blockIdx.x);
-    if (at >= count) {
-        return;
-    }
-    const Piece p = pieces[at];
     const uint64_t srcWord = Uniform(p.src);
     const uint64_t dstWord = Uniform(p.dst);
     const uint64_t src = srcWord & kPieceAddress;
@@ -709,7 +702,7 @@ __global__ __launch_bounds__(kLanes) void XcopyPieceKernel(uint64_t list, uint32
         }
 #pragma unroll
         for (uint32_t j = 0; j < kUnits; ++j) {
-            StoreUnit<kStoreStream>(d + (j * kLanes + tid) * kUnitBytes, v[j]);
+            StoreUnit<kStore>(d + (j * kLanes + tid) * kUnitBytes, v[j]);
         }
     } else if (apart == 0) {
 #pragma unroll
@@ -724,7 +717,7 @@ __global__ __launch_bounds__(kLanes) void XcopyPieceKernel(uint64_t list, uint32
 #pragma unroll
         for (uint32_t j = 0; j < kUnits; ++j) {
             if (j * kLanes + tid < body) {
-                StoreUnit<kStoreStream>(d + (j * kLanes + tid) * kUnitBytes, v[j]);
+                StoreUnit<kStore>(d + (j * kLanes + tid) * kUnitBytes, v[j]);
             }
         }
     } else if (body != 0) {
@@ -734,15 +727,41 @@ __global__ __launch_bounds__(kLanes) void XcopyPieceKernel(uint64_t list, uint32
         if (kHold) {
             HoldStores(t0, holdTicks);
         }
-        StoreApart<kStoreStream>(v, last, d, u0, body, apart);
+        StoreApart<kStore>(v, last, d, u0, body, apart);
     }
     if (tid < g.head) {
-        CopyByte<kStoreStream>(src + tid, dst + tid);
+        CopyByte<kStore>(src + tid, dst + tid);
     }
     if (tid < g.tail) {
         const uint64_t off = g.head + g.body * kUnitBytes + tid;
-        CopyByte<kStoreStream>(src + off, dst + off);
+        CopyByte<kStore>(src + off, dst + off);
     }
+}
+
+template <uint32_t kLanes, uint32_t kUnits, bool kHold>
+__global__ __launch_bounds__(kLanes) void XcopyPieceKernel(uint64_t list, uint32_t count, uint32_t holdTicks)
+{
+    const Piece *const pieces = Buffer<const Piece>(list);
+    const uint64_t t0 = kHold ? wall_clock64() : 0;
+    const uint32_t at = PieceOf(blockIdx.x);
+    if (at >= count) {
+        return;
+    }
+    CopyPiece<kLanes, kUnits, kHold, kStoreStream>(pieces[at], t0, holdTicks);
+}
+
+// A short blocking batch that says itself when it is done, as XcopySingleDoneKernel.  A blocking call with the signal launch / so, us:
+// 129 / 200 / 500 segments of 5000 bytes 14.0 / 15.2 / 19.7 and 12.5 / 13.4 / 17.0, 244 K and V blocks of 16 KiB 18.1 and 16.1, 200 of 16 000
+// bytes 17.0 and 13.8, 1000 ragged ones of up to 5000 bytes 23.6 and 22.8; 4000 of 2000 bytes 52.6 and 53.3, so not that many.
+__global__ __launch_bounds__(64) void XcopyPieceDoneKernel(uint64_t list, uint32_t count, uint64_t word, uint64_t counter, uint32_t value)
+{
+    const Piece *const pieces = Buffer<const Piece>(list);
+    const uint32_t at = PieceOf(blockIdx.x);
+    if (at >= count) {
+        return;
+    }
+    CopyPiece<64, kDepth, false, kStoreThrough>(pieces[at], 0, 0);
+    MarkDone(DoneMark{Buffer<uint64_t>(word), Buffer<uint32_t>(counter), value, count}, at);
 }
 
 // Pieces of kWindowUnits units in read and write windows, as XcopyWindowKernel walks chunks; every piece of the list begins on a
@@ -1622,6 +1641,17 @@ extern "C" int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t byt
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
+// The same of 4 KiB and their bytes beside; the last of them stores `value` in `word`.  counter: kDoneCounterBytes of device memory.
+extern "C" int mfk_xcopy_pieces_done(const void *pieces, uint32_t count, void *word, uint32_t value, void *counter, void *stream)
+{
+    using namespace mf;
+    if (pieces == nullptr || count == 0 || count > kPieceMaxCount || word == nullptr || counter == nullptr) {
+        return -1;
+    }
+    return Launch(XcopyPieceDoneKernel, (count + kPieceGroup - 1) / kPieceGroup * kPieceGroup, 64, 0, static_cast<hipStream_t>(stream), At(pieces),
+                  count, At(word), At(counter), value);
+}
+
 // The same pieces, of up to kWindowUnits units, in windows cut for windowMBps.
 extern "C" int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t windowMBps, void *mask, uint32_t maskValue,
                                          void *stream, void *event)
@@ -1741,6 +1771,7 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
                 (void)Launch(XcopyPieceKernel<128, 4, false>, 1, 128, 0, s, 0, 0u, 0u);
                 (void)Launch(XcopyPieceKernel<128, 4, true>, 1, 128, 0, s, 0, 0u, 0u);
                 (void)Launch(XcopyPieceKernel<256, 4, false>, 1, 256, 0, s, 0, 0u, 0u);
+                (void)Launch(XcopyPieceDoneKernel, 1, 64, 0, s, 0, 0u, 0, 0, 0u);
                 (void)Launch(XcopyPieceWindowKernel, 1, 64, 0, s, 0, 0u, 64u, NextWindowSeq(), 1u);
                 (void)Launch(XcopyPlannedKernel<1, kPlannedShortRun>, 1, 64, 64, s, 0, 0u, TablePace{});
                 (void)Launch(XcopyPlannedKernel<kPlannedWaves, kPlannedRun>, 1, 64 * kPlannedWaves, 64, s, 0, 0u, TablePace{});

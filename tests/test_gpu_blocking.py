@@ -177,7 +177,8 @@ def test_copies_whose_workgroups_count_in_two_steps(lib, pool, threads):
                 assert handle.copy_data(source + s, target + d, size, bm.BmCopyType.G2G) == 0, native.last_error()
                 got = _read(lib, target, size + 512)
                 assert np.array_equal(got[d:d + size], data[s:s + size]) and np.all(got[d + size:] == 0xA5), (size, s, d)
-            for count, each in [(128, 32768), (100, 41000), (2, 2 * mib), (2, 2 * mib + 8), (64, 16385)]:
+            for count, each in [(128, 32768), (100, 41000), (2, 2 * mib), (2, 2 * mib + 8), (64, 16385), (129, 32513), (129, 32514), (2048, 2000), (2049, 2000),
+                                (300, 4096), (700, 4099)]:
                 assert lib.mfrt_memset(target, 0xA5, room) == 0
                 at = rng.permutation(count) * (each + 7)
                 to = rng.permutation(count) * (each + 9)
