@@ -617,7 +617,9 @@ __global__ __launch_bounds__(64) void MoePermuteTileKernel(const u32x4 *__restri
 // elements at top-2 12.1 / 7.1, 4096 at top-2 14.8 / 18.6.  It ends where counting is the quicker (MoeDispatchCountKernel): at 4096 entries, and
 // at 16384 comparisons per part (2048 elements, dispatch and combine: 256 tokens at top-8 11.6 here and 12.0 there, 300 12.6 and 11.1;
 // 1000 at top-4 12.5 and 12.3).  Plain stores leave the rows in
-// the caches, where the experts' kernel finds them (dispatch and combine in turn, 512 tokens: 27.9 us, 29.5 with nontemporal stores).
+// the caches, where the experts' kernel finds them (dispatch and combine in turn, 256 tokens of 7168 elements: 15.1 us), and up to kQuickBytes
+// nontemporal ones do not wait for the launch's end: dispatch / both with plain stores and so, 8 tokens 4.4 / 7.0, 3.9 / 6.4, 64 5.1 / 9.9, 4.5 /
+// 9.2, 160 7.7 / 12.7, 6.5 / 12.1; 300 at top-2 4.5 / 8.6, 3.5 / 8.2, 500 5.5 / 10.2, 4.3 / 10.4.
 constexpr uint32_t kSmallThreads = 256;
 constexpr uint32_t kSmallHold = 2;                      // 128-bit pieces of the row per lane: a part is 512 units at most
 constexpr uint32_t kSmallEntries = 4096;                // the largest such call
@@ -632,7 +634,7 @@ __device__ __forceinline__ uint32_t SmallKey(int32_t id, uint32_t index, uint32_
     return static_cast<uint32_t>(id) < experts ? static_cast<uint32_t>(id) << 16 | index : 0xFFFFFFFFu;
 }
 
-template <uint32_t kSlots>
+template <uint32_t kSlots, int kMode>
 __global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(uint64_t x, uint64_t topkAt, uint32_t total, uint32_t topK,
                                                                         uint32_t experts, uint32_t unitsPerRow, uint32_t parts,
                                                                         uint32_t perPart, uint32_t groups, uint64_t out,
@@ -795,7 +797,7 @@ __global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(uint64_t
             for (uint32_t j = 0; j < kSmallHold; ++j) {
                 const uint32_t u = begin + j * kSmallThreads + threadIdx.x;
                 if (u < end) {
-                    RowStore<0>(dst + static_cast<uint64_t>(row) * unitsPerRow + u, v[j]);
+                    RowStore<kMode>(dst + static_cast<uint64_t>(row) * unitsPerRow + u, v[j]);
                 }
             }
         }
@@ -835,7 +837,7 @@ constexpr uint32_t CountLdsWords(uint32_t experts, uint32_t ownMost)
 }
 
 // The lines lie where the token rows and the stored rows together, in bytes, change what a store should do.
-// Up to kCountQuickBytes nontemporal stores: they are on their way at once, where plain ones wait in an XCD's L2 for the end of
+// Up to kQuickBytes nontemporal stores: they are on their way at once, where plain ones wait in an XCD's L2 for the end of
 // the launch (dispatch and combine in turn, 400 tokens of 2048 elements at top-8: 10.7 us, 11.4 with plain ones).  Beyond, plain
 // stores leave the rows in the last-level cache, where the next kernel finds them (1000 of 5120 at top-8: 31.2, 35.5 with
 // nontemporal ones; 1500 of 2048 21.8, 23.6).  From kCountNearBytes on nontemporal loads and twice as many of them ahead keep the token rows
@@ -845,7 +847,8 @@ constexpr uint32_t CountLdsWords(uint32_t experts, uint32_t ownMost)
 // What does not fit the last-level cache (256 MiB) goes to the tiles: 8192 of 2048 at top-8 57 us, 61 to 63 with this.  Below that
 // the tiles may be the quicker dispatch, but not the quicker pair: 2000 of 7168 at top-8 47.0 / 91.1, with this 51.1 / 80.0; 1500 37.5 / 70.6
 // and 39.1 / 61.3.  Rows that are not whole cache lines are always stored plainly: two waves share a line.
-constexpr uint64_t kCountQuickBytes = 24ull << 20;
+constexpr uint64_t kQuickBytes = 24ull << 20;            // also of the dispatch above
+constexpr uint64_t kQuickFewBytes = 16ull << 20;         // with up to two slots, whose next kernel reads the rows sooner
 constexpr uint64_t kCountNearBytes = 96ull << 20;
 constexpr uint64_t kCountDeepBytes = 150ull << 20;
 constexpr uint64_t kCountBytes = 256ull << 20;
@@ -1343,6 +1346,9 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
     const size_t histLds = static_cast<size_t>(kRankSlices) * experts * sizeof(uint32_t);
     const uint32_t upr = hidden / 8;
     const bool rows = x != nullptr && out != nullptr && hidden != 0;
+    const uint64_t moved = rows ? (static_cast<uint64_t>(tokens) + total) * upr * 16 : 0;
+    const bool lines = hidden % 64 == 0;                // rows of whole cache lines
+    const bool quick = lines && moved <= (topK <= 2 ? kQuickFewBytes : kQuickBytes);
     if (total <= kSmallEntries && total * topK <= kSmallCompares) {   // where the lines lie: see the kernel
         const uint32_t least = (upr + kSmallHold * kSmallThreads - 1) / (kSmallHold * kSmallThreads);
         const uint32_t most = (upr + 63) / 64;
@@ -1351,8 +1357,9 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
         const uint32_t perPart = rows ? ((upr + parts - 1) / parts + 7) / 8 * 8 : 0;   // whole cache lines
         parts = rows ? (upr + perPart - 1) / perPart : 1;
 #define MF_DISPATCH_SMALL(SLOTS)                                                                                       \
-    return Launch(MoeDispatchSmallKernel<SLOTS>, tokens * parts + 1, kSmallThreads, 0, s, At(x), At(topk), total, topK, experts, upr, parts, \
-                  perPart, tokens * parts + 1, At(out), At(counts), At(offsets), At(rowOf), At(srcOf), At(workspace))
+    return Launch(quick ? MoeDispatchSmallKernel<SLOTS, 1> : MoeDispatchSmallKernel<SLOTS, 0>, tokens * parts + 1, kSmallThreads, 0, s, At(x), \
+                  At(topk), total, topK, experts, upr, parts, perPart, tokens * parts + 1, At(out), At(counts), At(offsets), At(rowOf),          \
+                  At(srcOf), At(workspace))
         if (topK <= 2) {
             MF_DISPATCH_SMALL(2);
         } else if (topK <= 4) {
@@ -1364,7 +1371,6 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
         }
 #undef MF_DISPATCH_SMALL
     }
-    const uint64_t moved = rows ? (static_cast<uint64_t>(tokens) + total) * upr * 16 : 0;
     if (total <= kCountEntries && moved <= kCountBytes) {   // where the lines lie: see those
         const uint32_t cus = static_cast<uint32_t>(mfrt_cu_count() > 0 ? mfrt_cu_count() : 256);
         const uint32_t most = cus < kCountLeastGroups ? kCountLeastGroups : cus;
@@ -1373,8 +1379,7 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
 #define MF_DISPATCH_COUNT(AHEAD, MODE, NT)                                                                             \
     return Launch(MoeDispatchCountKernel<AHEAD, MODE, NT>, (tokens + perGroup - 1) / perGroup, kCountThreads, lds, s, rows ? At(x) : 0, \
                   At(topk), total, topK, experts, upr, perGroup, At(out), At(counts), At(offsets), At(rowOf), At(srcOf), At(workspace))
-        const bool lines = hidden % 64 == 0;
-        if (lines && (moved <= kCountQuickBytes || (topK <= 4 && moved > kCountDeepBytes))) {
+        if (quick || (lines && topK <= 4 && moved > kCountDeepBytes)) {
             MF_DISPATCH_COUNT(4, 1, false);
         } else if (moved <= kCountNearBytes) {
             MF_DISPATCH_COUNT(4, 0, false);

@@ -449,6 +449,7 @@ def test_rows_read_ahead_of_the_permute(gpu, oracle, T, H, K, E):
 
 
 @pytest.mark.parametrize("T,H,K,E", [
+    (185, 7168, 8, 256), (196, 7168, 8, 256), (383, 7168, 2, 8), (395, 7168, 2, 8),   # rows that its stores leave in the caches, or not
     (256, 72, 8, 256), (257, 72, 8, 256), (1025, 8, 16, 512),       # the last call whose tokens look at one another, the first that counts
     (1171, 24, 7, 65), (3073, 16, 3, 1), (2201, 1032, 2, 16),       # ids that end inside a vector; one expert; rows that end inside a wave
     (49152, 8, 1, 17), (49153, 8, 1, 17), (6145, 520, 8, 64),       # the last call that counts, and the first beyond
