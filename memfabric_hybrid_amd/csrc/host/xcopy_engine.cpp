@@ -27,9 +27,12 @@ std::atomic<uint64_t> g_launches{0};
 // kernel moves it to `dev` first.  The slot may be rewritten once an event recorded behind its
 // kernels has fired.  Recording an event costs the stream about 3 us, as much as the launch gap
 // it sits in, so one event guards kGuardEvery consecutive launches: a slot is Queued until that
-// event is recorded and Guarded (by the slot that owns the event) afterwards.
+// event is recorded and Guarded (by the slot that owns the event) afterwards.  A launch of pieces on the thread's
+// own stream needs none: the next one there says in a pinned word, when it starts, that this one has ended, and until then
+// its slot is Followed (batches of 129 to 1000 segments 0.8 to 1.1 us a launch less than with an event per four, which the stream
+// executes too: 168 K and V blocks 6.5 -> 5.5 us, 200 pages of 8 KiB 5.3 -> 4.7).
 struct StagingSlot {
-    enum State : uint8_t { kFree, kQueued, kGuarded };
+    enum State : uint8_t { kFree, kQueued, kGuarded, kFollowed };
     void *host = nullptr;
     void *dev = nullptr;
     void *rest = nullptr;       // RestList of device-resident tables, in device memory
@@ -38,6 +41,7 @@ struct StagingSlot {
     void *event = nullptr;
     State state = kFree;
     StagingSlot *guard = nullptr;
+    uint32_t startSeq = 0;      // of its launch, where it is Followed
 };
 
 // GPU resources of one calling thread: its stream, its staging slots, its bounce area.  They are
@@ -56,6 +60,7 @@ struct ThreadLease {
     bool adopted = false;           // taken over from a thread that ended: its queued kernels ran on streams unknown here
     uint64_t *doneWord = nullptr;   // pinned; a one-lane launch stores doneSeq there behind a blocking copy
     uint32_t doneSeq = 0;
+    uint32_t startSeq = 0;          // of the latest launch of pieces on `stream` that stores it in StartedWord() when it starts
     void *doneCounter = nullptr;    // device memory, for launches that store the word themselves
     void *graphRests = nullptr;     // kSlots RestLists for the device-table calls that become nodes of a graph: not those plain calls use
     uint32_t graphCursor = 0;
@@ -597,6 +602,42 @@ int MarkQueued(ThreadLease &ctx, StagingSlot *slot, void *stream, bool sealNow, 
     return sealNow || ctx.queued >= kGuardEvery ? SealQueued(ctx) : BM_OK;
 }
 
+// Behind the word of the blocking copies, which the GPU stores too.
+uint64_t *StartedWord(ThreadLease &lease)
+{
+    return lease.doneWord + 4;
+}
+
+// Waits until the kernel that reads a Followed slot has ended: until a later launch has started, in which the thread may sleep as long as
+// it likes, or, if there is none or none that starts, by an event.
+int AwaitFollower(ThreadLease &ctx, StagingSlot &slot)
+{
+    constexpr auto kSpin = std::chrono::microseconds(100);
+    constexpr auto kSleep = std::chrono::microseconds(20);
+    constexpr auto kMost = std::chrono::milliseconds(200);
+    if (ctx.startSeq != slot.startSeq) {
+        const auto from = std::chrono::steady_clock::now();
+        for (uint32_t polls = 1;; ++polls) {
+            const auto seen = static_cast<uint32_t>(__atomic_load_n(StartedWord(ctx), __ATOMIC_ACQUIRE));
+            if (static_cast<int32_t>(seen - slot.startSeq) > 0) {
+                return 0;
+            }
+            if ((polls & 63u) == 0) {
+                const auto waited = std::chrono::steady_clock::now() - from;
+                if (waited > kMost) {
+                    break;
+                }
+                if (waited > kSpin) {
+                    std::this_thread::sleep_for(kSleep);
+                    polls |= 62u;           // two looks, then the next sleep
+                }
+            }
+        }
+    }
+    const int err = mfrt_event_record(slot.event, ctx.stream);
+    return err != 0 ? err : mfrt_event_sync(slot.event);
+}
+
 // The next slot of the ring, free to be rewritten, with at least `bytes` of pinned host memory.  Not for launches that become nodes
 // of a graph: a replay would read what a later call has left in the slot, memory may not be allocated while a stream records, and
 // an event recorded there is none that anybody could wait for.
@@ -631,6 +672,13 @@ int AcquireSlot(ThreadLease &ctx, uint64_t bytes, void *stream, StagingSlot *&ou
         if (ret != BM_OK) {
             return ret;
         }
+    }
+    if (slot.state == StagingSlot::kFollowed) {
+        const int err = AwaitFollower(ctx, slot);
+        if (err != 0) {
+            MF_FAIL(BM_ERROR, "staging slot wait failed: " << mfrt_error_string(err));
+        }
+        slot.state = StagingSlot::kFree;
     }
     if (slot.state == StagingSlot::kGuarded) {
         StagingSlot *guard = slot.guard;
@@ -1308,6 +1356,7 @@ bool HasDoneWord(ThreadLease &lease)
         if (lease.doneWord != nullptr) {
             *lease.doneWord = 0;
             lease.doneSeq = 0;
+            *StartedWord(lease) = lease.startSeq;
         }
     }
     return lease.doneWord != nullptr;
@@ -2145,6 +2194,19 @@ int XcopyEngine::SubmitPieces(const uint64_t *src, const uint64_t *dst, const ui
     }
     void *event = EventOfLaunch(lease, *slot, stream);
     const uint32_t rate = PieceWindowRate(stats, dst, len, n, count, units, unordered);
+    if (stream == lease.stream && mask == nullptr && HasDoneWord(lease)) {
+        const uint32_t hold = rate != 0 ? 0 : HoldForPieces(stats, n, count, units, unordered);
+        const int failed = mfk_xcopy_pieces_followed(pieces, count, total, units, hold, rate, StartedWord(lease), lease.startSeq + 1, stream);
+        if (failed != 0) {
+            (void)MarkQueued(lease, slot, stream, true);
+            MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(failed));
+        }
+        slot->startSeq = ++lease.startSeq;
+        slot->state = StagingSlot::kFollowed;
+        g_launches.fetch_add(1, std::memory_order_relaxed);
+        NotePending(stream, total);
+        return BM_OK;
+    }
     const int err = rate != 0 ? mfk_xcopy_pieces_windowed(pieces, count, total, rate, mask, maskValue, stream, event)
                               : mfk_xcopy_pieces(pieces, count, total, units, mask, maskValue, stream, HoldForPieces(stats, n, count, units, unordered), event);
     if (err != 0) {

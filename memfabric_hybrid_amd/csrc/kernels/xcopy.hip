@@ -738,10 +738,20 @@ __device__ __forceinline__ void CopyPiece(const Piece &p, uint64_t t0, uint32_t 
     }
 }
 
+// A launch of a stream starts when those before it have ended, and has then no more use for what they have read: one that is
+// told a word in host memory says so there.
+__device__ __forceinline__ void MarkStarted(uint64_t started, uint32_t value)
+{
+    if (started != 0 && blockIdx.x == 0 && threadIdx.x == 0) {
+        __hip_atomic_store(Buffer<uint64_t>(started), static_cast<uint64_t>(value), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 template <uint32_t kLanes, uint32_t kUnits, bool kHold>
-__global__ __launch_bounds__(kLanes) void XcopyPieceKernel(uint64_t list, uint32_t count, uint32_t holdTicks)
+__global__ __launch_bounds__(kLanes) void XcopyPieceKernel(uint64_t list, uint32_t count, uint32_t holdTicks, uint32_t value, uint64_t started)
 {
     const Piece *const pieces = Buffer<const Piece>(list);
+    MarkStarted(started, value);
     const uint64_t t0 = kHold ? wall_clock64() : 0;
     const uint32_t at = PieceOf(blockIdx.x);
     if (at >= count) {
@@ -775,8 +785,10 @@ __global__ __launch_bounds__(64) void XcopyPieceDoneKernel(uint64_t list, uint32
 // (A schedule that stretches when sampled waves fall behind it was tried: it overshoots, 20 to 50 % slower than none.)
 // What a lane past the end of its piece loads is the last unit: a load under a condition would leave the registers of the
 // loop's last round alive in the others and take more of them than sixteen waves per CU have.
-__global__ __launch_bounds__(64) void XcopyPieceWindowKernel(uint64_t list, uint32_t count, uint32_t period, uint32_t seq, uint32_t groups)
+__global__ __launch_bounds__(64) void XcopyPieceWindowKernel(uint64_t list, uint32_t count, uint32_t period, uint32_t seq, uint32_t groups,
+                                                              uint32_t value, uint64_t started)
 {
+    MarkStarted(started, value);
     const Piece *const pieces = Buffer<const Piece>(list);
     uint32_t at = PieceOf(blockIdx.x);
     if (at >= count) {
@@ -1492,10 +1504,10 @@ int LaunchWithEvent(void (*kernel)(Params...), uint32_t grid, uint32_t lanes, hi
 }
 
 template <uint32_t kLanes, uint32_t kUnits, bool kHold>
-int LaunchPieces(const void *pieces, uint32_t count, uint32_t ticks, hipStream_t stream, hipEvent_t event)
+int LaunchPieces(const void *pieces, uint32_t count, uint32_t ticks, hipStream_t stream, hipEvent_t event, void *started, uint32_t value)
 {
     const uint32_t grid = (count + kPieceGroup - 1) / kPieceGroup * kPieceGroup;
-    return LaunchWithEvent(XcopyPieceKernel<kLanes, kUnits, kHold>, grid, kLanes, stream, event, At(pieces), count, ticks);
+    return LaunchWithEvent(XcopyPieceKernel<kLanes, kUnits, kHold>, grid, kLanes, stream, event, At(pieces), count, ticks, value, At(started));
 }
 
 template <bool kNtLoad, int kStore>
@@ -1612,40 +1624,68 @@ extern "C" int mfk_xcopy_signal(void *word, uint32_t value, void *stream)
     return mf::Signal(word, value, static_cast<hipStream_t>(stream));
 }
 
+namespace mf {
+namespace {
+
+bool IsList(const void *pieces, uint32_t count)
+{
+    return pieces != nullptr && count != 0 && count <= kPieceMaxCount;
+}
+
+// In the form that `units` and the hold ask for, or in windows of windowMBps where that is not 0.
+int SubmitPieceList(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, uint32_t holdNanos, uint32_t windowMBps, hipStream_t s,
+                    hipEvent_t end, void *started, uint32_t value)
+{
+    if (!IsList(pieces, count) || (units != 256 && units != 512 && units != 1024)) {
+        return -1;
+    }
+    if (windowMBps != 0) {
+        // whole groups of pieces, evenly over the rounds; the last group of the list may be short
+        const uint32_t grid = (WindowGrid(count, kWindowWaves) + kPieceGroup - 1) / kPieceGroup * kPieceGroup;
+        const uint32_t period = WindowPeriodTicks(2 * bytes * grid / (count > grid ? count : grid), windowMBps);
+        return period == 0 ? static_cast<int>(hipErrorInvalidValue)
+                           : LaunchWithEvent(XcopyPieceWindowKernel, grid, 64, s, end, At(pieces), count, period, NextWindowSeq(), grid, value,
+                                             At(started));
+    }
+    const uint32_t ticks = HoldTicks(PieceHoldNanos(holdNanos, count, bytes, units));
+    if (units == 256) {
+        return ticks != 0 ? LaunchPieces<64, 4, true>(pieces, count, ticks, s, end, started, value)
+                          : LaunchPieces<64, 4, false>(pieces, count, 0, s, end, started, value);
+    }
+    if (units == 512) {
+        return ticks != 0 ? LaunchPieces<128, 4, true>(pieces, count, ticks, s, end, started, value)
+                          : LaunchPieces<128, 4, false>(pieces, count, 0, s, end, started, value);
+    }
+    return ticks != 0 ? LaunchPieces<64, 16, true>(pieces, count, ticks, s, end, started, value)
+                      : LaunchPieces<256, 4, false>(pieces, count, 0, s, end, started, value);
+}
+
+}  // namespace
+}  // namespace mf
+
 // pieces: `count` mf::Piece of together `bytes` bytes, none longer than `units` units and the bytes beside them; holdNanos: what a
 // table of as many chunks would wait.
 extern "C" int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, void *mask, uint32_t maskValue,
                                 void *stream, uint32_t holdNanos, void *event)
 {
     using namespace mf;
-    if (pieces == nullptr || count == 0 || count > kPieceMaxCount || (units != 256 && units != 512 && units != 1024)) {
-        return -1;
-    }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const uint32_t ticks = HoldTicks(PieceHoldNanos(holdNanos, count, bytes, units));
-    const hipEvent_t end = static_cast<hipEvent_t>(event);
-    int err;
-    if (units == 256 && ticks != 0) {
-        err = LaunchPieces<64, 4, true>(pieces, count, ticks, s, end);
-    } else if (units == 256) {
-        err = LaunchPieces<64, 4, false>(pieces, count, 0, s, end);
-    } else if (units == 512 && ticks != 0) {
-        err = LaunchPieces<128, 4, true>(pieces, count, ticks, s, end);
-    } else if (units == 512) {
-        err = LaunchPieces<128, 4, false>(pieces, count, 0, s, end);
-    } else if (ticks != 0) {
-        err = LaunchPieces<64, 16, true>(pieces, count, ticks, s, end);
-    } else {
-        err = LaunchPieces<256, 4, false>(pieces, count, 0, s, end);
-    }
+    const int err = SubmitPieceList(pieces, count, bytes, units, holdNanos, 0, s, static_cast<hipEvent_t>(event), nullptr, 0);
     return err != 0 ? err : Signal(mask, maskValue, s);
+}
+
+// The same, in either form, with a word of pinned host memory that gets `value` when what is in front of them in the stream has ended.
+extern "C" int mfk_xcopy_pieces_followed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, uint32_t holdNanos,
+                                         uint32_t windowMBps, void *started, uint32_t value, void *stream)
+{
+    return mf::SubmitPieceList(pieces, count, bytes, units, holdNanos, windowMBps, static_cast<hipStream_t>(stream), nullptr, started, value);
 }
 
 // The same of 4 KiB and their bytes beside; the last of them stores `value` in `word`.  counter: kDoneCounterBytes of device memory.
 extern "C" int mfk_xcopy_pieces_done(const void *pieces, uint32_t count, void *word, uint32_t value, void *counter, void *stream)
 {
     using namespace mf;
-    if (pieces == nullptr || count == 0 || count > kPieceMaxCount || word == nullptr || counter == nullptr) {
+    if (!IsList(pieces, count) || word == nullptr || counter == nullptr) {
         return -1;
     }
     return Launch(XcopyPieceDoneKernel, (count + kPieceGroup - 1) / kPieceGroup * kPieceGroup, 64, 0, static_cast<hipStream_t>(stream), At(pieces),
@@ -1657,18 +1697,8 @@ extern "C" int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uin
                                          void *stream, void *event)
 {
     using namespace mf;
-    if (pieces == nullptr || count == 0 || count > kPieceMaxCount) {
-        return -1;
-    }
-    // whole groups of pieces, evenly over the rounds; the last group of the list may be short
-    const uint32_t grid = (WindowGrid(count, kWindowWaves) + kPieceGroup - 1) / kPieceGroup * kPieceGroup;
-    const uint32_t ticks = WindowPeriodTicks(2 * bytes * grid / (count > grid ? count : grid), windowMBps);
-    if (ticks == 0) {
-        return static_cast<int>(hipErrorInvalidValue);
-    }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int err = LaunchWithEvent(XcopyPieceWindowKernel, grid, 64, s, static_cast<hipEvent_t>(event), At(pieces), count, ticks,
-                                    NextWindowSeq(), grid);
+    const int err = windowMBps == 0 ? -1 : SubmitPieceList(pieces, count, bytes, kWindowUnits, 0, windowMBps, s, static_cast<hipEvent_t>(event), nullptr, 0);
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
@@ -1765,14 +1795,14 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
                 hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, empty, 1u);
                 hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 1u, 64u, 1u);
                 hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kWindowUnits, 1u, 64u, 1u);
-                (void)Launch(XcopyPieceKernel<64, 4, false>, 1, 64, 0, s, 0, 0u, 0u);
-                (void)Launch(XcopyPieceKernel<64, 4, true>, 1, 64, 0, s, 0, 0u, 0u);
-                (void)Launch(XcopyPieceKernel<64, 16, true>, 1, 64, 0, s, 0, 0u, 0u);
-                (void)Launch(XcopyPieceKernel<128, 4, false>, 1, 128, 0, s, 0, 0u, 0u);
-                (void)Launch(XcopyPieceKernel<128, 4, true>, 1, 128, 0, s, 0, 0u, 0u);
-                (void)Launch(XcopyPieceKernel<256, 4, false>, 1, 256, 0, s, 0, 0u, 0u);
+                (void)Launch(XcopyPieceKernel<64, 4, false>, 1, 64, 0, s, 0, 0u, 0u, 0u, 0);
+                (void)Launch(XcopyPieceKernel<64, 4, true>, 1, 64, 0, s, 0, 0u, 0u, 0u, 0);
+                (void)Launch(XcopyPieceKernel<64, 16, true>, 1, 64, 0, s, 0, 0u, 0u, 0u, 0);
+                (void)Launch(XcopyPieceKernel<128, 4, false>, 1, 128, 0, s, 0, 0u, 0u, 0u, 0);
+                (void)Launch(XcopyPieceKernel<128, 4, true>, 1, 128, 0, s, 0, 0u, 0u, 0u, 0);
+                (void)Launch(XcopyPieceKernel<256, 4, false>, 1, 256, 0, s, 0, 0u, 0u, 0u, 0);
                 (void)Launch(XcopyPieceDoneKernel, 1, 64, 0, s, 0, 0u, 0, 0, 0u);
-                (void)Launch(XcopyPieceWindowKernel, 1, 64, 0, s, 0, 0u, 64u, NextWindowSeq(), 1u);
+                (void)Launch(XcopyPieceWindowKernel, 1, 64, 0, s, 0, 0u, 64u, NextWindowSeq(), 1u, 0u, 0);
                 (void)Launch(XcopyPlannedKernel<1, kPlannedShortRun>, 1, 64, 64, s, 0, 0u, TablePace{});
                 (void)Launch(XcopyPlannedKernel<kPlannedWaves, kPlannedRun>, 1, 64 * kPlannedWaves, 64, s, 0, 0u, TablePace{});
                 hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());

@@ -69,3 +69,39 @@ def test_batch_in_pieces(gpu, oracle, kind, odd):
         b.free()
     gpu_util.oracle_batch(oracle, source, before, src, dst, lens)
     assert np.array_equal(got, before)
+
+
+@pytest.mark.parametrize("each", [512, 40000])
+@pytest.mark.parametrize("order", ["own", "own and a caller's", "own, blocking between", "own, a long copy in front"])
+def test_slots_whose_followers_say_that_they_are_free(gpu, order, each):
+    """More batches in flight than there are slots, none of them waited for: what each was told must stay in its slot until it has run."""
+    rng = np.random.default_rng(each)
+    batches, n = 40, 260
+    room = n * (each + 64)
+    a, b = gpu_util.DeviceBuffer(gpu, room), gpu_util.DeviceBuffer(gpu, batches * room)
+    long_from, long_to = gpu_util.DeviceBuffer(gpu, 256 << 20), gpu_util.DeviceBuffer(gpu, 256 << 20)
+    other = gpu.mfrt_stream_create()
+    try:
+        data = rng.integers(0, 256, room, dtype=np.uint8)
+        a.upload(data)
+        b.fill(0xA5)
+        want = np.full(batches * room, 0xA5, dtype=np.uint8)
+        if order == "own, a long copy in front":
+            for _ in range(20):
+                gpu_util.xcopy(gpu, [long_from.ptr], [long_to.ptr], [256 << 20], native.ROUTE_HBM, sync=False)
+        for k in range(batches):
+            lens = rng.integers(1, each, n).astype(np.uint64)
+            src = rng.integers(0, room - each, n).astype(np.uint64)
+            dst = rng.permutation(n).astype(np.uint64) * np.uint64(each + 64) + np.uint64(k * room)
+            for s, d, l in zip(src.tolist(), dst.tolist(), lens.tolist()):
+                want[d:d + l] = data[s:s + l]
+            stream = other if order == "own and a caller's" and k % 5 > 2 else None
+            gpu_util.xcopy(gpu, a.ptr + src, b.ptr + dst, lens, native.ROUTE_HBM, stream, sync=False)
+            if order == "own, blocking between" and k % 9 == 4:
+                assert gpu.mfrt_stream_sync(gpu.mf_xcopy_thread_stream()) == 0
+        assert gpu.mfrt_device_sync() == 0
+        assert np.array_equal(b.download(), want)
+    finally:
+        gpu.mfrt_stream_destroy(other)
+        for buffer in (a, b, long_from, long_to):
+            buffer.free()
