@@ -30,9 +30,11 @@ std::atomic<uint64_t> g_launches{0};
 // event is recorded and Guarded (by the slot that owns the event) afterwards.  A launch of pieces on the thread's
 // own stream needs none: the next one there says in a pinned word, when it starts, that this one has ended, and until then
 // its slot is Followed (batches of 129 to 1000 segments 0.8 to 1.1 us a launch less than with an event per four, which the stream
-// executes too: 168 K and V blocks 6.5 -> 5.5 us, 200 pages of 8 KiB 5.3 -> 4.7).
+// executes too: 168 K and V blocks 6.5 -> 5.5 us, 200 pages of 8 KiB 5.3 -> 4.7).  On a caller's stream, which may be gone before
+// there is a next one, the launch itself says in a word of the slot when every wave has read its piece (Reported), for an event of
+// its own costs 2.7 us of the host (129 / 500 / 1000 ragged segments of up to 40 000 bytes 7.4 / 11.0 / 15.7 us, so 6.2 / 9.6 / 14.4).
 struct StagingSlot {
-    enum State : uint8_t { kFree, kQueued, kGuarded, kFollowed };
+    enum State : uint8_t { kFree, kQueued, kGuarded, kFollowed, kReported };
     void *host = nullptr;
     void *dev = nullptr;
     void *rest = nullptr;       // RestList of device-resident tables, in device memory
@@ -42,6 +44,7 @@ struct StagingSlot {
     State state = kFree;
     StagingSlot *guard = nullptr;
     uint32_t startSeq = 0;      // of its launch, where it is Followed
+    uint32_t readSeq = 0;       // of its latest launch that reports
 };
 
 // GPU resources of one calling thread: its stream, its staging slots, its bounce area.  They are
@@ -62,6 +65,8 @@ struct ThreadLease {
     uint32_t doneSeq = 0;
     uint32_t startSeq = 0;          // of the latest launch of pieces on `stream` that stores it in StartedWord() when it starts
     void *doneCounter = nullptr;    // device memory, for launches that store the word themselves
+    uint64_t *readWords = nullptr;  // pinned, a line for every slot,
+    void *readCounters = nullptr;   // and counters in device memory, for launches that report that they have read it
     void *graphRests = nullptr;     // kSlots RestLists for the device-table calls that become nodes of a graph: not those plain calls use
     uint32_t graphCursor = 0;
     uint64_t pendingBytes = 0;      // bytes of the copies queued on `stream` since the thread last waited for it
@@ -120,6 +125,14 @@ struct ThreadLease {
         if (doneCounter != nullptr) {
             (void)mfrt_free_device(doneCounter);
             doneCounter = nullptr;
+        }
+        if (readWords != nullptr) {
+            (void)mfrt_free_host(readWords);
+            readWords = nullptr;
+        }
+        if (readCounters != nullptr) {
+            (void)mfrt_free_device(readCounters);
+            readCounters = nullptr;
         }
         if (graphRests != nullptr) {
             (void)mfrt_free_device(graphRests);
@@ -608,31 +621,66 @@ uint64_t *StartedWord(ThreadLease &lease)
     return lease.doneWord + 4;
 }
 
-// Waits until the kernel that reads a Followed slot has ended: until a later launch has started, in which the thread may sleep as long as
-// it likes, or, if there is none or none that starts, by an event.
-int AwaitFollower(ThreadLease &ctx, StagingSlot &slot)
+constexpr uint32_t kReadWordStride = 8;     // 64-bit words
+
+bool HasReadMarks(ThreadLease &lease)
+{
+    if (lease.readWords == nullptr) {
+        lease.readWords = static_cast<uint64_t *>(mfrt_alloc_host(kSlots * kReadWordStride * sizeof(uint64_t)));
+        if (lease.readWords == nullptr) {
+            return false;
+        }
+        std::fill_n(lease.readWords, kSlots * kReadWordStride, 0);
+    }
+    if (lease.readCounters == nullptr) {
+        lease.readCounters = mfrt_alloc_device(kSlots * kDoneCounterBytes);
+        if (lease.readCounters != nullptr && mfrt_memset(lease.readCounters, 0, kSlots * kDoneCounterBytes) != 0) {
+            (void)mfrt_free_device(lease.readCounters);
+            lease.readCounters = nullptr;
+        }
+    }
+    return lease.readCounters != nullptr;
+}
+
+uint64_t *ReadWord(ThreadLease &lease, const StagingSlot &slot)
+{
+    return lease.readWords + (&slot - lease.slots) * kReadWordStride;
+}
+
+void *ReadCounter(ThreadLease &lease, const StagingSlot &slot)
+{
+    return static_cast<uint8_t *>(lease.readCounters) + (&slot - lease.slots) * kDoneCounterBytes;
+}
+
+// Polls a word until it has come to `value`; after a while the thread sleeps between looks, as long as it takes or for `most`.
+bool AwaitWord(const uint64_t *word, uint32_t value, std::chrono::milliseconds most)
 {
     constexpr auto kSpin = std::chrono::microseconds(100);
     constexpr auto kSleep = std::chrono::microseconds(20);
-    constexpr auto kMost = std::chrono::milliseconds(200);
-    if (ctx.startSeq != slot.startSeq) {
-        const auto from = std::chrono::steady_clock::now();
-        for (uint32_t polls = 1;; ++polls) {
-            const auto seen = static_cast<uint32_t>(__atomic_load_n(StartedWord(ctx), __ATOMIC_ACQUIRE));
-            if (static_cast<int32_t>(seen - slot.startSeq) > 0) {
-                return 0;
+    const auto from = std::chrono::steady_clock::now();
+    for (uint32_t polls = 1;; ++polls) {
+        if (static_cast<int32_t>(static_cast<uint32_t>(__atomic_load_n(word, __ATOMIC_ACQUIRE)) - value) >= 0) {
+            return true;
+        }
+        if ((polls & 63u) == 0) {
+            const auto waited = std::chrono::steady_clock::now() - from;
+            if (most.count() != 0 && waited > most) {
+                return false;
             }
-            if ((polls & 63u) == 0) {
-                const auto waited = std::chrono::steady_clock::now() - from;
-                if (waited > kMost) {
-                    break;
-                }
-                if (waited > kSpin) {
-                    std::this_thread::sleep_for(kSleep);
-                    polls |= 62u;           // two looks, then the next sleep
-                }
+            if (waited > kSpin) {
+                std::this_thread::sleep_for(kSleep);
+                polls |= 62u;           // two looks, then the next sleep
             }
         }
+    }
+}
+
+// Waits until the kernel that reads a Followed slot has ended: until a later launch has started or, if there is none or none that
+// starts, by an event.
+int AwaitFollower(ThreadLease &ctx, StagingSlot &slot)
+{
+    if (ctx.startSeq != slot.startSeq && AwaitWord(StartedWord(ctx), slot.startSeq + 1, std::chrono::milliseconds(200))) {
+        return 0;
     }
     const int err = mfrt_event_record(slot.event, ctx.stream);
     return err != 0 ? err : mfrt_event_sync(slot.event);
@@ -678,6 +726,10 @@ int AcquireSlot(ThreadLease &ctx, uint64_t bytes, void *stream, StagingSlot *&ou
         if (err != 0) {
             MF_FAIL(BM_ERROR, "staging slot wait failed: " << mfrt_error_string(err));
         }
+        slot.state = StagingSlot::kFree;
+    }
+    if (slot.state == StagingSlot::kReported) {
+        (void)AwaitWord(ReadWord(ctx, slot), slot.readSeq, std::chrono::milliseconds(0));
         slot.state = StagingSlot::kFree;
     }
     if (slot.state == StagingSlot::kGuarded) {
@@ -2192,23 +2244,30 @@ int XcopyEngine::SubmitPieces(const uint64_t *src, const uint64_t *dst, const ui
         (void)BuildInlinePlan(none, kXcopyThreads, empty);
         return mfk_xcopy_inline(&empty, MFRT_ROUTE_HBM, 1, mask, maskValue, stream, 0, 0) == 0 ? BM_OK : BM_ERROR;
     }
-    void *event = EventOfLaunch(lease, *slot, stream);
     const uint32_t rate = PieceWindowRate(stats, dst, len, n, count, units, unordered);
-    if (stream == lease.stream && mask == nullptr && HasDoneWord(lease)) {
-        const uint32_t hold = rate != 0 ? 0 : HoldForPieces(stats, n, count, units, unordered);
-        const int failed = mfk_xcopy_pieces_followed(pieces, count, total, units, hold, rate, StartedWord(lease), lease.startSeq + 1, stream);
+    const uint32_t hold = rate != 0 ? 0 : HoldForPieces(stats, n, count, units, unordered);
+    const bool own = stream == lease.stream;
+    // Reporting costs the GPU the atomics of every wave (200 x 128 KiB 9.9 us with an event, 10.4 so, 2000 x 40 000 34.0 / 37.4), the
+    // event costs the host: for batches that the GPU copies in less time than the host needs for the next (4 us and some ns a segment).
+    const bool reports = !own && rate == 0 && total <= kReportBytes + kReportSegmentBytes * n;
+    if (mask == nullptr && (own ? HasDoneWord(lease) : reports && HasReadMarks(lease))) {
+        const uint32_t seq = own ? lease.startSeq + 1 : slot->readSeq + 1;
+        const int failed = mfk_xcopy_pieces_reported(pieces, count, total, units, hold, rate, own ? StartedWord(lease) : ReadWord(lease, *slot), seq,
+                                                     own ? nullptr : ReadCounter(lease, *slot), stream);
         if (failed != 0) {
             (void)MarkQueued(lease, slot, stream, true);
             MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(failed));
         }
-        slot->startSeq = ++lease.startSeq;
-        slot->state = StagingSlot::kFollowed;
+        (own ? lease.startSeq : slot->readSeq) = seq;
+        slot->startSeq = own ? seq : 0;
+        slot->state = own ? StagingSlot::kFollowed : StagingSlot::kReported;
         g_launches.fetch_add(1, std::memory_order_relaxed);
         NotePending(stream, total);
         return BM_OK;
     }
+    void *event = EventOfLaunch(lease, *slot, stream);
     const int err = rate != 0 ? mfk_xcopy_pieces_windowed(pieces, count, total, rate, mask, maskValue, stream, event)
-                              : mfk_xcopy_pieces(pieces, count, total, units, mask, maskValue, stream, HoldForPieces(stats, n, count, units, unordered), event);
+                              : mfk_xcopy_pieces(pieces, count, total, units, mask, maskValue, stream, hold, event);
     if (err != 0) {
         (void)MarkQueued(lease, slot, stream, true);   // the launch may have gone out with only the word behind it failing
         MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(err));

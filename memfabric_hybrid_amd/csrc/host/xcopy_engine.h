@@ -63,6 +63,8 @@ constexpr uint64_t kPieceLongMinBytes = 4ull << 20;
 constexpr uint64_t kPieceWindowMinBytes = 80ull << 20;
 constexpr uint64_t kDonePiecesBytes = 4ull << 20; // blocking batches up to here report their own end,
 constexpr uint32_t kDonePiecesSegments = 2048;    // and up to so many segments: every piece counts itself done
+constexpr uint64_t kReportBytes = 12000000;       // launches on callers' streams up to here,
+constexpr uint64_t kReportSegmentBytes = 16000;    // and this much more per segment, report that their list has been read
 constexpr uint64_t kSliceMinNanos = 6000;         // planning that a blocking batch is not sliced for
 constexpr uint64_t kPieceListMin = 1ull << 18;     // pieces that any batch may be cut into, 4 MiB of descriptors
 

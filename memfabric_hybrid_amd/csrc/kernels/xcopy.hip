@@ -486,10 +486,31 @@ struct DoneMark {
     uint32_t groups;        // of the launch
 };
 
-// Counts the caller in; true for the last of `expect`, which leaves the counter at 0.
-__device__ __forceinline__ bool LastIn(uint32_t *counter, uint32_t expect)
+// Workgroup `group` of `groups` counts itself in, on its own of kDoneCounters lines where they are many.  Every counter is 0 again when
+// the last has come.
+__device__ __forceinline__ bool InTwoSteps(uint32_t groups)
 {
-    return atomicInc(counter, expect - 1) == expect - 1;
+    return groups > kDoneFewGroups;
+}
+
+__device__ __forceinline__ uint32_t ArrivalLimit(uint32_t groups, uint32_t group)
+{
+    return (InTwoSteps(groups) ? (groups + kDoneCounters - 1 - group % kDoneCounters) / kDoneCounters : groups) - 1;
+}
+
+__device__ __forceinline__ uint32_t Arrive(uint32_t *counter, uint32_t groups, uint32_t group)
+{
+    uint32_t *own = InTwoSteps(groups) ? counter + (1 + group % kDoneCounters) * kDoneCounterWords : counter;
+    return atomicInc(own, ArrivalLimit(groups, group));
+}
+
+// Whether it was the last of all; `seen` is what Arrive() returned.
+__device__ __forceinline__ bool LastArrival(uint32_t *counter, uint32_t groups, uint32_t group, uint32_t seen)
+{
+    if (seen != ArrivalLimit(groups, group)) {
+        return false;
+    }
+    return !InTwoSteps(groups) || atomicInc(counter, kDoneCounters - 1) == kDoneCounters - 1;
 }
 
 // Every store of the launch is written through (kStoreThrough), so it has reached memory once vmcnt says so, and the last
@@ -501,15 +522,7 @@ __device__ __forceinline__ void MarkDone(const DoneMark &mark, uint32_t group = 
     if (threadIdx.x != 0) {
         return;
     }
-    uint32_t expect = mark.groups;
-    if (expect > kDoneFewGroups) {
-        const uint32_t sub = group % kDoneCounters;
-        if (!LastIn(mark.counter + (1 + sub) * kDoneCounterWords, (expect + kDoneCounters - 1 - sub) / kDoneCounters)) {
-            return;
-        }
-        expect = kDoneCounters;
-    }
-    if (expect > 1 && !LastIn(mark.counter, expect)) {
+    if (mark.groups > 1 && !LastArrival(mark.counter, mark.groups, group, Arrive(mark.counter, mark.groups, group))) {
         return;
     }
     __hip_atomic_store(mark.word, static_cast<uint64_t>(mark.value), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -678,8 +691,9 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyTableKernel(const TablePla
 // single waves of 16 KiB, held, beyond; and without hold four waves of 16 KiB, or as many as the usual segment fills: 4096 pages of 32 KiB
 // gathered 45.8 / 49.4 / 46.4 us with 4 KiB waves / 16 KiB waves / four waves, scattered 49.9 / 51.4 / 49.2, and a quarter of the
 // descriptors for the host to write.
-template <uint32_t kLanes, uint32_t kUnits, bool kHold, int kStore>
-__device__ __forceinline__ void CopyPiece(const Piece &p, uint64_t t0, uint32_t holdTicks)
+// `meanwhile`: what is done while the loads are on their way.
+template <uint32_t kLanes, uint32_t kUnits, bool kHold, int kStore, class F>
+__device__ __forceinline__ void CopyPiece(const Piece &p, uint64_t t0, uint32_t holdTicks, F meanwhile)
 {
     const uint64_t srcWord = Uniform(p.src);
     const uint64_t dstWord = Uniform(p.dst);
@@ -697,6 +711,7 @@ __device__ __forceinline__ void CopyPiece(const Piece &p, uint64_t t0, uint32_t 
         for (uint32_t j = 0; j < kUnits; ++j) {
             v[j] = LoadAligned(s + (j * kLanes + tid) * kUnitBytes);
         }
+        meanwhile();
         if (kHold) {
             HoldStores(t0, holdTicks);
         }
@@ -711,6 +726,7 @@ __device__ __forceinline__ void CopyPiece(const Piece &p, uint64_t t0, uint32_t 
                 v[j] = LoadAligned(s + (j * kLanes + tid) * kUnitBytes);
             }
         }
+        meanwhile();
         if (kHold) {
             HoldStores(t0, holdTicks);
         }
@@ -724,10 +740,13 @@ __device__ __forceinline__ void CopyPiece(const Piece &p, uint64_t t0, uint32_t 
         u32x4 last;
         const uint32_t u0 = (tid >> 6) * kUnits * 64;
         LoadApart(v, last, s - apart, u0, body);
+        meanwhile();
         if (kHold) {
             HoldStores(t0, holdTicks);
         }
         StoreApart<kStore>(v, last, d, u0, body, apart);
+    } else {
+        meanwhile();
     }
     if (tid < g.head) {
         CopyByte<kStore>(src + tid, dst + tid);
@@ -747,17 +766,37 @@ __device__ __forceinline__ void MarkStarted(uint64_t started, uint32_t value)
     }
 }
 
+// `word` gets `value` when the launch starts or, with a counter, when every wave has its piece: the list is the host's again then.
+// The counting is done beside the loads.
 template <uint32_t kLanes, uint32_t kUnits, bool kHold>
-__global__ __launch_bounds__(kLanes) void XcopyPieceKernel(uint64_t list, uint32_t count, uint32_t holdTicks, uint32_t value, uint64_t started)
+__global__ __launch_bounds__(kLanes) void XcopyPieceKernel(uint64_t list, uint32_t count, uint32_t holdTicks, uint32_t value, uint64_t word,
+                                                           uint64_t counter)
 {
     const Piece *const pieces = Buffer<const Piece>(list);
-    MarkStarted(started, value);
     const uint64_t t0 = kHold ? wall_clock64() : 0;
     const uint32_t at = PieceOf(blockIdx.x);
+    if (counter == 0) {
+        MarkStarted(word, value);
+    }
     if (at >= count) {
         return;
     }
-    CopyPiece<kLanes, kUnits, kHold, kStoreStream>(pieces[at], t0, holdTicks);
+    const Piece p = pieces[at];
+    // every wave fetches the piece for itself
+    constexpr uint32_t kWaves = kLanes / 64;
+    const uint32_t waves = count * kWaves;
+    const uint32_t wave = at * kWaves + threadIdx.x / 64;
+    const bool counts = counter != 0 && threadIdx.x % 64 == 0;
+    uint32_t seen = 0;
+    if (counts) {
+        asm volatile("" : : "s"(Uniform(p.src)), "s"(Uniform(p.dst)));      // has arrived
+        seen = Arrive(Buffer<uint32_t>(counter), waves, wave);
+    }
+    CopyPiece<kLanes, kUnits, kHold, kStoreStream>(p, t0, holdTicks, [&] {
+        if (counts && LastArrival(Buffer<uint32_t>(counter), waves, wave, seen)) {
+            __hip_atomic_store(Buffer<uint64_t>(word), static_cast<uint64_t>(value), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    });
 }
 
 // A short blocking batch that says itself when it is done, as XcopySingleDoneKernel.  A blocking call with the signal launch / so, us:
@@ -770,7 +809,7 @@ __global__ __launch_bounds__(64) void XcopyPieceDoneKernel(uint64_t list, uint32
     if (at >= count) {
         return;
     }
-    CopyPiece<64, kDepth, false, kStoreThrough>(pieces[at], 0, 0);
+    CopyPiece<64, kDepth, false, kStoreThrough>(pieces[at], 0, 0, [] {});
     MarkDone(DoneMark{Buffer<uint64_t>(word), Buffer<uint32_t>(counter), value, count}, at);
 }
 
@@ -1504,10 +1543,11 @@ int LaunchWithEvent(void (*kernel)(Params...), uint32_t grid, uint32_t lanes, hi
 }
 
 template <uint32_t kLanes, uint32_t kUnits, bool kHold>
-int LaunchPieces(const void *pieces, uint32_t count, uint32_t ticks, hipStream_t stream, hipEvent_t event, void *started, uint32_t value)
+int LaunchPieces(const void *pieces, uint32_t count, uint32_t ticks, hipStream_t stream, hipEvent_t event, void *word, uint32_t value,
+                 void *counter)
 {
     const uint32_t grid = (count + kPieceGroup - 1) / kPieceGroup * kPieceGroup;
-    return LaunchWithEvent(XcopyPieceKernel<kLanes, kUnits, kHold>, grid, kLanes, stream, event, At(pieces), count, ticks, value, At(started));
+    return LaunchWithEvent(XcopyPieceKernel<kLanes, kUnits, kHold>, grid, kLanes, stream, event, At(pieces), count, ticks, value, At(word), At(counter));
 }
 
 template <bool kNtLoad, int kStore>
@@ -1634,7 +1674,7 @@ bool IsList(const void *pieces, uint32_t count)
 
 // In the form that `units` and the hold ask for, or in windows of windowMBps where that is not 0.
 int SubmitPieceList(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, uint32_t holdNanos, uint32_t windowMBps, hipStream_t s,
-                    hipEvent_t end, void *started, uint32_t value)
+                    hipEvent_t end, void *word, uint32_t value, void *counter)
 {
     if (!IsList(pieces, count) || (units != 256 && units != 512 && units != 1024)) {
         return -1;
@@ -1645,19 +1685,19 @@ int SubmitPieceList(const void *pieces, uint32_t count, uint64_t bytes, uint32_t
         const uint32_t period = WindowPeriodTicks(2 * bytes * grid / (count > grid ? count : grid), windowMBps);
         return period == 0 ? static_cast<int>(hipErrorInvalidValue)
                            : LaunchWithEvent(XcopyPieceWindowKernel, grid, 64, s, end, At(pieces), count, period, NextWindowSeq(), grid, value,
-                                             At(started));
+                                             At(word));
     }
     const uint32_t ticks = HoldTicks(PieceHoldNanos(holdNanos, count, bytes, units));
     if (units == 256) {
-        return ticks != 0 ? LaunchPieces<64, 4, true>(pieces, count, ticks, s, end, started, value)
-                          : LaunchPieces<64, 4, false>(pieces, count, 0, s, end, started, value);
+        return ticks != 0 ? LaunchPieces<64, 4, true>(pieces, count, ticks, s, end, word, value, counter)
+                          : LaunchPieces<64, 4, false>(pieces, count, 0, s, end, word, value, counter);
     }
     if (units == 512) {
-        return ticks != 0 ? LaunchPieces<128, 4, true>(pieces, count, ticks, s, end, started, value)
-                          : LaunchPieces<128, 4, false>(pieces, count, 0, s, end, started, value);
+        return ticks != 0 ? LaunchPieces<128, 4, true>(pieces, count, ticks, s, end, word, value, counter)
+                          : LaunchPieces<128, 4, false>(pieces, count, 0, s, end, word, value, counter);
     }
-    return ticks != 0 ? LaunchPieces<64, 16, true>(pieces, count, ticks, s, end, started, value)
-                      : LaunchPieces<256, 4, false>(pieces, count, 0, s, end, started, value);
+    return ticks != 0 ? LaunchPieces<64, 16, true>(pieces, count, ticks, s, end, word, value, counter)
+                      : LaunchPieces<256, 4, false>(pieces, count, 0, s, end, word, value, counter);
 }
 
 }  // namespace
@@ -1670,15 +1710,19 @@ extern "C" int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t byt
 {
     using namespace mf;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int err = SubmitPieceList(pieces, count, bytes, units, holdNanos, 0, s, static_cast<hipEvent_t>(event), nullptr, 0);
+    const int err = SubmitPieceList(pieces, count, bytes, units, holdNanos, 0, s, static_cast<hipEvent_t>(event), nullptr, 0, nullptr);
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
-// The same, in either form, with a word of pinned host memory that gets `value` when what is in front of them in the stream has ended.
-extern "C" int mfk_xcopy_pieces_followed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, uint32_t holdNanos,
-                                         uint32_t windowMBps, void *started, uint32_t value, void *stream)
+// The same, in either form, with a word of pinned host memory that gets `value`: when what is in front of them in the stream has ended
+// or, with a counter (kDoneCounterBytes of device memory, 0; not in windows), when they have been read.
+extern "C" int mfk_xcopy_pieces_reported(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, uint32_t holdNanos,
+                                         uint32_t windowMBps, void *word, uint32_t value, void *counter, void *stream)
 {
-    return mf::SubmitPieceList(pieces, count, bytes, units, holdNanos, windowMBps, static_cast<hipStream_t>(stream), nullptr, started, value);
+    if (word == nullptr || (counter != nullptr && windowMBps != 0)) {
+        return -1;
+    }
+    return mf::SubmitPieceList(pieces, count, bytes, units, holdNanos, windowMBps, static_cast<hipStream_t>(stream), nullptr, word, value, counter);
 }
 
 // The same of 4 KiB and their bytes beside; the last of them stores `value` in `word`.  counter: kDoneCounterBytes of device memory.
@@ -1698,7 +1742,7 @@ extern "C" int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uin
 {
     using namespace mf;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int err = windowMBps == 0 ? -1 : SubmitPieceList(pieces, count, bytes, kWindowUnits, 0, windowMBps, s, static_cast<hipEvent_t>(event), nullptr, 0);
+    const int err = windowMBps == 0 ? -1 : SubmitPieceList(pieces, count, bytes, kWindowUnits, 0, windowMBps, s, static_cast<hipEvent_t>(event), nullptr, 0, nullptr);
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
@@ -1795,12 +1839,12 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
                 hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, empty, 1u);
                 hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 1u, 64u, 1u);
                 hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kWindowUnits, 1u, 64u, 1u);
-                (void)Launch(XcopyPieceKernel<64, 4, false>, 1, 64, 0, s, 0, 0u, 0u, 0u, 0);
-                (void)Launch(XcopyPieceKernel<64, 4, true>, 1, 64, 0, s, 0, 0u, 0u, 0u, 0);
-                (void)Launch(XcopyPieceKernel<64, 16, true>, 1, 64, 0, s, 0, 0u, 0u, 0u, 0);
-                (void)Launch(XcopyPieceKernel<128, 4, false>, 1, 128, 0, s, 0, 0u, 0u, 0u, 0);
-                (void)Launch(XcopyPieceKernel<128, 4, true>, 1, 128, 0, s, 0, 0u, 0u, 0u, 0);
-                (void)Launch(XcopyPieceKernel<256, 4, false>, 1, 256, 0, s, 0, 0u, 0u, 0u, 0);
+                (void)Launch(XcopyPieceKernel<64, 4, false>, 1, 64, 0, s, 0, 0u, 0u, 0u, 0, 0);
+                (void)Launch(XcopyPieceKernel<64, 4, true>, 1, 64, 0, s, 0, 0u, 0u, 0u, 0, 0);
+                (void)Launch(XcopyPieceKernel<64, 16, true>, 1, 64, 0, s, 0, 0u, 0u, 0u, 0, 0);
+                (void)Launch(XcopyPieceKernel<128, 4, false>, 1, 128, 0, s, 0, 0u, 0u, 0u, 0, 0);
+                (void)Launch(XcopyPieceKernel<128, 4, true>, 1, 128, 0, s, 0, 0u, 0u, 0u, 0, 0);
+                (void)Launch(XcopyPieceKernel<256, 4, false>, 1, 256, 0, s, 0, 0u, 0u, 0u, 0, 0);
                 (void)Launch(XcopyPieceDoneKernel, 1, 64, 0, s, 0, 0u, 0, 0, 0u);
                 (void)Launch(XcopyPieceWindowKernel, 1, 64, 0, s, 0, 0u, 64u, NextWindowSeq(), 1u, 0u, 0);
                 (void)Launch(XcopyPlannedKernel<1, kPlannedShortRun>, 1, 64, 64, s, 0, 0u, TablePace{});

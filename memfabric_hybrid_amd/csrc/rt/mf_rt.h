@@ -102,8 +102,8 @@ int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_
                      uint32_t holdNanos, void *event);
 /* The same pieces, of up to mfk_xcopy_window_units() units, which all begin on cache lines in source and destination, in read and
  * write windows cut for `windowMBps` MB/s of HBM traffic. */
-int mfk_xcopy_pieces_followed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, uint32_t holdNanos, uint32_t windowMBps,
-                              void *started, uint32_t value, void *stream);
+int mfk_xcopy_pieces_reported(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, uint32_t holdNanos, uint32_t windowMBps,
+                              void *word, uint32_t value, void *counter, void *stream);
 int mfk_xcopy_pieces_done(const void *pieces, uint32_t count, void *word, uint32_t value, void *counter, void *stream);
 int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t windowMBps, void *mask, uint32_t maskValue,
                               void *stream, void *event);

@@ -454,15 +454,21 @@ int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uint64_t bytes
     return windowMBps == 0 ? -1 : mfk_xcopy_pieces(pieces, count, bytes, 1024, mask, maskValue, stream, 0, event);
 }
 
-// When this launch starts, those before it have ended.
-int mfk_xcopy_pieces_followed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, uint32_t holdNanos, uint32_t windowMBps,
-                              void *started, uint32_t value, void *stream)
+// When this launch starts, those before it have ended; with a counter its own list has been read when it says so.
+int mfk_xcopy_pieces_reported(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, uint32_t holdNanos, uint32_t windowMBps,
+                              void *word, uint32_t value, void *counter, void *stream)
 {
-    Retire(g_flightSeq);
+    if (counter == nullptr) {
+        Retire(g_flightSeq);
+    }
     const int err = windowMBps != 0 ? mfk_xcopy_pieces_windowed(pieces, count, bytes, windowMBps, nullptr, 0, stream, nullptr)
                                     : mfk_xcopy_pieces(pieces, count, bytes, units, nullptr, 0, stream, holdNanos, nullptr);
     if (err == 0) {
-        __atomic_store_n(static_cast<uint64_t *>(started), static_cast<uint64_t>(value), __ATOMIC_RELEASE);
+        if (counter != nullptr) {
+            std::lock_guard<std::mutex> guard(g_flightLock);
+            g_inFlight.pop_back();
+        }
+        __atomic_store_n(static_cast<uint64_t *>(word), static_cast<uint64_t>(value), __ATOMIC_RELEASE);
     }
     return err;
 }

@@ -72,7 +72,8 @@ def test_batch_in_pieces(gpu, oracle, kind, odd):
 
 
 @pytest.mark.parametrize("each", [512, 40000])
-@pytest.mark.parametrize("order", ["own", "own and a caller's", "own, blocking between", "own, a long copy in front"])
+@pytest.mark.parametrize("order", ["own", "a caller's", "own and a caller's", "own, blocking between", "own, a long copy in front",
+                                   "a caller's, a long copy in front"])
 def test_slots_whose_followers_say_that_they_are_free(gpu, order, each):
     """More batches in flight than there are slots, none of them waited for: what each was told must stay in its slot until it has run."""
     rng = np.random.default_rng(each)
@@ -86,16 +87,16 @@ def test_slots_whose_followers_say_that_they_are_free(gpu, order, each):
         a.upload(data)
         b.fill(0xA5)
         want = np.full(batches * room, 0xA5, dtype=np.uint8)
-        if order == "own, a long copy in front":
+        if order.endswith("a long copy in front"):
             for _ in range(20):
-                gpu_util.xcopy(gpu, [long_from.ptr], [long_to.ptr], [256 << 20], native.ROUTE_HBM, sync=False)
+                gpu_util.xcopy(gpu, [long_from.ptr], [long_to.ptr], [256 << 20], native.ROUTE_HBM, other if order[0] == "a" else None, sync=False)
         for k in range(batches):
             lens = rng.integers(1, each, n).astype(np.uint64)
             src = rng.integers(0, room - each, n).astype(np.uint64)
             dst = rng.permutation(n).astype(np.uint64) * np.uint64(each + 64) + np.uint64(k * room)
             for s, d, l in zip(src.tolist(), dst.tolist(), lens.tolist()):
                 want[d:d + l] = data[s:s + l]
-            stream = other if order == "own and a caller's" and k % 5 > 2 else None
+            stream = other if order.startswith("a caller's") or (order == "own and a caller's" and k % 5 > 2) else None
             gpu_util.xcopy(gpu, a.ptr + src, b.ptr + dst, lens, native.ROUTE_HBM, stream, sync=False)
             if order == "own, blocking between" and k % 9 == 4:
                 assert gpu.mfrt_stream_sync(gpu.mf_xcopy_thread_stream()) == 0
