@@ -612,8 +612,8 @@ __global__ __launch_bounds__(64) void MoePermuteTileKernel(const u32x4 *__restri
 // the comparison.  Nothing is exchanged between workgroups.
 // What bounds it: the chain of a launch and of its memory round trips (kernel arguments; the ids and the row, side by side; the
 // stores), not bytes, as long as the comparisons stay few: with all parts they grow with tokens * entries.  Dispatch
-// alone, with the rank launch and the permute launch / in one: 16 tokens of 7168 elements at top-8 over 256 experts 12.0 / 4.3 us,
-// 64: 12.3 / 4.9, 128: 13.6 / 6.1, 256: 15.3 / 9.3, 512 (4096 entries): 19.6 / 16.0, 1024: 31.8 / 35.0; 2000 tokens of 1024
+// alone, with the rank launch and the permute launch / in one (both with plain stores, see below): 16 tokens of 7168 elements at
+// top-8 over 256 experts 12.0 / 4.3 us, 64: 12.3 / 4.9, 128: 13.6 / 6.1, 256: 15.3 / 9.3, 512 (4096 entries): 19.6 / 16.0, 1024: 31.8 / 35.0; 2000 tokens of 1024
 // elements at top-2 12.1 / 7.1, 4096 at top-2 14.8 / 18.6.  It ends where counting is the quicker (MoeDispatchCountKernel): at 4096 entries, and
 // at 16384 comparisons per part (2048 elements, dispatch and combine: 256 tokens at top-8 11.6 here and 12.0 there, 300 12.6 and 11.1;
 // 1000 at top-4 12.5 and 12.3).  Plain stores leave the rows in

@@ -1131,8 +1131,8 @@ __device__ __forceinline__ bool PlannedQuad(const uint64_t *__restrict__ triples
 // every workgroup reads the lengths of all of it and has their chunk prefix in LDS after two sums over its lanes.  So it knows what a
 // host that could read the table would: the total, which chooses the form, and the owner of every chunk.  No list of long segments,
 // no second launch, no event.  Bound: the chain of launch, lengths, prefix, descriptor and first load (4 us) for short tables, HBM for
-// long ones.  With the two launches of XcopyDirectKernel / so, us: 64 pages of 8 KiB 9.2 / 4.6, 1000 9.7 / 6.1, 4096 17.2 / 15.2; 500 of
-// 32 KiB 11.6 / 8.0, 2000 29.8 / 24.9, 4096 scattered 55.7 / 50.6; 1952 K and V blocks 65.4 / 53.9; 1000 / 4000 ragged segments of up to
+// long ones.  With the two launches of XcopyDirectKernel / so, us: 64 pages of 8 KiB 9.2 / 3.8, 1000 9.7 / 6.6, 4096 17.7 / 15.5; 500 of
+// 32 KiB 11.7 / 8.0, 2000 29.7 / 25.2, 4096 scattered 55.6 / 50.3; 1952 K and V blocks 65.4 / 53.9; 1000 / 4000 ragged segments of up to
 // 70 000 bytes 24.0 / 16.6, 71.2 / 65.6; 300 of 2 MB 240 / 206.  Longer tables cost each workgroup more lanes' worth of lengths: with
 // kPlannedRun 16, 8000 pages of 8 KiB 28.3 / 30.9, 16 384 ragged of 14 000 bytes 60.3 / 68.9, and that much more code made all others
 // 1 to 3 us slower.  Looking four chunks ahead of a quad up while it loads: registers spill, 8000 pages of 8 KiB 33.3.
