@@ -407,8 +407,8 @@ def extras_block(lib, pool, dev, batches, tables, steps):
                       "frac_of_hbm_peak": frac(2 * group[0].payload / entry["us_per_call"] / 1e3, HBM_PEAK_GBPS)})
         multi[f"ragged_{count}_segments_{lo // 1000}_to_{hi // 1000}_KB"] = entry
     multi["note"] = ("asynchronous smem_bm_copy_batch calls back to back on one stream, 16 tables in turn, HIP events, median of 5 runs; more than "
-                     "128 segments take the table form (descriptors read from the pinned staging slot), up to 24 MiB in 4 KiB chunks and up "
-                     "to 64 MiB in 16 KiB chunks with the stores held back until the loads of the launch are out")
+                     "128 segments go out as pieces cut by the host (descriptors read from the pinned staging slot), of 16 KiB from 4 MiB on, up "
+                     "to 64 MiB with the stores held back until the loads of the launch are out")
     out["batches_of_several_requests"] = multi
 
     # ---- the grid the reference publishes for its transfer benchmark (example/trans/perf/README.md:61-70 there:
