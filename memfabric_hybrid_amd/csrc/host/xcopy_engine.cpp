@@ -2299,6 +2299,17 @@ int XcopyEngine::SubmitDeviceTable(const void *triples, uint32_t n, int route, v
         int err = mfk_xcopy_inline(&empty, route, 1, mask, maskValue, stream, 0, 0);
         return err == 0 ? BM_OK : BM_ERROR;
     }
+    // Calls that become nodes of a graph have lists of their own, for a graph may be replayed beside plain calls.  They are made by the
+    // thread's first plain call whichever way that goes: the recorded one may have more segments, or another thread may submit by then.
+    // (A call that needs no list goes out without room for them.)
+    ThreadLease &lease = t_ctx.Lease();
+    int ret = BM_OK;
+    if (lease.graphRests == nullptr && mfrt_stream_capturing(stream) == 0) {
+        ret = EnsureRestLists(lease.graphRests, kSlots, kRestGraphCapacity);
+        if (ret != BM_OK && ret != BM_MALLOC_FAILED) {
+            return ret;
+        }
+    }
     // Up to kPlannedSegments segments one launch plans and copies.  Where it may not pace itself for the whole chip, because other
     // threads submit too, only the shorter ones.
     uint32_t hold = 0;
@@ -2315,13 +2326,10 @@ int XcopyEngine::SubmitDeviceTable(const void *triples, uint32_t n, int route, v
         NotePending(stream, ~0ull);   // sizes unknown here: the next wait sleeps on the stream
         return BM_OK;
     }
-    // The list of long segments belongs to a slot: the next call of another stream gets another one.  Calls that become
-    // nodes of a graph have lists of their own, made by the thread's first call: a graph may be replayed beside plain calls.
-    ThreadCtx &ctx = t_ctx;
+    // The list of long segments belongs to a slot: the next call of another stream gets another one.
     StagingSlot *slot = nullptr;
-    ThreadLease &lease = ctx.Lease();
     const bool recorded = mfrt_stream_capturing(stream) != 0;
-    int ret = EnsureRestLists(lease.graphRests, kSlots, kRestGraphCapacity);
+    ret = ret == BM_OK ? EnsureRestLists(lease.graphRests, kSlots, kRestGraphCapacity) : ret;
     if (ret == BM_OK && !recorded) {
         ret = AcquireSlot(lease, 0, stream, slot);
         ret = ret == BM_OK ? EnsureRestLists(slot->rest, 1, kRestCapacity) : ret;

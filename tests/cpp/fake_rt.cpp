@@ -44,9 +44,14 @@ void NoteRecorded(const void *stream)
 }
 const void *g_lastRestList = nullptr;
 
+bool g_failAllocations = false;
+
 void *Track(uint64_t bytes, int kind)
 {
     NoteRecorded(g_capturing);
+    if (g_failAllocations) {
+        return nullptr;
+    }
     void *p = nullptr;
     if (posix_memalign(&p, 4096, bytes == 0 ? 4096 : bytes) != 0) {
         return nullptr;
@@ -142,6 +147,7 @@ static void Guard(const char *what)
 void fake_rt_capture(void *stream) { g_capturing = stream; }
 uint64_t fake_rt_capture_errors(void) { return g_captureErrors; }
 const void *fake_rt_last_rest_list(void) { return g_lastRestList; }
+void fake_rt_fail_allocations(int on) { g_failAllocations = on != 0; }
 uint64_t fake_rt_launches(void) { return g_launches; }
 uint32_t fake_rt_last_hold(void) { return g_lastHold; }
 uint32_t fake_rt_last_window(void) { const uint32_t w = g_lastWindow; g_lastWindow = 0; return w; }

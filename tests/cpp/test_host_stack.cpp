@@ -47,6 +47,7 @@ extern "C" uint64_t fake_rt_in_flight(void);
 extern "C" void fake_rt_capture(void *stream);
 extern "C" uint64_t fake_rt_capture_errors(void);
 extern "C" const void *fake_rt_last_rest_list(void);
+extern "C" void fake_rt_fail_allocations(int on);
 
 using namespace mf;
 using ock::mf::DataOperatorPtr;
@@ -1393,6 +1394,90 @@ static void TestRecordedCalls()
     hybm_uninit();
 }
 
+// A device table is captured after a plain call that took another of its routes: the lists of recorded calls are there all the same.
+static void TestRecordedTablesAfterPlainCallsOfAnotherRoute()
+{
+    const uint64_t bytes = 16ull << 20;
+    for (bool beside : {true, false}) {
+        CHECK(hybm_init(0, 0) == BM_OK);
+        auto *a = static_cast<uint8_t *>(mfrt_alloc_device(bytes));
+        auto *b = static_cast<uint8_t *>(mfrt_alloc_device(bytes));
+        const uint32_t most = kPlannedSegments + 900;
+        auto *table = static_cast<uint64_t *>(mfrt_alloc_device(24ull * most));
+        CHECK(a != nullptr && b != nullptr && table != nullptr);
+        std::vector<uint8_t> ref(bytes);
+        Fill(ref, 32);
+        std::memcpy(a, ref.data(), bytes);
+        std::memset(b, 0, bytes);
+        for (uint32_t i = 0; i < most; ++i) {
+            table[3 * i] = reinterpret_cast<uint64_t>(a) + i * 3000ull + 1;
+            table[3 * i + 1] = reinterpret_cast<uint64_t>(b) + i * 3000ull;
+            table[3 * i + 2] = 1 + i * 37 % 3000;
+        }
+        void *stream = mfrt_stream_create();
+        // in one launch, which has no list
+        const uint32_t warm = 64 * kPlannedShortRun + 500;
+        uint64_t before = fake_rt_launches();
+        CHECK(mf_xcopy_device_table(table, warm, MF_ROUTE_HBM, stream) == BM_OK);
+        CHECK(fake_rt_launches() - before == 1);
+        std::memset(b, 0, bytes);
+        std::atomic<int> stage{0};
+        std::thread second;
+        if (beside) {           // a second thread that copies: the same call now takes two launches
+            second = std::thread([&] {
+                CHECK(mf_xcopy_thread_stream() != nullptr);
+                stage = 1;
+                while (stage != 2) {
+                    std::this_thread::yield();
+                }
+            });
+            while (stage != 1) {
+                std::this_thread::yield();
+            }
+        }
+        const uint32_t n = beside ? warm : most;        // or the table has grown
+        const uint64_t errors = fake_rt_capture_errors();
+        before = fake_rt_launches();
+        fake_rt_capture(stream);
+        CHECK(mf_xcopy_device_table(table, n, MF_ROUTE_HBM, stream) == BM_OK);
+        fake_rt_capture(nullptr);
+        CHECK(fake_rt_launches() - before == 2);
+        CHECK(fake_rt_capture_errors() == errors);
+        bool same = true;
+        for (uint32_t i = 0; i < n; ++i) {
+            same = same && std::memcmp(reinterpret_cast<void *>(table[3 * i + 1]), reinterpret_cast<void *>(table[3 * i]), table[3 * i + 2]) == 0;
+        }
+        CHECK(same);
+        if (beside) {
+            stage = 2;
+            second.join();
+        }
+        CHECK(mfrt_device_sync() == 0);
+        mfrt_stream_destroy(stream);
+        mfrt_free_device(a);
+        mfrt_free_device(b);
+        mfrt_free_device(table);
+        hybm_uninit();
+    }
+    // without room for the lists a call that needs none goes out as before
+    CHECK(hybm_init(0, 0) == BM_OK);
+    uint64_t row[3];
+    auto *a = static_cast<uint8_t *>(mfrt_alloc_device(8192));
+    CHECK(a != nullptr);
+    std::memset(a, 7, 4096);
+    std::memset(a + 4096, 0, 4096);
+    row[0] = reinterpret_cast<uint64_t>(a);
+    row[1] = row[0] + 4096;
+    row[2] = 4096;
+    fake_rt_fail_allocations(1);
+    CHECK(mf_xcopy_device_table(row, 1, MF_ROUTE_HBM, nullptr) == BM_OK);
+    fake_rt_fail_allocations(0);
+    CHECK(std::memcmp(a, a + 4096, 4096) == 0);
+    CHECK(mfrt_device_sync() == 0);
+    mfrt_free_device(a);
+    hybm_uninit();
+}
+
 // The two-symbol plugin over the same engine: the completion word of a table the CPU can read is
 // stored before the call returns; a failed launch leaves the word alone and is counted.
 static void TestPlugin()
@@ -1828,6 +1913,7 @@ int main()
     TestHostCopy();
     TestSlotRing();
     TestRecordedCalls();
+    TestRecordedTablesAfterPlainCallsOfAnotherRoute();
     TestCApi();                                  // device window: reserved address space, HBM mapped in
     setenv("MF_HIP_GVA_WINDOW", "malloc", 1);
     TestCApi();                                  // device window: one ordinary allocation

@@ -2,6 +2,8 @@
 they point to: a batch must travel in the arguments, whatever its size, and a replay must not share the list of long
 segments with a plain call.  Every replay is compared with the oracle, after plain calls of other batches that go through
 all the library's descriptor slots."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -97,4 +99,61 @@ def test_captured_and_replayed_between_plain_calls(gpu, oracle, form, kind):
     finally:
         pool.free()
         other.free()
+        table.free()
+
+
+@pytest.mark.parametrize("change", ["a second thread copies", "the table grows"])
+def test_table_captured_after_a_plain_call_of_another_route(gpu, oracle, change):
+    """The plain call before the capture goes out in one launch, the captured one in two, which need a list."""
+    torch = pytest.importorskip("torch")
+    pool = gpu_util.DeviceBuffer(gpu, POOL)
+    src, dst, lens = _batch("20000 short", 3)
+    table = gpu_util.DeviceBuffer(gpu, 24 * len(lens))
+    stream = torch.cuda.Stream()
+    raw = stream.cuda_stream
+    warm = 1000
+    n = warm if change == "a second thread copies" else len(lens)
+    table.upload(np.stack([pool.ptr + src, pool.ptr + dst, lens], axis=1).astype(np.uint64).view(np.uint8).reshape(-1))
+    ready, done = threading.Event(), threading.Event()
+
+    def beside():
+        assert gpu.mf_xcopy_thread_stream()
+        ready.set()
+        done.wait(60)
+
+    second = threading.Thread(target=beside)
+    graph = torch.cuda.CUDAGraph()
+    try:
+        gpu.hybm_uninit()                                    # a thread that has no lists from calls before
+        assert gpu.hybm_init(0, 0) == 0, native.last_error()
+        launches = gpu.mf_xcopy_launch_count()
+        assert gpu.mf_xcopy_device_table(table.ptr, warm, native.ROUTE_HBM, raw) == 0, native.last_error()
+        assert gpu.mf_xcopy_launch_count() - launches == 1
+        torch.cuda.synchronize()
+        if change == "a second thread copies":
+            second.start()
+            assert ready.wait(60)
+        launches = gpu.mf_xcopy_launch_count()
+        with torch.cuda.graph(graph, stream=stream):
+            ret = gpu.mf_xcopy_device_table(table.ptr, n, native.ROUTE_HBM, raw)
+        assert ret == 0, native.last_error()
+        assert gpu.mf_xcopy_launch_count() - launches == (2 if n == warm else 4)
+        for replay in range(3):
+            init = np.empty(POOL, dtype=np.uint8)
+            oracle.orc_fill_random(init.ctypes.data, POOL, 800 + replay)
+            pool.upload(init)
+            assert gpu.mf_xcopy_device_table(table.ptr, n, native.ROUTE_HBM, raw) == 0, native.last_error()
+            torch.cuda.synchronize()
+            pool.upload(init)
+            graph.replay()
+            torch.cuda.synchronize()
+            expect = init.copy()
+            gpu_util.oracle_batch(oracle, init, expect, src[:n], dst[:n], lens[:n])
+            assert np.array_equal(pool.download(), expect), f"replay {replay} differs"
+    finally:
+        done.set()
+        if second.is_alive():
+            second.join()
+        del graph
+        pool.free()
         table.free()
