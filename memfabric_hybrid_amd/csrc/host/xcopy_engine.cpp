@@ -652,7 +652,7 @@ void *ReadCounter(ThreadLease &lease, const StagingSlot &slot)
     return static_cast<uint8_t *>(lease.readCounters) + (&slot - lease.slots) * kDoneCounterBytes;
 }
 
-// Polls a word until it has come to `value`; after a while the thread sleeps between looks, as long as it takes or for `most`.
+// Polls a word until it has come to `value`, for `most` at the longest; after a while the thread sleeps between looks.
 bool AwaitWord(const uint64_t *word, uint32_t value, std::chrono::milliseconds most)
 {
     constexpr auto kSpin = std::chrono::microseconds(100);
@@ -664,7 +664,7 @@ bool AwaitWord(const uint64_t *word, uint32_t value, std::chrono::milliseconds m
         }
         if ((polls & 63u) == 0) {
             const auto waited = std::chrono::steady_clock::now() - from;
-            if (most.count() != 0 && waited > most) {
+            if (waited > most) {
                 return false;
             }
             if (waited > kSpin) {
@@ -675,15 +675,30 @@ bool AwaitWord(const uint64_t *word, uint32_t value, std::chrono::milliseconds m
     }
 }
 
+constexpr auto kWordPatience = std::chrono::milliseconds(200);
+
 // Waits until the kernel that reads a Followed slot has ended: until a later launch has started or, if there is none or none that
 // starts, by an event.
 int AwaitFollower(ThreadLease &ctx, StagingSlot &slot)
 {
-    if (ctx.startSeq != slot.startSeq && AwaitWord(StartedWord(ctx), slot.startSeq + 1, std::chrono::milliseconds(200))) {
+    if (ctx.startSeq != slot.startSeq && AwaitWord(StartedWord(ctx), slot.startSeq + 1, kWordPatience)) {
         return 0;
     }
     const int err = mfrt_event_record(slot.event, ctx.stream);
     return err != 0 ? err : mfrt_event_sync(slot.event);
+}
+
+// Waits until the kernel that reads a Reported slot says that it has read it, however much work is queued in front of it.  A GPU that
+// has failed never gets there: it shows on `stream`, which the next launch goes to (the kernel's own may be gone).
+int AwaitReport(ThreadLease &ctx, const StagingSlot &slot, void *stream)
+{
+    while (!AwaitWord(ReadWord(ctx, slot), slot.readSeq, kWordPatience)) {
+        const int state = mfrt_stream_done(stream);
+        if (state < 0) {
+            return -state;
+        }
+    }
+    return 0;
 }
 
 // The next slot of the ring, free to be rewritten, with at least `bytes` of pinned host memory.  Not for launches that become nodes
@@ -729,7 +744,10 @@ int AcquireSlot(ThreadLease &ctx, uint64_t bytes, void *stream, StagingSlot *&ou
         slot.state = StagingSlot::kFree;
     }
     if (slot.state == StagingSlot::kReported) {
-        (void)AwaitWord(ReadWord(ctx, slot), slot.readSeq, std::chrono::milliseconds(0));
+        const int err = AwaitReport(ctx, slot, stream);
+        if (err != 0) {
+            MF_FAIL(BM_ERROR, "staging slot wait failed: " << mfrt_error_string(err));
+        }
         slot.state = StagingSlot::kFree;
     }
     if (slot.state == StagingSlot::kGuarded) {

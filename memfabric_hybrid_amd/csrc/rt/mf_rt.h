@@ -55,6 +55,7 @@ int mfrt_window_last_error(void);                       /* failed step (1 create
 void *mfrt_stream_create(void);
 int mfrt_stream_destroy(void *stream);
 int mfrt_stream_sync(void *stream);
+int mfrt_stream_done(void *stream);                     /* 1 nothing left to run, 0 pending, <0 error */
 int mfrt_stream_capturing(void *stream);                /* 1: launches on the stream become nodes of a HIP graph */
 int mfrt_device_sync(void);
 

@@ -276,6 +276,19 @@ extern "C" int mfrt_stream_sync(void *stream)
     return Code(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
 }
 
+extern "C" int mfrt_stream_done(void *stream)
+{
+    hipError_t err = hipStreamQuery(static_cast<hipStream_t>(stream));
+    if (err == hipSuccess) {
+        return 1;
+    }
+    if (err == hipErrorNotReady) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return -Code(err);
+}
+
 extern "C" int mfrt_stream_capturing(void *stream)
 {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;

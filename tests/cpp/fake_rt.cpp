@@ -147,6 +147,23 @@ static void Guard(const char *what)
 void fake_rt_capture(void *stream) { g_capturing = stream; }
 uint64_t fake_rt_capture_errors(void) { return g_captureErrors; }
 const void *fake_rt_last_rest_list(void) { return g_lastRestList; }
+// Launches that say when they have read their list do so from now on only at fake_rt_release_reports().
+static std::mutex g_reportLock;
+static bool g_withholdReports = false;
+static std::vector<std::pair<uint64_t *, uint64_t>> g_withheldReports;
+void fake_rt_withhold_reports(void) { g_withholdReports = true; }
+void fake_rt_release_reports(void)
+{
+    std::lock_guard<std::mutex> guard(g_reportLock);
+    g_withholdReports = false;
+    Retire(~0ull);
+    for (const auto &report : g_withheldReports) {
+        __atomic_store_n(report.first, report.second, __ATOMIC_RELEASE);
+    }
+    g_withheldReports.clear();
+}
+static std::atomic<int> g_streamState{1};
+void fake_rt_stream_state(int state) { g_streamState = state; }
 void fake_rt_fail_allocations(int on) { g_failAllocations = on != 0; }
 uint64_t fake_rt_launches(void) { return g_launches; }
 uint32_t fake_rt_last_hold(void) { return g_lastHold; }
@@ -258,6 +275,7 @@ uint64_t fake_rt_in_flight(void)
 extern "C" void fake_rt_count_stream_sync(void);
 int mfrt_stream_sync(void *) { Guard("mfrt_stream_sync"); Retire(~0ull); fake_rt_count_stream_sync(); return 0; }
 int mfrt_stream_capturing(void *stream) { return g_capturing != nullptr && stream == g_capturing ? 1 : 0; }
+int mfrt_stream_done(void *) { return g_streamState; }
 int mfrt_device_sync(void) { Guard("mfrt_device_sync"); Retire(~0ull); return 0; }
 void *mfrt_event_create(void) { return calloc(1, 8); }
 int mfrt_event_destroy(void *e) { Guard("mfrt_event_destroy"); free(e); return 0; }
@@ -469,6 +487,11 @@ int mfk_xcopy_pieces_reported(const void *pieces, uint32_t count, uint64_t bytes
     }
     const int err = windowMBps != 0 ? mfk_xcopy_pieces_windowed(pieces, count, bytes, windowMBps, nullptr, 0, stream, nullptr)
                                     : mfk_xcopy_pieces(pieces, count, bytes, units, nullptr, 0, stream, holdNanos, nullptr);
+    if (err == 0 && counter != nullptr && g_withholdReports) {
+        std::lock_guard<std::mutex> guard(g_reportLock);
+        g_withheldReports.emplace_back(static_cast<uint64_t *>(word), value);
+        return 0;
+    }
     if (err == 0) {
         if (counter != nullptr) {
             std::lock_guard<std::mutex> guard(g_flightLock);

@@ -9,6 +9,7 @@
 #include <cstring>
 #include <random>
 #include <atomic>
+#include <chrono>
 #include <thread>
 #include <vector>
 
@@ -48,6 +49,9 @@ extern "C" void fake_rt_capture(void *stream);
 extern "C" uint64_t fake_rt_capture_errors(void);
 extern "C" const void *fake_rt_last_rest_list(void);
 extern "C" void fake_rt_fail_allocations(int on);
+extern "C" void fake_rt_withhold_reports(void);
+extern "C" void fake_rt_release_reports(void);
+extern "C" void fake_rt_stream_state(int state);
 
 using namespace mf;
 using ock::mf::DataOperatorPtr;
@@ -1298,6 +1302,67 @@ static void TestSlotRing()
     hybm_uninit();
 }
 
+// A slot whose launch does not say that its list has been read: the call that needs it next fails when the GPU has, and waits otherwise.
+static void TestReportsThatDoNotCome()
+{
+    CHECK(hybm_init(0, 0) == BM_OK);
+    const uint32_t n = 200;
+    const uint64_t each = 4096;
+    auto *a = static_cast<uint8_t *>(mfrt_alloc_device(n * each));
+    auto *b = static_cast<uint8_t *>(mfrt_alloc_device(n * each));
+    CHECK(a != nullptr && b != nullptr);
+    std::vector<uint8_t> ref(n * each);
+    Fill(ref, 33);
+    std::memcpy(a, ref.data(), ref.size());
+    std::vector<uint64_t> s(n), d(n), l(n, each);
+    for (uint32_t i = 0; i < n; ++i) {
+        s[i] = reinterpret_cast<uint64_t>(a) + i * each;
+        d[i] = reinterpret_cast<uint64_t>(b) + (n - 1 - i) * each;
+    }
+    auto call = [&](void *stream) { return mf_xcopy_batch(s.data(), d.data(), l.data(), n, MF_ROUTE_HBM, stream); };
+    void *stream = mfrt_stream_create();
+    CHECK(call(stream) == BM_OK);
+    const uint64_t violations = fake_rt_violations();
+    fake_rt_withhold_reports();
+    uint32_t accepted = 0;
+    int32_t ret = BM_OK;
+    fake_rt_stream_state(-719);
+    for (; accepted < 64; ++accepted) {
+        ret = call(stream);
+        if (ret != BM_OK) {
+            break;
+        }
+    }
+    CHECK(ret == BM_ERROR && accepted >= 4 && accepted < 64);       // every slot of the ring once
+    for (int state : {0, 1}) {          // work pending; or none left, on a stream that need not be the launch's
+        fake_rt_withhold_reports();
+        fake_rt_stream_state(state);
+        std::memset(b, 0, n * each);
+        std::atomic<bool> released{false};
+        std::thread gpu([&] {
+            std::this_thread::sleep_for(std::chrono::milliseconds(500));
+            released = true;
+            fake_rt_release_reports();
+        });
+        for (uint32_t k = 0; k <= accepted; ++k) {
+            CHECK(call(stream) == BM_OK);
+        }
+        CHECK(released);
+        gpu.join();
+        bool same = true;
+        for (uint32_t i = 0; i < n; ++i) {
+            same = same && std::memcmp(reinterpret_cast<void *>(d[i]), reinterpret_cast<void *>(s[i]), each) == 0;
+        }
+        CHECK(same);
+    }
+    CHECK(mfrt_device_sync() == 0);
+    CHECK(fake_rt_violations() == violations);
+    mfrt_stream_destroy(stream);
+    mfrt_free_device(a);
+    mfrt_free_device(b);
+    hybm_uninit();
+}
+
 // Calls on a stream that records a graph: nothing they launch may read host memory that a later call rewrites, nothing may be
 // allocated and no event recorded; and plain calls afterwards find their slots as they left them.
 static void TestRecordedCalls()
@@ -1912,6 +1977,7 @@ int main()
     TestPlanners();
     TestHostCopy();
     TestSlotRing();
+    TestReportsThatDoNotCome();
     TestRecordedCalls();
     TestRecordedTablesAfterPlainCallsOfAnotherRoute();
     TestCApi();                                  // device window: reserved address space, HBM mapped in

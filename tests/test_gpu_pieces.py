@@ -1,5 +1,7 @@
 """Batches of more than 128 segments between HBM addresses: every way a source and a destination can differ modulo 16, lengths at
 the edges of the pieces they are cut into, and sizes that take each of the launch's shapes, with stores held and not."""
+import time
+
 import numpy as np
 import pytest
 
@@ -103,6 +105,47 @@ def test_slots_whose_followers_say_that_they_are_free(gpu, order, each):
         assert gpu.mfrt_device_sync() == 0
         assert np.array_equal(b.download(), want)
     finally:
+        gpu.mfrt_stream_destroy(other)
+        for buffer in (a, b, long_from, long_to):
+            buffer.free()
+
+
+@pytest.mark.parametrize("order", ["a caller's"])
+def test_slots_whose_launches_do_not_start_for_a_while(gpu, order):
+    """A third of a second of copies to the host in front: a call that needs a slot again looks for its word longer than it is polled for,
+    and where no launch follows on the own stream it waits for an event."""
+    rng = np.random.default_rng(len(order))
+    batches, n, each, long = 12, 260, 20000, 256 << 20
+    room = n * (each + 64)
+    a, b = gpu_util.DeviceBuffer(gpu, room), gpu_util.DeviceBuffer(gpu, batches * room)
+    long_from, long_to = gpu_util.DeviceBuffer(gpu, long), gpu_util.PinnedBuffer(gpu, long)
+    other = gpu.mfrt_stream_create()
+    try:
+        data = rng.integers(0, 256, room, dtype=np.uint8)
+        a.upload(data)
+        b.fill(0xA5)
+        want = np.full(batches * room, 0xA5, dtype=np.uint8)
+        plans = []
+        for k in range(batches):
+            lens = rng.integers(1, each, n).astype(np.uint64)
+            src = rng.integers(0, room - each, n).astype(np.uint64)
+            dst = rng.permutation(n).astype(np.uint64) * np.uint64(each + 64) + np.uint64(k * room)
+            for s, d, l in zip(src.tolist(), dst.tolist(), lens.tolist()):
+                want[d:d + l] = data[s:s + l]
+            plans.append([native.u64_array(v) for v in (a.ptr + src, b.ptr + dst, lens)])
+        assert gpu.mfrt_device_sync() == 0
+        first = other if order == "a caller's" else None
+        for _ in range(75):                                  # 4.7 ms each
+            gpu_util.xcopy(gpu, [long_from.ptr], [long_to.ptr], [long], native.ROUTE_TO_HOST, first, sync=False)
+        began = time.monotonic()
+        for k, plan in enumerate(plans):
+            stream = other if order == "a caller's" or (k > 0 and order != "own") else None
+            assert gpu.mf_xcopy_batch(*plan, n, native.ROUTE_HBM, stream) == 0, native.last_error()
+        assert time.monotonic() - began > 0.25
+        assert gpu.mfrt_device_sync() == 0
+        assert np.array_equal(b.download(), want)
+    finally:
+        gpu.mfrt_device_sync()
         gpu.mfrt_stream_destroy(other)
         for buffer in (a, b, long_from, long_to):
             buffer.free()
