@@ -110,7 +110,7 @@ def test_slots_whose_followers_say_that_they_are_free(gpu, order, each):
             buffer.free()
 
 
-@pytest.mark.parametrize("order", ["a caller's"])
+@pytest.mark.parametrize("order", ["a caller's", "own", "own, followed by a caller's"])
 def test_slots_whose_launches_do_not_start_for_a_while(gpu, order):
     """A third of a second of copies to the host in front: a call that needs a slot again looks for its word longer than it is polled for,
     and where no launch follows on the own stream it waits for an event."""
