@@ -1170,13 +1170,13 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
         const uint32_t seg = r * 64 * kWaves + threadIdx.x;
         len[r] = r < run ? triples[3ull * (seg < nseg ? seg : 0) + 2] : 0;
     }
-    uint64_t size = 0;          // of 256 bytes
+    uint32_t spare = 0;
 #pragma unroll
     for (uint32_t r = 0; r < kRun; ++r) {
         const uint32_t seg = r * 64 * kWaves + threadIdx.x;
         if (r < run && seg < nseg) {
             first[seg] = static_cast<uint32_t>((len[r] + 4095) >> 12);
-            size += len[r] >> 8;
+            spare += PlannedSpare(len[r]);
         }
     }
     __syncthreads();
@@ -1192,8 +1192,7 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
     }
     const uint32_t shallowUpTo = LanesUpTo(shallow);
     const uint32_t deepUpTo = LanesUpTo(deep);
-    // in 4 KiB, from lanes of up to 512 MiB
-    uint32_t total = __builtin_amdgcn_readlane(LanesUpTo(static_cast<uint32_t>(size < 1u << 21 ? size : 1u << 21)), 63) / 16;
+    uint32_t spareAll = __builtin_amdgcn_readlane(LanesUpTo(spare), 63);
     uint32_t shallowAll = __builtin_amdgcn_readlane(shallowUpTo, 63);
     uint32_t deepAll = __builtin_amdgcn_readlane(deepUpTo, 63);
     uint32_t shallowBase = 0;
@@ -1202,13 +1201,13 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
         if (lane == 0) {
             sums[wave] = shallowAll;
             sums[kWaves + wave] = deepAll;
-            sums[2 * kWaves + wave] = total;
+            sums[2 * kWaves + wave] = spareAll;
         }
         __syncthreads();
         const uint32_t at = lane < kWaves ? lane : 0;
         const uint32_t a = LanesUpTo(lane < kWaves ? sums[at] : 0);
         const uint32_t b = LanesUpTo(lane < kWaves ? sums[kWaves + at] : 0);
-        total = __builtin_amdgcn_readlane(LanesUpTo(lane < kWaves ? sums[2 * kWaves + at] : 0), 63);
+        spareAll = __builtin_amdgcn_readlane(LanesUpTo(lane < kWaves ? sums[2 * kWaves + at] : 0), 63);
         shallowBase = wave == 0 ? 0 : __builtin_amdgcn_readlane(a, wave == 0 ? 0 : wave - 1);
         deepBase = wave == 0 ? 0 : __builtin_amdgcn_readlane(b, wave == 0 ? 0 : wave - 1);
         shallowAll = __builtin_amdgcn_readlane(a, 63);
@@ -1217,7 +1216,8 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
     // The form: short tables a chunk of 4 KiB per wave; others 16 KiB, of one segment where those are nearly full or where a source and
     // its destination may differ modulo 16, else of up to four.
     const bool aligned = __ballot(bits % kUnitBytes != 0) == 0;
-    const bool full = static_cast<uint64_t>(total) * 100 >= static_cast<uint64_t>(deepAll) * (4 * kPlannedFullPercent);
+    const uint32_t total = PlannedTotal(deepAll, spareAll);
+    const bool full = PlannedFull(total, deepAll);
     const bool large = total > kPlannedShallowChunks;
     const bool quads = large && aligned && !full;
     const bool byDeep = large && !quads;
@@ -1239,8 +1239,7 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
     constexpr uint32_t grid = kWindowWaves;
     const uint32_t items = quads ? (nchunk + 3) / 4 : nchunk;
     const bool held = large && items <= grid && total <= kPlannedHeldChunks;
-    const bool paced = large && total > kPlannedHeldChunks && aligned && pace.windowTicks != 0 &&
-                       static_cast<uint64_t>(total) * 100 >= static_cast<uint64_t>(items) * (4 * kPlannedFullPercent);
+    const bool paced = large && total > kPlannedHeldChunks && aligned && pace.windowTicks != 0 && PlannedFull(total, items);
     const uint32_t rounds = (items + grid - 1) / grid;
     const uint32_t waves = paced ? (items + rounds - 1) / rounds : grid;
     uint32_t item = wave * kGroups + blockIdx.x;          // neighbouring ones on neighbouring XCDs

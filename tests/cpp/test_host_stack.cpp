@@ -736,6 +736,36 @@ static void TestMappedWindow()
 }
 
 // The one-pass planners must produce exactly what normalisation followed by planning produces.
+// The payload of a device table, as its launch sums it in 32 bits, is that of a 64-bit sum whatever the lengths are.
+static void TestPayloadOfPlannedTables()
+{
+    std::mt19937_64 rng(0x91ed);
+    const uint64_t lengths[] = {0, 1, 255, 256, 257, 4096, 16383, 16384, 16385, 100000, 260ull << 20, (512ull << 20) - 256, 512ull << 20,
+                                (512ull << 20) + 1, 1ull << 30, (4ull << 30) - 1, 4ull << 30, 17ull << 30};
+    for (uint32_t n : {1u, 3u, 16u, 64u, 65u, 512u, 4096u}) {
+        for (uint32_t kind = 0; kind <= std::size(lengths); ++kind) {
+            uint32_t deep = 0;
+            uint32_t spare = 0;
+            uint64_t exact = 0;
+            uint64_t pieces = 0;
+            for (uint32_t i = 0; i < n; ++i) {
+                const uint64_t len = kind < std::size(lengths) ? lengths[kind] : rng() % (2ull << 30) >> rng() % 31;
+                deep += static_cast<uint32_t>((len + 16383) / 16384);
+                spare += PlannedSpare(len);
+                exact += len >> 8;
+                pieces += (len + 16383) / 16384;
+            }
+            if (pieces >= 1ull << 30) {
+                continue;           // 16 TiB
+            }
+            const uint32_t total = PlannedTotal(deep, spare);
+            CHECK(total == exact / 16);
+            CHECK(PlannedFull(total, deep) == (exact / 16 * 100 >= pieces * 4 * kPlannedFullPercent));
+            CHECK(kind >= std::size(lengths) || lengths[kind] < (1u << 20) || PlannedFull(total, deep));
+        }
+    }
+}
+
 static void TestPlanners()
 {
     std::mt19937_64 rng(0x9142);
@@ -1975,6 +2005,7 @@ int main()
     SetLogSink([](int, const char *) {});
     TestCompose();
     TestPlanners();
+    TestPayloadOfPlannedTables();
     TestHostCopy();
     TestSlotRing();
     TestReportsThatDoNotCome();

@@ -85,7 +85,8 @@ def test_table_unlike_its_first_segments(gpu, oracle, kind, route, static):
         table.free()
 
 
-@pytest.mark.parametrize("count,size,static", [(3, (256 << 20) + 48, True), (20, (260 << 20) + 16, False), (20, (130 << 20) + 3, True)])
+@pytest.mark.parametrize("count,size,static", [(3, (256 << 20) + 48, True), (20, (260 << 20) + 16, False), (20, (130 << 20) + 3, True),
+                                               (3, (2 << 30) + 80, False)])
 def test_table_of_a_few_very_long_segments(gpu, count, size, static):
     """Gigabytes in a few segments, compared on the GPU."""
     torch = pytest.importorskip("torch")
