@@ -641,8 +641,8 @@ def extras_paged(lib):
         lib.mfrt_device_sync()
         lib.mfrt_free_device(tab)
         lib.mfrt_free_device(big)
-    table_path["note"] = ("device_table_*: mf_xcopy_device_table, the table copied without a plan and a second launch for what long segments hold "
-                          "beyond their share; ragged_16384: mf_xcopy_batch from host arrays (cut into pieces by the host) "
+    table_path["note"] = ("device_table_*: mf_xcopy_device_table, up to 4096 segments planned and copied by one launch, more copied without a "
+                          "plan and with a second launch for what long segments hold beyond their share; ragged_16384: mf_xcopy_batch from host arrays (cut into pieces by the host) "
                           "and the same table resident in device memory")
     res["table_path"] = table_path
     lib.mfrt_free_device(pool)

@@ -67,8 +67,9 @@ int32_t mf_xcopy_batch(const uint64_t *src, const uint64_t *dst, const uint64_t 
                        void *stream);
 
 /* An enqueue of mf_xcopy_batch for a {src,dst,len} triple table that already lives in device memory.  Under
- * stream capture the call uses lists of its own (eight per thread, made by the thread's first plain call):
- * replays of two graphs that hold such a call must not run at the same time, replays beside plain calls may. */
+ * stream capture the call uses lists of its own (eight per thread, made by the thread's first plain call of this
+ * function or of the plugin with a table in device memory, whatever its size): replays of two graphs that hold
+ * such a call must not run at the same time, replays beside plain calls may. */
 int32_t mf_xcopy_device_table(const void *triples, uint32_t n, int32_t route, void *stream);
 
 /* No counterpart in the reference.  mf_xcopy_device_table for callers that cannot allocate: code

@@ -230,9 +230,9 @@ private:
     // Rate of the windows a list of `count` pieces of `units` units is copied in, 0: in none.
     uint32_t PieceWindowRate(const BatchStats &stats, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t count, uint32_t units,
                              bool unordered) const;
-    // Whether a batch of `bytes` in n segments is planned in chunks of kDeepUnits units, to hold the stores of 16 KiB per wave.
     // How a launch of a device table paces itself: the waits of its waves and the rate of its windows.
     void TablePaceFor(uint32_t &holdNanos, uint32_t &holdMoreNanos, uint32_t &windowMBps) const;
+    // Whether a batch of `bytes` in n segments is planned in chunks of kDeepUnits units, to hold the stores of 16 KiB per wave.
     bool DeepHoldApplies(uint64_t bytes, uint32_t n, int route, bool unordered) const;
     // A launch that stores the thread's word itself, where that is the faster form: kNotLaunched where it is not.
     static constexpr int kNotLaunched = 1;

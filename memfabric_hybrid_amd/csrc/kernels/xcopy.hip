@@ -443,9 +443,9 @@ __global__ __launch_bounds__(64) void XcopyWindowKernel(const InlinePlan p, uint
 }
 
 // A single segment needs no table: its three words travel as plain kernel arguments (28 bytes instead of
-// the 3080-byte plan), which is cheaper for the host to hand over and spares every wave the table fetch
-// (an 8 MiB copy: 13.7 instead of 15.4 us per blocking call).  From about 200 MiB on the table form is
-// 1 % faster, hence the limit.
+// the 3080-byte plan), which is cheaper for the host to hand over and spares every wave the table fetch (one copy behind the
+// other, us, against the same bytes as two halves in a table: 8 MiB 3.8 / 5.1, 24 MiB 8.0 / 9.0, 64 MiB 21.2 / 21.5; short ones that
+// are waited for take XcopySingleDoneKernel).  From about 200 MiB on the table form is 1 % faster, hence the limit.
 constexpr uint32_t kSingleMaxChunks = 49152;
 template <bool kNtLoad, int kStore, int kHold = kHoldNone>
 __global__ __launch_bounds__(kXcopyThreads) void XcopySingleKernel(uint64_t src, uint64_t dst, uint32_t len, uint32_t nchunk,

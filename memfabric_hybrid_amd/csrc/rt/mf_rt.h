@@ -63,10 +63,10 @@ void *mfrt_event_create(void);
 int mfrt_event_destroy(void *event);
 int mfrt_event_record(void *event, void *stream);
 int mfrt_event_sync(void *event);
-int mfrt_stream_wait_event(void *stream, void *event);
+int mfrt_stream_wait_event(void *stream, void *event);   /* work queued on `stream` afterwards waits for the event */
 /* 1: launches on the two (idle) streams run one after the other because the streams share a hardware queue; 0: they
  * run side by side; -1: not known.  About 50 us. */
-int mfrt_streams_share_queue(void *a, void *b);   /* work queued on `stream` afterwards waits for the event */
+int mfrt_streams_share_queue(void *a, void *b);
 int mfrt_event_done(void *event);       /* 1 finished, 0 pending, <0 error */
 float mfrt_event_elapsed_ms(void *start, void *stop);
 
@@ -101,11 +101,17 @@ int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, void *mask,
  * event (may be NULL): completes with the launch.  The stream must not be one that records a graph, whose launches cannot carry one. */
 int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, void *mask, uint32_t maskValue, void *stream,
                      uint32_t holdNanos, void *event);
-/* The same pieces, of up to mfk_xcopy_window_units() units, which all begin on cache lines in source and destination, in read and
- * write windows cut for `windowMBps` MB/s of HBM traffic. */
+/* The same pieces; the launch stores `value` into `word` (pinned host memory) once `pieces` may be rewritten.  Without a counter when
+ * it has started: the launches before it on `stream` have then ended, and theirs may be.  With one (kDoneCounterBytes of device memory,
+ * 0 between launches that follow one another) when every wave has its descriptor.  windowMBps != 0, which takes no counter: in
+ * windows, as mfk_xcopy_pieces_windowed. */
 int mfk_xcopy_pieces_reported(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, uint32_t holdNanos, uint32_t windowMBps,
                               void *word, uint32_t value, void *counter, void *stream);
+/* The same pieces, of 4 KiB each; the launch stores `value` into `word` once every byte is in memory.  `counter`: as for
+ * mfk_xcopy_done. */
 int mfk_xcopy_pieces_done(const void *pieces, uint32_t count, void *word, uint32_t value, void *counter, void *stream);
+/* The same pieces, of up to mfk_xcopy_window_units() units, which all begin on cache lines in source and destination, in read and
+ * write windows cut for `windowMBps` MB/s of HBM traffic. */
 int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t windowMBps, void *mask, uint32_t maskValue,
                               void *stream, void *event);
 /* Launches every copy kernel once on empty plans (a kernel's first launch is not capturable into a HIP graph). */

@@ -460,11 +460,12 @@ int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_
     return 0;
 }
 
-// The same in windows: the rate is noted, and a piece that begins between cache lines fails the launch.
+// The same with a word for the end of the copy.
 int mfk_xcopy_pieces_done(const void *pieces, uint32_t count, void *word, uint32_t value, void *counter, void *stream)
 {
     return counter == nullptr || word == nullptr ? -1 : mfk_xcopy_pieces(pieces, count, 0, 256, word, value, stream, 0, nullptr);
 }
+// The same in windows: the rate is noted, and a piece that begins between cache lines fails the launch.
 int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t windowMBps, void *mask, uint32_t maskValue,
                               void *stream, void *event)
 {
