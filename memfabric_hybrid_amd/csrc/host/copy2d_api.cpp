@@ -22,6 +22,116 @@ bool Aligned16(const mf_copy2d_desc &d)
     return RectFitsPlan(d.src, d.dst, d.width, d.height, d.spitch, d.dpitch);
 }
 
+// Rows of whole cache lines.
+bool OnLines(const mf_copy2d_desc &d)
+{
+    return ((d.src | d.dst | d.width | d.spitch | d.dpitch) & (kWindowAlignBytes - 1)) == 0;
+}
+
+// Two rectangles that are one entry of a RectChunkPlan.
+bool RectsPair(const mf_copy2d_desc &a, const mf_copy2d_desc &b)
+{
+    return RectsSideBySide(a.dst, b.dst, a.width, b.width, a.height, b.height, a.dpitch, b.dpitch) && a.spitch == b.spitch &&
+           RectPayloadChunks(2 * (a.width / 16), a.height, 1) != 0;
+}
+
+struct RectRun {
+    uint32_t rects = 0;            // of the list, from its front
+    uint32_t entries = 0;
+    uint64_t bytes = 0;
+    uint64_t looseBytes = 0;       // of single rectangles that are not OnLines()
+};
+
+// As many rectangles as the entries of a plan hold, or as make `target` bytes; none of 2^32 units.
+RectRun FillRectChunks(const mf_copy2d_desc *rects, size_t n, uint64_t target, RectChunkPlan &plan)
+{
+    RectRun run;
+    while (run.rects < n && run.entries < kRectInline && run.bytes < target) {
+        const mf_copy2d_desc &d = rects[run.rects];
+        const bool pair = run.rects + 1 < n && RectsPair(d, rects[run.rects + 1]);
+        const uint32_t half = static_cast<uint32_t>(d.width / 16);
+        const uint64_t row = pair ? 2ull * half : half;
+        if (RectPayloadChunks(row, d.height, 1) == 0) {
+            break;
+        }
+        const uint32_t e = run.entries++;
+        plan.src[e] = d.src;
+        plan.other[e] = pair ? rects[run.rects + 1].src : d.src;
+        plan.dst[e] = d.dst;
+        plan.spitchUnits[e] = static_cast<uint32_t>(d.spitch / 16);
+        plan.dpitchUnits[e] = static_cast<uint32_t>(d.dpitch / 16);
+        plan.halfUnits[e] = half;
+        plan.rowUnits[e] = static_cast<uint32_t>(row);
+        plan.height[e] = static_cast<uint32_t>(d.height);
+        plan.magic[e] = RectMagic(plan.rowUnits[e]);
+        run.rects += pair ? 2 : 1;
+        run.bytes += row * 16 * d.height;
+        run.looseBytes += pair || OnLines(d) ? 0 : row * 16 * d.height;
+    }
+    return run;
+}
+
+// The chunk prefix; false for a launch of 2^32 chunks.
+bool CountRectChunks(const RectRun &run, uint32_t units, RectChunkPlan &plan)
+{
+    uint64_t chunks = 0;
+    for (uint32_t i = 0; i < kRectInline; ++i) {
+        plan.first[i] = i < run.entries ? static_cast<uint32_t>(chunks) : 0xFFFFFFFFu;
+        chunks += i < run.entries ? RectPayloadChunks(plan.rowUnits[i], plan.height[i], units) : 0;
+        if (chunks >= 0xFFFFFFFFull) {
+            return false;
+        }
+    }
+    plan.nchunk = static_cast<uint32_t>(chunks);
+    return true;
+}
+
+// The first rectangles of the list in groups of whole rows, one launch; `taken` of them.
+int LaunchRectRows(const mf_copy2d_desc *rects, size_t n, uint32_t gridCap, void *stream, uint32_t &taken)
+{
+    RectPlan plan;
+    uint64_t run = 0;
+    uint32_t used = 0;
+    while (used < n && used < kRectInline) {
+        const mf_copy2d_desc &d = rects[used];
+        const uint32_t rows = RectRowsPerChunk(d.width);
+        const uint64_t chunks = (d.height + rows - 1) / rows;
+        if (used != 0 && run + chunks >= 0xFFFFFFFFull) {
+            break;
+        }
+        plan.src[used] = d.src;
+        plan.dst[used] = d.dst;
+        plan.spitchUnits[used] = static_cast<uint32_t>(d.spitch / 16);
+        plan.dpitchUnits[used] = static_cast<uint32_t>(d.dpitch / 16);
+        plan.widthUnits[used] = static_cast<uint32_t>(d.width / 16);
+        plan.height[used] = static_cast<uint32_t>(d.height);
+        plan.rowsPerChunk[used] = rows;
+        plan.magic[used] = RectMagic(plan.widthUnits[used]);
+        plan.first[used] = static_cast<uint32_t>(run);
+        plan.mate[used] = 0;
+        if (used > 0 && plan.mate[used - 1] == 0) {
+            const mf_copy2d_desc &a = rects[used - 1];
+            if (RectsSideBySide(a.dst, d.dst, a.width, d.width, a.height, d.height, a.dpitch, d.dpitch)) {
+                plan.mate[used - 1] = 1;
+                plan.mate[used] = 2;
+            }
+        }
+        run += chunks;
+        ++used;
+    }
+    for (uint32_t i = used; i < kRectInline; ++i) {
+        plan.src[i] = plan.dst[i] = 0;
+        plan.spitchUnits[i] = plan.dpitchUnits[i] = plan.widthUnits[i] = plan.height[i] = 0;
+        plan.rowsPerChunk[i] = 1;
+        plan.magic[i] = 0;
+        plan.first[i] = 0xFFFFFFFFu;
+        plan.mate[i] = 0;
+    }
+    taken = used;
+    plan.nchunk = static_cast<uint32_t>(run);
+    return mfk_copy2d(&plan, static_cast<uint32_t>(gridCap == 0 || run < gridCap ? run : gridCap), stream);
+}
+
 }  // namespace
 
 MF_EXPORT void mf_copy2d_describe(uint64_t width, uint32_t *rowsPerChunk, uint32_t *magic)
@@ -66,101 +176,52 @@ MF_EXPORT int32_t mf_xcopy_2d_batch(const mf_copy2d_desc *descs, uint32_t n, int
             MF_FAIL(BM_INVALID_PARAM, "rectangle " << i << ": width exceeds the destination pitch");
         }
     }
-    const uint32_t cu = mfrt_cu_count() == 0 ? 256 : mfrt_cu_count();
+    std::vector<mf_copy2d_desc> rects;
     std::vector<uint64_t> rs;
     std::vector<uint64_t> rd;
     std::vector<uint64_t> rl;
-    RectPlan plan;
-    uint32_t used = 0;
-    uint64_t run = 0;
-    // the same launch in the chunks of the windowed form (RectWindowChunks), which a launch of kWindowRectMinBytes and
-    // more between device addresses takes where the segment path would
-    uint32_t firstWindowed[kRectInline];
-    uint64_t runWindowed = 0;
-    uint64_t bytes = 0;
-    bool allWindowable = true;
-    auto flush = [&]() -> int {
-        if (used == 0) {
-            return 0;
-        }
-        const bool windowed = allWindowable && runWindowed < 0xFFFFFFFFull && engine.WindowsApply(bytes, route);
-        for (uint32_t i = used; i < kRectInline; ++i) {
-            plan.src[i] = plan.dst[i] = 0;
-            plan.spitchUnits[i] = plan.dpitchUnits[i] = plan.widthUnits[i] = plan.height[i] = 0;
-            plan.rowsPerChunk[i] = 1;
-            plan.magic[i] = 0;
-            plan.first[i] = 0xFFFFFFFFu;
-            plan.mate[i] = 0;
-        }
-        int err;
-        if (windowed) {
-            for (uint32_t i = 0; i < used; ++i) {
-                plan.first[i] = firstWindowed[i];
-            }
-            plan.nchunk = static_cast<uint32_t>(runWindowed);
-            err = mfk_copy2d_windowed(&plan, engine.Tuning().windowMBps, stream);
-        } else {
-            plan.nchunk = static_cast<uint32_t>(run);
-            const uint32_t perCu = engine.Tuning().wgPerCu;   // 0: one workgroup per row group
-            const uint64_t cap = perCu == 0 ? run : static_cast<uint64_t>(cu) * perCu;
-            err = mfk_copy2d(&plan, static_cast<uint32_t>(run < cap ? run : cap), stream);
-        }
-        used = 0;
-        run = 0;
-        runWindowed = 0;
-        bytes = 0;
-        allWindowable = true;
-        return err;
-    };
+    rects.reserve(n);
+    uint64_t total = 0;
     for (uint32_t i = 0; i < n; ++i) {
         const mf_copy2d_desc &d = descs[i];
         if (d.width == 0 || d.height == 0) {
             continue;
         }
-        if (!Aligned16(d)) {
-            for (uint64_t r = 0; r < d.height; ++r) {
-                rs.push_back(d.src + r * d.spitch);
-                rd.push_back(d.dst + r * d.dpitch);
-                rl.push_back(d.width);
-            }
+        if (Aligned16(d)) {
+            rects.push_back(d);
+            total += d.width * d.height;
             continue;
         }
-        const uint32_t wu = static_cast<uint32_t>(d.width / 16);
-        const uint32_t rpc = RectRowsPerChunk(d.width);
-        const uint64_t chunks = (d.height + rpc - 1) / rpc;
-        if (run + chunks >= 0xFFFFFFFFull || used == kRectInline) {
-            int err = flush();
-            if (err != 0) {
-                MF_FAIL(BM_ERROR, "2-D copy launch failed: " << mfrt_error_string(err));
-            }
+        for (uint64_t r = 0; r < d.height; ++r) {
+            rs.push_back(d.src + r * d.spitch);
+            rd.push_back(d.dst + r * d.dpitch);
+            rl.push_back(d.width);
         }
-        plan.src[used] = d.src;
-        plan.dst[used] = d.dst;
-        plan.spitchUnits[used] = static_cast<uint32_t>(d.spitch / 16);
-        plan.dpitchUnits[used] = static_cast<uint32_t>(d.dpitch / 16);
-        plan.widthUnits[used] = wu;
-        plan.height[used] = static_cast<uint32_t>(d.height);
-        plan.rowsPerChunk[used] = rpc;
-        plan.magic[used] = RectMagic(wu);
-        plan.first[used] = static_cast<uint32_t>(run);
-        plan.mate[used] = 0;
-        const uint64_t windowChunks = RectWindowChunks(wu, d.height);
-        firstWindowed[used] = static_cast<uint32_t>(runWindowed < 0xFFFFFFFFull ? runWindowed : 0xFFFFFFFFull);
-        allWindowable = allWindowable && windowChunks != 0;
-        runWindowed += windowChunks;
-        bytes += d.width * d.height;
-        if (used > 0 && plan.mate[used - 1] == 0 &&
-            RectsSideBySide(plan.dst[used - 1], d.dst, static_cast<uint64_t>(plan.widthUnits[used - 1]) * 16, d.width,
-                            plan.height[used - 1], d.height, static_cast<uint64_t>(plan.dpitchUnits[used - 1]) * 16, d.dpitch)) {
-            plan.mate[used - 1] = 1;
-            plan.mate[used] = 2;
-        }
-        run += chunks;
-        ++used;
     }
-    int err = flush();
-    if (err != 0) {
-        MF_FAIL(BM_ERROR, "2-D copy launch failed: " << mfrt_error_string(err));
+    const uint32_t cu = mfrt_cu_count() == 0 ? 256 : mfrt_cu_count();
+    const uint32_t gridCap = cu * engine.Tuning().wgPerCu;   // 0: one workgroup per row group
+    // A windowed launch loses its schedule the likelier the longer it runs, so long lists go in even parts.
+    const uint64_t parts = (total + kRectLaunchBytes / 2) / kRectLaunchBytes;
+    const uint64_t target = parts < 2 ? ~0ull : (total + parts - 1) / parts;
+    RectChunkPlan plan{};
+    for (size_t at = 0; at < rects.size();) {
+        int err = 0;
+        uint32_t taken = 0;
+        const RectRun run = route == MFRT_ROUTE_HBM && gridCap == 0 && total >= kRectChunksMinBytes
+                                ? FillRectChunks(&rects[at], rects.size() - at, target, plan)
+                                : RectRun{};
+        const bool windowed = run.looseBytes <= run.bytes / 4 && engine.WindowsApply(run.bytes, route, kRectChunksMinBytes);
+        if (run.bytes >= (windowed ? kRectChunksMinBytes : kRectPlainChunksMinBytes) &&
+            CountRectChunks(run, windowed ? kRectWindowUnits : 64 * kRectChunkDepth, plan)) {
+            taken = run.rects;
+            err = mfk_copy2d_chunks(&plan, windowed ? engine.Tuning().windowMBps : 0, stream);
+        } else {
+            err = LaunchRectRows(&rects[at], rects.size() - at, gridCap, stream, taken);
+        }
+        if (err != 0) {
+            MF_FAIL(BM_ERROR, "2-D copy launch failed: " << mfrt_error_string(err));
+        }
+        at += taken;
     }
     if (!rs.empty()) {
         return engine.Submit(rs.data(), rd.data(), rl.data(), static_cast<uint32_t>(rs.size()), route, stream, nullptr, 0);

@@ -82,7 +82,7 @@ struct XcopyTuning {
     int32_t holdPinnedExtraNanos = kHoldLookupExtraNanos;   // added to the rule for launches of more than kInlineSegs segments
     bool stageUnordered = true;  // the upload of a ragged table's descriptors is launched without a barrier
     uint32_t deviceTableWgPerCu = 0;   // grid of a device-resident table in workgroups per CU, 0 = four per segment between 16 and 1024 per CU
-    uint32_t windowMBps = 6800000;   // HBM copies of kWindowRectMinBytes and more alternate between read and write windows cut for this rate; 0 = never
+    uint32_t windowMBps = 6800000;   // long HBM copies alternate between read and write windows cut for this rate; 0 = never
     uint32_t windowAlignedMBps = 7100000;   // the same for launches of segments that all start at multiples of kWindowAlignBytes in source and destination, which hold more; 0 = the rate above
     uint32_t windowLongMBps = 7400000;      // and for those of them whose segments are kWindowLongSegmentBytes and longer on average, which hold more still; 0 = the rate above
 };
@@ -93,10 +93,13 @@ struct XcopyTuning {
 // 6.94 against 6.14, 256 MiB 7.14 against 6.37, 600 MiB 7.20 against 6.31 (at 64 MiB and below the held stores are
 // as fast).  A launch on its own gains less and less steadily below 128 MiB (80 MiB: 32.4 against 31.9 us), hence
 // the limit.  Segments between cache lines, paced for windowMBps, gain 5 to 7 % from there on (136 MB 43.7 against
-// 46.8 us, 272 MB 85 against 91.5, 407 MB 129.5 against 137).  Rectangles do not below 512 MiB (136 MB 45 against
-// 47 us, but 407 MB 141 against 136): they keep the limit they were measured at.
+// 46.8 us, 272 MB 85 against 91.5, 407 MB 129.5 against 137).
 constexpr uint64_t kWindowMinBytes = 128ull << 20;
-constexpr uint64_t kWindowRectMinBytes = 512ull << 20;
+// Rectangles in chunks of their payload: in windows, and without (several threads, rows between cache lines), where whole rows are as
+// fast up to 40 MB (Copy2dChunkKernel has the figures).
+constexpr uint64_t kRectChunksMinBytes = 32ull << 20;
+constexpr uint64_t kRectPlainChunksMinBytes = 48ull << 20;
+constexpr uint64_t kRectLaunchBytes = 640ull << 20;
 constexpr uint64_t kWindowPieceBytes = 512ull << 20;          // launches into which long segments are cut
 constexpr uint64_t kWindowLongSegmentBytes = 64ull << 20;     // launches whose segments average this much go out in pieces of kWindowPieceBytes and more
 constexpr uint64_t kWindowAlignBytes = 128;                   // a cache line: segments that start on one are read and written in whole lines by every wave
@@ -166,7 +169,7 @@ public:
     int Calibrate();
 
     // Whether an ordered launch that moves `bytes` on `route` takes the form with read and write windows.
-    bool WindowsApply(uint64_t bytes, int route, uint64_t minBytes = kWindowRectMinBytes) const;
+    bool WindowsApply(uint64_t bytes, int route, uint64_t minBytes) const;
     // Hardware queue (numbered in order of appearance) of each of the streams made at Start(), in the order they are handed out; returns their number.
     uint32_t StreamQueues(uint32_t *queues, uint32_t capacity) const;
     // No second thread holds a stream of the library: kernels that pace themselves for the whole chip may be used.

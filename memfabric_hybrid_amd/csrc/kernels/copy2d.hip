@@ -1,12 +1,13 @@
 // Batched strided 2-D copy for gfx950: up to 64 rectangles per launch, work cut
 // into groups of rows of about 16 KiB so that narrow rows (a few hundred bytes)
-// still fill every lane with 128-bit accesses.  HBM bound, 2 bytes of traffic
-// per payload byte; no LDS, no MFMA.
+// still fill every lane with 128-bit accesses, or from 32 MiB on into chunks of
+// the payload.  HBM bound, 2 bytes of traffic per payload byte; no LDS, no MFMA.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "../rt/mf_rt.h"
 #include "copy2d_plan.h"
+#include "launch.h"
 #include "window_clock.h"
 
 namespace mf {
@@ -87,86 +88,97 @@ __global__ __launch_bounds__(kRectThreads) void Copy2dKernel(const RectPlan p)
     } while (c < nchunk);
 }
 
-// The same rectangles in read and write windows (the form XcopyWindowKernel gives long segments): single-wave
-// workgroups walk chunks of kRectWindowUnits units of a rectangle's payload taken row-major, whatever the width,
-// one chunk per period each; sixteen loads per lane at the wave's offset into the read half of the period, the
-// stores at the same offset into the write half.  plan.first counts these chunks (RectWindowChunks), a
-// rectangle holds fewer than 2^32 units, rowsPerChunk is not used.
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void Copy2dWindowKernel(const RectPlan p, uint32_t period, uint32_t seq)
+// Rectangles in chunks of their payload (RectChunkPlan).  HBM bounds it.  A chunk of 4 KiB or 16 KiB of the payload is whole cache lines
+// of the destination wherever its rows lie against one another, those of a pair included, where groups of whole rows, and the two
+// halves of a pair's rows written by workgroups apart, end inside a line whenever the width is not a multiple of 128 bytes.
+// us per launch, back to back on buffers that no cache holds, whole rows (Copy2dKernel) / 4 KiB chunks / in windows cut for 6.8 TB/s:
+// pairs of 896 and 4736 bytes, 161 MB 57.5 / - / 51.4, 646 MB 215 / - / 200; of 480 and 2992, 107 MB 45.6 / 38.2 / 34.7, 213 MB 87.6 / - / 67.7; of
+// 736 and 1888, 62 MB 27.0 / 23.7 / 21.3, 247 MB 99.3 / 81.4 / 77.2.  Single rectangles of 896 or 4736 bytes a row with strided source,
+// strided destination or both, 40 MB 17.1 to 17.8 / 16.6 to 17.0 / 14.9 to 15.2, 400 MB 134 to 146 / 129 to 133 / 123 to 129; rows of 480, 2992 or
+// 20 000 bytes, 400 MB 147 to 197 / 129 to 190 / 126 to 201: those go without windows.  Below 32 MiB whole rows are as fast or faster (24 MB
+// 9.0 to 9.5 / 11.2 to 11.6 / 10.1 to 10.7).
+// kPaced: sixteen loads per lane at the wave's offset into the read half of the period, the stores at the same offset into the
+// write half, as XcopyWindowKernel does for long segments.  Rates of 7.1 TB/s and more fall apart for half of these geometries.
+template <bool kPaced>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPaced ? 5 : 8))) void Copy2dChunkKernel(const RectChunkPlan p, uint32_t groups,
+                                                                                                        uint32_t period, uint32_t seq)
 {
+    constexpr uint32_t kDepth = kPaced ? kRectWindowDepth : kRectChunkDepth;
+    constexpr uint32_t kUnits = 64 * kDepth;
     // Only what the search needs stays in vector registers; the rectangle a chunk belongs to is read from the
     // argument block by scalar loads once it is known (a period is microseconds long, their latency does not show).
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t first = p.first[lane];
-    const uint32_t mt = p.mate[lane];
     const uint32_t nchunk = p.nchunk;
     const uint32_t half = period / 2;
-    uint64_t slot = AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * half / gridDim.x;
-    for (uint32_t c = blockIdx.x; c < nchunk; c += gridDim.x) {
-        uint32_t r = __popcll(__ballot(first <= c)) - 1;
-        uint32_t k = c - __builtin_amdgcn_readlane(first, r);
-        const uint32_t m = __builtin_amdgcn_readlane(mt, r);
-        if (m != 0) {
-            const uint32_t r0 = r - (m - 1);
-            const uint32_t both = c - __builtin_amdgcn_readlane(first, r0);
-            r = r0 + (both & 1u);
-            k = both >> 1;
-        }
-        r &= kRectInline - 1;
-        const uint64_t rs = p.src[r];
-        const uint64_t rd = p.dst[r];
-        const uint32_t rsp = p.spitchUnits[r];
-        const uint32_t rdp = p.dpitchUnits[r];
-        const uint32_t rwu = p.widthUnits[r];
-        const uint32_t rht = p.height[r];
-        const uint32_t rmg = p.magic[r];
-        const uint32_t base = k * kRectWindowUnits;
-        const uint32_t left = rht * rwu - base;
-        const uint32_t n = left < kRectWindowUnits ? left : kRectWindowUnits;
-        const uint32_t row0 = base / rwu;
-        const uint32_t col0 = base - row0 * rwu;
-        const MF_GLOBAL u32x4 *s = reinterpret_cast<const MF_GLOBAL u32x4 *>(rs) + static_cast<uint64_t>(row0) * rsp;
-        MF_GLOBAL u32x4 *d = reinterpret_cast<MF_GLOBAL u32x4 *>(rd) + static_cast<uint64_t>(row0) * rdp;
+    uint64_t slot = kPaced ? AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * half / groups : 0;
+    for (uint32_t c = blockIdx.x; c < nchunk; c += groups) {
+        const uint32_t r = (__popcll(__ballot(first <= c)) - 1) & (kRectInline - 1);
+        const uint32_t base = (c - __builtin_amdgcn_readlane(first, r)) * kUnits;
+        const uint32_t sp = p.spitchUnits[r];
+        const uint32_t dp = p.dpitchUnits[r];
+        const uint32_t split = p.halfUnits[r];
+        const uint32_t ru = p.rowUnits[r];
+        const uint32_t mg = p.magic[r];
+        const uint32_t left = p.height[r] * ru - base;
+        const uint32_t n = left < kUnits ? left : kUnits;
+        const uint32_t row0 = base / ru;
+        const uint64_t down = static_cast<uint64_t>(row0) * sp;
+        const MF_GLOBAL u32x4 *s = reinterpret_cast<const MF_GLOBAL u32x4 *>(p.src[r]) + down;
+        const MF_GLOBAL u32x4 *o = reinterpret_cast<const MF_GLOBAL u32x4 *>(p.other[r]) + down - split;
+        MF_GLOBAL u32x4 *d = reinterpret_cast<MF_GLOBAL u32x4 *>(p.dst[r]) + static_cast<uint64_t>(row0) * dp;
         // Row and column of a unit are worked out where its address is needed, before the loads and again before the
         // stores, from a lane offset the compiler cannot see through: kept across the waits (or worked out ahead of them,
         // as it prefers) sixteen rows or thirty-two addresses beside the data take the kernel past the registers at which
         // all kRectWindowWaves waves are resident together with room to spare, which the schedule needs.
-        uint32_t x0 = col0 + lane;
-        auto unitOffset = [&](uint32_t j, uint32_t pitch) -> uint64_t {
+        uint32_t x0 = base - row0 * ru + lane;
+        auto load = [&](uint32_t j) -> u32x4 {
             uint32_t row;
             uint32_t col;
-            RectWindowRowCol(x0 + j * 64, rwu, rmg, row, col);
-            return static_cast<uint64_t>(row) * pitch + col;
+            RectWindowRowCol(x0 + j * 64, ru, mg, row, col);
+            const MF_GLOBAL u32x4 *from = col < split ? s : o;
+            return __builtin_nontemporal_load(from + (static_cast<uint64_t>(row) * sp + col));
         };
-        u32x4 v[kRectWindowDepth];
-        WaitForClock(slot);
-        asm volatile("" : "+v"(x0));
-        if (n == kRectWindowUnits) {
-#pragma unroll
-            for (uint32_t j = 0; j < kRectWindowDepth; ++j) {
-                v[j] = __builtin_nontemporal_load(s + unitOffset(j, rsp));
+        auto store = [&](uint32_t j, u32x4 v) {
+            uint32_t row;
+            uint32_t col;
+            RectWindowRowCol(x0 + j * 64, ru, mg, row, col);
+            __builtin_nontemporal_store(v, d + (static_cast<uint64_t>(row) * dp + col));
+        };
+        auto between = [&] {
+            if (kPaced) {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                WaitForClock(slot + half);
             }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            WaitForClock(slot + half);
             asm volatile("" : "+v"(x0));
+        };
+        u32x4 v[kDepth];
+        if (kPaced) {
+            WaitForClock(slot);
+        }
+        asm volatile("" : "+v"(x0));
+        if (n == kUnits) {
 #pragma unroll
-            for (uint32_t j = 0; j < kRectWindowDepth; ++j) {
-                __builtin_nontemporal_store(v[j], d + unitOffset(j, rdp));
+            for (uint32_t j = 0; j < kDepth; ++j) {
+                v[j] = load(j);
+            }
+            between();
+#pragma unroll
+            for (uint32_t j = 0; j < kDepth; ++j) {
+                store(j, v[j]);
             }
         } else {
 #pragma unroll
-            for (uint32_t j = 0; j < kRectWindowDepth; ++j) {
+            for (uint32_t j = 0; j < kDepth; ++j) {
                 if (j * 64 + lane < n) {
-                    v[j] = __builtin_nontemporal_load(s + unitOffset(j, rsp));
+                    v[j] = load(j);
                 }
             }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            WaitForClock(slot + half);
-            asm volatile("" : "+v"(x0));
+            between();
 #pragma unroll
-            for (uint32_t j = 0; j < kRectWindowDepth; ++j) {
+            for (uint32_t j = 0; j < kDepth; ++j) {
                 if (j * 64 + lane < n) {
-                    __builtin_nontemporal_store(v[j], d + unitOffset(j, rdp));
+                    store(j, v[j]);
                 }
             }
         }
@@ -177,23 +189,29 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void Co
 }  // namespace
 }  // namespace mf
 
-extern "C" int mfk_copy2d_windowed(const void *rectPlan, uint32_t windowMBps, void *stream)
+// In windows cut for windowMBps over chunks of kRectWindowUnits units or, with 0, in chunks of kRectChunkDepth loads per lane.
+extern "C" int mfk_copy2d_chunks(const void *rectChunkPlan, uint32_t windowMBps, void *stream)
 {
-    const mf::RectPlan &plan = *static_cast<const mf::RectPlan *>(rectPlan);
+    using namespace mf;
+    const RectChunkPlan &plan = *static_cast<const RectChunkPlan *>(rectChunkPlan);
+    hipStream_t s = static_cast<hipStream_t>(stream);
     if (plan.nchunk == 0) {
         return 0;
     }
-    const uint32_t grid = mf::WindowGrid(plan.nchunk, mf::kRectWindowWaves);
-    const uint32_t ticks = mf::WindowPeriodTicks(2ull * grid * mf::kRectWindowUnits * 16u, windowMBps);
+    if (windowMBps == 0) {
+        constexpr uint32_t kMost = (1u << 24) - 1;   // the grid size in lanes must stay below 2^32; workgroups loop over the rest
+        const uint32_t grid = plan.nchunk < kMost ? plan.nchunk : kMost;
+        return Launch(Copy2dChunkKernel<false>, grid, 64, 0, s, plan, grid, 0u, 0u);
+    }
+    const uint32_t grid = WindowGrid(plan.nchunk, kRectWindowWaves);
+    const uint32_t ticks = WindowPeriodTicks(2ull * grid * kRectWindowUnits * 16u, windowMBps);
     if (ticks == 0) {
         return static_cast<int>(hipErrorInvalidValue);
     }
-    hipLaunchKernelGGL(mf::Copy2dWindowKernel, dim3(grid), dim3(64), 0, static_cast<hipStream_t>(stream), plan, ticks,
-                       mf::NextWindowSeq());
-    return static_cast<int>(hipGetLastError());
+    return Launch(Copy2dChunkKernel<true>, grid, 64, 0, s, plan, grid, ticks, NextWindowSeq());
 }
 
-// Both kernels once on a plan that holds nothing: a kernel's first launch is not capturable.
+// Every kernel once on a plan that holds nothing: a kernel's first launch is not capturable.
 extern "C" int mfk_copy2d_prelaunch(void *stream)
 {
     mf::RectPlan empty{};
@@ -202,8 +220,12 @@ extern "C" int mfk_copy2d_prelaunch(void *stream)
         empty.rowsPerChunk[i] = 1;
     }
     hipLaunchKernelGGL(mf::Copy2dKernel, dim3(1), dim3(mf::kRectThreads), 0, static_cast<hipStream_t>(stream), empty);
-    hipLaunchKernelGGL(mf::Copy2dWindowKernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream), empty, 64u,
-                       mf::NextWindowSeq());
+    mf::RectChunkPlan none{};
+    for (uint32_t i = 0; i < mf::kRectInline; ++i) {
+        none.first[i] = 0xFFFFFFFFu;
+    }
+    (void)mf::Launch(mf::Copy2dChunkKernel<false>, 1, 64, 0, static_cast<hipStream_t>(stream), none, 1u, 0u, 0u);
+    (void)mf::Launch(mf::Copy2dChunkKernel<true>, 1, 64, 0, static_cast<hipStream_t>(stream), none, 1u, 64u, mf::NextWindowSeq());
     return static_cast<int>(hipGetLastError());
 }
 

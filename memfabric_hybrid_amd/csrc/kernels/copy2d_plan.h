@@ -65,20 +65,36 @@ MF_RECT_HD inline void RectRowCol(uint32_t u, uint32_t widthUnits, uint32_t rows
     col = u - row * widthUnits;
 }
 
-// The windowed form cuts a rectangle's payload, taken row-major, into chunks of kRectWindowUnits units
-// regardless of row ends (16 loads per lane of a single wave).
-constexpr uint32_t kRectWindowDepth = 16;
+// The chunked form: the payload of a rectangle, taken row-major, cut into chunks of one wave whatever the row ends.  Two rectangles that
+// RectsPair() are one entry: their rows, a first and a second half each, are taken as rows of twice the width, so that a chunk writes
+// what lies together in the destination and reads the two sources in turn.
+constexpr uint32_t kRectChunkDepth = 4;           // 128-bit loads per lane: 4 KiB chunks, handed out by the dispatcher
+constexpr uint32_t kRectWindowDepth = 16;         // 16 KiB chunks, walked by resident waves in read and write windows
 constexpr uint32_t kRectWindowUnits = 64 * kRectWindowDepth;
-constexpr uint32_t kRectWindowWaves = 4096;   // 16 per CU
+constexpr uint32_t kRectWindowWaves = 4096;       // 16 per CU
 
-// Chunks of the windowed form, or 0 for a rectangle it cannot take (2^32 units and more).
-MF_RECT_HD inline uint64_t RectWindowChunks(uint64_t widthUnits, uint64_t height)
+struct RectChunkPlan {
+    uint64_t src[kRectInline];
+    uint64_t other[kRectInline];          // the pair's second source; the first again for one rectangle
+    uint64_t dst[kRectInline];
+    uint32_t spitchUnits[kRectInline];    // of both sources
+    uint32_t dpitchUnits[kRectInline];
+    uint32_t halfUnits[kRectInline];      // columns below come from src, the others from `other`; the whole row for one rectangle
+    uint32_t rowUnits[kRectInline];
+    uint32_t height[kRectInline];
+    uint32_t magic[kRectInline];          // RectMagic(rowUnits)
+    uint32_t first[kRectInline];          // exclusive prefix of chunk counts, 0xFFFFFFFF past the end
+    uint32_t nchunk;
+};
+
+// Chunks of `units` units, or 0 for a payload that is not below 2^32 - kRectWindowUnits units.
+MF_RECT_HD inline uint64_t RectPayloadChunks(uint64_t rowUnits, uint64_t height, uint32_t units)
 {
-    const uint64_t units = widthUnits * height;
-    if (widthUnits == 0 || units / widthUnits != height || units > 0xFFFFFFFFull) {
+    const uint64_t all = rowUnits * height;
+    if (rowUnits == 0 || rowUnits > 0xFFFFFFFFull || height > 0xFFFFFFFFull || all > 0xFFFFFFFFull - kRectWindowUnits) {
         return 0;
     }
-    return (units + kRectWindowUnits - 1) / kRectWindowUnits;
+    return (all + units - 1) / units;
 }
 
 // Row (relative to the row the chunk starts in) and column of the unit x units past the start of that row,

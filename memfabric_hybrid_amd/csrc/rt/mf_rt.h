@@ -160,8 +160,9 @@ void mfk_moe_combine_windows(uint32_t readMBps, uint32_t writeMBps);
 
 /* ---- 2-D copy launcher (kernels/copy2d.hip) ----------------------------------- */
 int mfk_copy2d(const void *rectPlan, uint32_t grid, void *stream);
-/* The same rectangles in read and write windows cut for windowMBps; plan.first counts chunks of RectWindowChunks(). */
-int mfk_copy2d_windowed(const void *rectPlan, uint32_t windowMBps, void *stream);
+/* rectChunkPlan: mf::RectChunkPlan; in read and write windows cut for windowMBps over chunks of kRectWindowUnits units, or with 0 in
+ * chunks of 64 * kRectChunkDepth.  Between HBM addresses. */
+int mfk_copy2d_chunks(const void *rectChunkPlan, uint32_t windowMBps, void *stream);
 /* Both rectangle kernels once on an empty plan. */
 int mfk_copy2d_prelaunch(void *stream);
 

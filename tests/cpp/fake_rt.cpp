@@ -639,32 +639,34 @@ int mfk_copy2d(const void *rectPlan, uint32_t, void *)
     return 0;
 }
 
-// The windowed form: chunks of kRectWindowUnits units of the payload taken row-major, unit by unit as the kernel's lanes do.
+// Chunks of the payload taken row-major, unit by unit as the kernel's lanes do; pairs of rectangles as rows of two halves.
 static uint32_t g_rectWindowed = 0;
+static uint32_t g_rectChunked = 0;
 extern "C" uint32_t fake_rt_rect_windowed_launches() { return g_rectWindowed; }
-int mfk_copy2d_windowed(const void *rectPlan, uint32_t windowMBps, void *)
+extern "C" uint32_t fake_rt_rect_chunked_launches() { return g_rectChunked; }
+int mfk_copy2d_chunks(const void *rectChunkPlan, uint32_t windowMBps, void *)
 {
-    const mf::RectPlan &p = *static_cast<const mf::RectPlan *>(rectPlan);
-    if (windowMBps == 0) {
-        return -1;
-    }
+    const mf::RectChunkPlan &p = *static_cast<const mf::RectChunkPlan *>(rectChunkPlan);
+    const uint32_t units = windowMBps != 0 ? mf::kRectWindowUnits : 64 * mf::kRectChunkDepth;
     ++g_launches;
-    ++g_rectWindowed;
+    ++g_rectChunked;
+    g_rectWindowed += windowMBps != 0 ? 1 : 0;
     for (uint32_t c = 0; c < p.nchunk; ++c) {
         uint32_t r = 0;
-        uint32_t k = 0;
-        mf::RectOfChunk(p, c, r, k);
-        const uint32_t wu = p.widthUnits[r];
-        const uint32_t base = k * mf::kRectWindowUnits;
-        const uint32_t total = p.height[r] * wu;
-        const uint32_t row0 = base / wu;
-        const uint32_t col0 = base - row0 * wu;
-        for (uint32_t u = 0; u < mf::kRectWindowUnits && base + u < total; ++u) {
+        while (r + 1 < mf::kRectInline && p.first[r + 1] <= c) {
+            ++r;
+        }
+        const uint32_t ru = p.rowUnits[r];
+        const uint32_t base = (c - p.first[r]) * units;
+        const uint32_t total = p.height[r] * ru;
+        const uint32_t row0 = base / ru;
+        for (uint32_t u = 0; u < units && base + u < total; ++u) {
             uint32_t row = 0;
             uint32_t col = 0;
-            mf::RectWindowRowCol(col0 + u, wu, p.magic[r], row, col);
+            mf::RectWindowRowCol(base - row0 * ru + u, ru, p.magic[r], row, col);
+            const uint64_t from = col < p.halfUnits[r] ? p.src[r] : p.other[r] - 16ull * p.halfUnits[r];
             std::memmove(reinterpret_cast<void *>(p.dst[r] + 16ull * (static_cast<uint64_t>(p.dpitchUnits[r]) * (row0 + row) + col)),
-                         reinterpret_cast<void *>(p.src[r] + 16ull * (static_cast<uint64_t>(p.spitchUnits[r]) * (row0 + row) + col)), 16);
+                         reinterpret_cast<void *>(from + 16ull * (static_cast<uint64_t>(p.spitchUnits[r]) * (row0 + row) + col)), 16);
         }
     }
     return 0;

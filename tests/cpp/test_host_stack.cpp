@@ -27,6 +27,7 @@ extern "C" uint64_t fake_rt_launches(void);
 extern "C" uint32_t fake_rt_last_hold(void);
 extern "C" uint32_t fake_rt_last_rect_mates(void);
 extern "C" uint32_t fake_rt_rect_windowed_launches(void);
+extern "C" uint32_t fake_rt_rect_chunked_launches(void);
 extern "C" void fake_rt_queue_answers(int mode);
 extern "C" int fake_rt_last_combine_paced(void);
 extern "C" uint64_t fake_rt_signals(void);
@@ -1074,6 +1075,78 @@ static void TestWindowedRectangles()
     hybm_uninit();
 }
 
+// Lists of 32 MiB and more go in chunks of the payload, pairs of rectangles as one: every form of list, in windows, without them and
+// (a grid set by hand) as whole rows, leaves the same destination as a copy row by row.
+static void TestRectangleChunks()
+{
+    CHECK(hybm_init(0, 0) == BM_OK);
+    constexpr uint64_t kBytes = 36ull << 20;
+    std::vector<unsigned char> src(3 * kBytes);
+    for (uint64_t i = 0; i < src.size(); i += 8) {
+        const uint64_t word = i * 0x9E3779B97F4A7C15ull + 1;
+        std::memcpy(&src[i], &word, 8);
+    }
+    struct Form { uint64_t width, gap, sgap; int pairs; bool windows; };   // gap: behind a (pair's) row of the destination, sgap: of the source
+    const Form forms[] = {
+        {480, 0, 0, 1, true},      // pairs whose rows are no whole lines, against one another
+        {416, 32, 16, 1, true},    // pairs with gaps on both sides
+        {896, 0, 0, 1, true},      {16, 0, 0, 1, true},       // pairs on lines; of one unit a row
+        {20000, 0, 16, 1, true},   // rows longer than a chunk
+        {896, 128, 0, 0, true},    // single ones on lines
+        {480, 480, 0, 0, false},   // single ones between lines: without windows, and as whole rows below 48 MiB
+        {2992, 0, 16, 0, false},
+        {480, 0, 0, 2, false},     // pairs and single ones in turn: a third of the payload is single
+    };
+    for (const Form &f : forms) {
+        const uint64_t spitch = f.width + f.sgap;
+        const uint64_t height = (f.windows ? kBytes : 50ull << 20) / 14 / f.width + 3;     // fourteen rectangles
+        std::vector<mf_copy2d_desc> rects;
+        uint64_t at = 0;
+        const uint64_t dpitch = 2 * f.width + f.gap;
+        for (uint64_t i = 0; i < 15; ++i) {
+            const bool second = f.pairs == 1 ? i % 2 == 1 : f.pairs == 2 && i % 3 == 1;
+            const bool single = f.pairs == 0 || (f.pairs == 2 && i % 3 == 2);
+            const uint64_t from = i * spitch * height % (src.size() - spitch * height) / 16 * 16;
+            rects.push_back({from, second ? rects.back().dst + f.width : at, f.width, height, spitch, single ? f.width + f.gap : dpitch});
+            if (!second) {
+                at += rects.back().dpitch * height + (f.width % 128 == 0 ? 128 : 48);
+            }
+        }
+        std::vector<unsigned char> expect(at + 16, 0xEE);
+        for (const mf_copy2d_desc &d : rects) {
+            for (uint64_t r = 0; r < d.height; ++r) {
+                std::memcpy(&expect[d.dst + r * d.dpitch], &src[d.src + r * d.spitch], d.width);
+            }
+        }
+        void *memory = nullptr;
+        CHECK(posix_memalign(&memory, 128, at + 16) == 0);
+        unsigned char *dst = static_cast<unsigned char *>(memory);
+        std::vector<unsigned char> spare(src.size() + 128);
+        unsigned char *from = reinterpret_cast<unsigned char *>((reinterpret_cast<uint64_t>(spare.data()) + 127) & ~127ull);
+        std::memcpy(from, src.data(), src.size());
+        for (mf_copy2d_desc &d : rects) {
+            d.src += reinterpret_cast<uint64_t>(from);
+            d.dst += reinterpret_cast<uint64_t>(dst);
+        }
+        for (int mode = 0; mode < 3; ++mode) {   // windows, none, whole rows
+            CHECK(mf_xcopy_windows(mode == 0 ? 6800000 : 0) == BM_OK);
+            CHECK(mf_xcopy_tune(0, mode == 2 ? 4096 : 0, 0) == BM_OK);
+            std::memset(dst, 0xEE, at + 16);
+            const uint32_t windowed = fake_rt_rect_windowed_launches();
+            const uint32_t chunked = fake_rt_rect_chunked_launches();
+            CHECK(mf_xcopy_2d_batch(rects.data(), static_cast<uint32_t>(rects.size()), MF_ROUTE_HBM, nullptr) == BM_OK);
+            CHECK(std::memcmp(dst, expect.data(), expect.size()) == 0);
+            CHECK(fake_rt_rect_windowed_launches() == windowed + (mode == 0 && f.windows ? 1 : 0));
+            CHECK(mode != 2 || fake_rt_rect_chunked_launches() == chunked);
+            CHECK(mode != 0 || fake_rt_rect_chunked_launches() == chunked + 1);
+        }
+        free(memory);
+    }
+    CHECK(mf_xcopy_tune(0, 0, 0) == BM_OK);
+    CHECK(mf_xcopy_windows(1) == BM_OK);
+    hybm_uninit();
+}
+
 // Streams are dealt out one per hardware queue before the second of any.  The stand-in runtime puts the first eight
 // streams of a process on queues A B C C B A D C, as the GPU did.
 static void TestStreamDeck()
@@ -2025,6 +2098,7 @@ int main()
     TestLongSegments();
     TestStreamDeck();
     TestWindowedRectangles();
+    TestRectangleChunks();
     TestCalibration();
     TestUnorderedFanOut();
     TestHostLaunchCosts();

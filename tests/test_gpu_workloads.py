@@ -132,6 +132,37 @@ def test_2d_batch_in_read_and_write_windows(gpu, oracle):
     assert np.array_equal(got, expect)
 
 
+@pytest.mark.parametrize("width, pairs, gap, total_mib", [
+    (480, True, 0, 33), (896, True, 0, 36), (16, True, 16, 33), (20000, True, 0, 64),      # in windows, one period and two
+    (896, False, 128, 40), (480, False, 16, 56), (2992, False, 0, 56),                     # single: on lines, and between them without windows
+    (16368, True, 0, 70), (8192, True, 32, 33)], ids=str)
+def test_2d_batch_in_chunks_of_the_payload(gpu, oracle, width, pairs, gap, total_mib):
+    """Lists of 32 MiB and more are cut into chunks of their payload whatever the row ends; two rectangles side by side
+    in the destination are one, and their rows two halves.  Nine rectangles of `width` bytes a row, all but the last in
+    pairs or all single, `gap` bytes behind every row of the destination.  Byte for byte, gaps included."""
+    n = 9
+    height = total_mib * MIB // n // width + 1
+    dpitch = (2 if pairs else 1) * width + gap
+    each = (dpitch * height + 127) // 128 * 128 + (0 if width % 128 == 0 else 16)
+    sbytes, dbytes = n * width * height, n * each
+    src = _rand(oracle, sbytes, 79)
+    rects = [(i * width * height, (i - i % 2 if pairs else i) * each + (width * (i % 2) if pairs else 0)) for i in range(n)]
+    sbuf = gpu_util.DeviceBuffer(gpu, sbytes)
+    dbuf = gpu_util.DeviceBuffer(gpu, dbytes)
+    try:
+        sbuf.upload(src)
+        dbuf.fill(0x5C)
+        _copy2d(gpu, [(sbuf.ptr + s, dbuf.ptr + d, width, height, width, dpitch) for s, d in rects])
+        got = dbuf.download()
+    finally:
+        sbuf.free()
+        dbuf.free()
+    expect = np.full(dbytes, 0x5C, dtype=np.uint8)
+    for s, d in rects:
+        oracle.orc_copy_2d(np_ptr(expect) + d, dpitch, np_ptr(src) + s, width, width, height)
+    assert np.array_equal(got, expect)
+
+
 def test_2d_argument_errors(gpu):
     d = (native.Copy2dDesc * 1)(native.Copy2dDesc(0x1000, 0x2000, 64, 4, 32, 64))
     assert gpu.mf_xcopy_2d_batch(d, 1, 0, None) == native.BM_INVALID_PARAM      # width > source pitch
