@@ -1724,12 +1724,17 @@ uint32_t XcopyEngine::HoldFor(const InlinePlan &plan, uint32_t grid, int route, 
 
 BatchStats StatsOf(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n)
 {
+    constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kDeepUnits) * kUnitBytes;
     BatchStats st;
     for (uint32_t i = 0; i < n; ++i) {
         st.total += len[i];
         st.longest = len[i] > st.longest ? len[i] : st.longest;
         st.addressBits |= src[i] | dst[i];
         st.lengthBits |= len[i];
+        st.deepPieces += (len[i] + kPieceAlign - 1 + kDeepBytes - 1) / kDeepBytes;
+    }
+    if (st.longest + kPieceAlign <= kDeepBytes) {
+        st.deepPieces = n;
     }
     return st;
 }
@@ -1756,12 +1761,14 @@ uint32_t XcopyEngine::HoldForPieces(const BatchStats &stats, uint32_t n, uint32_
     if ((count > kHoldSharedMaxChunks || units != kXcopyThreads) && g_leasesOut.load(std::memory_order_relaxed) > 1) {
         return 0;
     }
-    const bool byChunks = stats.total <= kDeepMinBytes && units != kXcopyThreads && count <= kDeepMaxChunks;
+    const bool byChunks = stats.total <= kDeepMinBytes && units != kXcopyThreads && count <= (units == kDeepUnits ? kHeldMaxPieces : kDeepMaxChunks);
     constexpr uint64_t kChunkBytes = static_cast<uint64_t>(kXcopyThreads) * kUnitBytes;
     const uint64_t allChunks = (stats.total + kChunkBytes - 1) / kChunkBytes + (stats.lengthBits % kChunkBytes != 0 ? n / 2 : 0);
     const uint32_t chunks = static_cast<uint32_t>(std::min<uint64_t>(allChunks, kHoldMaxChunks));
     // pieces of 8 KiB, two waves of four loads per lane, wait as those of 16 KiB for the same bytes
+    const bool deep = units == kDeepUnits && !byChunks;
     const uint32_t rule = byChunks ? HoldNanosFor(chunks, chunks, kXcopyThreads, false)
+                          : deep ? (count >= kHoldMinChunks / 4 && count <= kHeldMaxPieces ? DeepRuleNanos(count) : 0)
                           : units != kDeepUnits / 2 ? HoldNanosFor(count, count, units, false)
                           : count <= kDeepMaxChunks ? HoldNanosFor(count / 2, count / 2, kDeepUnits, false)
                                                     : 0;
@@ -1774,14 +1781,15 @@ uint32_t XcopyEngine::HoldForPieces(const BatchStats &stats, uint32_t n, uint32_
     if (tuning_.holdCalibratedOff) {
         return 0;
     }
-    const int32_t extra = tuning_.holdPinnedExtraNanos + (!byChunks && units != kXcopyThreads ? kHoldPinnedDeepExtraNanos : 0);
+    const int32_t extra = tuning_.holdPinnedExtraNanos + (!byChunks && units != kXcopyThreads ? kHoldPinnedDeepExtraNanos : 0) +
+                          (deep && (stats.addressBits & (kUnitBytes - 1)) != 0 ? static_cast<int32_t>(PieceOddNanos(count, stats.total)) : 0);
     const int64_t with = static_cast<int64_t>(rule) + extra + tuning_.holdDeltaNanos;
     return with > 0 ? static_cast<uint32_t>(with) : 0;
 }
 
 // Units of the pieces of a batch.  Waves that are resident together hold their stores, and from kPieceLongMinBytes on the longer
-// pieces are the better shape for that (see there) as long as 4096 of them hold the batch: one wave of 16 KiB, or two of 4 KiB
-// where no segment has more than 8 KiB (4096 pages of 8 KiB 12.0 us, 14.5 without hold, 12.9 in waves of 16 KiB).  Beyond, what the
+// pieces are the better shape for that (see there) as long as the chip holds the batch: kHeldMaxPieces waves of 16 KiB or,
+// where no segment has more than 8 KiB, up to 4096 times two of 4 KiB (4096 pages of 8 KiB 12.0 us, 14.5 without hold, 12.9 in waves of 16 KiB).  Beyond, what the
 // usual segment fills: each workgroup twice the size halves the descriptors the host writes and the link carries, but lanes
 // without a unit cost (16 080 pages of 8 KiB 45.2 / 46.1 / 47.0 us with one, two and four waves; 4096 of 32 KiB 45.8 / 46.8 / 46.4).
 // Threads with streams of their own hold nothing but 4 KiB pieces (HoldFor).
@@ -1789,11 +1797,10 @@ uint32_t XcopyEngine::PieceUnits(const BatchStats &stats, uint32_t n, bool unord
 {
     const uint64_t mean = stats.total / n;
     const bool holds = !unordered && tuning_.holdNanos != 0 && tuning_.deepHold && g_leasesOut.load(std::memory_order_relaxed) <= 1;
-    constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kDeepUnits) * kUnitBytes;
-    const uint64_t deepPieces = n + (stats.longest + kPieceAlign <= kDeepBytes ? 0 : stats.total / kDeepBytes);   // at the most
-    if (holds && stats.total > kPieceLongMinBytes && stats.total <= kDeepMaxBytes && stats.longest > kXcopyThreads * kUnitBytes &&
-        deepPieces <= kDeepMaxChunks) {
-        return mean > 6144 && stats.longest <= kDeepUnits / 2 * kUnitBytes ? kDeepUnits / 2 : kDeepUnits;
+    const bool twoWaves = mean > 6144 && stats.longest <= kDeepUnits / 2 * kUnitBytes;
+    if (holds && stats.total > kPieceLongMinBytes && stats.longest > kXcopyThreads * kUnitBytes &&
+        stats.deepPieces <= (twoWaves ? kDeepMaxChunks : kHeldMaxPieces)) {
+        return twoWaves ? kDeepUnits / 2 : kDeepUnits;
     }
     if (stats.total <= kDeepMinBytes) {
         return kXcopyThreads;
@@ -2262,8 +2269,8 @@ int XcopyEngine::SubmitPieces(const uint64_t *src, const uint64_t *dst, const ui
         (void)BuildInlinePlan(none, kXcopyThreads, empty);
         return mfk_xcopy_inline(&empty, MFRT_ROUTE_HBM, 1, mask, maskValue, stream, 0, 0) == 0 ? BM_OK : BM_ERROR;
     }
-    const uint32_t rate = PieceWindowRate(stats, dst, len, n, count, units, unordered);
-    const uint32_t hold = rate != 0 ? 0 : HoldForPieces(stats, n, count, units, unordered);
+    const uint32_t hold = HoldForPieces(stats, n, count, units, unordered);
+    const uint32_t rate = hold != 0 ? 0 : PieceWindowRate(stats, dst, len, n, count, units, unordered);
     const bool own = stream == lease.stream;
     // Reporting costs the GPU the atomics of every wave (200 x 128 KiB 9.9 us with an event, 10.4 so, 2000 x 40 000 34.0 / 37.4), the
     // event costs the host: for batches that the GPU copies in less time than the host needs for the next (4 us and some ns a segment).

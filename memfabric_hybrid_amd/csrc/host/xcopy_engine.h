@@ -48,6 +48,7 @@ struct BatchStats {
     uint64_t longest = 0;
     uint64_t addressBits = 0;       // low bits that any address has set
     uint64_t lengthBits = 0;        // and any length
+    uint64_t deepPieces = 0;        // of 16 KiB, at the most
 };
 BatchStats StatsOf(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n);
 // Whether most of the first segments of a batch are written one behind the other.

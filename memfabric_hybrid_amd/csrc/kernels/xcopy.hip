@@ -688,7 +688,7 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyTableKernel(const TablePla
 // front of the first load: descriptors are fetched in one step from the host's memory, where a table with a chunk prefix and
 // an owner map had to be moved to HBM by a launch of its own first, and no wave looks anything up.
 // Shapes, measured on the kernel alone: single waves of 4 KiB as long as those are resident together, for their held stores;
-// single waves of 16 KiB, held, beyond; and without hold four waves of 16 KiB, or as many as the usual segment fills: 4096 pages of 32 KiB
+// single waves of 16 KiB, held (XcopyPieceHeldKernel), beyond; and without hold four waves of 16 KiB, or as many as the usual segment fills: 4096 pages of 32 KiB
 // gathered 45.8 / 49.4 / 46.4 us with 4 KiB waves / 16 KiB waves / four waves, scattered 49.9 / 51.4 / 49.2, and a quarter of the
 // descriptors for the host to write.
 // `meanwhile`: what is done while the loads are on their way.
@@ -805,6 +805,138 @@ __global__ __launch_bounds__(kLanes) void XcopyPieceKernel(uint64_t list, uint32
     }
     CopyPiece<kLanes, kUnits, kHold, kStoreStream>(p, t0, holdTicks, [&] {
         if (counts && LastArrival(Buffer<uint32_t>(counter), waves, wave, seen)) {
+            __hip_atomic_store(Buffer<uint64_t>(word), static_cast<uint64_t>(value), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    });
+}
+
+// A piece of up to kUnits * 64 units by one wave that holds all of it, in as few registers as there can be: every access is a
+// scalar base and the lane's offset, lanes past the end load the last unit, what lane 63 lacks of the unit behind its last
+// one comes by a scalar load, and the lane is hidden from the compiler, which would work all offsets out at the start.
+template <uint32_t kUnits, class F>
+__device__ __forceinline__ void CopyPieceHeld(const Piece &p, uint64_t t0, uint32_t holdTicks, F meanwhile)
+{
+    const uint64_t src = p.src & kPieceAddress;
+    const uint64_t dst = p.dst & kPieceAddress;
+    const SegGeom g = SegmentGeometry(dst, PieceLength(p.src, p.dst));
+    const uint32_t body = static_cast<uint32_t>(g.body);
+    const uint32_t lane = threadIdx.x;
+    const uint64_t d = dst + g.head;
+    const uint32_t apart = static_cast<uint32_t>(src + g.head) & (kUnitBytes - 1);
+    const uint64_t s = src + g.head - apart;
+    auto hidden = [&] {
+        uint32_t l = lane;
+        asm volatile("" : "+v"(l));
+        return l;
+    };
+    auto load = [&](uint64_t base, uint32_t unit) {
+        return __builtin_nontemporal_load(
+            reinterpret_cast<const MF_GLOBAL u32x4 *>(reinterpret_cast<const MF_GLOBAL uint8_t *>(base) + unit * kUnitBytes));
+    };
+    auto store = [&](uint32_t j, uint32_t unit, u32x4 v) {
+        __builtin_nontemporal_store(
+            v, reinterpret_cast<MF_GLOBAL u32x4 *>(reinterpret_cast<MF_GLOBAL uint8_t *>(d + j * 64 * kUnitBytes) + unit * kUnitBytes));
+    };
+    auto hold = [&] {       // `meanwhile` once the loads have landed: what it needs meets no address or load of theirs
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        meanwhile();
+        HoldStores(t0, holdTicks);
+    };
+    u32x4 v[kUnits];
+    if (body == 0) {
+        meanwhile();
+    } else if (apart == 0 && body == kUnits * 64) {
+#pragma unroll
+        for (uint32_t j = 0; j < kUnits; ++j) {
+            v[j] = load(s + j * 64 * kUnitBytes, lane);
+        }
+        hold();
+#pragma unroll
+        for (uint32_t j = 0; j < kUnits; ++j) {
+            store(j, lane, v[j]);
+        }
+    } else {
+        const uint32_t end = apart != 0 ? body : body - 1;      // the last unit that holds any of the bytes
+        const uint32_t behind = kUnits * 64 < end ? kUnits * 64 : end;
+        const auto *lacks = reinterpret_cast<const __attribute__((address_space(4))) uint32_t *>(s + behind * kUnitBytes);
+        uint32_t last[4] = {lacks[0], lacks[1], lacks[2], lacks[3]};
+#pragma unroll
+        for (uint32_t j = 0; j < kUnits; ++j) {
+            if (j * 64 <= end) {
+                const uint32_t u = j * 64 + hidden();
+                v[j] = load(s, u < end ? u : end);
+            }
+        }
+        asm volatile("" : "+s"(last[0]), "+s"(last[1]), "+s"(last[2]), "+s"(last[3]));
+        hold();
+        if (apart == 0) {
+#pragma unroll
+            for (uint32_t j = 0; j < kUnits; ++j) {
+                const uint32_t l = hidden();
+                if (j * 64 + l < body) {
+                    store(j, l, v[j]);
+                }
+            }
+        } else {
+            auto shifted = [&](auto words) {
+#pragma unroll
+                for (uint32_t j = 0; j < kUnits; ++j) {
+                    u32x4 next;
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; ++i) {
+                        const uint32_t wrap = j + 1 < kUnits ? __builtin_amdgcn_readfirstlane(v[j + 1 < kUnits ? j + 1 : 0][i]) : last[i];
+                        next[i] = NextLane(v[j][i], wrap);
+                    }
+                    const u32x4 r = Straddle<decltype(words)::value>(v[j], next, apart & 3u);
+                    const uint32_t l = hidden();
+                    if (j * 64 + l < body) {
+                        store(j, l, r);
+                    }
+                }
+            };
+            switch (apart >> 2) {
+                case 0: shifted(std::integral_constant<uint32_t, 0>()); break;
+                case 1: shifted(std::integral_constant<uint32_t, 1>()); break;
+                case 2: shifted(std::integral_constant<uint32_t, 2>()); break;
+                default: shifted(std::integral_constant<uint32_t, 3>()); break;
+            }
+        }
+    }
+    if (lane < g.head) {
+        CopyByte<kStoreStream>(src + lane, dst + lane);
+    }
+    if (lane < g.tail) {
+        const uint64_t off = g.head + g.body * kUnitBytes + lane;
+        CopyByte<kStoreStream>(src + off, dst + off);
+    }
+}
+
+// Waves of 16 KiB that hold their stores: 72 registers, 28 waves per CU, so kHeldMaxPieces (112 MiB, most of the chip's registers) are
+// resident and the launch reads all of the batch before it writes any of it.  HBM is the bound.  XcopyPieceKernel's form of sixteen
+// units has 100 registers, 4096 waves.  us back to back, without hold (4 KiB a wave or four waves of them, the better) / in windows cut for 6.0
+// or 6.4 TB/s, the better / XcopyPieceKernel<64, 16, true> / so.  Pages of 32 KiB scattered 28 MB 12.9 / - / 10.8 / 10.8, 72 MB 29.5 / 26.7 / - / 25.7,
+// 88 MB 35.5 / 32.0 / - / 31.2, 104 MB 41.8 / 37.4 / - / 37.0, gathered 56 MB 21.7 / - / 19.7 / 18.9, 104 MB 38.0 / 35.1 / - / 33.9.  Ragged segments of
+// up to 70 000 bytes, 8 MB 6.8 / - / 6.3 / 5.9, 22 MB 12.0 / - / 10.5 / 9.9, 55 MB 25.2 / - / - / 22.1, 74 MB 32.1 / - / - / 28.4, 89 MB 38.0 / - / - / 34.1;
+// of up to 8000, 28 MB 15.3 / - / - / 14.0; of up to 16 000, 57 MB 26.6 / - / - / 25.2.  What is short of full is skipped unit by unit by the whole
+// wave: lanes that loaded the last unit over and over cost 50 MB in segments of 50 688 bytes 20.3, so 18.2.
+// Not taken: 12 KiB in eight waves per SIMD or 20 and 24 KiB in five and four, within 2 %; units beyond the registers kept in LDS (28 and 4 KiB
+// in four waves per SIMD, 4096 pages of 32 KiB 44.5, two launches of 4096 waves 45.2).
+constexpr uint32_t kHeldWavesPerSimd = 7;
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kHeldWavesPerSimd, kHeldWavesPerSimd))) void XcopyPieceHeldKernel(
+    uint64_t list, uint32_t count, uint32_t holdTicks, uint32_t value, uint64_t word, uint64_t counter)
+{
+    const uint64_t t0 = wall_clock64();
+    const uint32_t at = PieceOf(blockIdx.x);
+    if (at >= count) {
+        return;
+    }
+    if (counter == 0) {
+        MarkStarted(word, value);
+    }
+    const Piece p = PieceAt(list, at);
+    CopyPieceHeld<kDeepUnits / 64>(p, t0, holdTicks, [&] {
+        if (counter != 0 && threadIdx.x == 0 &&
+            LastArrival(Buffer<uint32_t>(counter), count, at, Arrive(Buffer<uint32_t>(counter), count, at))) {
             __hip_atomic_store(Buffer<uint64_t>(word), static_cast<uint64_t>(value), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     });
@@ -1482,7 +1614,7 @@ uint32_t HoldTicks(uint32_t nanos)
     if (khz < 0) {
         return 0;
     }
-    const uint64_t capped = nanos < 10000 ? nanos : 10000;   // no wave ever waits longer than 10 us
+    const uint64_t capped = nanos < kHoldMaxNanos ? nanos : kHoldMaxNanos;   // no wave ever waits longer
     return static_cast<uint32_t>(capped * static_cast<uint64_t>(khz) / 1000000u);
 }
 
@@ -1551,12 +1683,11 @@ int LaunchWithEvent(void (*kernel)(Params...), uint32_t grid, uint32_t lanes, hi
     return static_cast<int>(hipGetLastError());
 }
 
-template <uint32_t kLanes, uint32_t kUnits, bool kHold>
-int LaunchPieces(const void *pieces, uint32_t count, uint32_t ticks, hipStream_t stream, hipEvent_t event, void *word, uint32_t value,
-                 void *counter)
+int LaunchPieces(void (*kernel)(uint64_t, uint32_t, uint32_t, uint32_t, uint64_t, uint64_t), uint32_t lanes, const void *pieces, uint32_t count,
+                 uint32_t ticks, hipStream_t stream, hipEvent_t event, void *word, uint32_t value, void *counter)
 {
     const uint32_t grid = (count + kPieceGroup - 1) / kPieceGroup * kPieceGroup;
-    return LaunchWithEvent(XcopyPieceKernel<kLanes, kUnits, kHold>, grid, kLanes, stream, event, At(pieces), count, ticks, value, At(word), At(counter));
+    return LaunchWithEvent(kernel, grid, lanes, stream, event, At(pieces), count, ticks, value, At(word), At(counter));
 }
 
 template <bool kNtLoad, int kStore>
@@ -1698,15 +1829,15 @@ int SubmitPieceList(const void *pieces, uint32_t count, uint64_t bytes, uint32_t
     }
     const uint32_t ticks = HoldTicks(PieceHoldNanos(holdNanos, count, bytes, units));
     if (units == 256) {
-        return ticks != 0 ? LaunchPieces<64, 4, true>(pieces, count, ticks, s, end, word, value, counter)
-                          : LaunchPieces<64, 4, false>(pieces, count, 0, s, end, word, value, counter);
+        return ticks != 0 ? LaunchPieces(XcopyPieceKernel<64, 4, true>, 64, pieces, count, ticks, s, end, word, value, counter)
+                          : LaunchPieces(XcopyPieceKernel<64, 4, false>, 64, pieces, count, 0, s, end, word, value, counter);
     }
     if (units == 512) {
-        return ticks != 0 ? LaunchPieces<128, 4, true>(pieces, count, ticks, s, end, word, value, counter)
-                          : LaunchPieces<128, 4, false>(pieces, count, 0, s, end, word, value, counter);
+        return ticks != 0 ? LaunchPieces(XcopyPieceKernel<128, 4, true>, 128, pieces, count, ticks, s, end, word, value, counter)
+                          : LaunchPieces(XcopyPieceKernel<128, 4, false>, 128, pieces, count, 0, s, end, word, value, counter);
     }
-    return ticks != 0 ? LaunchPieces<64, 16, true>(pieces, count, ticks, s, end, word, value, counter)
-                      : LaunchPieces<256, 4, false>(pieces, count, 0, s, end, word, value, counter);
+    return ticks != 0 ? LaunchPieces(XcopyPieceHeldKernel, 64, pieces, count, ticks, s, end, word, value, counter)
+                      : LaunchPieces(XcopyPieceKernel<256, 4, false>, 256, pieces, count, 0, s, end, word, value, counter);
 }
 
 }  // namespace
@@ -1850,7 +1981,7 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
                 hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kWindowUnits, 1u, 64u, 1u);
                 (void)Launch(XcopyPieceKernel<64, 4, false>, 1, 64, 0, s, 0, 0u, 0u, 0u, 0, 0);
                 (void)Launch(XcopyPieceKernel<64, 4, true>, 1, 64, 0, s, 0, 0u, 0u, 0u, 0, 0);
-                (void)Launch(XcopyPieceKernel<64, 16, true>, 1, 64, 0, s, 0, 0u, 0u, 0u, 0, 0);
+                (void)Launch(XcopyPieceHeldKernel, 1, 64, 0, s, 0, 0u, 0u, 0u, 0, 0);
                 (void)Launch(XcopyPieceKernel<128, 4, false>, 1, 128, 0, s, 0, 0u, 0u, 0u, 0, 0);
                 (void)Launch(XcopyPieceKernel<128, 4, true>, 1, 128, 0, s, 0, 0u, 0u, 0u, 0, 0);
                 (void)Launch(XcopyPieceKernel<256, 4, false>, 1, 256, 0, s, 0, 0u, 0u, 0u, 0, 0);

@@ -100,13 +100,19 @@ constexpr uint32_t kDeepUnits = 1024;
 constexpr uint32_t kDeepMaxChunks = 4096;
 constexpr uint64_t kDeepMinBytes = static_cast<uint64_t>(kHoldMaxChunks) * kXcopyThreads * kUnitBytes;   // 24 MiB
 constexpr uint64_t kDeepMaxBytes = static_cast<uint64_t>(kDeepMaxChunks) * kDeepUnits * kUnitBytes;      // 64 MiB
+constexpr uint32_t kHeldMaxPieces = 7168;          // waves of XcopyPieceHeldKernel that are resident together, 28 per CU
+constexpr uint32_t kHoldMaxNanos = 20000;
 constexpr uint64_t kDeepMinSegmentBytes = 32768;   // on average: short segments make chunks that are not whole
+inline uint32_t DeepRuleNanos(uint32_t count)
+{
+    return 600 + count * 215 / 100;
+}
 inline uint32_t HoldNanosFor(uint32_t nchunk, uint32_t grid, uint32_t units, bool single)
 {
     if (units == kDeepUnits && grid == nchunk && nchunk <= kDeepMaxChunks) {
         // fitted to sweeps over 1664 ... 4096 waves (26 to 64 MiB in 32 segments, one segment, 100 ragged ones): the best wait is
         // 600 ns and 2.15 ns per 16 KiB, a read rate of 7.6 TB/s; up to 10 % beyond costs 1 to 3 %, 10 % short loses half the gain
-        return nchunk < kHoldMinChunks / 4 ? 0 : 600 + nchunk * 215 / 100;
+        return nchunk < kHoldMinChunks / 4 ? 0 : DeepRuleNanos(nchunk);
     }
     if (units != kXcopyThreads || grid != nchunk || nchunk > kHoldMaxChunks) {
         return 0;   // only launches of one chunk per single-wave workgroup were measured
@@ -135,19 +141,44 @@ constexpr uint64_t kDoneCounterBytes = (1 + kDoneCounters) * kDoneCounterWords *
 constexpr int32_t kHoldLookupExtraNanos = 1600;
 constexpr int32_t kHoldLookupDeepExtraNanos = 2000;
 
+// Wait of a launch of pieces of 16 KiB beyond kDeepMinBytes.  Best waits in steps of 400 ns, us: 28 / 40 / 56 / 72 / 88 / 104 MB of pages or blocks
+// gathered and scattered 4.9 / 6.4 to 6.9 / 8.9 / 11.2 / 13.5 / 15.8, a read rate of 6.9 TB/s; where pieces are not full 0.7 ns less for each that
+// is missing (88 MB in segments of 100 000 bytes 12.7); and at odd addresses, where a piece reads lines at both ends that others read too,
+// nothing less (28 / 55 / 74 / 89 MB in segments of up to 70 000 bytes 4.9 / 8.9 / 11.4 / 13.6).  400 ns more or less cost 1 to 2 %.
+inline uint32_t PieceMissing(uint32_t count, uint64_t bytes)
+{
+    const uint64_t full = bytes / (kDeepUnits * kUnitBytes);
+    return count > full ? count - static_cast<uint32_t>(full) : 0;
+}
+inline uint64_t PieceDeepNanos(uint32_t count, uint64_t bytes)
+{
+    const uint64_t wait = 830 + bytes / 6930;
+    const uint64_t less = PieceMissing(count, bytes) * 7ull / 10;
+    return wait > less ? wait - less : 0;
+}
+inline uint32_t PieceOddNanos(uint32_t count, uint64_t bytes)
+{
+    return PieceMissing(count, bytes) * 8 / 10;
+}
+
 // What a launch of `count` pieces waits of the time a table of as many chunks would.  Its descriptors arrive eight to a line, and
 // kPieceLeadNanos sooner than three words per wave did; and ragged pieces are not full, so that the reads are over sooner: by
 // the rate of the rule above for the bytes that are not there.  Best waits beyond HoldNanosFor(count): K and V blocks of 10 / 18 /
-// 24 MB +400 / 200 / 400 ns, 27 / 36 / 45 / 54 / 63 MB on 16 KiB +400 / 800 / 800 / 1200 / 1000; ragged segments of 14 / 21 MB 0, 31 / 41 /
-// 52 MB -800 / -800 / -1200, where the bytes that are not there make 1000 / 1300 / 1700.
+// 24 MB +400 / 200 / 400 ns; ragged segments of 14 / 21 MB 0.
 // Pieces of 8 and 16 KiB of a batch of up to kDeepMinBytes wait as its chunks of 4 KiB would, but for the knee of that rule: best
 // waits beyond it with K and V blocks of 18 / 20 / 22 MB 0 / 40 / 250 ns, 23 MB of pages 300, on 8 KiB 8 / 16 / 25 MB of pages 200 / -100 / 300.
+// Of 16 KiB beyond, PieceDeepNanos.
 constexpr uint32_t kPieceLeadNanos = 1400;
 constexpr uint64_t kPieceKneeBytes = 18000000;
 inline uint32_t PieceLessNanos(uint32_t count, uint64_t bytes, uint32_t units)
 {
     if (units != kXcopyThreads && bytes <= kDeepMinBytes) {
         return kPieceLeadNanos - (bytes > kPieceKneeBytes ? static_cast<uint32_t>((bytes - kPieceKneeBytes) * 7 / 100000) : 0);
+    }
+    if (units == kDeepUnits && count <= kHeldMaxPieces) {
+        const uint64_t rule = DeepRuleNanos(count) + kHoldLookupDeepExtraNanos;
+        const uint64_t wait = PieceDeepNanos(count, bytes);
+        return rule > wait ? static_cast<uint32_t>(rule - wait) : 0;
     }
     const uint64_t full = static_cast<uint64_t>(count) * units * kUnitBytes;
     const uint64_t missing = full > bytes ? (full - bytes) / kUnitBytes : 0;                 // units

@@ -36,13 +36,19 @@ def _lengths(kind, rng):
         return np.concatenate([rng.integers(111000, 131000, 760), EDGES])
     if kind == "windows, three rounds":
         return np.concatenate([np.full(8193, 16384), [16384 + 15, 16383, 1, 0]])
+    if kind == "held, all that are resident":                    # 7168 pieces of 16 KiB at the most hold their stores
+        return np.concatenate([np.full(7168 - len(EDGES), 16256), np.minimum(EDGES, 16256)])
+    if kind == "one too many to hold":
+        return np.concatenate([np.full(7169 - len(EDGES), 16256), np.minimum(np.maximum(EDGES, 1), 16256)])
+    if kind == "more than are held":
+        return np.concatenate([rng.integers(1, 90000, 2700), EDGES])
     if kind == "two waves":
         return np.concatenate([rng.integers(1, 20000, 3000), EDGES])
     return np.concatenate([rng.integers(1, 90000, 2000), EDGES])   # "four waves"
 
 
 @pytest.mark.parametrize("kind", ["every shift", "held 4 KiB", "held 16 KiB", "held 8 KiB", "one wave", "two waves", "four waves", "windows",
-                                  "windows, three rounds"])
+                                  "windows, three rounds", "held, all that are resident", "one too many to hold", "more than are held"])
 @pytest.mark.parametrize("odd", [True, False])
 def test_batch_in_pieces(gpu, oracle, kind, odd):
     rng = np.random.default_rng(len(kind) + odd)
