@@ -1782,14 +1782,15 @@ uint32_t XcopyEngine::HoldForPieces(const BatchStats &stats, uint32_t n, uint32_
         return 0;
     }
     const int32_t extra = tuning_.holdPinnedExtraNanos + (!byChunks && units != kXcopyThreads ? kHoldPinnedDeepExtraNanos : 0) +
-                          (deep && (stats.addressBits & (kUnitBytes - 1)) != 0 ? static_cast<int32_t>(PieceOddNanos(count, stats.total)) : 0);
+                          (deep && ((stats.addressBits & (kUnitBytes - 1)) != 0 || count <= n) ? static_cast<int32_t>(PieceWholeNanos(count, stats.total)) : 0);
     const int64_t with = static_cast<int64_t>(rule) + extra + tuning_.holdDeltaNanos;
     return with > 0 ? static_cast<uint32_t>(with) : 0;
 }
 
 // Units of the pieces of a batch.  Waves that are resident together hold their stores, and from kPieceLongMinBytes on the longer
-// pieces are the better shape for that (see there) as long as the chip holds the batch: kHeldMaxPieces waves of 16 KiB or,
-// where no segment has more than 8 KiB, up to 4096 times two of 4 KiB (4096 pages of 8 KiB 12.0 us, 14.5 without hold, 12.9 in waves of 16 KiB).  Beyond, what the
+// pieces are the better shape for that (see there) as long as the chip holds the batch: kHeldMaxPieces waves of 16 KiB, or two of 4 KiB
+// for each of up to 4096 segments of 6 to 8 KiB (4000 pages of 8 KiB 11.6 to 12.4 us, 13.8 to 15.4 without hold, 11.9
+// to 12.5 in waves of 16 KiB; 4000 of 5120 bytes 10.0, 10.4 and 8.6; 5500 of 8 KiB 17.9 to 19.8 without hold, 15.5 to 17.5 so).  Beyond, what the
 // usual segment fills: each workgroup twice the size halves the descriptors the host writes and the link carries, but lanes
 // without a unit cost (16 080 pages of 8 KiB 45.2 / 46.1 / 47.0 us with one, two and four waves; 4096 of 32 KiB 45.8 / 46.8 / 46.4).
 // Threads with streams of their own hold nothing but 4 KiB pieces (HoldFor).
@@ -1797,9 +1798,8 @@ uint32_t XcopyEngine::PieceUnits(const BatchStats &stats, uint32_t n, bool unord
 {
     const uint64_t mean = stats.total / n;
     const bool holds = !unordered && tuning_.holdNanos != 0 && tuning_.deepHold && g_leasesOut.load(std::memory_order_relaxed) <= 1;
-    const bool twoWaves = mean > 6144 && stats.longest <= kDeepUnits / 2 * kUnitBytes;
-    if (holds && stats.total > kPieceLongMinBytes && stats.longest > kXcopyThreads * kUnitBytes &&
-        stats.deepPieces <= (twoWaves ? kDeepMaxChunks : kHeldMaxPieces)) {
+    if (holds && stats.total > kPieceLongMinBytes && stats.longest > kXcopyThreads * kUnitBytes && stats.deepPieces <= kHeldMaxPieces) {
+        const bool twoWaves = mean > 6144 && stats.longest <= kDeepUnits / 2 * kUnitBytes && stats.deepPieces <= kDeepMaxChunks;
         return twoWaves ? kDeepUnits / 2 : kDeepUnits;
     }
     if (stats.total <= kDeepMinBytes) {
