@@ -566,10 +566,16 @@ uint32_t MemEntity::FirstOutside(void *const *ptrs, const uint64_t *lengths, uin
     uint64_t rangeHi = 0;
     uint32_t checked = 0;
 #if defined(__x86_64__)
-    // the usual batch lies in the windows entirely: four elements a step say so; one that does not is found by the loop below
+    // The usual batch lies in the windows entirely, or in one registered range (the memory of a transfer session): four elements a
+    // step say so, and one that does not is found by the loop below.
     static const bool haveAvx2 = __builtin_cpu_supports("avx2") != 0;
-    if (haveAvx2 && n >= 8 && AllInsideAvx2(ptrs, lengths, n, devLo, devHi, hostLo, hostHi)) {
-        checked = n & ~3u;
+    if (haveAvx2 && n >= 8) {
+        const uint64_t a = reinterpret_cast<uint64_t>(ptrs[0]);
+        const bool windows = (a >= devLo && a < devHi) || (a >= hostLo && a < hostHi) || !haveRanges;
+        if (windows ? AllInsideAvx2(ptrs, lengths, n, devLo, devHi, hostLo, hostHi)
+                    : InRanges(a, lengths[0], &rangeLo, &rangeHi) && AllInsideAvx2(ptrs, lengths, n, rangeLo, rangeHi, rangeLo, rangeHi)) {
+            checked = n & ~3u;
+        }
     }
 #endif
     for (uint32_t i = checked; i < n; ++i) {

@@ -165,11 +165,11 @@ public:
                 PyErr_SetString(PyExc_RuntimeError, "sequence changed while it was read");
                 return nullptr;
             }
-            PyObject *item = PySequence_Fast_GET_ITEM(items_, static_cast<Py_ssize_t>(i));
-            if (PyLong_CheckExact(item)) {
-                room[i] = WordOfInt(item);
-                continue;
+            i += PlainInts(PySequence_Fast_ITEMS(items_) + i, n - i, room + i);
+            if (i == n) {
+                break;
             }
+            PyObject *item = PySequence_Fast_GET_ITEM(items_, static_cast<Py_ssize_t>(i));
             Py_INCREF(item);
             const bool ok = WordOf(item, room[i]);
             Py_DECREF(item);
@@ -181,6 +181,20 @@ public:
     }
 
 private:
+    // The ints in front of the first element that is none.  No Python code runs meanwhile, so the sequence stays as it is.
+    static size_t PlainInts(PyObject *const *__restrict items, size_t n, uint64_t *__restrict room)
+    {
+        constexpr size_t kAhead = 24;
+        size_t i = 0;
+        for (; i < n && PyLong_CheckExact(items[i]); ++i) {
+            if (i + kAhead < n) {
+                __builtin_prefetch(items[i + kAhead]);
+            }
+            room[i] = WordOfInt(items[i]);
+        }
+        return i;
+    }
+
     static bool Integer64(const char *format)
     {
         if (format == nullptr) {

@@ -561,6 +561,51 @@ static void TestTrans()
     CHECK(smem_trans_batch_write(sender, oneLocal, receiverName, outside, one, 1, 0) == SM_INVALID_PARAM);
     one[0] = 8;
     CHECK(smem_trans_batch_write(sender, oneLocal, receiverName, outside, one, 1, 0) == SM_OK);           // ends exactly at the end
+    {
+        // Eleven elements, the first and the last of them at the edges of the registered run; then each of them wrong in one way.
+        constexpr uint32_t m = 11;
+        const std::vector<uint8_t> before(dst, dst + n);
+        const void *from[m];
+        void *to[m];
+        size_t lens[m];
+        auto fill = [&] {
+            for (uint32_t i = 0; i < m; ++i) {
+                from[i] = src + i * 1000;
+                lens[i] = 100 + i;
+                to[i] = dst + 4096 + i * 2000;
+            }
+            to[m - 1] = dst + n - 4096 - lens[m - 1];
+        };
+        fill();
+        std::memset(dst, 0x3C, n);
+        CHECK(smem_trans_batch_write(sender, from, receiverName, to, lens, m, 0) == SM_OK);
+        for (uint32_t i = 0; i < m; ++i) {
+            CHECK(std::memcmp(to[i], from[i], lens[i]) == 0);
+        }
+        for (uint32_t i = 0; i < m; ++i) {
+            for (int wrong = 0; wrong < 8; ++wrong) {
+                fill();
+                switch (wrong) {
+                    case 0: from[i] = nullptr; break;
+                    case 1: to[i] = nullptr; break;
+                    case 2: lens[i] = 0; break;
+                    case 3: lens[i] = ~0ull - 5; break;
+                    case 4: lens[i] = n; break;
+                    case 5: to[i] = dst + 4095; break;
+                    case 6: to[i] = dst + n - 4096 - lens[i] + 1; break;
+                    default: to[i] = reinterpret_cast<void *>(~0ull - 50); break;
+                }
+                std::memset(dst, 0x3C, n);
+                CHECK(smem_trans_batch_write(sender, from, receiverName, to, lens, m, 0) == SM_INVALID_PARAM);
+                bool untouched = true;
+                for (size_t b = 0; b < n; ++b) {
+                    untouched = untouched && dst[b] == 0x3C;
+                }
+                CHECK(untouched);
+            }
+        }
+        std::memcpy(dst, before.data(), n);
+    }
 
     // read back through the single-element calls, into pinned and into pageable memory
     CHECK(smem_trans_read(sender, pinned, receiverName, dst + 4096, 70001, 0) == SM_OK);
