@@ -64,6 +64,16 @@ __device__ __forceinline__ uint64_t AgreedStart(uint32_t seq)
 
 // Period (ticks of the constant-rate clock) in which `bytes` of HBM traffic, read + written, pass at windowMBps
 // MB/s; 0 when the clock rate is unknown or the result is out of range.
+inline uint32_t WindowPeriodTicksAt(uint64_t bytes, uint32_t windowMBps, uint32_t khz)
+{
+    if (windowMBps == 0) {
+        return 0;
+    }
+    // bytes / (MB/s) = microseconds; ticks = microseconds * kHz / 1000
+    const uint64_t ticks = bytes * static_cast<uint64_t>(khz) / (static_cast<uint64_t>(windowMBps) * 1000u);
+    return ticks < 16 || ticks > 1000000 ? 0 : static_cast<uint32_t>(ticks);
+}
+
 inline uint32_t WindowPeriodTicks(uint64_t bytes, uint32_t windowMBps)
 {
     int dev = 0;
@@ -72,9 +82,7 @@ inline uint32_t WindowPeriodTicks(uint64_t bytes, uint32_t windowMBps)
         hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0) {
         return 0;
     }
-    // bytes / (MB/s) = microseconds; ticks = microseconds * kHz / 1000
-    const uint64_t ticks = bytes * static_cast<uint64_t>(khz) / (static_cast<uint64_t>(windowMBps) * 1000u);
-    return ticks < 16 || ticks > 1000000 ? 0 : static_cast<uint32_t>(ticks);
+    return WindowPeriodTicksAt(bytes, windowMBps, static_cast<uint32_t>(khz));
 }
 
 // Waves of a windowed launch of nchunk chunks, at most maxWaves: the chunks are shared out evenly over the fewest

@@ -1105,7 +1105,9 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_
 // How a launch of a device table paces itself; 0: not.
 struct TablePace {
     uint32_t holdTicks;         // of the clock, what a wave waits before it stores, where all waves of the launch are resident together,
-    uint32_t holdMoreTicks;     // and what more per 64 MiB of the table
+    uint32_t holdMoreTicks;     // and what more per 64 MiB of the table;
+    uint32_t equalTicks;        // the same where its segments are of one length, whose descriptors are there sooner
+    uint32_t equalMoreTicks;
     uint32_t windowTicks;       // period in which 64 MiB pass at the rate of random blocks
     uint32_t seq;               // of AgreedStart
 };
@@ -1160,8 +1162,10 @@ __device__ __forceinline__ void CopyDeepChunk(uint64_t src, uint64_t dst, uint64
         WaitForClock(loadAt);
 #pragma unroll
         for (uint32_t j = 0; j < kWindowDepth; ++j) {
-            const uint32_t u = j * 64 + tid < most ? j * 64 + tid : most;
-            v[j] = LoadAligned(from + u * kUnitBytes);
+            if (j * 64 <= most) {
+                const uint32_t u = j * 64 + tid < most ? j * 64 + tid : most;
+                v[j] = LoadAligned(from + u * kUnitBytes);
+            }
         }
         const u32x4 last = LoadAligned(from + most * kUnitBytes);
         meanwhile();
@@ -1228,17 +1232,21 @@ __device__ __forceinline__ void CopyCountedChunk(uint64_t src, uint64_t dst, uin
     }
 }
 
-// Chunk c of a table whose chunk prefix is `first`.
+// Chunk c of a table whose chunk prefix is `first`, and of one whose segments have `each` chunks.
+__device__ __forceinline__ ChunkRef ChunkOf(const uint64_t *__restrict__ triples, uint32_t seg, uint32_t k)
+{
+    const uint64_t *t = triples + 3ull * seg;
+    return ChunkRef{Uniform(t[0]), Uniform(t[1]), Uniform(t[2]), k};
+}
 __device__ __forceinline__ ChunkRef PlannedOwner(const uint64_t *__restrict__ triples, const uint32_t *first, uint32_t nseg, uint32_t c)
 {
     const uint32_t seg = Uniform(LastUpTo(first, nseg, c));
-    const uint64_t *t = triples + 3ull * seg;
-    ChunkRef r;
-    r.src = Uniform(t[0]);
-    r.dst = Uniform(t[1]);
-    r.len = Uniform(t[2]);
-    r.k = c - Uniform(first[seg]);
-    return r;
+    return ChunkOf(triples, seg, c - Uniform(first[seg]));
+}
+__device__ __forceinline__ ChunkRef EqualOwner(const uint64_t *__restrict__ triples, uint32_t each, uint32_t c)
+{
+    const uint32_t seg = Uniform(c / each);
+    return ChunkOf(triples, seg, c - seg * each);
 }
 
 // The chunks c to c + 3, of 4 KiB; false unless all four are there, begin on units and end with one.
@@ -1278,6 +1286,13 @@ __device__ __forceinline__ bool PlannedQuad(const uint64_t *__restrict__ triples
 // 70 000 bytes 24.0 / 16.6, 71.2 / 65.6; 300 of 2 MB 240 / 206.  Longer tables cost each workgroup more lanes' worth of lengths: with
 // kPlannedRun 16, 8000 pages of 8 KiB 28.3 / 30.9, 16 384 ragged of 14 000 bytes 60.3 / 68.9, and that much more code made all others
 // 1 to 3 us slower.  Looking four chunks ahead of a quad up while it loads: registers spill, 8000 pages of 8 KiB 33.3.
+// Segments of one length, as pages are, take a shorter way: one barrier says that they are, and the owner of a chunk is a division instead of
+// a prefix and a search.  us before / so, gathered and scattered: 300 of 32 KiB 5.8 / 5.2, 700 / 1000 / 2000 / 4096 pages of 8 KiB 5.8 / 4.3,
+// 6.6 / 4.8, 8.8 / 7.5, 15.4 and 16.1 / 12.9 and 14.1; 1000 of 32 KiB 13.1 and 13.8 / 12.3 and 12.9, 1000 of 64 KiB 24.1 and 26.3 / 22.7 and
+// 24.3; 3000 of 8200 bytes at odd addresses 13.5 / 11.4.  Finding that out costs other tables 0.1 to 0.2 us, of which the shorter chunks' skipped
+// units give back more to short ones: ragged segments 600 / 1000 of up to 70 000 bytes 10.6 / 10.75, 16.4 / 16.6, 4000 of up to 9000 13.4 / 12.6.  Not
+// taken: descriptors fetched ahead of that barrier, and all lengths requested by one stretch of code, whatever their number (each
+// request of 64 lengths is 24 lines of the L1): 600 / 1000 ragged ones 11.6 / 17.8.
 template <uint32_t kWaves, uint32_t kRun>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
@@ -1291,108 +1306,140 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
     const uint64_t t0 = wall_clock64();
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = threadIdx.x >> 6;
-    uint32_t *sums = words;                                 // [3][kWaves]
-    uint32_t *first = words + 3 * kWaves;                   // [nseg + 1]: chunks of 4 KiB of each segment, then the prefix of its chunks
+    uint32_t *sums = words;                                 // [4][kWaves]
+    uint32_t *first = words + 4 * kWaves;                   // [nseg + 1]: chunks of 4 KiB of each segment, then the prefix of its chunks
     const uint32_t run = (nseg + 64 * kWaves - 1) / (64 * kWaves);
+    const uint64_t len0 = reinterpret_cast<const __attribute__((address_space(4))) uint64_t *>(table)[2];     // by a scalar load
     const uint64_t *t = triples + 3ull * (lane < nseg ? lane : 0);
     const uint32_t bits = static_cast<uint32_t>(t[0] | t[1]);      // of the first 64 segments, the same for every wave
     uint64_t len[kRun];
 #pragma unroll
     for (uint32_t r = 0; r < kRun; ++r) {
         const uint32_t seg = r * 64 * kWaves + threadIdx.x;
-        len[r] = r < run ? triples[3ull * (seg < nseg ? seg : 0) + 2] : 0;
+        // (a branch waits for what is on its way: one wave asks for all, sixteen for no more than they need)
+        len[r] = kWaves == 1 || r < run ? triples[3ull * (seg < nseg ? seg : 0) + 2] : 0;
     }
     uint32_t spare = 0;
+    bool other = false;
 #pragma unroll
     for (uint32_t r = 0; r < kRun; ++r) {
         const uint32_t seg = r * 64 * kWaves + threadIdx.x;
         if (r < run && seg < nseg) {
             first[seg] = static_cast<uint32_t>((len[r] + 4095) >> 12);
             spare += PlannedSpare(len[r]);
+            other = other || len[r] != len0;
         }
-    }
-    __syncthreads();
-    uint32_t count[kRun];
-    uint32_t shallow = 0;       // chunks of 4 KiB,
-    uint32_t deep = 0;          // of 16 KiB
-#pragma unroll
-    for (uint32_t r = 0; r < kRun; ++r) {
-        const uint32_t seg = threadIdx.x * run + r;
-        count[r] = r < run && seg < nseg ? first[seg] : 0;
-        shallow += count[r];
-        deep += (count[r] + 3) / 4;
-    }
-    const uint32_t shallowUpTo = LanesUpTo(shallow);
-    const uint32_t deepUpTo = LanesUpTo(deep);
-    uint32_t spareAll = __builtin_amdgcn_readlane(LanesUpTo(spare), 63);
-    uint32_t shallowAll = __builtin_amdgcn_readlane(shallowUpTo, 63);
-    uint32_t deepAll = __builtin_amdgcn_readlane(deepUpTo, 63);
-    uint32_t shallowBase = 0;
-    uint32_t deepBase = 0;
-    if (kWaves > 1) {
-        if (lane == 0) {
-            sums[wave] = shallowAll;
-            sums[kWaves + wave] = deepAll;
-            sums[2 * kWaves + wave] = spareAll;
-        }
-        __syncthreads();
-        const uint32_t at = lane < kWaves ? lane : 0;
-        const uint32_t a = LanesUpTo(lane < kWaves ? sums[at] : 0);
-        const uint32_t b = LanesUpTo(lane < kWaves ? sums[kWaves + at] : 0);
-        spareAll = __builtin_amdgcn_readlane(LanesUpTo(lane < kWaves ? sums[2 * kWaves + at] : 0), 63);
-        shallowBase = wave == 0 ? 0 : __builtin_amdgcn_readlane(a, wave == 0 ? 0 : wave - 1);
-        deepBase = wave == 0 ? 0 : __builtin_amdgcn_readlane(b, wave == 0 ? 0 : wave - 1);
-        shallowAll = __builtin_amdgcn_readlane(a, 63);
-        deepAll = __builtin_amdgcn_readlane(b, 63);
     }
     // The form: short tables a chunk of 4 KiB per wave; others 16 KiB, of one segment where those are nearly full or where a source and
     // its destination may differ modulo 16, else of up to four.
+    constexpr uint32_t grid = kWindowWaves;
+    uint32_t item = wave * kGroups + blockIdx.x;            // neighbouring ones on neighbouring XCDs
     const bool aligned = __ballot(bits % kUnitBytes != 0) == 0;
-    const uint32_t total = PlannedTotal(deepAll, spareAll);
-    const bool full = PlannedFull(total, deepAll);
-    const bool large = total > kPlannedShallowChunks;
-    const bool quads = large && aligned && !full;
-    const bool byDeep = large && !quads;
-    uint32_t before = byDeep ? deepBase + deepUpTo - deep : shallowBase + shallowUpTo - shallow;
-#pragma unroll
-    for (uint32_t r = 0; r < kRun; ++r) {
-        const uint32_t seg = threadIdx.x * run + r;
-        if (r < run && seg < nseg) {
-            first[seg] = before;
-            before += byDeep ? (count[r] + 3) / 4 : count[r];
-        }
-    }
-    const uint32_t nchunk = byDeep ? deepAll : shallowAll;
-    if (threadIdx.x == 0) {
-        first[nseg] = nchunk;
+    uint32_t shallowAll = 0;
+    uint32_t deepAll = 0;
+    uint32_t total = 0;
+    bool large = false;
+    bool quads = false;
+    auto choose = [&](uint32_t shallowCount, uint32_t deepCount, uint32_t spareCount) {
+        shallowAll = shallowCount;
+        deepAll = deepCount;
+        total = PlannedTotal(deepAll, spareCount);
+        large = total > kPlannedShallowChunks;
+        quads = large && aligned && !PlannedFull(total, deepAll);
+    };
+    bool equal = __ballot(other) == 0;
+    if (kWaves > 1 && lane == 0) {
+        sums[3 * kWaves + wave] = equal ? 1 : 0;
     }
     __syncthreads();
+    if (kWaves > 1) {
+        equal = __ballot(lane < kWaves && sums[3 * kWaves + (lane < kWaves ? lane : 0)] == 0) == 0;
+    }
+    // Segments that all have the length of the first need neither sums nor a prefix.  Pages of up to 16 KiB never go as quads.
+    uint32_t each = 0;
+    if (equal) {
+        const uint32_t shallow0 = static_cast<uint32_t>((len0 + 4095) >> 12);
+        choose(nseg * shallow0, nseg * ((shallow0 + 3) / 4), nseg * PlannedSpare(len0));
+        quads = quads && shallow0 > 4;
+        each = quads ? 0 : large ? (shallow0 + 3) / 4 : shallow0;
+    }
+    if (each == 0) {
+        uint32_t count[kRun];
+        uint32_t shallow = 0;       // chunks of 4 KiB,
+        uint32_t deep = 0;          // of 16 KiB
+#pragma unroll
+        for (uint32_t r = 0; r < kRun; ++r) {
+            const uint32_t seg = threadIdx.x * run + r;
+            count[r] = r < run && seg < nseg ? first[seg] : 0;
+            shallow += count[r];
+            deep += (count[r] + 3) / 4;
+        }
+        const uint32_t shallowUpTo = LanesUpTo(shallow);
+        const uint32_t deepUpTo = LanesUpTo(deep);
+        uint32_t spareAll = __builtin_amdgcn_readlane(LanesUpTo(spare), 63);
+        uint32_t shallowSum = __builtin_amdgcn_readlane(shallowUpTo, 63);
+        uint32_t deepSum = __builtin_amdgcn_readlane(deepUpTo, 63);
+        uint32_t shallowBase = 0;
+        uint32_t deepBase = 0;
+        if (kWaves > 1) {
+            if (lane == 0) {
+                sums[wave] = shallowSum;
+                sums[kWaves + wave] = deepSum;
+                sums[2 * kWaves + wave] = spareAll;
+            }
+            __syncthreads();
+            const uint32_t at = lane < kWaves ? lane : 0;
+            const uint32_t a = LanesUpTo(lane < kWaves ? sums[at] : 0);
+            const uint32_t b = LanesUpTo(lane < kWaves ? sums[kWaves + at] : 0);
+            spareAll = __builtin_amdgcn_readlane(LanesUpTo(lane < kWaves ? sums[2 * kWaves + at] : 0), 63);
+            shallowBase = wave == 0 ? 0 : __builtin_amdgcn_readlane(a, wave == 0 ? 0 : wave - 1);
+            deepBase = wave == 0 ? 0 : __builtin_amdgcn_readlane(b, wave == 0 ? 0 : wave - 1);
+            shallowSum = __builtin_amdgcn_readlane(a, 63);
+            deepSum = __builtin_amdgcn_readlane(b, 63);
+        }
+        choose(shallowSum, deepSum, spareAll);
+        uint32_t before = large && !quads ? deepBase + deepUpTo - deep : shallowBase + shallowUpTo - shallow;
+#pragma unroll
+        for (uint32_t r = 0; r < kRun; ++r) {
+            const uint32_t seg = threadIdx.x * run + r;
+            if (r < run && seg < nseg) {
+                first[seg] = before;
+                before += large && !quads ? (count[r] + 3) / 4 : count[r];
+            }
+        }
+        if (threadIdx.x == 0) {
+            first[nseg] = large && !quads ? deepAll : shallowAll;
+        }
+        __syncthreads();
+    }
+    const bool byDeep = large && !quads;
+    const uint32_t nchunk = byDeep ? deepAll : shallowAll;
 
-    constexpr uint32_t grid = kWindowWaves;
     const uint32_t items = quads ? (nchunk + 3) / 4 : nchunk;
     const bool held = large && items <= grid && total <= kPlannedHeldChunks;
     const bool paced = large && total > kPlannedHeldChunks && aligned && pace.windowTicks != 0 && PlannedFull(total, items);
     const uint32_t rounds = (items + grid - 1) / grid;
     const uint32_t waves = paced ? (items + rounds - 1) / rounds : grid;
-    uint32_t item = wave * kGroups + blockIdx.x;          // neighbouring ones on neighbouring XCDs
     if (item >= items || item >= waves) {
         return;
     }
     constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kWindowUnits) * kUnitBytes;
     const uint32_t period = static_cast<uint32_t>(pace.windowTicks * (waves * kDeepBytes) >> 26);
-    const uint32_t hold = pace.holdTicks + static_cast<uint32_t>(static_cast<uint64_t>(pace.holdMoreTicks) * total >> 14);
+    const uint32_t hold = (each != 0 ? pace.equalTicks : pace.holdTicks) +
+                          static_cast<uint32_t>(static_cast<uint64_t>(each != 0 ? pace.equalMoreTicks : pace.holdMoreTicks) * total >> 14);
     uint64_t loadAt = paced ? AgreedStart(pace.seq) + static_cast<uint64_t>(item) * (period / 2) / waves : 0;
     uint64_t storeAt = paced ? loadAt + period / 2 : held && pace.holdTicks != 0 ? t0 + hold : 0;
     const uint32_t step = paced ? period : 0;
-    if (byDeep) {
+    // (Each owner with a loop of its own: code that a wave only steps over is fetched all the same, at 0.3 us.)
+    auto deepChunks = [&](auto owner) {
         // the next chunk's owner is looked up while the loads of this one are on their way
-        ChunkRef r = PlannedOwner(triples, first, nseg, item);
+        ChunkRef r = owner(item);
         for (;;) {
             const bool more = items - item > waves;
             ChunkRef next = r;
             CopyDeepChunk(r.src, r.dst, r.len, r.k, loadAt, storeAt, [&] {
                 if (more) {
-                    next = PlannedOwner(triples, first, nseg, item + waves);
+                    next = owner(item + waves);
                 }
             });
             if (!more) {
@@ -1403,6 +1450,26 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
             loadAt += step;
             storeAt += step;
         }
+    };
+    auto shallowChunks = [&](auto owner) {
+        for (; item < items; item += waves) {
+            const ChunkRef r = owner(item);
+            CopyCountedChunk(r.src, r.dst, r.len, r.k, lane);
+        }
+    };
+    auto planned = [&](uint32_t c) { return PlannedOwner(triples, first, nseg, c); };
+    auto divided = [&](uint32_t c) { return EqualOwner(triples, each, c); };
+    if (__builtin_expect(each != 0, 0)) {
+        if (byDeep) {
+            deepChunks(divided);
+        } else {
+            shallowChunks(divided);
+        }
+        return;
+    }
+    if (byDeep) {
+        deepChunks(planned);
+        return;
     }
     if (quads) {
         for (; item < items; item += waves) {
@@ -1414,7 +1481,7 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
                 const uint32_t end = item * 4 + 4 < nchunk ? item * 4 + 4 : nchunk;
 #pragma unroll 1
                 for (uint32_t c = item * 4; c < end; ++c) {
-                    const ChunkRef r = PlannedOwner(triples, first, nseg, c);
+                    const ChunkRef r = planned(c);
                     CopyCountedChunk(r.src, r.dst, r.len, r.k, lane);
                 }
             }
@@ -1423,10 +1490,7 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
         }
         return;
     }
-    for (; item < items; item += waves) {
-        const ChunkRef r = PlannedOwner(triples, first, nseg, item);
-        CopyCountedChunk(r.src, r.dst, r.len, r.k, lane);
-    }
+    shallowChunks(planned);
 }
 
 // The segments of a list that a wave is at, one per lane, so that the owner of a piece is found without a load.
@@ -1596,26 +1660,33 @@ uint32_t LanesFor(uint32_t units, int route)
     return lanes <= 64 ? 64u : (lanes <= 128 ? 128u : kXcopyThreads);
 }
 
-// Ticks of the device's constant-rate clock (the one wall_clock64() reads) in `nanos`.
-uint32_t HoldTicks(uint32_t nanos)
+// Rate of the current device's constant-rate clock, the one wall_clock64() reads; 0 where it is not known, and nothing waits.
+uint32_t ClockKhz()
 {
     static std::atomic<int> khzOf[64];
     int dev = 0;
-    if (nanos == 0 || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
         return 0;
     }
     int khz = khzOf[dev].load(std::memory_order_relaxed);
     if (khz == 0) {
         if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0) {
-            khz = -1;   // unknown clock: no hold on this device
+            khz = -1;
         }
         khzOf[dev].store(khz, std::memory_order_relaxed);
     }
-    if (khz < 0) {
-        return 0;
-    }
+    return khz < 0 ? 0 : static_cast<uint32_t>(khz);
+}
+
+uint32_t TicksOf(uint32_t nanos, uint32_t khz)
+{
     const uint64_t capped = nanos < kHoldMaxNanos ? nanos : kHoldMaxNanos;   // no wave ever waits longer
-    return static_cast<uint32_t>(capped * static_cast<uint64_t>(khz) / 1000000u);
+    return static_cast<uint32_t>(capped * khz / 1000000u);
+}
+
+uint32_t HoldTicks(uint32_t nanos)
+{
+    return nanos == 0 ? 0 : TicksOf(nanos, ClockKhz());
 }
 
 // anyOrder: the launch carries no barrier, so the command processor may start it while launches queued
@@ -1935,7 +2006,15 @@ extern "C" int mfk_xcopy_planned(const void *triples, uint32_t nseg, uint32_t ho
         return -1;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const TablePace pace{HoldTicks(holdNanos), HoldTicks(holdMoreNanos), WindowPeriodTicks(2ull << 26, windowMBps), NextWindowSeq()};
+    const uint32_t sooner = holdMoreNanos != 0 ? kTableHoldNanos - kTableEqualNanos : 0;     // a wait set by hand is what it is
+    const uint32_t equalNanos = holdNanos > sooner ? holdNanos - sooner : holdNanos;
+    const uint32_t khz = ClockKhz();
+    const TablePace pace{TicksOf(holdNanos, khz),
+                         TicksOf(holdMoreNanos, khz),
+                         TicksOf(equalNanos, khz),
+                         TicksOf(holdMoreNanos != 0 ? holdMoreNanos + kTableEqualMoreNanos - kTableHoldMoreNanos : 0, khz),
+                         WindowPeriodTicksAt(2ull << 26, windowMBps, khz),
+                         NextWindowSeq()};
     const int err = nseg <= 64 * kPlannedShortRun
                         ? Launch(XcopyPlannedKernel<1, kPlannedShortRun>, kWindowWaves, 64, PlannedLds(1, nseg), s, At(triples), nseg, pace)
                         : Launch(XcopyPlannedKernel<kPlannedWaves, kPlannedRun>, kWindowWaves / kPlannedWaves, 64 * kPlannedWaves,

@@ -367,12 +367,14 @@ MF_HD inline bool PlannedFull(uint32_t total, uint32_t deep)
 {
     return static_cast<uint64_t>(total) * 100 >= static_cast<uint64_t>(deep) * (4 * kPlannedFullPercent);
 }
-constexpr uint32_t PlannedLds(uint32_t waves, uint32_t nseg)          // bytes: the prefix, and three sums of each wave
+constexpr uint32_t PlannedLds(uint32_t waves, uint32_t nseg)          // bytes: the prefix, and four words of each wave
 {
-    return (nseg + 1 + 3 * waves) * 4;
+    return (nseg + 1 + 4 * waves) * 4;
 }
 constexpr int32_t kTableHoldNanos = 2000;             // held stores of device tables: the wait,
-constexpr uint32_t kTableHoldMoreNanos = 8800;        // and what more for 64 MiB
+constexpr uint32_t kTableHoldMoreNanos = 9400;        // and what more for 64 MiB;
+constexpr int32_t kTableEqualNanos = 850;             // of tables of segments of one length, whose waves load that much sooner: best
+constexpr uint32_t kTableEqualMoreNanos = 9850;       // waits in steps of 400 ns 5.6 to 5.9 us at 33 MB, 10.2 to 10.6 at 62 to 65 MB
 
 struct RestSegment {                                  // what is left of a long segment
     uint64_t first;                                   // pieces of those listed before

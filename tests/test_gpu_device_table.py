@@ -125,6 +125,17 @@ PLANNED = {
     "sixteen, windows": (4096, lambda rng, n: np.full(n, 32768), 0),
     "sixteen, more than held, between units": (3001, lambda rng, n: rng.integers(1, 70000, n), 16),
     "sixteen, more than held, not full": (2500, lambda rng, n: rng.integers(1, 4000, n) * 16, 0),
+    "one wave, equal, short": (65, lambda rng, n: np.full(n, 4097), 16),
+    "one wave, equal, one chunk each": (512, lambda rng, n: np.full(n, 16385), 16),
+    "one wave, equal but the last": (512, lambda rng, n: np.where(np.arange(n) == n - 1, 100, 12000), 16),
+    "sixteen, equal, short": (513, lambda rng, n: np.full(n, 15), 16),
+    "sixteen, equal, half chunks": (4095, lambda rng, n: np.full(n, 8192), 0),
+    "sixteen, equal, odd": (1025, lambda rng, n: np.full(n, 16400), 16),
+    "sixteen, equal, quads": (1100, lambda rng, n: np.full(n, 20000), 0),
+    "sixteen, equal, several rounds": (3000, lambda rng, n: np.full(n, 40001), 16),
+    "sixteen, equal but one of the last wave": (1024, lambda rng, n: np.where(np.arange(n) == 1000, 4096, 8192), 0),
+    "sixteen, equal but the first": (1500, lambda rng, n: np.where(np.arange(n) == 0, 1, 30000), 16),
+    "sixteen, all empty but one": (2000, lambda rng, n: np.where(np.arange(n) == 1999, 70000, 0), 16),
     "beyond": (4097, lambda rng, n: rng.integers(1, 9000, n), 16),
 }
 
