@@ -230,6 +230,9 @@ private:
 
     uint32_t HoldFor(const InlinePlan &plan, uint32_t grid, int route, bool unordered) const;
     uint32_t HoldForPieces(const BatchStats &stats, uint32_t n, uint32_t count, uint32_t units, bool unordered) const;
+    uint32_t HeldLaunches(const BatchStats &stats, const uint64_t *dst, const uint64_t *len, uint32_t n, bool unordered) const;
+    int SubmitHeld(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, const BatchStats &stats, uint32_t parts, void *stream,
+                   void *mask, uint32_t maskValue);
     uint32_t PieceUnits(const BatchStats &stats, uint32_t n, bool unordered) const;
     // Rate of the windows a list of `count` pieces of `units` units is copied in, 0: in none.
     uint32_t PieceWindowRate(const BatchStats &stats, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t count, uint32_t units,

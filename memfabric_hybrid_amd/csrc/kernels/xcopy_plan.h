@@ -143,7 +143,7 @@ constexpr int32_t kHoldLookupDeepExtraNanos = 2000;
 
 // Wait of a launch of pieces of 16 KiB beyond kDeepMinBytes.  Best waits in steps of 400 ns, us: 28 / 40 / 56 / 72 / 88 / 104 MB of pages or blocks
 // gathered and scattered 4.9 / 6.4 to 6.9 / 8.9 / 11.2 / 13.5 / 15.8, a read rate of 6.9 TB/s; where segments are cut into pieces that are not full
-// 0.7 ns less for each that is missing (88 MB in segments of 100 000 bytes 12.7); nothing less at odd addresses, where a piece reads lines
+// 0.7 ns less for each that is missing, up to a thousand (88 MB in segments of 100 000 bytes 12.7); nothing less at odd addresses, where a piece reads lines
 // at both ends that others read too (28 / 55 / 74 / 89 MB in segments of up to 70 000 bytes 4.9 / 8.9 / 11.4 / 13.6), nor where a segment is a piece (28 /
 // 36 MB in segments of 5120 bytes 4.5 / 5.8, 45 / 58 MB of 8 KiB 7.3 / 9.2).  400 ns more or less cost 1 to 2 %.
 inline uint32_t PieceMissing(uint32_t count, uint64_t bytes)
@@ -151,15 +151,18 @@ inline uint32_t PieceMissing(uint32_t count, uint64_t bytes)
     const uint64_t full = bytes / (kDeepUnits * kUnitBytes);
     return count > full ? count - static_cast<uint32_t>(full) : 0;
 }
+constexpr uint32_t kPieceLessMissing = 1000;
 inline uint64_t PieceDeepNanos(uint32_t count, uint64_t bytes)
 {
     const uint64_t wait = 830 + bytes / 6930;
-    const uint64_t less = PieceMissing(count, bytes) * 7ull / 10;
+    const uint64_t missing = PieceMissing(count, bytes);
+    const uint64_t less = missing < kPieceLessMissing ? missing * 7 / 10 : kPieceLessMissing * 7 / 10;
     return wait > less ? wait - less : 0;
 }
 inline uint32_t PieceWholeNanos(uint32_t count, uint64_t bytes)
 {
-    return PieceMissing(count, bytes) * 8 / 10;
+    const uint32_t missing = PieceMissing(count, bytes);
+    return (missing < kPieceLessMissing ? missing * 7 / 10 : kPieceLessMissing * 7 / 10) + missing / 10;
 }
 
 // What a launch of `count` pieces waits of the time a table of as many chunks would.  Its descriptors arrive eight to a line, and

@@ -70,7 +70,7 @@ def test_batch_in_pieces(gpu, oracle, kind, odd):
         b.upload(before)
         launches = gpu.mf_xcopy_launch_count()
         gpu_util.xcopy(gpu, a.ptr + src, b.ptr + dst, lens, native.ROUTE_HBM)
-        assert gpu.mf_xcopy_launch_count() - launches == 1
+        assert gpu.mf_xcopy_launch_count() - launches == (2 if kind == "more than are held" else 1)
         got = b.download()
     finally:
         a.free()
