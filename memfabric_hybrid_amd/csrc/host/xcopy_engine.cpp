@@ -1711,7 +1711,7 @@ uint32_t XcopyEngine::HoldFor(const InlinePlan &plan, uint32_t grid, int route, 
     if ((plan.nchunk > kHoldSharedMaxChunks || plan.units == kDeepUnits) && g_leasesOut.load(std::memory_order_relaxed) > 1) {
         return 0;
     }
-    const uint32_t rule = HoldNanosFor(plan.nchunk, grid, plan.units, plan.first[1] == kNoChunk && plan.units != kDeepUnits);
+    const uint32_t rule = HoldNanosFor(plan.nchunk, grid, plan.units, plan.first[1] == kNoChunk);
     if (rule == 0 || tuning_.holdNanos > 0) {
         return rule != 0 ? static_cast<uint32_t>(tuning_.holdNanos) : 0;
     }
@@ -1904,7 +1904,7 @@ void XcopyEngine::TablePaceFor(uint32_t &holdNanos, uint32_t &holdMoreNanos, uin
 bool XcopyEngine::DeepHoldApplies(uint64_t bytes, uint32_t n, int route, bool unordered) const
 {
     return route == MFRT_ROUTE_HBM && !unordered && tuning_.holdNanos != 0 && tuning_.unitsOverride == 0 && tuning_.deepHold &&
-           bytes > kDeepMinBytes && bytes <= kDeepMaxBytes && n != 0 && bytes / n >= kDeepMinSegmentBytes &&
+           bytes > kDeepMinBytes && n != 0 && bytes <= (n == 1 ? kHeldSingleBytes : kDeepMaxBytes) && bytes / n >= kDeepMinSegmentBytes &&
            g_leasesOut.load(std::memory_order_relaxed) <= 1;
 }
 
@@ -2089,16 +2089,16 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
             units = mfk_xcopy_window_units();
         }
         const bool deep = !windowed && DeepHoldApplies(total, n, route, unordered);
-        if (deep && (apartBits & (kUnitBytes - 1)) != 0 && mfrt_stream_capturing(stream) == 0) {
+        if (deep && n != 1 && (apartBits & (kUnitBytes - 1)) != 0 && mfrt_stream_capturing(stream) == 0) {
             // as pieces: sixteen loads per lane of aligned units and what shifts them, with the table of the kernel arguments, take
-            // more registers than sixteen waves per CU have (42 MB 17.5 us with straddling loads)
+            // more registers than sixteen waves per CU have (42 MB 17.5 us with straddling loads); one segment has no table
             const int ret = SubmitPieces(src, dst, len, n, StatsOf(src, dst, len, n), kDeepUnits, stream, mask, maskValue, unordered);
             if (ret != kNotLaunched) {
                 return ret;
             }
         }
         inlined = BuildInlineDirect(src, dst, len, n, deep ? kDeepUnits : units, plan);
-        if (inlined && deep && HoldNanosFor(plan.nchunk, plan.nchunk, kDeepUnits, false) == 0) {
+        if (inlined && deep && HoldNanosFor(plan.nchunk, plan.nchunk, kDeepUnits, plan.first[1] == kNoChunk) == 0) {
             inlined = BuildInlineDirect(src, dst, len, n, units, plan);   // ragged enough to exceed the waves that hold: the usual chunks
         }
     }

@@ -343,6 +343,22 @@ constexpr uint32_t kWindowDepth = 16;                       // 128-bit loads per
 constexpr uint32_t kWindowUnits = 64 * kWindowDepth;        // 16 KiB chunks, one wave each
 constexpr uint32_t kWindowWaves = 4096;                     // 16 per CU
 
+// Chunk c of a segment; with onLines one of LineChunks(), as a segment of its own.
+struct SegChunk {
+    uint64_t src;
+    uint64_t dst;
+    uint64_t len;
+    uint32_t k;
+};
+__device__ __forceinline__ SegChunk ChunkOn(bool onLines, uint64_t src, uint64_t dst, uint64_t len, uint32_t c, uint32_t units)
+{
+    if (!onLines) {
+        return SegChunk{src, dst, len, c};
+    }
+    const LineSpan span = LineChunk(dst, len, c, units);
+    return SegChunk{src + span.begin, dst + span.begin, span.end - span.begin, 0};
+}
+
 // Copy chunk k (kWindowUnits units) of one segment: loads at `slot`, stores at `slot + half`.  A chunk that is
 // not whole (the last one of a segment, or one with head or tail bytes) goes through CopyChunk in the
 // write half: there are at most two such chunks per segment.
@@ -429,7 +445,7 @@ __device__ __forceinline__ void CopyChunkHeld(uint64_t src, uint64_t dst, uint64
 // The inline plan (chunks of kWindowUnits units) copied by gridDim.x single-wave workgroups that walk
 // the chunks with stride gridDim.x, one chunk per period each.
 template <bool kNtLoad, int kStore>
-__global__ __launch_bounds__(64) void XcopyWindowKernel(const InlinePlan p, uint32_t period, uint32_t seq)
+__global__ __launch_bounds__(64) void XcopyWindowKernel(const InlinePlan p, uint32_t period, uint32_t seq, uint32_t onLines)
 {
     const InlineRows rows(p);
     const uint32_t nchunk = p.nchunk;
@@ -437,7 +453,8 @@ __global__ __launch_bounds__(64) void XcopyWindowKernel(const InlinePlan p, uint
     uint64_t slot = AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * half / gridDim.x;
     for (uint32_t c = blockIdx.x; c < nchunk; c += gridDim.x) {
         const InlineChunk r = rows.Owner(c);
-        CopyChunkWindowed<kNtLoad, kStore>(r.src, r.dst, r.len, r.k, slot, half);
+        const SegChunk m = ChunkOn(onLines != 0, r.src, r.dst, r.len, r.k, kWindowUnits);
+        CopyChunkWindowed<kNtLoad, kStore>(m.src, m.dst, m.len, m.k, slot, half);
         slot += period;
     }
 }
@@ -446,15 +463,20 @@ __global__ __launch_bounds__(64) void XcopyWindowKernel(const InlinePlan p, uint
 // the 3080-byte plan), which is cheaper for the host to hand over and spares every wave the table fetch (one copy behind the
 // other, us, against the same bytes as two halves in a table: 8 MiB 3.8 / 5.1, 24 MiB 8.0 / 9.0, 64 MiB 21.2 / 21.5; short ones that
 // are waited for take XcopySingleDoneKernel).  From about 200 MiB on the table form is 1 % faster, hence the limit.
+// A destination off a line has its chunks cut on the lines (onLines): chunks that begin with the segment end inside lines that two workgroups
+// write, each a part.  Back to back, us, chunks of the segment / of the lines: 12 / 16 / 20 / 24 MB 5.7 / 5.0, 6.9 / 6.1, 8.2 / 7.2, 9.5 / 8.3, as long
+// as with a destination on a line; where the source differs modulo 16 too 130 / 200 / 400 MB 46.3 / 43.8, 70.1 / 65.9, 138 / 131, so beyond the limit too.
 constexpr uint32_t kSingleMaxChunks = 49152;
 template <bool kNtLoad, int kStore, int kHold = kHoldNone>
 __global__ __launch_bounds__(kXcopyThreads) void XcopySingleKernel(uint64_t src, uint64_t dst, uint32_t len, uint32_t nchunk,
-                                                                   uint32_t units, uint32_t holdTicks, uint32_t lanes, uint32_t groups)
+                                                                   uint32_t units, uint32_t holdTicks, uint32_t lanes, uint32_t groups,
+                                                                   uint32_t onLines)
 {
     const uint64_t t0 = kHold != kHoldNone ? wall_clock64() : 0;
     uint32_t c = blockIdx.x;
     do {
-        CopyChunkHeld<kNtLoad, kStore, kHold>(src, dst, len, c, units, t0, holdTicks, lanes);
+        const SegChunk m = ChunkOn(onLines != 0, src, dst, len, c, units);
+        CopyChunkHeld<kNtLoad, kStore, kHold>(m.src, m.dst, m.len, m.k, units, t0, holdTicks, lanes);
         c += groups;
     } while (c < nchunk);
 }
@@ -814,11 +836,9 @@ __global__ __launch_bounds__(kLanes) void XcopyPieceKernel(uint64_t list, uint32
 // scalar base and the lane's offset, lanes past the end load the last unit, what lane 63 lacks of the unit behind its last
 // one comes by a scalar load, and the lane is hidden from the compiler, which would work all offsets out at the start.
 template <uint32_t kUnits, class F>
-__device__ __forceinline__ void CopyPieceHeld(const Piece &p, uint64_t t0, uint32_t holdTicks, F meanwhile)
+__device__ __forceinline__ void CopyPieceHeld(uint64_t src, uint64_t dst, uint32_t length, uint64_t t0, uint32_t holdTicks, F meanwhile)
 {
-    const uint64_t src = p.src & kPieceAddress;
-    const uint64_t dst = p.dst & kPieceAddress;
-    const SegGeom g = SegmentGeometry(dst, PieceLength(p.src, p.dst));
+    const SegGeom g = SegmentGeometry(dst, length);
     const uint32_t body = static_cast<uint32_t>(g.body);
     const uint32_t lane = threadIdx.x;
     const uint64_t d = dst + g.head;
@@ -934,12 +954,26 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kHeldWavesPe
         MarkStarted(word, value);
     }
     const Piece p = PieceAt(list, at);
-    CopyPieceHeld<kDeepUnits / 64>(p, t0, holdTicks, [&] {
+    CopyPieceHeld<kDeepUnits / 64>(p.src & kPieceAddress, p.dst & kPieceAddress, PieceLength(p.src, p.dst), t0, holdTicks, [&] {
         if (counter != 0 && threadIdx.x == 0 &&
             LastArrival(Buffer<uint32_t>(counter), count, at, Arrive(Buffer<uint32_t>(counter), count, at))) {
             __hip_atomic_store(Buffer<uint64_t>(word), static_cast<uint64_t>(value), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     });
+}
+
+// A single segment in chunks of LineChunks(), one a wave of the kernel above without a list.  HBM bounds it.  us back to back, from 16 KiB in
+// 100 registers up to 64 MiB and 4 KiB without hold beyond, the chunks the segment's / so: 32 MB 10.9 / 10.3, 48 16.3 / 15.4, 66 20.9 / 20.6, 90
+// 29.9 / 28.4, 110 36.2 / 34.0; destination off a line by 48 bytes 12.1 / 10.4, 18.1 / 15.7, 23.8 / 20.6, 31.7 / 28.8, 38.4 / 34.3; source and destination
+// different modulo 16, before from a list of pieces up to 64 MiB, 11.9 / 10.9, 17.0 / 15.7, 22.9 / 21.0, 32.9 / 29.4, 40.0 / 35.2.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kHeldWavesPerSimd, kHeldWavesPerSimd))) void XcopySingleHeldKernel(
+    uint64_t src, uint64_t dst, uint32_t len, uint32_t holdTicks)
+{
+    const uint64_t t0 = wall_clock64();
+    const LineSpan span = LineChunk(dst, len, blockIdx.x, kDeepUnits);
+    if (span.begin < len) {
+        CopyPieceHeld<kDeepUnits / 64>(src + span.begin, dst + span.begin, static_cast<uint32_t>(span.end - span.begin), t0, holdTicks, [] {});
+    }
 }
 
 // A short blocking batch that says itself when it is done, as XcopySingleDoneKernel.  A blocking call with the signal launch / so, us:
@@ -1702,16 +1736,24 @@ int LaunchInline(const InlinePlan &plan, uint32_t grid, uint32_t lanes, hipStrea
         lanes = 64;
     }
     const uint32_t ticks = grid == plan.nchunk && lanes == 64 ? HoldTicks(holdNanos) : 0;
-    if (plan.first[1] == kNoChunk && plan.nchunk <= kSingleMaxChunks) {
+    const bool single = plan.first[1] == kNoChunk;
+    const uint32_t lineChunks = single ? static_cast<uint32_t>(LineChunks(plan.dst[0], plan.len[0], plan.units)) : 0;
+    if (single && deep && ticks != 0 && lineChunks <= kHeldMaxPieces) {
+        return Launch(XcopySingleHeldKernel, lineChunks, 64, 0, stream, plan.src[0], plan.dst[0], plan.len[0], ticks);
+    }
+    const bool offLine = kStore == kStoreStream && single && (plan.dst[0] & (kLineBytes - 1)) != 0;
+    if (single && (offLine || plan.nchunk <= kSingleMaxChunks)) {
+        // (A chunk more than the waves that hold their stores together would be read when all others have been stored.)
+        const uint32_t onLines = offLine && (ticks == 0 || lineChunks <= kHoldMaxChunks) ? 1 : 0;
+        const uint32_t nchunk = onLines != 0 ? lineChunks : plan.nchunk;
+        grid = grid == plan.nchunk ? nchunk : grid;
         if (anyOrder) {
             hipExtLaunchKernelGGL((XcopySingleKernel<kNtLoad, kStore>), dim3(grid), dim3(lanes), 0, stream, nullptr, nullptr, flags,
-                                  plan.src[0], plan.dst[0], plan.len[0], plan.nchunk, plan.units, 0u, lanes, grid);
+                                  plan.src[0], plan.dst[0], plan.len[0], nchunk, plan.units, 0u, lanes, grid, onLines);
             return static_cast<int>(hipGetLastError());
         }
-        const auto kernel = ticks == 0 ? XcopySingleKernel<kNtLoad, kStore, kHoldNone>
-                            : deep     ? XcopySingleKernel<kNtLoad, kStore, kHoldDeep>
-                                       : XcopySingleKernel<kNtLoad, kStore, kHoldShallow>;
-        return Launch(kernel, grid, lanes, 0, stream, plan.src[0], plan.dst[0], plan.len[0], plan.nchunk, plan.units, ticks, lanes, grid);
+        const auto kernel = ticks == 0 ? XcopySingleKernel<kNtLoad, kStore, kHoldNone> : XcopySingleKernel<kNtLoad, kStore, kHoldShallow>;
+        return Launch(kernel, grid, lanes, 0, stream, plan.src[0], plan.dst[0], plan.len[0], nchunk, plan.units, ticks, lanes, grid, onLines);
     }
     // The ordered launches go through hipLaunchKernel with an argument array: the triple-chevron form pushes and pops a
     // launch configuration around the same call, 0.15 us of host time per launch with this 3 KiB argument block.
@@ -1730,15 +1772,35 @@ int LaunchInline(const InlinePlan &plan, uint32_t grid, uint32_t lanes, hipStrea
     return static_cast<int>(hipLaunchKernel(kernel, dim3(grid), dim3(lanes), args, 0, stream));
 }
 
+// The plan with the chunks of LineChunks(); false where all destinations begin on a line, whose chunks are whole lines as they are.
+bool CutOnLines(const InlinePlan &plan, InlinePlan &lines)
+{
+    uint64_t bits = 0;
+    for (uint32_t i = 0; i < kInlineSegs && plan.first[i] != kNoChunk; ++i) {
+        bits |= plan.dst[i];
+    }
+    if ((bits & (kLineBytes - 1)) == 0) {
+        return false;
+    }
+    lines = plan;
+    uint64_t chunks = 0;
+    for (uint32_t i = 0; i < kInlineSegs && plan.first[i] != kNoChunk; ++i) {
+        lines.first[i] = static_cast<uint32_t>(chunks);
+        chunks += LineChunks(plan.dst[i], plan.len[i], plan.units);
+    }
+    lines.nchunk = static_cast<uint32_t>(chunks);
+    return true;
+}
+
 // windowMBps: the rate (MB/s of HBM traffic, read + written) the period of a windowed launch is cut for.
 template <bool kNtLoad, int kStore>
-int LaunchWindowed(const InlinePlan &plan, uint32_t grid, uint32_t windowMBps, hipStream_t stream)
+int LaunchWindowed(const InlinePlan &plan, uint32_t grid, uint32_t onLines, uint32_t windowMBps, hipStream_t stream)
 {
     const uint32_t ticks = WindowPeriodTicks(2ull * grid * kWindowUnits * kUnitBytes, windowMBps);
     if (ticks == 0) {
         return static_cast<int>(hipErrorInvalidValue);
     }
-    hipLaunchKernelGGL((XcopyWindowKernel<kNtLoad, kStore>), dim3(grid), dim3(64), 0, stream, plan, ticks, NextWindowSeq());
+    hipLaunchKernelGGL((XcopyWindowKernel<kNtLoad, kStore>), dim3(grid), dim3(64), 0, stream, plan, ticks, NextWindowSeq(), onLines);
     return static_cast<int>(hipGetLastError());
 }
 
@@ -1858,14 +1920,17 @@ extern "C" uint32_t mfk_xcopy_window_waves(void)
 
 extern "C" int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream)
 {
-    const mf::InlinePlan &plan = *static_cast<const mf::InlinePlan *>(inlinePlan);
+    const mf::InlinePlan &given = *static_cast<const mf::InlinePlan *>(inlinePlan);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (plan.units != mf::kWindowUnits || plan.nchunk == 0 || windowMBps == 0) {
+    if (given.units != mf::kWindowUnits || given.nchunk == 0 || windowMBps == 0) {
         return -1;
     }
+    mf::InlinePlan lines;
+    const bool onLines = mf::CutOnLines(given, lines);
+    const mf::InlinePlan &plan = onLines ? lines : given;
     const uint32_t grid = mf::WindowGrid(plan.nchunk, mf::kWindowWaves);
     const int err = mf::WithPolicy(mf::PolicyOf(MFRT_ROUTE_HBM), [&](auto ntLoad, auto store) {
-        return mf::LaunchWindowed<decltype(ntLoad)::value, decltype(store)::value>(plan, grid, windowMBps, s);
+        return mf::LaunchWindowed<decltype(ntLoad)::value, decltype(store)::value>(plan, grid, onLines ? 1 : 0, windowMBps, s);
     });
     return err != 0 ? err : mf::Signal(mask, maskValue, s);
 }
@@ -2051,13 +2116,13 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
             constexpr bool kNt = decltype(ntLoad)::value;
             constexpr int kSt = decltype(store)::value;
             hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, empty, 0u);
-            hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 0u, 64u, 1u);
+            hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldNone>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 0u, 64u, 1u, 0u);
             hipLaunchKernelGGL((XcopyTableKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, none);
             if (route == MFRT_ROUTE_HBM) {
                 hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, empty, 1u);
                 hipLaunchKernelGGL((XcopyInlineKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, empty, 1u);
-                hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 1u, 64u, 1u);
-                hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldDeep>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kWindowUnits, 1u, 64u, 1u);
+                hipLaunchKernelGGL((XcopySingleKernel<kNt, kSt, kHoldShallow>), dim3(1), dim3(64), 0, s, 0ull, 0ull, 0u, 0u, kXcopyThreads, 1u, 64u, 1u, 0u);
+                (void)Launch(XcopySingleHeldKernel, 1, 64, 0, s, 0ull, 0ull, 0u, 1u);
                 (void)Launch(XcopyPieceKernel<64, 4, false>, 1, 64, 0, s, 0, 0u, 0u, 0u, 0, 0);
                 (void)Launch(XcopyPieceKernel<64, 4, true>, 1, 64, 0, s, 0, 0u, 0u, 0u, 0, 0);
                 (void)Launch(XcopyPieceHeldKernel, 1, 64, 0, s, 0, 0u, 0u, 0u, 0, 0);
@@ -2068,7 +2133,7 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
                 (void)Launch(XcopyPieceWindowKernel, 1, 64, 0, s, 0, 0u, 64u, NextWindowSeq(), 1u, 0u, 0);
                 (void)Launch(XcopyPlannedKernel<1, kPlannedShortRun>, 1, 64, 64, s, 0, 0u, TablePace{});
                 (void)Launch(XcopyPlannedKernel<kPlannedWaves, kPlannedRun>, 1, 64 * kPlannedWaves, 64, s, 0, 0u, TablePace{});
-                hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
+                hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq(), 0u);
             }
             return 0;
         });
@@ -2194,7 +2259,7 @@ extern "C" int mfk_xcopy_calibrate(void *stream, const uint32_t *holdNanos, cons
                 big.units = kWindowUnits;
                 big.nchunk = static_cast<uint32_t>(half / (kWindowUnits * kUnitBytes));
                 const uint32_t rate = windowMBps[v - 1];
-                err = timed([&](int) { (void)LaunchWindowed<true, kStoreStream>(big, kWindowWaves, rate, s); }, round == 0 ? 1 : 0, 1,
+                err = timed([&](int) { (void)LaunchWindowed<true, kStoreStream>(big, kWindowWaves, 0, rate, s); }, round == 0 ? 1 : 0, 1,
                             out[4 + v]);
             }
             if (err != hipSuccess) {

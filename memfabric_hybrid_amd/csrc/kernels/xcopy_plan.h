@@ -65,6 +65,28 @@ MF_HD inline uint64_t SegmentChunks(uint64_t dst, uint64_t len, uint32_t units)
     return n == 0 ? 1 : n;
 }
 
+// The same with its cuts where the destination reaches a multiple of kLineBytes: the first chunk is shorter by what the
+// destination lies behind one, and no two chunks write one cache line.
+constexpr uint32_t kLineBytes = 128;
+MF_HD inline uint64_t LineChunks(uint64_t dst, uint64_t len, uint32_t units)
+{
+    const uint64_t each = static_cast<uint64_t>(units) * kUnitBytes;
+    return len == 0 ? 0 : ((dst & (kLineBytes - 1)) + len + each - 1) / each;
+}
+
+// Bytes [begin, end) of such a segment that chunk k < LineChunks() holds.
+struct LineSpan {
+    uint64_t begin;
+    uint64_t end;
+};
+MF_HD inline LineSpan LineChunk(uint64_t dst, uint64_t len, uint64_t k, uint32_t units)
+{
+    const uint64_t each = static_cast<uint64_t>(units) * kUnitBytes;
+    const uint64_t skip = dst & (kLineBytes - 1);
+    const uint64_t end = (k + 1) * each - skip;
+    return LineSpan{k == 0 ? 0 : k * each - skip, end < len ? end : len};
+}
+
 // Everything a launch of up to kInlineSegs segments needs, passed by value in
 // the kernel-argument block (3080 bytes of the 4096 available): no table
 // upload, no extra dependent memory round trip before the first data load.
@@ -101,6 +123,7 @@ constexpr uint32_t kDeepMaxChunks = 4096;
 constexpr uint64_t kDeepMinBytes = static_cast<uint64_t>(kHoldMaxChunks) * kXcopyThreads * kUnitBytes;   // 24 MiB
 constexpr uint64_t kDeepMaxBytes = static_cast<uint64_t>(kDeepMaxChunks) * kDeepUnits * kUnitBytes;      // 64 MiB
 constexpr uint32_t kHeldMaxPieces = 7168;          // waves of XcopyPieceHeldKernel that are resident together, 28 per CU
+constexpr uint64_t kHeldSingleBytes = static_cast<uint64_t>(kHeldMaxPieces) * kDeepUnits * kUnitBytes - kLineBytes;   // wherever its lines begin
 constexpr uint32_t kHoldMaxNanos = 20000;
 constexpr uint64_t kDeepMinSegmentBytes = 32768;   // on average: short segments make chunks that are not whole
 inline uint32_t DeepRuleNanos(uint32_t count)
@@ -109,10 +132,12 @@ inline uint32_t DeepRuleNanos(uint32_t count)
 }
 inline uint32_t HoldNanosFor(uint32_t nchunk, uint32_t grid, uint32_t units, bool single)
 {
-    if (units == kDeepUnits && grid == nchunk && nchunk <= kDeepMaxChunks) {
+    if (units == kDeepUnits && grid == nchunk && nchunk <= (single ? kHeldMaxPieces : kDeepMaxChunks)) {
         // fitted to sweeps over 1664 ... 4096 waves (26 to 64 MiB in 32 segments, one segment, 100 ragged ones): the best wait is
         // 600 ns and 2.15 ns per 16 KiB, a read rate of 7.6 TB/s; up to 10 % beyond costs 1 to 3 %, 10 % short loses half the gain
-        return nchunk < kHoldMinChunks / 4 ? 0 : DeepRuleNanos(nchunk);
+        // (a single segment's waves know their chunk at once, so the reads are over sooner: best waits of 26 to 117 MB in steps of
+        // 500 ns 500 to 1000 shorter, 500 where source and destination differ modulo 16; that much more costs 2 to 4 %)
+        return nchunk < kHoldMinChunks / 4 ? 0 : DeepRuleNanos(nchunk) - (single ? 500 : 0);
     }
     if (units != kXcopyThreads || grid != nchunk || nchunk > kHoldMaxChunks) {
         return 0;   // only launches of one chunk per single-wave workgroup were measured

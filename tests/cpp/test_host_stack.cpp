@@ -923,6 +923,31 @@ static void TestPlanners()
     }
 }
 
+// Chunks cut on the destination's lines: side by side over the whole segment, each no longer than a chunk, all cuts on lines.
+static void TestLineChunks()
+{
+    const uint64_t lens[] = {1, 15, 16, 127, 128, 129, 4095, 4096, 4097, 16383, 16384, 16385, 100000, kHeldSingleBytes, 0xFFFFFFFFull};
+    for (uint32_t units : {256u, 512u, kDeepUnits}) {
+        for (uint64_t off : {0u, 1u, 15u, 16u, 48u, 77u, 112u, 127u}) {
+            for (uint64_t len : lens) {
+                const uint64_t dst = (1ull << 40) + off;
+                const uint64_t count = LineChunks(dst, len, units);
+                uint64_t at = 0;
+                bool ok = count != 0;
+                for (uint64_t k = 0; k < count && ok; ++k) {
+                    const LineSpan s = LineChunk(dst, len, k, units);
+                    ok = s.begin == at && s.end > at && s.end - at <= units * 16ull && (s.end == len || (dst + s.end) % kLineBytes == 0);
+                    at = s.end;
+                }
+                CHECK(ok && at == len);
+            }
+        }
+    }
+    CHECK(LineChunks(5, 0, 256) == 0);
+    CHECK(LineChunks(127, kHeldSingleBytes, kDeepUnits) <= kHeldMaxPieces);
+    CHECK(HoldNanosFor(kHeldMaxPieces, kHeldMaxPieces, kDeepUnits, true) != 0 && HoldNanosFor(kHeldMaxPieces, kHeldMaxPieces, kDeepUnits, false) == 0);
+}
+
 // The choice hybm_init makes from what it measures on its GPU.
 static void TestCalibration()
 {
@@ -2144,6 +2169,7 @@ int main()
     TestStreamDeck();
     TestWindowedRectangles();
     TestRectangleChunks();
+    TestLineChunks();
     TestCalibration();
     TestUnorderedFanOut();
     TestHostLaunchCosts();

@@ -208,6 +208,18 @@ def test_single_large_copy_with_odd_edges(gpu, oracle):
     _check_d2d(gpu, oracle, pool, np.array([3]), np.array([96 * MIB + 5]), np.array([80 * MIB + 123]), 0xB2)
 
 
+@pytest.mark.parametrize("src_off,dst_off", [(0, 0), (16, 48), (128, 112), (3, 19), (37, 100), (5, 127)])
+@pytest.mark.parametrize("length", [5000, 4 * MIB + 1, 24 * MIB - 1, 24 * MIB + 4096, 64 * MIB, 112 * MIB - 128, 112 * MIB - 127,
+                                    127 * MIB, 128 * MIB + 77, 193 * MIB + 5])
+def test_single_copies_whose_chunks_are_cut_on_lines(gpu, oracle, length, src_off, dst_off):
+    """One segment at each limit of the forms that copy it, destinations on a line, off it by whole units and by bytes, sources
+    that agree modulo 16 and that do not."""
+    half = 256 + (length + 255) // 256 * 256
+    one = np.array([length], dtype=np.uint64)
+    _check_d2d(gpu, oracle, 2 * half, np.array([src_off], dtype=np.uint64), half + np.array([dst_off], dtype=np.uint64), one,
+               seed=0x77 + length % 1000)
+
+
 def test_adjacent_segments_are_merged_without_changing_bytes(gpu, oracle):
     pool = 32 * MIB
     n = 300
