@@ -1812,24 +1812,26 @@ uint32_t XcopyEngine::PieceUnits(const BatchStats &stats, uint32_t n, bool unord
     return mean <= 6144 ? kXcopyThreads : mean <= 12288 ? kDeepUnits / 2 : kDeepUnits;
 }
 
-// Of 6.0 TB/s, which blocks at random places hold; of 6.4 for long ones that are written one behind the other, which leaves the
-// rows of HBM open (short ones hold that in some places of the pool only, and gain nothing at 6.0: 16 384 pages of 32 KiB gathered 182 us
-// without windows, 171 to 194 at 6.4, 181 at 6.0; the kernel has the other figures).  Pieces that are much less than full gain
+// Of 6.0 TB/s, which blocks at random places hold; of 6.4 for such of one length from 64 KiB on; of 6.6 for long ones that are written one
+// behind the other, which leaves the rows of HBM open (short ones hold that in some places of the pool only, and gain nothing at 6.0: 16 384
+// pages of 32 KiB gathered 182 us without windows, 171 to 194 at 6.4, 181 at 6.0).  At 6.0 / 6.2 / 6.4 / 6.6 / 6.8, the same to 1 % in four
+// processes: 64 KiB gathered, 2048 47.6 / 46.3 / 44.9 / 43.7 / 44.1, 16 000 355 / 344 / 333 / 328 / 350; scattered, 4096 92.6 / 90.0 / 87.7 / 86.0 / 96, 16 000
+// 355 / 344 / 345 / 375 / 402; 2000 of 128 KiB gathered and scattered 90.7 / 87.8 / 85.4 / 83.3 / 85.  Pieces that are much less than full gain
 // nothing; segments between cache lines keep the launch without windows, as they do in launches of kInlineSegs segments up to
 // kWindowSliceMinSegmentBytes.
 uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t count, uint32_t units,
                                       bool unordered) const
 {
-    constexpr uint64_t kLongBytes = 64ull << 10;
     const bool full = stats.total >= static_cast<uint64_t>(count) * (kDeepUnits * kUnitBytes) / 100 * 85;
     if (unordered || units != kDeepUnits || !full || (stats.addressBits & (kWindowAlignBytes - 1)) != 0 ||
         !WindowsApply(stats.total, MFRT_ROUTE_HBM, kPieceWindowMinBytes)) {
         return 0;
     }
     if (WrittenInOrder(dst, len, n)) {
-        return stats.total / n >= kLongBytes ? tuning_.windowMBps / 17 * 16 : 0;
+        return stats.total / n >= kWindowLongBlockBytes ? tuning_.windowMBps / 34 * 33 : 0;
     }
-    return tuning_.windowMBps / 17 * 15;
+    const bool longBlocks = stats.longest >= kWindowLongBlockBytes && stats.total == stats.longest * n;
+    return tuning_.windowMBps / 17 * (longBlocks ? 16 : 15);
 }
 
 // In how many launches, each of as many pieces as are held, a list of more goes out; 1 where one that holds nothing is as fast.  Back to back,

@@ -1142,7 +1142,9 @@ struct TablePace {
     uint32_t holdMoreTicks;     // and what more per 64 MiB of the table;
     uint32_t equalTicks;        // the same where its segments are of one length, whose descriptors are there sooner
     uint32_t equalMoreTicks;
-    uint32_t windowTicks;       // period in which 64 MiB pass at the rate of random blocks
+    uint32_t windowTicks;       // period in which 64 MiB pass at the rate of random blocks,
+    uint32_t longTicks;         // of such of one length, kWindowLongBlockBytes or more,
+    uint32_t orderedTicks;      // and of blocks of one length that are written one behind the other
     uint32_t seq;               // of AgreedStart
 };
 
@@ -1327,6 +1329,9 @@ __device__ __forceinline__ bool PlannedQuad(const uint64_t *__restrict__ triples
 // units give back more to short ones: ragged segments 600 / 1000 of up to 70 000 bytes 10.6 / 10.75, 16.4 / 16.6, 4000 of up to 9000 13.4 / 12.6.  Not
 // taken: descriptors fetched ahead of that barrier, and all lengths requested by one stretch of code, whatever their number (each
 // request of 64 lengths is 24 lines of the L1): 600 / 1000 ragged ones 11.6 / 17.8.
+// In windows cut for 6.0 / 6.2 / 6.4 / 6.6 / 6.8 TB/s, the same to 0.5 in four processes: 4096 pages of 32 KiB gathered 49.8 / 48.4 / 47.1 / 46.0 / 45.3,
+// scattered 50.2 / 51.2 / 54 / 54 / 54; of 64 KiB gathered 94.5 / 91.7 / 89.4 / 87.3 / 85.7 (7.0: 91), scattered 95.0 / 92.8 / 90.5 / 87.8 / 97 to 102;
+// 1000 of 256 KiB scattered 92.0 / 89.6 / 87.1 / 85.2 / 86.7 to 91.6: 6.6 for what is written in order, 6.4 for scattered pages of 64 KiB and more.
 template <uint32_t kWaves, uint32_t kRun>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
@@ -1345,7 +1350,8 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
     const uint32_t run = (nseg + 64 * kWaves - 1) / (64 * kWaves);
     const uint64_t len0 = reinterpret_cast<const __attribute__((address_space(4))) uint64_t *>(table)[2];     // by a scalar load
     const uint64_t *t = triples + 3ull * (lane < nseg ? lane : 0);
-    const uint32_t bits = static_cast<uint32_t>(t[0] | t[1]);      // of the first 64 segments, the same for every wave
+    const uint32_t to = static_cast<uint32_t>(t[1]);
+    const uint32_t bits = static_cast<uint32_t>(t[0]) | to;        // of the first 64 segments, the same for every wave
     uint64_t len[kRun];
 #pragma unroll
     for (uint32_t r = 0; r < kRun; ++r) {
@@ -1458,7 +1464,14 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
         return;
     }
     constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kWindowUnits) * kUnitBytes;
-    const uint32_t period = static_cast<uint32_t>(pace.windowTicks * (waves * kDeepBytes) >> 26);
+    // Whether the first segments are written one behind the other, which leaves the rows of HBM open: they hold a higher rate.
+    const uint32_t sample = nseg < 64 ? nseg : 64;
+    const uint32_t follow = __popcll(__ballot(lane + 1 < sample && __shfl_down(to, 1, 64) - to == static_cast<uint32_t>(len0)));
+    const uint32_t windowTicks = each == 0                       ? pace.windowTicks
+                                 : follow * 4 >= (sample - 1) * 3 ? pace.orderedTicks
+                                 : len0 >= kWindowLongBlockBytes  ? pace.longTicks
+                                                                  : pace.windowTicks;
+    const uint32_t period = static_cast<uint32_t>(windowTicks * (waves * kDeepBytes) >> 26);
     const uint32_t hold = (each != 0 ? pace.equalTicks : pace.holdTicks) +
                           static_cast<uint32_t>(static_cast<uint64_t>(each != 0 ? pace.equalMoreTicks : pace.holdMoreTicks) * total >> 14);
     uint64_t loadAt = paced ? AgreedStart(pace.seq) + static_cast<uint64_t>(item) * (period / 2) / waves : 0;
@@ -2079,6 +2092,8 @@ extern "C" int mfk_xcopy_planned(const void *triples, uint32_t nseg, uint32_t ho
                          TicksOf(equalNanos, khz),
                          TicksOf(holdMoreNanos != 0 ? holdMoreNanos + kTableEqualMoreNanos - kTableHoldMoreNanos : 0, khz),
                          WindowPeriodTicksAt(2ull << 26, windowMBps, khz),
+                         WindowPeriodTicksAt(2ull << 26, windowMBps / 15 * 16, khz),
+                         WindowPeriodTicksAt(2ull << 26, windowMBps / 20 * 22, khz),
                          NextWindowSeq()};
     const int err = nseg <= 64 * kPlannedShortRun
                         ? Launch(XcopyPlannedKernel<1, kPlannedShortRun>, kWindowWaves, 64, PlannedLds(1, nseg), s, At(triples), nseg, pace)

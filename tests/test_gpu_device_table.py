@@ -168,3 +168,22 @@ def test_tables_that_their_launch_plans(gpu, kind):
     for s, d, l in zip(at, place, lens):
         expect[d:d + l] = data[s:s + l]
     assert np.array_equal(target.cpu().numpy(), expect)
+
+
+@pytest.mark.parametrize("count,size", [(2049, 32768), (1025, 65536), (513, 163840), (64, 1 << 21)])
+@pytest.mark.parametrize("ordered", [True, False])
+def test_windowed_tables_of_pages_in_order_and_not(gpu, count, size, ordered):
+    """Just beyond what is held: the rates of pages that are written one behind the other, and of long ones that are not."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(count)
+    at = rng.permutation(2 * count)[:count].astype(np.int64) * size
+    place = (np.arange(count, dtype=np.int64) if ordered else rng.permutation(count)) * size
+    source = torch.randint(-2**63, 2**63 - 1, (2 * count * size // 8,), dtype=torch.int64, device="cuda").view(torch.uint8)
+    target = torch.zeros(count * size, dtype=torch.uint8, device="cuda")
+    table = torch.from_numpy(np.stack([source.data_ptr() + at, target.data_ptr() + place, np.full(count, size)], axis=1)).cuda()
+    torch.cuda.synchronize()
+    assert gpu.mf_xcopy_device_table(table.data_ptr(), count, native.ROUTE_HBM, None) == 0, native.last_error()
+    assert gpu.mfrt_device_sync() == 0
+    index = torch.from_numpy(at // size).cuda()
+    to = torch.from_numpy(place // size).cuda()
+    assert torch.equal(target.view(count, size)[to], source.view(2 * count, size)[index])
