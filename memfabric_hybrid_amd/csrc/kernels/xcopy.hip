@@ -1143,7 +1143,8 @@ struct TablePace {
     uint32_t equalTicks;        // the same where its segments are of one length, whose descriptors are there sooner
     uint32_t equalMoreTicks;
     uint32_t windowTicks;       // period in which 64 MiB pass at the rate of random blocks,
-    uint32_t longTicks;         // of such of one length, kWindowLongBlockBytes or more,
+    uint32_t shortTicks;        // of such of one length below kWindowLongBlockBytes, whose write part is the longer one,
+    uint32_t longTicks;         // of such of one length from there on,
     uint32_t orderedTicks;      // and of blocks of one length that are written one behind the other
     uint32_t seq;               // of AgreedStart
 };
@@ -1332,6 +1333,9 @@ __device__ __forceinline__ bool PlannedQuad(const uint64_t *__restrict__ triples
 // In windows cut for 6.0 / 6.2 / 6.4 / 6.6 / 6.8 TB/s, the same to 0.5 in four processes: 4096 pages of 32 KiB gathered 49.8 / 48.4 / 47.1 / 46.0 / 45.3,
 // scattered 50.2 / 51.2 / 54 / 54 / 54; of 64 KiB gathered 94.5 / 91.7 / 89.4 / 87.3 / 85.7 (7.0: 91), scattered 95.0 / 92.8 / 90.5 / 87.8 / 97 to 102;
 // 1000 of 256 KiB scattered 92.0 / 89.6 / 87.1 / 85.2 / 86.7 to 91.6: 6.6 for what is written in order, 6.4 for scattered pages of 64 KiB and more.
+// Shorter ones are stored at random places no faster than 5.6, but read faster: with a read part of 0.40 / 0.44 / 0.47 / 0.50 / 0.53 of the period, 4096
+// of 32 KiB at 6.0 50.6 / 50.1 / 50.2 / 50.1 / 51.5, at 6.2 50.5 / 48.9 / 48.9 / 49.8 / 53.8, at 6.4 51.6 / 48.7 / 48.8 / 53.2 / 54.7; so 29/64 at 6.3, 47.9.  The others
+// gain nothing from uneven parts.
 template <uint32_t kWaves, uint32_t kRun>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
@@ -1467,15 +1471,16 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
     // Whether the first segments are written one behind the other, which leaves the rows of HBM open: they hold a higher rate.
     const uint32_t sample = nseg < 64 ? nseg : 64;
     const uint32_t follow = __popcll(__ballot(lane + 1 < sample && __shfl_down(to, 1, 64) - to == static_cast<uint32_t>(len0)));
-    const uint32_t windowTicks = each == 0                       ? pace.windowTicks
-                                 : follow * 4 >= (sample - 1) * 3 ? pace.orderedTicks
-                                 : len0 >= kWindowLongBlockBytes  ? pace.longTicks
-                                                                  : pace.windowTicks;
+    const bool inOrder = each != 0 && follow * 4 >= (sample - 1) * 3;
+    const bool shortPages = each != 0 && !inOrder && len0 < kWindowLongBlockBytes;
+    const uint32_t windowTicks = each == 0 ? pace.windowTicks : inOrder ? pace.orderedTicks : shortPages ? pace.shortTicks : pace.longTicks;
     const uint32_t period = static_cast<uint32_t>(windowTicks * (waves * kDeepBytes) >> 26);
+    const uint32_t reading = shortPages ? period / 64 * 29 : period / 2;
     const uint32_t hold = (each != 0 ? pace.equalTicks : pace.holdTicks) +
                           static_cast<uint32_t>(static_cast<uint64_t>(each != 0 ? pace.equalMoreTicks : pace.holdMoreTicks) * total >> 14);
-    uint64_t loadAt = paced ? AgreedStart(pace.seq) + static_cast<uint64_t>(item) * (period / 2) / waves : 0;
-    uint64_t storeAt = paced ? loadAt + period / 2 : held && pace.holdTicks != 0 ? t0 + hold : 0;
+    const uint64_t start = paced ? AgreedStart(pace.seq) : 0;
+    uint64_t loadAt = paced ? start + static_cast<uint64_t>(item) * reading / waves : 0;
+    uint64_t storeAt = paced ? start + reading + static_cast<uint64_t>(item) * (period - reading) / waves : held && pace.holdTicks != 0 ? t0 + hold : 0;
     const uint32_t step = paced ? period : 0;
     // (Each owner with a loop of its own: code that a wave only steps over is fetched all the same, at 0.3 us.)
     auto deepChunks = [&](auto owner) {
@@ -2092,6 +2097,7 @@ extern "C" int mfk_xcopy_planned(const void *triples, uint32_t nseg, uint32_t ho
                          TicksOf(equalNanos, khz),
                          TicksOf(holdMoreNanos != 0 ? holdMoreNanos + kTableEqualMoreNanos - kTableHoldMoreNanos : 0, khz),
                          WindowPeriodTicksAt(2ull << 26, windowMBps, khz),
+                         WindowPeriodTicksAt(2ull << 26, windowMBps / 20 * 21, khz),
                          WindowPeriodTicksAt(2ull << 26, windowMBps / 15 * 16, khz),
                          WindowPeriodTicksAt(2ull << 26, windowMBps / 20 * 22, khz),
                          NextWindowSeq()};
