@@ -1813,8 +1813,10 @@ uint32_t XcopyEngine::PieceUnits(const BatchStats &stats, uint32_t n, bool unord
 }
 
 // Of 6.0 TB/s, which blocks at random places hold; of 6.4 for such of one length from 64 KiB on; of 6.6 for long ones that are written one
-// behind the other, which leaves the rows of HBM open (short ones hold that in some places of the pool only, and gain nothing at 6.0: 16 384
-// pages of 32 KiB gathered 182 us without windows, 171 to 194 at 6.4, 181 at 6.0).  At 6.0 / 6.2 / 6.4 / 6.6 / 6.8, the same to 1 % in four
+// behind the other, which leaves the rows of HBM open (short ones hold that in some places of the pool only: from
+// kOrderedWindowPieces on 6.0, where two held launches or none are slower; without windows / at 6.0 / at 6.4, back to back 10 000 of 48 KiB 170.6 / 167.2 / -,
+// 16 384 of 32 KiB 186 / 182 / 179 to 185, of 16 KiB 94.3 / 92.1 / 91 to 95, alone 258 / 248 / 238 and 148 / 143 / 138; 7300 and 8192 of 32 KiB 82 / 83 / -, 92 /
+// 92 / -).  At 6.0 / 6.2 / 6.4 / 6.6 / 6.8, the same to 1 % in four
 // processes: 64 KiB gathered, 2048 47.6 / 46.3 / 44.9 / 43.7 / 44.1, 16 000 355 / 344 / 333 / 328 / 350; scattered, 4096 92.6 / 90.0 / 87.7 / 86.0 / 96, 16 000
 // 355 / 344 / 345 / 375 / 402; 2000 of 128 KiB gathered and scattered 90.7 / 87.8 / 85.4 / 83.3 / 85.  Pieces that are much less than full gain
 // nothing; segments between cache lines keep the launch without windows, as they do in launches of kInlineSegs segments up to
@@ -1827,10 +1829,14 @@ uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *d
         !WindowsApply(stats.total, MFRT_ROUTE_HBM, kPieceWindowMinBytes)) {
         return 0;
     }
+    constexpr uint64_t kOrderedWindowPieces = 16384;
+    const bool equal = stats.total == stats.longest * n;
     if (WrittenInOrder(dst, len, n)) {
-        return stats.total / n >= kWindowLongBlockBytes ? tuning_.windowMBps / 34 * 33 : 0;
+        return stats.total / n >= kWindowLongBlockBytes             ? tuning_.windowMBps / 34 * 33
+               : equal && stats.deepPieces >= kOrderedWindowPieces ? tuning_.windowMBps / 17 * 15
+                                                                    : 0;
     }
-    const bool longBlocks = stats.longest >= kWindowLongBlockBytes && stats.total == stats.longest * n;
+    const bool longBlocks = stats.longest >= kWindowLongBlockBytes && equal;
     return tuning_.windowMBps / 17 * (longBlocks ? 16 : 15);
 }
 
