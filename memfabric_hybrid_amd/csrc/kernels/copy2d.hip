@@ -98,7 +98,8 @@ __global__ __launch_bounds__(kRectThreads) void Copy2dKernel(const RectPlan p)
 // 20 000 bytes, 400 MB 147 to 197 / 129 to 190 / 126 to 201: those go without windows.  Below 32 MiB whole rows are as fast or faster (24 MB
 // 9.0 to 9.5 / 11.2 to 11.6 / 10.1 to 10.7).
 // kPaced: sixteen loads per lane at the wave's offset into the read half of the period, the stores at the same offset into the
-// write half, as XcopyWindowKernel does for long segments.  Rates of 7.1 TB/s and more fall apart for half of these geometries.
+// write half, as XcopyWindowKernel does for long segments.  Rates of 7.1 TB/s and more fall apart for half of these geometries;
+// uneven parts lose (a read part of 0.42 / 0.45 / 0.475 / 0.5 / 0.525 / 0.55 / 0.58 of a period at 7.0, 161 MB 56.2 / 54.5 / 51.4 / 50.8 / 51.0 / 54.1 / 59.4).
 template <bool kPaced>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPaced ? 5 : 8))) void Copy2dChunkKernel(const RectChunkPlan p, uint32_t groups,
                                                                                                         uint32_t period, uint32_t seq)
