@@ -1180,14 +1180,13 @@ __global__ __launch_bounds__(kThreads) void MoeCombineKernel(uint64_t rowsIn, ui
 // keeps the result, 8 registers per item; in the write part it stores the kItems results at
 // its own offset of that part (top-6: six rows, twelve pieces).  The start of the first period is agreed through
 // AgreedStart(); after that every wave goes by the constant-rate clock alone.  8192 tokens of 7168
-// elements at top-8: 164-168 us against 177-181 us for one workgroup per item; from about six items per
-// wave on it is the faster form.  Read parts are paced at 6.8 TB/s, write parts at 6.2 (reads at 7.0
+// elements at top-8: 164-168 us against 177-181 us for one workgroup per item.  Read parts are paced at 6.8 TB/s, write parts at 6.2 (reads at 7.0
 // make the waves fall behind now and then).
 // Arithmetic and the rule for slots without a row are MoeCombineKernel's.
 constexpr uint32_t kCombineItems = 4;                  // 32 result registers, 116 in all: sixteen waves per CU
 constexpr uint32_t kCombineWavesPerCu = 16;
 constexpr uint32_t kCombineSliceUnits = 128;           // two column positions per lane
-constexpr uint32_t kCombineMinItemsPerWave = 6;
+constexpr uint32_t kCombineMinItemsPerWave = 3;
 
 template <uint32_t kItems, uint32_t kSlots>
 __global__ __launch_bounds__(64) void MoeCombineWindowKernel(const u32x4 *__restrict__ rowsIn,
@@ -1502,17 +1501,20 @@ extern "C" int mfk_moe_combine(const void *rows, const void *rowOf, const void *
         const uint32_t perPart = (upr + parts - 1) / parts;
         const uint64_t items = static_cast<uint64_t>(tokens) * parts;
         const uint32_t waves = static_cast<uint32_t>(mfrt_cu_count() > 0 ? mfrt_cu_count() : 256) * kCombineWavesPerCu;
-        // From six items per wave on, waves that stay and keep reads and writes apart in time; below that the
-        // first read part and the last write part, in which the chip only reads or only writes for want of
-        // work, cost what the separation gains (top-8, 16 800 items on 4096 waves: 51.4 against 50.5 us; 19 200: the
-        // same; 25 200: 74.4 against 76.7 us).
+        // Waves that stay and keep reads and writes apart in time, for rows that come from HBM: more than a dispatch leaves in the
+        // last-level cache (kCountBytes), or dispatched by the tiles, whose stores pass it.  us of the combine / of dispatch and combine, one workgroup per
+        // item and so: top-8, 3.6 items per wave (2106 x 7168) 46.6, 107.4 / 44.2, 104.6; 4 (8192 x 2048) 51.8, 110.9 / 48.5, 107.2; 4.3 (4403 x 4096) 55.5,
+        // 123.7 / 54.1, 121.7; 5.8 (5939 x 4096) 74.5, 159.5 / 71.6, 156.3; top-6, 3.6 (2106 x 7168) 35.8, 72.4 / 35.3, 69.3; 5 (2925) 49.8, 106.2 / 50.9,
+        // 106.5.  Rows in the cache want no windows: 1872 x 7168 at top-8 75.0 and 78.4, at top-6 59.7 and 62.8.
         const uint32_t readTicks = WindowPeriodTicks(static_cast<uint64_t>(waves) * topK * perPart * 16,
                                                      g_combineReadMBps.load(std::memory_order_relaxed));
         const uint32_t writeTicks = WindowPeriodTicks(static_cast<uint64_t>(waves) * kCombineItems * perPart * 16,
                                                       g_combineWriteMBps.load(std::memory_order_relaxed));
         // Top-6 gains as top-8 does (8192 x 7168: 131-133 against 138-140 us); top-4 gains nothing (98 against 97 us)
         // and top-2 loses (16 384 x 4096: 79 against 66 us): their read parts are too short for the switch to pay.
-        const bool windows = paced != 0 && topK >= 6 && items >= static_cast<uint64_t>(waves) * kCombineMinItemsPerWave &&
+        const uint64_t entries = static_cast<uint64_t>(tokens) * topK;
+        const bool fromHbm = entries > kCountEntries || (entries + tokens) * upr * 16 > kCountBytes;
+        const bool windows = paced != 0 && topK >= 6 && fromHbm && items >= static_cast<uint64_t>(waves) * kCombineMinItemsPerWave &&
                              items < 0x40000000ull && readTicks != 0 && writeTicks != 0;
         const uint32_t grid = windows ? waves : tokens * parts;
 #define MF_COMBINE_SLICES(K)                                                                                           \

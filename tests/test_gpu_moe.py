@@ -317,6 +317,16 @@ def test_combine_of_rows_that_differ_within_a_token(gpu, oracle, T, H, K):
             b.free()
 
 
+@pytest.mark.parametrize("T,H,K", [
+    (2080, 7168, 8),   # the most rows that a dispatch leaves in the last-level cache
+    (2081, 7168, 8),   # one token more: one period of three read parts and a part of the fourth
+    (6145, 2048, 8),   # the fewest entries beyond the dispatch that counts, three items per wave and two more
+    (2700, 7168, 6),
+])
+def test_combine_where_its_waves_begin_to_stay(gpu, oracle, T, H, K):
+    test_combine_of_rows_that_differ_within_a_token(gpu, oracle, T, H, K)
+
+
 def test_same_workspace_reused_by_calls_of_different_sizes(gpu, oracle):
     """Histograms and status of one call must not leak into the next call on the same workspace."""
     E, K, H = 64, 4, 64
