@@ -844,14 +844,20 @@ constexpr uint32_t CountLdsWords(uint32_t experts, uint32_t ownMost)
 // from taking turns with them (2400 of 7168 at top-2: dispatch 19.4, 25.9 without; before kCountNearBytes the longer code
 // costs 0.5).  Calls of few slots read most: from kCountDeepBytes on plain stores cost them more than the next kernel
 // gains (4096 of 7168 at top-2, dispatch / both: nontemporal 28.6 / 57.4, plain 36.5 / 56.0).
-// What does not fit the last-level cache (256 MiB) goes to the tiles: 8192 of 2048 at top-8 57 us, 61 to 63 with this.  Below that
-// the tiles may be the quicker dispatch, but not the quicker pair: 2000 of 7168 at top-8 47.0 / 91.1, with this 51.1 / 80.0; 1500 37.5 / 70.6
-// and 39.1 / 61.3.  Rows that are not whole cache lines are always stored plainly: two waves share a line.
+// What fits the last-level cache (256 MiB) too little goes to the tiles: they are the quicker dispatch from about 280 MiB on, but as long as the next kernel
+// finds a part of the rows in the cache not the quicker pair.  Dispatch / both with the tiles and so, us, three sets of buffers in turn: top-8 over 256 experts,
+// 262 MiB 61.4 / 105.6, 54.1 / 85.0; 310 64.7 / 118.2, 64.7 / 102.4; 350 66.8 / 127.2, 75.5 / 118.7; 400 84.8 / 153.1, 86.7 / 138.8; 450 85.0 / 161.6, 98.9 / 161.1; 500
+// 91.6 / 173.6, 109.7 / 183.9.  Top-6 310 56.6 / 110.9, 66.1 / 101.1; 350 66.2 / 126.9, 76.7 / 118.6; 400 75.0 / 143.2, 88.8 / 143.5.  Top-4 310 59.4 / 113.2, 54.6 /
+// 108.1; 350 61.4 / 122.5, 61.2 / 121.9; 450 88.0 / 165.6, 100.7 / 180.9.  Top-2 230 45.7 / 84.7, 38.5 / 77.6; 262 59.0 / 102.9, 57.1 / 102.2; 280 61.8 / 108.4,
+// 60.4 / 109.4.  Rows that are not whole cache lines are always stored plainly: two waves share a line.
 constexpr uint64_t kQuickBytes = 24ull << 20;            // also of the dispatch above
 constexpr uint64_t kQuickFewBytes = 16ull << 20;         // with up to two slots, whose next kernel reads the rows sooner
 constexpr uint64_t kCountNearBytes = 96ull << 20;
 constexpr uint64_t kCountDeepBytes = 150ull << 20;
-constexpr uint64_t kCountBytes = 256ull << 20;
+constexpr uint64_t CountBytes(uint32_t topK, bool lines)
+{
+    return (topK <= 2 || !lines ? 256ull : topK <= 4 ? 336ull : topK <= 6 ? 368ull : 432ull) << 20;
+}
 
 template <bool kNt>
 __device__ __forceinline__ u32x4 RowLoad(const MF_GLOBAL u32x4 *p)
@@ -1370,7 +1376,7 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
         }
 #undef MF_DISPATCH_SMALL
     }
-    if (total <= kCountEntries && moved <= kCountBytes) {   // where the lines lie: see those
+    if (total <= kCountEntries && moved <= CountBytes(topK, lines)) {   // where the lines lie: see those
         const uint32_t cus = static_cast<uint32_t>(mfrt_cu_count() > 0 ? mfrt_cu_count() : 256);
         const uint32_t most = cus < kCountLeastGroups ? kCountLeastGroups : cus;
         const uint32_t perGroup = (tokens + most - 1) / most;
@@ -1502,10 +1508,10 @@ extern "C" int mfk_moe_combine(const void *rows, const void *rowOf, const void *
         const uint64_t items = static_cast<uint64_t>(tokens) * parts;
         const uint32_t waves = static_cast<uint32_t>(mfrt_cu_count() > 0 ? mfrt_cu_count() : 256) * kCombineWavesPerCu;
         // Waves that stay and keep reads and writes apart in time, for rows that come from HBM: more than a dispatch leaves in the
-        // last-level cache (kCountBytes), or dispatched by the tiles, whose stores pass it.  us of the combine / of dispatch and combine, one workgroup per
-        // item and so: top-8, 3.6 items per wave (2106 x 7168) 46.6, 107.4 / 44.2, 104.6; 4 (8192 x 2048) 51.8, 110.9 / 48.5, 107.2; 4.3 (4403 x 4096) 55.5,
-        // 123.7 / 54.1, 121.7; 5.8 (5939 x 4096) 74.5, 159.5 / 71.6, 156.3; top-6, 3.6 (2106 x 7168) 35.8, 72.4 / 35.3, 69.3; 5 (2925) 49.8, 106.2 / 50.9,
-        // 106.5.  Rows in the cache want no windows: 1872 x 7168 at top-8 75.0 and 78.4, at top-6 59.7 and 62.8.
+        // last-level cache (CountBytes), or dispatched by the tiles, whose stores pass it.  us of dispatch and combine, one workgroup per item and so: top-8, 3
+        // to 4 items per wave (6600 / 8192 x 2048) 94.6 / 92.4, 110.1 / 106.5; 7 (4063 x 7168) 179.4 / 173.6; top-6, 5.9 (6000 x 4096) 122.4 / 121.0; 8 (4702 x 7168)
+        // 154.4 / 150.0.  Rows in the cache want no windows, at top-8 3.6 items per wave (2129 x 7168) 85.0 / 87.8, 5.6 (3250) 138.8 / 144.1, at top-6 6.3 (3657)
+        // 118.6 / 120.3.
         const uint32_t readTicks = WindowPeriodTicks(static_cast<uint64_t>(waves) * topK * perPart * 16,
                                                      g_combineReadMBps.load(std::memory_order_relaxed));
         const uint32_t writeTicks = WindowPeriodTicks(static_cast<uint64_t>(waves) * kCombineItems * perPart * 16,
@@ -1513,7 +1519,7 @@ extern "C" int mfk_moe_combine(const void *rows, const void *rowOf, const void *
         // Top-6 gains as top-8 does (8192 x 7168: 131-133 against 138-140 us); top-4 gains nothing (98 against 97 us)
         // and top-2 loses (16 384 x 4096: 79 against 66 us): their read parts are too short for the switch to pay.
         const uint64_t entries = static_cast<uint64_t>(tokens) * topK;
-        const bool fromHbm = entries > kCountEntries || (entries + tokens) * upr * 16 > kCountBytes;
+        const bool fromHbm = entries > kCountEntries || (entries + tokens) * upr * 16 > CountBytes(topK, hidden % 64 == 0);
         const bool windows = paced != 0 && topK >= 6 && fromHbm && items >= static_cast<uint64_t>(waves) * kCombineMinItemsPerWave &&
                              items < 0x40000000ull && readTicks != 0 && writeTicks != 0;
         const uint32_t grid = windows ? waves : tokens * parts;

@@ -492,6 +492,15 @@ def test_dispatch_that_counts_in_one_launch(gpu, T, H, K, E):
             _free(bufs)
 
 
+@pytest.mark.parametrize("T,H,K,E", [
+    (3510, 7168, 8, 256), (3511, 7168, 8, 256), (6144, 4096, 8, 64),    # at top-8, the most rows for the dispatch that counts, and a token more
+    (3845, 7168, 6, 64), (3846, 7168, 6, 64), (4915, 7168, 4, 8), (4916, 7168, 4, 8),
+    (6241, 7168, 2, 8), (6242, 7168, 2, 8),
+])
+def test_dispatch_where_the_tiles_begin(gpu, T, H, K, E):
+    test_dispatch_that_counts_in_one_launch(gpu, T, H, K, E)
+
+
 @pytest.mark.parametrize("T,H,K", [
     (1, 7168, 8), (3, 2048, 2), (33, 2056, 4),           # few entries: one column position per lane, rows of 256 and 257 units
     (512, 2048, 8), (513, 2048, 8),                      # the last call of 4096 entries and one beyond
