@@ -1912,7 +1912,7 @@ void XcopyEngine::TablePaceFor(uint32_t &holdNanos, uint32_t &holdMoreNanos, uin
 bool XcopyEngine::DeepHoldApplies(uint64_t bytes, uint32_t n, int route, bool unordered) const
 {
     return route == MFRT_ROUTE_HBM && !unordered && tuning_.holdNanos != 0 && tuning_.unitsOverride == 0 && tuning_.deepHold &&
-           bytes > kDeepMinBytes && n != 0 && bytes <= (n == 1 ? kHeldSingleBytes : kDeepMaxBytes) && bytes / n >= kDeepMinSegmentBytes &&
+           bytes > kDeepMinBytes && n != 0 && bytes <= (n == 1 && !tuning_.holdCalibratedOff ? kHeldSingleBytes : kDeepMaxBytes) && bytes / n >= kDeepMinSegmentBytes &&
            g_leasesOut.load(std::memory_order_relaxed) <= 1;
 }
 

@@ -444,8 +444,8 @@ __device__ __forceinline__ void CopyChunkHeld(uint64_t src, uint64_t dst, uint64
 
 // The inline plan (chunks of kWindowUnits units) copied by gridDim.x single-wave workgroups that walk
 // the chunks with stride gridDim.x, one chunk per period each.
-template <bool kNtLoad, int kStore>
-__global__ __launch_bounds__(64) void XcopyWindowKernel(const InlinePlan p, uint32_t period, uint32_t seq, uint32_t onLines)
+template <bool kNtLoad, int kStore, bool kOnLines>
+__global__ __launch_bounds__(64) void XcopyWindowKernel(const InlinePlan p, uint32_t period, uint32_t seq)
 {
     const InlineRows rows(p);
     const uint32_t nchunk = p.nchunk;
@@ -453,7 +453,7 @@ __global__ __launch_bounds__(64) void XcopyWindowKernel(const InlinePlan p, uint
     uint64_t slot = AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * half / gridDim.x;
     for (uint32_t c = blockIdx.x; c < nchunk; c += gridDim.x) {
         const InlineChunk r = rows.Owner(c);
-        const SegChunk m = ChunkOn(onLines != 0, r.src, r.dst, r.len, r.k, kWindowUnits);
+        const SegChunk m = ChunkOn(kOnLines, r.src, r.dst, r.len, r.k, kWindowUnits);
         CopyChunkWindowed<kNtLoad, kStore>(m.src, m.dst, m.len, m.k, slot, half);
         slot += period;
     }
@@ -1812,13 +1812,14 @@ bool CutOnLines(const InlinePlan &plan, InlinePlan &lines)
 
 // windowMBps: the rate (MB/s of HBM traffic, read + written) the period of a windowed launch is cut for.
 template <bool kNtLoad, int kStore>
-int LaunchWindowed(const InlinePlan &plan, uint32_t grid, uint32_t onLines, uint32_t windowMBps, hipStream_t stream)
+int LaunchWindowed(const InlinePlan &plan, uint32_t grid, bool onLines, uint32_t windowMBps, hipStream_t stream)
 {
     const uint32_t ticks = WindowPeriodTicks(2ull * grid * kWindowUnits * kUnitBytes, windowMBps);
     if (ticks == 0) {
         return static_cast<int>(hipErrorInvalidValue);
     }
-    hipLaunchKernelGGL((XcopyWindowKernel<kNtLoad, kStore>), dim3(grid), dim3(64), 0, stream, plan, ticks, NextWindowSeq(), onLines);
+    const auto kernel = onLines ? XcopyWindowKernel<kNtLoad, kStore, true> : XcopyWindowKernel<kNtLoad, kStore, false>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, stream, plan, ticks, NextWindowSeq());
     return static_cast<int>(hipGetLastError());
 }
 
@@ -1948,7 +1949,7 @@ extern "C" int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, v
     const mf::InlinePlan &plan = onLines ? lines : given;
     const uint32_t grid = mf::WindowGrid(plan.nchunk, mf::kWindowWaves);
     const int err = mf::WithPolicy(mf::PolicyOf(MFRT_ROUTE_HBM), [&](auto ntLoad, auto store) {
-        return mf::LaunchWindowed<decltype(ntLoad)::value, decltype(store)::value>(plan, grid, onLines ? 1 : 0, windowMBps, s);
+        return mf::LaunchWindowed<decltype(ntLoad)::value, decltype(store)::value>(plan, grid, onLines, windowMBps, s);
     });
     return err != 0 ? err : mf::Signal(mask, maskValue, s);
 }
@@ -2154,7 +2155,8 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
                 (void)Launch(XcopyPieceWindowKernel, 1, 64, 0, s, 0, 0u, 64u, NextWindowSeq(), 1u, 0u, 0);
                 (void)Launch(XcopyPlannedKernel<1, kPlannedShortRun>, 1, 64, 64, s, 0, 0u, TablePace{});
                 (void)Launch(XcopyPlannedKernel<kPlannedWaves, kPlannedRun>, 1, 64 * kPlannedWaves, 64, s, 0, 0u, TablePace{});
-                hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq(), 0u);
+                hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt, false>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
+                hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt, true>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
             }
             return 0;
         });
@@ -2280,7 +2282,7 @@ extern "C" int mfk_xcopy_calibrate(void *stream, const uint32_t *holdNanos, cons
                 big.units = kWindowUnits;
                 big.nchunk = static_cast<uint32_t>(half / (kWindowUnits * kUnitBytes));
                 const uint32_t rate = windowMBps[v - 1];
-                err = timed([&](int) { (void)LaunchWindowed<true, kStoreStream>(big, kWindowWaves, 0, rate, s); }, round == 0 ? 1 : 0, 1,
+                err = timed([&](int) { (void)LaunchWindowed<true, kStoreStream>(big, kWindowWaves, false, rate, s); }, round == 0 ? 1 : 0, 1,
                             out[4 + v]);
             }
             if (err != hipSuccess) {
