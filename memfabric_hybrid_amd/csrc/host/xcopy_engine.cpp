@@ -1816,7 +1816,8 @@ uint32_t XcopyEngine::PieceUnits(const BatchStats &stats, uint32_t n, bool unord
 }
 
 // Of 6.0 TB/s, which blocks at random places hold; of 6.4 for such of one length from 64 KiB on; of 6.6 for long ones that are written one
-// behind the other, which leaves the rows of HBM open (short ones hold that in some places of the pool only: from
+// behind the other, which leaves the rows of HBM open, up to kOrderedFastBytes, beyond which not every launch holds that (16 384 of 64 KiB 338 to 352 us, at
+// 6.4 340, 12 000 248 to 252 and 253 to 256), so 6.4 (short ones hold that in some places of the pool only: from
 // kOrderedWindowPieces on 6.0, where two held launches or none are slower; without windows / at 6.0 / at 6.4, back to back 10 000 of 48 KiB 170.6 / 167.2 / -,
 // 16 384 of 32 KiB 186 / 182 / 179 to 185, of 16 KiB 94.3 / 92.1 / 91 to 95, alone 258 / 248 / 238 and 148 / 143 / 138; 7300 and 8192 of 32 KiB 82 / 83 / -, 92 /
 // 92 / -).  At 6.0 / 6.2 / 6.4 / 6.6 / 6.8, the same to 1 % in four
@@ -1833,9 +1834,10 @@ uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *d
         return 0;
     }
     constexpr uint64_t kOrderedWindowPieces = 16384;
+    constexpr uint64_t kOrderedFastBytes = 800ull << 20;
     const bool equal = stats.total == stats.longest * n;
     if (WrittenInOrder(dst, len, n)) {
-        return stats.total / n >= kWindowLongBlockBytes             ? tuning_.windowMBps / 34 * 33
+        return stats.total / n >= kWindowLongBlockBytes             ? tuning_.windowMBps / 34 * (stats.total < kOrderedFastBytes ? 33 : 32)
                : equal && stats.deepPieces >= kOrderedWindowPieces ? tuning_.windowMBps / 17 * 15
                                                                     : 0;
     }
