@@ -1815,16 +1815,18 @@ uint32_t XcopyEngine::PieceUnits(const BatchStats &stats, uint32_t n, bool unord
     return mean <= 6144 ? kXcopyThreads : mean <= 12288 ? kDeepUnits / 2 : kDeepUnits;
 }
 
-// Of 6.0 TB/s, which blocks at random places hold; of 6.4 for such of one length from 64 KiB on; of 6.6 for long ones that are written one
-// behind the other, which leaves the rows of HBM open, up to kOrderedFastBytes, beyond which not every launch holds that (16 384 of 64 KiB 338 to 352 us, at
-// 6.4 340, 12 000 248 to 252 and 253 to 256), so 6.4 (short ones hold that in some places of the pool only: from
-// kOrderedWindowPieces on 6.0, where two held launches or none are slower; without windows / at 6.0 / at 6.4, back to back 10 000 of 48 KiB 170.6 / 167.2 / -,
-// 16 384 of 32 KiB 186 / 182 / 179 to 185, of 16 KiB 94.3 / 92.1 / 91 to 95, alone 258 / 248 / 238 and 148 / 143 / 138; 7300 and 8192 of 32 KiB 82 / 83 / -, 92 /
-// 92 / -).  At 6.0 / 6.2 / 6.4 / 6.6 / 6.8, the same to 1 % in four
-// processes: 64 KiB gathered, 2048 47.6 / 46.3 / 44.9 / 43.7 / 44.1, 16 000 355 / 344 / 333 / 328 / 350; scattered, 4096 92.6 / 90.0 / 87.7 / 86.0 / 96, 16 000
-// 355 / 344 / 345 / 375 / 402; 2000 of 128 KiB gathered and scattered 90.7 / 87.8 / 85.4 / 83.3 / 85.  Pieces that are much less than full gain
-// nothing; segments between cache lines keep the launch without windows, as they do in launches of kInlineSegs segments up to
-// kWindowSliceMinSegmentBytes.
+// Of 6.0 TB/s, which blocks at random places hold.  Blocks that begin and end on multiples of kWindowLongBlockBytes hold more: 6.4 where they
+// have one length, and 6.6 where they are written one behind the other, which leaves the rows of HBM open, up to kOrderedFastBytes, beyond which
+// not every launch holds that (8000 of 64 KiB 168 to 173 us, at 6.4 169; 16 384 345 to 355 and 345 to 349).  At 6.0 / 6.2 / 6.4 / 6.6 / 6.8, the same to 1 % in
+// four processes: 64 KiB gathered, 2048 47.6 / 46.3 / 44.9 / 43.7 / 44.1; scattered, 4096 92.6 / 90.0 / 87.7 / 86.0 / 96; 2000 of 128 KiB gathered and
+// scattered 90.7 / 87.8 / 85.4 / 83.3 / 85.  Elsewhere those rates fall apart.  300 and 700 MB at random places on both sides, at 6.0 / 6.4: 65 536 bytes at
+// multiples of 64 KiB 104.5 / 102.2, 238.7 / 235.3, at multiples of 4 KiB or 256 105.7 / 112.5, 246 / 275; 81 920 106.3 / 113.5, 247 / 277; 90 112 109.0 / 119.5,
+// 270 / 282; 110 776 107.1 / 117.5, 253 / 279; 163 840 240 / 249.  Written in order at 6.4 / 6.6: 73 728 100.7 / 106.8, 110 720 100.7 / 102.4, 81 920 98.4 / 96.6, but 226 / 232
+// at 700 MB; those stay at 6.4.  Short blocks in order hold 6.4 in some places of the pool only: from kOrderedWindowPieces on 6.0, where two held
+// launches or none are slower; without windows / at 6.0 / at 6.4, back to back 10 000 of 48 KiB 170.6 / 167.2 / -, 16 384 of 32 KiB 186 / 182 / 179 to
+// 185, of 16 KiB 94.3 / 92.1 / 91 to 95, alone 258 / 248 / 238 and 148 / 143 / 138; 7300 and 8192 of 32 KiB 82 / 83 / -, 92 / 92 / -.  Pieces that are
+// much less than full gain nothing; segments between cache lines keep the launch without windows, as they do in launches of
+// kInlineSegs segments up to kWindowSliceMinSegmentBytes.
 uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t count, uint32_t units,
                                       bool unordered) const
 {
@@ -1834,15 +1836,15 @@ uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *d
         return 0;
     }
     constexpr uint64_t kOrderedWindowPieces = 16384;
-    constexpr uint64_t kOrderedFastBytes = 800ull << 20;
+    constexpr uint64_t kOrderedFastBytes = 400ull << 20;
     const bool equal = stats.total == stats.longest * n;
+    const bool onGrid = ((stats.addressBits | stats.lengthBits) & (kWindowLongBlockBytes - 1)) == 0;
     if (WrittenInOrder(dst, len, n)) {
-        return stats.total / n >= kWindowLongBlockBytes             ? tuning_.windowMBps / 34 * (stats.total < kOrderedFastBytes ? 33 : 32)
+        return stats.total / n >= kWindowLongBlockBytes             ? tuning_.windowMBps / 34 * (onGrid && stats.total < kOrderedFastBytes ? 33 : 32)
                : equal && stats.deepPieces >= kOrderedWindowPieces ? tuning_.windowMBps / 17 * 15
                                                                     : 0;
     }
-    const bool longBlocks = stats.longest >= kWindowLongBlockBytes && equal;
-    return tuning_.windowMBps / 17 * (longBlocks ? 16 : 15);
+    return tuning_.windowMBps / 17 * (equal && onGrid ? 16 : 15);
 }
 
 // In how many launches, each of as many pieces as are held, a list of more goes out; 1 where one that holds nothing is as fast.  Back to back,

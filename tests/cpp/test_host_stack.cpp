@@ -2142,6 +2142,51 @@ static void TestWindows()
     hybm_uninit();
 }
 
+// Lists whose segments no memory of the test backs: from(i) and to(i) are where segment i lies.
+template <class From, class To>
+static int SubmitList(uint32_t n, uint64_t bytes, From from, To to)
+{
+    std::vector<uint64_t> s(n), d(n), l(n, bytes);
+    for (uint32_t i = 0; i < n; ++i) {
+        s[i] = (1ull << 40) + from(i);
+        d[i] = (1ull << 42) + to(i);
+    }
+    XcopyEngine &engine = XcopyEngine::Instance();
+    void *stream = mf_xcopy_thread_stream();
+    const int ret = engine.Submit(s.data(), d.data(), l.data(), n, MF_ROUTE_HBM, stream, nullptr, 0);
+    return ret != BM_OK ? ret : engine.DrainThread();
+}
+
+// The rates of lists in windows: those that only blocks at multiples of 64 KiB hold, and where they do not apply.
+static void TestWindowRatesOfLists()
+{
+    CHECK(hybm_init(0, 0) == BM_OK);
+    fake_rt_skip_copies(1);
+    constexpr uint64_t k = 1024;
+    const uint32_t rate = XcopyTuning{}.windowMBps;
+    const uint32_t random = rate / 17 * 15, grid = rate / 17 * 16, ordered = rate / 34 * 32, orderedGrid = rate / 34 * 33;
+    struct Form { uint32_t n; uint64_t bytes, step; bool inOrder; uint32_t rate; };
+    const Form forms[] = {
+        {4096, 64 * k, 64 * k, false, grid}, {2400, 128 * k, 192 * k, false, grid}, {9000, 64 * k, 64 * k, false, grid},
+        {4600, 64 * k, 68 * k, false, random}, {4600, 64 * k, 64 * k + 256, false, random},        // off the grid by pages and by lines
+        {2708, 110776, 110848, false, random}, {2708, 110720, 110720, false, random}, {4308, 68 * k, 128 * k, false, random}, {3662, 80 * k, 80 * k, false, random},
+        {4096, 64 * k, 64 * k, true, orderedGrid}, {8000, 64 * k, 64 * k, true, ordered},
+        {4308, 68 * k, 68 * k, true, ordered}, {3662, 80 * k, 80 * k, true, ordered},
+    };
+    for (const Form &f : forms) {
+        (void)fake_rt_last_window();
+        CHECK(SubmitList(f.n, f.bytes, [&](uint32_t i) { return (i * 7919ull % f.n) * 2 * f.step; },
+                         [&](uint32_t i) { return f.inOrder ? i * f.bytes : (i * 5077ull % f.n) * f.step; }) == BM_OK);
+        const uint32_t got = fake_rt_last_window();
+        CHECK(got == f.rate);
+        if (got != f.rate) {
+            std::printf("  %u segments of %llu bytes: rate %u, expected %u\n", f.n, static_cast<unsigned long long>(f.bytes), got, f.rate);
+        }
+    }
+    fake_rt_skip_copies(0);
+    hybm_uninit();
+}
+
 int main()
 {
     SetLogLevel(3);
@@ -2165,6 +2210,7 @@ int main()
     TestPlugin();
     TestHeldStores();
     TestWindows();
+    TestWindowRatesOfLists();
     TestLongSegments();
     TestStreamDeck();
     TestWindowedRectangles();
