@@ -1470,7 +1470,8 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
     constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kWindowUnits) * kUnitBytes;
     // Whether the first segments are written one behind the other, which leaves the rows of HBM open: they hold a higher rate.
     const uint32_t sample = nseg < 64 ? nseg : 64;
-    const uint32_t follow = __popcll(__ballot(lane + 1 < sample && __shfl_down(to, 1, 64) - to == static_cast<uint32_t>(len0)));
+    const uint32_t behind = __shfl_down(to, 1, 64);         // with all lanes: what one that is switched off holds is not defined
+    const uint32_t follow = __popcll(__ballot(lane + 1 < sample && behind - to == static_cast<uint32_t>(len0)));
     const bool inOrder = each != 0 && follow * 4 >= (sample - 1) * 3;
     const bool shortPages = each != 0 && !inOrder && len0 < kWindowLongBlockBytes;
     const uint32_t windowTicks = each == 0 ? pace.windowTicks : inOrder ? pace.orderedTicks : shortPages ? pace.shortTicks : pace.longTicks;

@@ -170,7 +170,8 @@ def test_tables_that_their_launch_plans(gpu, kind):
     assert np.array_equal(target.cpu().numpy(), expect)
 
 
-@pytest.mark.parametrize("count,size", [(2049, 32768), (1025, 65536), (513, 163840), (64, 1 << 21)])
+@pytest.mark.parametrize("count,size", [(2049, 32768), (1025, 65536), (513, 163840), (64, 1 << 21), (5, 1 << 24), (4, 1 << 25),
+                                        (3, 1 << 25), (2, 1 << 26), (1, 1 << 27)])
 @pytest.mark.parametrize("ordered", [True, False])
 def test_windowed_tables_of_pages_in_order_and_not(gpu, count, size, ordered):
     """Just beyond what is held: the rates of pages that are written one behind the other, and of long ones that are not."""
