@@ -1333,7 +1333,11 @@ __device__ __forceinline__ bool PlannedQuad(const uint64_t *__restrict__ triples
 // In windows cut for 6.0 / 6.2 / 6.4 / 6.6 / 6.8 TB/s, the same to 0.5 in four processes: 4096 pages of 32 KiB gathered 49.8 / 48.4 / 47.1 / 46.0 / 45.3,
 // scattered 50.2 / 51.2 / 54 / 54 / 54; of 64 KiB gathered 94.5 / 91.7 / 89.4 / 87.3 / 85.7 (7.0: 91), scattered 95.0 / 92.8 / 90.5 / 87.8 / 97 to 102;
 // 1000 of 256 KiB scattered 92.0 / 89.6 / 87.1 / 85.2 / 86.7 to 91.6: 6.6 for what is written in order, 6.4 for scattered pages of 64 KiB and more.
-// Shorter ones are stored at random places no faster than 5.6, but read faster: with a read part of 0.40 / 0.44 / 0.47 / 0.50 / 0.53 of the period, 4096
+// Blocks that are neither read nor written in order hold 6.4 only on multiples of 64 KiB (300 MB at 6.0 / 6.4: 128 KiB there 106.3 / 101.5, on lines 107.4 /
+// 114.4; 80 KiB 108.2 / 119.6; 500 and 700 MB of 256 KiB on lines 173.7 / 177.5, 247 / 253) or where their last pieces are so short, which the
+// period does not count on, that all have less than kPlannedLoosePercent (72 KiB, 90 %, 117.1 / 110.2; 200 000 bytes, 94 %, 112.0 / 107.3; 110 776, 97 %, 110.1
+// / 107.5 to 114.2), and shorter ones of them no uneven parts (32 KiB, 130 MB 50.1 / 53.4).
+// Shorter ones that are read in order are stored at random places no faster than 5.6, but read faster: with a read part of 0.40 / 0.44 / 0.47 / 0.50 / 0.53 of the period, 4096
 // of 32 KiB at 6.0 50.6 / 50.1 / 50.2 / 50.1 / 51.5, at 6.2 50.5 / 48.9 / 48.9 / 49.8 / 53.8, at 6.4 51.6 / 48.7 / 48.8 / 53.2 / 54.7; so 29/64 at 6.3, 47.9.  The others
 // gain nothing from uneven parts.
 template <uint32_t kWaves, uint32_t kRun>
@@ -1354,8 +1358,9 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
     const uint32_t run = (nseg + 64 * kWaves - 1) / (64 * kWaves);
     const uint64_t len0 = reinterpret_cast<const __attribute__((address_space(4))) uint64_t *>(table)[2];     // by a scalar load
     const uint64_t *t = triples + 3ull * (lane < nseg ? lane : 0);
+    const uint32_t from = static_cast<uint32_t>(t[0]);      // of the first 64 segments, the same for every wave
     const uint32_t to = static_cast<uint32_t>(t[1]);
-    const uint32_t bits = static_cast<uint32_t>(t[0]) | to;        // of the first 64 segments, the same for every wave
+    const uint32_t bits = from | to;
     uint64_t len[kRun];
 #pragma unroll
     for (uint32_t r = 0; r < kRun; ++r) {
@@ -1468,13 +1473,19 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
         return;
     }
     constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kWindowUnits) * kUnitBytes;
-    // Whether the first segments are written one behind the other, which leaves the rows of HBM open: they hold a higher rate.
+    // Whether the first segments are written, or read, one behind the other, and whether they all lie on multiples of kWindowLongBlockBytes:
+    // the rates that a table of one length holds differ by that.  (With all lanes: what one that is switched off holds is not defined.)
     const uint32_t sample = nseg < 64 ? nseg : 64;
-    const uint32_t behind = __shfl_down(to, 1, 64);         // with all lanes: what one that is switched off holds is not defined
-    const uint32_t follow = __popcll(__ballot(lane + 1 < sample && behind - to == static_cast<uint32_t>(len0)));
-    const bool inOrder = each != 0 && follow * 4 >= (sample - 1) * 3;
-    const bool shortPages = each != 0 && !inOrder && len0 < kWindowLongBlockBytes;
-    const uint32_t windowTicks = each == 0 ? pace.windowTicks : inOrder ? pace.orderedTicks : shortPages ? pace.shortTicks : pace.longTicks;
+    const uint32_t length = static_cast<uint32_t>(len0);
+    const bool pair = lane + 1 < sample;
+    const uint32_t behind = __shfl_down(to, 1, 64);
+    const uint32_t ahead = __shfl_down(from, 1, 64);
+    const bool inOrder = each != 0 && __popcll(__ballot(pair && behind - to == length)) * 4 >= static_cast<int>(sample - 1) * 3;
+    const bool readInOrder = __popcll(__ballot(pair && ahead - from == length)) * 4 >= static_cast<int>(sample - 1) * 3;
+    const bool onGrid = __ballot(((from | to | length) & (kWindowLongBlockBytes - 1)) != 0) == 0;
+    const bool faster = each != 0 && !inOrder && (readInOrder || onGrid || (len0 >= kWindowLongBlockBytes && total * 25ull < items * static_cast<uint64_t>(kPlannedLoosePercent)));
+    const bool shortPages = faster && len0 < kWindowLongBlockBytes;
+    const uint32_t windowTicks = inOrder ? pace.orderedTicks : !faster ? pace.windowTicks : shortPages ? pace.shortTicks : pace.longTicks;
     const uint32_t period = static_cast<uint32_t>(windowTicks * (waves * kDeepBytes) >> 26);
     const uint32_t reading = shortPages ? period / 64 * 29 : period / 2;
     const uint32_t hold = (each != 0 ? pace.equalTicks : pace.holdTicks) +

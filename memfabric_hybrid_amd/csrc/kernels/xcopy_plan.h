@@ -376,7 +376,8 @@ constexpr uint32_t kPlannedShortRun = 8;
 constexpr uint32_t kPlannedWaves = 16;
 constexpr uint32_t kPlannedRun = 4;
 constexpr uint32_t kPlannedSegments = 64 * kPlannedWaves * kPlannedRun;
-constexpr uint32_t kPlannedFullPercent = 85;          // pieces of 16 KiB that are less full gain nothing from windows
+constexpr uint32_t kPlannedFullPercent = 85;          // pieces of 16 KiB that are less full gain nothing from windows,
+constexpr uint32_t kPlannedLoosePercent = 94;         // and those that are less full than this hold a higher rate wherever they lie
 constexpr uint64_t kWindowLongBlockBytes = 64ull << 10;   // blocks of one length from here on, at multiples of it, hold a higher rate in any order
 constexpr uint32_t kPlannedShallowChunks = 1024;
 constexpr uint32_t kPlannedHeldChunks = 16384;

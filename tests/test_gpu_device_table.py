@@ -171,14 +171,14 @@ def test_tables_that_their_launch_plans(gpu, kind):
 
 
 @pytest.mark.parametrize("count,size", [(2049, 32768), (1025, 65536), (513, 163840), (64, 1 << 21), (5, 1 << 24), (4, 1 << 25),
-                                        (3, 1 << 25), (2, 1 << 26), (1, 1 << 27)])
-@pytest.mark.parametrize("ordered", [True, False])
+                                        (3, 1 << 25), (2, 1 << 26), (1, 1 << 27), (1030, 73728)])
+@pytest.mark.parametrize("ordered", [True, False, "read"])
 def test_windowed_tables_of_pages_in_order_and_not(gpu, count, size, ordered):
-    """Just beyond what is held: the rates of pages that are written one behind the other, and of long ones that are not."""
+    """Just beyond what is held: the rates of pages that are written, or read, one behind the other, and of long ones that are not."""
     torch = pytest.importorskip("torch")
     rng = np.random.default_rng(count)
-    at = rng.permutation(2 * count)[:count].astype(np.int64) * size
-    place = (np.arange(count, dtype=np.int64) if ordered else rng.permutation(count)) * size
+    at = (np.arange(count, dtype=np.int64) if ordered == "read" else rng.permutation(2 * count)[:count].astype(np.int64)) * size
+    place = (np.arange(count, dtype=np.int64) if ordered is True else rng.permutation(count)) * size
     source = torch.randint(-2**63, 2**63 - 1, (2 * count * size // 8,), dtype=torch.int64, device="cuda").view(torch.uint8)
     target = torch.zeros(count * size, dtype=torch.uint8, device="cuda")
     table = torch.from_numpy(np.stack([source.data_ptr() + at, target.data_ptr() + place, np.full(count, size)], axis=1)).cuda()
