@@ -2,6 +2,7 @@
 // include/mf_hip_dataplane.h).  Rectangles whose addresses, pitches and width
 // are all multiples of 16 go to the 2-D kernel; anything else is expanded into
 // one segment per row and takes the ordinary batch path.
+#include <algorithm>
 #include <vector>
 
 #include "../../../include/mf_hip_dataplane_internal.h"
@@ -77,9 +78,13 @@ RectRun FillRectChunks(const mf_copy2d_desc *rects, size_t n, uint64_t target, R
 // 6.8 / 6.9 / 7.0 / 7.1 TB/s, us, the same to 1 % in three processes: on lines 161 MB 51.8 / 51.7 / 50.8 / 50.7, 419 MB 133 / 131 / 130.4 / 128.6, 969 MB 305 / 302 / 299 / 315,
 // 4.5 GB 1405 / 1390 / 1369 / 1353; not on lines 248 MB 78.7 / 77.5 / 77.1 / 80.8, 344 MB 108.2 / 108.1 / 111.7 / 120.7, 363 MB 113.7 / 112.7 / 114.3 / 122, 963 MB
 // 300 / 297 / 292 / 290.
-uint32_t RectRate(const RectRun &run, uint32_t windowMBps)
+// Where no higher rate than windowMBps is in force (this GPU did not hold it, or a caller has set one for all), windowMBps it is.
+uint32_t RectRate(const RectRun &run, const XcopyTuning &tuning)
 {
-    return run.lines ? windowMBps / 34 * 35 : windowMBps / 68 * 69;
+    if (tuning.windowAlignedMBps <= tuning.windowMBps) {
+        return tuning.windowMBps;
+    }
+    return run.lines ? std::min(tuning.windowMBps / 34 * 35, tuning.windowAlignedMBps) : tuning.windowMBps / 68 * 69;
 }
 
 // The chunk prefix; false for a launch of 2^32 chunks.
@@ -225,7 +230,7 @@ MF_EXPORT int32_t mf_xcopy_2d_batch(const mf_copy2d_desc *descs, uint32_t n, int
         if (run.bytes >= (windowed ? kRectChunksMinBytes : kRectPlainChunksMinBytes) &&
             CountRectChunks(run, windowed ? kRectWindowUnits : 64 * kRectChunkDepth, plan)) {
             taken = run.rects;
-            err = mfk_copy2d_chunks(&plan, windowed ? RectRate(run, engine.Tuning().windowMBps) : 0, stream);
+            err = mfk_copy2d_chunks(&plan, windowed ? RectRate(run, engine.Tuning()) : 0, stream);
         } else {
             err = LaunchRectRows(&rects[at], rects.size() - at, gridCap, stream, taken);
         }

@@ -651,7 +651,8 @@ int mfk_copy2d_chunks(const void *rectChunkPlan, uint32_t windowMBps, void *)
     ++g_launches;
     ++g_rectChunked;
     g_rectWindowed += windowMBps != 0 ? 1 : 0;
-    for (uint32_t c = 0; c < p.nchunk; ++c) {
+    g_lastWindow = windowMBps;
+    for (uint32_t c = 0; c < p.nchunk && !g_skipCopies; ++c) {
         uint32_t r = 0;
         while (r + 1 < mf::kRectInline && p.first[r + 1] <= c) {
             ++r;

@@ -1198,6 +1198,25 @@ static void TestRectangleChunks()
             d.src += reinterpret_cast<uint64_t>(from);
             d.dst += reinterpret_cast<uint64_t>(dst);
         }
+        {
+            // the library's own rates; a rate set by hand is the rate; and where the GPU holds none above the general one, that
+            struct { uint32_t general, aligned; bool scaled; } const rates[] = {
+                {6800000, 7100000, true}, {6400000, 6400000, false}, {16000000, 16000000, false}, {6392000, 6392000, false}, {6800000, 0, false}};
+            bool lines = true;
+            for (const mf_copy2d_desc &d : rects) {
+                lines = lines && ((d.src | d.dst | d.width | d.spitch | d.dpitch) & 127) == 0;
+            }
+            CHECK(mf_xcopy_tune(0, 0, 0) == BM_OK);
+            fake_rt_skip_copies(1);
+            for (const auto &r : rates) {
+                XcopyEngine::Instance().Tuning().windowMBps = r.general;
+                XcopyEngine::Instance().Tuning().windowAlignedMBps = r.aligned;
+                (void)fake_rt_last_window();
+                CHECK(mf_xcopy_2d_batch(rects.data(), static_cast<uint32_t>(rects.size()), MF_ROUTE_HBM, nullptr) == BM_OK);
+                CHECK(fake_rt_last_window() == (!f.windows ? 0 : !r.scaled ? r.general : lines ? 7000000 : 6900000));
+            }
+            fake_rt_skip_copies(0);
+        }
         for (int mode = 0; mode < 3; ++mode) {   // windows, none, whole rows
             CHECK(mf_xcopy_windows(mode == 0 ? 6800000 : 0) == BM_OK);
             CHECK(mf_xcopy_tune(0, mode == 2 ? 4096 : 0, 0) == BM_OK);
@@ -1213,7 +1232,7 @@ static void TestRectangleChunks()
         free(memory);
     }
     CHECK(mf_xcopy_tune(0, 0, 0) == BM_OK);
-    CHECK(mf_xcopy_windows(1) == BM_OK);
+    CHECK(mf_xcopy_windows(MF_XCOPY_WINDOWS_OWN_CHOICE) == BM_OK);
     hybm_uninit();
 }
 
