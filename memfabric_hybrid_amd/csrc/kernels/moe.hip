@@ -1192,7 +1192,7 @@ __global__ __launch_bounds__(kThreads) void MoeCombineKernel(uint64_t rowsIn, ui
 constexpr uint32_t kCombineItems = 4;                  // 32 result registers, 116 in all: sixteen waves per CU
 constexpr uint32_t kCombineWavesPerCu = 16;
 constexpr uint32_t kCombineSliceUnits = 128;           // two column positions per lane
-constexpr uint32_t kCombineMinItemsPerWave = 3;
+constexpr uint32_t kCombineMinItemsPerWave = 6;
 
 template <uint32_t kItems, uint32_t kSlots>
 __global__ __launch_bounds__(64) void MoeCombineWindowKernel(const u32x4 *__restrict__ rowsIn,
@@ -1318,6 +1318,44 @@ std::atomic<int> g_xcdStreams{0};
 std::atomic<uint32_t> g_combineReadMBps{6800000};
 std::atomic<uint32_t> g_combineWriteMBps{6200000};
 
+uint32_t CombineWaves()
+{
+    return static_cast<uint32_t>(mfrt_cu_count() > 0 ? mfrt_cu_count() : 256) * kCombineWavesPerCu;
+}
+
+// The dispatch in one launch that counts: where the lines lie, see those.
+bool DispatchCounts(uint64_t entries, uint64_t moved, uint32_t topK, bool lines)
+{
+    return entries <= kCountEntries && moved <= CountBytes(topK, lines);
+}
+
+// Whether waves that stay and keep reads and writes apart in time combine rows of at least 256 units: from six slices per wave on (top-8, 16 800 items
+// on 4096 waves 51.4 us, one workgroup per item 50.5; 19 200 the same; 25 200 74.4 / 76.7), below which the first read part and the last write part, in
+// which the chip only reads or only writes for want of work, cost what the separation gains; and where the last-level cache does not hold the rows that
+// the kernel before has just written.  Rows written by an elementwise kernel and combined, with windows from three items on / from six on / in rows
+// that a dispatch leaves there, us: top-8 3.6 to 5.9 items of 2048 elements a row, 262 MiB of rows and tokens 125.1 / 119.4, 310 146.3 / 141.2, 430 201.7 / 196.9; top-6
+// 290 MiB 132.7 / 127.9; and 6.2 items of 7168 elements at top-6, 350 MiB - / 163.8 / 159.8, 366 - / 171.1 / 166.5.  (Directly behind a dispatch
+// whose stores pass that cache windows gain 2 to 3 % from three items on; a program's experts lie between.)
+// Top-6 gains as top-8 does (8192 x 7168: 131-133 against 138-140 us); top-4 gains nothing (98 against 97 us)
+// and top-2 loses (16 384 x 4096: 79 against 66 us): their read parts are too short for the switch to pay.
+bool CombineInWindows(uint32_t tokens, uint32_t hidden, uint32_t topK, uint32_t &readTicks, uint32_t &writeTicks)
+{
+    const uint32_t upr = hidden / 8;
+    const uint32_t parts = (upr + kCombineSliceUnits - 1) / kCombineSliceUnits;
+    const uint32_t perPart = (upr + parts - 1) / parts;
+    const uint64_t items = static_cast<uint64_t>(tokens) * parts;
+    const uint64_t entries = static_cast<uint64_t>(tokens) * topK;
+    const uint32_t waves = CombineWaves();
+    if ((topK != 6 && topK != 8) || upr < 256 || items < static_cast<uint64_t>(waves) * kCombineMinItemsPerWave || items >= 0x40000000ull ||
+        DispatchCounts(entries, (entries + tokens) * upr * 16, topK, hidden % 64 == 0)) {
+        return false;
+    }
+    readTicks = WindowPeriodTicks(static_cast<uint64_t>(waves) * topK * perPart * 16, g_combineReadMBps.load(std::memory_order_relaxed));
+    writeTicks = WindowPeriodTicks(static_cast<uint64_t>(waves) * kCombineItems * perPart * 16,
+                                   g_combineWriteMBps.load(std::memory_order_relaxed));
+    return readTicks != 0 && writeTicks != 0;
+}
+
 }  // namespace
 }  // namespace mf
 
@@ -1376,7 +1414,7 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
         }
 #undef MF_DISPATCH_SMALL
     }
-    if (total <= kCountEntries && moved <= CountBytes(topK, lines)) {   // where the lines lie: see those
+    if (DispatchCounts(total, moved, topK, lines)) {
         const uint32_t cus = static_cast<uint32_t>(mfrt_cu_count() > 0 ? mfrt_cu_count() : 256);
         const uint32_t most = cus < kCountLeastGroups ? kCountLeastGroups : cus;
         const uint32_t perGroup = (tokens + most - 1) / most;
@@ -1504,24 +1542,11 @@ extern "C" int mfk_moe_combine(const void *rows, const void *rowOf, const void *
         // top-4 8192 x 7168 96 against 106 us, top-6 139 against 152 us (against the kernel that walks a run-time
         // number of slots).
         const uint32_t parts = (upr + kCombineSliceUnits - 1) / kCombineSliceUnits;
-        const uint32_t perPart = (upr + parts - 1) / parts;
         const uint64_t items = static_cast<uint64_t>(tokens) * parts;
-        const uint32_t waves = static_cast<uint32_t>(mfrt_cu_count() > 0 ? mfrt_cu_count() : 256) * kCombineWavesPerCu;
-        // Waves that stay and keep reads and writes apart in time, for rows that come from HBM: more than a dispatch leaves in the
-        // last-level cache (CountBytes), or dispatched by the tiles, whose stores pass it.  us of dispatch and combine, one workgroup per item and so: top-8, 3
-        // to 4 items per wave (6600 / 8192 x 2048) 94.6 / 92.4, 110.1 / 106.5; 7 (4063 x 7168) 179.4 / 173.6; top-6, 5.9 (6000 x 4096) 122.4 / 121.0; 8 (4702 x 7168)
-        // 154.4 / 150.0.  Rows in the cache want no windows, at top-8 3.6 items per wave (2129 x 7168) 85.0 / 87.8, 5.6 (3250) 138.8 / 144.1, at top-6 6.3 (3657)
-        // 118.6 / 120.3.
-        const uint32_t readTicks = WindowPeriodTicks(static_cast<uint64_t>(waves) * topK * perPart * 16,
-                                                     g_combineReadMBps.load(std::memory_order_relaxed));
-        const uint32_t writeTicks = WindowPeriodTicks(static_cast<uint64_t>(waves) * kCombineItems * perPart * 16,
-                                                      g_combineWriteMBps.load(std::memory_order_relaxed));
-        // Top-6 gains as top-8 does (8192 x 7168: 131-133 against 138-140 us); top-4 gains nothing (98 against 97 us)
-        // and top-2 loses (16 384 x 4096: 79 against 66 us): their read parts are too short for the switch to pay.
-        const uint64_t entries = static_cast<uint64_t>(tokens) * topK;
-        const bool fromHbm = entries > kCountEntries || (entries + tokens) * upr * 16 > CountBytes(topK, hidden % 64 == 0);
-        const bool windows = paced != 0 && topK >= 6 && fromHbm && items >= static_cast<uint64_t>(waves) * kCombineMinItemsPerWave &&
-                             items < 0x40000000ull && readTicks != 0 && writeTicks != 0;
+        const uint32_t waves = CombineWaves();
+        uint32_t readTicks = 0;
+        uint32_t writeTicks = 0;
+        const bool windows = paced != 0 && CombineInWindows(tokens, hidden, topK, readTicks, writeTicks);
         const uint32_t grid = windows ? waves : tokens * parts;
 #define MF_COMBINE_SLICES(K)                                                                                           \
     return Launch(MoeCombineKernel<K, 64, true, 2>, grid, 64, 0, s, At(rows), At(rowOf), At(weights), topK, upr, parts, At(y))
@@ -1562,6 +1587,13 @@ extern "C" int mfk_moe_combine(const void *rows, const void *rowOf, const void *
 #undef MF_COMBINE_TOKEN
     }
     return static_cast<int>(hipGetLastError());
+}
+
+extern "C" int mfk_moe_combine_stays(uint32_t tokens, uint32_t hidden, uint32_t topK)
+{
+    uint32_t readTicks = 0;
+    uint32_t writeTicks = 0;
+    return mf::CombineInWindows(tokens, hidden, topK, readTicks, writeTicks) ? 1 : 0;
 }
 
 extern "C" void mfk_moe_combine_windows(uint32_t readMBps, uint32_t writeMBps)

@@ -278,12 +278,13 @@ def test_out_of_range_expert_ids_are_flagged_not_followed(gpu, oracle):
     (500, 4096, 2),    # the slice kernel compiled for top-2
     (400, 7168, 4),    # ... top-4
     (300, 5120, 6),    # ... top-6
-    (5100, 5120, 6),   # top-6, 25 500 slices: waves that stay, as in the first shape
+    (5100, 5120, 6),   # top-6, 25 500 slices of rows that a dispatch leaves in the last-level cache
+    (5400, 5120, 6),   # top-6, 27 000 slices of more rows than that: waves that stay, as in the first shape
     (3600, 7168, 4),   # top-4 with as many slices: still one workgroup per slice
 ])
 def test_combine_of_rows_that_differ_within_a_token(gpu, oracle, T, H, K):
     """After a dispatch the rows of a token are copies of one another, so a combine that mixed them up would still pass
-    the dispatch-then-combine tests; here every row is different.  The first two shapes and the top-6 shape of 5100 tokens have enough tokens of wide rows
+    the dispatch-then-combine tests; here every row is different.  The first two shapes and the top-6 shape of 5400 tokens have enough tokens of wide rows
     for the combine whose waves stay and alternate between reading and writing: same bits as the oracle at the
     default pace, at a slow and at an absurdly fast one, with slots without a row, and with the form switched off."""
     rng = np.random.default_rng(T)
@@ -317,14 +318,23 @@ def test_combine_of_rows_that_differ_within_a_token(gpu, oracle, T, H, K):
             b.free()
 
 
-@pytest.mark.parametrize("T,H,K", [
-    (2080, 7168, 8),   # the most rows that a dispatch leaves in the last-level cache
-    (2081, 7168, 8),   # one token more: one period of three read parts and a part of the fourth
-    (6145, 2048, 8),   # the fewest entries beyond the dispatch that counts, three items per wave and two more
-    (2700, 7168, 6),
+@pytest.mark.parametrize("T,H,K,stays", [
+    (3510, 7168, 8, False),   # one token short of six slices a wave, and the most rows that a dispatch leaves in the last-level cache
+    (3511, 7168, 8, True),    # one token more: a full period, two read parts and one slice of a third
+    (2081, 7168, 8, False),   # more than 256 MiB, 3.6 slices a wave
+    (6145, 2048, 8, False),   # the fewest entries beyond the dispatch that counts, three slices a wave
+    (3845, 7168, 6, False), (3846, 7168, 6, True),      # where those rows end at top-6
+    (8192, 3072, 6, False), (8193, 3072, 6, True),      # the fewest entries beyond the dispatch that counts, at six slices a wave
+    (8200, 3072, 4, False),
 ])
-def test_combine_where_its_waves_begin_to_stay(gpu, oracle, T, H, K):
+def test_combine_where_its_waves_begin_to_stay(gpu, oracle, T, H, K, stays):
+    assert gpu.mf_moe_combine_stays(T, H, K) == stays
     test_combine_of_rows_that_differ_within_a_token(gpu, oracle, T, H, K)
+    assert gpu.mf_moe_combine_windows(0, 0) == 0
+    try:
+        assert gpu.mf_moe_combine_stays(T, H, K) == 0
+    finally:
+        assert gpu.mf_moe_combine_windows(*native.MOE_COMBINE_WINDOWS_DEFAULT) == 0
 
 
 def test_same_workspace_reused_by_calls_of_different_sizes(gpu, oracle):
