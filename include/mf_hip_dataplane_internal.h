@@ -116,7 +116,7 @@ int32_t mf_xcopy_tune_hold(uint32_t deepHold, int32_t pinnedExtraNanos, uint32_t
 
 /* A combine of topK == 8 or 6 with rows of 2048 elements and more, on enough tokens to give every wave of the chip six
  * slices of 128 x 8 elements (about 3500 tokens of 7168 elements on 256 CUs) and more rows than a dispatch leaves in the
- * last-level cache (432 MiB with their tokens at top-8, 368 MiB at top-6), runs as waves that stay for the whole
+ * last-level cache (400 MiB with their tokens at top-8, 368 MiB at top-6), runs as waves that stay for the whole
  * launch and alternate, chip-wide and by the clock, between reading rows and writing results.  readMBps / writeMBps
  * (MB/s of HBM traffic, 1 000 000 ... 16 000 000) set the pace of the two parts; the defaults are 6 800 000 and
  * 6 200 000, both 0 turns the form off (one workgroup per slice, as for smaller inputs, and as long as a second
@@ -124,6 +124,8 @@ int32_t mf_xcopy_tune_hold(uint32_t deepHold, int32_t pinnedExtraNanos, uint32_t
 int32_t mf_moe_combine_windows(uint32_t readMBps, uint32_t writeMBps);
 /* 1 if such a combine by this thread would take that form now. */
 int32_t mf_moe_combine_stays(uint32_t tokens, uint32_t hidden, uint32_t topK);
+/* 1 if a dispatch with rows is one launch whose workgroups each count all ids (and is none of the few-token form). */
+int32_t mf_moe_dispatch_counts(uint32_t tokens, uint32_t hidden, uint32_t topK, uint32_t experts);
 /* 1 if hybm_init found that the GPU deals consecutive workgroups to its eight XCDs in turn (an MI355X in its default
  * partition does): the dispatch of rows of whole cache lines then writes its output in runs of consecutive rows, one stream of runs
  * per XCD; 0: it keeps to the token-ordered permute.  No counterpart in the reference. */

@@ -109,6 +109,11 @@ MF_EXPORT int32_t mf_moe_combine_windows(uint32_t readMBps, uint32_t writeMBps)
     return BM_OK;
 }
 
+MF_EXPORT int32_t mf_moe_dispatch_counts(uint32_t tokens, uint32_t hidden, uint32_t topK, uint32_t experts)
+{
+    return mfk_moe_dispatch_counts(tokens, hidden, topK, experts);
+}
+
 MF_EXPORT int32_t mf_moe_combine_stays(uint32_t tokens, uint32_t hidden, uint32_t topK)
 {
     return XcopyEngine::Instance().SingleSubmitter() ? mfk_moe_combine_stays(tokens, hidden, topK) : 0;

@@ -844,19 +844,22 @@ constexpr uint32_t CountLdsWords(uint32_t experts, uint32_t ownMost)
 // from taking turns with them (2400 of 7168 at top-2: dispatch 19.4, 25.9 without; before kCountNearBytes the longer code
 // costs 0.5).  Calls of few slots read most: from kCountDeepBytes on plain stores cost them more than the next kernel
 // gains (4096 of 7168 at top-2, dispatch / both: nontemporal 28.6 / 57.4, plain 36.5 / 56.0).
-// What fits the last-level cache (256 MiB) too little goes to the tiles: they are the quicker dispatch from about 280 MiB on, but as long as the next kernel
-// finds a part of the rows in the cache not the quicker pair.  Dispatch / both with the tiles and so, us, three sets of buffers in turn: top-8 over 256 experts,
-// 262 MiB 61.4 / 105.6, 54.1 / 85.0; 310 64.7 / 118.2, 64.7 / 102.4; 350 66.8 / 127.2, 75.5 / 118.7; 400 84.8 / 153.1, 86.7 / 138.8; 450 85.0 / 161.6, 98.9 / 161.1; 500
-// 91.6 / 173.6, 109.7 / 183.9.  Top-6 310 56.6 / 110.9, 66.1 / 101.1; 350 66.2 / 126.9, 76.7 / 118.6; 400 75.0 / 143.2, 88.8 / 143.5.  Top-4 310 59.4 / 113.2, 54.6 /
-// 108.1; 350 61.4 / 122.5, 61.2 / 121.9; 450 88.0 / 165.6, 100.7 / 180.9.  Top-2 230 45.7 / 84.7, 38.5 / 77.6; 262 59.0 / 102.9, 57.1 / 102.2; 280 61.8 / 108.4,
-// 60.4 / 109.4.  Rows that are not whole cache lines are always stored plainly: two waves share a line.
+// What fits the last-level cache (256 MiB) too little goes to the tiles: they are the quicker dispatch from about 300 MiB on, but pass that cache with their
+// stores, where this leaves a part of the rows for the next kernel.  The line follows the whole: dispatch, a kernel that reads the rows and writes
+// others of their size, and the combine of those.  Dispatch / all three with the tiles and so, us, three sets of buffers in turn, 7168 elements: top-8 over
+// 256 experts, 262 MiB 60.9 / 191, 53.7 / 180; 310 65.1 / 222, 64.3 / 211; 350 67.3 / 246, 75.6 / 240; 400 84.7 / 289, 86.6 / 274; 430 85.4 / 304, 93.3 / 297, but of 4096
+// elements over 64 72.5 / 292, 94.6 / 295.  Top-6 310 58.2 / 215, 66.9 / 206; 366 69.9 / 261, 80.4 / 246.  Top-4 290 59.6 / 199, 51.3 / 196; 310 60.4 / 211, 54.3 / 208; 334
+// 61.4 / 225, 58.6 / 227.  Top-2 270 59.2 / 164, 58.9 / 164.  64 and 128 experts as 256; over 8 the next kernel finds the rows of the tiles better: top-8 270
+// 62.1 / 185, 56.7 / 180, 310 62.8 / 204, 65.2 / 206, 350 63.2 / 225, 75.8 / 234; top-4 270 50.0 / 173, 48.4 / 178.  Rows that are not whole cache lines are always
+// stored plainly: two waves share a line.
 constexpr uint64_t kQuickBytes = 24ull << 20;            // also of the dispatch above
 constexpr uint64_t kQuickFewBytes = 16ull << 20;         // with up to two slots, whose next kernel reads the rows sooner
 constexpr uint64_t kCountNearBytes = 96ull << 20;
 constexpr uint64_t kCountDeepBytes = 150ull << 20;
-constexpr uint64_t CountBytes(uint32_t topK, bool lines)
+constexpr uint32_t kCountFewExperts = 64;                // below
+constexpr uint64_t CountBytes(uint32_t topK, uint32_t experts, bool lines)
 {
-    return (topK <= 2 || !lines ? 256ull : topK <= 4 ? 336ull : topK <= 6 ? 368ull : 432ull) << 20;
+    return (topK <= 2 || experts < kCountFewExperts || !lines ? 256ull : topK <= 4 ? 320ull : topK <= 6 ? 368ull : 400ull) << 20;
 }
 
 template <bool kNt>
@@ -1324,9 +1327,9 @@ uint32_t CombineWaves()
 }
 
 // The dispatch in one launch that counts: where the lines lie, see those.
-bool DispatchCounts(uint64_t entries, uint64_t moved, uint32_t topK, bool lines)
+bool DispatchCounts(uint64_t entries, uint64_t moved, uint32_t topK, uint32_t experts, bool lines)
 {
-    return entries <= kCountEntries && moved <= CountBytes(topK, lines);
+    return entries <= kCountEntries && moved <= CountBytes(topK, experts, lines);
 }
 
 // Whether waves that stay and keep reads and writes apart in time combine rows of at least 256 units: from six slices per wave on (top-8, 16 800 items
@@ -1347,7 +1350,7 @@ bool CombineInWindows(uint32_t tokens, uint32_t hidden, uint32_t topK, uint32_t 
     const uint64_t entries = static_cast<uint64_t>(tokens) * topK;
     const uint32_t waves = CombineWaves();
     if ((topK != 6 && topK != 8) || upr < 256 || items < static_cast<uint64_t>(waves) * kCombineMinItemsPerWave || items >= 0x40000000ull ||
-        DispatchCounts(entries, (entries + tokens) * upr * 16, topK, hidden % 64 == 0)) {
+        DispatchCounts(entries, (entries + tokens) * upr * 16, topK, kMaxExperts, hidden % 64 == 0)) {
         return false;
     }
     readTicks = WindowPeriodTicks(static_cast<uint64_t>(waves) * topK * perPart * 16, g_combineReadMBps.load(std::memory_order_relaxed));
@@ -1414,7 +1417,7 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
         }
 #undef MF_DISPATCH_SMALL
     }
-    if (DispatchCounts(total, moved, topK, lines)) {
+    if (DispatchCounts(total, moved, topK, experts, lines)) {
         const uint32_t cus = static_cast<uint32_t>(mfrt_cu_count() > 0 ? mfrt_cu_count() : 256);
         const uint32_t most = cus < kCountLeastGroups ? kCountLeastGroups : cus;
         const uint32_t perGroup = (tokens + most - 1) / most;
@@ -1587,6 +1590,13 @@ extern "C" int mfk_moe_combine(const void *rows, const void *rowOf, const void *
 #undef MF_COMBINE_TOKEN
     }
     return static_cast<int>(hipGetLastError());
+}
+
+extern "C" int mfk_moe_dispatch_counts(uint32_t tokens, uint32_t hidden, uint32_t topK, uint32_t experts)
+{
+    const uint64_t entries = static_cast<uint64_t>(tokens) * topK;
+    const bool small = entries <= mf::kSmallEntries && entries * topK <= mf::kSmallCompares;
+    return !small && mf::DispatchCounts(entries, (entries + tokens) * (hidden / 8) * 16, topK, experts, hidden % 64 == 0) ? 1 : 0;
 }
 
 extern "C" int mfk_moe_combine_stays(uint32_t tokens, uint32_t hidden, uint32_t topK)

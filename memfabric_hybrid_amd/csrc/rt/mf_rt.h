@@ -155,6 +155,8 @@ int mfk_moe_combine(const void *rows, const void *rowOf, const void *weights, ui
  * of the dispatch needs it); mfk_moe_xcd_streams() is 1 if they do */
 int mfk_moe_setup(void);
 int mfk_moe_xcd_streams(void);
+/* 1 where mfk_moe_dispatch with rows is the one launch in which every workgroup counts all ids */
+int mfk_moe_dispatch_counts(uint32_t tokens, uint32_t hidden, uint32_t topK, uint32_t experts);
 /* 1 where mfk_moe_combine takes the form that keeps reads and writes apart in time, if it may pace itself */
 int mfk_moe_combine_stays(uint32_t tokens, uint32_t hidden, uint32_t topK);
 /* pace of that form, MB/s for its read and write parts; 0 = never */

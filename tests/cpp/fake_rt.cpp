@@ -685,6 +685,7 @@ int mfk_moe_combine(const void *, const void *, const void *, uint32_t, uint32_t
     return 0;
 }
 void mfk_moe_combine_windows(uint32_t, uint32_t) {}
+int mfk_moe_dispatch_counts(uint32_t, uint32_t, uint32_t, uint32_t) { return 0; }
 int mfk_moe_combine_stays(uint32_t, uint32_t, uint32_t) { return 0; }
 int mfk_moe_setup(void) { return 0; }
 int mfk_moe_xcd_streams(void) { return 0; }

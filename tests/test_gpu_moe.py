@@ -319,7 +319,7 @@ def test_combine_of_rows_that_differ_within_a_token(gpu, oracle, T, H, K):
 
 
 @pytest.mark.parametrize("T,H,K,stays", [
-    (3510, 7168, 8, False),   # one token short of six slices a wave, and the most rows that a dispatch leaves in the last-level cache
+    (3510, 7168, 8, False),   # one token short of six slices a wave
     (3511, 7168, 8, True),    # one token more: a full period, two read parts and one slice of a third
     (2081, 7168, 8, False),   # more than 256 MiB, 3.6 slices a wave
     (6145, 2048, 8, False),   # the fewest entries beyond the dispatch that counts, three slices a wave
@@ -502,12 +502,15 @@ def test_dispatch_that_counts_in_one_launch(gpu, T, H, K, E):
             _free(bufs)
 
 
-@pytest.mark.parametrize("T,H,K,E", [
-    (3510, 7168, 8, 256), (3511, 7168, 8, 256), (6144, 4096, 8, 64),    # at top-8, the most rows for the dispatch that counts, and a token more
-    (3845, 7168, 6, 64), (3846, 7168, 6, 64), (4915, 7168, 4, 8), (4916, 7168, 4, 8),
-    (6241, 7168, 2, 8), (6242, 7168, 2, 8),
+@pytest.mark.parametrize("T,H,K,E,counts", [
+    (3250, 7168, 8, 256, True), (3251, 7168, 8, 256, False),    # at top-8, the most rows for the dispatch that counts, and a token more
+    (3510, 7168, 8, 256, False), (3511, 7168, 8, 256, False), (6144, 4096, 8, 64, False),
+    (2080, 7168, 8, 63, True), (2081, 7168, 8, 63, False),      # over few experts
+    (3845, 7168, 6, 64, True), (3846, 7168, 6, 64, False), (4681, 7168, 4, 64, True), (4682, 7168, 4, 64, False),
+    (4915, 7168, 4, 8, False), (4916, 7168, 4, 8, False), (6241, 7168, 2, 8, True), (6242, 7168, 2, 8, False),
 ])
-def test_dispatch_where_the_tiles_begin(gpu, T, H, K, E):
+def test_dispatch_where_the_tiles_begin(gpu, T, H, K, E, counts):
+    assert gpu.mf_moe_dispatch_counts(T, H, K, E) == counts
     test_dispatch_that_counts_in_one_launch(gpu, T, H, K, E)
 
 
