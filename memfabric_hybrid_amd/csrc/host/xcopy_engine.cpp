@@ -1722,6 +1722,13 @@ uint32_t XcopyEngine::HoldFor(const InlinePlan &plan, uint32_t grid, int route, 
     return with > 0 ? static_cast<uint32_t>(with) : 0;
 }
 
+// Pieces of 16 KiB that a segment of a batch whose addresses have these bits set is cut into, at the most.
+static uint64_t DeepPiecesOf(uint64_t bytes, uint64_t addressBits)
+{
+    constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kDeepUnits) * kUnitBytes;
+    return bytes == 0 ? 0 : (bytes + ((addressBits & (kPieceAlign - 1)) == 0 ? 0 : kPieceAlign - 1) + kDeepBytes - 1) / kDeepBytes;
+}
+
 BatchStats StatsOf(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n)
 {
     constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kDeepUnits) * kUnitBytes;
@@ -1733,14 +1740,13 @@ BatchStats StatsOf(const uint64_t *src, const uint64_t *dst, const uint64_t *len
         st.lengthBits |= len[i];
     }
     // (Pages need no second pass, which costs 0.4 ns a segment: 4096 of 8 KiB 14.5 us with it.)
-    const uint64_t more = ((st.addressBits & (kPieceAlign - 1)) == 0 ? 0 : kPieceAlign - 1) + kDeepBytes - 1;
     if (st.longest + kPieceAlign <= kDeepBytes) {
         st.deepPieces = n;
     } else if (st.total == st.longest * n) {
-        st.deepPieces = n * ((st.longest + more) / kDeepBytes);
+        st.deepPieces = n * DeepPiecesOf(st.longest, st.addressBits);
     } else {
         for (uint32_t i = 0; i < n; ++i) {
-            st.deepPieces += (len[i] + more) / kDeepBytes;
+            st.deepPieces += DeepPiecesOf(len[i], st.addressBits);
         }
     }
     return st;
@@ -1866,41 +1872,53 @@ uint32_t XcopyEngine::HeldLaunches(const BatchStats &stats, const uint64_t *dst,
     if (mean < (equal ? kDeepBytes : kDeepBytes / 4 * 7) || mean >= kWindowSliceMinAlignedSegmentBytes) {
         return 1;
     }
+    // A launch ends with a segment, so a share that surely fits is less than a launch holds by what that one may exceed it.
+    const uint64_t longest = DeepPiecesOf(stats.longest, stats.addressBits);
+    if (longest > kHeldMaxPieces / 4) {
+        return 1;
+    }
     const uint32_t pieces = static_cast<uint32_t>(stats.deepPieces);
-    const uint32_t parts = (pieces + kHeldMaxPieces - 1) / kHeldMaxPieces;
+    const uint32_t room = static_cast<uint32_t>(equal ? kHeldMaxPieces / longest * longest : kHeldMaxPieces + 1 - longest);
+    const uint32_t fewest = (pieces + kHeldMaxPieces - 1) / kHeldMaxPieces;
+    uint32_t parts = (pieces + room - 1) / room;
+    if (parts != fewest) {
+        const uint64_t share = (pieces + fewest - 1) / fewest;
+        uint64_t taken = 0;
+        uint64_t most = 0;
+        for (uint32_t i = 0; i < n; ++i) {
+            taken = (taken < share ? taken : 0) + DeepPiecesOf(len[i], stats.addressBits);
+            most = std::max(most, taken);
+        }
+        parts = most <= kHeldMaxPieces ? fewest : parts;
+    }
     const bool odd = (stats.addressBits & (kUnitBytes - 1)) != 0;
-    if ((parts > 2 && (odd ? mean < 3 * kDeepBytes : WrittenInOrder(dst, len, n))) || PieceWindowRate(stats, dst, len, n, pieces, kDeepUnits, false) != 0 ||
-        HoldForPieces(stats, n, pieces / parts, kDeepUnits, false) == 0) {
+    if (parts > kSlots / 2 || (parts > 2 && (odd ? mean < 3 * kDeepBytes : WrittenInOrder(dst, len, n))) ||
+        PieceWindowRate(stats, dst, len, n, pieces, kDeepUnits, false) != 0 || HoldForPieces(stats, n, pieces / parts, kDeepUnits, false) == 0) {
         return 1;
     }
     return parts;
 }
 
-// The same bytes to each of them.  (What the whole list's lengths and addresses rule out for none of its segments holds for each part.)
+// The same number of pieces to each of them, up to a segment.  (What the whole list's lengths and addresses rule out for none of its
+// segments holds for each part.)
 int XcopyEngine::SubmitHeld(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, const BatchStats &stats, uint32_t parts,
                             void *stream, void *mask, uint32_t maskValue)
 {
-    uint32_t at = 0;
-    uint64_t before = 0;
-    uint64_t taken = 0;
-    for (uint32_t p = 1; p <= parts; ++p) {
-        const uint64_t until = stats.total / parts * p;
-        uint32_t end = at;
-        while (end < n && (p == parts || taken < until)) {
-            taken += len[end++];
-        }
-        if (end == at) {
-            continue;
-        }
+    const uint64_t share = (stats.deepPieces + parts - 1) / parts;
+    for (uint32_t at = 0; at < n;) {
         BatchStats part = stats;
-        part.total = taken - before;
-        part.deepPieces = stats.deepPieces / parts;
+        part.total = 0;
+        part.deepPieces = 0;
+        uint32_t end = at;
+        while (end < n && (part.deepPieces < share || len[end] == 0)) {
+            part.total += len[end];
+            part.deepPieces += DeepPiecesOf(len[end++], stats.addressBits);
+        }
         const int ret = SubmitPieces(src + at, dst + at, len + at, end - at, part, kDeepUnits, stream, end == n ? mask : nullptr, maskValue, false);
         if (ret != BM_OK) {
             return ret;
         }
         at = end;
-        before = taken;
     }
     return BM_OK;
 }

@@ -31,6 +31,8 @@ bool g_skipCopies = false;       // launches count and check their plans but mov
 uint32_t g_lastTableShift = 0;   // group shift of the latest table launch that used a group map, 0 under a pattern
 uint64_t g_groupMapErrors = 0;
 uint32_t g_lastPieceWait = 0;    // what the waves of the latest launch of pieces wait
+uint32_t g_mostPieces = 0;       // the most pieces of one launch, and the least its waves wait, since fake_rt_piece_launches()
+uint32_t g_leastPieceWait = ~0u;
 uint32_t g_lastTableHold = 0;    // holdNanos of the latest table launch
 std::atomic<uint64_t> g_streamsMade{0};   // streams made since mfrt_init
 
@@ -176,6 +178,13 @@ void fake_rt_skip_copies(int on) { g_skipCopies = on != 0; }
 uint32_t fake_rt_last_table_shift(void) { return g_lastTableShift; }
 uint64_t fake_rt_group_map_errors(void) { return g_groupMapErrors; }
 uint32_t fake_rt_last_piece_wait(void) { return g_lastPieceWait; }
+void fake_rt_piece_launches(uint32_t *mostPieces, uint32_t *leastWait)
+{
+    *mostPieces = g_mostPieces;
+    *leastWait = g_leastPieceWait;
+    g_mostPieces = 0;
+    g_leastPieceWait = ~0u;
+}
 uint32_t fake_rt_last_table_hold(void) { return g_lastTableHold; }
 
 int mfrt_init(int device)
@@ -421,6 +430,8 @@ int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t bytes, uint32_
     NoteRecorded(stream);
     g_lastTableHold = holdNanos;
     g_lastPieceWait = mf::PieceHoldNanos(holdNanos, count, bytes, units);
+    g_mostPieces = count > g_mostPieces ? count : g_mostPieces;
+    g_leastPieceWait = g_lastPieceWait < g_leastPieceWait ? g_lastPieceWait : g_leastPieceWait;
     if (pieces == nullptr || count == 0 || (units != 256 && units != 512 && units != 1024)) {
         return -1;
     }

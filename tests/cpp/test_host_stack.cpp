@@ -44,6 +44,7 @@ extern "C" const uint32_t *fake_rt_calibration_holds(void);
 extern "C" uint32_t fake_rt_last_table_shift(void);
 extern "C" uint32_t fake_rt_last_table_hold(void);
 extern "C" uint32_t fake_rt_last_piece_wait(void);
+extern "C" void fake_rt_piece_launches(uint32_t *mostPieces, uint32_t *leastWait);
 extern "C" uint64_t fake_rt_group_map_errors(void);
 extern "C" uint64_t fake_rt_in_flight(void);
 extern "C" void fake_rt_capture(void *stream);
@@ -2206,6 +2207,112 @@ static void TestWindowRatesOfLists()
     hybm_uninit();
 }
 
+// Lists of more pieces than the chip holds go out in two to four launches, none of more than it holds, whatever lies where in the list.
+static void TestHeldLaunches()
+{
+    CHECK(hybm_init(0, 0) == BM_OK);
+    XcopyEngine &engine = XcopyEngine::Instance();
+    std::mt19937 rng(5);
+    auto some = [&](uint32_t n, uint64_t least, uint64_t most) {
+        std::vector<uint64_t> l(n);
+        for (uint64_t &v : l) {
+            v = least + rng() % (most - least + 1);
+        }
+        return l;
+    };
+    auto then = [](std::vector<uint64_t> a, const std::vector<uint64_t> &b) {
+        a.insert(a.end(), b.begin(), b.end());
+        return a;
+    };
+    struct List { const char *name; std::vector<uint64_t> len; uint64_t align; uint32_t launches; };
+    std::vector<List> lists;
+    lists.push_back({"ragged", some(2700, 1, 90000), 1, 2});
+    lists.push_back({"ragged, three", some(3000, 60000, 120000), 1, 3});
+    lists.push_back({"ragged, four", some(4200, 60000, 120000), 16, 4});
+    lists.push_back({"equal, as many as two launches hold", std::vector<uint64_t>(3584, 50000), 256, 2});
+    lists.push_back({"equal, one too many", std::vector<uint64_t>(3585, 50000), 256, 3});
+    lists.push_back({"short ones first", then(some(3000, 3000, 4000), some(4000, 55000, 63000)), 16, 3});
+    lists.push_back({"short ones last", then(some(4000, 55000, 63000), some(3000, 3000, 4000)), 16, 3});
+    lists.push_back({"empty ones last", then(some(3000, 60000, 120000), std::vector<uint64_t>(2000, 0)), 16, 3});
+    lists.push_back({"empty ones at a cut", then(then(std::vector<uint64_t>(1790, 50000), std::vector<uint64_t>(70, 0)), std::vector<uint64_t>(1790, 50000)), 256, 2});
+    lists.push_back({"a long one among them", then(then(some(1200, 50000, 60000), {1100 * 16384 + 7}), some(1600, 50000, 60000)), 16, 2});
+    lists.push_back({"a long one at the cut", then(then(some(1530, 50000, 60000), {1100 * 16384 + 7}), some(1270, 50000, 60000)), 16, 3});
+    // just below what two launches hold: a cut cannot meet their limits
+    std::vector<uint64_t> full = some(3300, 60000, 80000);
+    uint64_t pieces = 0;
+    size_t kept = 0;
+    while (pieces + 5 <= 2 * kHeldMaxPieces) {
+        pieces += (full[kept++] + 127 + 16383) / 16384;
+    }
+    full.resize(kept);
+    lists.push_back({"nearly what two launches hold", full, 16, 3});
+    void *other = mfrt_stream_create();
+    CHECK(other != nullptr);
+    for (const List &list : lists) {
+        const uint32_t n = static_cast<uint32_t>(list.len.size());
+        std::vector<uint64_t> src(n), dst(n);
+        std::vector<uint32_t> order(n);
+        for (uint32_t i = 0; i < n; ++i) {
+            order[i] = (i * 2657ull + 11) % n;
+        }
+        uint64_t room = 0;
+        for (uint32_t i = 0; i < n; ++i) {
+            src[i] = room + (list.align == 1 ? 1 : 0);
+            room += (list.len[i] + 2 + list.align) / list.align * list.align;
+        }
+        uint64_t to = 0;
+        std::vector<char> taken(n, 0);
+        auto place = [&](uint32_t i) {
+            if (taken[i] == 0) {
+                taken[i] = 1;
+                dst[i] = to + (list.align == 1 ? 2 : 0);
+                to += (list.len[i] + 3 + list.align) / list.align * list.align;
+            }
+        };
+        for (uint32_t i : order) {
+            place(i);
+        }
+        for (uint32_t i = 0; i < n; ++i) {
+            place(i);
+        }
+        uint8_t *a = static_cast<uint8_t *>(mfrt_alloc_device(room + 64));
+        uint8_t *b = static_cast<uint8_t *>(mfrt_alloc_device(to + 64));
+        for (uint64_t i = 0; i + 8 <= room; i += 8) {
+            const uint64_t word = (i + 1) * 0x9E3779B97F4A7C15ull;
+            std::memcpy(a + i, &word, 8);
+        }
+        for (uint32_t i = 0; i < n; ++i) {
+            src[i] += reinterpret_cast<uint64_t>(a);
+            dst[i] += reinterpret_cast<uint64_t>(b);
+        }
+        for (int way = 0; way < 3; ++way) {     // the thread's stream, the same with a word for the end, a stream of the caller's
+            uint64_t word = 0;
+            std::memset(b, 0xA5, to);
+            uint32_t most = 0;
+            uint32_t wait = 0;
+            fake_rt_piece_launches(&most, &wait);
+            const uint64_t before = mf_xcopy_launch_count();
+            void *stream = way == 2 ? other : mf_xcopy_thread_stream();
+            CHECK(engine.Submit(src.data(), dst.data(), list.len.data(), n, MF_ROUTE_HBM, stream, way == 1 ? &word : nullptr, 32) == BM_OK);
+            CHECK(mfrt_stream_sync(stream) == 0 && engine.DrainThread() == BM_OK);
+            const uint64_t launches = mf_xcopy_launch_count() - before;
+            fake_rt_piece_launches(&most, &wait);
+            bool ok = launches == list.launches && most <= kHeldMaxPieces && wait != 0 && wait != ~0u && word == (way == 1 ? 32 : 0);
+            for (uint32_t i = 0; i < n && ok; ++i) {
+                ok = std::memcmp(reinterpret_cast<void *>(dst[i]), reinterpret_cast<void *>(src[i]), list.len[i]) == 0;
+            }
+            CHECK(ok);
+            if (!ok) {
+                std::printf("  %s, way %d: %llu launches, most pieces %u, least wait %u\n", list.name, way, static_cast<unsigned long long>(launches), most, wait);
+            }
+        }
+        CHECK(mfrt_free_device(a) == 0 && mfrt_free_device(b) == 0);
+    }
+    CHECK(fake_rt_violations() == 0);
+    (void)mfrt_stream_destroy(other);
+    hybm_uninit();
+}
+
 int main()
 {
     SetLogLevel(3);
@@ -2230,6 +2337,7 @@ int main()
     TestHeldStores();
     TestWindows();
     TestWindowRatesOfLists();
+    TestHeldLaunches();
     TestLongSegments();
     TestStreamDeck();
     TestWindowedRectangles();
