@@ -1722,11 +1722,14 @@ uint32_t XcopyEngine::HoldFor(const InlinePlan &plan, uint32_t grid, int route, 
     return with > 0 ? static_cast<uint32_t>(with) : 0;
 }
 
-// Pieces of 16 KiB that a segment of a batch whose addresses have these bits set is cut into, at the most.
-static uint64_t DeepPiecesOf(uint64_t bytes, uint64_t addressBits)
+// Pieces of 16 KiB that a segment of a batch is cut into, at the most; `over` is DeepOver() of its addresses.
+static uint64_t DeepOver(uint64_t addressBits)
 {
-    constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kDeepUnits) * kUnitBytes;
-    return bytes == 0 ? 0 : (bytes + ((addressBits & (kPieceAlign - 1)) == 0 ? 0 : kPieceAlign - 1) + kDeepBytes - 1) / kDeepBytes;
+    return static_cast<uint64_t>(kDeepUnits) * kUnitBytes - 1 + ((addressBits & (kPieceAlign - 1)) == 0 ? 0 : kPieceAlign - 1);
+}
+static uint64_t DeepPiecesOf(uint64_t bytes, uint64_t over)
+{
+    return (bytes + over) / (static_cast<uint64_t>(kDeepUnits) * kUnitBytes);
 }
 
 BatchStats StatsOf(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n)
@@ -1740,13 +1743,14 @@ BatchStats StatsOf(const uint64_t *src, const uint64_t *dst, const uint64_t *len
         st.lengthBits |= len[i];
     }
     // (Pages need no second pass, which costs 0.4 ns a segment: 4096 of 8 KiB 14.5 us with it.)
+    const uint64_t over = DeepOver(st.addressBits);
     if (st.longest + kPieceAlign <= kDeepBytes) {
         st.deepPieces = n;
     } else if (st.total == st.longest * n) {
-        st.deepPieces = n * DeepPiecesOf(st.longest, st.addressBits);
+        st.deepPieces = n * DeepPiecesOf(st.longest, over);
     } else {
         for (uint32_t i = 0; i < n; ++i) {
-            st.deepPieces += DeepPiecesOf(len[i], st.addressBits);
+            st.deepPieces += DeepPiecesOf(len[i], over);
         }
     }
     return st;
@@ -1873,7 +1877,8 @@ uint32_t XcopyEngine::HeldLaunches(const BatchStats &stats, const uint64_t *dst,
         return 1;
     }
     // A launch ends with a segment, so a share that surely fits is less than a launch holds by what that one may exceed it.
-    const uint64_t longest = DeepPiecesOf(stats.longest, stats.addressBits);
+    const uint64_t over = DeepOver(stats.addressBits);
+    const uint64_t longest = DeepPiecesOf(stats.longest, over);
     if (longest > kHeldMaxPieces / 4) {
         return 1;
     }
@@ -1886,7 +1891,7 @@ uint32_t XcopyEngine::HeldLaunches(const BatchStats &stats, const uint64_t *dst,
         uint64_t taken = 0;
         uint64_t most = 0;
         for (uint32_t i = 0; i < n; ++i) {
-            taken = (taken < share ? taken : 0) + DeepPiecesOf(len[i], stats.addressBits);
+            taken = (taken < share || len[i] == 0 ? taken : 0) + DeepPiecesOf(len[i], over);
             most = std::max(most, taken);
         }
         parts = most <= kHeldMaxPieces ? fewest : parts;
@@ -1905,15 +1910,25 @@ int XcopyEngine::SubmitHeld(const uint64_t *src, const uint64_t *dst, const uint
                             void *stream, void *mask, uint32_t maskValue)
 {
     const uint64_t share = (stats.deepPieces + parts - 1) / parts;
+    const uint64_t over = DeepOver(stats.addressBits);
+    const uint64_t longest = DeepPiecesOf(stats.longest, over);
+    const bool equal = stats.total == stats.longest * n;
     for (uint32_t at = 0; at < n;) {
-        BatchStats part = stats;
-        part.total = 0;
-        part.deepPieces = 0;
+        uint64_t bytes = 0;
+        uint64_t pieces = 0;
         uint32_t end = at;
-        while (end < n && (part.deepPieces < share || len[end] == 0)) {
-            part.total += len[end];
-            part.deepPieces += DeepPiecesOf(len[end++], stats.addressBits);
+        if (equal) {
+            end = static_cast<uint32_t>(std::min<uint64_t>(n, at + (share + longest - 1) / longest));
+            bytes = (end - at) * stats.longest;
+            pieces = (end - at) * longest;
         }
+        while (end < n && (pieces < share || len[end] == 0)) {
+            bytes += len[end];
+            pieces += DeepPiecesOf(len[end++], over);
+        }
+        BatchStats part = stats;
+        part.total = bytes;
+        part.deepPieces = pieces;
         const int ret = SubmitPieces(src + at, dst + at, len + at, end - at, part, kDeepUnits, stream, end == n ? mask : nullptr, maskValue, false);
         if (ret != BM_OK) {
             return ret;
