@@ -2191,6 +2191,9 @@ static void TestWindowRatesOfLists()
         {4600, 64 * k, 68 * k, false, random}, {4600, 64 * k, 64 * k + 256, false, random},        // off the grid by pages and by lines
         {2708, 110776, 110848, false, random}, {2708, 110720, 110720, false, random}, {4308, 68 * k, 128 * k, false, random}, {3662, 80 * k, 80 * k, false, random},
         {4096, 64 * k, 64 * k, true, orderedGrid}, {8000, 64 * k, 64 * k, true, ordered},
+        {16384, 16 * k, 16 * k, true, random}, {8193, 32 * k, 32 * k, true, random},                  // short ones in order: from 16 384 pieces on
+        {7169, 32 * k, 32 * k, true, 0}, {7169, 16 * k, 16 * k, true, 0}, {7169, 16 * k, 16 * k, false, random},
+        {3584, 32 * k, 32 * k, false, 0}, {3585, 32 * k, 32 * k, false, random}, {1000, 110720, 110720, false, 0},    // what is held takes no windows
         {4308, 68 * k, 68 * k, true, ordered}, {3662, 80 * k, 80 * k, true, ordered},
     };
     for (const Form &f : forms) {
@@ -2202,6 +2205,24 @@ static void TestWindowRatesOfLists()
         if (got != f.rate) {
             std::printf("  %u segments of %llu bytes: rate %u, expected %u\n", f.n, static_cast<unsigned long long>(f.bytes), got, f.rate);
         }
+    }
+    for (const bool more : {false, true}) {      // part-filled pieces: held up to 7168 of them, in windows beyond
+        std::mt19937 rng(3);
+        const uint32_t n = more ? 1100 : 760;
+        std::vector<uint64_t> s(n), d(n), l(n);
+        for (uint32_t i = 0; i < n; ++i) {
+            s[i] = (1ull << 40) + i * 128 * k;
+            d[i] = (1ull << 42) + (i * 7ull % n) * 128 * k;
+            l[i] = 111000 + rng() % 20000;
+        }
+        uint32_t most = 0;
+        uint32_t wait = 0;
+        fake_rt_piece_launches(&most, &wait);
+        (void)fake_rt_last_window();
+        CHECK(XcopyEngine::Instance().Submit(s.data(), d.data(), l.data(), n, MF_ROUTE_HBM, mf_xcopy_thread_stream(), nullptr, 0) == BM_OK);
+        CHECK(XcopyEngine::Instance().DrainThread() == BM_OK);
+        fake_rt_piece_launches(&most, &wait);
+        CHECK(fake_rt_last_window() == (more ? random : 0) && (wait != 0) == !more && (most > kHeldMaxPieces) == more);
     }
     fake_rt_skip_copies(0);
     hybm_uninit();

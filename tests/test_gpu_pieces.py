@@ -32,8 +32,10 @@ def _lengths(kind, rng):
         return np.concatenate([rng.integers(1, 9000, 7000), EDGES])
     if kind == "held 8 KiB":                                     # no segment longer, 4096 pieces at the most
         return np.concatenate([rng.integers(7000, 8065, 2900), [1, 0, 8064, 8065, 17, 4096]])
-    if kind == "windows":                                        # nearly full pieces, 80 MiB and more; a round and a fraction of 4096
+    if kind == "held, nearly full":
         return np.concatenate([rng.integers(111000, 131000, 760), EDGES])
+    if kind == "windows":                                        # nearly full pieces, more than are held; two rounds and a fraction of 4096
+        return np.concatenate([rng.integers(111000, 131000, 1100), EDGES])
     if kind == "windows, three rounds":
         return np.concatenate([np.full(8193, 16384), [16384 + 15, 16383, 1, 0]])
     if kind == "held, all that are resident":                    # 7168 pieces of 16 KiB at the most hold their stores
@@ -42,13 +44,20 @@ def _lengths(kind, rng):
         return np.concatenate([np.full(7169 - len(EDGES), 16256), np.minimum(np.maximum(EDGES, 1), 16256)])
     if kind == "more than are held":
         return np.concatenate([rng.integers(1, 90000, 2700), EDGES])
+    if kind == "three times what is held":
+        return np.concatenate([rng.integers(50000, 110000, 3000), EDGES])
+    if kind == "three times what is held, part-filled":
+        return np.concatenate([rng.integers(33000, 40000, 5000), EDGES])
+    if kind == "four times what is held":
+        return np.concatenate([rng.integers(50000, 110000, 4400), EDGES])
     if kind == "two waves":
         return np.concatenate([rng.integers(1, 20000, 3000), EDGES])
     return np.concatenate([rng.integers(1, 90000, 2000), EDGES])   # "four waves"
 
 
 @pytest.mark.parametrize("kind", ["every shift", "held 4 KiB", "held 16 KiB", "held 8 KiB", "one wave", "two waves", "four waves", "windows",
-                                  "windows, three rounds", "held, all that are resident", "one too many to hold", "more than are held"])
+                                  "held, nearly full", "windows, three rounds", "held, all that are resident", "one too many to hold", "more than are held",
+                                  "three times what is held", "three times what is held, part-filled", "four times what is held"])
 @pytest.mark.parametrize("odd", [True, False])
 def test_batch_in_pieces(gpu, oracle, kind, odd):
     rng = np.random.default_rng(len(kind) + odd)
@@ -70,13 +79,31 @@ def test_batch_in_pieces(gpu, oracle, kind, odd):
         b.upload(before)
         launches = gpu.mf_xcopy_launch_count()
         gpu_util.xcopy(gpu, a.ptr + src, b.ptr + dst, lens, native.ROUTE_HBM)
-        assert gpu.mf_xcopy_launch_count() - launches == (2 if kind == "more than are held" else 1)
+        expect = {"more than are held": 2}       # nearly full pieces on lines go in windows; short segments at odd bytes in one launch that holds nothing
+        expect.update({"windows": 2, "three times what is held": 3, "four times what is held": 4} if odd else {"three times what is held, part-filled": 3})
+        assert gpu.mf_xcopy_launch_count() - launches == expect.get(kind, 1)
         got = b.download()
     finally:
         a.free()
         b.free()
     gpu_util.oracle_batch(oracle, source, before, src, dst, lens)
     assert np.array_equal(got, before)
+
+
+@pytest.mark.parametrize("count,size", [(1700, 65536), (1000, 131072), (1030, 110720), (16384, 16384), (7169, 16384), (8193, 32768)])
+@pytest.mark.parametrize("where", ["in order", "read in order", "scattered"])
+def test_lists_of_blocks_in_windows(gpu, count, size, where):
+    """Blocks of one length, written one behind the other, read so, or neither, at the rates that each of them is given."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(count)
+    at = (np.arange(count) if where == "read in order" else rng.permutation(2 * count)[:count]).astype(np.int64)
+    place = (np.arange(count) if where == "in order" else rng.permutation(count)).astype(np.int64)
+    source = torch.randint(-2**63, 2**63 - 1, (2 * count * size // 8,), dtype=torch.int64, device="cuda").view(torch.uint8)
+    target = torch.zeros(count * size, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    lens = np.full(count, size, dtype=np.uint64)
+    gpu_util.xcopy(gpu, (source.data_ptr() + at * size).astype(np.uint64), (target.data_ptr() + place * size).astype(np.uint64), lens, native.ROUTE_HBM)
+    assert torch.equal(target.view(count, size)[torch.from_numpy(place).cuda()], source.view(2 * count, size)[torch.from_numpy(at).cuda()])
 
 
 @pytest.mark.parametrize("each", [512, 40000])
