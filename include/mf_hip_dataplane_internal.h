@@ -52,7 +52,7 @@ int32_t mf_xcopy_tune(uint32_t units, uint32_t wgPerCu, uint32_t wgPerCuLink);
  * 0 = never wait, otherwise that many ns for every launch the rule would pick, also of more than 128 segments.  Other launches, and
  * batches submitted with MF_COPY_UNORDERED_FLAG, never wait. */
 int32_t mf_xcopy_hold_stores(int32_t nanos);
-/* Read and write windows.  A batch of up to 128 segments and 512 MiB or more between HBM addresses is copied
+/* Read and write windows.  A batch of up to 128 segments and 128 MiB or more between HBM addresses is copied
  * by 4096 waves that alternate, all together and by the GPU's constant-rate clock, between a read half and a
  * write half of a period, so that HBM sees long bursts of one direction: 6.65-6.75 TB/s instead of 6.1-6.35 on
  * aligned copies of 512 MiB to 2 GiB, 6.05-6.3 instead of 5.75-5.85 when sources sit at odd addresses.  The
@@ -63,7 +63,9 @@ int32_t mf_xcopy_hold_stores(int32_t nanos);
  * 7 100 000 (32 x 16 MiB back to back: 6.95 instead of 6.65 TB/s), those of 64 MiB and
  * more on average for 7 400 000, and a batch of 1 GiB and more of such long segments is cut into launches of
  * about 512 MiB, which hold their schedule more often than longer ones (1 GiB: 7.1-7.2 instead of 6.7 TB/s).
- * Segments whose source and destination differ modulo 16 take no windows.  The call sets all three rates; 0
+ * Segments whose source and destination differ modulo 16 take no windows.  Rectangles of 32 MiB and more go at
+ * 35/34 of the default rate where all rows are whole lines and at 69/68 elsewhere, lists of more than 128 segments and device
+ * tables at 15/17 to 33/34 of it.  The call sets all three rates, rectangles take the rate that is set, and the parts are of it; 0
  * switches the form off, MF_XCOPY_WINDOWS_OWN_CHOICE brings back the rates the library chose itself (what
  * hybm_init measured, else the defaults above).  While several threads submit on streams of their own the
  * form is not used. */

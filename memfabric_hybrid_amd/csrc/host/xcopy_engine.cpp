@@ -1859,14 +1859,18 @@ uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *d
 
 // In how many launches, each of as many pieces as are held, a list of more goes out; 1 where one that holds nothing is as fast.  Back to back,
 // us in one launch / so: pages of 32 KiB gathered 121 / 138 / 213 MB 43.4 / 41.8, 49.1 / 47.3, 75.7 / 74.2 (but 311 MB 110.2 / 110.5 and 360 MB
-// 125.7 / 127.8: no more than two launches for what is written in order); segments of 50 000 bytes at random places 130 / 150 MB 53.3 / 48.9, 61.1 /
-// 56.1, of 24 000 132 / 168 MB 54.3 / 50.2, 69.0 / 63.8, of 33 333, 68 % full, 153 MB 62.8 / 57.7, of 20 000, 61 %, 122 / 180 MB 50.8 / 52.5, 74.3 / 79.8; ragged ones
-// at odd addresses of up to 63 000 / 100 000 / 120 000 / 200 000 bytes 49.7 / 47.5, 62.2 / 58.5, 73.6 / 69.2, 148 / 145, of up to 45 000 58.0 / 62.9:
-// the host writes those no faster than the GPU copies them, and the second launch is 4 us of its time.
+// 125.7 / 127.8); segments of 50 000 bytes at random places 130 / 150 MB 53.3 / 48.9, 61.1 / 56.1, of 24 000 132 / 168 MB 54.3 / 50.2, 69.0 / 63.8, of
+// 33 333, 68 % full, 153 MB 62.8 / 57.7, of 20 000, 61 %, 122 / 180 MB 50.8 / 52.5, 74.3 / 79.8; ragged ones at odd addresses of up to 63 000 / 100 000 /
+// 120 000 / 200 000 bytes 49.7 / 47.5, 62.2 / 58.5, 73.6 / 69.2, 148 / 145, of up to 45 000 58.0 / 62.9: the host writes those no faster than the GPU
+// copies them, and the second launch is 4 us of its time.  The ratio over 125 to 450 MB in two to four launches, lengths of one size and ragged ones of 30 000 to
+// 900 000 bytes: at random places 0.92 to 0.99, at odd addresses from 640 000 bytes on 0.98 to 1.02; read in order 0.93 to 1.00, at odd addresses from
+// 400 000 on 0.98 to 1.06; written in order, where the one launch finds the rows of HBM open, in two launches of nearly full pieces 0.94 to 1.00, of others 1.00
+// to 1.04, in three or four 1.00 to 1.07, at odd addresses from 400 000 bytes on 1.00 to 1.08.
 // Every launch has a slot of its own, so half of them are left for other calls.
 uint32_t XcopyEngine::HeldLaunches(const BatchStats &stats, const uint64_t *dst, const uint64_t *len, uint32_t n, bool unordered) const
 {
     constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kDeepUnits) * kUnitBytes;
+    constexpr uint64_t kHeldOddBytes = 24 * kDeepBytes;
     if (unordered || tuning_.unitsOverride != 0 || !tuning_.deepHold || stats.deepPieces <= kHeldMaxPieces ||
         stats.deepPieces > kSlots / 2 * kHeldMaxPieces || stats.total < stats.deepPieces * kDeepBytes / 100 * 65) {
         return 1;
@@ -1897,8 +1901,10 @@ uint32_t XcopyEngine::HeldLaunches(const BatchStats &stats, const uint64_t *dst,
         parts = most <= kHeldMaxPieces ? fewest : parts;
     }
     const bool odd = (stats.addressBits & (kUnitBytes - 1)) != 0;
-    if (parts > kSlots / 2 || (parts > 2 && (odd ? mean < 3 * kDeepBytes : WrittenInOrder(dst, len, n))) ||
-        PieceWindowRate(stats, dst, len, n, pieces, kDeepUnits, false) != 0 || HoldForPieces(stats, n, pieces / parts, kDeepUnits, false) == 0) {
+    const bool refused = WrittenInOrder(dst, len, n) ? parts > 2 || stats.total < stats.deepPieces * kDeepBytes / 100 * 92
+                                                      : parts > 2 && odd && mean < 3 * kDeepBytes;
+    if (parts > kSlots / 2 || refused || (odd && mean >= kHeldOddBytes) || PieceWindowRate(stats, dst, len, n, pieces, kDeepUnits, false) != 0 ||
+        HoldForPieces(stats, n, pieces / parts, kDeepUnits, false) == 0) {
         return 1;
     }
     return parts;

@@ -965,7 +965,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kHeldWavesPe
 // A single segment in chunks of LineChunks(), one a wave of the kernel above without a list.  HBM bounds it.  us back to back, from 16 KiB in
 // 100 registers up to 64 MiB and 4 KiB without hold beyond, the chunks the segment's / so: 32 MB 10.9 / 10.3, 48 16.3 / 15.4, 66 20.9 / 20.6, 90
 // 29.9 / 28.4, 110 36.2 / 34.0; destination off a line by 48 bytes 12.1 / 10.4, 18.1 / 15.7, 23.8 / 20.6, 31.7 / 28.8, 38.4 / 34.3; source and destination
-// different modulo 16, before from a list of pieces up to 64 MiB, 11.9 / 10.9, 17.0 / 15.7, 22.9 / 21.0, 32.9 / 29.4, 40.0 / 35.2.
+// different modulo 16, before from a list of pieces up to 64 MiB, 11.9 / 10.9, 17.0 / 15.7, 22.9 / 21.0, 32.9 / 29.4, 40.0 / 35.2.  Beside a kernel of another
+// stream that holds half the CUs 63 MB 27.8 / 24.1, 72 28.7 / 26.6, 110 42.0 / 45.0; 32 of 72 MB beside eight elementwise kernels over 1 GiB, both together
+// 2151 / 2237.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kHeldWavesPerSimd, kHeldWavesPerSimd))) void XcopySingleHeldKernel(
     uint64_t src, uint64_t dst, uint32_t len, uint32_t holdTicks)
 {

@@ -167,7 +167,7 @@ int mfk_copy2d(const void *rectPlan, uint32_t grid, void *stream);
 /* rectChunkPlan: mf::RectChunkPlan; in read and write windows cut for windowMBps over chunks of kRectWindowUnits units, or with 0 in
  * chunks of 64 * kRectChunkDepth.  Between HBM addresses. */
 int mfk_copy2d_chunks(const void *rectChunkPlan, uint32_t windowMBps, void *stream);
-/* Both rectangle kernels once on an empty plan. */
+/* Every rectangle kernel once on an empty plan. */
 int mfk_copy2d_prelaunch(void *stream);
 
 #ifndef MF_RT_HIDDEN

@@ -2245,7 +2245,7 @@ static void TestHeldLaunches()
         a.insert(a.end(), b.begin(), b.end());
         return a;
     };
-    struct List { const char *name; std::vector<uint64_t> len; uint64_t align; uint32_t launches; };
+    struct List { const char *name; std::vector<uint64_t> len; uint64_t align; uint32_t launches; bool inOrder = false; };
     std::vector<List> lists;
     lists.push_back({"ragged", some(2700, 1, 90000), 1, 2});
     lists.push_back({"ragged, three", some(3000, 60000, 120000), 1, 3});
@@ -2267,6 +2267,12 @@ static void TestHeldLaunches()
     }
     full.resize(kept);
     lists.push_back({"nearly what two launches hold", full, 16, 3});
+    // where one launch that holds nothing is the faster form
+    lists.push_back({"long ones at odd addresses", some(300, 350000, 500000), 1, 1});
+    lists.push_back({"long ones on units", some(300, 350000, 500000), 16, 2});
+    lists.push_back({"in order, nearly full", some(1300, 110000, 130000), 16, 2, true});
+    lists.push_back({"in order, part-filled", some(3000, 40000, 56000), 16, 1, true});
+    lists.push_back({"in order, three", some(2200, 110000, 130000), 1, 1, true});
     void *other = mfrt_stream_create();
     CHECK(other != nullptr);
     for (const List &list : lists) {
@@ -2290,11 +2296,16 @@ static void TestHeldLaunches()
                 to += (list.len[i] + 3 + list.align) / list.align * list.align;
             }
         };
-        for (uint32_t i : order) {
-            place(i);
+        for (uint32_t i = 0; i < n && !list.inOrder; ++i) {
+            place(order[i]);
         }
         for (uint32_t i = 0; i < n; ++i) {
-            place(i);
+            if (list.inOrder) {
+                dst[i] = to;
+                to += list.len[i];
+            } else {
+                place(i);
+            }
         }
         uint8_t *a = static_cast<uint8_t *>(mfrt_alloc_device(room + 64));
         uint8_t *b = static_cast<uint8_t *>(mfrt_alloc_device(to + 64));
@@ -2318,7 +2329,7 @@ static void TestHeldLaunches()
             CHECK(mfrt_stream_sync(stream) == 0 && engine.DrainThread() == BM_OK);
             const uint64_t launches = mf_xcopy_launch_count() - before;
             fake_rt_piece_launches(&most, &wait);
-            bool ok = launches == list.launches && most <= kHeldMaxPieces && wait != 0 && wait != ~0u && word == (way == 1 ? 32 : 0);
+            bool ok = launches == list.launches && word == (way == 1 ? 32 : 0) && (most <= kHeldMaxPieces && wait != 0 && wait != ~0u) == (launches != 1);
             for (uint32_t i = 0; i < n && ok; ++i) {
                 ok = std::memcmp(reinterpret_cast<void *>(dst[i]), reinterpret_cast<void *>(src[i]), list.len[i]) == 0;
             }
