@@ -2228,6 +2228,34 @@ static void TestWindowRatesOfLists()
     hybm_uninit();
 }
 
+// The pieces a list is said to have at the most: never fewer than it is cut into, and on the side of kHeldMaxPieces on which they are.
+static void TestPiecesOfLists()
+{
+    std::mt19937 rng(9);
+    constexpr uint64_t deep = kDeepUnits * 16ull;
+    for (int round = 0; round < 400; ++round) {
+        const uint32_t n = 129 + rng() % (round % 2 == 0 ? 2000 : 12000);
+        const uint64_t mean = 1 + rng() % (round % 3 == 0 ? 5000 : round % 3 == 1 ? 40000 : 200000);
+        const uint64_t align = round % 5 < 2 ? 128 : 1;
+        std::vector<uint64_t> s(n), d(n), l(n);
+        uint64_t pieces = 0;
+        for (uint32_t i = 0; i < n; ++i) {
+            l[i] = round % 7 == 0 ? mean : round % 7 == 1 && i % 2 == 0 ? 1 + rng() % 100 : 1 + rng() % (2 * mean);
+            s[i] = (1ull << 40) + i * 1000000ull / align * align;
+            d[i] = (1ull << 42) + i * 1000000ull / align * align + (align == 1 ? rng() % 128 : 0);
+            pieces += ((d[i] & (kPieceAlign - 1)) + l[i] + deep - 1) / deep;
+        }
+        const BatchStats st = StatsOf(s.data(), d.data(), l.data(), n);
+        CHECK(st.deepPieces >= pieces);
+        const uint64_t over = align == 1 ? kPieceAlign - 1 : 0;
+        uint64_t most = 0;
+        for (uint32_t i = 0; i < n; ++i) {
+            most += (l[i] + over + deep - 1) / deep;
+        }
+        CHECK((st.deepPieces <= kHeldMaxPieces) == (most <= kHeldMaxPieces));
+    }
+}
+
 // Lists of more pieces than the chip holds go out in two to four launches, none of more than it holds, whatever lies where in the list.
 static void TestHeldLaunches()
 {
@@ -2369,6 +2397,7 @@ int main()
     TestHeldStores();
     TestWindows();
     TestWindowRatesOfLists();
+    TestPiecesOfLists();
     TestHeldLaunches();
     TestLongSegments();
     TestStreamDeck();
