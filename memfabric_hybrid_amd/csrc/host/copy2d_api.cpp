@@ -40,9 +40,32 @@ struct RectRun {
     uint32_t rects = 0;            // of the list, from its front
     uint32_t entries = 0;
     uint64_t bytes = 0;
-    uint64_t looseBytes = 0;       // of single rectangles that are not OnLines()
-    bool lines = true;             // all of them are
+    uint64_t looseBytes = 0;       // of what does not hold a schedule: see RectHolds
+    uint64_t shortBytes = 0;       // of that, of what does in short launches
+    uint64_t linesBytes = 0;       // of rows of whole cache lines that lie against one another in the destination
+    uint64_t againstBytes = 0;     // of other pairs whose rows do
 };
+
+// Whether a rectangle, or a pair with rows of `row` bytes, holds a schedule: where the destination's rows lie against one another (a pair), or begin and end on
+// 64 bytes, and where lines that are only touched in part are few.  600 MB, us, in windows cut for 6.8 TB/s / in 4 KiB chunks without: pairs of 2736 bytes 182.7 /
+// 194.1, 16 bytes between their rows 235 / 212, of 896 and 16 246 / 218, of 896 and 896 184 / 195; single ones of 896, 5120, 4736 bytes read from
+// rows 16 bytes longer 184 / 194, 185 / 191, 185 / 191, of 480, 2736 and 20 000 185 / 198, 199 / 194, 186 / 195 but at 900 MB 345 / 309, 336 / 304, 334 / 305; of 64
+// bytes 64 apart 308 / 264, of 192 read from rows of 256 281 / 243.  Pairs hold it in short launches whatever their rows: 40 MB of 2736 and 16 16.2 / 18.4 as whole rows.
+enum class Holds { kAlways, kShort, kNever };
+Holds RectHolds(const mf_copy2d_desc &d, bool pair)
+{
+    const uint64_t row = pair ? 2 * d.width : d.width;
+    const bool against = d.dpitch == row;
+    const bool on64 = ((d.dst | d.dpitch | row) & 63) == 0;
+    const bool dstLines = ((d.dst | d.dpitch | row) & (kWindowAlignBytes - 1)) == 0;
+    const bool srcLines = ((d.src | d.spitch | d.width) & (kWindowAlignBytes - 1)) == 0;
+    const uint64_t dstPart = against || dstLines ? 0 : std::min(d.dpitch - row, kWindowAlignBytes);
+    const uint64_t srcPart = d.spitch == d.width || srcLines ? 0 : std::min(d.spitch - d.width, kWindowAlignBytes);
+    if ((on64 || (pair && against)) && dstPart * 5 <= row && srcPart * 10 <= d.width) {
+        return Holds::kAlways;
+    }
+    return pair && dstPart * 3 <= row && srcPart * 3 <= d.width ? Holds::kShort : Holds::kNever;
+}
 
 // As many rectangles as the entries of a plan hold, or as make `target` bytes; none of 2^32 units.
 RectRun FillRectChunks(const mf_copy2d_desc *rects, size_t n, uint64_t target, RectChunkPlan &plan)
@@ -68,23 +91,39 @@ RectRun FillRectChunks(const mf_copy2d_desc *rects, size_t n, uint64_t target, R
         plan.magic[e] = RectMagic(plan.rowUnits[e]);
         run.rects += pair ? 2 : 1;
         run.bytes += row * 16 * d.height;
-        run.looseBytes += pair || OnLines(d) ? 0 : row * 16 * d.height;
-        run.lines = run.lines && OnLines(d) && (!pair || OnLines(rects[run.rects - 1]));
+        const Holds holds = RectHolds(d, pair);
+        run.looseBytes += holds == Holds::kAlways ? 0 : row * 16 * d.height;
+        run.shortBytes += holds == Holds::kShort ? row * 16 * d.height : 0;
+        const bool against = d.dpitch == row * 16;
+        const bool lines = against && OnLines(d) && (!pair || OnLines(rects[run.rects - 1]));
+        run.linesBytes += lines ? row * 16 * d.height : 0;
+        run.againstBytes += !lines && pair && against ? row * 16 * d.height : 0;
     }
     return run;
 }
 
-// Rows of whole cache lines hold more than others, and these more than segments at any place, whose rate the tuning is.  Rectangles of a reshard cut for
+// Whether the launch goes in windows.
+bool RectsHold(const RectRun &run)
+{
+    return run.looseBytes - (run.bytes < kRectShortBytes ? run.shortBytes : 0) <= run.bytes / 4;
+}
+
+// Rows of whole cache lines that lie against one another in the destination hold more than segments at any place, whose rate the tuning is, and other pairs whose
+// rows do a little more.  Rectangles of a reshard cut for
 // 6.8 / 6.9 / 7.0 / 7.1 TB/s, us, the same to 1 % in three processes: on lines 161 MB 51.8 / 51.7 / 50.8 / 50.7, 419 MB 133 / 131 / 130.4 / 128.6, 969 MB 305 / 302 / 299 / 315,
 // 4.5 GB 1405 / 1390 / 1369 / 1353; not on lines 248 MB 78.7 / 77.5 / 77.1 / 80.8, 344 MB 108.2 / 108.1 / 111.7 / 120.7, 363 MB 113.7 / 112.7 / 114.3 / 122, 963 MB
-// 300 / 297 / 292 / 290.
+// 300 / 297 / 292 / 290.  With room between their rows they fall apart above the tuning's: 600 MB of single ones of 896, 4736 and 5120 bytes, as much apart, 186.5 /
+// 186.3 / 186.7 at 6.8, 209.5 / 199.6 / 212.8 at 7.0, of pairs of 256 and of 128 bytes, as much apart, 189.5 / 190.3 and 222 / 208.
 // Where no higher rate than windowMBps is in force (this GPU did not hold it, or a caller has set one for all), windowMBps it is.
 uint32_t RectRate(const RectRun &run, const XcopyTuning &tuning)
 {
     if (tuning.windowAlignedMBps <= tuning.windowMBps) {
         return tuning.windowMBps;
     }
-    return run.lines ? std::min(tuning.windowMBps / 34 * 35, tuning.windowAlignedMBps) : tuning.windowMBps / 68 * 69;
+    if (run.linesBytes == run.bytes) {
+        return std::min(tuning.windowMBps / 34 * 35, tuning.windowAlignedMBps);
+    }
+    return run.linesBytes + run.againstBytes >= run.bytes / 4 * 3 ? tuning.windowMBps / 68 * 69 : tuning.windowMBps;
 }
 
 // The chunk prefix; false for a launch of 2^32 chunks.
@@ -226,7 +265,7 @@ MF_EXPORT int32_t mf_xcopy_2d_batch(const mf_copy2d_desc *descs, uint32_t n, int
         const RectRun run = route == MFRT_ROUTE_HBM && gridCap == 0 && total >= kRectChunksMinBytes
                                 ? FillRectChunks(&rects[at], rects.size() - at, target, plan)
                                 : RectRun{};
-        const bool windowed = run.looseBytes <= run.bytes / 4 && engine.WindowsApply(run.bytes, route, kRectChunksMinBytes);
+        const bool windowed = RectsHold(run) && engine.WindowsApply(run.bytes, route, kRectChunksMinBytes);
         if (run.bytes >= (windowed ? kRectChunksMinBytes : kRectPlainChunksMinBytes) &&
             CountRectChunks(run, windowed ? kRectWindowUnits : 64 * kRectChunkDepth, plan)) {
             taken = run.rects;

@@ -100,6 +100,7 @@ constexpr uint64_t kWindowMinBytes = 128ull << 20;
 // fast up to 40 MB (Copy2dChunkKernel has the figures).
 constexpr uint64_t kRectChunksMinBytes = 32ull << 20;
 constexpr uint64_t kRectPlainChunksMinBytes = 48ull << 20;
+constexpr uint64_t kRectShortBytes = 64ull << 20;             // launches below keep their schedule where longer ones of such rows lose it
 constexpr uint64_t kRectLaunchBytes = 640ull << 20;
 constexpr uint64_t kWindowPieceBytes = 512ull << 20;          // launches into which long segments are cut
 constexpr uint64_t kWindowLongSegmentBytes = 64ull << 20;     // launches whose segments average this much go out in pieces of kWindowPieceBytes and more

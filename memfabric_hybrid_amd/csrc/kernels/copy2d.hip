@@ -95,7 +95,7 @@ __global__ __launch_bounds__(kRectThreads) void Copy2dKernel(const RectPlan p)
 // pairs of 896 and 4736 bytes, 161 MB 57.5 / - / 51.4, 646 MB 215 / - / 200; of 480 and 2992, 107 MB 45.6 / 38.2 / 34.7, 213 MB 87.6 / - / 67.7; of
 // 736 and 1888, 62 MB 27.0 / 23.7 / 21.3, 247 MB 99.3 / 81.4 / 77.2.  Single rectangles of 896 or 4736 bytes a row with strided source,
 // strided destination or both, 40 MB 17.1 to 17.8 / 16.6 to 17.0 / 14.9 to 15.2, 400 MB 134 to 146 / 129 to 133 / 123 to 129; rows of 480, 2992 or
-// 20 000 bytes, 400 MB 147 to 197 / 129 to 190 / 126 to 201: those go without windows.  Below 32 MiB whole rows are as fast or faster (24 MB
+// 20 000 bytes, 400 MB 147 to 197 / 129 to 190 / 126 to 201: which rows go without windows is RectHolds.  Below 32 MiB whole rows are as fast or faster (24 MB
 // 9.0 to 9.5 / 11.2 to 11.6 / 10.1 to 10.7).
 // kPaced: sixteen loads per lane at the wave's offset into the read half of the period, the stores at the same offset into the
 // write half, as XcopyWindowKernel does for long segments.  Rates of 7.1 TB/s and more fall apart for half of these geometries;

@@ -1157,20 +1157,25 @@ static void TestRectangleChunks()
         const uint64_t word = i * 0x9E3779B97F4A7C15ull + 1;
         std::memcpy(&src[i], &word, 8);
     }
-    struct Form { uint64_t width, gap, sgap; int pairs; bool windows; };   // gap: behind a (pair's) row of the destination, sgap: of the source
+    // gap: behind a (pair's) row of the destination, sgap: of the source
+    struct Form { uint64_t width, gap, sgap; int pairs; bool windows; uint64_t mib = 0; };
     const Form forms[] = {
         {480, 0, 0, 1, true},      // pairs whose rows are no whole lines, against one another
         {416, 32, 16, 1, true},    // pairs with gaps on both sides
         {896, 0, 0, 1, true},      {16, 0, 0, 1, true},       // pairs on lines; of one unit a row
         {20000, 0, 16, 1, true},   // rows longer than a chunk
-        {896, 128, 0, 0, true},    // single ones on lines
+        {896, 128, 0, 0, true},    {896, 0, 128, 0, true},    // single ones on lines, with room between their rows and without
         {480, 480, 0, 0, false},   // single ones between lines: without windows, and as whole rows below 48 MiB
         {2992, 0, 16, 0, false},
         {480, 0, 0, 2, false},     // pairs and single ones in turn: a third of the payload is single
+        {2736, 16, 0, 1, true},    {2736, 16, 0, 1, false, 68},   // pairs that only touch some lines at their rows' ends: in windows while short
+        {960, 64, 0, 1, true, 68}, {2736, 0, 16, 1, true, 68},    // rows that end on 64 bytes, and rows against one another, whatever the length
+        {960, 0, 16, 0, true},     {960, 64, 0, 0, true},         // single ones whose rows end on 64 bytes
+        {960, 0, 128, 0, false},   {192, 64, 0, 0, false},        // lines of which a good part is not read, or not written
     };
     for (const Form &f : forms) {
         const uint64_t spitch = f.width + f.sgap;
-        const uint64_t height = (f.windows ? kBytes : 50ull << 20) / 14 / f.width + 3;     // fourteen rectangles
+        const uint64_t height = (f.mib != 0 ? f.mib << 20 : f.windows ? kBytes : 50ull << 20) / 14 / f.width + 3;     // fourteen rectangles
         std::vector<mf_copy2d_desc> rects;
         uint64_t at = 0;
         const uint64_t dpitch = 2 * f.width + f.gap;
@@ -1180,7 +1185,7 @@ static void TestRectangleChunks()
             const uint64_t from = i * spitch * height % (src.size() - spitch * height) / 16 * 16;
             rects.push_back({from, second ? rects.back().dst + f.width : at, f.width, height, spitch, single ? f.width + f.gap : dpitch});
             if (!second) {
-                at += rects.back().dpitch * height + (f.width % 128 == 0 ? 128 : 48);
+                at += (rects.back().dpitch * height + 127) / 128 * 128 + (f.width % 128 == 0 ? 128 : f.width % 64 == 0 ? 64 : 48);
             }
         }
         std::vector<unsigned char> expect(at + 16, 0xEE);
@@ -1214,7 +1219,8 @@ static void TestRectangleChunks()
                 XcopyEngine::Instance().Tuning().windowAlignedMBps = r.aligned;
                 (void)fake_rt_last_window();
                 CHECK(mf_xcopy_2d_batch(rects.data(), static_cast<uint32_t>(rects.size()), MF_ROUTE_HBM, nullptr) == BM_OK);
-                CHECK(fake_rt_last_window() == (!f.windows ? 0 : !r.scaled ? r.general : lines ? 7000000 : 6900000));
+                const uint32_t scaled = lines && f.pairs == 0 && f.gap == 0 ? 7000000 : f.pairs == 1 && (lines || f.gap == 0) ? 6900000 : 6800000;
+                CHECK(fake_rt_last_window() == (!f.windows ? 0 : r.scaled ? scaled : r.general));
             }
             fake_rt_skip_copies(0);
         }
