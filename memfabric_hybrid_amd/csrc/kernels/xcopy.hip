@@ -1328,8 +1328,10 @@ __device__ __forceinline__ bool PlannedQuad(const uint64_t *__restrict__ triples
 // Segments of one length, as pages are, take a shorter way: one barrier says that they are, and the owner of a chunk is a division instead of
 // a prefix and a search.  us before / so, gathered and scattered: 300 of 32 KiB 5.8 / 5.2, 700 / 1000 / 2000 / 4096 pages of 8 KiB 5.8 / 4.3,
 // 6.6 / 4.8, 8.8 / 7.5, 15.4 and 16.1 / 12.9 and 14.1; 1000 of 32 KiB 13.1 and 13.8 / 12.3 and 12.9, 1000 of 64 KiB 24.1 and 26.3 / 22.7 and
-// 24.3; 3000 of 8200 bytes at odd addresses 13.5 / 11.4.  Finding that out costs other tables 0.1 to 0.2 us, of which the shorter chunks' skipped
-// units give back more to short ones: ragged segments 600 / 1000 of up to 70 000 bytes 10.6 / 10.75, 16.4 / 16.6, 4000 of up to 9000 13.4 / 12.6.  Not
+// 24.3; 3000 of 8200 bytes at odd addresses 13.5 / 11.4.  All of that way stands behind the other one's code: between its parts, instructions
+// that a wave only steps over cost short tables 0.3 us (K and V blocks of 3 MB: no shorter way 4.84, behind 4.91, between 5.28).  Finding out
+// that segments differ costs up to 0.25 us from 513 on (1281 blocks of 26 MB 12.70 / 12.95; 1240 of 32 912 bytes, equal but not full enough, 18.4 / 19.1), of which the shorter
+// chunks' skipped units give back more to short ones: 4000 ragged segments of up to 9000 bytes 13.4 / 12.6.  Not
 // taken: descriptors fetched ahead of that barrier, and all lengths requested by one stretch of code, whatever their number (each
 // request of 64 lengths is 24 lines of the L1): 600 / 1000 ragged ones 11.6 / 17.8.
 // In windows cut for 6.0 / 6.2 / 6.4 / 6.6 / 6.8 TB/s, the same to 0.5 in four processes: 4096 pages of 32 KiB gathered 49.8 / 48.4 / 47.1 / 46.0 / 45.3,
@@ -1384,120 +1386,11 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
     // The form: short tables a chunk of 4 KiB per wave; others 16 KiB, of one segment where those are nearly full or where a source and
     // its destination may differ modulo 16, else of up to four.
     constexpr uint32_t grid = kWindowWaves;
+    constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kWindowUnits) * kUnitBytes;
     uint32_t item = wave * kGroups + blockIdx.x;            // neighbouring ones on neighbouring XCDs
     const bool aligned = __ballot(bits % kUnitBytes != 0) == 0;
-    uint32_t shallowAll = 0;
-    uint32_t deepAll = 0;
-    uint32_t total = 0;
-    bool large = false;
-    bool quads = false;
-    auto choose = [&](uint32_t shallowCount, uint32_t deepCount, uint32_t spareCount) {
-        shallowAll = shallowCount;
-        deepAll = deepCount;
-        total = PlannedTotal(deepAll, spareCount);
-        large = total > kPlannedShallowChunks;
-        quads = large && aligned && !PlannedFull(total, deepAll);
-    };
-    bool equal = __ballot(other) == 0;
-    if (kWaves > 1 && lane == 0) {
-        sums[3 * kWaves + wave] = equal ? 1 : 0;
-    }
-    __syncthreads();
-    if (kWaves > 1) {
-        equal = __ballot(lane < kWaves && sums[3 * kWaves + (lane < kWaves ? lane : 0)] == 0) == 0;
-    }
-    // Segments that all have the length of the first need neither sums nor a prefix.  Pages of up to 16 KiB never go as quads.
-    uint32_t each = 0;
-    if (equal) {
-        const uint32_t shallow0 = static_cast<uint32_t>((len0 + 4095) >> 12);
-        choose(nseg * shallow0, nseg * ((shallow0 + 3) / 4), nseg * PlannedSpare(len0));
-        quads = quads && shallow0 > 4;
-        each = quads ? 0 : large ? (shallow0 + 3) / 4 : shallow0;
-    }
-    if (each == 0) {
-        uint32_t count[kRun];
-        uint32_t shallow = 0;       // chunks of 4 KiB,
-        uint32_t deep = 0;          // of 16 KiB
-#pragma unroll
-        for (uint32_t r = 0; r < kRun; ++r) {
-            const uint32_t seg = threadIdx.x * run + r;
-            count[r] = r < run && seg < nseg ? first[seg] : 0;
-            shallow += count[r];
-            deep += (count[r] + 3) / 4;
-        }
-        const uint32_t shallowUpTo = LanesUpTo(shallow);
-        const uint32_t deepUpTo = LanesUpTo(deep);
-        uint32_t spareAll = __builtin_amdgcn_readlane(LanesUpTo(spare), 63);
-        uint32_t shallowSum = __builtin_amdgcn_readlane(shallowUpTo, 63);
-        uint32_t deepSum = __builtin_amdgcn_readlane(deepUpTo, 63);
-        uint32_t shallowBase = 0;
-        uint32_t deepBase = 0;
-        if (kWaves > 1) {
-            if (lane == 0) {
-                sums[wave] = shallowSum;
-                sums[kWaves + wave] = deepSum;
-                sums[2 * kWaves + wave] = spareAll;
-            }
-            __syncthreads();
-            const uint32_t at = lane < kWaves ? lane : 0;
-            const uint32_t a = LanesUpTo(lane < kWaves ? sums[at] : 0);
-            const uint32_t b = LanesUpTo(lane < kWaves ? sums[kWaves + at] : 0);
-            spareAll = __builtin_amdgcn_readlane(LanesUpTo(lane < kWaves ? sums[2 * kWaves + at] : 0), 63);
-            shallowBase = wave == 0 ? 0 : __builtin_amdgcn_readlane(a, wave == 0 ? 0 : wave - 1);
-            deepBase = wave == 0 ? 0 : __builtin_amdgcn_readlane(b, wave == 0 ? 0 : wave - 1);
-            shallowSum = __builtin_amdgcn_readlane(a, 63);
-            deepSum = __builtin_amdgcn_readlane(b, 63);
-        }
-        choose(shallowSum, deepSum, spareAll);
-        uint32_t before = large && !quads ? deepBase + deepUpTo - deep : shallowBase + shallowUpTo - shallow;
-#pragma unroll
-        for (uint32_t r = 0; r < kRun; ++r) {
-            const uint32_t seg = threadIdx.x * run + r;
-            if (r < run && seg < nseg) {
-                first[seg] = before;
-                before += large && !quads ? (count[r] + 3) / 4 : count[r];
-            }
-        }
-        if (threadIdx.x == 0) {
-            first[nseg] = large && !quads ? deepAll : shallowAll;
-        }
-        __syncthreads();
-    }
-    const bool byDeep = large && !quads;
-    const uint32_t nchunk = byDeep ? deepAll : shallowAll;
-
-    const uint32_t items = quads ? (nchunk + 3) / 4 : nchunk;
-    const bool held = large && items <= grid && total <= kPlannedHeldChunks;
-    const bool paced = large && total > kPlannedHeldChunks && aligned && pace.windowTicks != 0 && PlannedFull(total, items);
-    const uint32_t rounds = (items + grid - 1) / grid;
-    const uint32_t waves = paced ? (items + rounds - 1) / rounds : grid;
-    if (item >= items || item >= waves) {
-        return;
-    }
-    constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kWindowUnits) * kUnitBytes;
-    // Whether the first segments are written, or read, one behind the other, and whether they all lie on multiples of kWindowLongBlockBytes:
-    // the rates that a table of one length holds differ by that.  (With all lanes: what one that is switched off holds is not defined.)
-    const uint32_t sample = nseg < 64 ? nseg : 64;
-    const uint32_t length = static_cast<uint32_t>(len0);
-    const bool pair = lane + 1 < sample;
-    const uint32_t behind = __shfl_down(to, 1, 64);
-    const uint32_t ahead = __shfl_down(from, 1, 64);
-    const bool inOrder = each != 0 && __popcll(__ballot(pair && behind - to == length)) * 4 >= static_cast<int>(sample - 1) * 3;
-    const bool readInOrder = __popcll(__ballot(pair && ahead - from == length)) * 4 >= static_cast<int>(sample - 1) * 3;
-    const bool onGrid = __ballot(((from | to | length) & (kWindowLongBlockBytes - 1)) != 0) == 0;
-    const bool faster = each != 0 && !inOrder && (readInOrder || onGrid || (len0 >= kWindowLongBlockBytes && total * 25ull < items * static_cast<uint64_t>(kPlannedLoosePercent)));
-    const bool shortPages = faster && len0 < kWindowLongBlockBytes;
-    const uint32_t windowTicks = inOrder ? pace.orderedTicks : !faster ? pace.windowTicks : shortPages ? pace.shortTicks : pace.longTicks;
-    const uint32_t period = static_cast<uint32_t>(windowTicks * (waves * kDeepBytes) >> 26);
-    const uint32_t reading = shortPages ? period / 64 * 29 : period / 2;
-    const uint32_t hold = (each != 0 ? pace.equalTicks : pace.holdTicks) +
-                          static_cast<uint32_t>(static_cast<uint64_t>(each != 0 ? pace.equalMoreTicks : pace.holdMoreTicks) * total >> 14);
-    const uint64_t start = paced ? AgreedStart(pace.seq) : 0;
-    uint64_t loadAt = paced ? start + static_cast<uint64_t>(item) * reading / waves : 0;
-    uint64_t storeAt = paced ? start + reading + static_cast<uint64_t>(item) * (period - reading) / waves : held && pace.holdTicks != 0 ? t0 + hold : 0;
-    const uint32_t step = paced ? period : 0;
     // (Each owner with a loop of its own: code that a wave only steps over is fetched all the same, at 0.3 us.)
-    auto deepChunks = [&](auto owner) {
+    auto deepChunks = [&](auto owner, uint32_t items, uint32_t waves, uint64_t loadAt, uint64_t storeAt, uint32_t step) {
         // the next chunk's owner is looked up while the loads of this one are on their way
         ChunkRef r = owner(item);
         for (;;) {
@@ -1517,24 +1410,139 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
             storeAt += step;
         }
     };
-    auto shallowChunks = [&](auto owner) {
+    auto shallowChunks = [&](auto owner, uint32_t items, uint32_t waves) {
         for (; item < items; item += waves) {
             const ChunkRef r = owner(item);
             CopyCountedChunk(r.src, r.dst, r.len, r.k, lane);
         }
     };
-    auto planned = [&](uint32_t c) { return PlannedOwner(triples, first, nseg, c); };
-    auto divided = [&](uint32_t c) { return EqualOwner(triples, each, c); };
-    if (__builtin_expect(each != 0, 0)) {
-        if (byDeep) {
-            deepChunks(divided);
-        } else {
-            shallowChunks(divided);
+    bool equal = __ballot(other) == 0;
+    if (kWaves > 1 && lane == 0) {
+        sums[3 * kWaves + wave] = equal ? 1 : 0;
+    }
+    __syncthreads();
+    if (kWaves > 1) {
+        equal = __ballot(lane < kWaves && sums[3 * kWaves + (lane < kWaves ? lane : 0)] == 0) == 0;
+    }
+    // Segments that all have the length of the first need neither sums nor a prefix.  Pages of up to 16 KiB never go as quads.
+    if (__builtin_expect(equal, 0)) {
+        const uint32_t shallow0 = static_cast<uint32_t>((len0 + 4095) >> 12);
+        const uint32_t deep0 = (shallow0 + 3) / 4;
+        const uint32_t total = PlannedTotal(nseg * deep0, nseg * PlannedSpare(len0));
+        const bool large = total > kPlannedShallowChunks;
+        if (shallow0 != 0 && !(large && aligned && shallow0 > 4 && !PlannedFull(total, nseg * deep0))) {
+            const uint32_t each = large ? deep0 : shallow0;
+            const uint32_t items = nseg * each;
+            const bool held = large && items <= grid && total <= kPlannedHeldChunks;
+            const bool paced = large && total > kPlannedHeldChunks && aligned && pace.windowTicks != 0 && PlannedFull(total, items);
+            const uint32_t rounds = (items + grid - 1) / grid;
+            const uint32_t waves = paced ? (items + rounds - 1) / rounds : grid;
+            if (item >= items || item >= waves) {
+                return;
+            }
+            auto divided = [&](uint32_t c) { return EqualOwner(triples, each, c); };
+            if (!large) {
+                shallowChunks(divided, items, waves);
+                return;
+            }
+            uint64_t loadAt = 0;
+            uint64_t storeAt = 0;
+            uint32_t period = 0;
+            if (paced) {
+                // Whether the first segments are written, or read, one behind the other, and whether they all lie on multiples of kWindowLongBlockBytes:
+                // the rates that the table holds differ by that.  (With all lanes: what one that is switched off holds is not defined.)
+                const uint32_t sample = nseg < 64 ? nseg : 64;
+                const uint32_t length = static_cast<uint32_t>(len0);
+                const bool pair = lane + 1 < sample;
+                const uint32_t behind = __shfl_down(to, 1, 64);
+                const uint32_t ahead = __shfl_down(from, 1, 64);
+                const bool inOrder = __popcll(__ballot(pair && behind - to == length)) * 4 >= static_cast<int>(sample - 1) * 3;
+                const bool readInOrder = __popcll(__ballot(pair && ahead - from == length)) * 4 >= static_cast<int>(sample - 1) * 3;
+                const bool onGrid = __ballot(((from | to | length) & (kWindowLongBlockBytes - 1)) != 0) == 0;
+                const bool faster = !inOrder && (readInOrder || onGrid ||
+                                                 (len0 >= kWindowLongBlockBytes && total * 25ull < items * static_cast<uint64_t>(kPlannedLoosePercent)));
+                const bool shortPages = faster && len0 < kWindowLongBlockBytes;
+                const uint32_t windowTicks = inOrder ? pace.orderedTicks : !faster ? pace.windowTicks : shortPages ? pace.shortTicks : pace.longTicks;
+                period = static_cast<uint32_t>(windowTicks * (waves * kDeepBytes) >> 26);
+                const uint32_t reading = shortPages ? period / 64 * 29 : period / 2;
+                const uint64_t start = AgreedStart(pace.seq);
+                loadAt = start + static_cast<uint64_t>(item) * reading / waves;
+                storeAt = start + reading + static_cast<uint64_t>(item) * (period - reading) / waves;
+            } else if (held && pace.holdTicks != 0) {
+                storeAt = t0 + pace.equalTicks + static_cast<uint32_t>(static_cast<uint64_t>(pace.equalMoreTicks) * total >> 14);
+            }
+            deepChunks(divided, items, waves, loadAt, storeAt, period);
+            return;
         }
+    }
+    uint32_t count[kRun];
+    uint32_t shallow = 0;       // chunks of 4 KiB,
+    uint32_t deep = 0;          // of 16 KiB
+#pragma unroll
+    for (uint32_t r = 0; r < kRun; ++r) {
+        const uint32_t seg = threadIdx.x * run + r;
+        count[r] = r < run && seg < nseg ? first[seg] : 0;
+        shallow += count[r];
+        deep += (count[r] + 3) / 4;
+    }
+    const uint32_t shallowUpTo = LanesUpTo(shallow);
+    const uint32_t deepUpTo = LanesUpTo(deep);
+    uint32_t spareAll = __builtin_amdgcn_readlane(LanesUpTo(spare), 63);
+    uint32_t shallowAll = __builtin_amdgcn_readlane(shallowUpTo, 63);
+    uint32_t deepAll = __builtin_amdgcn_readlane(deepUpTo, 63);
+    uint32_t shallowBase = 0;
+    uint32_t deepBase = 0;
+    if (kWaves > 1) {
+        if (lane == 0) {
+            sums[wave] = shallowAll;
+            sums[kWaves + wave] = deepAll;
+            sums[2 * kWaves + wave] = spareAll;
+        }
+        __syncthreads();
+        const uint32_t at = lane < kWaves ? lane : 0;
+        const uint32_t a = LanesUpTo(lane < kWaves ? sums[at] : 0);
+        const uint32_t b = LanesUpTo(lane < kWaves ? sums[kWaves + at] : 0);
+        spareAll = __builtin_amdgcn_readlane(LanesUpTo(lane < kWaves ? sums[2 * kWaves + at] : 0), 63);
+        shallowBase = wave == 0 ? 0 : __builtin_amdgcn_readlane(a, wave == 0 ? 0 : wave - 1);
+        deepBase = wave == 0 ? 0 : __builtin_amdgcn_readlane(b, wave == 0 ? 0 : wave - 1);
+        shallowAll = __builtin_amdgcn_readlane(a, 63);
+        deepAll = __builtin_amdgcn_readlane(b, 63);
+    }
+    const uint32_t total = PlannedTotal(deepAll, spareAll);
+    const bool large = total > kPlannedShallowChunks;
+    const bool quads = large && aligned && !PlannedFull(total, deepAll);
+    const bool byDeep = large && !quads;
+    uint32_t before = byDeep ? deepBase + deepUpTo - deep : shallowBase + shallowUpTo - shallow;
+#pragma unroll
+    for (uint32_t r = 0; r < kRun; ++r) {
+        const uint32_t seg = threadIdx.x * run + r;
+        if (r < run && seg < nseg) {
+            first[seg] = before;
+            before += byDeep ? (count[r] + 3) / 4 : count[r];
+        }
+    }
+    const uint32_t nchunk = byDeep ? deepAll : shallowAll;
+    if (threadIdx.x == 0) {
+        first[nseg] = nchunk;
+    }
+    __syncthreads();
+
+    const uint32_t items = quads ? (nchunk + 3) / 4 : nchunk;
+    const bool held = large && items <= grid && total <= kPlannedHeldChunks;
+    const bool paced = large && total > kPlannedHeldChunks && aligned && pace.windowTicks != 0 && PlannedFull(total, items);
+    const uint32_t rounds = (items + grid - 1) / grid;
+    const uint32_t waves = paced ? (items + rounds - 1) / rounds : grid;
+    if (item >= items || item >= waves) {
         return;
     }
+    const uint32_t period = static_cast<uint32_t>(pace.windowTicks * (waves * kDeepBytes) >> 26);
+    const uint32_t hold = pace.holdTicks + static_cast<uint32_t>(static_cast<uint64_t>(pace.holdMoreTicks) * total >> 14);
+    uint64_t loadAt = paced ? AgreedStart(pace.seq) + static_cast<uint64_t>(item) * (period / 2) / waves : 0;
+    uint64_t storeAt = paced ? loadAt + period / 2 : held && pace.holdTicks != 0 ? t0 + hold : 0;
+    const uint32_t step = paced ? period : 0;
+    auto planned = [&](uint32_t c) { return PlannedOwner(triples, first, nseg, c); };
     if (byDeep) {
-        deepChunks(planned);
+        deepChunks(planned, items, waves, loadAt, storeAt, step);
         return;
     }
     if (quads) {
@@ -1556,7 +1564,7 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
         }
         return;
     }
-    shallowChunks(planned);
+    shallowChunks(planned, items, waves);
 }
 
 // The segments of a list that a wave is at, one per lane, so that the owner of a piece is found without a load.

@@ -402,7 +402,7 @@ constexpr uint32_t PlannedLds(uint32_t waves, uint32_t nseg)          // bytes: 
     return (nseg + 1 + 4 * waves) * 4;
 }
 constexpr int32_t kTableHoldNanos = 2000;             // held stores of device tables: the wait,
-constexpr uint32_t kTableHoldMoreNanos = 9400;        // and what more for 64 MiB;
+constexpr uint32_t kTableHoldMoreNanos = 8800;        // and what more for 64 MiB (K and V blocks of 32, 48, 62 MB want 600 to 1200 less, ragged ones at odd addresses 300 more);
 constexpr int32_t kTableEqualNanos = 850;             // of tables of segments of one length, whose waves load that much sooner: best
 constexpr uint32_t kTableEqualMoreNanos = 9850;       // waits in steps of 400 ns 5.6 to 5.9 us at 33 MB, 10.2 to 10.6 at 62 to 65 MB
 
