@@ -63,8 +63,9 @@ int32_t mf_xcopy_hold_stores(int32_t nanos);
  * 7 100 000 (32 x 16 MiB back to back: 6.95 instead of 6.65 TB/s), those of 64 MiB and
  * more on average for 7 400 000, and a batch of 1 GiB and more of such long segments is cut into launches of
  * about 512 MiB, which hold their schedule more often than longer ones (1 GiB: 7.1-7.2 instead of 6.7 TB/s).
- * Segments whose source and destination differ modulo 16 take no windows.  Rectangles of 32 MiB and more go at
- * 35/34 of the default rate where all rows are whole lines and at 69/68 elsewhere, lists of more than 128 segments and device
+ * Segments whose source and destination differ modulo 16 take no windows.  Rectangles of 32 MiB and more whose rows hold
+ * windows go at 35/34 of the default rate where rows of whole lines lie against one another in the destination, pairs of
+ * others at 69/68 and those with room between their rows at the rate itself, lists of more than 128 segments and device
  * tables at 15/17 to 33/34 of it.  The call sets all three rates, rectangles take the rate that is set, and the parts are of it; 0
  * switches the form off, MF_XCOPY_WINDOWS_OWN_CHOICE brings back the rates the library chose itself (what
  * hybm_init measured, else the defaults above).  While several threads submit on streams of their own the
