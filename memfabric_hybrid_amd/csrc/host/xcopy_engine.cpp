@@ -2468,9 +2468,11 @@ int XcopyEngine::SubmitDeviceTable(const void *triples, uint32_t n, int route, v
     uint32_t hold = 0;
     uint32_t holdMore = 0;
     uint32_t windows = 0;
-    TablePaceFor(hold, holdMore, windows);
-    if (route == MFRT_ROUTE_HBM && tuning_.unitsOverride == 0 && tuning_.deviceTableWgPerCu == 0 &&
-        n <= (windows != 0 ? kPlannedSegments : 64 * kPlannedShortRun)) {
+    const bool own = route == MFRT_ROUTE_HBM && tuning_.unitsOverride == 0 && tuning_.deviceTableWgPerCu == 0;
+    if (own) {
+        TablePaceFor(hold, holdMore, windows);
+    }
+    if (own && n <= (windows != 0 ? kPlannedSegments : 64 * kPlannedShortRun)) {
         const int err = mfk_xcopy_planned(triples, n, hold, holdMore, windows, mask, maskValue, stream);
         if (err != 0) {
             MF_FAIL(BM_ERROR, "xcopy launch of a device table failed: " << mfrt_error_string(err));
@@ -2501,8 +2503,8 @@ int XcopyEngine::SubmitDeviceTable(const void *triples, uint32_t n, int route, v
         const uint32_t m = n - at < capacity ? n - at : capacity;
         const bool last = m == n - at;
         err = mfk_xcopy_direct(static_cast<const uint64_t *>(triples) + 3ull * at, m, units, route, DeviceTableGrid(m, cu, route, tuning_),
-                               DeviceTableRestGrid(cu, route, tuning_), list, capacity, last ? mask : nullptr, maskValue, stream,
-                               last ? event : nullptr);
+                               DeviceTableRestGrid(cu, route, tuning_), list, capacity, hold, holdMore, windows, last ? mask : nullptr,
+                               maskValue, stream, last ? event : nullptr);
         g_launches.fetch_add(err == 0 ? 2 : 0, std::memory_order_relaxed);
         at += m;
     }

@@ -1065,6 +1065,51 @@ __global__ __launch_bounds__(64) void XcopyPieceWindowKernel(uint64_t list, uint
     }
 }
 
+// How a launch of a device table paces itself; 0: not.
+struct TablePace {
+    uint32_t holdTicks;         // of the clock, what a wave waits before it stores, where all waves of the launch are resident together,
+    uint32_t holdMoreTicks;     // and what more per 64 MiB of the table;
+    uint32_t equalTicks;        // the same where its segments are of one length, whose descriptors are there sooner
+    uint32_t equalMoreTicks;
+    uint32_t windowTicks;       // period in which 64 MiB pass at the rate of random blocks,
+    uint32_t shortTicks;        // of such of one length below kWindowLongBlockBytes, whose write part is the longer one,
+    uint32_t longTicks;         // of such of one length from there on,
+    uint32_t orderedTicks;      // and of blocks of one length that are written one behind the other
+    uint32_t seq;               // of AgreedStart
+};
+
+// The windows that a table of segments of length len0 holds, by 64 segments of it, one a lane: whether they are written, or read, one behind the other, and
+// whether they all lie on multiples of kWindowLongBlockBytes.  `loose`: its chunks of 16 KiB are so short that it holds a higher rate anywhere.  (With all lanes: what
+// one that is switched off holds is not defined.)
+struct TableWindows {
+    uint32_t ticks;             // period in which 64 MiB pass
+    uint32_t reading;           // 64ths of it that are the read part
+};
+__device__ __forceinline__ TableWindows WindowsOf(const TablePace &pace, uint32_t from, uint32_t to, uint64_t len0, uint32_t sample, bool loose)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t length = static_cast<uint32_t>(len0);
+    const bool pair = lane + 1 < sample;
+    const uint32_t behind = __shfl_down(to, 1, 64);
+    const uint32_t ahead = __shfl_down(from, 1, 64);
+    const bool inOrder = __popcll(__ballot(pair && behind - to == length)) * 4 >= static_cast<int>(sample - 1) * 3;
+    const bool readInOrder = __popcll(__ballot(pair && ahead - from == length)) * 4 >= static_cast<int>(sample - 1) * 3;
+    const bool onGrid = __ballot(((from | to | length) & (kWindowLongBlockBytes - 1)) != 0) == 0;
+    const bool faster = !inOrder && (readInOrder || onGrid || (len0 >= kWindowLongBlockBytes && loose));
+    const bool shortPages = faster && len0 < kWindowLongBlockBytes;
+    return TableWindows{inOrder ? pace.orderedTicks : !faster ? pace.windowTicks : shortPages ? pace.shortTicks : pace.longTicks, shortPages ? 29u : 32u};
+}
+
+__device__ __forceinline__ void ListRest(RestList *rest, uint32_t capacity, uint64_t src, uint64_t dst, uint64_t left)
+{
+    if (threadIdx.x == 0) {
+        const uint64_t taken = __hip_atomic_fetch_add(&rest->taken, kRestEntry + RestPieces(left), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (taken / kRestEntry < capacity) {   // which nseg is not more than: calls that share a list against the rules stay inside it
+            rest->entry[taken / kRestEntry] = RestSegment{taken % kRestEntry, src, dst, left};
+        }
+    }
+}
+
 // A table that only the GPU can read, copied as xcopy_plan.h says: item (segment, part), parts in a row.  The launch is sized from
 // the segment count alone, so a workgroup walks the items with the grid as its stride; it fetches the next item's triple before
 // it copies the current item.  What bounds it is HBM; a launch in front of it that planned the table (chunk prefix, owner map,
@@ -1079,12 +1124,19 @@ __global__ __launch_bounds__(64) void XcopyPieceWindowKernel(uint64_t list, uint
 // part numbers that turn from segment to segment, pages 1 % slower; the triples of 64 items at a time, one per lane, so that
 // empty items cost no wait, more registers than eight waves per SIMD have, 10 to 60 % slower on short tables; two triples ahead
 // instead of one, 16 384 segments of 2 to 14 KB 4 % slower.
-template <bool kNtLoad, int kStore>
-__global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_t *__restrict__ triples, uint32_t nseg, uint32_t units,
-                                                                   RestList *__restrict__ rest, uint32_t capacity)
+// What the first kDirectSample segments of a table say of it.
+struct DirectSample {
+    uint32_t parts;             // chunks of the longest, up to kDirectMaxParts
+    bool equal;                 // they have one length, `length`,
+    uint64_t length;
+    bool aligned;               // and lie on units
+};
+__device__ __forceinline__ DirectSample SampleOf(const uint64_t *__restrict__ triples, uint32_t nseg, uint32_t units)
 {
-    const uint32_t sample = (threadIdx.x & 63u) < kDirectSample && (threadIdx.x & 63u) < nseg ? threadIdx.x & 63u : 0;
-    const uint64_t sampled = SegmentChunks(triples[3ull * sample + 1], triples[3ull * sample + 2], units);
+    const uint32_t row = (threadIdx.x & 63u) < kDirectSample && (threadIdx.x & 63u) < nseg ? threadIdx.x & 63u : 0;
+    const uint64_t dst = triples[3ull * row + 1];
+    const uint64_t len = triples[3ull * row + 2];
+    const uint64_t sampled = SegmentChunks(dst, len, units);
     uint32_t parts = 1;
     uint32_t least = kDirectMaxParts;
 #pragma unroll
@@ -1094,6 +1146,14 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_
         least = chunks < least ? chunks : least;
     }
     parts |= least == parts ? 0u : 1u;      // odd in a ragged table: every XCD gets each of them in turn
+    const uint64_t length = Uniform(len);
+    return DirectSample{parts, __ballot(len != length) == 0, length, __ballot(((dst | len) & (kUnitBytes - 1)) != 0) == 0};
+}
+
+template <bool kNtLoad, int kStore>
+__device__ __forceinline__ void CopyDirect(const uint64_t *__restrict__ triples, uint32_t nseg, uint32_t units, RestList *__restrict__ rest,
+                                           uint32_t capacity, uint32_t parts)
+{
     uint32_t seg = blockIdx.x / parts;
     uint32_t part = blockIdx.x - seg * parts;
     if (seg >= nseg) {
@@ -1119,13 +1179,7 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_
         }
         if (part == 0 && chunks > own) {
             const uint64_t at = SegmentGeometry(dst, len).head + own * units * kUnitBytes;
-            if (threadIdx.x == 0) {
-                const uint64_t taken = __hip_atomic_fetch_add(&rest->taken, kRestEntry + RestPieces(len - at), __ATOMIC_RELAXED,
-                                                              __HIP_MEMORY_SCOPE_AGENT);
-                if (taken / kRestEntry < capacity) {   // which nseg is not more than: calls that share a list against the rules stay inside it
-                    rest->entry[taken / kRestEntry] = RestSegment{taken % kRestEntry, src + at, dst + at, len - at};
-                }
-            }
+            ListRest(rest, capacity, src + at, dst + at, len - at);
         }
         if (!more) {
             return;
@@ -1138,18 +1192,144 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_
     }
 }
 
-// How a launch of a device table paces itself; 0: not.
-struct TablePace {
-    uint32_t holdTicks;         // of the clock, what a wave waits before it stores, where all waves of the launch are resident together,
-    uint32_t holdMoreTicks;     // and what more per 64 MiB of the table;
-    uint32_t equalTicks;        // the same where its segments are of one length, whose descriptors are there sooner
-    uint32_t equalMoreTicks;
-    uint32_t windowTicks;       // period in which 64 MiB pass at the rate of random blocks,
-    uint32_t shortTicks;        // of such of one length below kWindowLongBlockBytes, whose write part is the longer one,
-    uint32_t longTicks;         // of such of one length from there on,
-    uint32_t orderedTicks;      // and of blocks of one length that are written one behind the other
-    uint32_t seq;               // of AgreedStart
-};
+template <bool kNtLoad, int kStore>
+__global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_t *__restrict__ triples, uint32_t nseg, uint32_t units,
+                                                                   RestList *__restrict__ rest, uint32_t capacity)
+{
+    CopyDirect<kNtLoad, kStore>(triples, nseg, units, rest, capacity, SampleOf(triples, nseg, units).parts);
+}
+
+// kWindowUnits units on units, of kParts places, loads and stores by the clock.
+template <uint32_t kParts>
+__device__ __forceinline__ void CopyWholeWindowed(const uint64_t (&src)[kParts], const uint64_t (&dst)[kParts], uint64_t loadAt, uint64_t storeAt)
+{
+    constexpr uint32_t kEach = kWindowDepth / kParts;
+    const uint32_t lane = threadIdx.x * kUnitBytes;     // beside a scalar base in every access
+    u32x4 v[kWindowDepth];
+    WaitForClock(loadAt);
+#pragma unroll
+    for (uint32_t j = 0; j < kWindowDepth; ++j) {
+        const uint64_t at = src[j / kEach] + j % kEach * 64 * kUnitBytes;
+        v[j] = __builtin_nontemporal_load(reinterpret_cast<const MF_GLOBAL u32x4 *>(reinterpret_cast<const MF_GLOBAL uint8_t *>(at) + lane));
+    }
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+    WaitForClock(storeAt);
+#pragma unroll
+    for (uint32_t j = 0; j < kWindowDepth; ++j) {
+        const uint64_t at = dst[j / kEach] + j % kEach * 64 * kUnitBytes;
+        __builtin_nontemporal_store(v[j], reinterpret_cast<MF_GLOBAL u32x4 *>(reinterpret_cast<MF_GLOBAL uint8_t *>(at) + lane));
+    }
+}
+
+// The same for tables of more than kPlannedSegments between HBM addresses, one wave a workgroup.  Where the sampled segments are pages of one
+// length, whole chunks of 16 KiB or a half or a quarter of one, and lie on units, the first waves copy all of the table in windows as those of
+// XcopyPlannedKernel do, by the rates that it has measured, and the others leave.  A segment that is not what was seen is listed for the second launch, as
+// what long ones leave is.  HBM is the bound; without windows it sees reads and writes mixed.  us without / so, gathered, scattered: 5000 pages of 8 KiB 19.8 / 19.0,
+// 20.8 / 19.6, 16 384 54.5 / 47.7, 59.9 / 49.9; of 16 KiB 33.4 / 31.5, 35.8 / 33.7, 94.7 / 89.3, 106 / 94.5; of 32 KiB 60.9 / 56.8, 66.7 / 60.8, 187 / 175, 208 / 191;
+// 8000 of 64 KiB 188 / 169, 204 / 176; 5000 of 128 KiB 242 / 211, 258 / 219; of 4 KiB 8000 19.4 / 16.5, 20.0 / 17.0, 16 384 35.7 / 27.3, 37.9 / 28.1, but 4100 13.5 / 13.1,
+// 12.0 / 12.8, hence kSampledQuarters.  Every other table pays for its look at the rule only: 16 384 segments of 2 to 14 KB 56.4 / 56.4, at odd addresses 64.3 / 64.8.
+// That asks for six waves per SIMD, as the kernel without windows has (with five, and 64 segments looked at by every wave, 64.3 / 85.8).  Not taken: the
+// stores of up to 5120 waves held instead (8000 of 8 KiB 28.2 / 29.5: four workgroups a segment start, most of them only to leave, and take the place of
+// those that load); pages that are no whole chunks, whose code would cost the registers.
+constexpr uint32_t kSampledWavesPerSimd = 6;
+constexpr uint32_t kSampledQuarters = 6144;             // segments of 4 KiB, at the least
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSampledWavesPerSimd, kSampledWavesPerSimd))) void XcopySampledKernel(
+    uint64_t table, uint32_t nseg, uint64_t list, uint32_t capacity, TablePace pace)
+{
+    if (nseg == 0) {
+        return;
+    }
+    const uint64_t *const triples = Buffer<const uint64_t>(table);
+    RestList *const rest = Buffer<RestList>(list);
+    constexpr uint32_t kDeepBytes = kWindowUnits * kUnitBytes;
+    const DirectSample seen = SampleOf(triples, nseg, kXcopyThreads);
+    const uint64_t len0 = seen.length;
+    const uint32_t together = len0 == kDeepBytes / 2 ? 2 : len0 == kDeepBytes / 4 && nseg >= kSampledQuarters ? 4 : 1;    // segments a wave
+    const uint32_t each = together != 1 ? 1 : len0 % kDeepBytes == 0 && len0 <= kSampledMostBytes ? static_cast<uint32_t>(len0) / kDeepBytes : 0;
+    const uint32_t items = (nseg + together - 1) / together * each;
+    if (!seen.equal || !seen.aligned || each == 0) {
+        CopyDirect<true, kStoreStream>(triples, nseg, kXcopyThreads, rest, capacity, seen.parts);
+        return;
+    }
+    const uint32_t rounds = (items + kWindowWaves - 1) / kWindowWaves;
+    const uint32_t waves = (items + rounds - 1) / rounds;
+    uint32_t item = blockIdx.x;
+    if (item >= waves) {
+        return;
+    }
+    const uint64_t *t = triples + 3ull * threadIdx.x;           // more than kPlannedSegments: a row for every lane
+    const TableWindows w = WindowsOf(pace, static_cast<uint32_t>(t[0]), static_cast<uint32_t>(t[1]), len0, 64, false);
+    const uint32_t period = static_cast<uint32_t>(static_cast<uint64_t>(w.ticks) * (waves * kDeepBytes) >> 26);
+    const uint32_t reading = w.reading == 32 ? period / 2 : period / 64 * w.reading;
+    const uint64_t start = AgreedStart(pace.seq);
+    uint64_t loadAt = start + static_cast<uint64_t>(item) * reading / waves;
+    uint64_t storeAt = start + reading + static_cast<uint64_t>(item) * (period - reading) / waves;
+    // by scalar loads: a table is not written while a launch reads it
+    const auto *const rows = reinterpret_cast<const __attribute__((address_space(4))) uint64_t *>(table);
+    auto asSeen = [&](const uint64_t (&row)[3]) { return row[2] == len0 && ((row[0] | row[1]) & (kUnitBytes - 1)) == 0; };
+    auto leave = [&](const uint64_t (&row)[3]) {
+        if (row[2] != 0) {
+            ListRest(rest, capacity, row[0], row[1], row[2]);
+        }
+    };
+    auto shorter = [&](auto count) {
+        constexpr uint32_t kParts = decltype(count)::value;
+        for (;; item += waves, loadAt += period, storeAt += period) {
+            uint64_t src[kParts];
+            uint64_t dst[kParts];
+            bool all = true;
+#pragma unroll
+            for (uint32_t j = 0; j < kParts; ++j) {
+                const uint32_t seg = item * kParts + j < nseg ? item * kParts + j : nseg - 1;       // the last again rather than none
+                const uint64_t row[3] = {rows[3ull * seg], rows[3ull * seg + 1], rows[3ull * seg + 2]};
+                src[j] = row[0];
+                dst[j] = row[1];
+                all = all && asSeen(row);
+            }
+            if (all) {
+                CopyWholeWindowed<kParts>(src, dst, loadAt, storeAt);
+            } else {
+#pragma unroll 1
+                for (uint32_t seg = item * kParts; seg < nseg && seg < (item + 1) * kParts; ++seg) {
+                    leave({rows[3ull * seg], rows[3ull * seg + 1], rows[3ull * seg + 2]});        // those that are as seen too
+                }
+            }
+            if (items - item <= waves) {
+                return;
+            }
+        }
+    };
+    if (together == 2) {
+        shorter(std::integral_constant<uint32_t, 2>());
+        return;
+    }
+    if (together == 4) {
+        shorter(std::integral_constant<uint32_t, 4>());
+        return;
+    }
+    uint32_t seg = item / each;
+    uint64_t row[3] = {rows[3ull * seg], rows[3ull * seg + 1], rows[3ull * seg + 2]};
+    for (;;) {
+        const uint32_t k = item - seg * each;
+        const bool more = items - item > waves;
+        item += more ? waves : 0;
+        seg = item / each;
+        const uint64_t next[3] = {rows[3ull * seg], rows[3ull * seg + 1], rows[3ull * seg + 2]};      // requested now, needed after the copy
+        if (asSeen(row)) {
+            CopyWholeWindowed<1>({row[0] + k * kDeepBytes}, {row[1] + k * kDeepBytes}, loadAt, storeAt);
+        } else if (k == 0) {
+            leave(row);
+        }
+        if (!more) {
+            return;
+        }
+        row[0] = next[0];
+        row[1] = next[1];
+        row[2] = next[2];
+        loadAt += period;
+        storeAt += period;
+    }
+}
 
 // The sum of the lanes up to and with this one.
 __device__ __forceinline__ uint32_t LanesUpTo(uint32_t v)
@@ -1449,22 +1629,10 @@ void XcopyPlannedKernel(uint64_t table, uint32_t nseg, TablePace pace)
             uint64_t storeAt = 0;
             uint32_t period = 0;
             if (paced) {
-                // Whether the first segments are written, or read, one behind the other, and whether they all lie on multiples of kWindowLongBlockBytes:
-                // the rates that the table holds differ by that.  (With all lanes: what one that is switched off holds is not defined.)
-                const uint32_t sample = nseg < 64 ? nseg : 64;
-                const uint32_t length = static_cast<uint32_t>(len0);
-                const bool pair = lane + 1 < sample;
-                const uint32_t behind = __shfl_down(to, 1, 64);
-                const uint32_t ahead = __shfl_down(from, 1, 64);
-                const bool inOrder = __popcll(__ballot(pair && behind - to == length)) * 4 >= static_cast<int>(sample - 1) * 3;
-                const bool readInOrder = __popcll(__ballot(pair && ahead - from == length)) * 4 >= static_cast<int>(sample - 1) * 3;
-                const bool onGrid = __ballot(((from | to | length) & (kWindowLongBlockBytes - 1)) != 0) == 0;
-                const bool faster = !inOrder && (readInOrder || onGrid ||
-                                                 (len0 >= kWindowLongBlockBytes && total * 25ull < items * static_cast<uint64_t>(kPlannedLoosePercent)));
-                const bool shortPages = faster && len0 < kWindowLongBlockBytes;
-                const uint32_t windowTicks = inOrder ? pace.orderedTicks : !faster ? pace.windowTicks : shortPages ? pace.shortTicks : pace.longTicks;
-                period = static_cast<uint32_t>(windowTicks * (waves * kDeepBytes) >> 26);
-                const uint32_t reading = shortPages ? period / 64 * 29 : period / 2;
+                const TableWindows w = WindowsOf(pace, from, to, len0, nseg < 64 ? nseg : 64,
+                                                 total * 25ull < items * static_cast<uint64_t>(kPlannedLoosePercent));
+                period = static_cast<uint32_t>(w.ticks * (waves * kDeepBytes) >> 26);
+                const uint32_t reading = w.reading == 32 ? period / 2 : period / 64 * w.reading;
                 const uint64_t start = AgreedStart(pace.seq);
                 loadAt = start + static_cast<uint64_t>(item) * reading / waves;
                 storeAt = start + reading + static_cast<uint64_t>(item) * (period - reading) / waves;
@@ -1864,12 +2032,18 @@ int LaunchPieces(void (*kernel)(uint64_t, uint32_t, uint32_t, uint32_t, uint64_t
     return LaunchWithEvent(kernel, grid, lanes, stream, event, At(pieces), count, ticks, value, At(word), At(counter));
 }
 
+// `pace`: of tables that may go as XcopySampledKernel's, else null.
 template <bool kNtLoad, int kStore>
 int LaunchDirect(const uint64_t *triples, uint32_t nseg, uint32_t units, uint32_t grid, uint32_t restGrid, uint32_t lanes, RestList *rest,
-                 uint32_t capacity, hipStream_t stream, hipEvent_t event)
+                 uint32_t capacity, hipStream_t stream, hipEvent_t event, const TablePace *pace = nullptr)
 {
-    hipLaunchKernelGGL((XcopyDirectKernel<kNtLoad, kStore>), dim3(grid), dim3(lanes), 0, stream, triples, nseg, units, rest, capacity);
-    hipError_t err = hipGetLastError();
+    hipError_t err = hipSuccess;
+    if (kStore == kStoreStream && pace != nullptr && lanes == 64) {
+        err = static_cast<hipError_t>(Launch(XcopySampledKernel, grid, 64, 0, stream, At(triples), nseg, At(rest), capacity, *pace));
+    } else {
+        hipLaunchKernelGGL((XcopyDirectKernel<kNtLoad, kStore>), dim3(grid), dim3(lanes), 0, stream, triples, nseg, units, rest, capacity);
+        err = hipGetLastError();
+    }
     if (err != hipSuccess) {
         return static_cast<int>(err);
     }
@@ -1880,6 +2054,22 @@ int LaunchDirect(const uint64_t *triples, uint32_t nseg, uint32_t units, uint32_
         (void)Launch(XcopySignalKernel, 1, 64, 0, stream, At(&rest->taken), 0u);
     }
     return static_cast<int>(err);
+}
+
+TablePace PaceOf(uint32_t holdNanos, uint32_t holdMoreNanos, uint32_t windowMBps)
+{
+    const uint32_t sooner = holdMoreNanos != 0 ? kTableHoldNanos - kTableEqualNanos : 0;     // a wait set by hand is what it is
+    const uint32_t equalNanos = holdNanos > sooner ? holdNanos - sooner : holdNanos;
+    const uint32_t khz = ClockKhz();
+    return TablePace{TicksOf(holdNanos, khz),
+                     TicksOf(holdMoreNanos, khz),
+                     TicksOf(equalNanos, khz),
+                     TicksOf(holdMoreNanos != 0 ? holdMoreNanos + kTableEqualMoreNanos - kTableHoldMoreNanos : 0, khz),
+                     WindowPeriodTicksAt(2ull << 26, windowMBps, khz),
+                     WindowPeriodTicksAt(2ull << 26, windowMBps / 20 * 21, khz),
+                     WindowPeriodTicksAt(2ull << 26, windowMBps / 15 * 16, khz),
+                     WindowPeriodTicksAt(2ull << 26, windowMBps / 20 * 22, khz),
+                     NextWindowSeq()};
 }
 
 int Signal(void *mask, uint32_t maskValue, hipStream_t stream)
@@ -2089,17 +2279,21 @@ extern "C" int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, 
 
 // rest: a RestList with room for `capacity` segments, its counts 0.
 extern "C" int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *rest,
-                                uint32_t capacity, void *mask, uint32_t maskValue, void *stream, void *event)
+                                uint32_t capacity, uint32_t holdNanos, uint32_t holdMoreNanos, uint32_t windowMBps, void *mask, uint32_t maskValue,
+                                void *stream, void *event)
 {
     using namespace mf;
     if (nseg == 0 || nseg > capacity || grid == 0 || restGrid == 0 || rest == nullptr) {
         return -1;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
+    // (grid: the waves that are held or paced have to be there)
+    const bool sampled = windowMBps != 0 && route == MFRT_ROUTE_HBM && nseg > kPlannedSegments && grid >= kHeldMaxPieces;
+    const TablePace pace = sampled ? PaceOf(holdNanos, holdMoreNanos, windowMBps) : TablePace{};
     const int err = WithPolicy(PolicyOf(route), [&](auto ntLoad, auto store) {
         return LaunchDirect<decltype(ntLoad)::value, decltype(store)::value>(static_cast<const uint64_t *>(triples), nseg, units, grid, restGrid,
-                                                                             LanesFor(units, route), static_cast<RestList *>(rest),
-                                                                             capacity, s, static_cast<hipEvent_t>(event));
+                                                                             LanesFor(units, route), static_cast<RestList *>(rest), capacity, s,
+                                                                             static_cast<hipEvent_t>(event), sampled && pace.windowTicks != 0 ? &pace : nullptr);
     });
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
@@ -2112,18 +2306,7 @@ extern "C" int mfk_xcopy_planned(const void *triples, uint32_t nseg, uint32_t ho
         return -1;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const uint32_t sooner = holdMoreNanos != 0 ? kTableHoldNanos - kTableEqualNanos : 0;     // a wait set by hand is what it is
-    const uint32_t equalNanos = holdNanos > sooner ? holdNanos - sooner : holdNanos;
-    const uint32_t khz = ClockKhz();
-    const TablePace pace{TicksOf(holdNanos, khz),
-                         TicksOf(holdMoreNanos, khz),
-                         TicksOf(equalNanos, khz),
-                         TicksOf(holdMoreNanos != 0 ? holdMoreNanos + kTableEqualMoreNanos - kTableHoldMoreNanos : 0, khz),
-                         WindowPeriodTicksAt(2ull << 26, windowMBps, khz),
-                         WindowPeriodTicksAt(2ull << 26, windowMBps / 20 * 21, khz),
-                         WindowPeriodTicksAt(2ull << 26, windowMBps / 15 * 16, khz),
-                         WindowPeriodTicksAt(2ull << 26, windowMBps / 20 * 22, khz),
-                         NextWindowSeq()};
+    const TablePace pace = PaceOf(holdNanos, holdMoreNanos, windowMBps);
     const int err = nseg <= 64 * kPlannedShortRun
                         ? Launch(XcopyPlannedKernel<1, kPlannedShortRun>, kWindowWaves, 64, PlannedLds(1, nseg), s, At(triples), nseg, pace)
                         : Launch(XcopyPlannedKernel<kPlannedWaves, kPlannedRun>, kWindowWaves / kPlannedWaves, 64 * kPlannedWaves,
@@ -2177,6 +2360,7 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
                 (void)Launch(XcopyPieceWindowKernel, 1, 64, 0, s, 0, 0u, 64u, NextWindowSeq(), 1u, 0u, 0);
                 (void)Launch(XcopyPlannedKernel<1, kPlannedShortRun>, 1, 64, 64, s, 0, 0u, TablePace{});
                 (void)Launch(XcopyPlannedKernel<kPlannedWaves, kPlannedRun>, 1, 64 * kPlannedWaves, 64, s, 0, 0u, TablePace{});
+                (void)Launch(XcopySampledKernel, 1, 64, 0, s, 0, 0u, 0, 0u, TablePace{});
                 hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt, false>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
                 hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt, true>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
             }
@@ -2398,8 +2582,8 @@ extern "C" int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32
     if (guarded && g_staticUsed[dev] && g_staticLast[dev] != s && hipStreamWaitEvent(s, g_staticDone[dev], 0) != hipSuccess) {
         return static_cast<int>(hipGetLastError());
     }
-    const int err = mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, g_scratchOf[dev], kStaticRestCapacity, nullptr, 0, stream,
-                                     nullptr);
+    const int err = mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, g_scratchOf[dev], kStaticRestCapacity, 0, 0, 0, nullptr, 0,
+                                     stream, nullptr);
     if (guarded && hipEventRecord(g_staticDone[dev], s) == hipSuccess) {
         g_staticLast[dev] = s;
         g_staticUsed[dev] = true;

@@ -379,6 +379,7 @@ constexpr uint32_t kPlannedSegments = 64 * kPlannedWaves * kPlannedRun;
 constexpr uint32_t kPlannedFullPercent = 85;          // pieces of 16 KiB that are less full gain nothing from windows,
 constexpr uint32_t kPlannedLoosePercent = 94;         // and those that are less full than this hold a higher rate wherever they lie
 constexpr uint64_t kWindowLongBlockBytes = 64ull << 10;   // blocks of one length from here on, at multiples of it, hold a higher rate in any order
+constexpr uint64_t kSampledMostBytes = 1ull << 20;         // of a segment of a longer table that goes by what its first ones are: fewer than 2^32 chunks
 constexpr uint32_t kPlannedShallowChunks = 1024;
 constexpr uint32_t kPlannedHeldChunks = 16384;
 // What the last piece of 16 KiB of a segment lacks, in 256 bytes, and the payload of `deep` such pieces that lack `spare`, in 4 KiB.

@@ -517,7 +517,7 @@ int mfk_xcopy_pieces_reported(const void *pieces, uint32_t count, uint64_t bytes
 // The direct copy of a device-resident table restated: the parts of every segment, and the pieces of what long ones have left out
 // of a list.
 int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int, uint32_t grid, uint32_t restGrid, void *rest,
-                     uint32_t capacity, void *mask, uint32_t maskValue, void *stream, void *event)
+                     uint32_t capacity, uint32_t, uint32_t, uint32_t, void *mask, uint32_t maskValue, void *stream, void *event)
 {
     if (event != nullptr) {
         (void)mfrt_event_record(event, stream);
@@ -622,7 +622,7 @@ int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, i
     if (nseg == 0 || nseg > MFK_STATIC_TABLE_SEGMENTS) {
         return -1;
     }
-    return mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, list.data(), MFK_STATIC_TABLE_SEGMENTS, nullptr, 0, stream, nullptr);
+    return mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, list.data(), MFK_STATIC_TABLE_SEGMENTS, 0, 0, 0, nullptr, 0, stream, nullptr);
 }
 
 static uint32_t g_lastRectMates = 0;

@@ -188,3 +188,50 @@ def test_windowed_tables_of_pages_in_order_and_not(gpu, count, size, ordered):
     index = torch.from_numpy(at // size).cuda()
     to = torch.from_numpy(place // size).cuda()
     assert torch.equal(target.view(count, size)[to], source.view(2 * count, size)[index])
+
+
+# Longer tables whose first segments have one length and lie on units, and so decide what all are taken for, while others are shorter,
+# empty, a chunk of 16 KiB and a little, longer than their share, at odd addresses.
+ODD = [0, 1, 15, 16, 17, 16383, 16384, 16385, 32768, 32769, 49157, 100003, (1 << 20) + 5, 300007]
+
+
+@pytest.mark.parametrize("count,size,odd,launches", [
+    (4097, 8192, False, 2), (8191, 8192, True, 2), (8193, 8192, True, 2), (4097, 16384, True, 2), (4097, 14000, False, 2),
+    (4097, 32768, True, 2), (4500, 40960, True, 2), (9000, 16384, True, 2), (4097, 16, True, 2), (4097, 65536, False, 2),
+    (65600, 16384, True, 4), (10241, 8000, True, 2), (16385, 8192, True, 2), (16384, 4096, True, 2), (16387, 4096, True, 2), (6143, 4096, False, 2),
+    (6145, 4096, False, 2),
+])
+def test_longer_tables_by_what_their_first_segments_are(gpu, count, size, odd, launches):
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(count + size)
+    lens = np.full(count, size, dtype=np.int64)
+    shift = np.zeros((2, count), dtype=np.int64)
+    if odd:
+        which = 64 + rng.permutation(count - 64)[:5 * len(ODD)]
+        lens[which] = np.tile(ODD, 5)
+        shift[:, which] = rng.integers(0, 16, (2, len(which)))
+        lens[-1], shift[0, -1] = 100003, 3
+    steps = (lens + 191) // 128 * 128
+    order = rng.permutation(count)
+    at = np.cumsum(steps) - steps + shift[0]
+    place = np.empty(count, dtype=np.int64)
+    place[order] = np.cumsum(steps[order]) - steps[order]
+    place += shift[1]
+    room = int(steps.sum()) + 4096
+    source = torch.randint(0, 256, (room,), dtype=torch.uint8, device="cuda")
+    before = torch.randint(0, 256, (room,), dtype=torch.uint8, device="cuda")
+    target = before.clone()
+    table = torch.from_numpy(np.stack([source.data_ptr() + at, target.data_ptr() + place, lens], axis=1)).cuda()
+    torch.cuda.synchronize()
+    expect, data = before.cpu().numpy(), source.cpu().numpy()
+    for s, d, l in zip(at, place, lens):
+        expect[d:d + l] = data[s:s + l]
+    expect = torch.from_numpy(expect).cuda()
+    for _ in range(2):                                           # twice: a list that the first call leaves behind shows
+        target.copy_(before)
+        torch.cuda.synchronize()
+        counted = gpu.mf_xcopy_launch_count()
+        assert gpu.mf_xcopy_device_table(table.data_ptr(), count, native.ROUTE_HBM, None) == 0, native.last_error()
+        assert gpu.mfrt_device_sync() == 0
+        assert gpu.mf_xcopy_launch_count() - counted == launches
+        assert torch.equal(target, expect)
