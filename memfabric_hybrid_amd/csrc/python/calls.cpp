@@ -11,16 +11,19 @@
 // A call takes it out of the thread's hands: an element's __int__ may make a batch call of its own.  The module is linked against libmf_hip_dataplane.so.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
+#include <structmember.h>
 #if PY_VERSION_HEX < 0x030C0000
 #include <longintrepr.h>
 #endif
 
+#include <cstddef>
 #include <cstdint>
 #include <cstring>
 #include <memory>
 #include <new>
 #include <utility>
 
+#include "../../../include/mf_hip_dataplane.h"
 #include "../../../include/mf_xcopy_api.h"
 
 namespace {
@@ -420,12 +423,170 @@ PyCFunction AsMethod(F f)
     return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f));
 }
 
+// A function of the C API that takes addresses and numbers only, in the place of its ctypes object: plain ints, and None for an address, go to it as
+// they are; a call with anything else, and every attribute, is the ctypes object's.  ctypes looks a converter up and calls it for every argument: a dispatch
+// and a combine of the decode path, 22 arguments, FIGURES.
+struct Direct {
+    PyObject_HEAD
+    vectorcallfunc call;
+    PyObject *function;     // the ctypes object
+    PyObject *(*direct)(const uint64_t *args);      // null once something has been set on that: its types may be others
+    const char *kinds;      // an argument each: 'p' address, 'i' number
+};
+
+bool Plain(PyObject *const *args, const char *kinds, uint64_t *words)
+{
+    for (; *kinds != '\0'; ++kinds, ++args, ++words) {
+        if (PyLong_CheckExact(*args)) {
+            *words = WordOfInt(*args);
+        } else if (*args == Py_None && *kinds == 'p') {
+            *words = 0;
+        } else {
+            return false;
+        }
+    }
+    return true;
+}
+
+PyObject *CallDirect(PyObject *self, PyObject *const *args, size_t nargsf, PyObject *names)
+{
+    const auto *d = reinterpret_cast<const Direct *>(self);
+    constexpr size_t kMost = 16;
+    uint64_t words[kMost];
+    if (names == nullptr && d->direct != nullptr && static_cast<size_t>(PyVectorcall_NARGS(nargsf)) == std::strlen(d->kinds) &&
+        Plain(args, d->kinds, words)) {
+        return d->direct(words);
+    }
+    return PyObject_Vectorcall(d->function, args, nargsf, names);
+}
+
+template <class T>
+T *Address(uint64_t word)
+{
+    return reinterpret_cast<T *>(word);
+}
+
+uint32_t Number(uint64_t word)
+{
+    return static_cast<uint32_t>(word);
+}
+
+PyObject *MoeDispatch(const uint64_t *a)
+{
+    int32_t ret = 0;
+    Py_BEGIN_ALLOW_THREADS;
+    ret = mf_moe_dispatch(Address<const void>(a[0]), Address<const int32_t>(a[1]), Number(a[2]), Number(a[3]), Number(a[4]), Number(a[5]),
+                          Address<void>(a[6]), Address<int32_t>(a[7]), Address<int32_t>(a[8]), Address<int32_t>(a[9]), Address<int32_t>(a[10]),
+                          Address<void>(a[11]), a[12], Address<void>(a[13]));
+    Py_END_ALLOW_THREADS;
+    return PyLong_FromLong(ret);
+}
+
+PyObject *MoeCombine(const uint64_t *a)
+{
+    int32_t ret = 0;
+    Py_BEGIN_ALLOW_THREADS;
+    ret = mf_moe_combine(Address<const void>(a[0]), Address<const int32_t>(a[1]), Address<const float>(a[2]), Number(a[3]), Number(a[4]), Number(a[5]),
+                         Address<void>(a[6]), Address<void>(a[7]));
+    Py_END_ALLOW_THREADS;
+    return PyLong_FromLong(ret);
+}
+
+PyObject *DeviceTable(const uint64_t *a)
+{
+    int32_t ret = 0;
+    Py_BEGIN_ALLOW_THREADS;
+    ret = mf_xcopy_device_table(Address<const void>(a[0]), Number(a[1]), static_cast<int32_t>(Number(a[2])), Address<void>(a[3]));
+    Py_END_ALLOW_THREADS;
+    return PyLong_FromLong(ret);
+}
+
+struct DirectKind {
+    const char *name;
+    const char *kinds;
+    PyObject *(*direct)(const uint64_t *args);
+};
+constexpr DirectKind kDirects[] = {
+    {"mf_moe_dispatch", "ppiiiippppppip", MoeDispatch},
+    {"mf_moe_combine", "pppiiipp", MoeCombine},
+    {"mf_xcopy_device_table", "piip", DeviceTable},
+};
+
+void DirectDealloc(PyObject *self)
+{
+    PyTypeObject *type = Py_TYPE(self);
+    Py_XDECREF(reinterpret_cast<Direct *>(self)->function);
+    type->tp_free(self);
+    Py_DECREF(type);
+}
+
+PyObject *DirectGet(PyObject *self, PyObject *name)
+{
+    PyObject *function = reinterpret_cast<Direct *>(self)->function;
+    if (PyUnicode_CompareWithASCIIString(name, "_as_parameter_") == 0) {    // where ctypes is given a function
+        Py_INCREF(function);
+        return function;
+    }
+    return PyObject_GetAttr(function, name);
+}
+
+int DirectSet(PyObject *self, PyObject *name, PyObject *value)
+{
+    auto *d = reinterpret_cast<Direct *>(self);
+    d->direct = nullptr;
+    return PyObject_SetAttr(d->function, name, value);
+}
+
+PyMemberDef g_directMembers[] = {
+    {"__vectorcalloffset__", T_PYSSIZET, offsetof(Direct, call), READONLY, nullptr},
+    {nullptr, 0, 0, 0, nullptr},
+};
+PyType_Slot g_directSlots[] = {
+    {Py_tp_dealloc, reinterpret_cast<void *>(DirectDealloc)},
+    {Py_tp_getattro, reinterpret_cast<void *>(DirectGet)},
+    {Py_tp_setattro, reinterpret_cast<void *>(DirectSet)},
+    {Py_tp_call, reinterpret_cast<void *>(PyVectorcall_Call)},
+    {Py_tp_members, g_directMembers},
+    {0, nullptr},
+};
+PyType_Spec g_directSpec = {"_calls.Direct", sizeof(Direct), 0, Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_VECTORCALL, g_directSlots};
+PyTypeObject *g_directType = nullptr;
+
+// direct(name, function): what stands for the ctypes object of that function, or the object itself where there is nothing
+PyObject *MakeDirect(PyObject *, PyObject *const *args, Py_ssize_t given)
+{
+    if (!Arguments(given, 2)) {
+        return nullptr;
+    }
+    const char *name = PyUnicode_AsUTF8(args[0]);
+    if (name == nullptr) {
+        return nullptr;
+    }
+    for (const DirectKind &kind : kDirects) {
+        if (std::strcmp(kind.name, name) == 0) {
+            auto *d = PyObject_New(Direct, g_directType);
+            if (d == nullptr) {
+                return nullptr;
+            }
+            d->call = CallDirect;
+            Py_INCREF(args[1]);
+            d->function = args[1];
+            d->direct = kind.direct;
+            d->kinds = kind.kinds;
+            return reinterpret_cast<PyObject *>(d);
+        }
+    }
+    Py_INCREF(args[1]);
+    return args[1];
+}
+
 PyMethodDef g_methods[] = {
     {"copy", AsMethod(Copy), METH_FASTCALL, "copy(handle, source, destination, size, type, flags) -> code"},
     {"copy_batch", AsMethod(CopyBatch), METH_FASTCALL,
      "copy_batch(handle, sources, destinations, sizes, count, type, flags) -> code"},
     {"transfer_batch", AsMethod(TransferBatch), METH_FASTCALL,
      "transfer_batch(handle, write, peer, buffers, peer_buffers, lengths, submit, stream, flags) -> code"},
+    {"direct", AsMethod(MakeDirect), METH_FASTCALL, "direct(name, function): a function that is called without ctypes where that is possible"},
     {"fill", AsMethod(Fill), METH_FASTCALL, "fill(array, values): the values as 64-bit words in the array"},
     {nullptr, nullptr, 0, nullptr},
 };
@@ -437,5 +598,6 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_calls", "Native calls of the Py
 
 PyMODINIT_FUNC PyInit__calls(void)
 {
-    return PyModule_Create(&g_module);
+    g_directType = reinterpret_cast<PyTypeObject *>(PyType_FromSpec(&g_directSpec));
+    return g_directType == nullptr ? nullptr : PyModule_Create(&g_module);
 }

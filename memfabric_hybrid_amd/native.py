@@ -303,6 +303,9 @@ _YARDSTICK_SIGNATURES = {
     "mf_probe_hbm": (i32, [i32, vp, vp, u64, vp]),
 }
 
+# the short calls of a decode step and of a page table, which go past ctypes where their arguments are plain (csrc/python/calls.cpp)
+_DIRECT = ("mf_moe_dispatch", "mf_moe_combine", "mf_xcopy_device_table")
+
 _lock = threading.Lock()
 _lib = None
 _plugin = None
@@ -325,13 +328,19 @@ def _bind(handle, table):
 def lib():
     """The data-plane library; raises OSError if it has not been built."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is None:
             if not os.path.exists(DATAPLANE_PATH):
                 raise OSError(
                     f"{DATAPLANE_PATH} is missing: build it with `make -C memfabric_hybrid_amd/csrc` "
                     "(or __graft_entry__.build()); there is no fallback path")
-            _lib = _bind(ctypes.CDLL(DATAPLANE_PATH, mode=ctypes.RTLD_GLOBAL), _SIGNATURES)
+            handle = _bind(ctypes.CDLL(DATAPLANE_PATH, mode=ctypes.RTLD_GLOBAL), _SIGNATURES)
+            if os.path.exists(CALLS_PATH):
+                for name in _DIRECT:
+                    setattr(handle, name, _load_calls().direct(name, getattr(handle, name)))
+            _lib = handle
         return _lib
 
 
@@ -357,21 +366,26 @@ def yardstick():
         return _yardstick
 
 
+def _load_calls():
+    global _calls
+    if _calls is None:
+        loader = importlib.machinery.ExtensionFileLoader("_calls", CALLS_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_calls", loader))
+        loader.exec_module(module)
+        _calls = module
+    return _calls
+
+
 def calls():
     """The extension module behind the Python face: sequences of integers into the C API without a loop of the
     interpreter's (csrc/python/calls.cpp).  Linked against the data-plane library, which is loaded first."""
-    global _calls
     if _calls is None:
         lib()
         with _lock:
-            if _calls is None:
-                if not os.path.exists(CALLS_PATH):
-                    raise OSError(f"{CALLS_PATH} is missing: build it for this interpreter with `make -C memfabric_hybrid_amd/csrc "
-                                  f"PYTHON={sys.executable}`")
-                loader = importlib.machinery.ExtensionFileLoader("_calls", CALLS_PATH)
-                module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_calls", loader))
-                loader.exec_module(module)
-                _calls = module
+            if not os.path.exists(CALLS_PATH):
+                raise OSError(f"{CALLS_PATH} is missing: build it for this interpreter with `make -C memfabric_hybrid_amd/csrc "
+                              f"PYTHON={sys.executable}`")
+            _load_calls()
     return _calls
 
 

@@ -199,3 +199,46 @@ def test_a_batch_call_inside_a_batch_call_copies_both(lib, outer, inner):
     finally:
         pool.destroy()
         bm.uninitialize()
+
+
+class _Int(int):
+    pass
+
+
+@pytest.mark.parametrize("args", [
+    (0x1000, 0x2000, 0x3000, 0, 64, 8, 0x4000, None), (None, None, None, 1, 64, 1, None, None),
+    (0x1000, 0x2000, 0x3000, 1, 12, 8, 0x4000, 0), (0x1008, 0x2000, 0x3000, 1 << 32, 64, 8, 0x4000, 0),       # numbers modulo 2^32: no tokens
+    (0x1000, 0x2000, 0x3000, 1, 64, (1 << 32) + 17, 0x4000, 0), (0x1000, 0x2000, 0x3000, -1, -1, -1, 0x4000, 0),
+    ((1 << 64) + 0x1001, 0x2000, 0x3000, 1, 64, 8, 0x4000, 0), (-15, 0x2000, 0x3000, 1, 64, 8, 0x4000, 0),    # addresses modulo 2^64
+    (ctypes.c_void_p(0), 0x2000, 0x3000, 1, 64, 8, 0x4000, None), (_Int(0x1001), True, 0x3000, 1, 64, 8, 0x4000, None),
+    (0x1001, 0x2000, 0x3000, ctypes.c_uint32(1), 64, 8, 0x4000, None), (0x1001, 0x2000, 0x3000, 1, 64, 8, 0x4000, None, 5),
+    (0x1001, 0x2000, 0x3000, 1, 64, 8, 0x4000), (), (1.0, 0, 0, 0, 0, 0, 0, 0), (0, 0, 0, None, 0, 0, 0, 0), (0, "x", 0, 0, 0, 0, 0, 0),
+    (np.int64(4096), 0, 0, 0, 0, 0, 0, 0), (0, 0, 0, np.uint32(1), 0, 0, 0, 0),
+], ids=str)
+def test_calls_past_ctypes_are_what_ctypes_makes_of_them(lib, args):
+    """None of them gets to the GPU: what the library refuses, and why, and what ctypes refuses."""
+    def outcome(function):
+        try:
+            return function(*args), native.last_error()
+        except Exception as e:
+            return type(e), str(e)
+    direct, plain = lib.mf_moe_combine, lib["mf_moe_combine"]
+    plain.restype, plain.argtypes = native._SIGNATURES["mf_moe_combine"]
+    assert type(direct) is not type(plain)
+    lib.mf_moe_combine_windows(1, 1)                    # another message in between
+    expect = outcome(plain)
+    assert expect[0] != 0
+    lib.mf_moe_combine_windows(1, 1)
+    assert outcome(direct) == expect
+
+
+def test_a_call_past_ctypes_has_its_attributes(lib):
+    direct = lib.mf_moe_dispatch
+    assert (direct.restype, direct.argtypes) == native._SIGNATURES["mf_moe_dispatch"] and direct.__name__ == "mf_moe_dispatch" and callable(direct)
+    assert ctypes.cast(direct, ctypes.c_void_p).value == ctypes.cast(lib["mf_moe_dispatch"], ctypes.c_void_p).value
+    with pytest.raises(AttributeError):
+        direct.nothing
+    other = native.calls().direct("mf_moe_combine", lib["mf_moe_combine"])
+    other.restype, other.argtypes = ctypes.c_bool, native._SIGNATURES["mf_moe_combine"][1]      # what is set holds
+    assert other(0, 0, 0, 0, 0, 0, 0, 0) is True
+    assert native.calls().direct("hybm_uninit", lib.hybm_uninit) is lib.hybm_uninit
