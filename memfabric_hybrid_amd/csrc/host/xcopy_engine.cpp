@@ -2105,7 +2105,9 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
     uint32_t units = 0;
     bool oversized = false;      // a run the 32-bit length of the inline table cannot hold is possible
     bool windowed = false;
+    bool lineWindowed = false;
     uint32_t windowRate = tuning_.windowMBps;
+    uint32_t linesRate = windowRate;
     uint64_t queuedBytes = 0;
     if (n <= 4 * kInlineSegs) {  // small enough that a failed attempt costs next to nothing
         uint64_t total = 0;
@@ -2120,19 +2122,19 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         oversized = total > 0xFFFFFFFFull;
         units = ChooseUnits(total, cu, route, tuning_);
         // Large HBM copies of one submitter: 16 KiB chunks for the kernel that alternates between read and write windows.
-        // Not where a source and its destination differ modulo 16: the loads that straddle units cost twice the issue slots,
-        // and the waves keep no schedule at any rate that pays (100 segments of 10 MB: 5.35 TB/s in windows cut for 6.8, 5.26
-        // for 7.4, 5.51 to 5.56 without windows).
+        // Where a source and its destination differ modulo 16, and below kWindowMinBytes from where held stores end, by the kernel that
+        // takes any chunk (XcopyLineWindowKernel has the figures).
         const bool aligned = (addressBits & (kWindowAlignBytes - 1)) == 0;
-        windowed = !unordered && (apartBits & (kUnitBytes - 1)) == 0 && WindowsApply(total, route, kWindowMinBytes);
+        const bool apart = (apartBits & (kUnitBytes - 1)) != 0;
+        windowed = !unordered && !apart && WindowsApply(total, route, kWindowMinBytes);
+        lineWindowed = !unordered && !windowed && WindowsApply(total, route, kDeepMaxBytes + 1) && !DeepHoldApplies(total, n, route, unordered);
         // Segments that all start on cache lines, in source and destination, hold a higher rate.  Back to back at 6.8 / 7.1 /
         // 7.4 TB/s, the same in four processes: 2 GiB in one segment 6.65 / 6.95 / 7.02 to 7.27, 32 x 16 MiB 6.65 / 6.95 / 7.05 to
         // 7.26, 128 x 9 MiB 6.65 / 6.95 / 6.76 to 7.32.  The reshard's launches of 128 segments of 0.4 to 17 MB from eight
         // places hold 7.1 in every process (6.87 to 7.00) and 7.4 only in some (7.0 to 7.2 in one, 5.8 to 6.1 in three others):
         // long segments take the highest rate, other aligned ones the one between.  Where segments start between cache lines
-        // every wave's kilobyte straddles a line it shares with its neighbour; such launches hold 6.8 (6.24 to 6.27 against 5.65
-        // to 5.80 TB/s without windows) and fall apart at 7.4 (5.36 to 5.48).
-        const bool longSegments = windowed && total / n >= kWindowLongSegmentBytes;
+        // their chunks are cut on the lines and hold 7.1 too; shifted ones hold 6.8.
+        const bool longSegments = (windowed || lineWindowed) && total / n >= kWindowLongSegmentBytes;
         if (longSegments && maySlice && total >= 2 * kWindowPieceBytes) {
             // A windowed launch that loses its schedule runs the rest of its bytes at the rate without windows, and the longer
             // it runs the likelier that is: launches of kWindowPieceBytes to twice that, each with a schedule of its own, hold
@@ -2141,16 +2143,19 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
             // segments (600 to 900 MB) were no faster than in launches of 128.
             return SubmitInPieces(src, dst, len, n, total, route, stream, mask, maskValue);
         }
+        linesRate = !apart && tuning_.windowAlignedMBps != 0 ? tuning_.windowAlignedMBps : tuning_.windowMBps;
         windowRate = tuning_.windowMBps;
         if (aligned && longSegments && tuning_.windowLongMBps != 0) {
             windowRate = tuning_.windowLongMBps;
         } else if (aligned && tuning_.windowAlignedMBps != 0) {
             windowRate = tuning_.windowAlignedMBps;
+        } else if (lineWindowed) {
+            windowRate = linesRate;
         }
-        if (windowed) {
+        if (windowed || lineWindowed) {
             units = mfk_xcopy_window_units();
         }
-        const bool deep = !windowed && DeepHoldApplies(total, n, route, unordered);
+        const bool deep = !windowed && !lineWindowed && DeepHoldApplies(total, n, route, unordered);
         if (deep && n != 1 && (apartBits & (kUnitBytes - 1)) != 0 && mfrt_stream_capturing(stream) == 0) {
             // as pieces: sixteen loads per lane of aligned units and what shifts them, with the table of the kernel arguments, take
             // more registers than sixteen waves per CU have (42 MB 17.5 us with straddling loads); one segment has no table
@@ -2167,11 +2172,12 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
     if (!inlined && oversized) {
         // a run of 4 GiB and more may have made the one-pass attempt give up: the general inline path cuts it into pieces
         NormalizeSegments(src, dst, len, n, kInlinePiece, ctx.segs);
-        units = windowed ? mfk_xcopy_window_units() : ChooseUnits(ctx.segs.totalBytes, cu, route, tuning_);
+        units = windowed || lineWindowed ? mfk_xcopy_window_units() : ChooseUnits(ctx.segs.totalBytes, cu, route, tuning_);
         inlined = BuildInlinePlan(ctx.segs, units, plan);
     }
-    if (inlined && windowed) {
-        int err = mfk_xcopy_windowed(&plan, windowRate, mask, maskValue, stream);
+    if (inlined && (windowed || lineWindowed)) {
+        const int err = windowed ? mfk_xcopy_windowed(&plan, windowRate, linesRate, mask, maskValue, stream)
+                                 : mfk_xcopy_line_windowed(&plan, windowRate, mask, maskValue, stream);
         if (err != 0) {
             MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(err));
         }

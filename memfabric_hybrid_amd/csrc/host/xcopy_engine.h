@@ -88,13 +88,12 @@ struct XcopyTuning {
     uint32_t windowLongMBps = 7400000;      // and for those of them whose segments are kWindowLongSegmentBytes and longer on average, which hold more still; 0 = the rate above
 };
 
-// From this total on a batch of up to 128 segments between HBM addresses is copied in read and write windows.
-// Segments on cache lines, paced for windowAlignedMBps, gain from where the held stores of 16 KiB per wave end:
-// back to back, 32 segments, windows against none: 66 MiB 6.37 against 5.71 TB/s, 80 MiB 6.57 against 5.76, 130 MiB
-// 6.94 against 6.14, 256 MiB 7.14 against 6.37, 600 MiB 7.20 against 6.31 (at 64 MiB and below the held stores are
-// as fast).  A launch on its own gains less and less steadily below 128 MiB (80 MiB: 32.4 against 31.9 us), hence
-// the limit.  Segments between cache lines, paced for windowMBps, gain 5 to 7 % from there on (136 MB 43.7 against
-// 46.8 us, 272 MB 85 against 91.5, 407 MB 129.5 against 137).
+// From this total on a batch of up to 128 segments between HBM addresses that agree modulo 16 is copied by XcopyWindowKernel, or by
+// XcopyLineWindowKernel where a destination is off a cache line; below, and where source and destination differ modulo 16, by the latter from
+// where held stores end (64 MiB, 112 for one segment).  Back to back, 32 segments on lines, windows against none: 66 MiB 6.37
+// against 5.71 TB/s, 80 MiB 6.57 against 5.76, 130 MiB 6.94 against 6.14, 256 MiB 7.14 against 6.37, 600 MiB 7.20 against 6.31.  The limit
+// is where chunks that are not whole, which XcopyWindowKernel copies in its write half, stop to matter (100 segments of together 70 / 126 / 150 MiB
+// 29.0 / 43.4 / 47.6 us in that one, 24.6 / 43.4 / 48.5 in the other).
 constexpr uint64_t kWindowMinBytes = 128ull << 20;
 // Rectangles in chunks of their payload: in windows, and without (several threads, rows between cache lines), where whole rows are as
 // fast up to 40 MB (Copy2dChunkKernel has the figures).

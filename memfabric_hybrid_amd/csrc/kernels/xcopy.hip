@@ -442,9 +442,9 @@ __device__ __forceinline__ void CopyChunkHeld(uint64_t src, uint64_t dst, uint64
     }
 }
 
-// The inline plan (chunks of kWindowUnits units) copied by gridDim.x single-wave workgroups that walk
+// The inline plan (chunks of kWindowUnits units, destinations on lines) copied by gridDim.x single-wave workgroups that walk
 // the chunks with stride gridDim.x, one chunk per period each.
-template <bool kNtLoad, int kStore, bool kOnLines>
+template <bool kNtLoad, int kStore>
 __global__ __launch_bounds__(64) void XcopyWindowKernel(const InlinePlan p, uint32_t period, uint32_t seq)
 {
     const InlineRows rows(p);
@@ -453,8 +453,7 @@ __global__ __launch_bounds__(64) void XcopyWindowKernel(const InlinePlan p, uint
     uint64_t slot = AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * half / gridDim.x;
     for (uint32_t c = blockIdx.x; c < nchunk; c += gridDim.x) {
         const InlineChunk r = rows.Owner(c);
-        const SegChunk m = ChunkOn(kOnLines, r.src, r.dst, r.len, r.k, kWindowUnits);
-        CopyChunkWindowed<kNtLoad, kStore>(m.src, m.dst, m.len, m.k, slot, half);
+        CopyChunkWindowed<kNtLoad, kStore>(r.src, r.dst, r.len, r.k, slot, half);
         slot += period;
     }
 }
@@ -975,6 +974,30 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kHeldWavesPe
     const LineSpan span = LineChunk(dst, len, blockIdx.x, kDeepUnits);
     if (span.begin < len) {
         CopyPieceHeld<kDeepUnits / 64>(src + span.begin, dst + span.begin, static_cast<uint32_t>(span.end - span.begin), t0, holdTicks, [] {});
+    }
+}
+
+// XcopyWindowKernel in chunks of LineChunks(), whatever source and destination are modulo 16, a chunk as XcopyPieceHeldKernel's: one that is not
+// whole, or whose bytes are shifted, keeps to the windows too, where XcopyWindowKernel copies it in the write half and one kernel of straddling loads falls behind.
+// HBM is the bound.  us back to back, without windows or in those of XcopyWindowKernel / so.  Source and destination different modulo 16: one segment of 120 / 200 /
+// 500 / 1024 MB 40.4 / 38.9, 65.9 / 63.1, 160 / 154, 335 / 323, 16 of together 74 / 157 / 315 MB 28.1 / 25.8, 56.4 / 50.8, 108 / 98.5, 128 of them 29.8 / 26.6, 60.3 / 52.7,
+// 115 / 99.8.  Alike modulo 16, destinations between lines: one of 134 / 300 / 700 MB 42.7 / 41.2, 93.6 / 90.6, 217 / 210, 16 of 74 / 157 / 315 MB 27.3 / 24.0, 52.2 / 48.3,
+// 98.5 / 94.4, 128 of them 28.8 / 25.0, 54.7 / 48.9, 101.6 / 95.1.  On lines below kWindowMinBytes: one of 118 / 126 MB 38.8 / 35.3, 41.1 / 38.2, two of together 74 / 132 MB
+// 25.3 / 23.5, 43.1 / 40.2, 100 of them 27.1 / 24.6, 45.8 / 43.4; above, the kernel with less to compute is as fast or 1 % faster.
+// Rates, 6.5 / 6.8 / 6.95 / 7.1 TB/s where bytes are shifted: 200 MB 65.5 / 63.1 / 62.2 / 61.6, 1024 MB 333 / 325 / 332 / 352, 100 x 10 MB 323 / 317 / 318 / 343; and
+// 6.8 / 7.1 / 7.3 where they are not: 300 MB 93.6 / 90.6 / 88.6, 1024 MB 319 / 312 / 323, 100 x 10 MB 314 / 310 / 350.
+__global__ __launch_bounds__(64) void XcopyLineWindowKernel(const InlinePlan p, uint32_t period, uint32_t seq)
+{
+    const InlineRows rows(p);
+    const uint32_t nchunk = p.nchunk;
+    const uint32_t groups = gridDim.x;
+    const uint32_t half = period / 2;
+    uint64_t slot = AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * half / groups;
+    for (uint32_t c = blockIdx.x; c < nchunk; c += groups, slot += period) {
+        const InlineChunk r = rows.Owner(c);
+        const LineSpan span = LineChunk(r.dst, r.len, r.k, kDeepUnits);
+        WaitForClock(slot);
+        CopyPieceHeld<kDeepUnits / 64>(r.src + span.begin, r.dst + span.begin, static_cast<uint32_t>(span.end - span.begin), slot, half, [] {});
     }
 }
 
@@ -1980,35 +2003,37 @@ int LaunchInline(const InlinePlan &plan, uint32_t grid, uint32_t lanes, hipStrea
     return static_cast<int>(hipLaunchKernel(kernel, dim3(grid), dim3(lanes), args, 0, stream));
 }
 
-// The plan with the chunks of LineChunks(); false where all destinations begin on a line, whose chunks are whole lines as they are.
-bool CutOnLines(const InlinePlan &plan, InlinePlan &lines)
+// Whether all destinations begin on a line.
+bool OnLines(const InlinePlan &plan)
 {
     uint64_t bits = 0;
     for (uint32_t i = 0; i < kInlineSegs && plan.first[i] != kNoChunk; ++i) {
         bits |= plan.dst[i];
     }
-    if ((bits & (kLineBytes - 1)) == 0) {
-        return false;
-    }
-    lines = plan;
+    return (bits & (kLineBytes - 1)) == 0;
+}
+
+// The plan with the chunks of LineChunks(), which are others also where a segment on a line ends with a few bytes behind its last whole chunk.
+InlinePlan CutOnLines(const InlinePlan &plan)
+{
+    InlinePlan lines = plan;
     uint64_t chunks = 0;
     for (uint32_t i = 0; i < kInlineSegs && plan.first[i] != kNoChunk; ++i) {
         lines.first[i] = static_cast<uint32_t>(chunks);
         chunks += LineChunks(plan.dst[i], plan.len[i], plan.units);
     }
     lines.nchunk = static_cast<uint32_t>(chunks);
-    return true;
+    return lines;
 }
 
 // windowMBps: the rate (MB/s of HBM traffic, read + written) the period of a windowed launch is cut for.
-template <bool kNtLoad, int kStore>
-int LaunchWindowed(const InlinePlan &plan, uint32_t grid, bool onLines, uint32_t windowMBps, hipStream_t stream)
+int LaunchWindowed(void (*kernel)(const InlinePlan, uint32_t, uint32_t), const InlinePlan &plan, uint32_t windowMBps, hipStream_t stream)
 {
+    const uint32_t grid = WindowGrid(plan.nchunk, kWindowWaves);
     const uint32_t ticks = WindowPeriodTicks(2ull * grid * kWindowUnits * kUnitBytes, windowMBps);
     if (ticks == 0) {
         return static_cast<int>(hipErrorInvalidValue);
     }
-    const auto kernel = onLines ? XcopyWindowKernel<kNtLoad, kStore, true> : XcopyWindowKernel<kNtLoad, kStore, false>;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, stream, plan, ticks, NextWindowSeq());
     return static_cast<int>(hipGetLastError());
 }
@@ -2149,21 +2174,33 @@ extern "C" uint32_t mfk_xcopy_window_waves(void)
     return mf::kWindowWaves;
 }
 
-extern "C" int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream)
+extern "C" int mfk_xcopy_line_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream)
 {
-    const mf::InlinePlan &given = *static_cast<const mf::InlinePlan *>(inlinePlan);
+    using namespace mf;
+    const InlinePlan &plan = *static_cast<const InlinePlan *>(inlinePlan);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (given.units != mf::kWindowUnits || given.nchunk == 0 || windowMBps == 0) {
+    if (plan.units != kWindowUnits || plan.nchunk == 0 || windowMBps == 0) {
         return -1;
     }
-    mf::InlinePlan lines;
-    const bool onLines = mf::CutOnLines(given, lines);
-    const mf::InlinePlan &plan = onLines ? lines : given;
-    const uint32_t grid = mf::WindowGrid(plan.nchunk, mf::kWindowWaves);
-    const int err = mf::WithPolicy(mf::PolicyOf(MFRT_ROUTE_HBM), [&](auto ntLoad, auto store) {
-        return mf::LaunchWindowed<decltype(ntLoad)::value, decltype(store)::value>(plan, grid, onLines, windowMBps, s);
+    const int err = LaunchWindowed(XcopyLineWindowKernel, CutOnLines(plan), windowMBps, s);
+    return err != 0 ? err : Signal(mask, maskValue, s);
+}
+
+extern "C" int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, uint32_t linesMBps, void *mask, uint32_t maskValue, void *stream)
+{
+    using namespace mf;
+    const InlinePlan &plan = *static_cast<const InlinePlan *>(inlinePlan);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (plan.units != kWindowUnits || plan.nchunk == 0 || windowMBps == 0) {
+        return -1;
+    }
+    if (!OnLines(plan)) {
+        return mfk_xcopy_line_windowed(inlinePlan, linesMBps, mask, maskValue, stream);
+    }
+    const int err = WithPolicy(PolicyOf(MFRT_ROUTE_HBM), [&](auto ntLoad, auto store) {
+        return LaunchWindowed(XcopyWindowKernel<decltype(ntLoad)::value, decltype(store)::value>, plan, windowMBps, s);
     });
-    return err != 0 ? err : mf::Signal(mask, maskValue, s);
+    return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
 extern "C" int mfk_xcopy_signal(void *word, uint32_t value, void *stream)
@@ -2361,8 +2398,8 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
                 (void)Launch(XcopyPlannedKernel<1, kPlannedShortRun>, 1, 64, 64, s, 0, 0u, TablePace{});
                 (void)Launch(XcopyPlannedKernel<kPlannedWaves, kPlannedRun>, 1, 64 * kPlannedWaves, 64, s, 0, 0u, TablePace{});
                 (void)Launch(XcopySampledKernel, 1, 64, 0, s, 0, 0u, 0, 0u, TablePace{});
-                hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt, false>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
-                hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt, true>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
+                hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
+                hipLaunchKernelGGL(XcopyLineWindowKernel, dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
             }
             return 0;
         });
@@ -2488,7 +2525,7 @@ extern "C" int mfk_xcopy_calibrate(void *stream, const uint32_t *holdNanos, cons
                 big.units = kWindowUnits;
                 big.nchunk = static_cast<uint32_t>(half / (kWindowUnits * kUnitBytes));
                 const uint32_t rate = windowMBps[v - 1];
-                err = timed([&](int) { (void)LaunchWindowed<true, kStoreStream>(big, kWindowWaves, false, rate, s); }, round == 0 ? 1 : 0, 1,
+                err = timed([&](int) { (void)LaunchWindowed(XcopyWindowKernel<true, kStoreStream>, big, rate, s); }, round == 0 ? 1 : 0, 1,
                             out[4 + v]);
             }
             if (err != hipSuccess) {

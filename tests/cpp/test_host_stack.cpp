@@ -33,6 +33,7 @@ extern "C" int fake_rt_last_combine_paced(void);
 extern "C" uint64_t fake_rt_signals(void);
 extern "C" uint64_t fake_rt_stream_syncs(void);
 extern "C" uint32_t fake_rt_last_window(void);
+extern "C" uint32_t fake_rt_last_line_window(void);
 extern "C" void fake_rt_seal(void);
 extern "C" void fake_rt_fail_launches(int n);
 #include "../../include/mf_hip_copy_extend.h"
@@ -2007,7 +2008,7 @@ static void TestWindows()
     CHECK(ok && from[gib + 256 + gib - 1] == from[gib - 1]);
     {
         // odd addresses that agree modulo 16 (head and tail bytes): windows at the general rate;
-        // addresses that differ modulo 16: no windows, one launch
+        // addresses that differ modulo 16: those of TestLineWindows, one launch
         uint64_t so = s1 + 3;
         uint64_t dO = s1 + gib + 256 + 19;
         uint64_t lo = gib - 64;
@@ -2068,7 +2069,7 @@ static void TestWindows()
         CHECK(fake_rt_last_window() == 7100000);       // on cache lines, 16 MiB each: the rate between
         CHECK(engine.DrainThread() == BM_OK);
     }
-    l1 = (gib >> 3) - 1;                           // one byte below the limit of segments on cache lines: the ordinary form
+    l1 = (gib >> 3) - 1;                           // one byte below the limit: those of TestLineWindows
     CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
     CHECK(fake_rt_last_window() == 0);
     l1 = gib >> 3;
@@ -2181,6 +2182,58 @@ static int SubmitList(uint32_t n, uint64_t bytes, From from, To to)
     void *stream = mf_xcopy_thread_stream();
     const int ret = engine.Submit(s.data(), d.data(), l.data(), n, MF_ROUTE_HBM, stream, nullptr, 0);
     return ret != BM_OK ? ret : engine.DrainThread();
+}
+
+// Which batches take the windows whose chunks are cut on lines, and their rates: addresses that differ modulo 16, and all from where held
+// stores end up to the other windows.
+static void TestLineWindows()
+{
+    CHECK(hybm_init(0, 0) == BM_OK);
+    fake_rt_skip_copies(1);
+    XcopyEngine &engine = XcopyEngine::Instance();
+    void *stream = mf_xcopy_thread_stream();
+    const uint64_t mib = 1ull << 20;
+    const uint32_t general = XcopyTuning{}.windowMBps;
+    const uint32_t between = XcopyTuning{}.windowAlignedMBps;
+    const uint32_t most = XcopyTuning{}.windowLongMBps;
+    struct Form { uint32_t n; uint64_t bytes, from, to; uint32_t rate; bool other; };
+    const Form forms[] = {
+        {1, kHeldSingleBytes, 0, 0, 0, false},          {1, kHeldSingleBytes, 3, 16, 0, false},         // held
+        {1, kHeldSingleBytes + 1, 0, 0, most, false},   {1, kHeldSingleBytes + 1, 16, 48, between, false}, {1, kHeldSingleBytes + 1, 3, 16, general, false},
+        {1, 128 * mib - 1, 0, 0, most, false},          {1, 128 * mib, 0, 0, 0, true},                  {1, 128 * mib, 16, 48, 0, true},
+        {1, 128 * mib, 3, 16, general, false},          {1, 900 * mib + 5, 18, 7, general, false},      {1, 1024 * mib, 18, 7, general, false},
+        {2, 32 * mib, 0, 0, 0, false},                  {2, 32 * mib + 256, 0, 0, between, false},      {2, 32 * mib + 1, 16, 48, between, false},
+        {2, 64 * mib, 16, 48, 0, true},                 {2, 64 * mib - 1, 3, 16, general, false},       {128, mib + 77, 3, 16, general, false},
+        {128, 512 * 1024, 0, 0, 0, false},              {128, 512 * 1024 + 128, 0, 0, between, false},  {129, mib, 3, 16, 0, false},
+    };
+    for (const Form &f : forms) {
+        std::vector<uint64_t> s(f.n), d(f.n), l(f.n, f.bytes);
+        for (uint32_t i = 0; i < f.n; ++i) {
+            s[i] = (1ull << 40) + i * 8192 * mib + f.from;
+            d[i] = (1ull << 42) + i * 4096 * mib + f.to;
+        }
+        for (int mode = 0; mode < 2; ++mode) {      // declared independent of what is in flight: none
+            (void)fake_rt_last_window();
+            (void)fake_rt_last_line_window();
+            CHECK(engine.Submit(s.data(), d.data(), l.data(), f.n, MF_ROUTE_HBM, stream, nullptr, 0, mode == 1) == BM_OK);
+            CHECK(fake_rt_last_line_window() == (mode == 1 ? 0 : f.rate));
+            CHECK((fake_rt_last_window() != 0) == (mode == 0 && f.other));
+        }
+        CHECK(engine.DrainThread() == BM_OK);
+    }
+    CHECK(mf_xcopy_windows(0) == BM_OK);
+    uint64_t s1 = 1ull << 40;
+    uint64_t d1 = (1ull << 42) + 3;
+    uint64_t l1 = 300 * mib;
+    CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
+    CHECK(fake_rt_last_line_window() == 0);
+    CHECK(mf_xcopy_windows(6400000) == BM_OK);
+    CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
+    CHECK(fake_rt_last_line_window() == 6400000);
+    CHECK(mf_xcopy_windows(MF_XCOPY_WINDOWS_OWN_CHOICE) == BM_OK);
+    CHECK(engine.DrainThread() == BM_OK);
+    fake_rt_skip_copies(0);
+    hybm_uninit();
 }
 
 // The rates of lists in windows: those that only blocks at multiples of 64 KiB hold, and where they do not apply.
@@ -2402,6 +2455,7 @@ int main()
     TestPlugin();
     TestHeldStores();
     TestWindows();
+    TestLineWindows();
     TestWindowRatesOfLists();
     TestPiecesOfLists();
     TestHeldLaunches();

@@ -92,8 +92,8 @@ def test_ragged_batch_above_one_gib_in_read_and_write_windows(pool, lib, oracle,
     last chunks, head and tail bytes), with the default period, with a period too short for the waves to
     keep up (they then proceed late; the result must not depend on timing) and with the form switched off:
     what comes back equals the same slices cut on the CPU, and the bytes between and round the destinations
-    are untouched.  Sources and destinations either agree modulo 16 (the batch then takes the windows) or do not
-    (the engine then leaves the windows out, whatever the rate)."""
+    are untouched.  Sources and destinations either agree modulo 16 or do not (the batch then takes the windows
+    whose chunks are cut on lines)."""
     dev = pool.peer_rank_ptr(0, bm.BmMemType.DEVICE)
     host = pool.peer_rank_ptr(0, bm.BmMemType.HOST)
     span = 2 * GIB + GUARD
@@ -144,7 +144,7 @@ def test_batches_of_some_hundred_mib_in_windows_whose_last_period_is_full(pool, 
     """Device-to-device batches of 130 to 300 MiB in 37 ragged segments: sizes whose chunks do not fill a whole number
     of periods on 4096 waves, so the launch runs on fewer waves with every period full.  Segments on cache lines
     (the higher window rate), between cache lines (the general rate) and with sources apart from their destinations
-    modulo 16 (no windows): what arrives equals the same slices cut on the CPU, the gaps between destinations stay."""
+    modulo 16 (the general rate, chunks cut on lines): what arrives equals the same slices cut on the CPU, the gaps between destinations stay."""
     dev = pool.peer_rank_ptr(0, bm.BmMemType.DEVICE)
     host = pool.peer_rank_ptr(0, bm.BmMemType.HOST)
     span = 2 * GIB + GUARD

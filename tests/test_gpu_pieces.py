@@ -106,6 +106,37 @@ def test_lists_of_blocks_in_windows(gpu, count, size, where):
     assert torch.equal(target.view(count, size)[torch.from_numpy(place).cuda()], source.view(2 * count, size)[torch.from_numpy(at).cuda()])
 
 
+# Batches whose chunks are cut on the destinations' lines and go in windows: one segment just above what is held, at and beyond 128 MiB; chunks that
+# are not whole, segments shorter than one, than a unit, than a line.
+@pytest.mark.parametrize("lens", [[(112 << 20) + 1], [(112 << 20) - 127], [(128 << 20) + 77], [300000001], [(64 << 20) + 1 - 16500, 16500],
+                                  [700001] * 127 + [5], [1 << 20] * 66 + [16384, 16383, 16385, 1, 15, 16, 17, 127, 128, 129, 0, 0, 33000] * 4], ids=str)
+@pytest.mark.parametrize("shift", [(0, 0), (0, 16), (64, 48), (3, 19), (0, 1), (1, 0), (4, 0), (127, 120), (5, 11), "each another"], ids=str)
+def test_batches_cut_on_lines_in_windows(gpu, lens, shift):
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(len(lens))
+    lens = np.array(lens, dtype=np.int64)
+    steps = (lens + 511) // 256 * 256
+    order = rng.permutation(len(lens))
+    at = np.cumsum(steps) - steps
+    place = np.empty_like(at)
+    place[order] = np.cumsum(steps[order]) - steps[order]
+    if shift == "each another":
+        at, place = at + rng.integers(0, 128, len(lens)), place + rng.integers(0, 128, len(lens))
+    else:
+        at, place = at + shift[0], place + shift[1]
+    room = int(steps.sum()) + 256
+    source = torch.randint(-2**63, 2**63 - 1, (room // 8,), dtype=torch.int64, device="cuda").view(torch.uint8)
+    before = torch.randint(-2**63, 2**63 - 1, (room // 8,), dtype=torch.int64, device="cuda").view(torch.uint8)
+    target, expect = before.clone(), before.clone()
+    for s, d, l in zip(at.tolist(), place.tolist(), lens.tolist()):
+        expect[d:d + l] = source[s:s + l]
+    torch.cuda.synchronize()
+    launches = gpu.mf_xcopy_launch_count()
+    gpu_util.xcopy(gpu, (source.data_ptr() + at).astype(np.uint64), (target.data_ptr() + place).astype(np.uint64), lens.astype(np.uint64), native.ROUTE_HBM)
+    assert gpu.mf_xcopy_launch_count() - launches == 1
+    assert torch.equal(target, expect)
+
+
 @pytest.mark.parametrize("each", [512, 40000])
 @pytest.mark.parametrize("order", ["own", "a caller's", "own and a caller's", "own, blocking between", "own, a long copy in front",
                                    "a caller's, a long copy in front"])
