@@ -189,7 +189,8 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
                                                               int32_t *__restrict__ rowOf, int32_t *__restrict__ srcOf,
                                                               const uint32_t *__restrict__ blockBad,
                                                               uint32_t *__restrict__ status, uint32_t topK,
-                                                              int2 *__restrict__ runOrder, uint32_t stepSlices,
+                                                              int2 *__restrict__ runOrder, uint32_t restSlices,
+                                                              uint32_t together, uint32_t blocksTogether, uint32_t blocksWhole,
                                                               uint32_t blocks, const u32x4 *__restrict__ warm, uint64_t warmUnits)
 {
     if (blockIdx.x >= blocks) {
@@ -210,8 +211,12 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
     // (plain counts, so LDS atomics give the same result every time).
     const bool tabled = blockHist != nullptr;
     const bool counting = !tabled;
+    const uint32_t stepSlices = blockIdx.x < blocksWhole ? kRankSlices : restSlices;
     const uint32_t steps = runOrder != nullptr ? kRankSlices / stepSlices : 0;
     uint32_t *others = cum + steps * experts;             // [experts], counting only
+    const bool grouped = blockIdx.x < blocksTogether;     // a step is `together` blocks, from groupFirst on
+    const uint32_t groupFirst = grouped ? blockIdx.x / together * together : blockIdx.x;
+    uint32_t *groupBefore = cum + steps * experts;        // [experts] entries of the step's blocks before this one, grouped only
     for (uint32_t i = threadIdx.x; counting && i < experts; i += kRankThreads) {
         others[i] = 0;
     }
@@ -268,6 +273,8 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
             const uint32_t *rowHist = blockHist + static_cast<uint64_t>(x) * histStride;
             uint32_t t = 0;
             uint32_t b = 0;
+            uint32_t g = 0;
+            uint32_t gb = 0;
             if (counting) {
 #pragma unroll
                 for (uint32_t sl = 0; sl < kRankSlices; ++sl) {
@@ -292,10 +299,25 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
                         b += blk + 4 * q + i < blockIdx.x ? v[q][i] : 0u;
                     }
                 }
+                if (grouped && blk == groupFirst / kHistPad * kHistPad) {       // a step's blocks lie in one
+#pragma unroll
+                    for (uint32_t q = 0; q < kHistPad / 4; ++q) {
+#pragma unroll
+                        for (uint32_t i = 0; i < 4; ++i) {
+                            const uint32_t after = blk + 4 * q + i - groupFirst;    // wraps in front of it
+                            g += after < together ? v[q][i] : 0u;
+                            gb += after < blockIdx.x - groupFirst ? v[q][i] : 0u;
+                        }
+                    }
+                }
             }
             tot[j] = t;
             before[j] = b;
             mine += t;
+            if (grouped) {
+                cum[x] = g;
+                groupBefore[x] = gb;
+            }
         }
     }
     // exclusive scan of `mine` over the threads: shuffles inside each wave, LDS across the waves
@@ -329,7 +351,7 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
     __syncthreads();
     // Turn slice histograms into exclusive prefixes over the slices of this block.  For the run-ordered list the
     // block is cut into steps of stepSlices slices (the tile permute works through one step at a time); the
-    // entries per (step, expert) are what the prefix gains over a step.
+    // entries per (step, expert) are what the prefix gains over a step.  (Those of a step of several blocks are in cum already.)
     for (uint32_t x = threadIdx.x; x < experts; x += kRankThreads) {
         uint32_t acc = base[x];
         uint32_t stepStart = acc;
@@ -342,7 +364,7 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
         for (uint32_t s = 0; s < kRankSlices; ++s) {
             hist[s * experts + x] = acc;
             acc += v[s];
-            if (steps != 0 && (s + 1) % stepSlices == 0) {
+            if (steps != 0 && !grouped && (s + 1) % stepSlices == 0) {
                 cum[(s / stepSlices) * experts + x] = acc - stepStart;
                 stepStart = acc;
             }
@@ -353,7 +375,7 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
     const uint32_t wave = threadIdx.x >> 6;
     if (steps != 0) {
         // cum[j][x]: entries of step j routed to an expert below x, i.e. where the rows of expert x start in the list
-        // of the step's rows in ascending order.  One wave per step; a lane scans experts/64 neighbours itself.
+        // of the step's rows in ascending order; behind them those of the step's blocks before this one.  One wave per step; a lane scans experts/64 neighbours itself.
         const uint32_t perLane = (experts + 63) / 64;     // at most kMaxExperts / 64
         for (uint32_t j = wave; j < steps; j += kRankThreads / 64) {
             uint32_t mineOf[kMaxExperts / 64];
@@ -375,7 +397,7 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
             for (uint32_t i = 0; i < kMaxExperts / 64; ++i) {
                 const uint32_t x = lane * perLane + i;
                 if (i < perLane && x < experts) {
-                    cum[j * experts + x] = at;
+                    cum[j * experts + x] = at + (grouped ? groupBefore[x] : 0u);
                     at += mineOf[i];
                 }
             }
@@ -400,7 +422,7 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
                     const uint32_t j = slice / stepSlices;
                     const uint32_t firstOfStep = hist[j * stepSlices * experts + myExpert[r]];
                     const uint32_t at = cum[j * experts + myExpert[r]] + (static_cast<uint32_t>(row) - firstOfStep);
-                    runOrder[static_cast<uint64_t>(blockIdx.x) * kRankBlock + j * stepSlices * 64 + at] =
+                    runOrder[static_cast<uint64_t>(groupFirst) * kRankBlock + j * stepSlices * 64 + at] =
                         make_int2(row, static_cast<int32_t>(idx / topK));
                 }
             }
@@ -412,7 +434,7 @@ __global__ __launch_bounds__(kRankThreads) void MoeRankKernel(const int32_t *__r
         const uint32_t stepEntries = stepSlices * 64;
         for (uint32_t slot = threadIdx.x; slot < kRankBlock; slot += kRankThreads) {
             const uint32_t j = slot / stepEntries;
-            if (slot - j * stepEntries >= stepValid[j]) {
+            if (slot - j * stepEntries + (blockIdx.x - groupFirst) * kRankBlock >= stepValid[j]) {
                 runOrder[static_cast<uint64_t>(blockIdx.x) * kRankBlock + slot] = make_int2(-1, 0);
             }
         }
@@ -554,7 +576,7 @@ __global__ __launch_bounds__(64) void MoePermuteLoopKernel(const u32x4 *__restri
 }
 
 // The permute of wide rows when a block of kRankBlock entries holds no more of x than an XCD's L2 keeps:
-// output-ordered, in tiles.  runOrder lists, step by step (a step is a block of kRankBlock entries or a power-of-two
+// output-ordered, in tiles.  runOrder lists, step by step (a step is a block of kRankBlock entries, several or a power-of-two
 // part of one, chosen so that the token rows of a step fit), the step's output rows in ascending
 // order (runs of consecutive rows per expert) with the token each row is a copy of.  Workgroup i, a single
 // wave, belongs to stream i % 8 (the dispatcher deals consecutive workgroups to the eight XCDs in turn);
@@ -562,28 +584,70 @@ __global__ __launch_bounds__(64) void MoePermuteLoopKernel(const u32x4 *__restri
 // tiles of 128 units (2 KiB).  So an XCD writes runs of consecutive rows front to back, two stores per wave,
 // the store pattern this part takes fastest, and the K reads of a token row all come from the same XCD within
 // the time it spends on the block: the first from HBM, the others from its L2 (plain loads), which stores that
-// are written through pass without evicting x.  8192 x 7168, top-8, 256 experts: 163-166 us against 192 us for
+// are written through pass without evicting x.  8192 x 7168, top-8, 256 experts, one block a step: 163-166 us against 192 us for
 // the token-ordered loop kernel; streams that do not follow the XCDs 283 us.
 constexpr uint32_t kTileUnits = 128;
 constexpr uint32_t kTileStreams = 8;
+// The longer a step's runs the better HBM takes them, as long as its token rows stay in the L2: kTileStepBytes of them, all of it (8192 x 7168 in steps of
+// four blocks, 7.3 MB, 227 us and not 193).  So a step has several blocks, as many as make runs of kTileRunBytes, and blocks that their rows cut in two are
+// whole again from four slots on.  Dispatch, us, one block a step / so, top-8, 256 experts: 8192 x 7168 193 / 185, 16 384 382 / 368, 4100 110 / 96, 7300 x 5120 134 / 119,
+// 6200 x 4096 96.5 / 83.5, 16 384 232 / 213, 30 000 x 2048 233 / 214, 6200 56.0 / 51.1; 512 experts 8192 x 7168 204 / 194, x 2048 70.4 / 62.7.  128 experts have runs twice
+// as long as they are: 8192 x 7168 183 / 179, 6400 148 / 138, but x 2048 58.0 / 58.8, x 4096 99.9 / 100.0, hence kTileLongRowBytes; 64 lose (x 7168 174.0 / 174.7, x 5120
+// 120.9 / 123.2).  Rows of one tile lose with two and four blocks (7300 x 1024 38.4 / 39.4), and so do four slots, whose rows are read less often from the
+// L2 (9999 x 4096 77.2 / 78.5).
+// Steps that the streams do not divide leave XCDs idle at the end, 4 of 56 the half of them for a seventh of the time: what is left of the last round
+// is cut until they do (6900 x 7168 over 8 experts 148 / 144, 6500 at top-4 88.1 / 84.8, 7000 over 64 at top-6 127 / 122.5, 6300 x 1024 33.0 / 31.6; it is
+// most of what 4100, 6200 and 6400 tokens above gain).
+constexpr uint64_t kTileStepBytes = 4ull << 20;
+constexpr uint64_t kTileRunBytes = 128ull << 10;
+constexpr uint32_t kTileMostTogether = 8;
+constexpr uint32_t kTileFewExperts = 128;
+constexpr uint32_t kTileLongRowBytes = 12288;
+constexpr uint32_t kTileTogetherRowBytes = 4096;
+constexpr uint32_t kTileWholeSlots = 4;                 // the fewest for whole blocks of more than half of kTileStepBytes, and too few for several
+static_assert(kHistPad % kTileMostTogether == 0, "the counts of a step's blocks are fetched together");
+
+// Steps of longEntries entries first, then of kRankBlock, then of restEntries: rounds of a step for every stream, the last one what is left.
+struct TilePlan {
+    uint32_t entries;           // of the list, whole blocks
+    uint32_t longEntries;
+    uint32_t longRounds;
+    uint32_t wholeRounds;
+    uint32_t restEntries;
+};
 
 __global__ __launch_bounds__(64) void MoePermuteTileKernel(const u32x4 *__restrict__ x, const int2 *__restrict__ runOrder,
-                                                           uint32_t unitsPerRow, uint32_t tilesPerRow, uint32_t steps,
-                                                           uint32_t stepEntries, u32x4 *__restrict__ out)
+                                                           uint32_t unitsPerRow, uint32_t tilesPerRow, TilePlan plan, u32x4 *__restrict__ out)
 {
     const uint32_t stream = blockIdx.x % kTileStreams;
-    const uint32_t q = blockIdx.x / kTileStreams;
-    const uint32_t tilesPerStep = stepEntries * tilesPerRow;
-    const uint32_t step = (q / tilesPerStep) * kTileStreams + stream;
-    const uint32_t within = q % tilesPerStep;
-    if (step >= steps) {
+    uint32_t q = blockIdx.x / kTileStreams;
+    const uint32_t tilesLong = plan.longRounds * plan.longEntries * tilesPerRow;
+    const uint32_t tilesWhole = plan.wholeRounds * kRankBlock * tilesPerRow;
+    uint32_t each = plan.longEntries;
+    uint32_t from = 0;
+    if (q >= tilesLong) {
+        q -= tilesLong;
+        from = plan.longRounds * kTileStreams * plan.longEntries;
+        each = kRankBlock;
+        if (q >= tilesWhole) {
+            q -= tilesWhole;
+            from += plan.wholeRounds * kTileStreams * kRankBlock;
+            each = plan.restEntries;
+        }
+    }
+    const uint32_t tilesPerStep = each * tilesPerRow;
+    const uint32_t round = q / tilesPerStep;
+    const uint32_t within = q - round * tilesPerStep;
+    const uint32_t entry = within / tilesPerRow;
+    const uint32_t first = from + (round * kTileStreams + stream) * each;
+    if (first >= plan.entries) {
         return;
     }
-    const int2 rowAndToken = runOrder[static_cast<uint64_t>(step) * stepEntries + within / tilesPerRow];
+    const int2 rowAndToken = runOrder[static_cast<uint64_t>(first) + entry];
     if (rowAndToken.x < 0) {
         return;
     }
-    const uint32_t begin = (within % tilesPerRow) * kTileUnits;
+    const uint32_t begin = (within - entry * tilesPerRow) * kTileUnits;
     const MF_GLOBAL u32x4 *src = reinterpret_cast<const MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(x)) +
                                  static_cast<uint64_t>(rowAndToken.y) * unitsPerRow;
     MF_GLOBAL u32x4 *dst = reinterpret_cast<MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(out)) +
@@ -1440,30 +1504,54 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
     // that was measured (8192 tokens, top-8, 256 experts, 7168 elements: 174 against 208 us with the loop kernel;
     // 1024 elements: 44 against 49 us with one workgroup per token).  Rows that are not whole cache lines
     // (10 000 elements) lose, whatever the step: every tile then begins and ends inside a line; they keep the loop kernel.
-    uint32_t stepSlices = kRankSlices;
-    while (stepSlices > 1 && static_cast<uint64_t>(stepSlices * 64 / topK + 1) * hidden * 2 > 2200000ull) {
-        stepSlices /= 2;
+    // Where steps of whole blocks and of several lie, and why: see kTileStepBytes.
+    uint32_t restSlices = kRankSlices;
+    while (restSlices > 1 && static_cast<uint64_t>(restSlices * 64 / topK + 1) * hidden * 2 > 2200000ull) {
+        restSlices /= 2;
     }
     // a call of few blocks is cut finer, so that every XCD gets steps to work on
-    while (stepSlices > 1 && static_cast<uint64_t>(blocks) * (kRankSlices / stepSlices) < 2 * kTileStreams) {
-        stepSlices /= 2;
+    while (restSlices > 1 && static_cast<uint64_t>(blocks) * (kRankSlices / restSlices) < 2 * kTileStreams) {
+        restSlices /= 2;
     }
-    const uint32_t stepEntries = stepSlices * 64;
-    const uint32_t stepsPerBlock = kRankSlices / stepSlices;
-    const uint64_t steps = static_cast<uint64_t>(blocks) * stepsPerBlock;
     const uint32_t tilesPerRow = (upr + kTileUnits - 1) / kTileUnits;
-    const uint64_t tileGrid = (steps + kTileStreams - 1) / kTileStreams * kTileStreams * stepEntries * tilesPerRow;
+    const auto tileGridOf = [&](uint32_t longBlocks, uint32_t slices) {     // longBlocks: whole rounds of them
+        const uint64_t restSteps = static_cast<uint64_t>(blocks - longBlocks) * (kRankSlices / slices);
+        return (static_cast<uint64_t>(longBlocks) * kRankBlock + (restSteps + kTileStreams - 1) / kTileStreams * kTileStreams * slices * 64) * tilesPerRow;
+    };
     const bool tiles = g_xcdStreams.load(std::memory_order_relaxed) != 0 && x != nullptr && out != nullptr && upr >= kTileUnits &&
-                       hidden % 64 == 0 && static_cast<uint64_t>(stepEntries / topK + 1) * hidden * 2 <= 2200000ull &&
-                       stepsPerBlock * experts <= 4096 && tileGrid <= 0x7FFFFFFFull;
+                       hidden % 64 == 0 && static_cast<uint64_t>(restSlices * 64 / topK + 1) * hidden * 2 <= 2200000ull &&
+                       kRankSlices / restSlices * experts <= 4096 && tileGridOf(0, restSlices) <= 0x7FFFFFFFull;
     // Up to kCountingBlocks blocks rank without a histogram launch in front of them: every block counts the entries
     // of the others itself.  Dispatch of rows of 1024 elements, with the launch / so: 2200 tokens at top-8 over 256 experts (18 blocks)
     // 20.1 / 17.6 us, 3000 (24) 19.7 / 18.3, 4096 (32) 22.2 / 22.0 (of 7168 elements 90.3 / 90.6).  The counts of a wave land on few LDS
     // words when the experts are few: over 64, 12 blocks 15.7 / 13.8, 16 34.5 / 34.0, 24 63.6 / 63.9 (longer rows); over 8, 16 blocks
     // 19.7 / 20.2.  (The short ones of these have one launch by now.)
     const bool counting = blocks <= (experts >= 128 ? kCountingBlocks : experts >= 64 ? 16u : 8u);
+    uint32_t together = 1;
+    const auto stepFits = [&](uint32_t m) { return static_cast<uint64_t>(kRankBlock / topK) * m * hidden * 2 <= kTileStepBytes; };
+    if (tiles && !counting && topK > kTileWholeSlots && hidden * 2 >= kTileTogetherRowBytes &&
+        (experts > kTileFewExperts || (experts == kTileFewExperts && hidden * 2 >= kTileLongRowBytes))) {
+        while (static_cast<uint64_t>(kRankBlock) * together * hidden * 2 < kTileRunBytes * experts && stepFits(2 * together) &&
+               2 * together <= kTileMostTogether && blocks >= 2 * together * kTileStreams) {
+            together *= 2;
+        }
+    }
+    const uint32_t longRounds = together > 1 ? blocks / (together * kTileStreams) : 0;
+    const uint32_t blocksTogether = longRounds * together * kTileStreams;
+    uint32_t wholeRounds = 0;
+    if (tiles && (restSlices == kRankSlices || (topK >= kTileWholeSlots && stepFits(1))) && blocks >= 2 * kTileStreams) {
+        wholeRounds = (blocks - blocksTogether) / kTileStreams;
+    }
+    const uint32_t blocksWhole = blocksTogether + wholeRounds * kTileStreams;
+    if (wholeRounds != 0 || blocksTogether != 0) {
+        while ((blocks - blocksWhole) * (kRankSlices / restSlices) % kTileStreams != 0 &&
+               kRankSlices / restSlices * 2 * experts <= 4096) {
+            restSlices /= 2;
+        }
+    }
+    const uint32_t stepsPerBlock = kRankSlices / restSlices;
     const size_t rankLds = histLds + (experts + kRankThreads + kRankSlices + (tiles ? stepsPerBlock * experts : 0) +
-                                      (counting ? experts : 0)) * sizeof(uint32_t);
+                                      (counting || blocksTogether != 0 ? experts : 0)) * sizeof(uint32_t);
     const uint64_t tableBytes = 256 + histStride * sizeof(uint32_t) + static_cast<uint64_t>(histStride) * experts * sizeof(uint32_t);
     int2 *runOrder = tiles ? reinterpret_cast<int2 *>(static_cast<char *>(workspace) + (tableBytes + 15) / 16 * 16) : nullptr;
     const uint64_t rowBytes = static_cast<uint64_t>(upr) * 16;
@@ -1480,15 +1568,16 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
     }
     hipLaunchKernelGGL(MoeRankKernel, dim3(blocks + warmGroups), dim3(kRankThreads), rankLds, s, static_cast<const int32_t *>(topk),
                        total, experts, blockHist, histStride, static_cast<int32_t *>(counts), static_cast<int32_t *>(offsets),
-                       static_cast<int32_t *>(rowOf), static_cast<int32_t *>(srcOf), blockBad, status, topK, runOrder, stepSlices,
-                       blocks, warm + warmFirst, warmUnits - warmFirst);
+                       static_cast<int32_t *>(rowOf), static_cast<int32_t *>(srcOf), blockBad, status, topK, runOrder, restSlices,
+                       together, blocksTogether, blocksWhole, blocks, warm + warmFirst, warmUnits - warmFirst);
     if (x != nullptr && out != nullptr && hidden != 0) {
         const u32x4 *xi = static_cast<const u32x4 *>(x);
         const int32_t *ro = static_cast<const int32_t *>(rowOf);
         u32x4 *oo = static_cast<u32x4 *>(out);
         if (tiles) {
-            hipLaunchKernelGGL(MoePermuteTileKernel, dim3(static_cast<uint32_t>(tileGrid)), dim3(64), 0, s, xi, runOrder, upr,
-                               tilesPerRow, static_cast<uint32_t>(steps), stepEntries, oo);
+            const TilePlan plan{blocks * kRankBlock, together * kRankBlock, longRounds, wholeRounds, restSlices * 64};
+            hipLaunchKernelGGL(MoePermuteTileKernel, dim3(static_cast<uint32_t>(tileGridOf(blocksWhole, restSlices))), dim3(64), 0, s, xi, runOrder,
+                               upr, tilesPerRow, plan, oo);
         } else if (upr >= 512) {
             // Wide rows: single-wave workgroups that hold up to 14 pieces per lane (a whole 7168-element
             // row) and write them with plain stores; sixteen waves per CU that each take several tokens and

@@ -560,3 +560,40 @@ def test_combine_of_any_values(gpu, oracle, T, H, K):
 ])
 def test_more_blocks_that_count_one_anothers_entries(gpu, oracle, T, K, E):
     test_few_blocks_that_count_one_anothers_entries(gpu, oracle, T, K, E)
+
+
+# Rounds of steps of eight, four and two blocks, of whole ones and of the parts of those that are left: the fewest blocks of each, one to seven left,
+# blocks that end inside a token, a last one that is not full.
+@pytest.mark.parametrize("T,H,K,E", [
+    (8192, 2048, 8, 256), (8065, 2048, 8, 256), (8064, 2048, 8, 256), (6145, 2048, 8, 256), (16385, 2048, 8, 512), (9400, 2112, 7, 300), (6200, 2048, 16, 129),
+    (7300, 4096, 8, 512), (7040, 4096, 8, 129), (6300, 4096, 8, 128), (4100, 7168, 8, 256), (5150, 7168, 8, 128), (6400, 7168, 8, 127), (4000, 8192, 8, 512),
+    (6000, 7168, 6, 256), (5200, 7168, 4, 8), (5633, 7168, 4, 64), (9999, 4096, 4, 256), (8400, 1024, 8, 256),
+])
+@pytest.mark.parametrize("refused", [False, True])
+def test_tiles_in_steps_of_several_blocks(gpu, T, H, K, E, refused):
+    torch = pytest.importorskip("torch")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T + K)
+    x = torch.randint(-2**63, 2**63 - 1, (T, H // 4), dtype=torch.int64, device="cuda", generator=g)
+    ids = torch.randint(0, E, (T, K), dtype=torch.int32, device="cuda", generator=g)
+    if refused:                                             # entries without a row, some all of a slice
+        ids.view(-1)[torch.randint(0, T * K, (500,), device="cuda", generator=g)] = E
+        ids.view(-1)[4096:4160] = -1
+    flat = torch.where((ids < 0) | (ids >= E), E, ids).view(-1)
+    order = torch.sort(flat, stable=True).indices[:int((flat < E).sum())]
+    row_of = torch.full((T * K,), -1, dtype=torch.int32, device="cuda")
+    row_of[order] = torch.arange(len(order), dtype=torch.int32, device="cuda")
+    counts = torch.bincount(flat, minlength=E + 1)[:E].to(torch.int32)
+    room = gpu.mf_moe_workspace_bytes(T, K, E)
+    rows = torch.full((T * K + 1, H // 4), 0x5A, dtype=torch.int64, device="cuda")
+    got = {name: torch.full((n,), -7, dtype=torch.int32, device="cuda") for name, n in
+           (("counts", E), ("offsets", E), ("row_of", T * K), ("source_of", T * K), ("workspace", room // 4 + 1))}
+    torch.cuda.synchronize()
+    assert gpu.mf_moe_dispatch_counts(T, H, K, E) == 0
+    assert gpu.mf_moe_dispatch(x.data_ptr(), ids.data_ptr(), T, H, K, E, rows.data_ptr(), got["counts"].data_ptr(), got["offsets"].data_ptr(),
+                               got["row_of"].data_ptr(), got["source_of"].data_ptr(), got["workspace"].data_ptr(), room, None) == 0, native.last_error()
+    assert gpu.mfrt_device_sync() == 0
+    assert torch.equal(got["counts"], counts) and torch.equal(got["offsets"], (torch.cumsum(counts, 0) - counts).to(torch.int32))
+    assert torch.equal(got["row_of"], row_of) and torch.equal(got["source_of"][:len(order)], order.to(torch.int32))
+    assert int(got["workspace"][0]) == int(refused) and int(got["workspace"][-1]) == -7
+    assert torch.equal(rows[:len(order)], x[order // K]) and bool((rows[len(order):] == 0x5A).all())
