@@ -2121,29 +2121,30 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         queuedBytes = total;
         oversized = total > 0xFFFFFFFFull;
         units = ChooseUnits(total, cu, route, tuning_);
-        // Large HBM copies of one submitter: 16 KiB chunks for the kernel that alternates between read and write windows.
-        // Where a source and its destination differ modulo 16, and below kWindowMinBytes from where held stores end, by the kernel that
-        // takes any chunk (XcopyLineWindowKernel has the figures).
+        // Large HBM copies of one submitter: 16 KiB chunks for the kernel that alternates between read and write windows, from where
+        // held stores end (XcopyWindowKernel has the figures).
         const bool aligned = (addressBits & (kWindowAlignBytes - 1)) == 0;
         const bool apart = (apartBits & (kUnitBytes - 1)) != 0;
         windowed = !unordered && !apart && WindowsApply(total, route, kWindowMinBytes);
         lineWindowed = !unordered && !windowed && WindowsApply(total, route, kDeepMaxBytes + 1) && !DeepHoldApplies(total, n, route, unordered);
-        // Segments that all start on cache lines, in source and destination, hold a higher rate.  Back to back at 6.8 / 7.1 /
-        // 7.4 TB/s, the same in four processes: 2 GiB in one segment 6.65 / 6.95 / 7.02 to 7.27, 32 x 16 MiB 6.65 / 6.95 / 7.05 to
-        // 7.26, 128 x 9 MiB 6.65 / 6.95 / 6.76 to 7.32.  The reshard's launches of 128 segments of 0.4 to 17 MB from eight
-        // places hold 7.1 in every process (6.87 to 7.00) and 7.4 only in some (7.0 to 7.2 in one, 5.8 to 6.1 in three others):
-        // long segments take the highest rate, other aligned ones the one between.  Where segments start between cache lines
-        // their chunks are cut on the lines and hold 7.1 too; shifted ones hold 6.8.
+        // Segments that all start on cache lines, in source and destination, hold a higher rate, and long ones the highest; those whose
+        // destinations are off a line hold that of the first, as their chunks are cut on lines, and shifted ones a little more than the general one.
+        // Back to back, us, at 7.2 / 7.3 / 7.4 / 7.5 TB/s: one segment of 370 MB 110.0 / 108.8 / 107.9 / 107.0, 900 MB 269 / 266 / 264 / 262 (512 MiB at 7.6 158 to
+        // 162, 7.5 151 to 155); 128 x 9 MB 355 / 348 / 348 / 350, 128 x 2.4 MB 91.9 / 92.1 / 91.8 / 101.9; the column-parallel part of 28 layers with its rectangles
+        // 3986 / 3955 / 3952 / 3958; off a line 300 MB 89.0 / 87.7 / 87.1 / 86.1, 900 MB 271 / 269 / 262 / 262.  Shifted, at 6.8 / 7.0 / 7.2 / 7.3: 200 MB 63.4 / 62.1 / 61.0 / 61.2,
+        // 900 MB 282 / 278 / 276 / 281, 100 of 2 MB on average 35.4 / 35.2 / 36.2 / 36.8, of 4 MB 131 / 129 / 135 / 144.
         const bool longSegments = (windowed || lineWindowed) && total / n >= kWindowLongSegmentBytes;
         if (longSegments && maySlice && total >= 2 * kWindowPieceBytes) {
             // A windowed launch that loses its schedule runs the rest of its bytes at the rate without windows, and the longer
             // it runs the likelier that is: launches of kWindowPieceBytes to twice that, each with a schedule of its own, hold
-            // a target the whole copy in one launch does not (2 GiB at 7.4 TB/s: 7.1 TB/s on average in four launches,
+            // a target the whole copy in one launch does not (2 GiB at 7.4 TB/s on 4096 waves: 7.1 TB/s on average in four launches,
             // 6.6 to 6.8 in one).  Only long segments are worth it: 896 segments of some 10 MB in launches of 64 or 96
             // segments (600 to 900 MB) were no faster than in launches of 128.
             return SubmitInPieces(src, dst, len, n, total, route, stream, mask, maskValue);
         }
-        linesRate = !apart && tuning_.windowAlignedMBps != 0 ? tuning_.windowAlignedMBps : tuning_.windowMBps;
+        linesRate = tuning_.windowAlignedMBps == 0 ? tuning_.windowMBps
+                    : apart                          ? std::min(tuning_.windowMBps / 34 * 35, tuning_.windowAlignedMBps)
+                                                     : tuning_.windowAlignedMBps;
         windowRate = tuning_.windowMBps;
         if (aligned && longSegments && tuning_.windowLongMBps != 0) {
             windowRate = tuning_.windowLongMBps;

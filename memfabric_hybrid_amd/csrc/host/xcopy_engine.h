@@ -84,16 +84,13 @@ struct XcopyTuning {
     bool stageUnordered = true;  // the upload of a ragged table's descriptors is launched without a barrier
     uint32_t deviceTableWgPerCu = 0;   // grid of a device-resident table in workgroups per CU, 0 = four per segment between 16 and 1024 per CU
     uint32_t windowMBps = 6800000;   // long HBM copies alternate between read and write windows cut for this rate; 0 = never
-    uint32_t windowAlignedMBps = 7100000;   // the same for launches of segments that all start at multiples of kWindowAlignBytes in source and destination, which hold more; 0 = the rate above
-    uint32_t windowLongMBps = 7400000;      // and for those of them whose segments are kWindowLongSegmentBytes and longer on average, which hold more still; 0 = the rate above
+    uint32_t windowAlignedMBps = 7300000;   // the same for launches of segments that all start at multiples of kWindowAlignBytes in source and destination, which hold more; 0 = the rate above
+    uint32_t windowLongMBps = 7500000;      // and for those of them whose segments are kWindowLongSegmentBytes and longer on average, which hold more still; 0 = the rate above
 };
 
-// From this total on a batch of up to 128 segments between HBM addresses that agree modulo 16 is copied by XcopyWindowKernel, or by
-// XcopyLineWindowKernel where a destination is off a cache line; below, and where source and destination differ modulo 16, by the latter from
-// where held stores end (64 MiB, 112 for one segment).  Back to back, 32 segments on lines, windows against none: 66 MiB 6.37
-// against 5.71 TB/s, 80 MiB 6.57 against 5.76, 130 MiB 6.94 against 6.14, 256 MiB 7.14 against 6.37, 600 MiB 7.20 against 6.31.  The limit
-// is where chunks that are not whole, which XcopyWindowKernel copies in its write half, stop to matter (100 segments of together 70 / 126 / 150 MiB
-// 29.0 / 43.4 / 47.6 us in that one, 24.6 / 43.4 / 48.5 in the other).
+// A batch of up to 128 segments between HBM addresses is copied in windows from where held stores end (64 MiB, 112 for one segment); from this
+// total on the caller names a rate for segments on cache lines besides.  Back to back, 32 segments on lines, windows of 4096 waves against none:
+// 66 MiB 6.37 against 5.71 TB/s, 80 MiB 6.57 against 5.76, 130 MiB 6.94 against 6.14, 256 MiB 7.14 against 6.37, 600 MiB 7.20 against 6.31.
 constexpr uint64_t kWindowMinBytes = 128ull << 20;
 // Rectangles in chunks of their payload: in windows, and without (several threads, rows between cache lines), where whole rows are as
 // fast up to 40 MB (Copy2dChunkKernel has the figures).

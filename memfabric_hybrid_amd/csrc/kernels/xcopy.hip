@@ -342,6 +342,13 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyInlineKernel(const InlineP
 constexpr uint32_t kWindowDepth = 16;                       // 128-bit loads per lane and round
 constexpr uint32_t kWindowUnits = 64 * kWindowDepth;        // 16 KiB chunks, one wave each
 constexpr uint32_t kWindowWaves = 4096;                     // 16 per CU
+// XcopyWindowKernel's, 24 per CU.  A period of half as many waves again is as much longer, so a wave whose loads land late has more of it to
+// catch up in, and HBM turns round less often.  4096 / 5120 / 6144 waves, the mean of sixteen launches in pairs, us: 128 x 9 MB at 7.1 TB/s 359 / 355 / 346, at
+// 7.4 377 / 357 / 351; 128 x 2.4 MB at 7.4 102 / 93 / 90; 170 MiB at 7.6 56.4 / 55.8 / 52.2; shifted, 512 MiB at 7.1 164 / 168 / 161.  7168 waves are as many as there
+// are registers for the data of, and spill what else they need (170 MiB at 7.6 52.5).  The read and the write part as long as each other: 47 and 53 % of the period for reads are
+// no better; nor are parts that issue in 95 or 90 % of their time and leave the rest for stragglers (128 x 9 MB at 7.2 346, 379, at 100 % 348).
+constexpr uint32_t kLongWavesPerSimd = 6;
+constexpr uint32_t kLongWaves = 6144;
 
 // Chunk c of a segment; with onLines one of LineChunks(), as a segment of its own.
 struct SegChunk {
@@ -357,36 +364,6 @@ __device__ __forceinline__ SegChunk ChunkOn(bool onLines, uint64_t src, uint64_t
     }
     const LineSpan span = LineChunk(dst, len, c, units);
     return SegChunk{src + span.begin, dst + span.begin, span.end - span.begin, 0};
-}
-
-// Copy chunk k (kWindowUnits units) of one segment: loads at `slot`, stores at `slot + half`.  A chunk that is
-// not whole (the last one of a segment, or one with head or tail bytes) goes through CopyChunk in the
-// write half: there are at most two such chunks per segment.
-template <bool kNtLoad, int kStore>
-__device__ __forceinline__ void CopyChunkWindowed(uint64_t src, uint64_t dst, uint64_t len, uint64_t k, uint64_t slot, uint32_t half)
-{
-    const SegGeom g = SegmentGeometry(dst, len);
-    const uint64_t u0 = k * kWindowUnits;
-    const bool whole = u0 + kWindowUnits <= g.body && (k != 0 || g.head == 0) && (u0 + kWindowUnits < g.body || g.tail == 0);
-    WaitForClock(slot);
-    if (!whole) {
-        WaitForClock(slot + half);
-        CopyChunk<kNtLoad, kStore>(src, dst, len, k, kWindowUnits);
-        return;
-    }
-    const uint64_t s = src + g.head + u0 * kUnitBytes + threadIdx.x * kUnitBytes;
-    const uint64_t d = dst + g.head + u0 * kUnitBytes + threadIdx.x * kUnitBytes;
-    u32x4 v[kWindowDepth];
-#pragma unroll
-    for (uint32_t j = 0; j < kWindowDepth; ++j) {
-        v[j] = LoadUnit<kNtLoad>(s + j * 64 * kUnitBytes);
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    WaitForClock(slot + half);
-#pragma unroll
-    for (uint32_t j = 0; j < kWindowDepth; ++j) {
-        StoreUnit<kStore>(d + j * 64 * kUnitBytes, v[j]);
-    }
 }
 
 // One chunk under a hold mode.  kHoldDeep: a chunk of up to kWindowUnits units is read by a single wave with up to
@@ -439,22 +416,6 @@ __device__ __forceinline__ void CopyChunkHeld(uint64_t src, uint64_t dst, uint64
     if (u0 + kWindowUnits >= g.body && tid < g.tail) {
         const uint64_t off = g.head + g.body * kUnitBytes + tid;
         CopyByte<kStore>(src + off, dst + off);
-    }
-}
-
-// The inline plan (chunks of kWindowUnits units, destinations on lines) copied by gridDim.x single-wave workgroups that walk
-// the chunks with stride gridDim.x, one chunk per period each.
-template <bool kNtLoad, int kStore>
-__global__ __launch_bounds__(64) void XcopyWindowKernel(const InlinePlan p, uint32_t period, uint32_t seq)
-{
-    const InlineRows rows(p);
-    const uint32_t nchunk = p.nchunk;
-    const uint32_t half = period / 2;
-    uint64_t slot = AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * half / gridDim.x;
-    for (uint32_t c = blockIdx.x; c < nchunk; c += gridDim.x) {
-        const InlineChunk r = rows.Owner(c);
-        CopyChunkWindowed<kNtLoad, kStore>(r.src, r.dst, r.len, r.k, slot, half);
-        slot += period;
     }
 }
 
@@ -977,22 +938,54 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kHeldWavesPe
     }
 }
 
-// XcopyWindowKernel in chunks of LineChunks(), whatever source and destination are modulo 16, a chunk as XcopyPieceHeldKernel's: one that is not
-// whole, or whose bytes are shifted, keeps to the windows too, where XcopyWindowKernel copies it in the write half and one kernel of straddling loads falls behind.
-// HBM is the bound.  us back to back, without windows or in those of XcopyWindowKernel / so.  Source and destination different modulo 16: one segment of 120 / 200 /
-// 500 / 1024 MB 40.4 / 38.9, 65.9 / 63.1, 160 / 154, 335 / 323, 16 of together 74 / 157 / 315 MB 28.1 / 25.8, 56.4 / 50.8, 108 / 98.5, 128 of them 29.8 / 26.6, 60.3 / 52.7,
-// 115 / 99.8.  Alike modulo 16, destinations between lines: one of 134 / 300 / 700 MB 42.7 / 41.2, 93.6 / 90.6, 217 / 210, 16 of 74 / 157 / 315 MB 27.3 / 24.0, 52.2 / 48.3,
-// 98.5 / 94.4, 128 of them 28.8 / 25.0, 54.7 / 48.9, 101.6 / 95.1.  On lines below kWindowMinBytes: one of 118 / 126 MB 38.8 / 35.3, 41.1 / 38.2, two of together 74 / 132 MB
-// 25.3 / 23.5, 43.1 / 40.2, 100 of them 27.1 / 24.6, 45.8 / 43.4; above, the kernel with less to compute is as fast or 1 % faster.
-// Rates, 6.5 / 6.8 / 6.95 / 7.1 TB/s where bytes are shifted: 200 MB 65.5 / 63.1 / 62.2 / 61.6, 1024 MB 333 / 325 / 332 / 352, 100 x 10 MB 323 / 317 / 318 / 343; and
-// 6.8 / 7.1 / 7.3 where they are not: 300 MB 93.6 / 90.6 / 88.6, 1024 MB 319 / 312 / 323, 100 x 10 MB 314 / 310 / 350.
-__global__ __launch_bounds__(64) void XcopyLineWindowKernel(const InlinePlan p, uint32_t period, uint32_t seq)
+// The rows of an InlinePlan in LDS, for waves that look them up again and again: held in registers, as InlineRows does, they would take the
+// place of a wave.
+struct SharedRows {
+    uint64_t src[kInlineSegs];
+    uint64_t dst[kInlineSegs];
+    uint32_t len[kInlineSegs];
+    uint32_t first[kInlineSegs];
+
+    // by a workgroup of one wave
+    __device__ __forceinline__ void Keep(const InlineRows &r)
+    {
+        const uint32_t lane = threadIdx.x;
+        src[lane] = r.s0;
+        src[lane + 64] = r.s1;
+        dst[lane] = r.d0;
+        dst[lane + 64] = r.d1;
+        len[lane] = r.l0;
+        len[lane + 64] = r.l1;
+        first[lane] = r.f0;
+        first[lane + 64] = r.f1;
+        __syncthreads();
+    }
+    __device__ __forceinline__ InlineChunk Owner(uint32_t c) const
+    {
+        uint32_t lane = threadIdx.x;
+        asm volatile("" : "+v"(lane));      // read anew in every round
+        const uint32_t s = __popcll(__ballot(first[lane] <= c)) + __popcll(__ballot(first[lane + 64] <= c)) - 1;
+        return InlineChunk{Uniform(src[s]), Uniform(dst[s]), Uniform(len[s]), c - Uniform(first[s])};
+    }
+};
+
+// The inline plan in chunks of LineChunks(), whatever source and destination are modulo 16, in windows: single-wave workgroups walk the chunks
+// with stride gridDim.x, one per period each, as XcopyPieceHeldKernel copies a piece, so that a chunk that is not whole, or whose bytes are shifted, keeps to the windows too.
+// HBM is the bound.  us back to back, 4096 waves that keep the table in registers, cut for 7.1 (one segment on lines 7.4, shifted 6.8) TB/s / this, cut for 7.3 (7.5, 7.0):
+// one segment on lines of 136 / 370 / 900 MB 39.3 / 39.0, 104.0 / 102.4, 252.6 / 247.3; off a line 300 / 700 MB 90.6 / 85.3, 210 / 197; shifted 200 MB 63.1 / 60.5;
+// 128 of 2.4 / 9 MB 92.4 / 88.5, 337 / 326; reshards with their rectangles, 13 layers of 1280 548 / 533, 28 of 3584 3873 / 3831.
+// Beside eight elementwise kernels of another stream over 1 GiB, both together, 18 of 512 MiB 6333 / 6341, 31 of 128 x 2.4 MB 6485 / 6337; beside products of
+// matrices 3412 / 3478, 3495 / 3475.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kLongWavesPerSimd, kLongWavesPerSimd))) void XcopyWindowKernel(
+    const InlinePlan p, uint32_t period, uint32_t seq)
 {
-    const InlineRows rows(p);
+    __shared__ SharedRows rows;
+    const InlineRows fetched(p);            // on their way while the start is agreed
     const uint32_t nchunk = p.nchunk;
     const uint32_t groups = gridDim.x;
     const uint32_t half = period / 2;
     uint64_t slot = AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * half / groups;
+    rows.Keep(fetched);
     for (uint32_t c = blockIdx.x; c < nchunk; c += groups, slot += period) {
         const InlineChunk r = rows.Owner(c);
         const LineSpan span = LineChunk(r.dst, r.len, r.k, kDeepUnits);
@@ -2027,14 +2020,15 @@ InlinePlan CutOnLines(const InlinePlan &plan)
 }
 
 // windowMBps: the rate (MB/s of HBM traffic, read + written) the period of a windowed launch is cut for.
-int LaunchWindowed(void (*kernel)(const InlinePlan, uint32_t, uint32_t), const InlinePlan &plan, uint32_t windowMBps, hipStream_t stream)
+int LaunchWindowed(const InlinePlan &plan, uint32_t windowMBps, hipStream_t stream)
 {
-    const uint32_t grid = WindowGrid(plan.nchunk, kWindowWaves);
+    const InlinePlan lines = CutOnLines(plan);
+    const uint32_t grid = WindowGrid(lines.nchunk, kLongWaves);
     const uint32_t ticks = WindowPeriodTicks(2ull * grid * kWindowUnits * kUnitBytes, windowMBps);
     if (ticks == 0) {
         return static_cast<int>(hipErrorInvalidValue);
     }
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, stream, plan, ticks, NextWindowSeq());
+    hipLaunchKernelGGL(XcopyWindowKernel, dim3(grid), dim3(64), 0, stream, lines, ticks, NextWindowSeq());
     return static_cast<int>(hipGetLastError());
 }
 
@@ -2171,7 +2165,7 @@ extern "C" int mfk_xcopy_windows_available(void)
 
 extern "C" uint32_t mfk_xcopy_window_waves(void)
 {
-    return mf::kWindowWaves;
+    return mf::kLongWaves;
 }
 
 extern "C" int mfk_xcopy_line_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream)
@@ -2182,7 +2176,7 @@ extern "C" int mfk_xcopy_line_windowed(const void *inlinePlan, uint32_t windowMB
     if (plan.units != kWindowUnits || plan.nchunk == 0 || windowMBps == 0) {
         return -1;
     }
-    const int err = LaunchWindowed(XcopyLineWindowKernel, CutOnLines(plan), windowMBps, s);
+    const int err = LaunchWindowed(plan, windowMBps, s);
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
@@ -2194,12 +2188,7 @@ extern "C" int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, u
     if (plan.units != kWindowUnits || plan.nchunk == 0 || windowMBps == 0) {
         return -1;
     }
-    if (!OnLines(plan)) {
-        return mfk_xcopy_line_windowed(inlinePlan, linesMBps, mask, maskValue, stream);
-    }
-    const int err = WithPolicy(PolicyOf(MFRT_ROUTE_HBM), [&](auto ntLoad, auto store) {
-        return LaunchWindowed(XcopyWindowKernel<decltype(ntLoad)::value, decltype(store)::value>, plan, windowMBps, s);
-    });
+    const int err = LaunchWindowed(plan, OnLines(plan) ? windowMBps : linesMBps, s);
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
@@ -2398,8 +2387,7 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
                 (void)Launch(XcopyPlannedKernel<1, kPlannedShortRun>, 1, 64, 64, s, 0, 0u, TablePace{});
                 (void)Launch(XcopyPlannedKernel<kPlannedWaves, kPlannedRun>, 1, 64 * kPlannedWaves, 64, s, 0, 0u, TablePace{});
                 (void)Launch(XcopySampledKernel, 1, 64, 0, s, 0, 0u, 0, 0u, TablePace{});
-                hipLaunchKernelGGL((XcopyWindowKernel<kNt, kSt>), dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
-                hipLaunchKernelGGL(XcopyLineWindowKernel, dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
+                hipLaunchKernelGGL(XcopyWindowKernel, dim3(1), dim3(64), 0, s, empty, 64u, NextWindowSeq());
             }
             return 0;
         });
@@ -2525,7 +2513,7 @@ extern "C" int mfk_xcopy_calibrate(void *stream, const uint32_t *holdNanos, cons
                 big.units = kWindowUnits;
                 big.nchunk = static_cast<uint32_t>(half / (kWindowUnits * kUnitBytes));
                 const uint32_t rate = windowMBps[v - 1];
-                err = timed([&](int) { (void)LaunchWindowed(XcopyWindowKernel<true, kStoreStream>, big, rate, s); }, round == 0 ? 1 : 0, 1,
+                err = timed([&](int) { (void)LaunchWindowed(big, rate, s); }, round == 0 ? 1 : 0, 1,
                             out[4 + v]);
             }
             if (err != hipSuccess) {

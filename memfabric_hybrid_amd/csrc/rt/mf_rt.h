@@ -94,7 +94,7 @@ int mfk_xcopy_windows_available(void);   /* 1 when the current device's constant
 uint32_t mfk_xcopy_window_units(void);
 uint32_t mfk_xcopy_window_waves(void);
 int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, uint32_t linesMBps, void *mask, uint32_t maskValue, void *stream);
-/* The same with chunks cut on the destinations' cache lines, for any addresses (see XcopyLineWindowKernel). */
+/* The same at one rate, whatever the addresses. */
 int mfk_xcopy_line_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream);
 /* tablePlan: a mf::TablePlan (kernels/xcopy_plan.h).  Under a pattern its triples may live in pinned host
  * memory and neither prefix nor group map is read. */

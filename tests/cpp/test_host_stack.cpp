@@ -1998,7 +1998,7 @@ static void TestWindows()
     (void)fake_rt_last_window();
     uint64_t launchesBefore = mf_xcopy_launch_count();
     CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-    CHECK(fake_rt_last_window() == 7400000);                   // source and destination on cache lines: the higher rate
+    CHECK(fake_rt_last_window() == 7500000);                   // source and destination on cache lines: the higher rate
     CHECK(mf_xcopy_launch_count() - launchesBefore == 2);      // twice the minimum: two launches of 512 MiB, a schedule each
     CHECK(engine.DrainThread() == BM_OK);
     bool ok = true;
@@ -2066,7 +2066,7 @@ static void TestWindows()
             dst64[i] += 128 - 48;
         }
         CHECK(engine.Submit(src64.data(), dst64.data(), len64.data(), 64, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-        CHECK(fake_rt_last_window() == 7100000);       // on cache lines, 16 MiB each: the rate between
+        CHECK(fake_rt_last_window() == 7300000);       // on cache lines, 16 MiB each: the rate between
         CHECK(engine.DrainThread() == BM_OK);
     }
     l1 = (gib >> 3) - 1;                           // one byte below the limit: those of TestLineWindows
@@ -2074,7 +2074,7 @@ static void TestWindows()
     CHECK(fake_rt_last_window() == 0);
     l1 = gib >> 3;
     CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-    CHECK(fake_rt_last_window() == 7400000);
+    CHECK(fake_rt_last_window() == 7500000);
     {
         // between cache lines the same limit, at the general rate
         uint64_t so = s1 + 16;
@@ -2193,17 +2193,17 @@ static void TestLineWindows()
     XcopyEngine &engine = XcopyEngine::Instance();
     void *stream = mf_xcopy_thread_stream();
     const uint64_t mib = 1ull << 20;
-    const uint32_t general = XcopyTuning{}.windowMBps;
+    const uint32_t shifted = XcopyTuning{}.windowMBps / 34 * 35;
     const uint32_t between = XcopyTuning{}.windowAlignedMBps;
     const uint32_t most = XcopyTuning{}.windowLongMBps;
     struct Form { uint32_t n; uint64_t bytes, from, to; uint32_t rate; bool other; };
     const Form forms[] = {
         {1, kHeldSingleBytes, 0, 0, 0, false},          {1, kHeldSingleBytes, 3, 16, 0, false},         // held
-        {1, kHeldSingleBytes + 1, 0, 0, most, false},   {1, kHeldSingleBytes + 1, 16, 48, between, false}, {1, kHeldSingleBytes + 1, 3, 16, general, false},
+        {1, kHeldSingleBytes + 1, 0, 0, most, false},   {1, kHeldSingleBytes + 1, 16, 48, between, false}, {1, kHeldSingleBytes + 1, 3, 16, shifted, false},
         {1, 128 * mib - 1, 0, 0, most, false},          {1, 128 * mib, 0, 0, 0, true},                  {1, 128 * mib, 16, 48, 0, true},
-        {1, 128 * mib, 3, 16, general, false},          {1, 900 * mib + 5, 18, 7, general, false},      {1, 1024 * mib, 18, 7, general, false},
+        {1, 128 * mib, 3, 16, shifted, false},          {1, 900 * mib + 5, 18, 7, shifted, false},      {1, 1024 * mib, 18, 7, shifted, false},
         {2, 32 * mib, 0, 0, 0, false},                  {2, 32 * mib + 256, 0, 0, between, false},      {2, 32 * mib + 1, 16, 48, between, false},
-        {2, 64 * mib, 16, 48, 0, true},                 {2, 64 * mib - 1, 3, 16, general, false},       {128, mib + 77, 3, 16, general, false},
+        {2, 64 * mib, 16, 48, 0, true},                 {2, 64 * mib - 1, 3, 16, shifted, false},       {128, mib + 77, 3, 16, shifted, false},
         {128, 512 * 1024, 0, 0, 0, false},              {128, 512 * 1024 + 128, 0, 0, between, false},  {129, mib, 3, 16, 0, false},
     };
     for (const Form &f : forms) {

@@ -137,6 +137,20 @@ def test_batches_cut_on_lines_in_windows(gpu, lens, shift):
     assert torch.equal(target, expect)
 
 
+# Windows where a round of the waves ends: one of 6144 chunks of 16 KiB, two, and a chunk, a unit or a byte more or less.
+@pytest.mark.parametrize("n", [2 * 6144 * 16384 + more for more in (-16385, -1, 0, 1, 16, 16384, 16389)] + [6144 * 16384 * 3 // 2 + 5])
+@pytest.mark.parametrize("shift", [(0, 0), (16, 48), (3, 9)], ids=str)
+def test_windows_where_a_round_ends(gpu, n, shift):
+    torch = pytest.importorskip("torch")
+    source = torch.randint(-2**63, 2**63 - 1, (n // 8 + 32,), dtype=torch.int64, device="cuda").view(torch.uint8)
+    target = torch.zeros_like(source)
+    torch.cuda.synchronize()
+    gpu_util.xcopy(gpu, np.array([source.data_ptr() + shift[0]], dtype=np.uint64), np.array([target.data_ptr() + shift[1]], dtype=np.uint64),
+                   np.array([n], dtype=np.uint64), native.ROUTE_HBM)
+    assert torch.equal(target[shift[1]:shift[1] + n], source[shift[0]:shift[0] + n])
+    assert not target[:shift[1]].any() and not target[shift[1] + n:].any()
+
+
 @pytest.mark.parametrize("each", [512, 40000])
 @pytest.mark.parametrize("order", ["own", "a caller's", "own and a caller's", "own, blocking between", "own, a long copy in front",
                                    "a caller's, a long copy in front"])
