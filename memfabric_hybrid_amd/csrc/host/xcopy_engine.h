@@ -85,7 +85,7 @@ struct XcopyTuning {
     uint32_t deviceTableWgPerCu = 0;   // grid of a device-resident table in workgroups per CU, 0 = four per segment between 16 and 1024 per CU
     uint32_t windowMBps = 6800000;   // long HBM copies alternate between read and write windows cut for this rate; 0 = never
     uint32_t windowAlignedMBps = 7300000;   // the same for launches of segments that all start at multiples of kWindowAlignBytes in source and destination, which hold more; 0 = the rate above
-    uint32_t windowLongMBps = 7500000;      // and for those of them whose segments are kWindowLongSegmentBytes and longer on average, which hold more still; 0 = the rate above
+    uint32_t windowLongMBps = 7450000;      // and for those of them whose segments are kWindowLongSegmentBytes and longer on average, which hold more still; 0 = the rate above
 };
 
 // A batch of up to 128 segments between HBM addresses is copied in windows from where held stores end (64 MiB, 112 for one segment); from this

@@ -971,8 +971,8 @@ struct SharedRows {
 
 // The inline plan in chunks of LineChunks(), whatever source and destination are modulo 16, in windows: single-wave workgroups walk the chunks
 // with stride gridDim.x, one per period each, as XcopyPieceHeldKernel copies a piece, so that a chunk that is not whole, or whose bytes are shifted, keeps to the windows too.
-// HBM is the bound.  us back to back, 4096 waves that keep the table in registers, cut for 7.1 (one segment on lines 7.4, shifted 6.8) TB/s / this, cut for 7.3 (7.5, 7.0):
-// one segment on lines of 136 / 370 / 900 MB 39.3 / 39.0, 104.0 / 102.4, 252.6 / 247.3; off a line 300 / 700 MB 90.6 / 85.3, 210 / 197; shifted 200 MB 63.1 / 60.5;
+// HBM is the bound.  us back to back, 4096 waves that keep the table in registers, cut for 7.1 (one segment on lines 7.4, shifted 6.8) TB/s / this, cut for 7.3 (7.45, 7.0):
+// one segment on lines of 136 / 370 / 900 MB 39.3 / 39.3, 104.8 / 103.7, 257.2 / 253.7; off a line 300 / 700 MB 90.6 / 85.3, 210 / 197; shifted 200 MB 63.1 / 60.5;
 // 128 of 2.4 / 9 MB 92.4 / 88.5, 337 / 326; reshards with their rectangles, 13 layers of 1280 548 / 533, 28 of 3584 3873 / 3831.
 // Beside eight elementwise kernels of another stream over 1 GiB, both together, 18 of 512 MiB 6333 / 6341, 31 of 128 x 2.4 MB 6485 / 6337; beside products of
 // matrices 3412 / 3478, 3495 / 3475.

@@ -1998,7 +1998,7 @@ static void TestWindows()
     (void)fake_rt_last_window();
     uint64_t launchesBefore = mf_xcopy_launch_count();
     CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-    CHECK(fake_rt_last_window() == 7500000);                   // source and destination on cache lines: the higher rate
+    CHECK(fake_rt_last_window() == 7450000);                   // source and destination on cache lines: the higher rate
     CHECK(mf_xcopy_launch_count() - launchesBefore == 2);      // twice the minimum: two launches of 512 MiB, a schedule each
     CHECK(engine.DrainThread() == BM_OK);
     bool ok = true;
@@ -2074,7 +2074,7 @@ static void TestWindows()
     CHECK(fake_rt_last_window() == 0);
     l1 = gib >> 3;
     CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-    CHECK(fake_rt_last_window() == 7500000);
+    CHECK(fake_rt_last_window() == 7450000);
     {
         // between cache lines the same limit, at the general rate
         uint64_t so = s1 + 16;

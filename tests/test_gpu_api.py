@@ -451,7 +451,7 @@ def test_start_up_check_of_the_timing_rules(lib, pool):
     assert all(100.0 < t < 2000.0 for t in times[4:]), times      # a 512 MiB copy
     assert enabled.value in (0, 1) and delta.value in (-200, 0, 200)
     assert rate.value in (0, 6800000, 6800000 * 94 // 100)
-    assert (aligned_rate.value, long_rate.value) in ((rate.value, rate.value), (7300000, 7500000))
+    assert (aligned_rate.value, long_rate.value) in ((rate.value, rate.value), (7300000, 7450000))
     assert rate.value != 0 or aligned_rate.value == 0
     if enabled.value == 1:
         chosen = {0: times[1], -200: times[2], 200: times[3]}[delta.value]
