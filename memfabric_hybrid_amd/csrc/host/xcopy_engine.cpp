@@ -1835,36 +1835,49 @@ uint32_t XcopyEngine::PieceUnits(const BatchStats &stats, uint32_t n, bool unord
     return mean <= 6144 ? kXcopyThreads : mean <= 12288 ? kDeepUnits / 2 : kDeepUnits;
 }
 
-// Of 6.0 TB/s, which blocks at random places hold.  Blocks that begin and end on multiples of kWindowLongBlockBytes hold more: 6.4 where they
-// have one length, and 6.6 where they are written one behind the other, which leaves the rows of HBM open, up to kOrderedFastBytes, beyond which
-// not every launch holds that (8000 of 64 KiB 168 to 173 us, at 6.4 169; 16 384 345 to 355 and 345 to 349).  At 6.0 / 6.2 / 6.4 / 6.6 / 6.8, the same to 1 % in
-// four processes: 64 KiB gathered, 2048 47.6 / 46.3 / 44.9 / 43.7 / 44.1; scattered, 4096 92.6 / 90.0 / 87.7 / 86.0 / 96; 2000 of 128 KiB gathered and
-// scattered 90.7 / 87.8 / 85.4 / 83.3 / 85.  Elsewhere those rates fall apart.  300 and 700 MB at random places on both sides, at 6.0 / 6.4: 65 536 bytes at
-// multiples of 64 KiB 104.5 / 102.2, 238.7 / 235.3, at multiples of 4 KiB or 256 105.7 / 112.5, 246 / 275; 81 920 106.3 / 113.5, 247 / 277; 90 112 109.0 / 119.5,
-// 270 / 282; 110 776 107.1 / 117.5, 253 / 279; 163 840 240 / 249.  Written in order at 6.4 / 6.6: 73 728 100.7 / 106.8, 110 720 100.7 / 102.4, 81 920 98.4 / 96.6, but 226 / 232
-// at 700 MB; those stay at 6.4.  Short blocks in order hold 6.4 in some places of the pool only: from kOrderedWindowPieces on 6.0, where two held
-// launches or none are slower; without windows / at 6.0 / at 6.4, back to back 10 000 of 48 KiB 170.6 / 167.2 / -, 16 384 of 32 KiB 186 / 182 / 179 to
-// 185, of 16 KiB 94.3 / 92.1 / 91 to 95, alone 258 / 248 / 238 and 148 / 143 / 138; 7300 and 8192 of 32 KiB 82 / 83 / -, 92 / 92 / -.  Pieces that are
-// much less than full gain nothing; segments between cache lines keep the launch without windows, as they do in launches of
-// kInlineSegs segments up to kWindowSliceMinSegmentBytes.
+// What 6144 waves hold goes by where the segments are and how full their pieces.  us at 5.6 / 5.8 / 6.0 / 6.2 / 6.4 / 6.6 / 6.8 / 7.0 TB/s, back to back, the same to 1 %
+// in two or three processes.
+// Written one behind the other, which leaves the rows of HBM open.  Multiples of 64 KiB, 5000 of 64 KiB - / - / - / - / 105.9 / 102.8 / 100.4 / 98.1, 16 384 344 / 334 / 332 /
+// 326, but 2100 45.7 / 44.5 / 43.3 / 45.4: 6.8.  Others of one length, 4096 of 32 KiB 44.6 / 43.5 / 42.6 / 42.6, 16 384 173.4 / 170.0 / 166.7 / 190.3, 8000 of 40 960 bytes
+// 106.6 / 104.2 / 101.6 or 118.0 / 119.3, 7000 of 73 728 173.4 / 164.3 / 160.6 / 165.5, 3000 of 100 352 101.0 / 98.4 / 95.9 / -, 4500 of 32 896 50.0 / 49.7 / 52.9 / 56.4:
+// 6.6; 16 384 of 16 KiB 87.6 / 86.1 / 92.9 / 97.2, 9000 49.1 / 47.9 / 49.2 / 51.0: 6.4 below kOrderedSteadyBytes.  Of several lengths 6.4 where they are long, as it was.
+// Elsewhere multiples of 64 KiB of one length, 12 000 of 64 KiB scattered - / - / 272 / 259 / 254.7 / 248.5 / 250.5 / 289, 8000 - / - / 179.1 / 173.4 / 173.2 / 165.0 / 162.6 / 166.6: 6.6.
+// Others by how full their pieces are.  From 95 % on, long ones 6.3 (7000 of 65 536 bytes 157.9 / 154.3 / 152.1 / 165.6 from 6.0 on, at 6.4 160 in another process, 3500 of 81 920
+// 99.4 / 96.2 / 94.0 / 97.2, 6000 of 110 776 230 / 230 / 224 / 253, K and V blocks of 128 and 16 KiB 49.2 / 47.9 / 46.7 / 48.3); from 88 % on 6.0 (4500 of 32 KiB 54.1 / 54.1 / 54.1 / 54.4 / 57.0
+// from 5.6 on, 4000 of 73 728 103.3 / 100.7 / 102.8 / 113.4 from 6.0 on, 16 384 of 16 KiB scattered at 5.9 / 6.0 95.1 / 94.1), from 85 % on, and of one length from 75 %, 5.9 (8000 of 50 000 149.7 / 145.4 /
+// 144.6 / 158.6 from 5.6 on, at 6.0 158 in another process, 8000 of 24 576 at 5.8 / 5.9 / 6.0 71.7 / 70.9 / 77.8, 3800 of 28 000 39.4 / 39.5 / 41.2); below, of one length, 5.8 from three held
+// launches' worth on (8000 of 24 000 73.0 / 70.7 / 70.9 / 77.1 from 5.6 on, 6000 of 33 333 75.8 / 74.0 / 79.7 / 81.8; in two held launches 2500 of 33 333 31.8, so 32.1; of 20 000, 61 % full, none is better
+// than none).
+// At addresses off the lines held launches are as good or nearly (ragged ones of up to 131 072 bytes 262 MB 102.1, at 5.5 / 5.6 / 5.7 / 5.8 101.9 / 100.5 / 99.0 / 99.9; of up to
+// 101 706 169 MB 65.9, 66.7 / 66.1 / 66.4 / 67.4; of up to 60 000 240 MB 100.8, 104).
 uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t count, uint32_t units,
                                       bool unordered) const
 {
-    const bool full = stats.total >= static_cast<uint64_t>(count) * (kDeepUnits * kUnitBytes) / 100 * 85;
-    if (unordered || units != kDeepUnits || !full || (stats.addressBits & (kWindowAlignBytes - 1)) != 0 ||
+    constexpr uint64_t kOrderedSteadyBytes = 24000;
+    constexpr uint64_t kUnevenBytes = 24000;
+    if (unordered || units != kDeepUnits || (stats.addressBits & (kWindowAlignBytes - 1)) != 0 ||
         !WindowsApply(stats.total, MFRT_ROUTE_HBM, kPieceWindowMinBytes)) {
         return 0;
     }
-    constexpr uint64_t kOrderedWindowPieces = 16384;
-    constexpr uint64_t kOrderedFastBytes = 400ull << 20;
+    const uint32_t rate = tuning_.windowMBps / 68;      // of 68, what the general rate is
+    const uint64_t mean = stats.total / n;
+    const uint64_t percent = stats.total * 100 / (static_cast<uint64_t>(count) * (kDeepUnits * kUnitBytes));
     const bool equal = stats.total == stats.longest * n;
-    const bool onGrid = ((stats.addressBits | stats.lengthBits) & (kWindowLongBlockBytes - 1)) == 0;
+    const bool onGrid = equal && ((stats.addressBits | stats.lengthBits) & (kWindowLongBlockBytes - 1)) == 0;
+    const bool longBlocks = mean >= kWindowLongBlockBytes;
     if (WrittenInOrder(dst, len, n)) {
-        return stats.total / n >= kWindowLongBlockBytes             ? tuning_.windowMBps / 34 * (onGrid && stats.total < kOrderedFastBytes ? 33 : 32)
-               : equal && stats.deepPieces >= kOrderedWindowPieces ? tuning_.windowMBps / 17 * 15
-                                                                    : 0;
+        return onGrid ? rate * 68 : equal && mean >= kOrderedSteadyBytes ? rate * 66 : equal || (longBlocks && percent >= 85) ? rate * 64 : 0;
     }
-    return tuning_.windowMBps / 17 * (equal && onGrid ? 16 : 15);
+    if (onGrid) {
+        return rate * 66;
+    }
+    if (longBlocks && percent >= 95) {
+        return rate * 63;
+    }
+    if (percent >= 85 || (equal && percent >= 75)) {
+        return rate * (percent >= 88 ? 60 : 59);
+    }
+    return equal && mean >= kUnevenBytes && count > 2 * kHeldMaxPieces ? rate * 58 : 0;
 }
 
 // In how many launches, each of as many pieces as are held, a list of more goes out; 1 where one that holds nothing is as fast.  Back to back,

@@ -342,13 +342,14 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyInlineKernel(const InlineP
 constexpr uint32_t kWindowDepth = 16;                       // 128-bit loads per lane and round
 constexpr uint32_t kWindowUnits = 64 * kWindowDepth;        // 16 KiB chunks, one wave each
 constexpr uint32_t kWindowWaves = 4096;                     // 16 per CU
-// XcopyWindowKernel's, 24 per CU.  A period of half as many waves again is as much longer, so a wave whose loads land late has more of it to
+// XcopyWindowKernel's and XcopyPieceWindowKernel's, 24 per CU.  A period of half as many waves again is as much longer, so a wave whose loads land late has more of it to
 // catch up in, and HBM turns round less often.  4096 / 5120 / 6144 waves, the mean of sixteen launches in pairs, us: 128 x 9 MB at 7.1 TB/s 359 / 355 / 346, at
 // 7.4 377 / 357 / 351; 128 x 2.4 MB at 7.4 102 / 93 / 90; 170 MiB at 7.6 56.4 / 55.8 / 52.2; shifted, 512 MiB at 7.1 164 / 168 / 161.  7168 waves are as many as there
 // are registers for the data of, and spill what else they need (170 MiB at 7.6 52.5).  The read and the write part as long as each other: 47 and 53 % of the period for reads are
 // no better; nor are parts that issue in 95 or 90 % of their time and leave the rest for stragglers (128 x 9 MB at 7.2 346, 379, at 100 % 348).
 constexpr uint32_t kLongWavesPerSimd = 6;
 constexpr uint32_t kLongWaves = 6144;
+static_assert(kLongWaves % kPieceGroup == 0, "a round of pieces is whole groups");
 
 // Chunk c of a segment; with onLines one of LineChunks(), as a segment of its own.
 struct SegChunk {
@@ -1007,77 +1008,25 @@ __global__ __launch_bounds__(64) void XcopyPieceDoneKernel(uint64_t list, uint32
     MarkDone(DoneMark{Buffer<uint64_t>(word), Buffer<uint32_t>(counter), value, count}, at);
 }
 
-// Pieces of kWindowUnits units in read and write windows, as XcopyWindowKernel walks chunks; every piece of the list begins on a
-// cache line in source and destination.  A wave requests its next piece's descriptor before it copies the current piece.
+// Pieces of kWindowUnits units in read and write windows, as XcopyWindowKernel walks chunks, each copied as XcopyPieceHeldKernel copies it; every
+// piece of the list begins on a cache line in source and destination.  A wave fetches a descriptor across the link when it has issued its stores and has half a period for it.
 // Bound: HBM, whose rows a random place opens for 256 bytes a channel, so the rate that holds is lower than that of long segments.
-// Back to back, us without windows / in windows cut for 6.0 / 6.4 / 6.8 TB/s: 4096 pages of 32 KiB gathered 46.9 / 47.1 / 44.7 / 48.1,
-// scattered 50.6 / 47.5 / 48.4 / 51.0, 12 000 scattered 146 / 137 / 148 / 152, 4096 of 64 KiB scattered 97.0 / 91.9 / 86.9 / 88.8,
-// K and V blocks of 128 and 16 KiB, 90 MB 35.7 / 32.8 / 36.4 / 37.0 and 144 MB 55.8 / 51.0 / 56.2 / 57.3, 1500 segments of 120 000 bytes
-// 70.2 / 63.6 / 68.8 / 71.7.  Pieces that are four fifths full gain nothing (8192 x 40 000 130 / 128 / 133 / 133), ragged ones at odd
-// addresses lose (4000 of up to 131 072 bytes 106 / 108 / 110 / 111).
+// Back to back, us, held launches or 4096 waves at the rates those held / 6144 waves at theirs (PieceWindowRate), the same in two processes each.  Gathered 4096 / 8000 / 16 384
+// pages of 32 KiB 45.7 / 43.5, 90.8 / 83.3, 183 / 170, 16 384 of 16 KiB 92.6 / 87.5, 4900 of 24 064 bytes 43.0 / 39.1, 12 000 of 64 KiB 254 / 240; scattered 2500 / 12 000 of 64 KiB
+// 55.0 / 52.7, 258 / 249, 16 384 of 32 KiB 187 / 186, of 16 KiB 94.1 / 94.4.  At random places on both sides 8000 of 50 000 bytes 160 / 148, 6000 of 73 728 174 / 154, 3500 of 81 920 100.1 /
+// 95.7, 6000 of 110 776 234 / 224, K and V blocks of 128 and 16 KiB, 144 MB, 51.0 / 48.7.
+// Beside eight elementwise kernels of another stream over 1 GiB, both together, 37 x 8000 pages of 32 KiB 6159 / 6231, beside products of matrices 3992 / 3750.
 // (A schedule that stretches when sampled waves fall behind it was tried: it overshoots, 20 to 50 % slower than none.)
-// What a lane past the end of its piece loads is the last unit: a load under a condition would leave the registers of the
-// loop's last round alive in the others and take more of them than sixteen waves per CU have.
-__global__ __launch_bounds__(64) void XcopyPieceWindowKernel(uint64_t list, uint32_t count, uint32_t period, uint32_t seq, uint32_t groups,
-                                                              uint32_t value, uint64_t started)
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kLongWavesPerSimd, kLongWavesPerSimd))) void XcopyPieceWindowKernel(
+    uint64_t list, uint32_t count, uint32_t period, uint32_t seq, uint32_t groups, uint32_t value, uint64_t started)
 {
     MarkStarted(started, value);
-    const Piece *const pieces = Buffer<const Piece>(list);
-    uint32_t at = PieceOf(blockIdx.x);
-    if (at >= count) {
-        return;
-    }
-    Piece next = pieces[at];
     const uint32_t half = period / 2;
     uint64_t slot = AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * half / groups;
-    for (;;) {
-        uint32_t tid = threadIdx.x;
-        asm volatile("" : "+v"(tid));       // offsets are computed in each round instead of held through all of them
-        const uint64_t srcWord = Uniform(next.src);
-        const uint64_t dstWord = Uniform(next.dst);
-        const bool more = count - at > groups;
-        next = pieces[more ? at + groups : at];
-        const uint64_t src = srcWord & kPieceAddress;
-        const uint64_t dst = dstWord & kPieceAddress;
-        const uint32_t length = PieceLength(srcWord, dstWord);
-        const uint32_t body = length / kUnitBytes;
-        u32x4 v[kWindowDepth];
+    for (uint32_t at = PieceOf(blockIdx.x); at < count; at += groups, slot += period) {
+        const Piece p = PieceAt(list, at);
         WaitForClock(slot);
-        if (body == kWindowUnits) {
-#pragma unroll
-            for (uint32_t j = 0; j < kWindowDepth; ++j) {
-                v[j] = LoadAligned(src + (j * 64 + tid) * kUnitBytes);
-            }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            WaitForClock(slot + half);
-#pragma unroll
-            for (uint32_t j = 0; j < kWindowDepth; ++j) {
-                StoreUnit<kStoreStream>(dst + (j * 64 + tid) * kUnitBytes, v[j]);
-            }
-        } else if (body != 0) {
-#pragma unroll
-            for (uint32_t j = 0; j < kWindowDepth; ++j) {
-                const uint32_t u = j * 64 + tid < body ? j * 64 + tid : body - 1;
-                v[j] = LoadAligned(src + u * kUnitBytes);
-            }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            WaitForClock(slot + half);
-#pragma unroll
-            for (uint32_t j = 0; j < kWindowDepth; ++j) {
-                if (j * 64 + tid < body) {
-                    StoreUnit<kStoreStream>(dst + (j * 64 + tid) * kUnitBytes, v[j]);
-                }
-            }
-        }
-        if (tid < length % kUnitBytes) {
-            const uint64_t off = body * kUnitBytes + tid;
-            CopyByte<kStoreStream>(src + off, dst + off);
-        }
-        if (!more) {
-            return;
-        }
-        at += groups;
-        slot += period;
+        CopyPieceHeld<kDeepUnits / 64>(p.src & kPieceAddress, p.dst & kPieceAddress, PieceLength(p.src, p.dst), slot, half, [] {});
     }
 }
 
@@ -2214,7 +2163,7 @@ int SubmitPieceList(const void *pieces, uint32_t count, uint64_t bytes, uint32_t
     }
     if (windowMBps != 0) {
         // whole groups of pieces, evenly over the rounds; the last group of the list may be short
-        const uint32_t grid = (WindowGrid(count, kWindowWaves) + kPieceGroup - 1) / kPieceGroup * kPieceGroup;
+        const uint32_t grid = (WindowGrid(count, kLongWaves) + kPieceGroup - 1) / kPieceGroup * kPieceGroup;
         const uint32_t period = WindowPeriodTicks(2 * bytes * grid / (count > grid ? count : grid), windowMBps);
         return period == 0 ? static_cast<int>(hipErrorInvalidValue)
                            : LaunchWithEvent(XcopyPieceWindowKernel, grid, 64, s, end, At(pieces), count, period, NextWindowSeq(), grid, value,

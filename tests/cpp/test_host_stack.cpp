@@ -2243,17 +2243,21 @@ static void TestWindowRatesOfLists()
     fake_rt_skip_copies(1);
     constexpr uint64_t k = 1024;
     const uint32_t rate = XcopyTuning{}.windowMBps;
-    const uint32_t random = rate / 17 * 15, grid = rate / 17 * 16, ordered = rate / 34 * 32, orderedGrid = rate / 34 * 33;
+    const uint32_t part = rate / 68;
+    const uint32_t random = part * 60, partRandom = part * 59, uneven = part * 58, full = part * 63, grid = part * 66, brief = part * 64, ordered = part * 66, orderedGrid = part * 68;
     struct Form { uint32_t n; uint64_t bytes, step; bool inOrder; uint32_t rate; };
     const Form forms[] = {
         {4096, 64 * k, 64 * k, false, grid}, {2400, 128 * k, 192 * k, false, grid}, {9000, 64 * k, 64 * k, false, grid},
-        {4600, 64 * k, 68 * k, false, random}, {4600, 64 * k, 64 * k + 256, false, random},        // off the grid by pages and by lines
-        {2708, 110776, 110848, false, random}, {2708, 110720, 110720, false, random}, {4308, 68 * k, 128 * k, false, random}, {3662, 80 * k, 80 * k, false, random},
-        {4096, 64 * k, 64 * k, true, orderedGrid}, {8000, 64 * k, 64 * k, true, ordered},
-        {16384, 16 * k, 16 * k, true, random}, {8193, 32 * k, 32 * k, true, random},                  // short ones in order: from 16 384 pieces on
-        {7169, 32 * k, 32 * k, true, 0}, {7169, 16 * k, 16 * k, true, 0}, {7169, 16 * k, 16 * k, false, random},
+        {4600, 64 * k, 68 * k, false, full}, {4600, 64 * k, 64 * k + 256, false, full},        // off the grid by pages and by lines
+        {2708, 110776, 110848, false, full}, {2708, 110720, 110720, false, full}, {4308, 68 * k, 128 * k, false, partRandom}, {3662, 80 * k, 80 * k, false, full},
+        {4096, 64 * k, 64 * k, true, orderedGrid}, {8000, 64 * k, 64 * k, true, orderedGrid},
+        {16384, 16 * k, 16 * k, true, brief}, {8193, 32 * k, 32 * k, true, ordered},
+        {7169, 32 * k, 32 * k, true, ordered}, {7169, 16 * k, 16 * k, true, brief}, {7169, 16 * k, 16 * k, false, random},
         {3584, 32 * k, 32 * k, false, 0}, {3585, 32 * k, 32 * k, false, random}, {1000, 110720, 110720, false, 0},    // what is held takes no windows
         {4308, 68 * k, 68 * k, true, ordered}, {3662, 80 * k, 80 * k, true, ordered},
+        {8000, 24064, 24064, true, ordered}, {8000, 23936, 23936, true, brief}, {8000, 24064, 24064, false, uneven}, {8000, 23936, 23936, false, 0},   // part-filled pieces
+        {6000, 24064, 24064, false, 0}, {6000, 50048, 50048, false, partRandom}, {6000, 40192, 40192, true, ordered}, {8000, 24576, 24576, false, partRandom},
+        {6000, 64 * k, 64 * k + 16, false, 0}, {6000, 50000, 50000, true, 0},     // off the lines
     };
     for (const Form &f : forms) {
         (void)fake_rt_last_window();
@@ -2337,8 +2341,8 @@ static void TestHeldLaunches()
     lists.push_back({"ragged", some(2700, 1, 90000), 1, 2});
     lists.push_back({"ragged, three", some(3000, 60000, 120000), 1, 3});
     lists.push_back({"ragged, four", some(4200, 60000, 120000), 16, 4});
-    lists.push_back({"equal, as many as two launches hold", std::vector<uint64_t>(3584, 50000), 256, 2});
-    lists.push_back({"equal, one too many", std::vector<uint64_t>(3585, 50000), 256, 3});
+    lists.push_back({"equal, as many as two launches hold", std::vector<uint64_t>(3584, 50000), 16, 2});
+    lists.push_back({"equal, one too many", std::vector<uint64_t>(3585, 50000), 16, 3});
     lists.push_back({"short ones first", then(some(3000, 3000, 4000), some(4000, 55000, 63000)), 16, 3});
     lists.push_back({"short ones last", then(some(4000, 55000, 63000), some(3000, 3000, 4000)), 16, 3});
     lists.push_back({"empty ones last", then(some(3000, 60000, 120000), std::vector<uint64_t>(2000, 0)), 16, 3});

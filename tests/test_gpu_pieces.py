@@ -227,3 +227,26 @@ def test_slots_whose_launches_do_not_start_for_a_while(gpu, order):
         gpu.mfrt_stream_destroy(other)
         for buffer in (a, b, long_from, long_to):
             buffer.free()
+
+
+# Lists in windows of pieces that are not full, and as many as a round of 6144 waves has, a group of 64 more or less.
+@pytest.mark.parametrize("count, size", [(3072, 32896), (7232, 16400), (12288, 16384), (12287, 16384), (12352, 16384), (8000, 24576), (8000, 24001), (4000, 40000),
+                                         (3700, 49153), (2400, 50048), (2200, 65535), (1500, 100352)])
+@pytest.mark.parametrize("where", ["gathered", "scattered"])
+def test_lists_of_part_filled_pieces_in_windows(gpu, count, size, where):
+    torch = pytest.importorskip("torch")
+    step = (size + 127) // 128 * 128
+    rng = np.random.default_rng(count)
+    at = rng.permutation(count).astype(np.int64) * step
+    place = np.arange(count, dtype=np.int64) * step
+    if where == "scattered":
+        at, place = place, at
+    source = torch.randint(-2**63, 2**63 - 1, (count * step // 8,), dtype=torch.int64, device="cuda").view(torch.uint8)
+    target = torch.full_like(source, 0x5A)
+    torch.cuda.synchronize()
+    for _ in range(2):
+        gpu_util.xcopy(gpu, (source.data_ptr() + at).astype(np.uint64), (target.data_ptr() + place).astype(np.uint64),
+                       np.full(count, size, dtype=np.uint64), native.ROUTE_HBM)
+    got = target.view(count, step)[torch.from_numpy(place // step).cuda()]
+    assert torch.equal(got[:, :size], source.view(count, step)[torch.from_numpy(at // step).cuda()][:, :size])
+    assert bool((got[:, size:] == 0x5A).all())
