@@ -342,14 +342,14 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyInlineKernel(const InlineP
 constexpr uint32_t kWindowDepth = 16;                       // 128-bit loads per lane and round
 constexpr uint32_t kWindowUnits = 64 * kWindowDepth;        // 16 KiB chunks, one wave each
 constexpr uint32_t kWindowWaves = 4096;                     // 16 per CU
-// XcopyWindowKernel's and XcopyPieceWindowKernel's, 24 per CU.  A period of half as many waves again is as much longer, so a wave whose loads land late has more of it to
+// XcopyWindowKernel's, XcopyPieceWindowKernel's and XcopySampledKernel's, 24 per CU.  A period of half as many waves again is as much longer, so a wave whose loads land late has more of it to
 // catch up in, and HBM turns round less often.  4096 / 5120 / 6144 waves, the mean of sixteen launches in pairs, us: 128 x 9 MB at 7.1 TB/s 359 / 355 / 346, at
 // 7.4 377 / 357 / 351; 128 x 2.4 MB at 7.4 102 / 93 / 90; 170 MiB at 7.6 56.4 / 55.8 / 52.2; shifted, 512 MiB at 7.1 164 / 168 / 161.  7168 waves are as many as there
 // are registers for the data of, and spill what else they need (170 MiB at 7.6 52.5).  The read and the write part as long as each other: 47 and 53 % of the period for reads are
 // no better; nor are parts that issue in 95 or 90 % of their time and leave the rest for stragglers (128 x 9 MB at 7.2 346, 379, at 100 % 348).
 constexpr uint32_t kLongWavesPerSimd = 6;
 constexpr uint32_t kLongWaves = 6144;
-static_assert(kLongWaves % kPieceGroup == 0, "a round of pieces is whole groups");
+static_assert(kLongWaves <= kHeldMaxPieces && kLongWaves % kPieceGroup == 0, "a round of pieces is whole groups, and a table of more than kPlannedSegments has a workgroup for each wave");
 
 // Chunk c of a segment; with onLines one of LineChunks(), as a segment of its own.
 struct SegChunk {
@@ -1193,6 +1193,9 @@ __device__ __forceinline__ void CopyWholeWindowed(const uint64_t (&src)[kParts],
 // 20.8 / 19.6, 16 384 54.5 / 47.7, 59.9 / 49.9; of 16 KiB 33.4 / 31.5, 35.8 / 33.7, 94.7 / 89.3, 106 / 94.5; of 32 KiB 60.9 / 56.8, 66.7 / 60.8, 187 / 175, 208 / 191;
 // 8000 of 64 KiB 188 / 169, 204 / 176; 5000 of 128 KiB 242 / 211, 258 / 219; of 4 KiB 8000 19.4 / 16.5, 20.0 / 17.0, 16 384 35.7 / 27.3, 37.9 / 28.1, but 4100 13.5 / 13.1,
 // 12.0 / 12.8, hence kSampledQuarters.  Every other table pays for its look at the rule only: 16 384 segments of 2 to 14 KB 56.4 / 56.4, at odd addresses 64.3 / 64.8.
+// With kLongWaves instead of kWindowWaves, and what is read or written in order or lies on the grid at 6.7 instead of 6.4 and 6.6 TB/s, gathered, scattered: 9000 of 16 KiB 51.9 / 51.2, 58.6 / 54.3;
+// 4200 of 32 KiB 49.0 / 48.3, 54.7 / 50.8, 9000 97.5 / 96.3, 113.5 / 101.9, 16 384 174 / 174, 202 / 193 to 199; 9000 of 64 KiB 190 / 186, 196 / 188, 16 384 347 / 338, 354 / 341
+// (at 6.8 16 384 of 32 KiB gathered 168 to 185).
 // That asks for six waves per SIMD, as the kernel without windows has (with five, and 64 segments looked at by every wave, 64.3 / 85.8).  Not taken: the
 // stores of up to 5120 waves held instead (8000 of 8 KiB 28.2 / 29.5: four workgroups a segment start, most of them only to leave, and take the place of
 // those that load); pages that are no whole chunks, whose code would cost the registers.
@@ -1216,7 +1219,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSampledWave
         CopyDirect<true, kStoreStream>(triples, nseg, kXcopyThreads, rest, capacity, seen.parts);
         return;
     }
-    const uint32_t rounds = (items + kWindowWaves - 1) / kWindowWaves;
+    const uint32_t rounds = (items + kLongWaves - 1) / kLongWaves;
     const uint32_t waves = (items + rounds - 1) / rounds;
     uint32_t item = blockIdx.x;
     if (item >= waves) {
@@ -2024,7 +2027,8 @@ int LaunchDirect(const uint64_t *triples, uint32_t nseg, uint32_t units, uint32_
     return static_cast<int>(err);
 }
 
-TablePace PaceOf(uint32_t holdNanos, uint32_t holdMoreNanos, uint32_t windowMBps)
+// longWaves: for kLongWaves of them instead of kWindowWaves (XcopySampledKernel has the figures).
+TablePace PaceOf(uint32_t holdNanos, uint32_t holdMoreNanos, uint32_t windowMBps, bool longWaves)
 {
     const uint32_t sooner = holdMoreNanos != 0 ? kTableHoldNanos - kTableEqualNanos : 0;     // a wait set by hand is what it is
     const uint32_t equalNanos = holdNanos > sooner ? holdNanos - sooner : holdNanos;
@@ -2035,8 +2039,8 @@ TablePace PaceOf(uint32_t holdNanos, uint32_t holdMoreNanos, uint32_t windowMBps
                      TicksOf(holdMoreNanos != 0 ? holdMoreNanos + kTableEqualMoreNanos - kTableHoldMoreNanos : 0, khz),
                      WindowPeriodTicksAt(2ull << 26, windowMBps, khz),
                      WindowPeriodTicksAt(2ull << 26, windowMBps / 20 * 21, khz),
-                     WindowPeriodTicksAt(2ull << 26, windowMBps / 15 * 16, khz),
-                     WindowPeriodTicksAt(2ull << 26, windowMBps / 20 * 22, khz),
+                     WindowPeriodTicksAt(2ull << 26, longWaves ? windowMBps / 60 * 67 : windowMBps / 15 * 16, khz),
+                     WindowPeriodTicksAt(2ull << 26, longWaves ? windowMBps / 60 * 67 : windowMBps / 20 * 22, khz),
                      NextWindowSeq()};
 }
 
@@ -2262,9 +2266,9 @@ extern "C" int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t uni
         return -1;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // (grid: the waves that are held or paced have to be there)
+    // (grid: the waves that are paced have to be there)
     const bool sampled = windowMBps != 0 && route == MFRT_ROUTE_HBM && nseg > kPlannedSegments && grid >= kHeldMaxPieces;
-    const TablePace pace = sampled ? PaceOf(holdNanos, holdMoreNanos, windowMBps) : TablePace{};
+    const TablePace pace = sampled ? PaceOf(holdNanos, holdMoreNanos, windowMBps, true) : TablePace{};
     const int err = WithPolicy(PolicyOf(route), [&](auto ntLoad, auto store) {
         return LaunchDirect<decltype(ntLoad)::value, decltype(store)::value>(static_cast<const uint64_t *>(triples), nseg, units, grid, restGrid,
                                                                              LanesFor(units, route), static_cast<RestList *>(rest), capacity, s,
@@ -2281,7 +2285,7 @@ extern "C" int mfk_xcopy_planned(const void *triples, uint32_t nseg, uint32_t ho
         return -1;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const TablePace pace = PaceOf(holdNanos, holdMoreNanos, windowMBps);
+    const TablePace pace = PaceOf(holdNanos, holdMoreNanos, windowMBps, false);
     const int err = nseg <= 64 * kPlannedShortRun
                         ? Launch(XcopyPlannedKernel<1, kPlannedShortRun>, kWindowWaves, 64, PlannedLds(1, nseg), s, At(triples), nseg, pace)
                         : Launch(XcopyPlannedKernel<kPlannedWaves, kPlannedRun>, kWindowWaves / kPlannedWaves, 64 * kPlannedWaves,

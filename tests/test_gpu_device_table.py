@@ -235,3 +235,10 @@ def test_longer_tables_by_what_their_first_segments_are(gpu, count, size, odd, l
         assert gpu.mfrt_device_sync() == 0
         assert gpu.mf_xcopy_launch_count() - counted == launches
         assert torch.equal(target, expect)
+
+
+# As many chunks as a round of its 6144 waves, one more or less, two rounds of them.
+@pytest.mark.parametrize("count,size", [(6143, 16384), (6144, 16384), (6145, 16384), (12288, 16384), (12289, 16384), (12287, 8192), (12289, 8192), (6144, 32768)])
+@pytest.mark.parametrize("odd", [False, True])
+def test_longer_tables_where_a_round_of_waves_ends(gpu, count, size, odd):
+    test_longer_tables_by_what_their_first_segments_are(gpu, count, size, odd, 2)
