@@ -1766,12 +1766,12 @@ BatchStats StatsOf(const uint64_t *src, const uint64_t *dst, const uint64_t *len
     return st;
 }
 
-bool WrittenInOrder(const uint64_t *dst, const uint64_t *len, uint32_t n)
+bool InOrder(const uint64_t *at, const uint64_t *len, uint32_t n)
 {
     const uint32_t seen = n < 256 ? n : 256;
     uint32_t following = 0;
     for (uint32_t i = 1; i < seen; ++i) {
-        following += dst[i - 1] + len[i - 1] == dst[i] ? 1 : 0;
+        following += at[i - 1] + len[i - 1] == at[i] ? 1 : 0;
     }
     return following >= seen / 2;
 }
@@ -1848,13 +1848,18 @@ uint32_t XcopyEngine::PieceUnits(const BatchStats &stats, uint32_t n, bool unord
 // 144.6 / 158.6 from 5.6 on, at 6.0 158 in another process, 8000 of 24 576 at 5.8 / 5.9 / 6.0 71.7 / 70.9 / 77.8, 3800 of 28 000 39.4 / 39.5 / 41.2); below, of one length, 5.8 from three held
 // launches' worth on (8000 of 24 000 73.0 / 70.7 / 70.9 / 77.1 from 5.6 on, 6000 of 33 333 75.8 / 74.0 / 79.7 / 81.8; in two held launches 2500 of 33 333 31.8, so 32.1; of 20 000, 61 % full, none is better
 // than none).
+// Short ones, from 88 % on, that are read one behind the other are read faster than they are written at random places, and hold 6.2 with a read part of 30 / 64 of the period (parts of 28 / 29 / 30, each at 6.1 / 6.2 / 6.3, one half at
+// 6.0: 6000 of 32 KiB scattered 67.6 / 66.7 / 66.1, 67.6 / 66.6 / 65.7, 67.6 / 66.6 / 65.7, 69.9; 9889 111 / 112 / 119, 111 / 109 / 114, 111 / 109 / 109, 112.7; 16 384 184 / 186 / 199, 183 / 182 / 192,
+// - / 181 / 182, 186; of 16 KiB 92.0 / 92.6 / 97.5, 91.9 / 91.1 / 93.0, - / 90.9 / 90.8, 94.0; at random places on
+// both sides 3700 / 4500 / 8000 of 32 KiB 44.3 / 55.0 / 94.2 with even parts at 6.0, so 47.9 / 57.2 / 96.6).  Uneven parts do nothing for the others.
 // At addresses off the lines held launches are as good or nearly (ragged ones of up to 131 072 bytes 262 MB 102.1, at 5.5 / 5.6 / 5.7 / 5.8 101.9 / 100.5 / 99.0 / 99.9; of up to
 // 101 706 169 MB 65.9, 66.7 / 66.1 / 66.4 / 67.4; of up to 60 000 240 MB 100.8, 104).
-uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t count, uint32_t units,
-                                      bool unordered) const
+uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t count, uint32_t units,
+                                      bool unordered, uint32_t &reading) const
 {
     constexpr uint64_t kOrderedSteadyBytes = 24000;
     constexpr uint64_t kUnevenBytes = 24000;
+    constexpr uint32_t kShortReading = 30;
     if (unordered || units != kDeepUnits || (stats.addressBits & (kWindowAlignBytes - 1)) != 0 ||
         !WindowsApply(stats.total, MFRT_ROUTE_HBM, kPieceWindowMinBytes)) {
         return 0;
@@ -1865,7 +1870,7 @@ uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *d
     const bool equal = stats.total == stats.longest * n;
     const bool onGrid = equal && ((stats.addressBits | stats.lengthBits) & (kWindowLongBlockBytes - 1)) == 0;
     const bool longBlocks = mean >= kWindowLongBlockBytes;
-    if (WrittenInOrder(dst, len, n)) {
+    if (InOrder(dst, len, n)) {
         return onGrid ? rate * 68 : equal && mean >= kOrderedSteadyBytes ? rate * 66 : equal || (longBlocks && percent >= 85) ? rate * 64 : 0;
     }
     if (onGrid) {
@@ -1873,6 +1878,10 @@ uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *d
     }
     if (longBlocks && percent >= 95) {
         return rate * 63;
+    }
+    if (!longBlocks && percent >= 88 && InOrder(src, len, n)) {
+        reading = kShortReading;
+        return rate * 62;
     }
     if (percent >= 85 || (equal && percent >= 75)) {
         return rate * (percent >= 88 ? 60 : 59);
@@ -1890,7 +1899,7 @@ uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *d
 // 400 000 on 0.98 to 1.06; written in order, where the one launch finds the rows of HBM open, in two launches of nearly full pieces 0.94 to 1.00, of others 1.00
 // to 1.04, in three or four 1.00 to 1.07, at odd addresses from 400 000 bytes on 1.00 to 1.08.
 // Every launch has a slot of its own, so half of them are left for other calls.
-uint32_t XcopyEngine::HeldLaunches(const BatchStats &stats, const uint64_t *dst, const uint64_t *len, uint32_t n, bool unordered) const
+uint32_t XcopyEngine::HeldLaunches(const BatchStats &stats, const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, bool unordered) const
 {
     constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kDeepUnits) * kUnitBytes;
     constexpr uint64_t kHeldOddBytes = 24 * kDeepBytes;
@@ -1923,10 +1932,11 @@ uint32_t XcopyEngine::HeldLaunches(const BatchStats &stats, const uint64_t *dst,
         }
         parts = most <= kHeldMaxPieces ? fewest : parts;
     }
+    uint32_t reading = 0;
     const bool odd = (stats.addressBits & (kUnitBytes - 1)) != 0;
-    const bool refused = WrittenInOrder(dst, len, n) ? parts > 2 || stats.total < stats.deepPieces * kDeepBytes / 100 * 92
+    const bool refused = InOrder(dst, len, n) ? parts > 2 || stats.total < stats.deepPieces * kDeepBytes / 100 * 92
                                                       : parts > 2 && odd && mean < 3 * kDeepBytes;
-    if (parts > kSlots / 2 || refused || (odd && mean >= kHeldOddBytes) || PieceWindowRate(stats, dst, len, n, pieces, kDeepUnits, false) != 0 ||
+    if (parts > kSlots / 2 || refused || (odd && mean >= kHeldOddBytes) || PieceWindowRate(stats, src, dst, len, n, pieces, kDeepUnits, false, reading) != 0 ||
         HoldForPieces(stats, n, pieces / parts, kDeepUnits, false) == 0) {
         return 1;
     }
@@ -2251,7 +2261,7 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         }
         units = ChooseUnits(total, cu, route, tuning_);
         if (route == MFRT_ROUTE_HBM) {
-            const uint32_t parts = HeldLaunches(stats, dst, len, n, unordered);
+            const uint32_t parts = HeldLaunches(stats, src, dst, len, n, unordered);
             if (parts > 1) {
                 return SubmitHeld(src, dst, len, n, stats, parts, stream, mask, maskValue);
             }
@@ -2420,14 +2430,15 @@ int XcopyEngine::SubmitPieces(const uint64_t *src, const uint64_t *dst, const ui
         return mfk_xcopy_inline(&empty, MFRT_ROUTE_HBM, 1, mask, maskValue, stream, 0, 0) == 0 ? BM_OK : BM_ERROR;
     }
     const uint32_t hold = HoldForPieces(stats, n, count, units, unordered);
-    const uint32_t rate = hold != 0 ? 0 : PieceWindowRate(stats, dst, len, n, count, units, unordered);
+    uint32_t reading = 0;
+    const uint32_t rate = hold != 0 ? 0 : PieceWindowRate(stats, src, dst, len, n, count, units, unordered, reading);
     const bool own = stream == lease.stream;
     // Reporting costs the GPU the atomics of every wave (200 x 128 KiB 9.9 us with an event, 10.4 so, 2000 x 40 000 34.0 / 37.4), the
     // event costs the host: for batches that the GPU copies in less time than the host needs for the next (4 us and some ns a segment).
     const bool reports = !own && rate == 0 && total <= kReportBytes + kReportSegmentBytes * n;
     if (mask == nullptr && (own ? HasDoneWord(lease) : reports && HasReadMarks(lease))) {
         const uint32_t seq = own ? lease.startSeq + 1 : slot->readSeq + 1;
-        const int failed = mfk_xcopy_pieces_reported(pieces, count, total, units, hold, rate, own ? StartedWord(lease) : ReadWord(lease, *slot), seq,
+        const int failed = mfk_xcopy_pieces_reported(pieces, count, total, units, hold, rate, reading, own ? StartedWord(lease) : ReadWord(lease, *slot), seq,
                                                      own ? nullptr : ReadCounter(lease, *slot), stream);
         if (failed != 0) {
             (void)MarkQueued(lease, slot, stream, true);
@@ -2441,7 +2452,7 @@ int XcopyEngine::SubmitPieces(const uint64_t *src, const uint64_t *dst, const ui
         return BM_OK;
     }
     void *event = EventOfLaunch(lease, *slot, stream);
-    const int err = rate != 0 ? mfk_xcopy_pieces_windowed(pieces, count, total, rate, mask, maskValue, stream, event)
+    const int err = rate != 0 ? mfk_xcopy_pieces_windowed(pieces, count, total, rate, reading, mask, maskValue, stream, event)
                               : mfk_xcopy_pieces(pieces, count, total, units, mask, maskValue, stream, hold, event);
     if (err != 0) {
         (void)MarkQueued(lease, slot, stream, true);   // the launch may have gone out with only the word behind it failing

@@ -52,7 +52,7 @@ struct BatchStats {
 };
 BatchStats StatsOf(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n);
 // Whether most of the first segments of a batch are written one behind the other.
-bool WrittenInOrder(const uint64_t *dst, const uint64_t *len, uint32_t n);
+bool InOrder(const uint64_t *at, const uint64_t *len, uint32_t n);
 
 // A batch of this much and more is cut into pieces of 8 and 16 KiB.  Shorter ones keep 4 KiB, which more CUs share: 150 pages of 8 KiB
 // 2.8 us, 4.0 in waves of 16 KiB; 200 pages of 32 KiB 4.4 / 4.6.  From there on the longer pieces are as fast and a quarter of the
@@ -227,13 +227,14 @@ private:
 
     uint32_t HoldFor(const InlinePlan &plan, uint32_t grid, int route, bool unordered) const;
     uint32_t HoldForPieces(const BatchStats &stats, uint32_t n, uint32_t count, uint32_t units, bool unordered) const;
-    uint32_t HeldLaunches(const BatchStats &stats, const uint64_t *dst, const uint64_t *len, uint32_t n, bool unordered) const;
+    uint32_t HeldLaunches(const BatchStats &stats, const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, bool unordered) const;
     int SubmitHeld(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, const BatchStats &stats, uint32_t parts, void *stream,
                    void *mask, uint32_t maskValue);
     uint32_t PieceUnits(const BatchStats &stats, uint32_t n, bool unordered) const;
-    // Rate of the windows a list of `count` pieces of `units` units is copied in, 0: in none.
-    uint32_t PieceWindowRate(const BatchStats &stats, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t count, uint32_t units,
-                             bool unordered) const;
+    // Rate of the windows a list of `count` pieces of `units` units is copied in, 0: in none.  reading: 64ths of a period that are its read
+    // part, unchanged for half of it.
+    uint32_t PieceWindowRate(const BatchStats &stats, const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t count,
+                             uint32_t units, bool unordered, uint32_t &reading) const;
     // How a launch of a device table paces itself: the waits of its waves and the rate of its windows.
     void TablePaceFor(uint32_t &holdNanos, uint32_t &holdMoreNanos, uint32_t &windowMBps) const;
     // Whether a batch of `bytes` in n segments is planned in chunks of kDeepUnits units, to hold the stores of 16 KiB per wave.

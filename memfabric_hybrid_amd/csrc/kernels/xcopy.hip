@@ -1013,20 +1013,21 @@ __global__ __launch_bounds__(64) void XcopyPieceDoneKernel(uint64_t list, uint32
 // Bound: HBM, whose rows a random place opens for 256 bytes a channel, so the rate that holds is lower than that of long segments.
 // Back to back, us, held launches or 4096 waves at the rates those held / 6144 waves at theirs (PieceWindowRate), the same in two processes each.  Gathered 4096 / 8000 / 16 384
 // pages of 32 KiB 45.7 / 43.5, 90.8 / 83.3, 183 / 170, 16 384 of 16 KiB 92.6 / 87.5, 4900 of 24 064 bytes 43.0 / 39.1, 12 000 of 64 KiB 254 / 240; scattered 2500 / 12 000 of 64 KiB
-// 55.0 / 52.7, 258 / 249, 16 384 of 32 KiB 187 / 186, of 16 KiB 94.1 / 94.4.  At random places on both sides 8000 of 50 000 bytes 160 / 148, 6000 of 73 728 174 / 154, 3500 of 81 920 100.1 /
+// 55.0 / 52.7, 258 / 249, and with a shorter read part (PieceWindowRate) 4096 / 6000 / 16 384 of 32 KiB 47.8 / 46.3, 69.8 / 67.1, 189 / 186, 9000 / 16 384 of 16 KiB 52.6 / 51.1, 95.5 / 92.4.  At random places on both sides 8000 of 50 000 bytes 160 / 148, 6000 of 73 728 174 / 154, 3500 of 81 920 100.1 /
 // 95.7, 6000 of 110 776 234 / 224, K and V blocks of 128 and 16 KiB, 144 MB, 51.0 / 48.7.
 // Beside eight elementwise kernels of another stream over 1 GiB, both together, 37 x 8000 pages of 32 KiB 6159 / 6231, beside products of matrices 3992 / 3750.
 // (A schedule that stretches when sampled waves fall behind it was tried: it overshoots, 20 to 50 % slower than none.)
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kLongWavesPerSimd, kLongWavesPerSimd))) void XcopyPieceWindowKernel(
-    uint64_t list, uint32_t count, uint32_t period, uint32_t seq, uint32_t groups, uint32_t value, uint64_t started)
+    uint64_t list, uint32_t count, uint32_t period, uint32_t reading, uint32_t seq, uint32_t groups, uint32_t value, uint64_t started)
 {
     MarkStarted(started, value);
-    const uint32_t half = period / 2;
-    uint64_t slot = AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * half / groups;
+    uint64_t slot = AgreedStart(seq) + static_cast<uint64_t>(blockIdx.x) * reading / groups;
+    const uint32_t hold = reading + static_cast<uint32_t>(static_cast<uint64_t>(blockIdx.x) * (period - reading) / groups) -
+                          static_cast<uint32_t>(static_cast<uint64_t>(blockIdx.x) * reading / groups);
     for (uint32_t at = PieceOf(blockIdx.x); at < count; at += groups, slot += period) {
         const Piece p = PieceAt(list, at);
         WaitForClock(slot);
-        CopyPieceHeld<kDeepUnits / 64>(p.src & kPieceAddress, p.dst & kPieceAddress, PieceLength(p.src, p.dst), slot, half, [] {});
+        CopyPieceHeld<kDeepUnits / 64>(p.src & kPieceAddress, p.dst & kPieceAddress, PieceLength(p.src, p.dst), slot, hold, [] {});
     }
 }
 
@@ -2158,8 +2159,8 @@ bool IsList(const void *pieces, uint32_t count)
     return pieces != nullptr && count != 0 && count <= kPieceMaxCount;
 }
 
-// In the form that `units` and the hold ask for, or in windows of windowMBps where that is not 0.
-int SubmitPieceList(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, uint32_t holdNanos, uint32_t windowMBps, hipStream_t s,
+// In the form that `units` and the hold ask for, or in windows of windowMBps where that is not 0, whose read part is `reading` 64ths of a period (0: half of it).
+int SubmitPieceList(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, uint32_t holdNanos, uint32_t windowMBps, uint32_t reading, hipStream_t s,
                     hipEvent_t end, void *word, uint32_t value, void *counter)
 {
     if (!IsList(pieces, count) || (units != 256 && units != 512 && units != 1024)) {
@@ -2170,8 +2171,8 @@ int SubmitPieceList(const void *pieces, uint32_t count, uint64_t bytes, uint32_t
         const uint32_t grid = (WindowGrid(count, kLongWaves) + kPieceGroup - 1) / kPieceGroup * kPieceGroup;
         const uint32_t period = WindowPeriodTicks(2 * bytes * grid / (count > grid ? count : grid), windowMBps);
         return period == 0 ? static_cast<int>(hipErrorInvalidValue)
-                           : LaunchWithEvent(XcopyPieceWindowKernel, grid, 64, s, end, At(pieces), count, period, NextWindowSeq(), grid, value,
-                                             At(word));
+                           : LaunchWithEvent(XcopyPieceWindowKernel, grid, 64, s, end, At(pieces), count, period,
+                                             reading == 0 ? period / 2 : period / 64 * reading, NextWindowSeq(), grid, value, At(word));
     }
     const uint32_t ticks = HoldTicks(PieceHoldNanos(holdNanos, count, bytes, units));
     if (units == 256) {
@@ -2196,19 +2197,20 @@ extern "C" int mfk_xcopy_pieces(const void *pieces, uint32_t count, uint64_t byt
 {
     using namespace mf;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int err = SubmitPieceList(pieces, count, bytes, units, holdNanos, 0, s, static_cast<hipEvent_t>(event), nullptr, 0, nullptr);
+    const int err = SubmitPieceList(pieces, count, bytes, units, holdNanos, 0, 0, s, static_cast<hipEvent_t>(event), nullptr, 0, nullptr);
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
 // The same, in either form, with a word of pinned host memory that gets `value`: when what is in front of them in the stream has ended
 // or, with a counter (kDoneCounterBytes of device memory, 0; not in windows), when they have been read.
 extern "C" int mfk_xcopy_pieces_reported(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, uint32_t holdNanos,
-                                         uint32_t windowMBps, void *word, uint32_t value, void *counter, void *stream)
+                                         uint32_t windowMBps, uint32_t reading, void *word, uint32_t value, void *counter, void *stream)
 {
     if (word == nullptr || (counter != nullptr && windowMBps != 0)) {
         return -1;
     }
-    return mf::SubmitPieceList(pieces, count, bytes, units, holdNanos, windowMBps, static_cast<hipStream_t>(stream), nullptr, word, value, counter);
+    return mf::SubmitPieceList(pieces, count, bytes, units, holdNanos, windowMBps, reading, static_cast<hipStream_t>(stream), nullptr, word, value,
+                               counter);
 }
 
 // The same of 4 KiB and their bytes beside; the last of them stores `value` in `word`.  counter: kDoneCounterBytes of device memory.
@@ -2223,12 +2225,13 @@ extern "C" int mfk_xcopy_pieces_done(const void *pieces, uint32_t count, void *w
 }
 
 // The same pieces, of up to kWindowUnits units, in windows cut for windowMBps.
-extern "C" int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t windowMBps, void *mask, uint32_t maskValue,
-                                         void *stream, void *event)
+extern "C" int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t windowMBps, uint32_t reading, void *mask,
+                                         uint32_t maskValue, void *stream, void *event)
 {
     using namespace mf;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int err = windowMBps == 0 ? -1 : SubmitPieceList(pieces, count, bytes, kWindowUnits, 0, windowMBps, s, static_cast<hipEvent_t>(event), nullptr, 0, nullptr);
+    const int err = windowMBps == 0 ? -1 : SubmitPieceList(pieces, count, bytes, kWindowUnits, 0, windowMBps, reading, s, static_cast<hipEvent_t>(event),
+                                                            nullptr, 0, nullptr);
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
 
@@ -2336,7 +2339,7 @@ extern "C" int mfk_xcopy_prelaunch(void *stream)
                 (void)Launch(XcopyPieceKernel<128, 4, true>, 1, 128, 0, s, 0, 0u, 0u, 0u, 0, 0);
                 (void)Launch(XcopyPieceKernel<256, 4, false>, 1, 256, 0, s, 0, 0u, 0u, 0u, 0, 0);
                 (void)Launch(XcopyPieceDoneKernel, 1, 64, 0, s, 0, 0u, 0, 0, 0u);
-                (void)Launch(XcopyPieceWindowKernel, 1, 64, 0, s, 0, 0u, 64u, NextWindowSeq(), 1u, 0u, 0);
+                (void)Launch(XcopyPieceWindowKernel, 1, 64, 0, s, 0, 0u, 64u, 32u, NextWindowSeq(), 1u, 0u, 0);
                 (void)Launch(XcopyPlannedKernel<1, kPlannedShortRun>, 1, 64, 64, s, 0, 0u, TablePace{});
                 (void)Launch(XcopyPlannedKernel<kPlannedWaves, kPlannedRun>, 1, 64 * kPlannedWaves, 64, s, 0, 0u, TablePace{});
                 (void)Launch(XcopySampledKernel, 1, 64, 0, s, 0, 0u, 0, 0u, TablePace{});

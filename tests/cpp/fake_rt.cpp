@@ -25,6 +25,7 @@ std::map<uint64_t, std::pair<uint64_t, int>> g_allocs;  // base -> (size, kind)
 int g_device = -1;
 std::atomic<uint64_t> g_launches{0};   // launches may come from the engine's submit threads
 std::atomic<uint32_t> g_lastHold{0};
+uint32_t g_lastReading = 0;  // read part of the latest windowed list
 uint32_t g_lastWindow = 0;   // rate of the latest windowed launch, cleared by fake_rt_last_window()     // holdNanos of the latest inline launch
 std::atomic<uint64_t> g_chunksRun{0};
 bool g_skipCopies = false;       // launches count and check their plans but move nothing (tables of segments no test can back with memory)
@@ -169,6 +170,7 @@ void fake_rt_stream_state(int state) { g_streamState = state; }
 void fake_rt_fail_allocations(int on) { g_failAllocations = on != 0; }
 uint64_t fake_rt_launches(void) { return g_launches; }
 uint32_t fake_rt_last_hold(void) { return g_lastHold; }
+uint32_t fake_rt_last_reading(void) { return g_lastReading; }
 uint32_t fake_rt_last_window(void) { const uint32_t w = g_lastWindow; g_lastWindow = 0; return w; }
 // The next n xcopy launches fail with a runtime error code instead of running.
 static int g_failLaunches = 0;
@@ -493,8 +495,8 @@ int mfk_xcopy_pieces_done(const void *pieces, uint32_t count, void *word, uint32
     return counter == nullptr || word == nullptr ? -1 : mfk_xcopy_pieces(pieces, count, 0, 256, word, value, stream, 0, nullptr);
 }
 // The same in windows: the rate is noted, and a piece that begins between cache lines fails the launch.
-int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t windowMBps, void *mask, uint32_t maskValue,
-                              void *stream, void *event)
+int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t windowMBps, uint32_t reading, void *mask,
+                              uint32_t maskValue, void *stream, void *event)
 {
     const mf::Piece *p = static_cast<const mf::Piece *>(pieces);
     for (uint32_t i = 0; p != nullptr && i < count; ++i) {
@@ -503,17 +505,18 @@ int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uint64_t bytes
         }
     }
     g_lastWindow = windowMBps;
+    g_lastReading = reading;
     return windowMBps == 0 ? -1 : mfk_xcopy_pieces(pieces, count, bytes, 1024, mask, maskValue, stream, 0, event);
 }
 
 // When this launch starts, those before it have ended; with a counter its own list has been read when it says so.
 int mfk_xcopy_pieces_reported(const void *pieces, uint32_t count, uint64_t bytes, uint32_t units, uint32_t holdNanos, uint32_t windowMBps,
-                              void *word, uint32_t value, void *counter, void *stream)
+                              uint32_t reading, void *word, uint32_t value, void *counter, void *stream)
 {
     if (counter == nullptr) {
         Retire(g_flightSeq);
     }
-    const int err = windowMBps != 0 ? mfk_xcopy_pieces_windowed(pieces, count, bytes, windowMBps, nullptr, 0, stream, nullptr)
+    const int err = windowMBps != 0 ? mfk_xcopy_pieces_windowed(pieces, count, bytes, windowMBps, reading, nullptr, 0, stream, nullptr)
                                     : mfk_xcopy_pieces(pieces, count, bytes, units, nullptr, 0, stream, holdNanos, nullptr);
     if (err == 0 && counter != nullptr && g_withholdReports) {
         std::lock_guard<std::mutex> guard(g_reportLock);

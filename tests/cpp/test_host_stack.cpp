@@ -34,6 +34,7 @@ extern "C" uint64_t fake_rt_signals(void);
 extern "C" uint64_t fake_rt_stream_syncs(void);
 extern "C" uint32_t fake_rt_last_window(void);
 extern "C" uint32_t fake_rt_last_line_window(void);
+extern "C" uint32_t fake_rt_last_reading(void);
 extern "C" void fake_rt_seal(void);
 extern "C" void fake_rt_fail_launches(int n);
 #include "../../include/mf_hip_copy_extend.h"
@@ -2244,7 +2245,7 @@ static void TestWindowRatesOfLists()
     constexpr uint64_t k = 1024;
     const uint32_t rate = XcopyTuning{}.windowMBps;
     const uint32_t part = rate / 68;
-    const uint32_t random = part * 60, partRandom = part * 59, uneven = part * 58, full = part * 63, grid = part * 66, brief = part * 64, ordered = part * 66, orderedGrid = part * 68;
+    const uint32_t random = part * 60, readInOrder = part * 62, partRandom = part * 59, uneven = part * 58, full = part * 63, grid = part * 66, brief = part * 64, ordered = part * 66, orderedGrid = part * 68;
     struct Form { uint32_t n; uint64_t bytes, step; bool inOrder; uint32_t rate; };
     const Form forms[] = {
         {4096, 64 * k, 64 * k, false, grid}, {2400, 128 * k, 192 * k, false, grid}, {9000, 64 * k, 64 * k, false, grid},
@@ -2264,10 +2265,16 @@ static void TestWindowRatesOfLists()
         CHECK(SubmitList(f.n, f.bytes, [&](uint32_t i) { return (i * 7919ull % f.n) * 2 * f.step; },
                          [&](uint32_t i) { return f.inOrder ? i * f.bytes : (i * 5077ull % f.n) * f.step; }) == BM_OK);
         const uint32_t got = fake_rt_last_window();
-        CHECK(got == f.rate);
+        CHECK(got == f.rate && (got == 0 || fake_rt_last_reading() == 0));
         if (got != f.rate) {
             std::printf("  %u segments of %llu bytes: rate %u, expected %u\n", f.n, static_cast<unsigned long long>(f.bytes), got, f.rate);
         }
+    }
+    for (const Form &f : {Form{4096, 32 * k, 32 * k, false, readInOrder}, Form{7169, 16 * k, 16 * k, false, readInOrder}, Form{4308, 68 * k, 128 * k, false, partRandom},
+                          Form{4000, 60 * k, 60 * k, false, readInOrder}, Form{4096, 64 * k, 64 * k, false, grid}}) {      // read one behind the other
+        (void)fake_rt_last_window();
+        CHECK(SubmitList(f.n, f.bytes, [&](uint32_t i) { return i * f.bytes; }, [&](uint32_t i) { return (i * 5077ull % f.n) * f.step; }) == BM_OK);
+        CHECK(fake_rt_last_window() == f.rate && fake_rt_last_reading() == (f.rate == readInOrder ? 30u : 0u));
     }
     for (const bool more : {false, true}) {      // part-filled pieces: held up to 7168 of them, in windows beyond
         std::mt19937 rng(3);
