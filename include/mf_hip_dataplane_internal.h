@@ -52,21 +52,20 @@ int32_t mf_xcopy_tune(uint32_t units, uint32_t wgPerCu, uint32_t wgPerCuLink);
  * 0 = never wait, otherwise that many ns for every launch the rule would pick, also of more than 128 segments.  Other launches, and
  * batches submitted with MF_COPY_UNORDERED_FLAG, never wait. */
 int32_t mf_xcopy_hold_stores(int32_t nanos);
-/* Read and write windows.  A batch of up to 128 segments and 128 MiB or more between HBM addresses is copied
- * by 4096 waves that alternate, all together and by the GPU's constant-rate clock, between a read half and a
- * write half of a period, so that HBM sees long bursts of one direction: 6.65-6.75 TB/s instead of 6.1-6.35 on
- * aligned copies of 512 MiB to 2 GiB, 6.05-6.3 instead of 5.75-5.85 when sources sit at odd addresses.  The
- * period is cut for a rate of HBM traffic (read + written) in MB/s, 6 800 000 by default; at 7 000 000 the waves
- * of a 2 GiB copy now and then no longer keep up, the windows dissolve and the copy runs at about the rate it
- * has without them; at 7 200 000 and above most launches do.  That holds for segments that start between
- * cache lines.  Segments whose sources and destinations all start on 128-byte lines are paced for
- * 7 100 000 (32 x 16 MiB back to back: 6.95 instead of 6.65 TB/s), those of 64 MiB and
- * more on average for 7 400 000, and a batch of 1 GiB and more of such long segments is cut into launches of
+/* Read and write windows.  A batch of up to 128 segments and more than 64 MiB (one segment: 112) between HBM addresses is copied
+ * by 6144 waves that alternate, all together and by the GPU's constant-rate clock, between a read half and a
+ * write half of a period, so that HBM sees long bursts of one direction: 6.9-7.2 TB/s instead of 6.1-6.35 on
+ * aligned copies of 512 MiB to 2 GiB, 6.6-6.75 instead of 5.75-5.85 when sources sit at odd addresses.  The
+ * period is cut for a rate of HBM traffic (read + written) in MB/s, 6 800 000 by default; beyond what a launch holds the
+ * waves no longer keep up, the windows dissolve and the copy runs at about the rate it
+ * has without them.  Segments whose sources and destinations agree modulo 16 are paced for
+ * 7 300 000, those on 128-byte lines of 64 MiB and
+ * more on average for 7 450 000, and a batch of 1 GiB and more of such long segments is cut into launches of
  * about 512 MiB, which hold their schedule more often than longer ones (1 GiB: 7.1-7.2 instead of 6.7 TB/s).
- * Segments whose source and destination differ modulo 16 take no windows.  Rectangles of 32 MiB and more whose rows hold
+ * Segments whose source and destination differ modulo 16 go at 35/34 of the default rate.  Rectangles of 32 MiB and more whose rows hold
  * windows go at 35/34 of the default rate where rows of whole lines lie against one another in the destination, pairs of
  * others at 69/68 and those with room between their rows at the rate itself, lists of more than 128 segments and device
- * tables at 15/17 to 33/34 of it.  The call sets all three rates, rectangles take the rate that is set, and the parts are of it; 0
+ * tables at 58/68 of it up to all of it.  The call sets all three rates, rectangles take the rate that is set, and the parts are of it; 0
  * switches the form off, MF_XCOPY_WINDOWS_OWN_CHOICE brings back the rates the library chose itself (what
  * hybm_init measured, else the defaults above).  While several threads submit on streams of their own the
  * form is not used. */
