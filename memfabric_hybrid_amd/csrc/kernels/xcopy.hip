@@ -1090,16 +1090,22 @@ __device__ __forceinline__ void ListRest(RestList *rest, uint32_t capacity, uint
 // part numbers that turn from segment to segment, pages 1 % slower; the triples of 64 items at a time, one per lane, so that
 // empty items cost no wait, more registers than eight waves per SIMD have, 10 to 60 % slower on short tables; two triples ahead
 // instead of one, 16 384 segments of 2 to 14 KB 4 % slower.
-// What the first kDirectSample segments of a table say of it.
+// What the first kDirectSample segments of a table say of it, and, kAcross, as many that lie across it.
 struct DirectSample {
-    uint32_t parts;             // chunks of the longest, up to kDirectMaxParts
-    bool equal;                 // they have one length, `length`,
+    uint32_t parts;             // chunks of the longest of the first, up to kDirectMaxParts
+    bool equal;                 // all have one length, `length`,
     uint64_t length;
-    bool aligned;               // and lie on units
+    bool aligned;               // and lie on units, sources and destinations
 };
+// Of 2^32, the golden section: its multiples lie evenly, and not with the period of a table of layers or of powers of two.
+constexpr uint32_t kAcrossStep = 0x9E3779B9u;
+template <bool kAcross>
 __device__ __forceinline__ DirectSample SampleOf(const uint64_t *__restrict__ triples, uint32_t nseg, uint32_t units)
 {
-    const uint32_t row = (threadIdx.x & 63u) < kDirectSample && (threadIdx.x & 63u) < nseg ? threadIdx.x & 63u : 0;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t across = kAcross ? __umulhi(nseg, (lane % kDirectSample + 1) * kAcrossStep) : 0;
+    const uint32_t row = lane < kDirectSample && lane < nseg ? lane : across;
+    const uint64_t src = triples[3ull * row];
     const uint64_t dst = triples[3ull * row + 1];
     const uint64_t len = triples[3ull * row + 2];
     const uint64_t sampled = SegmentChunks(dst, len, units);
@@ -1113,7 +1119,7 @@ __device__ __forceinline__ DirectSample SampleOf(const uint64_t *__restrict__ tr
     }
     parts |= least == parts ? 0u : 1u;      // odd in a ragged table: every XCD gets each of them in turn
     const uint64_t length = Uniform(len);
-    return DirectSample{parts, __ballot(len != length) == 0, length, __ballot(((dst | len) & (kUnitBytes - 1)) != 0) == 0};
+    return DirectSample{parts, __ballot(len != length) == 0, length, __ballot(((src | dst | len) & (kUnitBytes - 1)) != 0) == 0};
 }
 
 template <bool kNtLoad, int kStore>
@@ -1162,7 +1168,7 @@ template <bool kNtLoad, int kStore>
 __global__ __launch_bounds__(kXcopyThreads) void XcopyDirectKernel(const uint64_t *__restrict__ triples, uint32_t nseg, uint32_t units,
                                                                    RestList *__restrict__ rest, uint32_t capacity)
 {
-    CopyDirect<kNtLoad, kStore>(triples, nseg, units, rest, capacity, SampleOf(triples, nseg, units).parts);
+    CopyDirect<kNtLoad, kStore>(triples, nseg, units, rest, capacity, SampleOf<false>(triples, nseg, units).parts);
 }
 
 // kWindowUnits units on units, of kParts places, loads and stores by the clock.
@@ -1187,19 +1193,56 @@ __device__ __forceinline__ void CopyWholeWindowed(const uint64_t (&src)[kParts],
     }
 }
 
+// The same of four places on units, `bytes` of each, up to a quarter of kWindowUnits units.
+__device__ __forceinline__ void CopyPartWindowed(const uint64_t (&src)[4], const uint64_t (&dst)[4], const uint32_t (&bytes)[4], uint64_t loadAt,
+                                                 uint64_t storeAt)
+{
+    constexpr uint32_t kEach = kWindowDepth / 4;
+    const uint32_t lane = threadIdx.x * kUnitBytes;
+    u32x4 v[kWindowDepth];
+    WaitForClock(loadAt);
+#pragma unroll
+    for (uint32_t j = 0; j < kWindowDepth; ++j) {
+        const uint64_t at = src[j / kEach] + j % kEach * 64 * kUnitBytes;
+        if (lane + j % kEach * 64 * kUnitBytes < bytes[j / kEach] / kUnitBytes * kUnitBytes) {
+            v[j] = __builtin_nontemporal_load(reinterpret_cast<const MF_GLOBAL u32x4 *>(reinterpret_cast<const MF_GLOBAL uint8_t *>(at) + lane));
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+    WaitForClock(storeAt);
+#pragma unroll
+    for (uint32_t j = 0; j < kWindowDepth; ++j) {
+        const uint64_t at = dst[j / kEach] + j % kEach * 64 * kUnitBytes;
+        if (lane + j % kEach * 64 * kUnitBytes < bytes[j / kEach] / kUnitBytes * kUnitBytes) {
+            __builtin_nontemporal_store(v[j], reinterpret_cast<MF_GLOBAL u32x4 *>(reinterpret_cast<MF_GLOBAL uint8_t *>(at) + lane));
+        }
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q) {
+        if (threadIdx.x < bytes[q] % kUnitBytes) {
+            const uint64_t at = bytes[q] / kUnitBytes * kUnitBytes + threadIdx.x;
+            CopyByte<kStoreStream>(src[q] + at, dst[q] + at);
+        }
+    }
+}
+
 // The same for tables of more than kPlannedSegments between HBM addresses, one wave a workgroup.  Where the sampled segments are pages of one
 // length, whole chunks of 16 KiB or a half or a quarter of one, and lie on units, the first waves copy all of the table in windows as those of
-// XcopyPlannedKernel do, by the rates that it has measured, and the others leave.  A segment that is not what was seen is listed for the second launch, as
-// what long ones leave is.  HBM is the bound; without windows it sees reads and writes mixed.  us without / so, gathered, scattered: 5000 pages of 8 KiB 19.8 / 19.0,
-// 20.8 / 19.6, 16 384 54.5 / 47.7, 59.9 / 49.9; of 16 KiB 33.4 / 31.5, 35.8 / 33.7, 94.7 / 89.3, 106 / 94.5; of 32 KiB 60.9 / 56.8, 66.7 / 60.8, 187 / 175, 208 / 191;
-// 8000 of 64 KiB 188 / 169, 204 / 176; 5000 of 128 KiB 242 / 211, 258 / 219; of 4 KiB 8000 19.4 / 16.5, 20.0 / 17.0, 16 384 35.7 / 27.3, 37.9 / 28.1, but 4100 13.5 / 13.1,
-// 12.0 / 12.8, hence kSampledQuarters.  Every other table pays for its look at the rule only: 16 384 segments of 2 to 14 KB 56.4 / 56.4, at odd addresses 64.3 / 64.8.
-// With kLongWaves instead of kWindowWaves, and what is read or written in order or lies on the grid at 6.7 instead of 6.4 and 6.6 TB/s, gathered, scattered: 9000 of 16 KiB 51.9 / 51.2, 58.6 / 54.3;
-// 4200 of 32 KiB 49.0 / 48.3, 54.7 / 50.8, 9000 97.5 / 96.3, 113.5 / 101.9, 16 384 174 / 174, 202 / 193 to 199; 9000 of 64 KiB 190 / 186, 196 / 188, 16 384 347 / 338, 354 / 341
-// (at 6.8 16 384 of 32 KiB gathered 168 to 185).
-// That asks for six waves per SIMD, as the kernel without windows has (with five, and 64 segments looked at by every wave, 64.3 / 85.8).  Not taken: the
-// stores of up to 5120 waves held instead (8000 of 8 KiB 28.2 / 29.5: four workgroups a segment start, most of them only to leave, and take the place of
-// those that load); pages that are no whole chunks, whose code would cost the registers.
+// XcopyPlannedKernel do, by the rates that it has measured, and the others leave.  HBM is the bound; without windows it sees reads and writes mixed.
+// us without / so, gathered, scattered: 16 384 pages of 4 KiB 35.8 / 28.2, 37.0 / 28.7, of 8 KiB 54.2 / 48.1, 58.5 / 50.5, of 16 KiB 94.6 / 90.5,
+// 104.6 / 96.6; 9000 of 32 KiB 105.8 / 97.7, 115.1 / 104.4, of 64 KiB 214 / 191, 230 / 198; 5000 of 8 KiB 20.0 / 19.1, 20.3 / 19.8; but 4100 of 4 KiB
+// 13.5 / 13.1, 12.0 / 12.8, hence kSampledQuarters.
+// A page that is unlike those sampled takes its slot if it is shorter and lies on units, else it is listed for the second launch.  Listing costs 11 ns of
+// one word that all XCDs count on, so tables with many such pages are not for this: that is what the segments across the table are looked at for.  8192 pages of 16 KiB
+// with all sources off units, all listed / by CopyDirect() 204 / 52.8; 4096 of 8 KiB and then 4096 of 32 KiB 118 / 66.2, of 16 and 128 KiB 278 / 243; 16 384 of
+// 8 KiB with 5 % shorter 72.2 listed, 52.6 in their slots.  Not taken: CopyDirect()'s code for an unlike page where it is met (1 % of 16 384 of 16 KiB, 95.9, 131: it is
+// in no instruction cache by then), and a second, longer look by the waves that stay (ones of 6144 copy what is left 4 to 18 % slower than all would).
+// Every other table pays for the look, and for six waves per SIMD where XcopyDirectKernel has eight: 16 384 segments of 2 to 14 KB 57.5 / 58.9, 8000 of 64 KiB and 8000
+// of 100 bytes 195 / 204.  (With 64 segments looked at by every wave 64.3 / 85.8.)
+// With kLongWaves instead of kWindowWaves, and what is read or written in order or lies on the grid at 6.7 instead of 6.4 and 6.6 TB/s, gathered, scattered: 9000 of
+// 16 KiB 51.9 / 51.2, 58.6 / 54.3; 4200 of 32 KiB 49.0 / 48.3, 54.7 / 50.8, 9000 97.5 / 96.3, 113.5 / 101.9; 9000 of 64 KiB 190 / 186, 196 / 188.
+// Not taken: the stores of up to 5120 waves held instead (8000 of 8 KiB 28.2 / 29.5: four workgroups a segment start, most of them only to leave, and take the
+// place of those that load); pages that are no whole chunks, whose code would cost the registers.
 constexpr uint32_t kSampledWavesPerSimd = 6;
 constexpr uint32_t kSampledQuarters = 6144;             // segments of 4 KiB, at the least
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSampledWavesPerSimd, kSampledWavesPerSimd))) void XcopySampledKernel(
@@ -1211,15 +1254,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSampledWave
     const uint64_t *const triples = Buffer<const uint64_t>(table);
     RestList *const rest = Buffer<RestList>(list);
     constexpr uint32_t kDeepBytes = kWindowUnits * kUnitBytes;
-    const DirectSample seen = SampleOf(triples, nseg, kXcopyThreads);
+    const DirectSample seen = SampleOf<true>(triples, nseg, kXcopyThreads);
     const uint64_t len0 = seen.length;
     const uint32_t together = len0 == kDeepBytes / 2 ? 2 : len0 == kDeepBytes / 4 && nseg >= kSampledQuarters ? 4 : 1;    // segments a wave
     const uint32_t each = together != 1 ? 1 : len0 % kDeepBytes == 0 && len0 <= kSampledMostBytes ? static_cast<uint32_t>(len0) / kDeepBytes : 0;
-    const uint32_t items = (nseg + together - 1) / together * each;
     if (!seen.equal || !seen.aligned || each == 0) {
         CopyDirect<true, kStoreStream>(triples, nseg, kXcopyThreads, rest, capacity, seen.parts);
         return;
     }
+    auto asSeen = [&](const uint64_t (&row)[3]) { return row[2] == len0 && ((row[0] | row[1]) & (kUnitBytes - 1)) == 0; };
+    // by scalar loads: a table is not written while a launch reads it
+    const auto *const rows = reinterpret_cast<const __attribute__((address_space(4))) uint64_t *>(table);
+    const uint32_t items = (nseg + together - 1) / together * each;
     const uint32_t rounds = (items + kLongWaves - 1) / kLongWaves;
     const uint32_t waves = (items + rounds - 1) / rounds;
     uint32_t item = blockIdx.x;
@@ -1233,68 +1279,74 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSampledWave
     const uint64_t start = AgreedStart(pace.seq);
     uint64_t loadAt = start + static_cast<uint64_t>(item) * reading / waves;
     uint64_t storeAt = start + reading + static_cast<uint64_t>(item) * (period - reading) / waves;
-    // by scalar loads: a table is not written while a launch reads it
-    const auto *const rows = reinterpret_cast<const __attribute__((address_space(4))) uint64_t *>(table);
-    auto asSeen = [&](const uint64_t (&row)[3]) { return row[2] == len0 && ((row[0] | row[1]) & (kUnitBytes - 1)) == 0; };
-    auto leave = [&](const uint64_t (&row)[3]) {
-        if (row[2] != 0) {
-            ListRest(rest, capacity, row[0], row[1], row[2]);
-        }
-    };
-    auto shorter = [&](auto count) {
+    auto several = [&](auto count) {
         constexpr uint32_t kParts = decltype(count)::value;
-        for (;; item += waves, loadAt += period, storeAt += period) {
-            uint64_t src[kParts];
-            uint64_t dst[kParts];
-            bool all = true;
+        uint64_t src[kParts];
+        uint64_t dst[kParts];
+        bool all = true;
 #pragma unroll
-            for (uint32_t j = 0; j < kParts; ++j) {
-                const uint32_t seg = item * kParts + j < nseg ? item * kParts + j : nseg - 1;       // the last again rather than none
-                const uint64_t row[3] = {rows[3ull * seg], rows[3ull * seg + 1], rows[3ull * seg + 2]};
-                src[j] = row[0];
-                dst[j] = row[1];
-                all = all && asSeen(row);
-            }
-            if (all) {
-                CopyWholeWindowed<kParts>(src, dst, loadAt, storeAt);
-            } else {
-#pragma unroll 1
-                for (uint32_t seg = item * kParts; seg < nseg && seg < (item + 1) * kParts; ++seg) {
-                    leave({rows[3ull * seg], rows[3ull * seg + 1], rows[3ull * seg + 2]});        // those that are as seen too
-                }
-            }
-            if (items - item <= waves) {
-                return;
-            }
+        for (uint32_t j = 0; j < kParts; ++j) {
+            const uint32_t at = item * kParts + j < nseg ? item * kParts + j : nseg - 1;       // the last again rather than none
+            const uint64_t row[3] = {rows[3ull * at], rows[3ull * at + 1], rows[3ull * at + 2]};
+            src[j] = row[0];
+            dst[j] = row[1];
+            all = all && asSeen(row);
         }
+        if (all) {
+            CopyWholeWindowed<kParts>(src, dst, loadAt, storeAt);
+        }
+        return all;
     };
-    if (together == 2) {
-        shorter(std::integral_constant<uint32_t, 2>());
-        return;
-    }
-    if (together == 4) {
-        shorter(std::integral_constant<uint32_t, 4>());
-        return;
-    }
     uint32_t seg = item / each;
     uint64_t row[3] = {rows[3ull * seg], rows[3ull * seg + 1], rows[3ull * seg + 2]};
     for (;;) {
+        uint32_t first = seg;
         const uint32_t k = item - seg * each;
         const bool more = items - item > waves;
-        item += more ? waves : 0;
-        seg = item / each;
-        const uint64_t next[3] = {rows[3ull * seg], rows[3ull * seg + 1], rows[3ull * seg + 2]};      // requested now, needed after the copy
-        if (asSeen(row)) {
-            CopyWholeWindowed<1>({row[0] + k * kDeepBytes}, {row[1] + k * kDeepBytes}, loadAt, storeAt);
-        } else if (k == 0) {
-            leave(row);
+        bool all = true;
+        if (together == 1) {
+            seg = more ? (item + waves) / each : seg;
+            const uint64_t next[3] = {rows[3ull * seg], rows[3ull * seg + 1], rows[3ull * seg + 2]};      // requested now, needed after the copy
+            all = asSeen(row);
+            if (all) {
+                CopyWholeWindowed<1>({row[0] + k * kDeepBytes}, {row[1] + k * kDeepBytes}, loadAt, storeAt);
+            }
+            row[0] = next[0];
+            row[1] = next[1];
+            row[2] = next[2];
+        } else {
+            first = item * together;
+            all = together == 2 ? several(std::integral_constant<uint32_t, 2>()) : several(std::integral_constant<uint32_t, 4>());
+        }
+        if (!all) {
+            // a quarter of 16 KiB at a time
+            uint64_t src[4];
+            uint64_t dst[4];
+            uint32_t bytes[4];
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q) {
+                const uint32_t at = first + q * together / 4;
+                const uint32_t begin = together == 1 ? k * kDeepBytes + q * (kDeepBytes / 4) : q * (kDeepBytes / 4) % (kDeepBytes / together);
+                const bool there = at < nseg;
+                const uint32_t r = there ? at : first;
+                const uint64_t len = there ? rows[3ull * r + 2] : 0;
+                src[q] = rows[3ull * r] + begin;
+                dst[q] = rows[3ull * r + 1] + begin;
+                const bool fits = len <= len0 && ((src[q] | dst[q]) & (kUnitBytes - 1)) == 0;
+                if (!fits && len != 0 && begin == 0) {
+                    ListRest(rest, capacity, src[q], dst[q], len);
+                }
+                const uint32_t left = fits && len > begin ? static_cast<uint32_t>(len) - begin : 0;
+                bytes[q] = left < kDeepBytes / 4 ? left : kDeepBytes / 4;
+            }
+            if ((bytes[0] | bytes[1] | bytes[2] | bytes[3]) != 0) {
+                CopyPartWindowed(src, dst, bytes, loadAt, storeAt);
+            }
         }
         if (!more) {
             return;
         }
-        row[0] = next[0];
-        row[1] = next[1];
-        row[2] = next[2];
+        item += waves;
         loadAt += period;
         storeAt += period;
     }

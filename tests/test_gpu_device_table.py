@@ -242,3 +242,81 @@ def test_longer_tables_by_what_their_first_segments_are(gpu, count, size, odd, l
 @pytest.mark.parametrize("odd", [False, True])
 def test_longer_tables_where_a_round_of_waves_ends(gpu, count, size, odd):
     test_longer_tables_by_what_their_first_segments_are(gpu, count, size, odd, 2)
+
+
+# What a page unlike the sampled ones becomes: its place's slot where it is shorter and begins on 16 bytes, an entry of the list elsewhere, on
+# both sides of a chunk's quarters and next to pages that are as sampled.
+@pytest.mark.parametrize("count,size", [(4097, 16384), (9001, 8192), (6145, 4096), (4200, 49152)])
+@pytest.mark.parametrize("shifted", [False, True])
+def test_longer_tables_with_a_few_shorter_pages(gpu, count, size, shifted):
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(count)
+    edges = [0, 1, 15, 16, 17] + [e + d for e in (4096, 8192, 12288, 16384, 32768, 49152) for d in (-17, -16, -1, 0, 1, 16) if e + d <= size]
+    looked_at = {count * (i * 0x9E3779B9 % 2**32) >> 32 for i in range(1, 9)}
+    free = np.array([i for i in range(64, count) if i not in looked_at])
+    which = np.concatenate([rng.choice(free[:-5], len(edges), replace=False), [count - 1]])
+    lens = np.full(count, size, dtype=np.int64)
+    lens[which] = edges + [size - 3]
+    step = size + 256
+    at = rng.permutation(count) * step
+    place = rng.permutation(count) * step
+    if shifted:                                                  # sources, destinations or both between units
+        at[which[::2]] += 5
+        place[which[::3]] += 9
+    source = torch.randint(0, 256, (count * step,), dtype=torch.uint8, device="cuda")
+    before = torch.randint(0, 256, (count * step,), dtype=torch.uint8, device="cuda")
+    expect, data = before.cpu().numpy(), source.cpu().numpy()
+    for s, d, l in zip(at, place, lens):
+        expect[d:d + l] = data[s:s + l]
+    target = before.clone()
+    table = torch.from_numpy(np.stack([source.data_ptr() + at, target.data_ptr() + place, lens], axis=1)).cuda()
+    for _ in range(2):
+        target.copy_(before)
+        torch.cuda.synchronize()
+        assert gpu.mf_xcopy_device_table(table.data_ptr(), count, native.ROUTE_HBM, None) == 0, native.last_error()
+        assert gpu.mfrt_device_sync() == 0
+        assert np.array_equal(target.cpu().numpy(), expect)
+
+
+# Tables that begin like pages of one length and are none: right, and at the rate they have without the look at their first segments
+# (a page that is listed costs eleven nanoseconds of one word; all of them listed took these two to four times as long).
+@pytest.mark.parametrize("name,lengths,off", [
+    ("sources off units", [(8192, 16384)], 4), ("longer ones behind", [(4096, 8192), (4096, 32768)], 0),
+    ("much longer ones behind", [(8192, 4096), (8192, 16384)], 0), ("eight long ones first", [(8, 65536), (9000, 4096)], 0),
+])
+def test_longer_tables_that_only_begin_like_pages(gpu, name, lengths, off):
+    torch = pytest.importorskip("torch")
+    import time
+    lens = np.concatenate([np.full(n, size, dtype=np.int64) for n, size in lengths])
+    count = len(lens)
+    order = np.random.default_rng(count).permutation(count)
+    at = np.cumsum(lens) - lens + off
+    place = np.empty(count, dtype=np.int64)
+    place[order] = np.cumsum(lens[order]) - lens[order]
+    size = int(lens.sum())
+    source = torch.randint(0, 256, (size + 64,), dtype=torch.uint8, device="cuda")
+    target = torch.zeros(size + 64, dtype=torch.uint8, device="cuda")
+    table = torch.from_numpy(np.stack([source.data_ptr() + at, target.data_ptr() + place, lens], axis=1)).cuda()
+    torch.cuda.synchronize()
+
+    def best():
+        times = []
+        for _ in range(5):
+            began = time.perf_counter()
+            for _ in range(20):
+                assert gpu.mf_xcopy_device_table(table.data_ptr(), count, native.ROUTE_HBM, None) == 0, native.last_error()
+            assert gpu.mfrt_device_sync() == 0
+            times.append((time.perf_counter() - began) / 20)
+        return min(times)
+
+    chosen = best()
+    expect, data = np.zeros(size + 64, dtype=np.uint8), source.cpu().numpy()
+    for s, d, l in zip(at, place, lens):
+        expect[d:d + l] = data[s:s + l]
+    assert np.array_equal(target.cpu().numpy(), expect)
+    assert gpu.mf_xcopy_tune_table(1, 256) == 0                  # a grid set by hand: no look
+    try:
+        plain = best()
+    finally:
+        assert gpu.mf_xcopy_tune_table(1, 0) == 0
+    assert chosen < 1.5 * plain, (chosen, plain)
