@@ -1999,7 +1999,7 @@ static void TestWindows()
     (void)fake_rt_last_window();
     uint64_t launchesBefore = mf_xcopy_launch_count();
     CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-    CHECK(fake_rt_last_window() == 7450000);                   // source and destination on cache lines: the higher rate
+    CHECK(fake_rt_last_window() == XcopyTuning{}.windowLongMBps);                   // source and destination on cache lines: the higher rate
     CHECK(mf_xcopy_launch_count() - launchesBefore == 2);      // twice the minimum: two launches of 512 MiB, a schedule each
     CHECK(engine.DrainThread() == BM_OK);
     bool ok = true;
@@ -2016,7 +2016,7 @@ static void TestWindows()
         std::memset(from + gib, 0, gib + 512);
         launchesBefore = mf_xcopy_launch_count();
         CHECK(engine.Submit(&so, &dO, &lo, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-        CHECK(fake_rt_last_window() == 6800000);
+        CHECK(fake_rt_last_window() == XcopyTuning{}.windowMBps);
         CHECK(mf_xcopy_launch_count() - launchesBefore == 1);      // 64 bytes short of twice the minimum
         CHECK(engine.DrainThread() == BM_OK);
         CHECK(std::memcmp(from + gib + 256 + 19, from + 3, lo) == 0 && from[gib + 256 + 18] == 0 && from[gib + 256 + 19 + lo] == 0);
@@ -2062,12 +2062,12 @@ static void TestWindows()
             same = std::memcmp(reinterpret_cast<void *>(dst64[i]), reinterpret_cast<void *>(src64[i]), len64[i]) == 0;
         }
         CHECK(same);
-        CHECK(fake_rt_last_window() == 6800000);       // destinations between cache lines: the general rate
+        CHECK(fake_rt_last_window() == XcopyTuning{}.windowMBps);       // destinations between cache lines: the general rate
         for (uint32_t i = 0; i < 64; ++i) {
             dst64[i] += 128 - 48;
         }
         CHECK(engine.Submit(src64.data(), dst64.data(), len64.data(), 64, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-        CHECK(fake_rt_last_window() == 7300000);       // on cache lines, 16 MiB each: the rate between
+        CHECK(fake_rt_last_window() == XcopyTuning{}.windowAlignedMBps);       // on cache lines, 16 MiB each: the rate between
         CHECK(engine.DrainThread() == BM_OK);
     }
     l1 = (gib >> 3) - 1;                           // one byte below the limit: those of TestLineWindows
@@ -2075,7 +2075,7 @@ static void TestWindows()
     CHECK(fake_rt_last_window() == 0);
     l1 = gib >> 3;
     CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-    CHECK(fake_rt_last_window() == 7450000);
+    CHECK(fake_rt_last_window() == XcopyTuning{}.windowLongMBps);
     {
         // between cache lines the same limit, at the general rate
         uint64_t so = s1 + 16;
@@ -2085,7 +2085,7 @@ static void TestWindows()
         CHECK(fake_rt_last_window() == 0);
         lo = gib >> 3;
         CHECK(engine.Submit(&so, &dO, &lo, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-        CHECK(fake_rt_last_window() == 6800000);
+        CHECK(fake_rt_last_window() == XcopyTuning{}.windowMBps);
     }
     l1 = gib;
     CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0, true) == BM_OK);
