@@ -549,7 +549,8 @@ PyType_Slot g_directSlots[] = {
     {Py_tp_members, g_directMembers},
     {0, nullptr},
 };
-PyType_Spec g_directSpec = {"_calls.Direct", sizeof(Direct), 0, Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_VECTORCALL, g_directSlots};
+PyType_Spec g_directSpec = {"_calls.Direct", sizeof(Direct), 0,
+                            Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_VECTORCALL | Py_TPFLAGS_DISALLOW_INSTANTIATION, g_directSlots};
 PyTypeObject *g_directType = nullptr;
 
 // direct(name, function): what stands for the ctypes object of that function, or the object itself where there is nothing

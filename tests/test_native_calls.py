@@ -99,6 +99,15 @@ def test_a_batch_call_inside_a_batch_call(lib, outer, inner):
     assert done.stdout.split() == [str(native.SM_NOT_INITIALIZED)] * 3
 
 
+def test_what_stands_for_a_function_is_made_for_one(lib):
+    """The type behind lib.mf_moe_combine cannot be instantiated: such an object would have no function to call."""
+    kind = type(lib.mf_moe_combine)
+    assert kind is not type(lib.mf_xcopy_batch)
+    for make in (kind, lambda: kind.__new__(kind), lambda: object.__new__(kind)):
+        with pytest.raises(TypeError):
+            make()
+
+
 def test_codes_without_a_pool_or_a_session(lib):
     pool = bm.BigMemory(None)
     assert pool.copy_data(1, 2, 3, bm.BmCopyType.G2G) == native.SM_INVALID_PARAM
