@@ -337,9 +337,9 @@ def lib():
                     f"{DATAPLANE_PATH} is missing: build it with `make -C memfabric_hybrid_amd/csrc` "
                     "(or __graft_entry__.build()); there is no fallback path")
             handle = _bind(ctypes.CDLL(DATAPLANE_PATH, mode=ctypes.RTLD_GLOBAL), _SIGNATURES)
-            if os.path.exists(CALLS_PATH):
-                for name in _DIRECT:
-                    setattr(handle, name, _load_calls().direct(name, getattr(handle, name)))
+            direct = _direct()
+            for name in _DIRECT if direct is not None else ():
+                setattr(handle, name, direct(name, getattr(handle, name)))
             _lib = handle
         return _lib
 
@@ -374,6 +374,17 @@ def _load_calls():
         loader.exec_module(module)
         _calls = module
     return _calls
+
+
+def _direct():
+    """direct() of the extension module; None where that is missing, does not load or is an older one: the library's functions
+    are then called through ctypes, and calls() says what is wrong."""
+    if not os.path.exists(CALLS_PATH):
+        return None
+    try:
+        return getattr(_load_calls(), "direct", None)
+    except (ImportError, OSError):
+        return None
 
 
 def calls():

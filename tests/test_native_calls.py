@@ -6,6 +6,7 @@ import os
 import shutil
 import subprocess
 import sys
+import types
 
 import numpy as np
 import pytest
@@ -106,6 +107,28 @@ def test_what_stands_for_a_function_is_made_for_one(lib):
     for make in (kind, lambda: kind.__new__(kind), lambda: object.__new__(kind)):
         with pytest.raises(TypeError):
             make()
+
+
+@pytest.mark.parametrize("content", [b"", b"no library", None])
+def test_the_library_loads_beside_a_module_that_does_not(lib, monkeypatch, tmp_path, content):
+    """The module's file missing, empty or broken: the library's functions are the ctypes ones, and calls() raises."""
+    path = tmp_path / os.path.basename(native.CALLS_PATH)
+    if content is not None:
+        path.write_bytes(content)
+    for name, value in (("CALLS_PATH", str(path)), ("_lib", None), ("_calls", None)):
+        monkeypatch.setattr(native, name, value)
+    assert issubclass(type(native.lib().mf_moe_combine), ctypes._CFuncPtr)
+    assert native.lib().mf_moe_combine(None, None, None, 1, 8, 1, None, None) == lib.mf_moe_combine(None, None, None, 1, 8, 1, None, None) != 0
+    with pytest.raises((ImportError, OSError)):
+        native.calls()
+
+
+def test_the_library_loads_beside_an_older_module(lib, monkeypatch):
+    older = types.SimpleNamespace(copy_batch=native.calls().copy_batch)
+    monkeypatch.setattr(native, "_lib", None)
+    monkeypatch.setattr(native, "_calls", older)
+    assert issubclass(type(native.lib().mf_moe_combine), ctypes._CFuncPtr)
+    assert native.calls() is older
 
 
 def test_codes_without_a_pool_or_a_session(lib):
