@@ -60,7 +60,7 @@ int32_t mf_xcopy_hold_stores(int32_t nanos);
  * waves no longer keep up, the windows dissolve and the copy runs at about the rate it
  * has without them.  Segments whose sources and destinations agree modulo 16 are paced for
  * 7 300 000, those on 128-byte lines of 64 MiB and
- * more on average for 7 450 000, and a batch of 1 GiB and more of such long segments is cut into launches of
+ * more on average for 7 375 000, and a batch of 1 GiB and more of such long segments is cut into launches of
  * about 512 MiB, which hold their schedule more often than longer ones (1 GiB: 7.1-7.2 instead of 6.7 TB/s).
  * Segments whose source and destination differ modulo 16 go at 35/34 of the default rate.  Rectangles of 32 MiB and more whose rows hold
  * windows go at 35/34 of the default rate where rows of whole lines lie against one another in the destination, pairs of

@@ -1269,10 +1269,7 @@ int XcopyEngine::Calibrate()
     const uint32_t holds[3] = {rule - kCalibrateHoldStepNanos, rule, rule + kCalibrateHoldStepNanos};
     const uint32_t defaultRate = XcopyTuning{}.windowMBps;
     const uint32_t defaultLong = XcopyTuning{}.windowLongMBps;
-    // The higher two are tried half-way between them: at 7.5 TB/s one process in some twenty-five saw none of its six copies keep the schedule, on
-    // memory that happened to lie badly, and would have run at the general rate for good, 5 % slower.
-    const uint32_t rates[3] = {defaultRate, static_cast<uint32_t>(static_cast<uint64_t>(defaultRate) * kCalibrateSlowerWindowPercent / 100),
-                               (XcopyTuning{}.windowAlignedMBps + defaultLong) / 2};
+    const uint32_t rates[3] = {defaultRate, static_cast<uint32_t>(static_cast<uint64_t>(defaultRate) * kCalibrateSlowerWindowPercent / 100), defaultLong};
     float us[8] = {};
     const int err = mfk_xcopy_calibrate(stream, holds, rates, us);
     if (err != 0) {

@@ -85,7 +85,10 @@ struct XcopyTuning {
     uint32_t deviceTableWgPerCu = 0;   // grid of a device-resident table in workgroups per CU, 0 = four per segment between 16 and 1024 per CU
     uint32_t windowMBps = 6800000;   // long HBM copies alternate between read and write windows cut for this rate; 0 = never
     uint32_t windowAlignedMBps = 7300000;   // the same for launches of segments that all start at multiples of kWindowAlignBytes in source and destination, which hold more; 0 = the rate above
-    uint32_t windowLongMBps = 7450000;      // and for those of them whose segments are kWindowLongSegmentBytes and longer on average, which hold more still; 0 = the rate above
+    // And for those of them whose segments are kWindowLongSegmentBytes and longer on average, which hold more still; 0 = the rate above.  The highest that copies kept
+    // to in each of ten processes; us, the mean back to back at 7.3 / 7.375 / 7.45 TB/s: one segment of 512 MiB 151.9 / 151.9 / 151.2, of 1 GiB 302 / 300 / 301,
+    // in one process of four 303 / 300 / 307; waited for one by one, 512 MiB 165 / 165 / 163 to 176, 1 GiB 317 / 314 / 312.  At 7.5 one in some twenty-five saw none of six keep to it.
+    uint32_t windowLongMBps = 7375000;
 };
 
 // A batch of up to 128 segments between HBM addresses is copied in windows from where held stores end (64 MiB, 112 for one segment); from this

@@ -346,11 +346,14 @@ int mfk_xcopy_prelaunch(void *) { return 0; }
 // The calibration "measures" what the test has put here (all zero: nothing measured, the defaults stay).
 static float g_calibration[8] = {};
 static uint32_t g_calibrationHolds[3] = {};
+static uint32_t g_calibrationRates[3] = {};
 extern "C" void fake_rt_set_calibration(const float *us) { std::memcpy(g_calibration, us, sizeof(g_calibration)); }
 extern "C" const uint32_t *fake_rt_calibration_holds(void) { return g_calibrationHolds; }
-int mfk_xcopy_calibrate(void *, const uint32_t *holdNanos, const uint32_t *, float *out)
+extern "C" const uint32_t *fake_rt_calibration_rates(void) { return g_calibrationRates; }
+int mfk_xcopy_calibrate(void *, const uint32_t *holdNanos, const uint32_t *windowMBps, float *out)
 {
     std::memcpy(g_calibrationHolds, holdNanos, sizeof(g_calibrationHolds));
+    std::memcpy(g_calibrationRates, windowMBps, sizeof(g_calibrationRates));
     std::memcpy(out, g_calibration, sizeof(g_calibration));
     return 0;
 }

@@ -43,6 +43,7 @@ extern "C" void fake_rt_skip_copies(int on);
 extern "C" uint64_t fake_rt_stream_waits(void);
 extern "C" void fake_rt_set_calibration(const float *us);
 extern "C" const uint32_t *fake_rt_calibration_holds(void);
+extern "C" const uint32_t *fake_rt_calibration_rates(void);
 extern "C" uint32_t fake_rt_last_table_shift(void);
 extern "C" uint32_t fake_rt_last_table_hold(void);
 extern "C" uint32_t fake_rt_last_piece_wait(void);
@@ -1008,6 +1009,7 @@ static void TestCalibration()
     float micros[8] = {};
     CHECK(mf_xcopy_calibration(&enabled, &delta, &mbps, &alignedMbps, &longMbps, micros) == 1);
     CHECK(enabled == 1 && delta == -200 && mbps == rate && alignedMbps == alignedRate && longMbps == longRate && micros[1] == 4.40f && micros[5] == 160.0f && micros[7] == 150.0f);
+    CHECK(fake_rt_calibration_rates()[0] == mbps && fake_rt_calibration_rates()[2] == longMbps);     // what is in force has been tried
     {
         std::vector<uint8_t> from(12 << 20), to(12 << 20);
         const uint64_t fromBase = (reinterpret_cast<uint64_t>(from.data()) + 4095) & ~4095ull;
