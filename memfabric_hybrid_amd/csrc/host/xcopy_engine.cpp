@@ -2127,9 +2127,7 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
     uint32_t units = 0;
     bool oversized = false;      // a run the 32-bit length of the inline table cannot hold is possible
     bool windowed = false;
-    bool lineWindowed = false;
     uint32_t windowRate = tuning_.windowMBps;
-    uint32_t linesRate = windowRate;
     uint64_t queuedBytes = 0;
     if (n <= 4 * kInlineSegs) {  // small enough that a failed attempt costs next to nothing
         uint64_t total = 0;
@@ -2147,15 +2145,14 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         // held stores end (XcopyWindowKernel has the figures).
         const bool aligned = (addressBits & (kWindowAlignBytes - 1)) == 0;
         const bool apart = (apartBits & (kUnitBytes - 1)) != 0;
-        windowed = !unordered && !apart && WindowsApply(total, route, kWindowMinBytes);
-        lineWindowed = !unordered && !windowed && WindowsApply(total, route, kDeepMaxBytes + 1) && !DeepHoldApplies(total, n, route, unordered);
-        // Segments that all start on cache lines, in source and destination, hold a higher rate, and long ones the highest; those whose
-        // destinations are off a line hold that of the first, as their chunks are cut on lines, and shifted ones a little more than the general one.
+        windowed = !unordered && WindowsApply(total, route, kDeepMaxBytes + 1) && !DeepHoldApplies(total, n, route, unordered);
+        // Segments whose sources and destinations agree modulo 16 hold a higher rate, as their chunks are cut on the destinations' lines; long ones that all
+        // start on cache lines, in source and destination, the highest, and shifted ones a little more than the general one.
         // Back to back, us, at 7.2 / 7.3 / 7.4 / 7.5 TB/s: one segment of 370 MB 110.0 / 108.8 / 107.9 / 107.0, 900 MB 269 / 266 / 264 / 262 (512 MiB at 7.6 158 to
         // 162, 7.5 151 to 155); 128 x 9 MB 355 / 348 / 348 / 350, 128 x 2.4 MB 91.9 / 92.1 / 91.8 / 101.9; the column-parallel part of 28 layers with its rectangles
         // 3986 / 3955 / 3952 / 3958; off a line 300 MB 89.0 / 87.7 / 87.1 / 86.1, 900 MB 271 / 269 / 262 / 262.  Shifted, at 6.8 / 7.0 / 7.2 / 7.3: 200 MB 63.4 / 62.1 / 61.0 / 61.2,
         // 900 MB 282 / 278 / 276 / 281, 100 of 2 MB on average 35.4 / 35.2 / 36.2 / 36.8, of 4 MB 131 / 129 / 135 / 144.
-        const bool longSegments = (windowed || lineWindowed) && total / n >= kWindowLongSegmentBytes;
+        const bool longSegments = windowed && total / n >= kWindowLongSegmentBytes;
         if (longSegments && maySlice && total >= 2 * kWindowPieceBytes) {
             // A windowed launch that loses its schedule runs the rest of its bytes at the rate without windows, and the longer
             // it runs the likelier that is: launches of kWindowPieceBytes to twice that, each with a schedule of its own, hold
@@ -2164,21 +2161,15 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
             // segments (600 to 900 MB) were no faster than in launches of 128.
             return SubmitInPieces(src, dst, len, n, total, route, stream, mask, maskValue);
         }
-        linesRate = tuning_.windowAlignedMBps == 0 ? tuning_.windowMBps
-                    : apart                          ? std::min(tuning_.windowMBps / 34 * 35, tuning_.windowAlignedMBps)
-                                                     : tuning_.windowAlignedMBps;
-        windowRate = tuning_.windowMBps;
         if (aligned && longSegments && tuning_.windowLongMBps != 0) {
             windowRate = tuning_.windowLongMBps;
-        } else if (aligned && tuning_.windowAlignedMBps != 0) {
-            windowRate = tuning_.windowAlignedMBps;
-        } else if (lineWindowed) {
-            windowRate = linesRate;
+        } else if (tuning_.windowAlignedMBps != 0) {
+            windowRate = apart ? std::min(tuning_.windowMBps / 34 * 35, tuning_.windowAlignedMBps) : tuning_.windowAlignedMBps;
         }
-        if (windowed || lineWindowed) {
+        if (windowed) {
             units = mfk_xcopy_window_units();
         }
-        const bool deep = !windowed && !lineWindowed && DeepHoldApplies(total, n, route, unordered);
+        const bool deep = !windowed && DeepHoldApplies(total, n, route, unordered);
         if (deep && n != 1 && (apartBits & (kUnitBytes - 1)) != 0 && mfrt_stream_capturing(stream) == 0) {
             // as pieces: sixteen loads per lane of aligned units and what shifts them, with the table of the kernel arguments, take
             // more registers than sixteen waves per CU have (42 MB 17.5 us with straddling loads); one segment has no table
@@ -2195,12 +2186,11 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
     if (!inlined && oversized) {
         // a run of 4 GiB and more may have made the one-pass attempt give up: the general inline path cuts it into pieces
         NormalizeSegments(src, dst, len, n, kInlinePiece, ctx.segs);
-        units = windowed || lineWindowed ? mfk_xcopy_window_units() : ChooseUnits(ctx.segs.totalBytes, cu, route, tuning_);
+        units = windowed ? mfk_xcopy_window_units() : ChooseUnits(ctx.segs.totalBytes, cu, route, tuning_);
         inlined = BuildInlinePlan(ctx.segs, units, plan);
     }
-    if (inlined && (windowed || lineWindowed)) {
-        const int err = windowed ? mfk_xcopy_windowed(&plan, windowRate, linesRate, mask, maskValue, stream)
-                                 : mfk_xcopy_line_windowed(&plan, windowRate, mask, maskValue, stream);
+    if (inlined && windowed) {
+        const int err = mfk_xcopy_windowed(&plan, windowRate, mask, maskValue, stream);
         if (err != 0) {
             MF_FAIL(BM_ERROR, "xcopy launch failed: " << mfrt_error_string(err));
         }

@@ -84,17 +84,18 @@ struct XcopyTuning {
     bool stageUnordered = true;  // the upload of a ragged table's descriptors is launched without a barrier
     uint32_t deviceTableWgPerCu = 0;   // grid of a device-resident table in workgroups per CU, 0 = four per segment between 16 and 1024 per CU
     uint32_t windowMBps = 6800000;   // long HBM copies alternate between read and write windows cut for this rate; 0 = never
-    uint32_t windowAlignedMBps = 7300000;   // the same for launches of segments that all start at multiples of kWindowAlignBytes in source and destination, which hold more; 0 = the rate above
-    // And for those of them whose segments are kWindowLongSegmentBytes and longer on average, which hold more still; 0 = the rate above.  The highest that copies kept
+    // The same for launches whose sources and destinations agree modulo 16, which hold more; 0 = the rate above.  300 MB, us, at 6.8 / 7.3 TB/s: with the source 64 bytes
+    // off a cache line 91.8 / 86.0, the destination 91.8 / 86.2; 100 segments of 3 MB, 48 bytes off 92.6 / 86.8, 92.6 / 86.9.
+    uint32_t windowAlignedMBps = 7300000;
+    // And for those of them that all start at multiples of kWindowAlignBytes in source and destination and are kWindowLongSegmentBytes and longer on average, which hold more still; 0 = the rate above.  The highest that copies kept
     // to in each of ten processes; us, the mean back to back at 7.3 / 7.375 / 7.45 TB/s: one segment of 512 MiB 151.9 / 151.9 / 151.2, of 1 GiB 302 / 300 / 301,
     // in one process of four 303 / 300 / 307; waited for one by one, 512 MiB 165 / 165 / 163 to 176, 1 GiB 317 / 314 / 312.  At 7.5 one in some twenty-five saw none of six keep to it.
     uint32_t windowLongMBps = 7375000;
 };
 
-// A batch of up to 128 segments between HBM addresses is copied in windows from where held stores end (64 MiB, 112 for one segment); from this
-// total on the caller names a rate for segments on cache lines besides.  Back to back, 32 segments on lines, windows of 4096 waves against none:
-// 66 MiB 6.37 against 5.71 TB/s, 80 MiB 6.57 against 5.76, 130 MiB 6.94 against 6.14, 256 MiB 7.14 against 6.37, 600 MiB 7.20 against 6.31.
-constexpr uint64_t kWindowMinBytes = 128ull << 20;
+// (A batch of up to 128 segments between HBM addresses is copied in windows from where held stores end, 64 MiB, 112 for one segment.  Back to back, 32
+// segments on lines, windows of 4096 waves against none: 66 MiB 6.37 against 5.71 TB/s, 80 MiB 6.57 against 5.76, 130 MiB 6.94 against 6.14, 256 MiB 7.14
+// against 6.37, 600 MiB 7.20 against 6.31.)
 // Rectangles in chunks of their payload: in windows, and without (several threads, rows between cache lines), where whole rows are as
 // fast up to 40 MB (Copy2dChunkKernel has the figures).
 constexpr uint64_t kRectChunksMinBytes = 32ull << 20;
@@ -105,7 +106,7 @@ constexpr uint64_t kWindowPieceBytes = 512ull << 20;          // launches into w
 constexpr uint64_t kWindowLongSegmentBytes = 64ull << 20;     // launches whose segments average this much go out in pieces of kWindowPieceBytes and more
 constexpr uint64_t kWindowAlignBytes = 128;                   // a cache line: segments that start on one are read and written in whole lines by every wave
 constexpr uint64_t kWindowSliceMinSegmentBytes = 4ull << 20;   // tables of segments this long on average are cut into windowed launches
-constexpr uint64_t kWindowSliceMinAlignedSegmentBytes = 1ull << 20;   // the same for segments on cache lines: kInlineSegs of them reach kWindowMinBytes
+constexpr uint64_t kWindowSliceMinAlignedSegmentBytes = 1ull << 20;   // the same for segments on cache lines: kInlineSegs of them are 128 MiB
 
 // What Start() measured on the GPU it runs on and chose from it (XcopyEngine::Calibrate).
 struct XcopyCalibration {

@@ -2001,16 +2001,6 @@ int LaunchInline(const InlinePlan &plan, uint32_t grid, uint32_t lanes, hipStrea
     return static_cast<int>(hipLaunchKernel(kernel, dim3(grid), dim3(lanes), args, 0, stream));
 }
 
-// Whether all destinations begin on a line.
-bool OnLines(const InlinePlan &plan)
-{
-    uint64_t bits = 0;
-    for (uint32_t i = 0; i < kInlineSegs && plan.first[i] != kNoChunk; ++i) {
-        bits |= plan.dst[i];
-    }
-    return (bits & (kLineBytes - 1)) == 0;
-}
-
 // The plan with the chunks of LineChunks(), which are others also where a segment on a line ends with a few bytes behind its last whole chunk.
 InlinePlan CutOnLines(const InlinePlan &plan)
 {
@@ -2169,12 +2159,7 @@ extern "C" int mfk_xcopy_windows_available(void)
     return mf::WindowPeriodTicks(2ull * mf::kWindowWaves * mf::kWindowUnits * mf::kUnitBytes, 6800000u) != 0 ? 1 : 0;
 }
 
-extern "C" uint32_t mfk_xcopy_window_waves(void)
-{
-    return mf::kLongWaves;
-}
-
-extern "C" int mfk_xcopy_line_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream)
+extern "C" int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream)
 {
     using namespace mf;
     const InlinePlan &plan = *static_cast<const InlinePlan *>(inlinePlan);
@@ -2183,18 +2168,6 @@ extern "C" int mfk_xcopy_line_windowed(const void *inlinePlan, uint32_t windowMB
         return -1;
     }
     const int err = LaunchWindowed(plan, windowMBps, s);
-    return err != 0 ? err : Signal(mask, maskValue, s);
-}
-
-extern "C" int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, uint32_t linesMBps, void *mask, uint32_t maskValue, void *stream)
-{
-    using namespace mf;
-    const InlinePlan &plan = *static_cast<const InlinePlan *>(inlinePlan);
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (plan.units != kWindowUnits || plan.nchunk == 0 || windowMBps == 0) {
-        return -1;
-    }
-    const int err = LaunchWindowed(plan, OnLines(plan) ? windowMBps : linesMBps, s);
     return err != 0 ? err : Signal(mask, maskValue, s);
 }
 

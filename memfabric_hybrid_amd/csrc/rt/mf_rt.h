@@ -87,15 +87,11 @@ int mfk_xcopy_inline(const void *inlinePlan, int route, uint32_t grid, void *mas
  * again when `word` has been stored: launches that share it follow one another on a stream. */
 int mfk_xcopy_done(const void *inlinePlan, int route, uint32_t grid, void *word, uint32_t value, void *counter, void *stream);
 /* HBM to HBM copies of hundreds of MiB: the plan's chunks are mfk_xcopy_window_units() units (16 KiB), copied by up to
- * mfk_xcopy_window_waves() single-wave workgroups that alternate, chip-wide and by the clock, between a read half and a
- * write half of a period cut for `windowMBps` MB/s of HBM traffic (see XcopyWindowKernel), for `linesMBps` where a destination is
- * off a cache line.  No source may differ from its destination modulo 16. */
+ * 6144 single-wave workgroups that alternate, chip-wide and by the clock, between a read half and a
+ * write half of a period cut for `windowMBps` MB/s of HBM traffic, whatever the addresses (see XcopyWindowKernel). */
 int mfk_xcopy_windows_available(void);   /* 1 when the current device's constant-rate clock is known, which the period is cut by */
 uint32_t mfk_xcopy_window_units(void);
-uint32_t mfk_xcopy_window_waves(void);
-int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, uint32_t linesMBps, void *mask, uint32_t maskValue, void *stream);
-/* The same at one rate, whatever the addresses. */
-int mfk_xcopy_line_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream);
+int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream);
 /* tablePlan: a mf::TablePlan (kernels/xcopy_plan.h).  Under a pattern its triples may live in pinned host
  * memory and neither prefix nor group map is read. */
 int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, void *mask, uint32_t maskValue, void *stream);

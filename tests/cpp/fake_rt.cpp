@@ -358,30 +358,13 @@ int mfk_xcopy_calibrate(void *, const uint32_t *holdNanos, const uint32_t *windo
     return 0;
 }
 uint32_t mfk_xcopy_window_units(void) { return 1024; }
-uint32_t mfk_xcopy_window_waves(void) { return 4096; }
-int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, uint32_t, void *mask, uint32_t maskValue, void *stream)
+int mfk_xcopy_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream)
 {
     const mf::InlinePlan &p = *static_cast<const mf::InlinePlan *>(inlinePlan);
     if (p.units != 1024 || p.nchunk == 0 || windowMBps == 0) {
         return -1;
     }
     g_lastWindow = windowMBps;
-    return mfk_xcopy_inline(inlinePlan, 0, p.nchunk, mask, maskValue, stream, 0, 0);
-}
-static uint32_t g_lastLineWindow = 0;
-extern "C" uint32_t fake_rt_last_line_window(void)
-{
-    const uint32_t last = g_lastLineWindow;
-    g_lastLineWindow = 0;
-    return last;
-}
-int mfk_xcopy_line_windowed(const void *inlinePlan, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream)
-{
-    const mf::InlinePlan &p = *static_cast<const mf::InlinePlan *>(inlinePlan);
-    if (p.units != 1024 || p.nchunk == 0 || windowMBps == 0) {
-        return -1;
-    }
-    g_lastLineWindow = windowMBps;
     return mfk_xcopy_inline(inlinePlan, 0, p.nchunk, mask, maskValue, stream, 0, 0);
 }
 

@@ -33,7 +33,6 @@ extern "C" int fake_rt_last_combine_paced(void);
 extern "C" uint64_t fake_rt_signals(void);
 extern "C" uint64_t fake_rt_stream_syncs(void);
 extern "C" uint32_t fake_rt_last_window(void);
-extern "C" uint32_t fake_rt_last_line_window(void);
 extern "C" uint32_t fake_rt_last_reading(void);
 extern "C" void fake_rt_seal(void);
 extern "C" void fake_rt_fail_launches(int n);
@@ -2010,15 +2009,15 @@ static void TestWindows()
     }
     CHECK(ok && from[gib + 256 + gib - 1] == from[gib - 1]);
     {
-        // odd addresses that agree modulo 16 (head and tail bytes): windows at the general rate;
-        // addresses that differ modulo 16: those of TestLineWindows, one launch
+        // odd addresses that agree modulo 16 (head and tail bytes): windows at the rate between;
+        // addresses that differ modulo 16: a little above the general one, one launch
         uint64_t so = s1 + 3;
         uint64_t dO = s1 + gib + 256 + 19;
         uint64_t lo = gib - 64;
         std::memset(from + gib, 0, gib + 512);
         launchesBefore = mf_xcopy_launch_count();
         CHECK(engine.Submit(&so, &dO, &lo, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-        CHECK(fake_rt_last_window() == XcopyTuning{}.windowMBps);
+        CHECK(fake_rt_last_window() == XcopyTuning{}.windowAlignedMBps);
         CHECK(mf_xcopy_launch_count() - launchesBefore == 1);      // 64 bytes short of twice the minimum
         CHECK(engine.DrainThread() == BM_OK);
         CHECK(std::memcmp(from + gib + 256 + 19, from + 3, lo) == 0 && from[gib + 256 + 18] == 0 && from[gib + 256 + 19 + lo] == 0);
@@ -2026,7 +2025,7 @@ static void TestWindows()
         std::memset(from + gib, 0, gib + 512);
         launchesBefore = mf_xcopy_launch_count();
         CHECK(engine.Submit(&so, &dO, &lo, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-        CHECK(fake_rt_last_window() == 0);
+        CHECK(fake_rt_last_window() == XcopyTuning{}.windowMBps / 34 * 35);
         CHECK(mf_xcopy_launch_count() - launchesBefore == 1);
         CHECK(engine.DrainThread() == BM_OK);
         CHECK(std::memcmp(from + gib + 256 + 5, from + 3, lo) == 0 && from[gib + 256 + 4] == 0 && from[gib + 256 + 5 + lo] == 0);
@@ -2064,30 +2063,13 @@ static void TestWindows()
             same = std::memcmp(reinterpret_cast<void *>(dst64[i]), reinterpret_cast<void *>(src64[i]), len64[i]) == 0;
         }
         CHECK(same);
-        CHECK(fake_rt_last_window() == XcopyTuning{}.windowMBps);       // destinations between cache lines: the general rate
+        CHECK(fake_rt_last_window() == XcopyTuning{}.windowAlignedMBps);       // destinations between cache lines: the rate between
         for (uint32_t i = 0; i < 64; ++i) {
             dst64[i] += 128 - 48;
         }
         CHECK(engine.Submit(src64.data(), dst64.data(), len64.data(), 64, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-        CHECK(fake_rt_last_window() == XcopyTuning{}.windowAlignedMBps);       // on cache lines, 16 MiB each: the rate between
+        CHECK(fake_rt_last_window() == XcopyTuning{}.windowAlignedMBps);       // on cache lines, 16 MiB each: the same
         CHECK(engine.DrainThread() == BM_OK);
-    }
-    l1 = (gib >> 3) - 1;                           // one byte below the limit: those of TestLineWindows
-    CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-    CHECK(fake_rt_last_window() == 0);
-    l1 = gib >> 3;
-    CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-    CHECK(fake_rt_last_window() == XcopyTuning{}.windowLongMBps);
-    {
-        // between cache lines the same limit, at the general rate
-        uint64_t so = s1 + 16;
-        uint64_t dO = d1 + 48;
-        uint64_t lo = (gib >> 3) - 1;
-        CHECK(engine.Submit(&so, &dO, &lo, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-        CHECK(fake_rt_last_window() == 0);
-        lo = gib >> 3;
-        CHECK(engine.Submit(&so, &dO, &lo, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-        CHECK(fake_rt_last_window() == XcopyTuning{}.windowMBps);
     }
     l1 = gib;
     CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0, true) == BM_OK);
@@ -2187,9 +2169,9 @@ static int SubmitList(uint32_t n, uint64_t bytes, From from, To to)
     return ret != BM_OK ? ret : engine.DrainThread();
 }
 
-// Which batches take the windows whose chunks are cut on lines, and their rates: addresses that differ modulo 16, and all from where held
-// stores end up to the other windows.
-static void TestLineWindows()
+// Which batches of up to 128 segments go in windows, and at which rate: all from where held stores end, by whether they are long and on cache lines, and
+// whether source and destination agree modulo 16.
+static void TestWindowRatesOfCopies()
 {
     CHECK(hybm_init(0, 0) == BM_OK);
     fake_rt_skip_copies(1);
@@ -2199,15 +2181,18 @@ static void TestLineWindows()
     const uint32_t shifted = XcopyTuning{}.windowMBps / 34 * 35;
     const uint32_t between = XcopyTuning{}.windowAlignedMBps;
     const uint32_t most = XcopyTuning{}.windowLongMBps;
-    struct Form { uint32_t n; uint64_t bytes, from, to; uint32_t rate; bool other; };
+    struct Form { uint32_t n; uint64_t bytes, from, to; uint32_t rate; };
     const Form forms[] = {
-        {1, kHeldSingleBytes, 0, 0, 0, false},          {1, kHeldSingleBytes, 3, 16, 0, false},         // held
-        {1, kHeldSingleBytes + 1, 0, 0, most, false},   {1, kHeldSingleBytes + 1, 16, 48, between, false}, {1, kHeldSingleBytes + 1, 3, 16, shifted, false},
-        {1, 128 * mib - 1, 0, 0, most, false},          {1, 128 * mib, 0, 0, 0, true},                  {1, 128 * mib, 16, 48, 0, true},
-        {1, 128 * mib, 3, 16, shifted, false},          {1, 900 * mib + 5, 18, 7, shifted, false},      {1, 1024 * mib, 18, 7, shifted, false},
-        {2, 32 * mib, 0, 0, 0, false},                  {2, 32 * mib + 256, 0, 0, between, false},      {2, 32 * mib + 1, 16, 48, between, false},
-        {2, 64 * mib, 16, 48, 0, true},                 {2, 64 * mib - 1, 3, 16, shifted, false},       {128, mib + 77, 3, 16, shifted, false},
-        {128, 512 * 1024, 0, 0, 0, false},              {128, 512 * 1024 + 128, 0, 0, between, false},  {129, mib, 3, 16, 0, false},
+        {1, kHeldSingleBytes, 0, 0, 0},          {1, kHeldSingleBytes, 3, 16, 0},         // held
+        {1, kHeldSingleBytes + 1, 0, 0, most},   {1, kHeldSingleBytes + 1, 16, 48, between}, {1, kHeldSingleBytes + 1, 3, 16, shifted},
+        {1, 128 * mib - 1, 0, 0, most},          {1, 128 * mib, 0, 0, most},              {1, 128 * mib, 16, 48, between},
+        {1, 128 * mib, 3, 16, shifted},          {1, 900 * mib + 5, 18, 7, shifted},      {1, 1024 * mib, 18, 7, shifted},
+        {1, 1024 * mib, 0, 0, most},             {1, 300 * mib, 64, 0, between},          {1, 300 * mib, 0, 64, between},    // one side off a line
+        {1, 120 * mib, 64, 0, between},          {1, 1024 * mib, 64, 0, between},         {1, 300 * mib, 64, 8, shifted},
+        {2, 32 * mib, 0, 0, 0},                  {2, 32 * mib + 256, 0, 0, between},      {2, 32 * mib + 1, 16, 48, between},
+        {2, 64 * mib, 16, 48, between},          {2, 64 * mib, 0, 0, most},               {2, 64 * mib - 1, 0, 0, between},
+        {2, 64 * mib - 1, 3, 16, shifted},       {128, mib + 77, 3, 16, shifted},         {128, 3 * mib, 48, 0, between},
+        {128, 512 * 1024, 0, 0, 0},              {128, 512 * 1024 + 128, 0, 0, between},  {129, mib, 3, 16, 0},
     };
     for (const Form &f : forms) {
         std::vector<uint64_t> s(f.n), d(f.n), l(f.n, f.bytes);
@@ -2217,10 +2202,8 @@ static void TestLineWindows()
         }
         for (int mode = 0; mode < 2; ++mode) {      // declared independent of what is in flight: none
             (void)fake_rt_last_window();
-            (void)fake_rt_last_line_window();
             CHECK(engine.Submit(s.data(), d.data(), l.data(), f.n, MF_ROUTE_HBM, stream, nullptr, 0, mode == 1) == BM_OK);
-            CHECK(fake_rt_last_line_window() == (mode == 1 ? 0 : f.rate));
-            CHECK((fake_rt_last_window() != 0) == (mode == 0 && f.other));
+            CHECK(fake_rt_last_window() == (mode == 1 ? 0 : f.rate));
         }
         CHECK(engine.DrainThread() == BM_OK);
     }
@@ -2229,10 +2212,10 @@ static void TestLineWindows()
     uint64_t d1 = (1ull << 42) + 3;
     uint64_t l1 = 300 * mib;
     CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-    CHECK(fake_rt_last_line_window() == 0);
+    CHECK(fake_rt_last_window() == 0);
     CHECK(mf_xcopy_windows(6400000) == BM_OK);
     CHECK(engine.Submit(&s1, &d1, &l1, 1, MF_ROUTE_HBM, stream, nullptr, 0) == BM_OK);
-    CHECK(fake_rt_last_line_window() == 6400000);
+    CHECK(fake_rt_last_window() == 6400000);
     CHECK(mf_xcopy_windows(MF_XCOPY_WINDOWS_OWN_CHOICE) == BM_OK);
     CHECK(engine.DrainThread() == BM_OK);
     fake_rt_skip_copies(0);
@@ -2468,7 +2451,7 @@ int main()
     TestPlugin();
     TestHeldStores();
     TestWindows();
-    TestLineWindows();
+    TestWindowRatesOfCopies();
     TestWindowRatesOfLists();
     TestPiecesOfLists();
     TestHeldLaunches();
