@@ -2523,8 +2523,8 @@ int XcopyEngine::SubmitDeviceTable(const void *triples, uint32_t n, int route, v
         const uint32_t m = n - at < capacity ? n - at : capacity;
         const bool last = m == n - at;
         err = mfk_xcopy_direct(static_cast<const uint64_t *>(triples) + 3ull * at, m, units, route, DeviceTableGrid(m, cu, route, tuning_),
-                               DeviceTableRestGrid(cu, route, tuning_), list, capacity, hold, holdMore, windows, last ? mask : nullptr,
-                               maskValue, stream, last ? event : nullptr);
+                               DeviceTableRestGrid(cu, route, tuning_), list, capacity, windows, last ? mask : nullptr, maskValue, stream,
+                               last ? event : nullptr);
         g_launches.fetch_add(err == 0 ? 2 : 0, std::memory_order_relaxed);
         at += m;
     }

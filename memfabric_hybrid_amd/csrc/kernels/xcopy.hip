@@ -2286,8 +2286,7 @@ extern "C" int mfk_xcopy_table(const void *tablePlan, int route, uint32_t grid, 
 
 // rest: a RestList with room for `capacity` segments, its counts 0.
 extern "C" int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *rest,
-                                uint32_t capacity, uint32_t holdNanos, uint32_t holdMoreNanos, uint32_t windowMBps, void *mask, uint32_t maskValue,
-                                void *stream, void *event)
+                                uint32_t capacity, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream, void *event)
 {
     using namespace mf;
     if (nseg == 0 || nseg > capacity || grid == 0 || restGrid == 0 || rest == nullptr) {
@@ -2296,7 +2295,7 @@ extern "C" int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t uni
     hipStream_t s = static_cast<hipStream_t>(stream);
     // (grid: the waves that are paced have to be there)
     const bool sampled = windowMBps != 0 && route == MFRT_ROUTE_HBM && nseg > kPlannedSegments && grid >= kHeldMaxPieces;
-    const TablePace pace = sampled ? PaceOf(holdNanos, holdMoreNanos, windowMBps, true) : TablePace{};
+    const TablePace pace = sampled ? PaceOf(0, 0, windowMBps, true) : TablePace{};
     const int err = WithPolicy(PolicyOf(route), [&](auto ntLoad, auto store) {
         return LaunchDirect<decltype(ntLoad)::value, decltype(store)::value>(static_cast<const uint64_t *>(triples), nseg, units, grid, restGrid,
                                                                              LanesFor(units, route), static_cast<RestList *>(rest), capacity, s,
@@ -2588,8 +2587,8 @@ extern "C" int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32
     if (guarded && g_staticUsed[dev] && g_staticLast[dev] != s && hipStreamWaitEvent(s, g_staticDone[dev], 0) != hipSuccess) {
         return static_cast<int>(hipGetLastError());
     }
-    const int err = mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, g_scratchOf[dev], kStaticRestCapacity, 0, 0, 0, nullptr, 0,
-                                     stream, nullptr);
+    const int err = mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, g_scratchOf[dev], kStaticRestCapacity, 0, nullptr, 0, stream,
+                                     nullptr);
     if (guarded && hipEventRecord(g_staticDone[dev], s) == hipSuccess) {
         g_staticLast[dev] = s;
         g_staticUsed[dev] = true;

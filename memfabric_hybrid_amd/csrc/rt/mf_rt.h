@@ -125,11 +125,10 @@ int mfk_xcopy_signal(void *word, uint32_t value, void *stream);
 /* A triple table in device memory, copied without a plan (kernels/xcopy_plan.h says how): `grid` workgroups walk its segments,
  * `restGrid` those of the second launch what is left of the long segments that the first has listed in `rest`, a mf::RestList in
  * device memory with room for `capacity` segments whose counts are 0 before and after.  One call at a time may use a list.
- * event: as for mfk_xcopy_pieces; NULL on a stream that records a graph.  windowMBps and the waits: as for mfk_xcopy_planned, for tables
- * between HBM addresses whose first segments have one length; 0: they go as all others. */
+ * event: as for mfk_xcopy_pieces; NULL on a stream that records a graph.  windowMBps: as for mfk_xcopy_planned, for longer tables
+ * between HBM addresses whose segments, as far as they are looked at, are pages of one length; 0: they go as all others. */
 int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *rest,
-                     uint32_t capacity, uint32_t holdNanos, uint32_t holdMoreNanos, uint32_t windowMBps, void *mask, uint32_t maskValue,
-                     void *stream, void *event);
+                     uint32_t capacity, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream, void *event);
 /* A triple table in device memory of up to kPlannedSegments (kernels/xcopy_plan.h) segments between HBM addresses, in one launch that
  * reads and plans it.  Waves that are resident together hold their stores for holdNanos and holdMoreNanos per 64 MiB; what is more goes
  * in read and write windows cut for `windowMBps`.  0: not held, no windows. */

@@ -24,9 +24,10 @@ std::mutex g_lock;
 std::map<uint64_t, std::pair<uint64_t, int>> g_allocs;  // base -> (size, kind)
 int g_device = -1;
 std::atomic<uint64_t> g_launches{0};   // launches may come from the engine's submit threads
-std::atomic<uint32_t> g_lastHold{0};
+std::atomic<uint32_t> g_lastHold{0};   // holdNanos of the latest inline launch
 uint32_t g_lastReading = 0;  // read part of the latest windowed list
-uint32_t g_lastWindow = 0;   // rate of the latest windowed launch, cleared by fake_rt_last_window()     // holdNanos of the latest inline launch
+uint32_t g_lastWindow = 0;   // rate of the latest windowed launch, cleared by fake_rt_last_window()
+uint32_t g_lastTableWindow = 0;   // rate handed to the latest launch of a long device table
 std::atomic<uint64_t> g_chunksRun{0};
 bool g_skipCopies = false;       // launches count and check their plans but move nothing (tables of segments no test can back with memory)
 uint32_t g_lastTableShift = 0;   // group shift of the latest table launch that used a group map, 0 under a pattern
@@ -170,6 +171,7 @@ void fake_rt_stream_state(int state) { g_streamState = state; }
 void fake_rt_fail_allocations(int on) { g_failAllocations = on != 0; }
 uint64_t fake_rt_launches(void) { return g_launches; }
 uint32_t fake_rt_last_hold(void) { return g_lastHold; }
+uint32_t fake_rt_last_table_window(void) { return g_lastTableWindow; }
 uint32_t fake_rt_last_reading(void) { return g_lastReading; }
 uint32_t fake_rt_last_window(void) { const uint32_t w = g_lastWindow; g_lastWindow = 0; return w; }
 // The next n xcopy launches fail with a runtime error code instead of running.
@@ -522,12 +524,13 @@ int mfk_xcopy_pieces_reported(const void *pieces, uint32_t count, uint64_t bytes
 // The direct copy of a device-resident table restated: the parts of every segment, and the pieces of what long ones have left out
 // of a list.
 int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int, uint32_t grid, uint32_t restGrid, void *rest,
-                     uint32_t capacity, uint32_t, uint32_t, uint32_t, void *mask, uint32_t maskValue, void *stream, void *event)
+                     uint32_t capacity, uint32_t windowMBps, void *mask, uint32_t maskValue, void *stream, void *event)
 {
     if (event != nullptr) {
         (void)mfrt_event_record(event, stream);
     }
     g_lastRestList = rest;
+    g_lastTableWindow = windowMBps;
     mf::RestList *list = static_cast<mf::RestList *>(rest);
     if (nseg == 0 || nseg > capacity || grid == 0 || restGrid == 0 || list == nullptr || list->taken != 0 || list->done[0].count != 0) {
         return -1;
@@ -627,7 +630,7 @@ int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, i
     if (nseg == 0 || nseg > MFK_STATIC_TABLE_SEGMENTS) {
         return -1;
     }
-    return mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, list.data(), MFK_STATIC_TABLE_SEGMENTS, 0, 0, 0, nullptr, 0, stream, nullptr);
+    return mfk_xcopy_direct(triples, nseg, units, route, grid, restGrid, list.data(), MFK_STATIC_TABLE_SEGMENTS, 0, nullptr, 0, stream, nullptr);
 }
 
 static uint32_t g_lastRectMates = 0;

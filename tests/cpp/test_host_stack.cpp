@@ -34,6 +34,7 @@ extern "C" uint64_t fake_rt_signals(void);
 extern "C" uint64_t fake_rt_stream_syncs(void);
 extern "C" uint32_t fake_rt_last_window(void);
 extern "C" uint32_t fake_rt_last_reading(void);
+extern "C" uint32_t fake_rt_last_table_window(void);
 extern "C" void fake_rt_seal(void);
 extern "C" void fake_rt_fail_launches(int n);
 #include "../../include/mf_hip_copy_extend.h"
@@ -1652,6 +1653,43 @@ static void TestRecordedCalls()
             same = same && std::memcmp(to, reinterpret_cast<void *>(rows[3 * i]), rows[3 * i + 2]) == 0 && to[rows[3 * i + 2]] == 0;
         }
         CHECK(same);
+    }
+    {
+        // Which long tables may go in windows: those between HBM addresses of one submitter, unless windows are off or a launch has been shaped by hand.
+        const uint32_t n = kPlannedSegments + 1;
+        std::vector<uint64_t> rows(3ull * n);
+        for (uint32_t i = 0; i < n; ++i) {
+            rows[3 * i] = reinterpret_cast<uint64_t>(a) + 64 * i;
+            rows[3 * i + 1] = reinterpret_cast<uint64_t>(b) + 64 * i;
+            rows[3 * i + 2] = 64;
+        }
+        const auto rateOf = [&](int route, bool isStatic) {
+            CHECK((isStatic ? mf_xcopy_device_table_static(rows.data(), n, route, stream) : mf_xcopy_device_table(rows.data(), n, route, stream)) == BM_OK);
+            return fake_rt_last_table_window();
+        };
+        const uint32_t rate = XcopyTuning{}.windowMBps / 17 * 15;
+        CHECK(rateOf(MF_ROUTE_HBM, false) == rate);
+        CHECK(rateOf(MF_ROUTE_HBM, true) == 0 && rateOf(MF_ROUTE_TO_HOST, false) == 0 && rateOf(MF_ROUTE_FROM_HOST, false) == 0);
+        CHECK(mf_xcopy_windows(0) == BM_OK && rateOf(MF_ROUTE_HBM, false) == 0);
+        CHECK(mf_xcopy_windows(3400000) == BM_OK && rateOf(MF_ROUTE_HBM, false) == rate / 2);
+        CHECK(mf_xcopy_windows(MF_XCOPY_WINDOWS_OWN_CHOICE) == BM_OK);
+        CHECK(mf_xcopy_tune_table(1, 256) == BM_OK && rateOf(MF_ROUTE_HBM, false) == 0 && mf_xcopy_tune_table(1, 0) == BM_OK);
+        CHECK(mf_xcopy_tune(256, 0, 0) == BM_OK && rateOf(MF_ROUTE_HBM, false) == 0 && mf_xcopy_tune(0, 0, 0) == BM_OK);
+        std::atomic<int> phase{0};
+        std::thread other([&] {
+            (void)mf_xcopy_thread_stream();
+            phase.store(1);
+            while (phase.load() != 2) {
+                std::this_thread::yield();
+            }
+        });
+        while (phase.load() != 1) {
+            std::this_thread::yield();
+        }
+        CHECK(rateOf(MF_ROUTE_HBM, false) == 0);
+        phase.store(2);
+        other.join();
+        CHECK(rateOf(MF_ROUTE_HBM, false) == rate);
     }
     CHECK(mfrt_device_sync() == 0);
     mfrt_stream_destroy(stream);
