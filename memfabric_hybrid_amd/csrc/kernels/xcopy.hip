@@ -1076,20 +1076,6 @@ __device__ __forceinline__ void ListRest(RestList *rest, uint32_t capacity, uint
     }
 }
 
-// A table that only the GPU can read, copied as xcopy_plan.h says: item (segment, part), parts in a row.  The launch is sized from
-// the segment count alone, so a workgroup walks the items with the grid as its stride; it fetches the next item's triple before
-// it copies the current item.  What bounds it is HBM; a launch in front of it that planned the table (chunk prefix, owner map,
-// repeating pattern) took 8 us, after which the copy was no faster: 4096 pages of 32 KiB scattered 60.0 / 52.8 us with the
-// planner / so, 16 080 pages of 8 KiB 76.7 / 57.9, 100 pages 10.0 / 7.1.
-// A ragged table has an odd number of parts: workgroups go to the eight XCDs in turn, and with an even number the first parts,
-// which every segment has, went to some and the last, which few have, to others.  In the slower / faster of the two modes that
-// the place of a pool decides, us with the planner, with an even number and so: 16 384 segments of 2 to 14 KB 87.1 / 77.5, 79.4 / 74.1,
-// 66 / 57.5; 4000 K and V blocks 139.4 / 138.1, 160 / 160, 135.5 / 135.5; 2000 of up to 70 KB 43.4 / 38.7, 40.2 / 35.4, 39.3 / 34.6 and spread over
-// 48 GiB 45.4 / 40.4, 50.5 / 46.3, 41.4 / 36.5.  16 384 of up to 262 KB are none the faster for it: 949 / 778, 967 / 774, 967 / 773.
-// Not taken: eight workgroups per segment, 1 to 7 % faster where segments have dozens of chunks, 16 080 pages of 8 KiB 24 % slower;
-// part numbers that turn from segment to segment, pages 1 % slower; the triples of 64 items at a time, one per lane, so that
-// empty items cost no wait, more registers than eight waves per SIMD have, 10 to 60 % slower on short tables; two triples ahead
-// instead of one, 16 384 segments of 2 to 14 KB 4 % slower.
 // What the first kDirectSample segments of a table say of it, and, kAcross, as many that lie across it.
 struct DirectSample {
     uint32_t parts;             // chunks of the longest of the first, up to kDirectMaxParts
@@ -1122,6 +1108,20 @@ __device__ __forceinline__ DirectSample SampleOf(const uint64_t *__restrict__ tr
     return DirectSample{parts, __ballot(len != length) == 0, length, __ballot(((src | dst | len) & (kUnitBytes - 1)) != 0) == 0};
 }
 
+// A table that only the GPU can read, copied as xcopy_plan.h says: item (segment, part), parts in a row.  The launch is sized from
+// the segment count alone, so a workgroup walks the items with the grid as its stride; it fetches the next item's triple before
+// it copies the current item.  What bounds it is HBM; a launch in front of it that planned the table (chunk prefix, owner map,
+// repeating pattern) took 8 us, after which the copy was no faster: 4096 pages of 32 KiB scattered 60.0 / 52.8 us with the
+// planner / so, 16 080 pages of 8 KiB 76.7 / 57.9, 100 pages 10.0 / 7.1.
+// A ragged table has an odd number of parts: workgroups go to the eight XCDs in turn, and with an even number the first parts,
+// which every segment has, went to some and the last, which few have, to others.  In the slower / faster of the two modes that
+// the place of a pool decides, us with the planner, with an even number and so: 16 384 segments of 2 to 14 KB 87.1 / 77.5, 79.4 / 74.1,
+// 66 / 57.5; 4000 K and V blocks 139.4 / 138.1, 160 / 160, 135.5 / 135.5; 2000 of up to 70 KB 43.4 / 38.7, 40.2 / 35.4, 39.3 / 34.6 and spread over
+// 48 GiB 45.4 / 40.4, 50.5 / 46.3, 41.4 / 36.5.  16 384 of up to 262 KB are none the faster for it: 949 / 778, 967 / 774, 967 / 773.
+// Not taken: eight workgroups per segment, 1 to 7 % faster where segments have dozens of chunks, 16 080 pages of 8 KiB 24 % slower;
+// part numbers that turn from segment to segment, pages 1 % slower; the triples of 64 items at a time, one per lane, so that
+// empty items cost no wait, more registers than eight waves per SIMD have, 10 to 60 % slower on short tables; two triples ahead
+// instead of one, 16 384 segments of 2 to 14 KB 4 % slower.
 template <bool kNtLoad, int kStore>
 __device__ __forceinline__ void CopyDirect(const uint64_t *__restrict__ triples, uint32_t nseg, uint32_t units, RestList *__restrict__ rest,
                                            uint32_t capacity, uint32_t parts)
@@ -1229,16 +1229,18 @@ __device__ __forceinline__ void CopyPartWindowed(const uint64_t (&src)[4], const
 // The same for tables of more than kPlannedSegments between HBM addresses, one wave a workgroup.  Where the sampled segments are pages of one
 // length, whole chunks of 16 KiB or a half or a quarter of one, and lie on units, the first waves copy all of the table in windows as those of
 // XcopyPlannedKernel do, by the rates that it has measured, and the others leave.  HBM is the bound; without windows it sees reads and writes mixed.
-// us without / so, gathered, scattered: 16 384 pages of 4 KiB 35.8 / 28.2, 37.0 / 28.7, of 8 KiB 54.2 / 48.1, 58.5 / 50.5, of 16 KiB 94.6 / 90.5,
-// 104.6 / 96.6; 9000 of 32 KiB 105.8 / 97.7, 115.1 / 104.4, of 64 KiB 214 / 191, 230 / 198; 5000 of 8 KiB 20.0 / 19.1, 20.3 / 19.8; but 4100 of 4 KiB
+// us without / so, gathered, scattered: 16 384 pages of 4 KiB 35.8 / 26.0, 37.0 / 30.9, of 8 KiB 54.2 / 46.2, 62.6 / 57.7, of 16 KiB 95.3 / 87.3,
+// - / 106.9; 9000 of 32 KiB 105.8 / 95.6, 121.7 / 115.9; 60 000 of 8 KiB - / 202; 5000 of 8 KiB 20.0 / 18.0, 20.3 / 20.0; but 4100 of 4 KiB
 // 13.5 / 13.1, 12.0 / 12.8, hence kSampledQuarters.
 // A page that is unlike those sampled takes its slot if it is shorter and lies on units, else it is listed for the second launch.  Listing costs 11 ns of
 // one word that all XCDs count on, so tables with many such pages are not for this: that is what the segments across the table are looked at for.  8192 pages of 16 KiB
 // with all sources off units, all listed / by CopyDirect() 204 / 52.8; 4096 of 8 KiB and then 4096 of 32 KiB 118 / 66.2, of 16 and 128 KiB 278 / 243; 16 384 of
-// 8 KiB with 5 % shorter 72.2 listed, 52.6 in their slots.  Not taken: CopyDirect()'s code for an unlike page where it is met (1 % of 16 384 of 16 KiB, 95.9, 131: it is
+// 8 KiB with 5 % shorter 72.2 listed, 52.6 in their slots.  Pages as sampled are copied in loops of their own, which are left for one that is not: in one loop with its
+// code 16 384 scattered pages of 8 KiB take 58.3 and not 57.7, 9000 of 32 KiB 117 and not 116.  Not taken: CopyDirect()'s code for an unlike page where it is met (1 % of 16 384 of 16 KiB, 95.9, 131: it is
 // in no instruction cache by then), and a second, longer look by the waves that stay (ones of 6144 copy what is left 4 to 18 % slower than all would).
-// Every other table pays for the look, and for six waves per SIMD where XcopyDirectKernel has eight: 16 384 segments of 2 to 14 KB 57.5 / 58.9, 8000 of 64 KiB and 8000
-// of 100 bytes 195 / 204.  (With 64 segments looked at by every wave 64.3 / 85.8.)
+// Every other table pays for the look, and for six waves per SIMD where XcopyDirectKernel has eight, and gains by a smaller grid (SubmitDeviceTable): 16 384 segments
+// of 2 to 14 KB 58.0 / 58.6, at odd addresses 64.1 / 64.0, of 2 KiB 25.6 / 23.0, 8000 of 64 KiB and 8000 of 100 bytes 214 to 216 / 217.5.  (With 64 segments looked at by
+// every wave 64.3 / 85.8.)
 // With kLongWaves instead of kWindowWaves, and what is read or written in order or lies on the grid at 6.7 instead of 6.4 and 6.6 TB/s, gathered, scattered: 9000 of
 // 16 KiB 51.9 / 51.2, 58.6 / 54.3; 4200 of 32 KiB 49.0 / 48.3, 54.7 / 50.8, 9000 97.5 / 96.3, 113.5 / 101.9; 9000 of 64 KiB 190 / 186, 196 / 188.
 // Not taken: the stores of up to 5120 waves held instead (8000 of 8 KiB 28.2 / 29.5: four workgroups a segment start, most of them only to leave, and take the
@@ -1276,80 +1278,89 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSampledWave
     const TableWindows w = WindowsOf(pace, static_cast<uint32_t>(t[0]), static_cast<uint32_t>(t[1]), len0, 64, false);
     const uint32_t period = static_cast<uint32_t>(static_cast<uint64_t>(w.ticks) * (waves * kDeepBytes) >> 26);
     const uint32_t reading = w.reading == 32 ? period / 2 : period / 64 * w.reading;
-    const uint64_t start = AgreedStart(pace.seq);
+    const uint64_t start = Uniform(AgreedStart(pace.seq));
     uint64_t loadAt = start + static_cast<uint64_t>(item) * reading / waves;
     uint64_t storeAt = start + reading + static_cast<uint64_t>(item) * (period - reading) / waves;
+    // To this wave's next item; false where it has none.
+    auto onward = [&] {
+        const bool more = items - item > waves;
+        item += more ? waves : 0;
+        loadAt += period;
+        storeAt += period;
+        return more;
+    };
+    // Copies items as seen, up to the first that is not; false: no item is left.
     auto several = [&](auto count) {
         constexpr uint32_t kParts = decltype(count)::value;
-        uint64_t src[kParts];
-        uint64_t dst[kParts];
-        bool all = true;
+        do {
+            uint64_t src[kParts];
+            uint64_t dst[kParts];
+            bool all = true;
 #pragma unroll
-        for (uint32_t j = 0; j < kParts; ++j) {
-            const uint32_t at = item * kParts + j < nseg ? item * kParts + j : nseg - 1;       // the last again rather than none
-            const uint64_t row[3] = {rows[3ull * at], rows[3ull * at + 1], rows[3ull * at + 2]};
-            src[j] = row[0];
-            dst[j] = row[1];
-            all = all && asSeen(row);
-        }
-        if (all) {
+            for (uint32_t j = 0; j < kParts; ++j) {
+                const uint32_t at = item * kParts + j < nseg ? item * kParts + j : nseg - 1;       // the last again rather than none
+                const uint64_t row[3] = {rows[3ull * at], rows[3ull * at + 1], rows[3ull * at + 2]};
+                src[j] = row[0];
+                dst[j] = row[1];
+                all = all && asSeen(row);
+            }
+            if (!all) {
+                return true;
+            }
             CopyWholeWindowed<kParts>(src, dst, loadAt, storeAt);
-        }
-        return all;
+        } while (onward());
+        return false;
     };
-    uint32_t seg = item / each;
-    uint64_t row[3] = {rows[3ull * seg], rows[3ull * seg + 1], rows[3ull * seg + 2]};
-    for (;;) {
-        uint32_t first = seg;
-        const uint32_t k = item - seg * each;
-        const bool more = items - item > waves;
-        bool all = true;
-        if (together == 1) {
-            seg = more ? (item + waves) / each : seg;
+    auto one = [&] {
+        uint32_t seg = item / each;
+        uint64_t row[3] = {rows[3ull * seg], rows[3ull * seg + 1], rows[3ull * seg + 2]};
+        for (;;) {
+            const uint32_t k = item - seg * each;
+            seg = items - item > waves ? (item + waves) / each : seg;
             const uint64_t next[3] = {rows[3ull * seg], rows[3ull * seg + 1], rows[3ull * seg + 2]};      // requested now, needed after the copy
-            all = asSeen(row);
-            if (all) {
-                CopyWholeWindowed<1>({row[0] + k * kDeepBytes}, {row[1] + k * kDeepBytes}, loadAt, storeAt);
+            if (!asSeen(row)) {
+                return true;
+            }
+            CopyWholeWindowed<1>({row[0] + k * kDeepBytes}, {row[1] + k * kDeepBytes}, loadAt, storeAt);
+            if (!onward()) {
+                return false;
             }
             row[0] = next[0];
             row[1] = next[1];
             row[2] = next[2];
-        } else {
-            first = item * together;
-            all = together == 2 ? several(std::integral_constant<uint32_t, 2>()) : several(std::integral_constant<uint32_t, 4>());
         }
-        if (!all) {
-            // a quarter of 16 KiB at a time
-            uint64_t src[4];
-            uint64_t dst[4];
-            uint32_t bytes[4];
-#pragma unroll
-            for (uint32_t q = 0; q < 4; ++q) {
-                const uint32_t at = first + q * together / 4;
-                const uint32_t begin = together == 1 ? k * kDeepBytes + q * (kDeepBytes / 4) : q * (kDeepBytes / 4) % (kDeepBytes / together);
-                const bool there = at < nseg;
-                const uint32_t r = there ? at : first;
-                const uint64_t len = there ? rows[3ull * r + 2] : 0;
-                src[q] = rows[3ull * r] + begin;
-                dst[q] = rows[3ull * r + 1] + begin;
-                const bool fits = len <= len0 && ((src[q] | dst[q]) & (kUnitBytes - 1)) == 0;
-                if (!fits && len != 0 && begin == 0) {
-                    ListRest(rest, capacity, src[q], dst[q], len);
-                }
-                const uint32_t left = fits && len > begin ? static_cast<uint32_t>(len) - begin : 0;
-                bytes[q] = left < kDeepBytes / 4 ? left : kDeepBytes / 4;
-            }
-            if ((bytes[0] | bytes[1] | bytes[2] | bytes[3]) != 0) {
-                CopyPartWindowed(src, dst, bytes, loadAt, storeAt);
-            }
-        }
-        if (!more) {
+    };
+    do {
+        const bool unlike = together == 1 ? one() : together == 2 ? several(std::integral_constant<uint32_t, 2>()) : several(std::integral_constant<uint32_t, 4>());
+        if (!unlike) {
             return;
         }
-        item += waves;
-        loadAt += period;
-        storeAt += period;
-    }
+        // a quarter of 16 KiB at a time
+        const uint32_t first = together == 1 ? item / each : item * together;
+        const uint32_t k = together == 1 ? item - first * each : 0;
+        uint64_t src[4];
+        uint64_t dst[4];
+        uint32_t bytes[4];
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            const uint32_t at = first + q * together / 4;
+            const uint32_t begin = together == 1 ? k * kDeepBytes + q * (kDeepBytes / 4) : q * (kDeepBytes / 4) % (kDeepBytes / together);
+            const bool there = at < nseg;
+            const uint32_t r = there ? at : first;
+            const uint64_t len = there ? rows[3ull * r + 2] : 0;
+            src[q] = rows[3ull * r] + begin;
+            dst[q] = rows[3ull * r + 1] + begin;
+            const bool fits = len <= len0 && ((src[q] | dst[q]) & (kUnitBytes - 1)) == 0;
+            if (!fits && len != 0 && begin == 0) {
+                ListRest(rest, capacity, src[q], dst[q], len);
+            }
+            const uint32_t left = fits && len > begin ? static_cast<uint32_t>(len) - begin : 0;
+            bytes[q] = left < kDeepBytes / 4 ? left : kDeepBytes / 4;
+        }
+        if ((bytes[0] | bytes[1] | bytes[2] | bytes[3]) != 0) {
+            CopyPartWindowed(src, dst, bytes, loadAt, storeAt);
+        }
+    } while (onward());
 }
 
 // The sum of the lanes up to and with this one.

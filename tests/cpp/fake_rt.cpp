@@ -27,7 +27,8 @@ std::atomic<uint64_t> g_launches{0};   // launches may come from the engine's su
 std::atomic<uint32_t> g_lastHold{0};   // holdNanos of the latest inline launch
 uint32_t g_lastReading = 0;  // read part of the latest windowed list
 uint32_t g_lastWindow = 0;   // rate of the latest windowed launch, cleared by fake_rt_last_window()
-uint32_t g_lastTableWindow = 0;   // rate handed to the latest launch of a long device table
+uint32_t g_lastTableWindow = 0;   // rate handed to the latest launch of a long device table, and its grid
+uint32_t g_lastTableGrid = 0;
 std::atomic<uint64_t> g_chunksRun{0};
 bool g_skipCopies = false;       // launches count and check their plans but move nothing (tables of segments no test can back with memory)
 uint32_t g_lastTableShift = 0;   // group shift of the latest table launch that used a group map, 0 under a pattern
@@ -171,6 +172,7 @@ void fake_rt_stream_state(int state) { g_streamState = state; }
 void fake_rt_fail_allocations(int on) { g_failAllocations = on != 0; }
 uint64_t fake_rt_launches(void) { return g_launches; }
 uint32_t fake_rt_last_hold(void) { return g_lastHold; }
+uint32_t fake_rt_last_table_grid(void) { return g_lastTableGrid; }
 uint32_t fake_rt_last_table_window(void) { return g_lastTableWindow; }
 uint32_t fake_rt_last_reading(void) { return g_lastReading; }
 uint32_t fake_rt_last_window(void) { const uint32_t w = g_lastWindow; g_lastWindow = 0; return w; }
@@ -531,6 +533,7 @@ int mfk_xcopy_direct(const void *triples, uint32_t nseg, uint32_t units, int, ui
     }
     g_lastRestList = rest;
     g_lastTableWindow = windowMBps;
+    g_lastTableGrid = grid;
     mf::RestList *list = static_cast<mf::RestList *>(rest);
     if (nseg == 0 || nseg > capacity || grid == 0 || restGrid == 0 || list == nullptr || list->taken != 0 || list->done[0].count != 0) {
         return -1;

@@ -35,6 +35,7 @@ extern "C" uint64_t fake_rt_stream_syncs(void);
 extern "C" uint32_t fake_rt_last_window(void);
 extern "C" uint32_t fake_rt_last_reading(void);
 extern "C" uint32_t fake_rt_last_table_window(void);
+extern "C" uint32_t fake_rt_last_table_grid(void);
 extern "C" void fake_rt_seal(void);
 extern "C" void fake_rt_fail_launches(int n);
 #include "../../include/mf_hip_copy_extend.h"
@@ -1656,9 +1657,11 @@ static void TestRecordedCalls()
     }
     {
         // Which long tables may go in windows: those between HBM addresses of one submitter, unless windows are off or a launch has been shaped by hand.
-        const uint32_t n = kPlannedSegments + 1;
-        std::vector<uint64_t> rows(3ull * n);
-        for (uint32_t i = 0; i < n; ++i) {
+        uint32_t n = kPlannedSegments + 1;
+        const uint32_t many = 60000;
+        std::vector<uint64_t> rows(3ull * many);
+        CHECK(64ull * many <= bytes);
+        for (uint32_t i = 0; i < many; ++i) {
             rows[3 * i] = reinterpret_cast<uint64_t>(a) + 64 * i;
             rows[3 * i + 1] = reinterpret_cast<uint64_t>(b) + 64 * i;
             rows[3 * i + 2] = 64;
@@ -1690,6 +1693,14 @@ static void TestRecordedCalls()
         phase.store(2);
         other.join();
         CHECK(rateOf(MF_ROUTE_HBM, false) == rate);
+        // their grid: four workgroups a segment, 192 a CU at the most, 1024 where they take no windows
+        const uint32_t cu = mfrt_cu_count();
+        for (const uint32_t segments : {kPlannedSegments + 1, 48 * cu, 48 * cu + 1, many}) {
+            n = std::max(segments, kPlannedSegments + 1);
+            CHECK(rateOf(MF_ROUTE_HBM, false) == rate && fake_rt_last_table_grid() == std::min(4 * n, 192 * cu));
+            CHECK(mf_xcopy_windows(0) == BM_OK && rateOf(MF_ROUTE_HBM, false) == 0 && fake_rt_last_table_grid() == std::min(4 * n, 1024 * cu));
+            CHECK(mf_xcopy_windows(MF_XCOPY_WINDOWS_OWN_CHOICE) == BM_OK);
+        }
     }
     CHECK(mfrt_device_sync() == 0);
     mfrt_stream_destroy(stream);
