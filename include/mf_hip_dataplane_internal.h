@@ -65,7 +65,7 @@ int32_t mf_xcopy_hold_stores(int32_t nanos);
  * Segments whose source and destination differ modulo 16 go at 35/34 of the default rate.  Rectangles of 32 MiB and more whose rows hold
  * windows go at 35/34 of the default rate where rows of whole lines lie against one another in the destination, pairs of
  * others at 69/68 and those with room between their rows at the rate itself, lists of more than 128 segments and device
- * tables at 58/68 of it up to all of it.  The call sets all three rates, rectangles take the rate that is set, and the parts are of it; 0
+ * tables at 59/68 of it up to all of it.  The call sets all three rates, rectangles take the rate that is set, and the parts are of it; 0
  * switches the form off, MF_XCOPY_WINDOWS_OWN_CHOICE brings back the rates the library chose itself (what
  * hybm_init measured, else the defaults above).  While several threads submit on streams of their own the
  * form is not used. */

@@ -1832,58 +1832,72 @@ uint32_t XcopyEngine::PieceUnits(const BatchStats &stats, uint32_t n, bool unord
     return mean <= 6144 ? kXcopyThreads : mean <= 12288 ? kDeepUnits / 2 : kDeepUnits;
 }
 
-// What 6144 waves hold goes by where the segments are and how full their pieces.  us at 5.6 / 5.8 / 6.0 / 6.2 / 6.4 / 6.6 / 6.8 / 7.0 TB/s, back to back, the same to 1 %
-// in two or three processes.
-// Written one behind the other, which leaves the rows of HBM open.  Multiples of 64 KiB, 5000 of 64 KiB - / - / - / - / 105.9 / 102.8 / 100.4 / 98.1, 16 384 344 / 334 / 332 /
-// 326, but 2100 45.7 / 44.5 / 43.3 / 45.4: 6.8.  Others of one length, 4096 of 32 KiB 44.6 / 43.5 / 42.6 / 42.6, 16 384 173.4 / 170.0 / 166.7 / 190.3, 8000 of 40 960 bytes
-// 106.6 / 104.2 / 101.6 or 118.0 / 119.3, 7000 of 73 728 173.4 / 164.3 / 160.6 / 165.5, 3000 of 100 352 101.0 / 98.4 / 95.9 / -, 4500 of 32 896 50.0 / 49.7 / 52.9 / 56.4:
-// 6.6; 16 384 of 16 KiB 87.6 / 86.1 / 92.9 / 97.2, 9000 49.1 / 47.9 / 49.2 / 51.0: 6.4 below kOrderedSteadyBytes.  Of several lengths 6.4 where they are long, as it was.
-// Elsewhere multiples of 64 KiB of one length, 12 000 of 64 KiB scattered - / - / 272 / 259 / 254.7 / 248.5 / 250.5 / 289, 8000 - / - / 179.1 / 173.4 / 173.2 / 165.0 / 162.6 / 166.6: 6.6.
-// Others by how full their pieces are.  From 95 % on, long ones 6.3 (7000 of 65 536 bytes 157.9 / 154.3 / 152.1 / 165.6 from 6.0 on, at 6.4 160 in another process, 3500 of 81 920
-// 99.4 / 96.2 / 94.0 / 97.2, 6000 of 110 776 230 / 230 / 224 / 253, K and V blocks of 128 and 16 KiB 49.2 / 47.9 / 46.7 / 48.3); from 88 % on 6.0 (4500 of 32 KiB 54.1 / 54.1 / 54.1 / 54.4 / 57.0
-// from 5.6 on, 4000 of 73 728 103.3 / 100.7 / 102.8 / 113.4 from 6.0 on, 16 384 of 16 KiB scattered at 5.9 / 6.0 95.1 / 94.1), from 85 % on, and of one length from 75 %, 5.9 (8000 of 50 000 149.7 / 145.4 /
-// 144.6 / 158.6 from 5.6 on, at 6.0 158 in another process, 8000 of 24 576 at 5.8 / 5.9 / 6.0 71.7 / 70.9 / 77.8, 3800 of 28 000 39.4 / 39.5 / 41.2); below, of one length, 5.8 from three held
-// launches' worth on (8000 of 24 000 73.0 / 70.7 / 70.9 / 77.1 from 5.6 on, 6000 of 33 333 75.8 / 74.0 / 79.7 / 81.8; in two held launches 2500 of 33 333 31.8, so 32.1; of 20 000, 61 % full, none is better
-// than none).
-// Short ones, from 88 % on, that are read one behind the other are read faster than they are written at random places, and hold 6.2 with a read part of 30 / 64 of the period (parts of 28 / 29 / 30, each at 6.1 / 6.2 / 6.3, one half at
-// 6.0: 6000 of 32 KiB scattered 67.6 / 66.7 / 66.1, 67.6 / 66.6 / 65.7, 67.6 / 66.6 / 65.7, 69.9; 9889 111 / 112 / 119, 111 / 109 / 114, 111 / 109 / 109, 112.7; 16 384 184 / 186 / 199, 183 / 182 / 192,
-// - / 181 / 182, 186; of 16 KiB 92.0 / 92.6 / 97.5, 91.9 / 91.1 / 93.0, - / 90.9 / 90.8, 94.0; at random places on
-// both sides 3700 / 4500 / 8000 of 32 KiB 44.3 / 55.0 / 94.2 with even parts at 6.0, so 47.9 / 57.2 / 96.6).  Uneven parts do nothing for the others.
-// At addresses off the lines held launches are as good or nearly (ragged ones of up to 131 072 bytes 262 MB 102.1, at 5.5 / 5.6 / 5.7 / 5.8 101.9 / 100.5 / 99.0 / 99.9; of up to
-// 101 706 169 MB 65.9, 66.7 / 66.1 / 66.4 / 67.4; of up to 60 000 240 MB 100.8, 104).
+// Rates of lists in windows of 6144 waves, in 68ths of the general rate, which is 6.8 TB/s: what holds by where the segments lie and how full their pieces
+// of 16 KiB are.  A rate is one or two steps below the one at which the list falls apart, so that a process whose memory lies badly keeps it too; one that does
+// not hold costs 8 to 12 %, a step 1.7 %.  us back to back, the mean of four to seven processes on two machines:
+//
+//                                              at   59     60     61     62     63     64     66     68    rate
+//   written one behind the other
+//     5000 of 64 KiB, at multiples of it         116.4  118.8  112.5  110.8  109.1  107.6  104.5  102.2   68
+//     5000 of 64 KiB                             116.3  120.1  112.5  110.8  109.1  107.5  104.7  102.4   66
+//     4096 of 32 KiB                              49.5   48.7   48.0   47.3   46.7   46.0   44.9   44.4   66
+//     4500 of 32 896 bytes                        55.0   54.2   53.5   52.8   52.3   51.5   50.2   50.7   66 (one process at 68: 53.0)
+//     9000 of 16 KiB                              54.7   53.8   53.0   52.4   51.6   51.0   49.8   50.1   66 (52.6)
+//     3000 of 64 to 128 KiB                      105.9  104.2  102.6  101.0   99.6   98.4   96.3   94.2   66
+//   elsewhere
+//     12 000 of 64 KiB, at multiples of it       274.1  273.6  265.0  260.7  256.9  254.0  250.2  246.0   66
+//     7000 of 64 KiB                             161.5  159.1  157.5  155.4  153.9  152.5  164.3  171.6   63
+//     6000 of 110 720 bytes                      233.1  231.3  231.4  225.6  224.3  221.6  224.3  257.6   63 (one at 66: 233.7)
+//     4000 of 73 728 bytes                       106.2  104.9  103.6  102.3  102.4  107.3  114.9  116.5   60
+//     2500 of 90 to 200 KiB                      137.6  128.7  126.7  125.2  123.8  124.6  124.6  134.8   60
+//     4308 of 68 KiB                             108.3  106.9  105.5  104.0  106.8  114.9  119.2  120.3   60
+//     16 384 of 32 KiB                           192.9  199.1  209.4  212.8  213.6  214.2  214.8  215.7   59
+//     16 384 of 16 KiB                           100.2  104.0  105.7  106.6  107.0  107.4  107.8  108.4   59
+//     8000 of 24 576 bytes                        73.2   73.0   77.2   80.4   81.4   81.4   81.5   81.6   59
+//     8000 of 24 064 bytes                        71.6   71.5   75.0   78.2   79.6   79.9   80.0   80.0   59
+//     6000 of 33 280 bytes                        73.8   73.2   75.1   78.8   80.9   81.6   81.8   82.0   59
+//   read one behind the other, a read part of 30/64 of the period
+//     16 384 of 32 KiB                           189.8  201.8  200.2  184.0  182.8  192.5  202.0  204.7   62
+//     16 384 of 16 KiB                            97.2   98.7   98.7   93.9   93.6   97.4  100.2  101.4   62
+//     8000 of 28 032 bytes                        81.9   80.8   79.7   78.6   77.8   78.5   85.4   87.4   62 (with even parts 80.7 at best)
+//     9000 of 14 080 bytes                        48.1   47.6   46.8   46.3   45.5   45.2   47.0   50.0   62 (46.9)
+//
+// Short segments that are read in order are written more slowly than they are read, hence their longer write part; it does nothing for the others.
+// Segments of one length that fill their pieces less than 75 % go in windows only where they would take three held launches (2500 of 33 333 bytes in two
+// 31.8, in windows 32.1; of 20 000 bytes, 61 % full, nothing is better than none).  At addresses off the lines held launches are as good or nearly: ragged
+// segments of up to 131 072 bytes, 262 MB, 102.1, at 5.7 TB/s 99.0; of up to 101 706, 169 MB, 65.9 and 66.4; of up to 60 000, 240 MB, 100.8 and 104.
 uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t count, uint32_t units,
                                       bool unordered, uint32_t &reading) const
 {
-    constexpr uint64_t kOrderedSteadyBytes = 24000;
-    constexpr uint64_t kUnevenBytes = 24000;
+    constexpr uint64_t kLessFullBytes = 24000;
     constexpr uint32_t kShortReading = 30;
     if (unordered || units != kDeepUnits || (stats.addressBits & (kWindowAlignBytes - 1)) != 0 ||
         !WindowsApply(stats.total, MFRT_ROUTE_HBM, kPieceWindowMinBytes)) {
         return 0;
     }
-    const uint32_t rate = tuning_.windowMBps / 68;      // of 68, what the general rate is
+    const uint32_t rate = tuning_.windowMBps / 68;
     const uint64_t mean = stats.total / n;
     const uint64_t percent = stats.total * 100 / (static_cast<uint64_t>(count) * (kDeepUnits * kUnitBytes));
     const bool equal = stats.total == stats.longest * n;
     const bool onGrid = equal && ((stats.addressBits | stats.lengthBits) & (kWindowLongBlockBytes - 1)) == 0;
     const bool longBlocks = mean >= kWindowLongBlockBytes;
     if (InOrder(dst, len, n)) {
-        return onGrid ? rate * 68 : equal && mean >= kOrderedSteadyBytes ? rate * 66 : equal || (longBlocks && percent >= 85) ? rate * 64 : 0;
+        return onGrid ? rate * 68 : equal || (longBlocks && percent >= 85) ? rate * 66 : 0;
     }
     if (onGrid) {
         return rate * 66;
     }
-    if (longBlocks && percent >= 95) {
-        return rate * 63;
+    if (percent < 85 && !(equal && (percent >= 75 || (mean >= kLessFullBytes && count > 2 * kHeldMaxPieces)))) {
+        return 0;
     }
-    if (!longBlocks && percent >= 88 && InOrder(src, len, n)) {
+    if (longBlocks) {
+        return rate * (percent >= 95 ? 63 : 60);
+    }
+    if (percent >= 85 && InOrder(src, len, n)) {
         reading = kShortReading;
         return rate * 62;
     }
-    if (percent >= 85 || (equal && percent >= 75)) {
-        return rate * (percent >= 88 ? 60 : 59);
-    }
-    return equal && mean >= kUnevenBytes && count > 2 * kHeldMaxPieces ? rate * 58 : 0;
+    return rate * 59;
 }
 
 // In how many launches, each of as many pieces as are held, a list of more goes out; 1 where one that holds nothing is as fast.  Back to back,

@@ -2279,19 +2279,20 @@ static void TestWindowRatesOfLists()
     constexpr uint64_t k = 1024;
     const uint32_t rate = XcopyTuning{}.windowMBps;
     const uint32_t part = rate / 68;
-    const uint32_t random = part * 60, readInOrder = part * 62, partRandom = part * 59, uneven = part * 58, full = part * 63, grid = part * 66, brief = part * 64, ordered = part * 66, orderedGrid = part * 68;
+    const uint32_t random = part * 59, readInOrder = part * 62, randomLong = part * 60, full = part * 63, grid = part * 66, ordered = part * 66, orderedGrid = part * 68;
     struct Form { uint32_t n; uint64_t bytes, step; bool inOrder; uint32_t rate; };
     const Form forms[] = {
         {4096, 64 * k, 64 * k, false, grid}, {2400, 128 * k, 192 * k, false, grid}, {9000, 64 * k, 64 * k, false, grid},
         {4600, 64 * k, 68 * k, false, full}, {4600, 64 * k, 64 * k + 256, false, full},        // off the grid by pages and by lines
-        {2708, 110776, 110848, false, full}, {2708, 110720, 110720, false, full}, {4308, 68 * k, 128 * k, false, partRandom}, {3662, 80 * k, 80 * k, false, full},
+        {2708, 110776, 110848, false, full}, {2708, 110720, 110720, false, full}, {4308, 68 * k, 128 * k, false, randomLong}, {3662, 80 * k, 80 * k, false, full},
+        {4308, 66 * k, 66 * k, false, randomLong}, {5000, 73728, 73728, false, randomLong},
         {4096, 64 * k, 64 * k, true, orderedGrid}, {8000, 64 * k, 64 * k, true, orderedGrid},
-        {16384, 16 * k, 16 * k, true, brief}, {8193, 32 * k, 32 * k, true, ordered},
-        {7169, 32 * k, 32 * k, true, ordered}, {7169, 16 * k, 16 * k, true, brief}, {7169, 16 * k, 16 * k, false, random},
+        {16384, 16 * k, 16 * k, true, ordered}, {8193, 32 * k, 32 * k, true, ordered},
+        {7169, 32 * k, 32 * k, true, ordered}, {7169, 16 * k, 16 * k, true, ordered}, {7169, 16 * k, 16 * k, false, random},
         {3584, 32 * k, 32 * k, false, 0}, {3585, 32 * k, 32 * k, false, random}, {1000, 110720, 110720, false, 0},    // what is held takes no windows
         {4308, 68 * k, 68 * k, true, ordered}, {3662, 80 * k, 80 * k, true, ordered},
-        {8000, 24064, 24064, true, ordered}, {8000, 23936, 23936, true, brief}, {8000, 24064, 24064, false, uneven}, {8000, 23936, 23936, false, 0},   // part-filled pieces
-        {6000, 24064, 24064, false, 0}, {6000, 50048, 50048, false, partRandom}, {6000, 40192, 40192, true, ordered}, {8000, 24576, 24576, false, partRandom},
+        {8000, 24064, 24064, true, ordered}, {8000, 23936, 23936, true, ordered}, {8000, 24064, 24064, false, random}, {8000, 23936, 23936, false, 0},   // part-filled pieces
+        {6000, 24064, 24064, false, 0}, {6000, 50048, 50048, false, random}, {6000, 40192, 40192, true, ordered}, {8000, 24576, 24576, false, random},
         {6000, 64 * k, 64 * k + 16, false, 0}, {6000, 50000, 50000, true, 0},     // off the lines
     };
     for (const Form &f : forms) {
@@ -2304,8 +2305,9 @@ static void TestWindowRatesOfLists()
             std::printf("  %u segments of %llu bytes: rate %u, expected %u\n", f.n, static_cast<unsigned long long>(f.bytes), got, f.rate);
         }
     }
-    for (const Form &f : {Form{4096, 32 * k, 32 * k, false, readInOrder}, Form{7169, 16 * k, 16 * k, false, readInOrder}, Form{4308, 68 * k, 128 * k, false, partRandom},
-                          Form{4000, 60 * k, 60 * k, false, readInOrder}, Form{4096, 64 * k, 64 * k, false, grid}}) {      // read one behind the other
+    for (const Form &f : {Form{4096, 32 * k, 32 * k, false, readInOrder}, Form{7169, 16 * k, 16 * k, false, readInOrder}, Form{4308, 68 * k, 128 * k, false, randomLong},
+                          Form{4000, 60 * k, 60 * k, false, readInOrder}, Form{8000, 28032, 28032, false, readInOrder}, Form{8000, 24576, 24576, false, random},
+                          Form{4096, 64 * k, 64 * k, false, grid}}) {      // read one behind the other
         (void)fake_rt_last_window();
         CHECK(SubmitList(f.n, f.bytes, [&](uint32_t i) { return i * f.bytes; }, [&](uint32_t i) { return (i * 5077ull % f.n) * f.step; }) == BM_OK);
         CHECK(fake_rt_last_window() == f.rate && fake_rt_last_reading() == (f.rate == readInOrder ? 30u : 0u));
@@ -2326,7 +2328,7 @@ static void TestWindowRatesOfLists()
         CHECK(XcopyEngine::Instance().Submit(s.data(), d.data(), l.data(), n, MF_ROUTE_HBM, mf_xcopy_thread_stream(), nullptr, 0) == BM_OK);
         CHECK(XcopyEngine::Instance().DrainThread() == BM_OK);
         fake_rt_piece_launches(&most, &wait);
-        CHECK(fake_rt_last_window() == (more ? random : 0) && (wait != 0) == !more && (most > kHeldMaxPieces) == more);
+        CHECK(fake_rt_last_window() == (more ? randomLong : 0) && (wait != 0) == !more && (most > kHeldMaxPieces) == more);
     }
     fake_rt_skip_copies(0);
     hybm_uninit();
