@@ -142,9 +142,9 @@ def test_ragged_batch_above_one_gib_in_read_and_write_windows(pool, lib, oracle,
 @pytest.mark.parametrize("total_mib", [130, 200, 300], ids=["130MiB", "200MiB", "300MiB"])
 def test_batches_of_some_hundred_mib_in_windows_whose_last_period_is_full(pool, lib, oracle, total_mib, layout):
     """Device-to-device batches of 130 to 300 MiB in 37 ragged segments: sizes whose chunks do not fill a whole number
-    of periods on 4096 waves, so the launch runs on fewer waves with every period full.  Segments on cache lines
-    (the higher window rate), between cache lines (the general rate) and with sources apart from their destinations
-    modulo 16 (the general rate, chunks cut on lines): what arrives equals the same slices cut on the CPU, the gaps between destinations stay."""
+    of periods on 6144 waves, so the launch runs on fewer waves with every period full.  Segments on cache lines and
+    between them (the higher window rate) and with sources apart from their destinations modulo 16 (a little above the
+    general rate): what arrives equals the same slices cut on the CPU, the gaps between destinations stay."""
     dev = pool.peer_rank_ptr(0, bm.BmMemType.DEVICE)
     host = pool.peer_rank_ptr(0, bm.BmMemType.HOST)
     span = 2 * GIB + GUARD

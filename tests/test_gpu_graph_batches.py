@@ -36,6 +36,9 @@ def _batch(kind, seed):
         lens = rng.integers(0, 150000, 300)
     elif kind == "20000 short":                              # a table beyond one of the lists for recorded calls
         lens = np.concatenate([rng.integers(0, 800, 19000), rng.integers(16385, 17000, 1000)])
+    elif kind == "5000 pages":                               # in windows, but for a few
+        lens = np.full(5000, 8192)
+        lens[1000:5000:500] = 8191
     elif kind == "4000 short":
         lens = rng.integers(0, 3000, 4000)
     else:                                                    # a table: one segment far beyond the others
@@ -53,7 +56,7 @@ def _batch(kind, seed):
 
 @pytest.mark.parametrize("form, kind", [("batch", "few, apart modulo 16"), ("batch", "128 ragged, apart"), ("batch", "129 pages"),
                                         ("batch", "300 ragged"), ("batch", "4000 short"), ("table", "300 ragged"), ("table", "one long"),
-                                        ("table", "20000 short")])
+                                        ("table", "20000 short"), ("table", "5000 pages")])
 def test_captured_and_replayed_between_plain_calls(gpu, oracle, form, kind):
     torch = pytest.importorskip("torch")
     assert torch.cuda.is_available()

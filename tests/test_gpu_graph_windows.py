@@ -21,7 +21,7 @@ def gpu(lib):
     lib.hybm_uninit()
 
 
-@pytest.mark.parametrize("layout", ["on-cache-lines", "between-cache-lines"])
+@pytest.mark.parametrize("layout", ["on-cache-lines", "between-cache-lines", "apart-modulo-16"])
 def test_windowed_copy_captured_in_a_graph_and_replayed(gpu, oracle, layout):
     torch = pytest.importorskip("torch")
     assert torch.cuda.is_available()
@@ -30,9 +30,10 @@ def test_windowed_copy_captured_in_a_graph_and_replayed(gpu, oracle, layout):
     stream = torch.cuda.Stream()
     raw = stream.cuda_stream
     shift = 0 if layout == "on-cache-lines" else 48
-    # three segments, 200 MiB in all (12 800 chunks of 16 KiB: four periods on 3200 waves), destinations in another order
+    # three segments, 200 MiB in all (12 800 chunks of 16 KiB: three periods), destinations in another order
     lens = np.array([90 * MIB, 10 * MIB + 4096, 100 * MIB - 4096], dtype=np.uint64)
-    src = np.array([shift, 100 * MIB + shift, 120 * MIB + shift], dtype=np.uint64)
+    apart = 5 if layout == "apart-modulo-16" else 0
+    src = np.array([shift + apart, 100 * MIB + shift + apart, 120 * MIB + shift + apart], dtype=np.uint64)
     dst = np.array([half + 110 * MIB + shift, half + shift, half + 10 * MIB + 8192 + shift], dtype=np.uint64)
     args = (native.u64_array(pool.ptr + src), native.u64_array(pool.ptr + dst), native.u64_array(lens), 3, native.ROUTE_HBM, raw)
     try:
