@@ -2160,12 +2160,13 @@ int XcopyEngine::SubmitOne(const uint64_t *src, const uint64_t *dst, const uint6
         const bool aligned = (addressBits & (kWindowAlignBytes - 1)) == 0;
         const bool apart = (apartBits & (kUnitBytes - 1)) != 0;
         windowed = !unordered && WindowsApply(total, route, kDeepMaxBytes + 1) && !DeepHoldApplies(total, n, route, unordered);
-        // Segments whose sources and destinations agree modulo 16 hold a higher rate, as their chunks are cut on the destinations' lines; long ones that all
-        // start on cache lines, in source and destination, the highest, and shifted ones a little more than the general one.
-        // Back to back, us, at 7.2 / 7.3 / 7.4 / 7.5 TB/s: one segment of 370 MB 110.0 / 108.8 / 107.9 / 107.0, 900 MB 269 / 266 / 264 / 262 (512 MiB at 7.6 158 to
-        // 162, 7.5 151 to 155); 128 x 9 MB 355 / 348 / 348 / 350, 128 x 2.4 MB 91.9 / 92.1 / 91.8 / 101.9; the column-parallel part of 28 layers with its rectangles
-        // 3986 / 3955 / 3952 / 3958; off a line 300 MB 89.0 / 87.7 / 87.1 / 86.1, 900 MB 271 / 269 / 262 / 262.  Shifted, at 6.8 / 7.0 / 7.2 / 7.3: 200 MB 63.4 / 62.1 / 61.0 / 61.2,
-        // 900 MB 282 / 278 / 276 / 281, 100 of 2 MB on average 35.4 / 35.2 / 36.2 / 36.8, of 4 MB 131 / 129 / 135 / 144.
+        // Segments whose sources and destinations agree modulo 16 hold a higher rate, as their chunks are cut on the destinations' lines; long
+        // ones that all start on cache lines, in source and destination, the highest, and shifted ones a little more than the general one.
+        // Back to back, us, at 7.2 / 7.3 / 7.4 / 7.5 TB/s: one segment of 370 MB 110.0 / 108.8 / 107.9 / 107.0, 900 MB 269 / 266 / 264 / 262 (512 MiB
+        // at 7.5 151 to 155, at 7.6 158 to 162); 128 x 9 MB 355 / 348 / 348 / 350, 128 x 2.4 MB 91.9 / 92.1 / 91.8 / 101.9; the column-parallel part of 28
+        // layers with its rectangles 3986 / 3955 / 3952 / 3958; off a line 300 MB 89.0 / 87.7 / 87.1 / 86.1, 900 MB 271 / 269 / 262 / 262.  Shifted, at
+        // 6.8 / 7.0 / 7.2 / 7.3: 200 MB 63.4 / 62.1 / 61.0 / 61.2, 900 MB 282 / 278 / 276 / 281, 100 of 2 MB on average 35.4 / 35.2 / 36.2 / 36.8, of 4 MB
+        // 131 / 129 / 135 / 144.
         const bool longSegments = windowed && total / n >= kWindowLongSegmentBytes;
         if (longSegments && maySlice && total >= 2 * kWindowPieceBytes) {
             // A windowed launch that loses its schedule runs the rest of its bytes at the rate without windows, and the longer
@@ -2532,10 +2533,10 @@ int XcopyEngine::SubmitDeviceTable(const void *triples, uint32_t n, int route, v
     const uint32_t cu = mfrt_cu_count();
     const uint32_t units = ChooseUnits(0, cu, route, tuning_);   // sizes are only known on the GPU
     const uint32_t capacity = recorded ? kRestGraphCapacity : kRestCapacity;
-    // Where the launch may go in windows all workgroups but those that then copy start only to look and leave, through the few places the others leave them.  us with four a
-    // segment and up to 1024 a CU / with up to 192: 16 384 pages scattered of 4 KiB 31.4 / 30.2, of 8 KiB 58.2 / 56.7, of 16 KiB 109.2 / 106.4, 16 080 segments of 2 KiB
-    // 25.8 / 22.6, of 6 KiB 50.6 / 47.4, 40 000 of up to 9 KB 86.6 / 84.2, 16 384 of 2 to 14 KB 58.0 / 58.4, at odd addresses 64.8 / 64.3, of up to 262 KB 925 / 928; with up to 128
-    // a CU 58.0 / 60.2 and 925 / 932.
+    // Where the launch may go in windows all workgroups but those that then copy start only to look and leave, through the few places
+    // the others leave them.  us with four a segment and up to 1024 a CU / with up to 192: 16 384 pages scattered of 4 KiB 31.4 / 30.2, of
+    // 8 KiB 58.2 / 56.7, of 16 KiB 109.2 / 106.4, 16 080 segments of 2 KiB 25.8 / 22.6, of 6 KiB 50.6 / 47.4, 40 000 of up to 9 KB 86.6 / 84.2,
+    // 16 384 of 2 to 14 KB 58.0 / 58.4, at odd addresses 64.8 / 64.3, of up to 262 KB 925 / 928; with up to 128 a CU 60.2 and 932.
     constexpr uint32_t kSampledPerCu = 192;
     const auto gridOf = [&](uint32_t segments) {
         const uint32_t grid = DeviceTableGrid(segments, cu, route, tuning_);

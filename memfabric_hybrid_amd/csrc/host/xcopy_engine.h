@@ -84,12 +84,15 @@ struct XcopyTuning {
     bool stageUnordered = true;  // the upload of a ragged table's descriptors is launched without a barrier
     uint32_t deviceTableWgPerCu = 0;   // grid of a device-resident table in workgroups per CU, 0 = four per segment between 16 and 1024 per CU
     uint32_t windowMBps = 6800000;   // long HBM copies alternate between read and write windows cut for this rate; 0 = never
-    // The same for launches whose sources and destinations agree modulo 16, which hold more; 0 = the rate above.  300 MB, us, at 6.8 / 7.3 TB/s: with the source 64 bytes
-    // off a cache line 91.8 / 86.0, the destination 91.8 / 86.2; 100 segments of 3 MB, 48 bytes off 92.6 / 86.8, 92.6 / 86.9.
+    // The same for launches whose sources and destinations agree modulo 16, which hold more; 0 = the rate above.  300 MB, us, at 6.8 / 7.3
+    // TB/s: with the source 64 bytes off a cache line 91.8 / 86.0, the destination 91.8 / 86.2; 100 segments of 3 MB, 48 bytes off 92.6 / 86.8,
+    // 92.6 / 86.9.
     uint32_t windowAlignedMBps = 7300000;
-    // And for those of them that all start at multiples of kWindowAlignBytes in source and destination and are kWindowLongSegmentBytes and longer on average, which hold more still; 0 = the rate above.  The highest that copies kept
-    // to in each of ten processes; us, the mean back to back at 7.3 / 7.375 / 7.45 TB/s: one segment of 512 MiB 151.9 / 151.9 / 151.2, of 1 GiB 302 / 300 / 301,
-    // in one process of four 303 / 300 / 307; waited for one by one, 512 MiB 165 / 165 / 163 to 176, 1 GiB 317 / 314 / 312.  At 7.5 one in some twenty-five saw none of six keep to it.
+    // And for those of them that all start at multiples of kWindowAlignBytes in source and destination and are kWindowLongSegmentBytes and
+    // longer on average, which hold more still; 0 = the rate above.  The highest that copies kept to in each of ten processes; us, the
+    // mean back to back at 7.3 / 7.375 / 7.45 TB/s: one segment of 512 MiB 151.9 / 151.9 / 151.2, of 1 GiB 302 / 300 / 301, in one process of
+    // four 303 / 300 / 307; waited for one by one, 512 MiB 165 / 165 / 163 to 176, 1 GiB 317 / 314 / 312.  At 7.5 one in some twenty-five saw
+    // none of six keep to it.
     uint32_t windowLongMBps = 7375000;
 };
 

@@ -342,14 +342,22 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyInlineKernel(const InlineP
 constexpr uint32_t kWindowDepth = 16;                       // 128-bit loads per lane and round
 constexpr uint32_t kWindowUnits = 64 * kWindowDepth;        // 16 KiB chunks, one wave each
 constexpr uint32_t kWindowWaves = 4096;                     // 16 per CU
-// XcopyWindowKernel's, XcopyPieceWindowKernel's and XcopySampledKernel's, 24 per CU.  A period of half as many waves again is as much longer, so a wave whose loads land late has more of it to
-// catch up in, and HBM turns round less often.  4096 / 5120 / 6144 waves, the mean of sixteen launches in pairs, us: 128 x 9 MB at 7.1 TB/s 359 / 355 / 346, at
-// 7.4 377 / 357 / 351; 128 x 2.4 MB at 7.4 102 / 93 / 90; 170 MiB at 7.6 56.4 / 55.8 / 52.2; shifted, 512 MiB at 7.1 164 / 168 / 161.  7168 waves are as many as there
-// are registers for the data of, and spill what else they need (170 MiB at 7.6 52.5).  The read and the write part as long as each other: 47 and 53 % of the period for reads are
-// no better; nor are parts that issue in 95 or 90 % of their time and leave the rest for stragglers (128 x 9 MB at 7.2 346, 379, at 100 % 348).
+// XcopyWindowKernel's, XcopyPieceWindowKernel's and XcopySampledKernel's, 24 per CU.  A period of half as many waves again is as much
+// longer, so a wave whose loads land late has more of it to catch up in, and HBM turns round less often.  The mean of sixteen launches in
+// pairs, us:
+//                                        waves   4096   5120   6144
+//   128 segments of 9 MB at 7.1 TB/s              359    355    346
+//   the same at 7.4                               377    357    351
+//   128 of 2.4 MB at 7.4                          102     93     90
+//   170 MiB at 7.6                               56.4   55.8   52.2
+//   512 MiB shifted at 7.1                        164    168    161
+// 7168 waves are as many as there are registers for the data of, and spill what else they need (170 MiB at 7.6 52.5).  The read and the
+// write part as long as each other: 47 and 53 % of the period for reads are no better; nor are parts that issue in 95 or 90 % of their
+// time and leave the rest for stragglers (128 segments of 9 MB at 7.2 346 and 379, at 100 % 348).
 constexpr uint32_t kLongWavesPerSimd = 6;
 constexpr uint32_t kLongWaves = 6144;
-static_assert(kLongWaves <= kHeldMaxPieces && kLongWaves % kPieceGroup == 0, "a round of pieces is whole groups, and a table of more than kPlannedSegments has a workgroup for each wave");
+static_assert(kLongWaves <= kHeldMaxPieces && kLongWaves % kPieceGroup == 0,
+              "a round of pieces is whole groups, and a table of more than kPlannedSegments has a workgroup for each wave");
 
 // Chunk c of a segment; with onLines one of LineChunks(), as a segment of its own.
 struct SegChunk {
@@ -970,13 +978,18 @@ struct SharedRows {
     }
 };
 
-// The inline plan in chunks of LineChunks(), whatever source and destination are modulo 16, in windows: single-wave workgroups walk the chunks
-// with stride gridDim.x, one per period each, as XcopyPieceHeldKernel copies a piece, so that a chunk that is not whole, or whose bytes are shifted, keeps to the windows too.
-// HBM is the bound.  us back to back, 4096 waves that keep the table in registers, cut for 7.1 (one segment on lines 7.4, shifted 6.8) TB/s / this, cut for 7.3 (7.45, 7.0):
-// one segment on lines of 136 / 370 / 900 MB 39.3 / 39.3, 104.8 / 103.7, 257.2 / 253.7; off a line 300 / 700 MB 90.6 / 85.3, 210 / 197; shifted 200 MB 63.1 / 60.5;
-// 128 of 2.4 / 9 MB 92.4 / 88.5, 337 / 326; reshards with their rectangles, 13 layers of 1280 548 / 533, 28 of 3584 3873 / 3831.
-// Beside eight elementwise kernels of another stream over 1 GiB, both together, 18 of 512 MiB 6333 / 6341, 31 of 128 x 2.4 MB 6485 / 6337; beside products of
-// matrices 3412 / 3478, 3495 / 3475.
+// The inline plan in chunks of LineChunks(), whatever source and destination are modulo 16, in windows: single-wave workgroups walk the
+// chunks with stride gridDim.x, one per period each, as XcopyPieceHeldKernel copies a piece, so that a chunk that is not whole, or whose
+// bytes are shifted, keeps to the windows too.  HBM is the bound.  us back to back, the mean of two processes, 4096 waves that keep the
+// table in registers and are cut for 7.1 TB/s (one segment on lines 7.4, shifted 6.8) / this, cut for 7.3 (7.375, 7.0):
+//   one segment on lines   136 MB 42.6 / 40.7, 370 MB 107.6 / 104.9, 512 MiB 154 / 151, 900 MB 281 / 254, 1 GiB 310 / 302
+//   off a line             300 MB 93.1 / 86.0, 700 MB 213 / 198, 1 GiB 323 / 303
+//   shifted                200 MB 65.7 / 61.2
+//   128 segments           of 2.4 MB 96.9 / 88.8, of 9 MB 338 / 327
+//   reshards with their rectangles   13 layers of 1280 548 / 533, 28 of 3584 3873 / 3831
+// Beside elementwise kernels of another stream over 1 GiB, both together, 18 of 512 MiB 6333 / 6341, 31 of 128 x 2.4 MB 6485 / 6337; over
+// 256 MB 13 of 512 MiB 4358 / 4288, 46 of 128 x 1 MB 3842 / 4048, 20 shifted of 300 MB 3700 / 3863; beside products of matrices the
+// same three 3643 / 3658, 3704 / 3466, 3513 / 3450.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kLongWavesPerSimd, kLongWavesPerSimd))) void XcopyWindowKernel(
     const InlinePlan p, uint32_t period, uint32_t seq)
 {
@@ -1008,14 +1021,18 @@ __global__ __launch_bounds__(64) void XcopyPieceDoneKernel(uint64_t list, uint32
     MarkDone(DoneMark{Buffer<uint64_t>(word), Buffer<uint32_t>(counter), value, count}, at);
 }
 
-// Pieces of kWindowUnits units in read and write windows, as XcopyWindowKernel walks chunks, each copied as XcopyPieceHeldKernel copies it; every
-// piece of the list begins on a cache line in source and destination.  A wave fetches a descriptor across the link when it has issued its stores and has half a period for it.
-// Bound: HBM, whose rows a random place opens for 256 bytes a channel, so the rate that holds is lower than that of long segments.
-// Back to back, us, held launches or 4096 waves at the rates those held / 6144 waves at theirs (PieceWindowRate), the same in two processes each.  Gathered 4096 / 8000 / 16 384
-// pages of 32 KiB 45.7 / 43.5, 90.8 / 83.3, 183 / 170, 16 384 of 16 KiB 92.6 / 87.5, 4900 of 24 064 bytes 43.0 / 39.1, 12 000 of 64 KiB 254 / 240; scattered 2500 / 12 000 of 64 KiB
-// 55.0 / 52.7, 258 / 249, and with a shorter read part (PieceWindowRate) 4096 / 6000 / 16 384 of 32 KiB 47.8 / 46.3, 69.8 / 67.1, 189 / 186, 9000 / 16 384 of 16 KiB 52.6 / 51.1, 95.5 / 92.4.  At random places on both sides 8000 of 50 000 bytes 160 / 148, 6000 of 73 728 174 / 154, 3500 of 81 920 100.1 /
-// 95.7, 6000 of 110 776 234 / 224, K and V blocks of 128 and 16 KiB, 144 MB, 51.0 / 48.7.
-// Beside eight elementwise kernels of another stream over 1 GiB, both together, 37 x 8000 pages of 32 KiB 6159 / 6231, beside products of matrices 3992 / 3750.
+// Pieces of kWindowUnits units in read and write windows, as XcopyWindowKernel walks chunks, each copied as XcopyPieceHeldKernel copies it;
+// every piece of the list begins on a cache line in source and destination.  A wave fetches a descriptor across the link when it has
+// issued its stores and has half a period for it.  Bound: HBM, whose rows a random place opens for 256 bytes a channel, so the rate that
+// holds is lower than that of long segments.  us back to back, held launches or 4096 waves at the rates those held / 6144 waves at
+// theirs (PieceWindowRate), two processes each:
+//   gathered    pages of 32 KiB, 4096 49.3 / 44.7, 16 384 185 / 171; 16 384 of 16 KiB 95.0 / 87.0; 12 000 of 20 KiB 85.7 / 80.5
+//   scattered   pages of 32 KiB, 4096 48.7 / 47.1, 16 384 186 / 180; 16 384 of 16 KiB 95.8 / 93.0; 12 000 of 64 KiB 255 / 245
+//   at random places on both sides   8000 of 50 048 bytes 158 / 142, 3500 of 81 920 100.0 / 95.5, 6000 of 110 720 230 / 218,
+//               16 384 of 32 KiB 213 / 190, K and V blocks of 128 and 16 KiB, 72 MB, 53.0 / 50.6; 3800 of 28 032 39.9 / 40.6
+// Beside elementwise kernels of another stream over 1 GiB, both together, 37 x 8000 pages of 32 KiB 6159 / 6231; over 256 MB 44 x 4096
+// scattered 3942 / 4006, gathered 3980 / 3941, 22 x 8000 gathered 3728 / 3867; beside products of matrices 3738 / 3680, 3600 / 3583,
+// 3555 / 3465.
 // (A schedule that stretches when sampled waves fall behind it was tried: it overshoots, 20 to 50 % slower than none.)
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kLongWavesPerSimd, kLongWavesPerSimd))) void XcopyPieceWindowKernel(
     uint64_t list, uint32_t count, uint32_t period, uint32_t reading, uint32_t seq, uint32_t groups, uint32_t value, uint64_t started)
@@ -1226,25 +1243,33 @@ __device__ __forceinline__ void CopyPartWindowed(const uint64_t (&src)[4], const
     }
 }
 
-// The same for tables of more than kPlannedSegments between HBM addresses, one wave a workgroup.  Where the sampled segments are pages of one
-// length, whole chunks of 16 KiB or a half or a quarter of one, and lie on units, the first waves copy all of the table in windows as those of
-// XcopyPlannedKernel do, by the rates that it has measured, and the others leave.  HBM is the bound; without windows it sees reads and writes mixed.
-// us without / so, gathered, scattered: 16 384 pages of 4 KiB 35.8 / 26.0, 37.0 / 30.9, of 8 KiB 54.2 / 46.2, 62.6 / 57.7, of 16 KiB 95.3 / 87.3,
-// - / 106.9; 9000 of 32 KiB 105.8 / 95.6, 121.7 / 115.9; 60 000 of 8 KiB - / 202; 5000 of 8 KiB 20.0 / 18.0, 20.3 / 20.0; but 4100 of 4 KiB
-// 13.5 / 13.1, 12.0 / 12.8, hence kSampledQuarters.
-// A page that is unlike those sampled takes its slot if it is shorter and lies on units, else it is listed for the second launch.  Listing costs 11 ns of
-// one word that all XCDs count on, so tables with many such pages are not for this: that is what the segments across the table are looked at for.  8192 pages of 16 KiB
-// with all sources off units, all listed / by CopyDirect() 204 / 52.8; 4096 of 8 KiB and then 4096 of 32 KiB 118 / 66.2, of 16 and 128 KiB 278 / 243; 16 384 of
-// 8 KiB with 5 % shorter 72.2 listed, 52.6 in their slots.  Pages as sampled are copied in loops of their own, which are left for one that is not: in one loop with its
-// code 16 384 scattered pages of 8 KiB take 58.3 and not 57.7, 9000 of 32 KiB 117 and not 116.  Not taken: CopyDirect()'s code for an unlike page where it is met (1 % of 16 384 of 16 KiB, 95.9, 131: it is
-// in no instruction cache by then), and a second, longer look by the waves that stay (ones of 6144 copy what is left 4 to 18 % slower than all would).
-// Every other table pays for the look, and for six waves per SIMD where XcopyDirectKernel has eight, and gains by a smaller grid (SubmitDeviceTable): 16 384 segments
-// of 2 to 14 KB 58.0 / 58.6, at odd addresses 64.1 / 64.0, of 2 KiB 25.6 / 23.0, 8000 of 64 KiB and 8000 of 100 bytes 214 to 216 / 217.5.  (With 64 segments looked at by
-// every wave 64.3 / 85.8.)
-// With kLongWaves instead of kWindowWaves, and what is read or written in order or lies on the grid at 6.7 instead of 6.4 and 6.6 TB/s, gathered, scattered: 9000 of
-// 16 KiB 51.9 / 51.2, 58.6 / 54.3; 4200 of 32 KiB 49.0 / 48.3, 54.7 / 50.8, 9000 97.5 / 96.3, 113.5 / 101.9; 9000 of 64 KiB 190 / 186, 196 / 188.
-// Not taken: the stores of up to 5120 waves held instead (8000 of 8 KiB 28.2 / 29.5: four workgroups a segment start, most of them only to leave, and take the
-// place of those that load); pages that are no whole chunks, whose code would cost the registers.
+// XcopyDirectKernel for tables of more than kPlannedSegments between HBM addresses, one wave a workgroup.  Where the sampled segments are
+// pages of one length, whole chunks of 16 KiB or a half or a quarter of one, and lie on units, the first waves copy all of the table in
+// windows as those of XcopyPlannedKernel do, by the rates that it has measured, and the others leave.  HBM is the bound; without windows
+// it sees reads and writes mixed.  us without / so:
+//               gathered                                           scattered
+//      4 KiB    16 384 35.3 / 25.8; 5000 12.5 / 12.9               16 384 38.2 / 30.8; 5000 13.1 / 13.5
+//      8 KiB    16 384 54.4 / 45.8; 5000 19.6 / 17.9               16 384 63.3 / 57.7, 60 000 226 / 201; 5000 20.8 / 19.9
+//     16 KiB    16 384 95.0 / 86.1; 9000 54.6 / 49.7               16 384 110 / 106; 9000 61.8 / 57.8
+//     32 KiB    16 384 188 / 167; 9000 105.6 / 94.0                16 384 217 / 216; 9000 121 / 115
+//     64 KiB    9000 212 / 182                                     9000 241 / 238
+// (Fewer than kSampledQuarters of 4 KiB go as all others: in windows 4100 13.1 and 12.8, without 13.5 and 12.0.)
+//
+// A page that is unlike those sampled takes its slot if it is shorter and lies on units, else it is listed for the second launch.
+// Listing costs 11 ns of one word that all XCDs count on, so tables with many such pages are not for this: that is what the segments
+// across the table are looked at for.  All listed / by CopyDirect(): 8192 pages of 16 KiB with all sources off units 204 / 52.8, 4096 of
+// 8 KiB and then 4096 of 32 KiB 118 / 66.2, of 16 and 128 KiB 278 / 243; 16 384 of 8 KiB with 5 % shorter 72.2 listed, 52.6 in their slots.
+// Pages as sampled are copied in loops of their own, which are left for one that is not: in one loop with its code 16 384 scattered pages
+// of 8 KiB take 58.3 and not 57.7, 9000 of 32 KiB 117 and not 116.
+//
+// Every other table pays for the look and for six waves per SIMD where XcopyDirectKernel has eight, and gains by a smaller grid
+// (SubmitDeviceTable): 16 384 segments of 2 to 14 KB 57.3 / 58.6, at odd addresses 63.7 / 63.7, of 2 KiB 25.4 / 23.0, 100 000 142 / 88,
+// 8000 of 64 KiB and 8000 of 100 bytes 214.5 / 217.5.
+//
+// Not taken: 64 segments looked at by every wave (16 384 of 2 to 14 KB 85.8); CopyDirect()'s code for an unlike page where it is met (1 % of
+// 16 384 of 16 KiB, 95.9, 131: it is in no instruction cache by then); a second, longer look by the waves that stay (ones of 6144 copy
+// what is left 4 to 18 % slower than all would); the look by scalar loads (sixteen rows take more scalar registers than there are); the
+// stores of up to 5120 waves held instead (8000 of 8 KiB 28.2 / 29.5); pages that are no whole chunks, whose code would cost the registers.
 constexpr uint32_t kSampledWavesPerSimd = 6;
 constexpr uint32_t kSampledQuarters = 6144;             // segments of 4 KiB, at the least
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSampledWavesPerSimd, kSampledWavesPerSimd))) void XcopySampledKernel(
