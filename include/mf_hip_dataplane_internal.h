@@ -103,8 +103,8 @@ uint32_t mf_xcopy_stream_queues(uint32_t *queues, uint32_t capacity);
 /* Table launches.  stageUnordered: 1 (default) launches the upload of a ragged table's descriptors without a
  * barrier, so that it runs while the caller's earlier copies still do; 0 orders it behind them.
  * deviceTableWgPerCu: workgroups per CU of the launch that copies a table in device memory, whose chunk
- * count only the GPU knows (0 = the default: four workgroups per segment, between 16 and 1024 per CU); each walks
- * the parts of the segments with the grid as its stride. */
+ * count only the GPU knows (0 = the default: four workgroups per segment, between 16 and 1024 per CU, up to 192 where
+ * the table may go in windows); each walks the parts of the segments with the grid as its stride. */
 int32_t mf_xcopy_tune_table(uint32_t stageUnordered, uint32_t deviceTableWgPerCu);
 /* Held stores beyond the kernel-argument form.  deepHold: 1 (default) lets batches of 24 to 64 MiB whose segments
  * average 32 KiB and more be copied in 16 KiB chunks, one single wave each with sixteen loads per lane in flight,

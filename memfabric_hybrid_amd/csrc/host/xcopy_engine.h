@@ -82,7 +82,7 @@ struct XcopyTuning {
     bool deepHold = true;        // batches of 24 to 64 MiB hold the stores of 16 KiB per wave
     int32_t holdPinnedExtraNanos = kHoldLookupExtraNanos;   // added to the rule for launches of more than kInlineSegs segments
     bool stageUnordered = true;  // the upload of a ragged table's descriptors is launched without a barrier
-    uint32_t deviceTableWgPerCu = 0;   // grid of a device-resident table in workgroups per CU, 0 = four per segment between 16 and 1024 per CU
+    uint32_t deviceTableWgPerCu = 0;   // grid of a device-resident table in workgroups per CU, 0 = four per segment between 16 and 1024 per CU, or 192 (SubmitDeviceTable)
     uint32_t windowMBps = 6800000;   // long HBM copies alternate between read and write windows cut for this rate; 0 = never
     // The same for launches whose sources and destinations agree modulo 16, which hold more; 0 = the rate above.  300 MB, us, at 6.8 / 7.3
     // TB/s: with the source 64 bytes off a cache line 91.8 / 86.0, the destination 91.8 / 86.2; 100 segments of 3 MB, 48 bytes off 92.6 / 86.8,
