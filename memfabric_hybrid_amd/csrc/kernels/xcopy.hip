@@ -1248,12 +1248,12 @@ __device__ __forceinline__ void CopyPartWindowed(const uint64_t (&src)[4], const
 // windows as those of XcopyPlannedKernel do, by the rates that it has measured, and the others leave.  HBM is the bound; without windows
 // it sees reads and writes mixed.  us without / so:
 //               gathered                                           scattered
-//      4 KiB    16 384 35.3 / 25.8; 5000 12.5 / 12.9               16 384 38.2 / 30.8; 5000 13.1 / 13.5
+//      4 KiB    16 384 35.3 / 25.8; 6140 14.8 / 12.9; 5000 12.6     16 384 38.2 / 30.8; 6140 15.3 / 14.2; 5000 12.7
+//               / 12.6; 4400 11.6 / 12.5                            / 12.6; 4400 11.6 / 12.1
 //      8 KiB    16 384 54.4 / 45.8; 5000 19.6 / 17.9               16 384 63.3 / 57.7, 60 000 226 / 201; 5000 20.8 / 19.9
 //     16 KiB    16 384 95.0 / 86.1; 9000 54.6 / 49.7               16 384 110 / 106; 9000 61.8 / 57.8
 //     32 KiB    16 384 188 / 167; 9000 105.6 / 94.0                16 384 217 / 216; 9000 121 / 115
 //     64 KiB    9000 212 / 182                                     9000 241 / 238
-// (Fewer than kSampledQuarters of 4 KiB go as all others: in windows 4100 13.1 and 12.8, without 13.5 and 12.0.)
 //
 // A page that is unlike those sampled takes its slot if it is shorter and lies on units, else it is listed for the second launch.
 // Listing costs 11 ns of one word that all XCDs count on, so tables with many such pages are not for this: that is what the segments
@@ -1271,7 +1271,6 @@ __device__ __forceinline__ void CopyPartWindowed(const uint64_t (&src)[4], const
 // what is left 4 to 18 % slower than all would); the look by scalar loads (sixteen rows take more scalar registers than there are); the
 // stores of up to 5120 waves held instead (8000 of 8 KiB 28.2 / 29.5); pages that are no whole chunks, whose code would cost the registers.
 constexpr uint32_t kSampledWavesPerSimd = 6;
-constexpr uint32_t kSampledQuarters = 6144;             // segments of 4 KiB, at the least
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSampledWavesPerSimd, kSampledWavesPerSimd))) void XcopySampledKernel(
     uint64_t table, uint32_t nseg, uint64_t list, uint32_t capacity, TablePace pace)
 {
@@ -1283,7 +1282,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSampledWave
     constexpr uint32_t kDeepBytes = kWindowUnits * kUnitBytes;
     const DirectSample seen = SampleOf<true>(triples, nseg, kXcopyThreads);
     const uint64_t len0 = seen.length;
-    const uint32_t together = len0 == kDeepBytes / 2 ? 2 : len0 == kDeepBytes / 4 && nseg >= kSampledQuarters ? 4 : 1;    // segments a wave
+    const uint32_t together = len0 == kDeepBytes / 2 ? 2 : len0 == kDeepBytes / 4 ? 4 : 1;    // segments a wave
     const uint32_t each = together != 1 ? 1 : len0 % kDeepBytes == 0 && len0 <= kSampledMostBytes ? static_cast<uint32_t>(len0) / kDeepBytes : 0;
     if (!seen.equal || !seen.aligned || each == 0) {
         CopyDirect<true, kStoreStream>(triples, nseg, kXcopyThreads, rest, capacity, seen.parts);

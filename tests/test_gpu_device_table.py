@@ -246,7 +246,7 @@ def test_longer_tables_where_a_round_of_waves_ends(gpu, count, size, odd):
 
 # What a page unlike the sampled ones becomes: its place's slot where it is shorter and begins on 16 bytes, an entry of the list elsewhere, on
 # both sides of a chunk's quarters and next to pages that are as sampled.
-@pytest.mark.parametrize("count,size", [(4097, 16384), (9001, 8192), (6145, 4096), (4200, 49152)])
+@pytest.mark.parametrize("count,size", [(4097, 16384), (9001, 8192), (4097, 4096), (6145, 4096), (4200, 49152)])
 @pytest.mark.parametrize("shifted", [False, True])
 def test_longer_tables_with_a_few_shorter_pages(gpu, count, size, shifted):
     torch = pytest.importorskip("torch")
