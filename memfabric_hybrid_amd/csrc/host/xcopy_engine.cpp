@@ -1805,8 +1805,9 @@ uint32_t XcopyEngine::HoldForPieces(const BatchStats &stats, uint32_t n, uint32_
     if (tuning_.holdCalibratedOff) {
         return 0;
     }
+    const int32_t whole = !deep ? 0 : static_cast<int32_t>(PieceWholeNanos(count, stats.total));
     const int32_t extra = tuning_.holdPinnedExtraNanos + (!byChunks && units != kXcopyThreads ? kHoldPinnedDeepExtraNanos : 0) +
-                          (deep && ((stats.addressBits & (kUnitBytes - 1)) != 0 || count <= n) ? static_cast<int32_t>(PieceWholeNanos(count, stats.total)) : 0);
+                          (count <= n ? whole : (stats.addressBits & (kUnitBytes - 1)) != 0 ? whole / 2 : 0);
     const int64_t with = static_cast<int64_t>(rule) + extra + tuning_.holdDeltaNanos;
     return with > 0 ? static_cast<uint32_t>(with) : 0;
 }

@@ -118,14 +118,14 @@ __device__ __forceinline__ u32x4 Straddle(u32x4 a, u32x4 b, uint32_t bytes)
 // A source that differs from its destination modulo 16, read in whole aligned units: loads that straddle units cost twice the cache
 // accesses (4.9 MB of ragged segments 4.7 / 3.9 us, 69 MB 30.4 / 29.2).  A wave takes kUnits * 64 consecutive ones from u0 on, of
 // those 0 ... end that hold any of the bytes, so that what a lane lacks is in the next lane's unit; `last` is what lane 63 of
-// its last unit lacks.  Up to 15 bytes beside the source are read, of units that hold some of its bytes.
+// its last unit lacks.  Up to 15 bytes beside the source are read, of units that hold some of its bytes, and none in front of unit `lead`.
 template <uint32_t kUnits>
-__device__ __forceinline__ void LoadApart(u32x4 (&v)[kUnits], u32x4 &last, uint64_t aligned, uint32_t u0, uint32_t end)
+__device__ __forceinline__ void LoadApart(u32x4 (&v)[kUnits], u32x4 &last, uint64_t aligned, uint32_t u0, uint32_t end, uint32_t lead = 0)
 {
     const uint32_t u = u0 + (threadIdx.x & 63u);
 #pragma unroll
     for (uint32_t j = 0; j < kUnits; ++j) {
-        if (u + j * 64 <= end) {
+        if (u + j * 64 - lead <= end - lead) {
             v[j] = LoadAligned(aligned + (u + j * 64) * kUnitBytes);
         }
     }
@@ -135,7 +135,7 @@ __device__ __forceinline__ void LoadApart(u32x4 (&v)[kUnits], u32x4 &last, uint6
 
 template <int kStore, uint32_t kUnits>
 __device__ __forceinline__ void StoreApart(const u32x4 (&v)[kUnits], u32x4 last, uint64_t dst, uint32_t u0, uint32_t end, uint32_t apart,
-                                           uint32_t lane = threadIdx.x & 63u)
+                                           uint32_t lane = threadIdx.x & 63u, uint32_t lead = 0)
 {
     const uint32_t u = u0 + lane;
     auto store = [&](auto words) {
@@ -148,7 +148,7 @@ __device__ __forceinline__ void StoreApart(const u32x4 (&v)[kUnits], u32x4 last,
                 next[i] = NextLane(v[j][i], __builtin_amdgcn_readfirstlane(wrap));
             }
             const u32x4 r = Straddle<decltype(words)::value>(v[j], next, apart & 3u);
-            if (u + j * 64 < end) {
+            if (u + j * 64 - lead < end - lead) {
                 StoreUnit<kStore>(dst + (u + j * 64) * kUnitBytes, r);
             }
         }
@@ -675,6 +675,17 @@ __global__ __launch_bounds__(kXcopyThreads) void XcopyTableKernel(const TablePla
     }
 }
 
+// Units of the destination's cache line in front of a piece's first one.  A piece that counts its units from the line on stores whole
+// lines with every instruction; counted from the first unit on, each instruction of a piece that begins inside a line, as a quarter to a
+// half of those of ragged segments do, ends in a line that the next one has to complete.  us back to back, counted from the first unit / from
+// the line: ragged segments of up to 70 000 bytes 35 / 70 / 95 / 140 MB 14.2 / 13.7, 27.2 / 25.7, 37.8 / 36.1, 55.9 / 53.2, of up to 128 KiB 26 / 66 /
+// 262 MB 10.7 / 10.5, 24.7 / 23.7, 101.5 / 98.2; in four waves that hold nothing 287 / 537 MB 119.7 / 117.5, 217.8 / 215.1.
+__device__ __forceinline__ uint32_t LeadUnits(uint64_t first, uint32_t body, uint32_t most)
+{
+    const uint32_t lead = static_cast<uint32_t>(first & (kLineBytes - 1)) / kUnitBytes;
+    return lead + body <= most ? lead : 0;
+}
+
 // Pieces of up to kLanes * kUnits units (xcopy_plan.h), one per workgroup.  HBM is the bound; what the form saves is everything in
 // front of the first load: descriptors are fetched in one step from the host's memory, where a table with a chunk prefix and
 // an owner map had to be moved to HBM by a launch of its own first, and no wave looks anything up.
@@ -692,8 +703,10 @@ __device__ __forceinline__ void CopyPiece(const Piece &p, uint64_t t0, uint32_t 
     const uint64_t dst = dstWord & kPieceAddress;
     const SegGeom g = SegmentGeometry(dst, PieceLength(srcWord, dstWord));
     const uint32_t body = static_cast<uint32_t>(g.body);
-    const uint64_t s = src + g.head;
-    const uint64_t d = dst + g.head;
+    const uint32_t lead = LeadUnits(dst + g.head, body, kLanes * kUnits);
+    const uint32_t units = lead + body;
+    const uint64_t s = src + g.head - lead * kUnitBytes;
+    const uint64_t d = dst + g.head - lead * kUnitBytes;
     const uint32_t tid = threadIdx.x;
     const uint32_t apart = static_cast<uint32_t>(s) & (kUnitBytes - 1);
     u32x4 v[kUnits];
@@ -713,7 +726,7 @@ __device__ __forceinline__ void CopyPiece(const Piece &p, uint64_t t0, uint32_t 
     } else if (apart == 0) {
 #pragma unroll
         for (uint32_t j = 0; j < kUnits; ++j) {
-            if (j * kLanes + tid < body) {
+            if (j * kLanes + tid - lead < body) {
                 v[j] = LoadAligned(s + (j * kLanes + tid) * kUnitBytes);
             }
         }
@@ -723,19 +736,19 @@ __device__ __forceinline__ void CopyPiece(const Piece &p, uint64_t t0, uint32_t 
         }
 #pragma unroll
         for (uint32_t j = 0; j < kUnits; ++j) {
-            if (j * kLanes + tid < body) {
+            if (j * kLanes + tid - lead < body) {
                 StoreUnit<kStore>(d + (j * kLanes + tid) * kUnitBytes, v[j]);
             }
         }
     } else if (body != 0) {
         u32x4 last;
         const uint32_t u0 = (tid >> 6) * kUnits * 64;
-        LoadApart(v, last, s - apart, u0, body);
+        LoadApart(v, last, s - apart, u0, units, lead);
         meanwhile();
         if (kHold) {
             HoldStores(t0, holdTicks);
         }
-        StoreApart<kStore>(v, last, d, u0, body, apart);
+        StoreApart<kStore>(v, last, d, u0, units, apart, tid & 63u, lead);
     } else {
         meanwhile();
     }
@@ -804,15 +817,18 @@ __global__ __launch_bounds__(kLanes) void XcopyPieceKernel(uint64_t list, uint32
 // A piece of up to kUnits * 64 units by one wave that holds all of it, in as few registers as there can be: every access is a
 // scalar base and the lane's offset, lanes past the end load the last unit, what lane 63 lacks of the unit behind its last
 // one comes by a scalar load, and the lane is hidden from the compiler, which would work all offsets out at the start.
+// Units are counted from the cache line that the piece begins in (LeadUnits).
 template <uint32_t kUnits, class F>
 __device__ __forceinline__ void CopyPieceHeld(uint64_t src, uint64_t dst, uint32_t length, uint64_t t0, uint32_t holdTicks, F meanwhile)
 {
     const SegGeom g = SegmentGeometry(dst, length);
     const uint32_t body = static_cast<uint32_t>(g.body);
     const uint32_t lane = threadIdx.x;
-    const uint64_t d = dst + g.head;
+    const uint32_t lead = LeadUnits(dst + g.head, body, kUnits * 64);
+    const uint32_t units = lead + body;
+    const uint64_t d = dst + g.head - lead * kUnitBytes;
     const uint32_t apart = static_cast<uint32_t>(src + g.head) & (kUnitBytes - 1);
-    const uint64_t s = src + g.head - apart;
+    const uint64_t s = src + g.head - apart - lead * kUnitBytes;
     auto hidden = [&] {
         uint32_t l = lane;
         asm volatile("" : "+v"(l));
@@ -845,7 +861,7 @@ __device__ __forceinline__ void CopyPieceHeld(uint64_t src, uint64_t dst, uint32
             store(j, lane, v[j]);
         }
     } else {
-        const uint32_t end = apart != 0 ? body : body - 1;      // the last unit that holds any of the bytes
+        const uint32_t end = apart != 0 ? units : units - 1;      // the last unit that holds any of the bytes
         const uint32_t behind = kUnits * 64 < end ? kUnits * 64 : end;
         const auto *lacks = reinterpret_cast<const __attribute__((address_space(4))) uint32_t *>(s + behind * kUnitBytes);
         uint32_t last[4] = {lacks[0], lacks[1], lacks[2], lacks[3]};
@@ -853,7 +869,8 @@ __device__ __forceinline__ void CopyPieceHeld(uint64_t src, uint64_t dst, uint32
         for (uint32_t j = 0; j < kUnits; ++j) {
             if (j * 64 <= end) {
                 const uint32_t u = j * 64 + hidden();
-                v[j] = load(s, u < end ? u : end);
+                const uint32_t upTo = u < end ? u : end;
+                v[j] = load(s, j == 0 && upTo < lead ? lead : upTo);
             }
         }
         asm volatile("" : "+s"(last[0]), "+s"(last[1]), "+s"(last[2]), "+s"(last[3]));
@@ -862,7 +879,7 @@ __device__ __forceinline__ void CopyPieceHeld(uint64_t src, uint64_t dst, uint32
 #pragma unroll
             for (uint32_t j = 0; j < kUnits; ++j) {
                 const uint32_t l = hidden();
-                if (j * 64 + l < body) {
+                if (j * 64 + l - lead < body) {
                     store(j, l, v[j]);
                 }
             }
@@ -878,7 +895,7 @@ __device__ __forceinline__ void CopyPieceHeld(uint64_t src, uint64_t dst, uint32
                     }
                     const u32x4 r = Straddle<decltype(words)::value>(v[j], next, apart & 3u);
                     const uint32_t l = hidden();
-                    if (j * 64 + l < body) {
+                    if (j * 64 + l - lead < body) {
                         store(j, l, r);
                     }
                 }

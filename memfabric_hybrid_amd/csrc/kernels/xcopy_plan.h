@@ -168,8 +168,9 @@ constexpr int32_t kHoldLookupDeepExtraNanos = 2000;
 
 // Wait of a launch of pieces of 16 KiB beyond kDeepMinBytes.  Best waits in steps of 400 ns, us: 28 / 40 / 56 / 72 / 88 / 104 MB of pages or blocks
 // gathered and scattered 4.9 / 6.4 to 6.9 / 8.9 / 11.2 / 13.5 / 15.8, a read rate of 6.9 TB/s; where segments are cut into pieces that are not full
-// 0.7 ns less for each that is missing, up to a thousand (88 MB in segments of 100 000 bytes 12.7); nothing less at odd addresses, where a piece reads lines
-// at both ends that others read too (28 / 55 / 74 / 89 MB in segments of up to 70 000 bytes 4.9 / 8.9 / 11.4 / 13.6), nor where a segment is a piece (28 /
+// 0.7 ns less for each that is missing, up to a thousand (88 MB in segments of 100 000 bytes 12.7); half as much less at odd addresses, where a piece reads
+// lines at both ends that others read too (70 MB in segments of up to 70 000 bytes 25.7 us without, 25.4 so, 66 / 92 MB of up to 128 KiB 23.7 / 23.6, 32.8 /
+// 32.5; two launches of 48 / 59 MB 36.1 / 36.4, 44.4 / 44.7), and nothing less where a segment is a piece (28 /
 // 36 MB in segments of 5120 bytes 4.5 / 5.8, 45 / 58 MB of 8 KiB 7.3 / 9.2).  400 ns more or less cost 1 to 2 %.
 inline uint32_t PieceMissing(uint32_t count, uint64_t bytes)
 {

@@ -106,6 +106,38 @@ def test_lists_of_blocks_in_windows(gpu, count, size, where):
     assert torch.equal(target.view(count, size)[torch.from_numpy(place).cuda()], source.view(2 * count, size)[torch.from_numpy(at).cuda()])
 
 
+@pytest.mark.parametrize("form", ["4 KiB", "8 KiB", "held 16 KiB", "four waves"])
+@pytest.mark.parametrize("shift", [0, 5, 16])
+def test_pieces_that_begin_inside_a_line(gpu, form, shift):
+    """Destinations at every unit of a cache line and beside it, and lengths that end a piece at its last unit, before and behind it.
+    shift: what the source is off the destination's place in its line."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(7)
+    offsets = np.array([o + b for o in range(0, 128, 16) for b in (0, 1, 8, 15)], dtype=np.int64)
+    most = {"4 KiB": 4096, "8 KiB": 8192, "held 16 KiB": 16384, "four waves": 16384}[form]
+    ends = [most - 1, most, most + 1, 2 * most + 33]
+    short = [] if form in ("8 KiB", "four waves") else [1, 16, 100, 128, 144]
+    lens = np.concatenate([np.concatenate((most - offsets + e, np.full(len(offsets), most + e))) for e in (-16, -1, 0, 1)] +
+                          [np.full(2 * len(offsets), e) for e in ends + short]).astype(np.int64)
+    at = np.tile(offsets, len(lens) // len(offsets))
+    times = {"4 KiB": 1, "8 KiB": 12, "held 16 KiB": 3, "four waves": 20}[form]
+    lens, at = np.tile(lens, times), np.tile(at, times)
+    order = rng.permutation(len(lens))
+    lens, at = lens[order], at[order]
+    steps = (at + shift + lens + 383) // 128 * 128
+    begin = np.cumsum(steps) - steps
+    size = int(steps.sum())
+    source = torch.randint(0, 256, (size,), dtype=torch.uint8, device="cuda")
+    target = torch.randint(0, 256, (size,), dtype=torch.uint8, device="cuda")
+    expect = target.clone()
+    for b, o, n in zip((begin + at).tolist(), (begin + at + shift).tolist(), lens.tolist()):
+        expect[b:b + n] = source[o:o + n]
+    torch.cuda.synchronize()
+    gpu_util.xcopy(gpu, (source.data_ptr() + begin + at + shift).astype(np.uint64), (target.data_ptr() + begin + at).astype(np.uint64),
+                   lens.astype(np.uint64), native.ROUTE_HBM)
+    assert torch.equal(target, expect)
+
+
 # Batches whose chunks are cut on the destinations' lines and go in windows: one segment just above what is held, at and beyond 128 MiB; chunks that
 # are not whole, segments shorter than one, than a unit, than a line.
 @pytest.mark.parametrize("lens", [[(112 << 20) + 1], [(112 << 20) - 127], [(128 << 20) + 77], [300000001], [(64 << 20) + 1 - 16500, 16500],
