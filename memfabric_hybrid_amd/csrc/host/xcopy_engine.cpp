@@ -1731,6 +1731,11 @@ static uint64_t DeepPiecesOf(uint64_t bytes, uint64_t over)
     return (bytes + over) / (static_cast<uint64_t>(kDeepUnits) * kUnitBytes);
 }
 
+static bool OnLines(const BatchStats &stats)
+{
+    return (stats.addressBits & (kWindowAlignBytes - 1)) == 0;
+}
+
 // Mean length from which a list of unequal segments may go in several held launches.
 constexpr uint64_t kHeldLaunchBytes = static_cast<uint64_t>(kDeepUnits) * kUnitBytes / 4 * 7;
 
@@ -1865,15 +1870,23 @@ uint32_t XcopyEngine::PieceUnits(const BatchStats &stats, uint32_t n, bool unord
 //
 // Short segments that are read in order are written more slowly than they are read, hence their longer write part; it does nothing for the others.
 // Segments of one length that fill their pieces less than 75 % go in windows only where they would take three held launches (2500 of 33 333 bytes in two
-// 31.8, in windows 32.1; of 20 000 bytes, 61 % full, nothing is better than none).  At addresses off the lines held launches are as good or nearly: ragged
-// segments of up to 131 072 bytes, 262 MB, 102.1, at 5.7 TB/s 99.0; of up to 101 706, 169 MB, 65.9 and 66.4; of up to 60 000, 240 MB, 100.8 and 104.
+// 31.8, in windows 32.1; of 20 000 bytes, 61 % full, nothing is better than none).
+// At addresses off the lines, in places without an order, 58 and, less than 85 % full, 57.  us back to back, unless held in two to four launches before / at
+//                                      before   54     56     57     58     60     62
+//     8192 of up to 70 000 bytes        117.2  114.3  112.0  108.0  110.7  117.2  118.9    (79 % full; 57 on another machine)
+//     8192 of up to 100 000             166.3  160.8  156.5     -   154.4  156.1  164.6
+//     8192 of up to 131 072             215.3  208.8  204.1     -   201.9  200.3  214.5    (195.3 on the other)
+//     8192 of up to 50 000               85.8   85.5   86.9     -    84.4   86.1   86.7    (73 %: left as it was)
+//     4000 of up to 70 000 (2 held)      53.3   56.6   55.3     -    53.7   53.7   55.9
+//     4000 of up to 131 072 (3 held)     98.5  102.5   99.6     -    98.5   94.7   92.9
+// so only those that are not held.
 uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t count, uint32_t units,
                                       bool unordered, uint32_t &reading) const
 {
     constexpr uint64_t kLessFullBytes = 24000;
     constexpr uint32_t kShortReading = 30;
-    if (unordered || units != kDeepUnits || (stats.addressBits & (kWindowAlignBytes - 1)) != 0 ||
-        !WindowsApply(stats.total, MFRT_ROUTE_HBM, kPieceWindowMinBytes)) {
+    constexpr uint64_t kOddPercent = 75;
+    if (unordered || units != kDeepUnits || !WindowsApply(stats.total, MFRT_ROUTE_HBM, kPieceWindowMinBytes)) {
         return 0;
     }
     const uint32_t rate = tuning_.windowMBps / 68;
@@ -1882,6 +1895,9 @@ uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *s
     const bool equal = stats.total == stats.longest * n;
     const bool onGrid = equal && ((stats.addressBits | stats.lengthBits) & (kWindowLongBlockBytes - 1)) == 0;
     const bool longBlocks = mean >= kWindowLongBlockBytes;
+    if (!OnLines(stats)) {
+        return count <= 2 * kHeldMaxPieces || percent < kOddPercent || InOrder(dst, len, n) || InOrder(src, len, n) ? 0 : rate * (percent >= 85 ? 58 : 57);
+    }
     if (InOrder(dst, len, n)) {
         return onGrid ? rate * 68 : equal || (longBlocks && percent >= 85) ? rate * 66 : 0;
     }
@@ -1948,8 +1964,8 @@ uint32_t XcopyEngine::HeldLaunches(const BatchStats &stats, const uint64_t *src,
     const bool odd = (stats.addressBits & (kUnitBytes - 1)) != 0;
     const bool refused = InOrder(dst, len, n) ? parts > 2 || stats.total < stats.deepPieces * kDeepBytes / 100 * 92
                                                       : parts > 2 && odd && mean < 3 * kDeepBytes;
-    if (parts > kSlots / 2 || refused || (odd && mean >= kHeldOddBytes) || PieceWindowRate(stats, src, dst, len, n, pieces, kDeepUnits, false, reading) != 0 ||
-        HoldForPieces(stats, n, pieces / parts, kDeepUnits, false) == 0) {
+    if (parts > kSlots / 2 || refused || (odd && mean >= kHeldOddBytes) ||
+        (OnLines(stats) && PieceWindowRate(stats, src, dst, len, n, pieces, kDeepUnits, false, reading) != 0) || HoldForPieces(stats, n, pieces / parts, kDeepUnits, false) == 0) {
         return 1;
     }
     return parts;

@@ -1038,9 +1038,8 @@ __global__ __launch_bounds__(64) void XcopyPieceDoneKernel(uint64_t list, uint32
     MarkDone(DoneMark{Buffer<uint64_t>(word), Buffer<uint32_t>(counter), value, count}, at);
 }
 
-// Pieces of kWindowUnits units in read and write windows, as XcopyWindowKernel walks chunks, each copied as XcopyPieceHeldKernel copies it;
-// every piece of the list begins on a cache line in source and destination.  A wave fetches a descriptor across the link when it has
-// issued its stores and has half a period for it.  Bound: HBM, whose rows a random place opens for 256 bytes a channel, so the rate that
+// Pieces of kWindowUnits units in read and write windows, as XcopyWindowKernel walks chunks, each copied as XcopyPieceHeldKernel copies it,
+// whatever its addresses.  A wave fetches a descriptor across the link when it has issued its stores and has half a period for it.  Bound: HBM, whose rows a random place opens for 256 bytes a channel, so the rate that
 // holds is lower than that of long segments.  us back to back, held launches or 4096 waves at the rates those held / 6144 waves at
 // theirs (PieceWindowRate), two processes each:
 //   gathered    pages of 32 KiB, 4096 49.3 / 44.7, 16 384 185 / 171; 16 384 of 16 KiB 95.0 / 87.0; 12 000 of 20 KiB 85.7 / 80.5

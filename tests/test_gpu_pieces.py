@@ -138,6 +138,32 @@ def test_pieces_that_begin_inside_a_line(gpu, form, shift):
     assert torch.equal(target, expect)
 
 
+@pytest.mark.parametrize("count,least,most", [(8000, 30000, 45000), (6700, 1, 131073), (4800, 93000, 98305)])
+def test_ragged_lists_at_odd_addresses_in_windows(gpu, count, least, most):
+    """Three held launches' worth of short segments, more than four of others: one launch each, pieces of every fill at every byte."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(count)
+    lens = rng.integers(least, most, count)
+    steps = lens + rng.integers(0, 300, count)
+    begin = np.cumsum(steps) - steps
+    order = rng.permutation(count)
+    size = int(steps.sum()) + 512
+    source = torch.randint(-2**63, 2**63 - 1, ((size + 7) // 8,), dtype=torch.int64, device="cuda").view(torch.uint8)
+    target = torch.zeros_like(source)
+    other = rng.permutation(count)                       # sources in another order, so neither side has one
+    src = np.empty(count, dtype=np.int64)
+    src[other] = np.cumsum(steps[other]) - steps[other]
+    expect = target.clone()
+    for b, o, n in zip(begin.tolist(), src.tolist(), lens.tolist()):
+        expect[b:b + n] = source[o:o + n]
+    torch.cuda.synchronize()
+    launches = gpu.mf_xcopy_launch_count()
+    gpu_util.xcopy(gpu, (source.data_ptr() + src[order]).astype(np.uint64), (target.data_ptr() + begin[order]).astype(np.uint64),
+                   lens[order].astype(np.uint64), native.ROUTE_HBM)
+    assert gpu.mf_xcopy_launch_count() - launches == 1
+    assert torch.equal(target, expect)
+
+
 # Batches whose chunks are cut on the destinations' lines and go in windows: one segment just above what is held, at and beyond 128 MiB; chunks that
 # are not whole, segments shorter than one, than a unit, than a line.
 @pytest.mark.parametrize("lens", [[(112 << 20) + 1], [(112 << 20) - 127], [(128 << 20) + 77], [300000001], [(64 << 20) + 1 - 16500, 16500],
