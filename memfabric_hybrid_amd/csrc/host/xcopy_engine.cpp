@@ -1738,6 +1738,8 @@ static bool OnLines(const BatchStats &stats)
 
 // Mean length from which a list of unequal segments may go in several held launches.
 constexpr uint64_t kHeldLaunchBytes = static_cast<uint64_t>(kDeepUnits) * kUnitBytes / 4 * 7;
+// Mean length of segments at odd addresses from which neither several held launches nor windows were faster.
+constexpr uint64_t kHeldOddBytes = static_cast<uint64_t>(kDeepUnits) * kUnitBytes * 24;
 
 BatchStats StatsOf(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n)
 {
@@ -1871,7 +1873,7 @@ uint32_t XcopyEngine::PieceUnits(const BatchStats &stats, uint32_t n, bool unord
 // Short segments that are read in order are written more slowly than they are read, hence their longer write part; it does nothing for the others.
 // Segments of one length that fill their pieces less than 75 % go in windows only where they would take three held launches (2500 of 33 333 bytes in two
 // 31.8, in windows 32.1; of 20 000 bytes, 61 % full, nothing is better than none).
-// At addresses off the lines, in places without an order, 58 and, less than 85 % full, 57.  us back to back, unless held in two to four launches before / at
+// At addresses off the lines, segments of several lengths in places without an order: 58 and, less than 85 % full, 57.  us back to back, before / at
 //                                      before   54     56     57     58     60     62
 //     8192 of up to 70 000 bytes        117.2  114.3  112.0  108.0  110.7  117.2  118.9    (79 % full; 57 on another machine)
 //     8192 of up to 100 000             166.3  160.8  156.5     -   154.4  156.1  164.6
@@ -1896,7 +1898,8 @@ uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *s
     const bool onGrid = equal && ((stats.addressBits | stats.lengthBits) & (kWindowLongBlockBytes - 1)) == 0;
     const bool longBlocks = mean >= kWindowLongBlockBytes;
     if (!OnLines(stats)) {
-        return count <= 2 * kHeldMaxPieces || percent < kOddPercent || InOrder(dst, len, n) || InOrder(src, len, n) ? 0 : rate * (percent >= 85 ? 58 : 57);
+        const bool holds = !equal && mean < kHeldOddBytes && count > 2 * kHeldMaxPieces && percent >= kOddPercent;
+        return holds && !InOrder(dst, len, n) && !InOrder(src, len, n) ? rate * (percent >= 85 ? 58 : 57) : 0;
     }
     if (InOrder(dst, len, n)) {
         return onGrid ? rate * 68 : equal || (longBlocks && percent >= 85) ? rate * 66 : 0;
@@ -1930,7 +1933,6 @@ uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *s
 uint32_t XcopyEngine::HeldLaunches(const BatchStats &stats, const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, bool unordered) const
 {
     constexpr uint64_t kDeepBytes = static_cast<uint64_t>(kDeepUnits) * kUnitBytes;
-    constexpr uint64_t kHeldOddBytes = 24 * kDeepBytes;
     if (unordered || tuning_.unitsOverride != 0 || !tuning_.deepHold || stats.deepPieces <= kHeldMaxPieces ||
         stats.deepPieces > kSlots / 2 * kHeldMaxPieces || stats.total < stats.deepPieces * kDeepBytes / 100 * 65) {
         return 1;
