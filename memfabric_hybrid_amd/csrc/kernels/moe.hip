@@ -677,17 +677,22 @@ __global__ __launch_bounds__(64) void MoePermuteTileKernel(const u32x4 *__restri
 // What bounds it: the chain of a launch and of its memory round trips (kernel arguments; the ids and the row, side by side; the
 // stores), not bytes, as long as the comparisons stay few: with all parts they grow with tokens * entries.  Dispatch
 // alone, with the rank launch and the permute launch / in one (both with plain stores, see below): 16 tokens of 7168 elements at
-// top-8 over 256 experts 12.0 / 4.3 us, 64: 12.3 / 4.9, 128: 13.6 / 6.1, 256: 15.3 / 9.3, 512 (4096 entries): 19.6 / 16.0, 1024: 31.8 / 35.0; 2000 tokens of 1024
-// elements at top-2 12.1 / 7.1, 4096 at top-2 14.8 / 18.6.  It ends where counting is the quicker (MoeDispatchCountKernel): at 4096 entries, and
-// at 16384 comparisons per part (2048 elements, dispatch and combine: 256 tokens at top-8 11.6 here and 12.0 there, 300 12.6 and 11.1;
-// 1000 at top-4 12.5 and 12.3).  Plain stores leave the rows in
+// top-8 over 256 experts 12.0 / 4.3 us, 64: 12.3 / 4.9, 128: 13.6 / 6.1, 256: 15.3 / 9.3; 2000 tokens of 1024 elements at top-2 12.1 / 7.1.  Then its
+// loads were put side by side: ids, the token's own ids and the row were waited for one after the other.  Dispatch / dispatch and combine, before /
+// so, 256 experts: 64 tokens of 7168 elements at top-8 4.4, 9.3 / 3.9, 8.5; 200 8.1, 13.7 / 6.7, 12.2; 400 at top-4 7.5, 13.3 / 6.5, 12.3; 1000 of 2048 at
+// top-4 over 128 6.6, 12.1 / 5.3, 10.7; 2000 of 1024 at top-2 6.4, 10.3 / 5.5, 9.4.
+// It ends where counting is the quicker (MoeDispatchCountKernel): at 4096 entries (1500 tokens of 1024 elements at top-4 7.3, 11.2 here and 5.8, 10.2 there,
+// 3000 at top-2 9.6, 14.1 and 6.9, 11.4), and at 20480 comparisons per part (at top-8 260 of 4096 elements over 8 experts 5.7, 11.2 and 6.9, 12.0, 300 of 2048 5.0,
+// 10.3 and 5.8, 10.8, 320 of 7168 9.2, 16.5 and 9.9, 17.2, but 400 11.4, 20.0 and 11.2, 19.8; at top-6 500 of 4096 7.4, 13.1 and 7.9, 13.6, but 600 9.1, 15.4 and 8.8,
+// 15.1), with more than eight slots at 16384 (128 of 4096 at top-12 5.6, 13.1 and 6.1, 12.4).  Plain stores leave the rows in
 // the caches, where the experts' kernel finds them (dispatch and combine in turn, 256 tokens of 7168 elements: 15.1 us), and up to kQuickBytes
 // nontemporal ones do not wait for the launch's end: dispatch / both with plain stores and so, 8 tokens 4.4 / 7.0, 3.9 / 6.4, 64 5.1 / 9.9, 4.5 /
 // 9.2, 160 7.7 / 12.7, 6.5 / 12.1; 300 at top-2 4.5 / 8.6, 3.5 / 8.2, 500 5.5 / 10.2, 4.3 / 10.4.
 constexpr uint32_t kSmallThreads = 256;
 constexpr uint32_t kSmallHold = 2;                      // 128-bit pieces of the row per lane: a part is 512 units at most
 constexpr uint32_t kSmallEntries = 4096;                // the largest such call
-constexpr uint32_t kSmallCompares = 16384;              // entries times slots: what a part of a token compares
+constexpr uint32_t kSmallCompares = 20480;              // entries times slots: what a part of a token compares
+constexpr uint32_t kSmallManyCompares = 16384;          // with more than eight slots
 constexpr uint32_t kSmallGroups = 256;                  // rows are cut until there are so many workgroups, one per CU
 constexpr uint32_t kSmallBatch = 4;                     // ids per lane requested together by the counting workgroup
 static_assert(kSmallEntries <= 1u << 16 && kMaxExperts <= 1u << 16, "an entry's expert and index share a word");
@@ -785,48 +790,68 @@ __global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(uint64_t
     const uint32_t part = blockIdx.x - token * parts;
     const uint32_t begin = part * perPart;
     const uint32_t end = begin + perPart < unitsPerRow ? begin + perPart : unitsPerRow;
-    const MF_GLOBAL u32x4 *src = reinterpret_cast<const MF_GLOBAL u32x4 *>(x) +
-                                 static_cast<uint64_t>(token) * unitsPerRow;
     MF_GLOBAL u32x4 *dst = reinterpret_cast<MF_GLOBAL u32x4 *>(out);
+    // An entry as one word, expert above index: what comes before the token's slots is what compares below their words.
+    // Every wave looks at a quarter of the ids, for all slots.  Loads return in the order of their requests, and a load that some path
+    // skips is waited for with all behind it: so the ids are requested in front of the row, and every lane requests the same number of
+    // loads, those past the end what is there already.  The ranks are then known when the row has come.
+    const uint32_t first = token * topK;
+    const int32_t idOfLane = topk[first + (lane < topK ? lane : 0)];
+    constexpr uint32_t kRound = 4 * kSmallThreads;
+    const uint32_t mineAt = wave * 256 + lane * 4;
+    const uint32_t lastAt = total >= 4 ? total - 4 : 0;
+    const auto idsAt = [&](uint32_t at) {
+        i32x4a id;
+        if (total >= 4) {
+            id = *reinterpret_cast<const i32x4a *>(topk + (at < lastAt ? at : lastAt));
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                id[i] = i < total ? topk[i] : -1;
+            }
+        }
+        return id;
+    };
+    i32x4a id = idsAt(mineAt);
+    i32x4a second = {-1, -1, -1, -1};
+    if (total > kRound) {
+        second = idsAt(mineAt + kRound);
+    }
+    const bool rows = perPart != 0;
+    const MF_GLOBAL u32x4 *src = reinterpret_cast<const MF_GLOBAL u32x4 *>(rows ? x + static_cast<uint64_t>(token) * unitsPerRow * sizeof(u32x4)
+                                                                                : topkAt & ~static_cast<uint64_t>(sizeof(u32x4) - 1));
+    const uint32_t lastUnit = rows ? end - 1 : 0;
     u32x4 v[kSmallHold];
 #pragma unroll
     for (uint32_t j = 0; j < kSmallHold; ++j) {
         const uint32_t u = begin + j * kSmallThreads + threadIdx.x;
-        if (u < end) {
-            v[j] = src[u];
-        }
+        v[j] = src[u < lastUnit ? u : lastUnit];
     }
-    // An entry as one word, expert above index: what comes before the token's slots is what compares below their words.
-    // Every wave looks at a quarter of the ids, for all slots.
-    const uint32_t first = token * topK;
-    const int32_t idOfLane = threadIdx.x < topK ? topk[first + threadIdx.x] : -1;
+    const uint32_t keyOfLane = lane < topK ? SmallKey(idOfLane, first + lane, experts) : 0u;
     uint32_t own[kSlots];
     uint32_t before[kSlots];
 #pragma unroll
     for (uint32_t k = 0; k < kSlots; ++k) {
-        own[k] = k < topK ? SmallKey(topk[first + k], first + k, experts) : 0u;
+        own[k] = __builtin_amdgcn_readlane(keyOfLane, k);
         before[k] = 0;
     }
-    for (uint32_t c = wave * 256; c < total; c += 4 * kSmallThreads) {
-        const uint32_t at = c + lane * 4;
-        i32x4a id = {-1, -1, -1, -1};
-        if (at + 3 < total) {
-            id = *reinterpret_cast<const i32x4a *>(topk + at);
-        } else {
-#pragma unroll
-            for (uint32_t i = 0; i < 3; ++i) {
-                if (at + i < total) {
-                    id[i] = topk[at + i];
-                }
-            }
-        }
+    const auto compare = [&](const i32x4a &ids, uint32_t at) {
+        const uint32_t from = at < lastAt ? at : lastAt;
+        const uint32_t skip = at - from;                // of these, what another lane has
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i) {
-            const uint32_t key = SmallKey(id[i], at + i, experts);
+            const uint32_t key = i >= skip ? SmallKey(ids[i], from + i, experts) : 0xFFFFFFFFu;
 #pragma unroll
             for (uint32_t k = 0; k < kSlots; ++k) {
                 before[k] += __popcll(__ballot(key < own[k]));
             }
+        }
+    };
+    compare(id, mineAt);
+    if (total > kRound) {
+        compare(second, mineAt + kRound);
+        for (uint32_t at = mineAt + 2 * kRound; at - mineAt < total; at += kRound) {
+            compare(idsAt(at), at);
         }
     }
     uint32_t mine = 0;
@@ -1396,6 +1421,12 @@ bool DispatchCounts(uint64_t entries, uint64_t moved, uint32_t topK, uint32_t ex
     return entries <= kCountEntries && moved <= CountBytes(topK, experts, lines);
 }
 
+// The dispatch in one launch that compares: where the lines lie, see MoeDispatchSmallKernel.
+bool DispatchCompares(uint64_t entries, uint32_t topK)
+{
+    return entries <= kSmallEntries && entries * topK <= (topK <= 8 ? kSmallCompares : kSmallManyCompares);
+}
+
 // Whether waves that stay and keep reads and writes apart in time combine rows of at least 256 units: from six slices per wave on (top-8, 16 800 items
 // on 4096 waves 51.4 us, one workgroup per item 50.5; 19 200 the same; 25 200 74.4 / 76.7), below which the first read part and the last write part, in
 // which the chip only reads or only writes for want of work, cost what the separation gains; and where the last-level cache does not hold the rows that
@@ -1459,7 +1490,7 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
     const uint64_t moved = rows ? (static_cast<uint64_t>(tokens) + total) * upr * 16 : 0;
     const bool lines = hidden % 64 == 0;                // rows of whole cache lines
     const bool quick = lines && moved <= (topK <= 2 ? kQuickFewBytes : kQuickBytes);
-    if (total <= kSmallEntries && total * topK <= kSmallCompares) {   // where the lines lie: see the kernel
+    if (DispatchCompares(total, topK)) {
         const uint32_t least = (upr + kSmallHold * kSmallThreads - 1) / (kSmallHold * kSmallThreads);
         const uint32_t most = (upr + 63) / 64;
         uint32_t parts = (kSmallGroups + tokens - 1) / tokens;
@@ -1684,8 +1715,7 @@ extern "C" int mfk_moe_combine(const void *rows, const void *rowOf, const void *
 extern "C" int mfk_moe_dispatch_counts(uint32_t tokens, uint32_t hidden, uint32_t topK, uint32_t experts)
 {
     const uint64_t entries = static_cast<uint64_t>(tokens) * topK;
-    const bool small = entries <= mf::kSmallEntries && entries * topK <= mf::kSmallCompares;
-    return !small && mf::DispatchCounts(entries, (entries + tokens) * (hidden / 8) * 16, topK, experts, hidden % 64 == 0) ? 1 : 0;
+    return !mf::DispatchCompares(entries, topK) && mf::DispatchCounts(entries, (entries + tokens) * (hidden / 8) * 16, topK, experts, hidden % 64 == 0) ? 1 : 0;
 }
 
 extern "C" int mfk_moe_combine_stays(uint32_t tokens, uint32_t hidden, uint32_t topK)

@@ -502,6 +502,16 @@ def test_dispatch_that_counts_in_one_launch(gpu, T, H, K, E):
             _free(bufs)
 
 
+@pytest.mark.parametrize("T,H,K,E", [
+    (1, 8, 2, 1), (1, 64, 2, 8), (1, 7168, 3, 256), (2, 1032, 2, 5), (5, 16, 1, 3),       # fewer ids than a lane's four, and a few more
+    (128, 4096, 8, 256), (129, 4096, 8, 8), (341, 520, 3, 37), (342, 520, 3, 37),         # a round of 1024 ids, and one that ends inside a vector
+    (512, 2056, 4, 64), (1025, 1024, 2, 512), (683, 136, 3, 9), (4096, 64, 1, 256), (2048, 128, 2, 8),    # rounds behind the row's loads
+    (320, 4096, 8, 256), (321, 4096, 8, 256), (568, 1024, 6, 64), (569, 1024, 6, 64), (64, 2048, 16, 256), (65, 2048, 16, 256),  # the last that compare
+])
+def test_dispatch_that_compares_in_one_launch(gpu, T, H, K, E):
+    test_dispatch_that_counts_in_one_launch(gpu, T, H, K, E)
+
+
 @pytest.mark.parametrize("T,H,K,E,counts", [
     (3250, 7168, 8, 256, True), (3251, 7168, 8, 256, False),    # at top-8, the most rows for the dispatch that counts, and a token more
     (3510, 7168, 8, 256, False), (3511, 7168, 8, 256, False), (6144, 4096, 8, 64, False),
