@@ -863,24 +863,23 @@ __global__ __launch_bounds__(kSmallThreads) void MoeDispatchSmallKernel(uint64_t
         lds[kMaxTopK * (1 + wave) + lane] = mine;
     }
     __syncthreads();
-    if (threadIdx.x < topK) {
-        uint32_t row = 0;
+    // every wave adds them up for itself, a slot a lane
+    uint32_t rowOfLane = 0;
 #pragma unroll
-        for (uint32_t w = 0; w < kSmallThreads / 64; ++w) {
-            row += lds[kMaxTopK * (1 + w) + threadIdx.x];
-        }
-        lds[threadIdx.x] = static_cast<uint32_t>(idOfLane) < experts ? row : 0xFFFFFFFFu;
+    for (uint32_t w = 0; w < kSmallThreads / 64; ++w) {
+        rowOfLane += lds[kMaxTopK * (1 + w) + (lane < kSlots ? lane : 0)];
     }
-    __syncthreads();
+    rowOfLane = static_cast<uint32_t>(idOfLane) < experts ? rowOfLane : 0xFFFFFFFFu;
     if (part == 0 && threadIdx.x < topK) {
-        const int32_t row = static_cast<int32_t>(lds[threadIdx.x]);
+        const int32_t row = static_cast<int32_t>(rowOfLane);
         rowOf[first + threadIdx.x] = row;
         if (srcOfAt != 0 && row >= 0) {
             srcOf[row] = static_cast<int32_t>(first + threadIdx.x);
         }
     }
+#pragma unroll 1
     for (uint32_t k = 0; k < topK; ++k) {
-        const uint32_t row = lds[k];
+        const uint32_t row = __builtin_amdgcn_readlane(rowOfLane, k);
         if (row != 0xFFFFFFFFu) {
 #pragma unroll
             for (uint32_t j = 0; j < kSmallHold; ++j) {
