@@ -37,8 +37,17 @@ public:
     }
 
     // The same for a set of pieces that do not overlap one another: the bytes of the set are cut
-    // into equal shares (inside a piece if need be), one for the caller and one per helper.
-    void CopySet(const Task *tasks, size_t count);
+    // into equal shares (inside a piece if need be), one for the caller and one per helper.  pastCaches: by StreamCopy() where it is shared.
+    void CopySet(const Task *tasks, size_t count, bool pastCaches = false);
+
+    // part(context) on the helper threads, where no other caller is using them, from Begin() on; what Begin() returned goes to End(), which
+    // returns when they have.  The caller does its own part in between, all of it if need be.
+    using Part = void (*)(void *context);
+    bool Begin(Part part, void *context);
+    void End(bool begun);
+
+    // memcpy past the caches, for copies whose target the CPU does not read again soon.
+    static void StreamCopy(void *dst, const void *src, size_t len);
 
     static constexpr size_t kSplitMin = 512u << 10;
     static constexpr uint32_t kWorkers = 3;
@@ -62,9 +71,12 @@ private:
         size_t count = 0;
         Cut begin;
         Cut end;
+        bool pastCaches = false;
     };
     struct Worker {
         Share share;                       // written by the caller before seq moves, read by the worker after it saw the move
+        Part part = nullptr;               // as is this: done instead of the share
+        void *context = nullptr;
         std::atomic<uint64_t> seq{0};      // shares posted
         std::atomic<uint64_t> done{0};     // shares finished
         std::atomic<bool> sleeping{false};
@@ -73,11 +85,15 @@ private:
     };
     static void Run(const Share &share);
     void Loop(Worker *worker);
+    bool HasWorkers();                 // with owner_ held
+    void Post(uint32_t worker);
+    void Join(uint32_t worker);
 
     std::mutex owner_;                 // one caller at a time hands work to the helpers
     uint32_t started_ = 0;             // workers running; guarded by owner_
     bool unavailable_ = false;         // a thread could not be started: no further attempts
     Worker workers_[kWorkers];
+    uint64_t tickets_[kWorkers] = {};  // of the shares posted last; guarded by owner_
     std::atomic<uint64_t> shared_{0};
 };
 

@@ -1386,7 +1386,7 @@ void *XcopyEngine::ThreadStream()
     return lease.stream;
 }
 
-void *XcopyEngine::ThreadBounce(uint64_t bytes)
+void *XcopyEngine::ThreadBounce(uint64_t bytes, bool *fresh)
 {
     ThreadLease &lease = t_ctx.Lease();
     if (lease.bounceBytes < bytes) {
@@ -1400,6 +1400,9 @@ void *XcopyEngine::ThreadBounce(uint64_t bytes)
         }
         lease.bounce = mfrt_alloc_host(bytes);
         lease.bounceBytes = lease.bounce != nullptr ? bytes : 0;
+        if (fresh != nullptr) {
+            *fresh = true;
+        }
     }
     return lease.bounce;
 }

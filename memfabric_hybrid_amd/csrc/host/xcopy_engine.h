@@ -187,8 +187,8 @@ public:
     static constexpr uint32_t kDeckStreams = 8;   // streams made at Start() and dealt out so that consecutive takers sit on different hardware queues
     static constexpr uint64_t kFanMaxBytes = 64ull << 20;   // larger batches gain nothing from a second queue
     // Pinned, device-mapped staging memory of the calling thread, at least `bytes` long; it lives
-    // until Stop().  NULL when it cannot be allocated.
-    void *ThreadBounce(uint64_t bytes);
+    // until Stop().  NULL when it cannot be allocated.  *fresh: whether this call has allocated it.
+    void *ThreadBounce(uint64_t bytes, bool *fresh = nullptr);
     // Wait for everything this thread enqueued on its own stream.
     int DrainThread();
     // Wait for everything queued on `stream` so far: what a blocking copy does after its launch.

@@ -144,6 +144,14 @@ int mfk_xcopy_clear_lists(void *lists, uint32_t count, uint64_t stride, void *st
 int mfk_xcopy_static_setup(void);
 int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, int route, uint32_t grid, uint32_t restGrid, void *stream);
 
+/* ---- staged copies (kernels/staging.hip) ---------------------------------- */
+/* `count` mf::StreamChunk (kernels/staging.h) in pinned host memory, chunk c between HBM and slot c % slots, of kStreamChunkBytes, of a ring
+ * in pinned host memory, where it begins `at` % kStreamLine bytes in; the launch runs while the CPU fills (toHost 0) or empties the slots.  hostWords and
+ * gpuWords: a 64-bit word per slot, kStreamWordBytes apart, in which the CPU and the GPU say base + c + 1 when they are done with chunk c
+ * there.  A workgroup that waits limitMillis for the CPU leaves, and the chunks it has left are not copied. */
+int mfk_stream_chunks(int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count, uint32_t slots,
+                      uint32_t limitMillis, void *stream);
+
 /* ---- MoE launchers (kernels/moe.hip) ---------------------------------------- */
 uint64_t mfk_moe_workspace_bytes(uint32_t tokens, uint32_t topK, uint32_t experts);
 int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens, uint32_t hidden, uint32_t topK, uint32_t experts,

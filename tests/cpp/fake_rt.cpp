@@ -10,12 +10,15 @@
 #include <cstdlib>
 #include <vector>
 #include <cstring>
+#include <chrono>
 #include <map>
 #include <mutex>
+#include <thread>
 
 #include <sys/mman.h>
 
 #include "../../memfabric_hybrid_amd/csrc/kernels/copy2d_plan.h"
+#include "../../memfabric_hybrid_amd/csrc/kernels/staging.h"
 #include "../../memfabric_hybrid_amd/csrc/kernels/xcopy_plan.h"
 #include "../../memfabric_hybrid_amd/csrc/rt/mf_rt.h"
 
@@ -50,6 +53,18 @@ void NoteRecorded(const void *stream)
 const void *g_lastRestList = nullptr;
 
 bool g_failAllocations = false;
+
+// Streamed copies run on a thread of their own; off unless a test asks for them, so that the others see copies in rounds.
+uint32_t g_streamChunks = 0;              // chunks after which such a launch leaves; 0: it cannot be launched
+std::atomic<uint32_t> g_streamsRunning{0};
+std::atomic<uint64_t> g_chunksStreamed{0};
+std::thread g_streamThread;
+void JoinStreamed()
+{
+    if (g_streamThread.joinable()) {
+        g_streamThread.join();
+    }
+}
 
 void *Track(uint64_t bytes, int kind)
 {
@@ -288,9 +303,9 @@ uint64_t fake_rt_in_flight(void)
 }
 
 extern "C" void fake_rt_count_stream_sync(void);
-int mfrt_stream_sync(void *) { Guard("mfrt_stream_sync"); Retire(~0ull); fake_rt_count_stream_sync(); return 0; }
+int mfrt_stream_sync(void *) { Guard("mfrt_stream_sync"); JoinStreamed(); Retire(~0ull); fake_rt_count_stream_sync(); return 0; }
 int mfrt_stream_capturing(void *stream) { return g_capturing != nullptr && stream == g_capturing ? 1 : 0; }
-int mfrt_stream_done(void *) { return g_streamState; }
+int mfrt_stream_done(void *) { return g_streamsRunning.load() != 0 ? 0 : g_streamState.load(); }
 int mfrt_device_sync(void) { Guard("mfrt_device_sync"); Retire(~0ull); return 0; }
 void *mfrt_event_create(void) { return calloc(1, 8); }
 int mfrt_event_destroy(void *e) { Guard("mfrt_event_destroy"); free(e); return 0; }
@@ -427,6 +442,53 @@ int mfk_xcopy_table(const void *tablePlan, int, uint32_t grid, void *mask, uint3
     if (mask != nullptr) {
         *static_cast<uint64_t *>(mask) = maskValue;
     }
+    return 0;
+}
+
+void fake_rt_stream_chunks(uint32_t most) { g_streamChunks = most; }
+uint64_t fake_rt_chunks_streamed(void) { return g_chunksStreamed.exchange(0); }
+
+// Chunk after chunk, with the words of both sides as the kernel reads and writes them.
+int mfk_stream_chunks(int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count, uint32_t slots,
+                      uint32_t limitMillis, void *)
+{
+    if (g_streamChunks == 0) {
+        return -1;
+    }
+    JoinStreamed();
+    ++g_launches;
+    ++g_streamsRunning;
+    const uint32_t most = g_streamChunks;
+    g_streamThread = std::thread([=] {
+        auto word = [](void *words, uint32_t slot) {
+            return reinterpret_cast<uint64_t *>(static_cast<uint8_t *>(words) + static_cast<uint64_t>(slot) * mf::kStreamWordBytes);
+        };
+        for (uint32_t c = 0; c < count && c < most; ++c) {
+            const mf::StreamChunk &chunk = static_cast<const mf::StreamChunk *>(chunks)[c];
+            const uint32_t slot = c % slots;
+            if (toHost == 0 || c >= slots) {
+                const uint64_t wanted = toHost != 0 ? base + c - slots + 1 : base + c + 1;
+                const auto start = std::chrono::steady_clock::now();
+                while (__atomic_load_n(word(hostWords, slot), __ATOMIC_ACQUIRE) != wanted) {
+                    if (std::chrono::steady_clock::now() - start > std::chrono::milliseconds(limitMillis)) {
+                        --g_streamsRunning;
+                        return;
+                    }
+                    std::this_thread::yield();
+                }
+            }
+            const uint64_t skip = chunk.at & (mf::kStreamLine - 1);
+            uint8_t *there = static_cast<uint8_t *>(ring) + static_cast<uint64_t>(slot) * mf::kStreamChunkBytes + skip;
+            if (chunk.len == 0 || skip + chunk.len > mf::kStreamChunkBytes) {
+                break;
+            }
+            uint8_t *at = reinterpret_cast<uint8_t *>(chunk.at);
+            std::memcpy(toHost != 0 ? there : at, toHost != 0 ? at : there, chunk.len);
+            ++g_chunksStreamed;
+            __atomic_store_n(word(gpuWords, slot), base + c + 1, __ATOMIC_RELEASE);
+        }
+        --g_streamsRunning;
+    });
     return 0;
 }
 

@@ -58,6 +58,8 @@ extern "C" void fake_rt_fail_allocations(int on);
 extern "C" void fake_rt_withhold_reports(void);
 extern "C" void fake_rt_release_reports(void);
 extern "C" void fake_rt_stream_state(int state);
+extern "C" void fake_rt_stream_chunks(uint32_t most);
+extern "C" uint64_t fake_rt_chunks_streamed(void);
 
 using namespace mf;
 using ock::mf::DataOperatorPtr;
@@ -2479,6 +2481,68 @@ static void TestHeldLaunches()
     hybm_uninit();
 }
 
+// Copies between ordinary memory and the pool while one launch runs: chunks at every byte, more than the ring has slots, several
+// segments, and a launch that leaves before it is done or cannot be made, whose copy is made in rounds.
+static void TestStreamedCopies()
+{
+    smem_bm_config_t cfg;
+    smem_bm_config_init(&cfg);
+    CHECK(smem_bm_init("tcp://127.0.0.1:1", 1, 0, &cfg) == SM_OK);
+    const uint64_t pool = 80ull << 20;
+    smem_bm_t bm = smem_bm_create(7, 1, SMEMB_DATA_OP_SDMA, 2u << 20, pool, 0);
+    CHECK(bm != nullptr && smem_bm_join(bm, 0) == SM_OK);
+    auto *dev = static_cast<uint8_t *>(smem_bm_ptr_by_mem_type(bm, SMEM_MEM_TYPE_DEVICE, 0));
+    const std::vector<std::vector<uint64_t>> lists = {
+        {256u << 10}, {(256u << 10) - 1}, {(864u << 10) + 1}, {(33u << 20) + 13}, {70u << 20}, {(12u << 20) - 1}, {12u << 20}, {512u << 10}, {(512u << 10) - 1}, {864u << 10}, {40000, 0, 16384, 1, 300000, 16385}, std::vector<uint64_t>(200, 32768), {8u << 20, 5, (25u << 20) + 1, 127},
+        std::vector<uint64_t>(40, 16383),
+    };
+    std::mt19937 rng(5);
+    for (const uint32_t most : {~0u, 1u, 900u, 1500u, 0u}) {
+        for (size_t k = 0; k < lists.size(); ++k) {
+            std::vector<uint64_t> len = lists[k];
+            const uint64_t total = [&] { uint64_t sum = 0; for (uint64_t l : len) { sum += l; } return sum; }();
+            if (most != ~0u && k > 5) {
+                continue;
+            }
+            std::vector<uint8_t> outside(total), image(total + 256 * len.size());
+            for (size_t i = 0; i < outside.size(); i += 3) {
+                outside[i] = static_cast<uint8_t>(rng());
+            }
+            std::vector<void *> in, out;
+            uint64_t at = 0, inside = 0;
+            for (uint64_t l : len) {
+                inside += 1 + rng() % 200;
+                in.push_back(dev + inside);
+                out.push_back(outside.data() + at);
+                at += l;
+                inside += l;
+            }
+            const uint64_t room = inside + 64;
+            std::memset(dev, 0xA5, room);
+            std::vector<uint8_t> expect(dev, dev + room);
+            for (size_t i = 0; i < len.size(); ++i) {
+                std::memcpy(expect.data() + (static_cast<uint8_t *>(in[i]) - dev), out[i], len[i]);
+            }
+            (void)fake_rt_chunks_streamed();
+            fake_rt_stream_chunks(most);
+            smem_batch_copy_params load{out.data(), in.data(), len.data(), static_cast<uint32_t>(len.size())};
+            CHECK(smem_bm_copy_batch(bm, &load, SMEMB_COPY_H2G, 0) == SM_OK);
+            CHECK(std::memcmp(dev, expect.data(), room) == 0);
+            const bool streams = total >= (256u << 10) && total / len.size() >= 16384 && !(total >= (512u << 10) && total <= (864u << 10));
+            CHECK((fake_rt_chunks_streamed() != 0) == (streams && most != 0));
+            const std::vector<uint8_t> before = outside;
+            std::fill(outside.begin(), outside.end(), 0);
+            smem_batch_copy_params save{in.data(), out.data(), len.data(), static_cast<uint32_t>(len.size())};
+            CHECK(smem_bm_copy_batch(bm, &save, SMEMB_COPY_G2H, 0) == SM_OK);
+            CHECK(outside == before);
+            CHECK((fake_rt_chunks_streamed() != 0) == (streams && total < (12u << 20) && most != 0));
+            fake_rt_stream_chunks(0);
+        }
+    }
+    smem_bm_destroy(bm);
+    smem_bm_uninit(0);
+}
+
 int main()
 {
     SetLogLevel(3);
@@ -2487,6 +2551,7 @@ int main()
     TestPlanners();
     TestPayloadOfPlannedTables();
     TestHostCopy();
+    TestStreamedCopies();
     TestSlotRing();
     TestReportsThatDoNotCome();
     TestRecordedCalls();

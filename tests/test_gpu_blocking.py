@@ -1,5 +1,6 @@
 """Short blocking copies, which report their own end: what they moved is where it belongs when the call returns."""
 
+import ctypes
 import threading
 
 import numpy as np
@@ -122,6 +123,43 @@ LEAST_ROUND = 576 << 10
 ], ids=lambda s: f"{len(s)}x{s[0]}")
 def test_staged_copies_at_the_edges_of_rounds(lib, pool, way, sizes):
     test_staged_copies_of_pageable_memory(lib, pool, way, sizes)
+
+
+@pytest.mark.parametrize("way", ["load", "save"])
+@pytest.mark.parametrize("sizes", [
+    [256 << 10], [(256 << 10) - 1], [16384] * 16, [16383] * 17, [3 * LEAST_ROUND // 2 + 1, 0],        # the least that streams, segments too short for it
+    [65536 - 64] * 14, [65536, 65535, 65537, 1, 131072, 130900] * 3,                                # a chunk or nearly one a segment
+    [(12 << 20) - 1], [12 << 20], [(33 << 20) + 1, 100000],                                         # the line of copies past the caches, more chunks than slots
+], ids=lambda s: f"{len(s)}x{s[0]}")
+def test_copies_while_the_ring_is_filled_or_emptied(lib, pool, way, sizes):
+    test_staged_copies_of_pageable_memory(lib, pool, way, sizes)
+
+
+def test_chunks_that_the_host_never_fills(lib, pool):
+    """The launch leaves when its wait is over, and what it would have written is as it was; what was filled is copied."""
+    chunk, slots, room = 64 << 10, 4, 4096
+    memory = pool.peer_rank_ptr(0)
+    before = _read(lib, memory, 3 * chunk)
+    host = lib.mfrt_alloc_host(slots * chunk + room)
+    try:
+        view = np.ctypeslib.as_array((ctypes.c_uint8 * (slots * chunk + room)).from_address(host))
+        view[:] = 7
+        words = view[slots * chunk:].view(np.uint64)
+        words[:] = 0
+        listed, host_words, gpu_words = slots * chunk, slots * chunk + 1024, slots * chunk + 2048
+        for c in range(2):
+            words[2 * c], words[2 * c + 1] = memory + c * chunk, 1000
+        words[1024 // 8] = 11                                                         # chunk 0 is filled, chunk 1 is not
+        err = lib.mfk_stream_chunks(0, ctypes.c_void_p(host), ctypes.c_void_p(host + listed), ctypes.c_void_p(host + host_words),
+                                    ctypes.c_void_p(host + gpu_words), ctypes.c_uint64(10), 2, slots, 2, None)
+        assert err == 0 and lib.mfrt_device_sync() == 0
+        assert words[2048 // 8] == 11 and words[2048 // 8 + 8] == 0
+        before[:1000] = 7
+        assert np.array_equal(_read(lib, memory, 3 * chunk), before)
+        assert lib.mfk_stream_chunks(0, ctypes.c_void_p(host), None, ctypes.c_void_p(host), ctypes.c_void_p(host), ctypes.c_uint64(0), 1, slots, 2, None) != 0
+    finally:
+        del view, words
+        lib.mfrt_free_host(host)
 
 
 @pytest.mark.parametrize("count, most, launches", [(513, 131072, 1), (1400, 65536, 2), (1601, 131072, 3)])
