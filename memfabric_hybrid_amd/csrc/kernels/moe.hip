@@ -1274,19 +1274,23 @@ __global__ __launch_bounds__(kThreads) void MoeCombineKernel(uint64_t rowsIn, ui
 // the two are kept apart in time: a period is kItems read parts and one write part.  In read
 // part j a wave requests the 16 pieces of its j-th item of the period (eight rows, two column
 // positions per lane) at its own offset of the part, reduces them when they have arrived and
-// keeps the result, 8 registers per item; in the write part it stores the kItems results at
+// keeps the result in LDS; in the write part it stores the kItems results at
 // its own offset of that part (top-6: six rows, twelve pieces).  The start of the first period is agreed through
 // AgreedStart(); after that every wave goes by the constant-rate clock alone.  8192 tokens of 7168
-// elements at top-8: 164-168 us against 177-181 us for one workgroup per item.  Read parts are paced at 6.8 TB/s, write parts at 6.2 (reads at 7.0
-// make the waves fall behind now and then).
+// elements at top-8: 162 us against 177-181 us for one workgroup per item.  Read parts are paced at 6.8 TB/s, write parts at 6.5.
+// HBM is the bound.  Results in registers, four an item (116 of them), left room for 4096 waves: 5120 have a quarter more time for loads that come late in as
+// much longer parts.  Dispatch and combine, us, 4096 waves at 6.8 and 6.2 / 5120 at 6.8 and 6.5: 8192 tokens of 7168 elements at top-8 over 256 experts 352 / 344, over 8 331 /
+// 329, at top-6 274 / 271, of 5120 246 / 244, of 4096 191.0 / 191.5; combine alone of 3600 of 7168 74.3 / 72.7.  Reads at 6.85 make the waves fall behind behind a
+// dispatch, whose rows are still on their way out of the last-level cache (350).  Not taken: 6144 waves (80 registers spill), four results (LDS for 18 waves, 346).
 // Arithmetic and the rule for slots without a row are MoeCombineKernel's.
-constexpr uint32_t kCombineItems = 4;                  // 32 result registers, 116 in all: sixteen waves per CU
-constexpr uint32_t kCombineWavesPerCu = 16;
+constexpr uint32_t kCombineItems = 3;                  // of which the results, 2 KiB each, wait in LDS
+constexpr uint32_t kCombineWavesPerSimd = 5;           // 90 registers
+constexpr uint32_t kCombineWavesPerCu = 4 * kCombineWavesPerSimd;
 constexpr uint32_t kCombineSliceUnits = 128;           // two column positions per lane
-constexpr uint32_t kCombineMinItemsPerWave = 6;
+constexpr uint32_t kCombineMinItemsPerCu = 96;
 
 template <uint32_t kItems, uint32_t kSlots>
-__global__ __launch_bounds__(64) void MoeCombineWindowKernel(const u32x4 *__restrict__ rowsIn,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kCombineWavesPerSimd, kCombineWavesPerSimd))) void MoeCombineWindowKernel(const u32x4 *__restrict__ rowsIn,
                                                              const int32_t *__restrict__ rowOf,
                                                              const float *__restrict__ weights, uint32_t unitsPerRow,
                                                              uint32_t parts, uint32_t items, u32x4 *__restrict__ y,
@@ -1300,6 +1304,7 @@ __global__ __launch_bounds__(64) void MoeCombineWindowKernel(const u32x4 *__rest
     const uint32_t perPart = (unitsPerRow + parts - 1) / parts;
     const MF_GLOBAL u32x4 *in = reinterpret_cast<const MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(rowsIn));
     MF_GLOBAL u32x4 *out = reinterpret_cast<MF_GLOBAL u32x4 *>(reinterpret_cast<uint64_t>(y));
+    __shared__ u32x4 o[kItems][kBatch][64];
     uint64_t t0 = start;
     for (uint32_t base = 0; base < items; base += kItems * gridDim.x, t0 += period) {
         if (base + blockIdx.x >= items) {
@@ -1314,7 +1319,6 @@ __global__ __launch_bounds__(64) void MoeCombineWindowKernel(const u32x4 *__rest
         const uint32_t lastPartTicks = inLastPart >= gridDim.x ? readTicks
             : static_cast<uint32_t>(static_cast<uint64_t>(inLastPart) * readTicks / gridDim.x);
         const uint32_t readEnd = (readParts - 1) * readTicks + lastPartTicks;
-        u32x4 o[kItems][kBatch];
 #pragma unroll
         for (uint32_t j = 0; j < kItems; ++j) {
             const uint32_t item = base + j * gridDim.x + blockIdx.x;
@@ -1352,6 +1356,7 @@ __global__ __launch_bounds__(64) void MoeCombineWindowKernel(const u32x4 *__rest
 #pragma unroll
                 for (uint32_t b = 0; b < kBatch; ++b) {
                     float acc[8];
+                    u32x4 sum;
 #pragma unroll
                     for (uint32_t i = 0; i < 8; ++i) {
                         acc[i] = 0.0f;
@@ -1367,8 +1372,9 @@ __global__ __launch_bounds__(64) void MoeCombineWindowKernel(const u32x4 *__rest
                     }
 #pragma unroll
                     for (uint32_t i = 0; i < 4; ++i) {
-                        o[j][b][i] = ToBf16Pair(acc[2 * i], acc[2 * i + 1]);
+                        sum[i] = ToBf16Pair(acc[2 * i], acc[2 * i + 1]);
                     }
+                    o[j][b][threadIdx.x] = sum;
                 }
             }
         }
@@ -1384,7 +1390,7 @@ __global__ __launch_bounds__(64) void MoeCombineWindowKernel(const u32x4 *__rest
                 for (uint32_t b = 0; b < kBatch; ++b) {
                     const uint32_t u = begin + b * 64 + threadIdx.x;
                     if (u < end) {
-                        __builtin_nontemporal_store(o[j][b], out + static_cast<uint64_t>(token) * unitsPerRow + u);
+                        __builtin_nontemporal_store(o[j][b][threadIdx.x], out + static_cast<uint64_t>(token) * unitsPerRow + u);
                     }
                 }
             }
@@ -1407,7 +1413,7 @@ std::atomic<int> g_xcdStreams{0};
 
 // Pace of the windowed combine, MB/s of HBM traffic in the read parts and in the write parts; 0 = never windowed.
 std::atomic<uint32_t> g_combineReadMBps{6800000};
-std::atomic<uint32_t> g_combineWriteMBps{6200000};
+std::atomic<uint32_t> g_combineWriteMBps{6500000};
 
 uint32_t CombineWaves()
 {
@@ -1426,8 +1432,8 @@ bool DispatchCompares(uint64_t entries, uint32_t topK)
     return entries <= kSmallEntries && entries * topK <= (topK <= 8 ? kSmallCompares : kSmallManyCompares);
 }
 
-// Whether waves that stay and keep reads and writes apart in time combine rows of at least 256 units: from six slices per wave on (top-8, 16 800 items
-// on 4096 waves 51.4 us, one workgroup per item 50.5; 19 200 the same; 25 200 74.4 / 76.7), below which the first read part and the last write part, in
+// Whether waves that stay and keep reads and writes apart in time combine rows of at least 256 units: from 96 slices per CU on (top-8, 16 800 items
+// on 4096 waves of 16 a CU 51.4 us, one workgroup per item 50.5; 19 200 the same; 25 200 74.4 / 76.7), below which the first read part and the last write part, in
 // which the chip only reads or only writes for want of work, cost what the separation gains; and where the last-level cache does not hold the rows that
 // the kernel before has just written.  Rows written by an elementwise kernel and combined, with windows from three items on / from six on / in rows
 // that a dispatch leaves there, us: top-8 3.6 to 5.9 items of 2048 elements a row, 262 MiB of rows and tokens 125.1 / 119.4, 310 146.3 / 141.2, 430 201.7 / 196.9; top-6
@@ -1443,7 +1449,7 @@ bool CombineInWindows(uint32_t tokens, uint32_t hidden, uint32_t topK, uint32_t 
     const uint64_t items = static_cast<uint64_t>(tokens) * parts;
     const uint64_t entries = static_cast<uint64_t>(tokens) * topK;
     const uint32_t waves = CombineWaves();
-    if ((topK != 6 && topK != 8) || upr < 256 || items < static_cast<uint64_t>(waves) * kCombineMinItemsPerWave || items >= 0x40000000ull ||
+    if ((topK != 6 && topK != 8) || upr < 256 || items < static_cast<uint64_t>(waves / kCombineWavesPerCu) * kCombineMinItemsPerCu || items >= 0x40000000ull ||
         DispatchCounts(entries, (entries + tokens) * upr * 16, topK, kMaxExperts, hidden % 64 == 0)) {
         return false;
     }

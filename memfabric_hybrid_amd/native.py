@@ -314,7 +314,7 @@ _calls = None
 
 
 # pace of the combine's read and write parts the library starts with (MB/s), for callers that switch it and back
-MOE_COMBINE_WINDOWS_DEFAULT = (6800000, 6200000)
+MOE_COMBINE_WINDOWS_DEFAULT = (6800000, 6500000)
 
 
 def _bind(handle, table):
