@@ -131,6 +131,12 @@ constexpr uint64_t kWarmMaxBytes = 224ull << 20;
 constexpr uint32_t kWarmGroups = 128;
 constexpr uint32_t kWarmPieces = 8;                     // 128-bit loads in flight per lane
 constexpr uint32_t kWarmHistPercent = 30;               // share of the shorter first launch
+// Rows of so many bytes are read by all CUs that rank nothing, as long as those are many: 8192 tokens of 7168 elements, 117 MB, dispatch with 128 groups and 30 % / so, top-8 over 256 experts
+// 181.0 / 177.1 us, over 8 170.0 / 165.6, top-4 115.0 / 109.7, top-2 74.4 / 73.7; but 84 MB, partly in that cache, 98.2 / 100.1.
+constexpr uint64_t kWarmMoreBytes = 96ull << 20;
+constexpr uint32_t kWarmMoreGroups = 192;
+constexpr uint32_t kWarmMoreBlocks = 64;                // with which they are 256 (16 384 tokens of 4096 elements, 128 blocks, dispatch 208.3 / 210.0)
+constexpr uint32_t kWarmMoreHistPercent = 40;
 
 __device__ __forceinline__ void WarmRows(const u32x4 *rows, uint64_t units, uint32_t group, uint32_t groups)
 {
@@ -1593,8 +1599,9 @@ extern "C" int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens
     const uint64_t rowBytes = static_cast<uint64_t>(upr) * 16;
     const bool warms = tiles && tokens * rowBytes >= kWarmMinBytes;
     const uint64_t warmUnits = !warms ? 0 : (tokens * rowBytes < kWarmMaxBytes ? tokens * rowBytes : kWarmMaxBytes) / 16;
-    const uint64_t warmFirst = counting ? 0 : warmUnits * kWarmHistPercent / 100;
-    const uint32_t warmGroups = warms ? kWarmGroups : 0;
+    const bool warmsMore = warmUnits * 16 >= kWarmMoreBytes && blocks <= kWarmMoreBlocks;
+    const uint64_t warmFirst = counting ? 0 : warmUnits * (warmsMore ? kWarmMoreHistPercent : kWarmHistPercent) / 100;
+    const uint32_t warmGroups = !warms ? 0 : warmsMore ? kWarmMoreGroups : kWarmGroups;
     const u32x4 *warm = static_cast<const u32x4 *>(x);
     if (counting) {
         blockHist = nullptr;
