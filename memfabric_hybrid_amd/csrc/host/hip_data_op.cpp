@@ -167,13 +167,15 @@ struct StreamArea {
     StreamChunk list[kStreamListChunks];
 };
 static_assert(sizeof(StreamArea::ring) == kBounceBytes, "the rounds use it too, and nothing behind it");
-// Below, one launch that is waited for and a copy of the whole are as fast, and so they are where the copy is one round that the cores share (512 KiB to the
-// host 21.9 us, streamed 24.5); shorter segments make chunks that are not worth their words.  Before / streamed, us, to the GPU and back: 300 KB in three parts 21.3 /
-// 19.2, 21.5 / 18.5, 1 MiB 37.7 / 32.5, 40.5 / 36.3, 2 MiB 64.5 / 53.5, 62.8 / 56.2.
-constexpr uint64_t kStreamMinBytes = 256ull << 10;
+// What is one round stays one: 512 KiB to the host 21.9 us, streamed 24.5, and below kSplitMin a copy of its own would wake the helpers for it (260 KB to the GPU 2 ms
+// behind the last 24 us, streamed 33).  Shorter segments make chunks that are not worth their words.  Before / streamed, us, to the GPU and back: 1 MiB 37.7 / 32.4, 40.8 /
+// 36.5, 2 MiB 65.6 / 54.4, 63.4 / 56.0; 2 ms behind the last 53.2 / 45.2, 54.5 / 50.0, 74.4 / 67.7, 73.1 / 68.0.
+constexpr uint64_t kStreamMinBytes = kRoundMinBytes / 2 * 3 + 1;
 constexpr uint64_t kStreamMinSegmentBytes = 16ull << 10;
-// Copies of so many bytes go past the CPU's caches, which they would sweep, ring and all; and those to the host in rounds, of which a core empties
-// 2 MiB in one piece, sooner than as many chunks.  us, rounds by memcpy / rounds past the caches / streamed: to the host 4 MiB 103 / 108 / 96, 8 MiB in 20
+// To the host rounds are the better from here on: a core empties its share of one, 2 MiB, in one piece, sooner than as many chunks (10 MiB 216 to 229 us, streamed 214 in
+// some processes and 245 in others; 8 MiB in 20 parts 188 / 175).
+constexpr uint64_t kStreamMostBytesOut = kRoundBytes;
+// Copies of so many bytes go past the CPU's caches, which they would sweep, ring and all.  us, rounds by memcpy / rounds past the caches / streamed: to the host 4 MiB 103 / 108 / 96, 8 MiB in 20
 // parts 188 / 191 / 172, 12 MiB 265 / 255 / 253, 16 MiB 376 / 338 / 334, 64 MiB 1273 / 1242 / 1352; to the GPU 4 MiB 109 / 114 / 101, 16 MiB 370 / 350 / 340, 64 MiB 1339 / 1286 /
 // 1262, 128 MiB 2559 / 2503 / 2490.
 constexpr uint64_t kPastCachesBytes = 12ull << 20;
@@ -278,8 +280,7 @@ bool Streams(const uint64_t *len, uint32_t n, bool toHost, void *stream)
     for (uint32_t i = 0; i < n; ++i) {
         total += len[i];
     }
-    const bool oneSharedRound = total >= HostCopyHelper::kSplitMin && total <= kRoundMinBytes / 2 * 3;
-    return total >= kStreamMinBytes && !oneSharedRound && !(toHost && total >= kPastCachesBytes) && total / n >= kStreamMinSegmentBytes &&
+    return total >= kStreamMinBytes && !(toHost && total > kStreamMostBytesOut) && total / n >= kStreamMinSegmentBytes &&
            mfrt_stream_capturing(stream) == 0;
 }
 

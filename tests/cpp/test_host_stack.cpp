@@ -2493,8 +2493,8 @@ static void TestStreamedCopies()
     CHECK(bm != nullptr && smem_bm_join(bm, 0) == SM_OK);
     auto *dev = static_cast<uint8_t *>(smem_bm_ptr_by_mem_type(bm, SMEM_MEM_TYPE_DEVICE, 0));
     const std::vector<std::vector<uint64_t>> lists = {
-        {256u << 10}, {(256u << 10) - 1}, {(864u << 10) + 1}, {(33u << 20) + 13}, {70u << 20}, {(12u << 20) - 1}, {12u << 20}, {512u << 10}, {(512u << 10) - 1}, {864u << 10}, {40000, 0, 16384, 1, 300000, 16385}, std::vector<uint64_t>(200, 32768), {8u << 20, 5, (25u << 20) + 1, 127},
-        std::vector<uint64_t>(40, 16383),
+        {256u << 10}, {(256u << 10) - 1}, {(864u << 10) + 1}, {(33u << 20) + 13}, {70u << 20}, {8u << 20}, {(8u << 20) + 1}, {512u << 10}, {(512u << 10) - 1}, {864u << 10}, {40000, 0, 16384, 1, 300000, 16385}, std::vector<uint64_t>(200, 32768), {8u << 20, 5, (25u << 20) + 1, 127},
+        std::vector<uint64_t>(60, 16383), std::vector<uint64_t>(60, 16384),
     };
     std::mt19937 rng(5);
     for (const uint32_t most : {~0u, 1u, 900u, 1500u, 0u}) {
@@ -2528,14 +2528,14 @@ static void TestStreamedCopies()
             smem_batch_copy_params load{out.data(), in.data(), len.data(), static_cast<uint32_t>(len.size())};
             CHECK(smem_bm_copy_batch(bm, &load, SMEMB_COPY_H2G, 0) == SM_OK);
             CHECK(std::memcmp(dev, expect.data(), room) == 0);
-            const bool streams = total >= (256u << 10) && total / len.size() >= 16384 && !(total >= (512u << 10) && total <= (864u << 10));
+            const bool streams = total > (864u << 10) && total / len.size() >= 16384;
             CHECK((fake_rt_chunks_streamed() != 0) == (streams && most != 0));
             const std::vector<uint8_t> before = outside;
             std::fill(outside.begin(), outside.end(), 0);
             smem_batch_copy_params save{in.data(), out.data(), len.data(), static_cast<uint32_t>(len.size())};
             CHECK(smem_bm_copy_batch(bm, &save, SMEMB_COPY_G2H, 0) == SM_OK);
             CHECK(outside == before);
-            CHECK((fake_rt_chunks_streamed() != 0) == (streams && total < (12u << 20) && most != 0));
+            CHECK((fake_rt_chunks_streamed() != 0) == (streams && total <= (8u << 20) && most != 0));
             fake_rt_stream_chunks(0);
         }
     }

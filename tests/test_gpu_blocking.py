@@ -127,9 +127,9 @@ def test_staged_copies_at_the_edges_of_rounds(lib, pool, way, sizes):
 
 @pytest.mark.parametrize("way", ["load", "save"])
 @pytest.mark.parametrize("sizes", [
-    [256 << 10], [(256 << 10) - 1], [16384] * 16, [16383] * 17, [3 * LEAST_ROUND // 2 + 1, 0],        # the least that streams, segments too short for it
+    [3 * LEAST_ROUND // 2], [3 * LEAST_ROUND // 2 + 1, 0], [16384] * 55, [16383] * 56,                # the least that streams, segments too short for it
     [65536 - 64] * 14, [65536, 65535, 65537, 1, 131072, 130900] * 3,                                # a chunk or nearly one a segment
-    [(12 << 20) - 1], [12 << 20], [(33 << 20) + 1, 100000],                                         # the line of copies past the caches, more chunks than slots
+    [8 << 20], [(8 << 20) + 1], [(12 << 20) - 1], [12 << 20], [(33 << 20) + 1, 100000],             # back in rounds, past the caches, more chunks than slots
 ], ids=lambda s: f"{len(s)}x{s[0]}")
 def test_copies_while_the_ring_is_filled_or_emptied(lib, pool, way, sizes):
     test_staged_copies_of_pageable_memory(lib, pool, way, sizes)
