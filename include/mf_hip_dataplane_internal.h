@@ -116,12 +116,12 @@ int32_t mf_xcopy_tune_table(uint32_t stageUnordered, uint32_t deviceTableWgPerCu
  * 0 (default): they overlap one another on purpose and store at once. */
 int32_t mf_xcopy_tune_hold(uint32_t deepHold, int32_t pinnedExtraNanos, uint32_t holdOnSideStreams);
 
-/* A combine of topK == 8 or 6 with rows of 2048 elements and more, on enough tokens to give every wave of the chip six
+/* A combine of topK == 8 or 6 with rows of 2048 elements and more, on enough tokens to give every CU 96
  * slices of 128 x 8 elements (about 3500 tokens of 7168 elements on 256 CUs) and more rows than a dispatch leaves in the
  * last-level cache (400 MiB with their tokens at top-8, 368 MiB at top-6), runs as waves that stay for the whole
  * launch and alternate, chip-wide and by the clock, between reading rows and writing results.  readMBps / writeMBps
  * (MB/s of HBM traffic, 1 000 000 ... 16 000 000) set the pace of the two parts; the defaults are 6 800 000 and
- * 6 200 000, both 0 turns the form off (one workgroup per slice, as for smaller inputs, and as long as a second
+ * 6 500 000, both 0 turns the form off (one workgroup per slice, as for smaller inputs, and as long as a second
  * thread holds a stream of the library).  Results do not depend on it.  No counterpart in the reference.  Returns BM_INVALID_PARAM for other values. */
 int32_t mf_moe_combine_windows(uint32_t readMBps, uint32_t writeMBps);
 /* 1 if such a combine by this thread would take that form now. */

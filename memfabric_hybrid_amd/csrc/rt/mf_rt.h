@@ -109,7 +109,7 @@ int mfk_xcopy_pieces_reported(const void *pieces, uint32_t count, uint64_t bytes
 /* The same pieces, of 4 KiB each; the launch stores `value` into `word` once every byte is in memory.  `counter`: as for
  * mfk_xcopy_done. */
 int mfk_xcopy_pieces_done(const void *pieces, uint32_t count, void *word, uint32_t value, void *counter, void *stream);
-/* The same pieces, of up to mfk_xcopy_window_units() units, which all begin on cache lines in source and destination, in read and
+/* The same pieces, of up to mfk_xcopy_window_units() units, whatever their addresses (those off cache lines hold a lower rate), in read and
  * write windows cut for `windowMBps` MB/s of HBM traffic.  reading: 64ths of a period that are its read part, 0 = half of it. */
 int mfk_xcopy_pieces_windowed(const void *pieces, uint32_t count, uint64_t bytes, uint32_t windowMBps, uint32_t reading, void *mask, uint32_t maskValue,
                               void *stream, void *event);
