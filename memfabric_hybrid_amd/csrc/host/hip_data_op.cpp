@@ -172,6 +172,11 @@ static_assert(sizeof(StreamArea::ring) == kBounceBytes, "the rounds use it too, 
 // 36.5, 2 MiB 65.6 / 54.4, 63.4 / 56.0; 2 ms behind the last 53.2 / 45.2, 54.5 / 50.0, 74.4 / 67.7, 73.1 / 68.0.
 constexpr uint64_t kStreamMinBytes = kRoundMinBytes / 2 * 3 + 1;
 constexpr uint64_t kStreamMinSegmentBytes = 16ull << 10;
+// A segment whose last chunk would be this short is cut into equal ones: full chunks and short ones in turn leave most of the work to a part of the launch's
+// workgroups, which take every eighth or sixteenth.  us, a launch a round / full chunks and a tail / equal ones: 22 segments of 68 181 bytes in 47.8 / 51.6 /
+// 46.9, out 46.4 / 47.6 / 46.1; 32 of 72 022 in 71.0 / 74.3 / 69.8; out 32 of 203 125 145.4 / 147.6 / 139.7, of 100 000 80.6 / 78.5 / 75.1; but 4 of 375 000, a tail of
+// 47 320, 46.0 / 43.9 / 45.8, and 32 of 250 000, one of 53 392, 179.0 / 168.5 / 170.9.
+constexpr uint64_t kStreamShortTail = kStreamChunkBytes / 8 * 5;
 // To the host rounds are the better from here on: a core empties its share of one, 2 MiB, in one piece, sooner than as many chunks (10 MiB 216 to 229 us, streamed 214 in
 // some processes and 245 in others; 8 MiB in 20 parts 188 / 175).
 constexpr uint64_t kStreamMostBytesOut = kRoundBytes;
@@ -314,7 +319,12 @@ int StreamAll(void *const *src, void *const *dst, const uint64_t *len, uint32_t 
             }
             const uint8_t *gpu = static_cast<const uint8_t *>(toHost ? src[i] : dst[i]) + at;
             const uint64_t skip = reinterpret_cast<uint64_t>(gpu) & (kStreamLine - 1);
-            const uint64_t take = std::min<uint64_t>(left, kStreamChunkBytes - skip);       // the next begins on a line
+            uint64_t end = kStreamChunkBytes;       // the next begins on a line
+            if ((skip + left) % kStreamChunkBytes <= kStreamShortTail) {
+                const uint64_t chunks = (skip + left + kStreamChunkBytes - 1) / kStreamChunkBytes;
+                end = ((skip + left + chunks - 1) / chunks + kStreamLine - 1) / kStreamLine * kStreamLine;
+            }
+            const uint64_t take = std::min<uint64_t>(left, end - skip);
             area->list[count++] = StreamChunk{reinterpret_cast<uint64_t>(gpu), static_cast<uint32_t>(take), 0};
             memory.push_back(static_cast<const uint8_t *>(toHost ? dst[i] : src[i]) + at);
             at += take;

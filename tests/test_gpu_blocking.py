@@ -129,6 +129,7 @@ def test_staged_copies_at_the_edges_of_rounds(lib, pool, way, sizes):
 @pytest.mark.parametrize("sizes", [
     [3 * LEAST_ROUND // 2], [3 * LEAST_ROUND // 2 + 1, 0], [16384] * 55, [16383] * 56,                # the least that streams, segments too short for it
     [65536 - 64] * 14, [65536, 65535, 65537, 1, 131072, 130900] * 3,                                # a chunk or nearly one a segment
+    [65536 + 40960 - 128, 65536 + 40960, 65536 + 40961, 65536 + 41088, 196608 + 1, 3 * 65536 - 1] * 3, [65536 + 130] * 16,   # a tail that is shared out and one that is not
     [8 << 20], [(8 << 20) + 1], [(12 << 20) - 1], [12 << 20], [(33 << 20) + 1, 100000],             # back in rounds, past the caches, more chunks than slots
 ], ids=lambda s: f"{len(s)}x{s[0]}")
 def test_copies_while_the_ring_is_filled_or_emptied(lib, pool, way, sizes):
