@@ -209,6 +209,7 @@ struct Streaming {
     void *stream;
     const uint8_t *const *memory;       // the caller's, by chunk
     std::atomic<uint32_t> next{0};
+    std::atomic<bool> launched{false};  // the helpers begin before: until then nothing has left, whatever the stream says
     std::atomic<bool> stopped{false};   // the launch has ended, or never began, with chunks left
 
     static uint64_t Load(const StreamArea::Word &word)
@@ -230,7 +231,7 @@ struct Streaming {
                 return false;
             }
             const auto now = std::chrono::steady_clock::now();
-            if (spins == 1024) {
+            if (spins == 1024 || !launched.load(std::memory_order_acquire)) {
                 since = now;
             } else if (now - since > std::chrono::milliseconds(kStreamLookMillis)) {
                 // the words of a launch that is over have all arrived
@@ -340,6 +341,7 @@ int StreamAll(void *const *src, void *const *dst, const uint64_t *len, uint32_t 
         if (err != 0) {
             job.stopped.store(true, std::memory_order_relaxed);
         } else {
+            job.launched.store(true, std::memory_order_release);
             Streaming::Part(&job);
             for (uint32_t c = toHost || count <= kStreamSlots ? 0 : count - kStreamSlots; !toHost && c < count && job.Wait(c); ++c) {
             }

@@ -58,6 +58,7 @@ bool g_failAllocations = false;
 uint32_t g_streamChunks = 0;              // chunks after which such a launch leaves; 0: it cannot be launched
 std::atomic<uint32_t> g_streamsRunning{0};
 std::atomic<uint64_t> g_chunksStreamed{0};
+uint32_t g_streamLaunchMillis = 0;        // what the call that launches one takes
 std::thread g_streamThread;
 void JoinStreamed()
 {
@@ -446,6 +447,7 @@ int mfk_xcopy_table(const void *tablePlan, int, uint32_t grid, void *mask, uint3
 }
 
 void fake_rt_stream_chunks(uint32_t most) { g_streamChunks = most; }
+void fake_rt_stream_launch_takes(uint32_t millis) { g_streamLaunchMillis = millis; }
 uint64_t fake_rt_chunks_streamed(void) { return g_chunksStreamed.exchange(0); }
 
 // Chunk after chunk, with the words of both sides as the kernel reads and writes them.
@@ -456,6 +458,7 @@ int mfk_stream_chunks(int toHost, void *ring, const void *chunks, void *hostWord
         return -1;
     }
     JoinStreamed();
+    std::this_thread::sleep_for(std::chrono::milliseconds(g_streamLaunchMillis));
     ++g_launches;
     ++g_streamsRunning;
     const uint32_t most = g_streamChunks;

@@ -59,6 +59,7 @@ extern "C" void fake_rt_withhold_reports(void);
 extern "C" void fake_rt_release_reports(void);
 extern "C" void fake_rt_stream_state(int state);
 extern "C" void fake_rt_stream_chunks(uint32_t most);
+extern "C" void fake_rt_stream_launch_takes(uint32_t millis);
 extern "C" uint64_t fake_rt_chunks_streamed(void);
 
 using namespace mf;
@@ -2543,6 +2544,49 @@ static void TestStreamedCopies()
     smem_bm_uninit(0);
 }
 
+// A launch that comes late, later than the helpers look for one that has left, still makes the copy.
+static void TestStreamedCopiesLaunchedLate()
+{
+    smem_bm_config_t cfg;
+    smem_bm_config_init(&cfg);
+    CHECK(smem_bm_init("tcp://127.0.0.1:1", 1, 0, &cfg) == SM_OK);
+    smem_bm_t bm = smem_bm_create(7, 1, SMEMB_DATA_OP_SDMA, 2u << 20, 80ull << 20, 0);
+    CHECK(bm != nullptr && smem_bm_join(bm, 0) == SM_OK);
+    auto *dev = static_cast<uint8_t *>(smem_bm_ptr_by_mem_type(bm, SMEM_MEM_TYPE_DEVICE, 0));
+    std::mt19937 rng(11);
+    fake_rt_stream_chunks(~0u);
+    fake_rt_stream_launch_takes(150);
+    for (const uint64_t bytes : {70ull << 20, 5ull << 20}) {
+        std::vector<uint8_t> outside(bytes);
+        for (size_t i = 0; i < bytes; i += 5) {
+            outside[i] = static_cast<uint8_t>(rng());
+        }
+        const std::vector<uint8_t> before = outside;
+        void *there = outside.data();
+        void *here = dev;
+        uint64_t len = bytes;
+        (void)fake_rt_chunks_streamed();
+        uint64_t launches = fake_rt_launches();
+        smem_batch_copy_params load{&there, &here, &len, 1};
+        CHECK(smem_bm_copy_batch(bm, &load, SMEMB_COPY_H2G, 0) == SM_OK);
+        CHECK(std::memcmp(dev, before.data(), bytes) == 0);
+        CHECK(fake_rt_launches() - launches == 1 && fake_rt_chunks_streamed() == bytes >> 16);
+        if (bytes > (8u << 20)) {
+            continue;
+        }
+        std::fill(outside.begin(), outside.end(), 0);
+        launches = fake_rt_launches();
+        smem_batch_copy_params save{&here, &there, &len, 1};
+        CHECK(smem_bm_copy_batch(bm, &save, SMEMB_COPY_G2H, 0) == SM_OK);
+        CHECK(outside == before);
+        CHECK(fake_rt_launches() - launches == 1 && fake_rt_chunks_streamed() == bytes >> 16);
+    }
+    fake_rt_stream_launch_takes(0);
+    fake_rt_stream_chunks(0);
+    smem_bm_destroy(bm);
+    smem_bm_uninit(0);
+}
+
 int main()
 {
     SetLogLevel(3);
@@ -2552,6 +2596,7 @@ int main()
     TestPayloadOfPlannedTables();
     TestHostCopy();
     TestStreamedCopies();
+    TestStreamedCopiesLaunchedLate();
     TestSlotRing();
     TestReportsThatDoNotCome();
     TestRecordedCalls();
