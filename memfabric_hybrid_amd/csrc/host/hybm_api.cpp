@@ -47,10 +47,11 @@ MF_EXPORT int32_t hybm_init(uint16_t deviceId, uint64_t flags)
     }
     VaManager::Global().SetDeviceProbe(HipDeviceProbe);
     {
-        // the rectangle kernels once, as the engine did with the copy kernels: a kernel's first launch is not capturable
+        // the rectangle kernels once, as the engine did with the copy kernels: a kernel's first launch is not capturable; and those of the
+        // staged copies: a first launch takes long
         void *stream = XcopyEngine::Instance().ThreadStream();
-        if (stream == nullptr || mfk_copy2d_prelaunch(stream) != 0 || mfrt_stream_sync(stream) != 0) {
-            MF_ERROR("the rectangle kernels could not be launched once at start");
+        if (stream == nullptr || mfk_copy2d_prelaunch(stream) != 0 || mfk_stream_prelaunch(stream) != 0 || mfrt_stream_sync(stream) != 0) {
+            MF_ERROR("the rectangle and staging kernels could not be launched once at start");
         }
     }
     if (mfk_moe_setup() != 0) {

@@ -132,6 +132,16 @@ __global__ __launch_bounds__(kStreamThreads) void StreamChunksKernel(uint64_t ri
 }  // namespace
 }  // namespace mf
 
+// Both kernels once, on no chunks: what a first launch costs, this file's code has to be loaded for it, is not paid in a copy, whose helpers
+// would wait for it.
+extern "C" int mfk_stream_prelaunch(void *stream)
+{
+    using namespace mf;
+    const int in = Launch(StreamChunksKernel<false>, 1, kStreamThreads, 0, static_cast<hipStream_t>(stream), 0, 0, 0, 0, 0, 0u, 1u, 1u, 1u);
+    const int out = Launch(StreamChunksKernel<true>, 1, kStreamThreads, 0, static_cast<hipStream_t>(stream), 0, 0, 0, 0, 0, 0u, 1u, 1u, 1u);
+    return in != 0 ? in : out;
+}
+
 extern "C" int mfk_stream_chunks(int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count,
                                  uint32_t slots, uint32_t limitMillis, void *stream)
 {

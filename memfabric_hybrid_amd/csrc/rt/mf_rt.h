@@ -152,6 +152,9 @@ int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, i
 int mfk_stream_chunks(int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count, uint32_t slots,
                       uint32_t limitMillis, void *stream);
 
+/* Every kernel of theirs once, on nothing. */
+int mfk_stream_prelaunch(void *stream);
+
 /* ---- MoE launchers (kernels/moe.hip) ---------------------------------------- */
 uint64_t mfk_moe_workspace_bytes(uint32_t tokens, uint32_t topK, uint32_t experts);
 int mfk_moe_dispatch(const void *x, const void *topk, uint32_t tokens, uint32_t hidden, uint32_t topK, uint32_t experts,

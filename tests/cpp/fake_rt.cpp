@@ -450,6 +450,10 @@ void fake_rt_stream_chunks(uint32_t most) { g_streamChunks = most; }
 void fake_rt_stream_launch_takes(uint32_t millis) { g_streamLaunchMillis = millis; }
 uint64_t fake_rt_chunks_streamed(void) { return g_chunksStreamed.exchange(0); }
 
+uint32_t g_streamPrelaunches = 0;
+uint32_t fake_rt_stream_prelaunches(void) { return g_streamPrelaunches; }
+int mfk_stream_prelaunch(void *) { ++g_streamPrelaunches; return 0; }
+
 // Chunk after chunk, with the words of both sides as the kernel reads and writes them.
 int mfk_stream_chunks(int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count, uint32_t slots,
                       uint32_t limitMillis, void *)

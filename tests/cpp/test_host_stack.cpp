@@ -60,6 +60,7 @@ extern "C" void fake_rt_release_reports(void);
 extern "C" void fake_rt_stream_state(int state);
 extern "C" void fake_rt_stream_chunks(uint32_t most);
 extern "C" void fake_rt_stream_launch_takes(uint32_t millis);
+extern "C" uint32_t fake_rt_stream_prelaunches(void);
 extern "C" uint64_t fake_rt_chunks_streamed(void);
 
 using namespace mf;
@@ -2489,6 +2490,7 @@ static void TestStreamedCopies()
     smem_bm_config_t cfg;
     smem_bm_config_init(&cfg);
     CHECK(smem_bm_init("tcp://127.0.0.1:1", 1, 0, &cfg) == SM_OK);
+    CHECK(fake_rt_stream_prelaunches() != 0);       // no copy waits for the first launch of its kernel
     const uint64_t pool = 80ull << 20;
     smem_bm_t bm = smem_bm_create(7, 1, SMEMB_DATA_OP_SDMA, 2u << 20, pool, 0);
     CHECK(bm != nullptr && smem_bm_join(bm, 0) == SM_OK);
