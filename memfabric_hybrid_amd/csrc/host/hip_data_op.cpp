@@ -186,6 +186,9 @@ constexpr uint64_t kStreamMostBytesOut = kRoundBytes;
 constexpr uint64_t kPastCachesBytes = 12ull << 20;
 constexpr uint32_t kStreamLimitMillis = 1000;
 constexpr uint32_t kStreamLookMillis = 50;              // without a word from the GPU: then whether it has left
+constexpr uint32_t kStreamIdleMicros = 100;             // a launch on an idle stream says its first word after some 20
+constexpr uint32_t kStreamPollMicros = 1000;
+constexpr uint32_t kStreamSleepMicros = 100;            // what the ring holds keeps the GPU busy for as long and longer
 
 StreamArea *AreaOf(XcopyEngine &engine)
 {
@@ -199,7 +202,10 @@ StreamArea *AreaOf(XcopyEngine &engine)
     return area;
 }
 
-// One launch's copy.  The caller and the helpers take chunk after chunk.
+// One launch's copy.  The caller and the helpers take chunk after chunk, each only when the GPU is done with its slot, so that whoever
+// finds nothing to do can leave at any time.  The helpers do so after kStreamIdleMicros: a stream that has other work in front of the
+// launch is waited for by the caller alone, which polls as long as it does for a round, and then sleeps.  CPU time of a call behind 30 ms
+// of matrix products, with all of them polling for it / so: 1 MiB to the host 115 ms / 31 (the runtime polls too), 64 MiB to the GPU 127 / 6.
 struct Streaming {
     StreamArea *area;
     bool toHost;
@@ -209,41 +215,15 @@ struct Streaming {
     void *stream;
     const uint8_t *const *memory;       // the caller's, by chunk
     std::atomic<uint32_t> next{0};
-    std::atomic<bool> launched{false};  // the helpers begin before: until then nothing has left, whatever the stream says
-    std::atomic<bool> stopped{false};   // the launch has ended, or never began, with chunks left
+    bool stopped = false;               // the launch has ended, or never began, with chunks left
 
-    static uint64_t Load(const StreamArea::Word &word)
+    bool Done(uint32_t c) const         // the GPU with chunk c in its slot
     {
-        return __atomic_load_n(&word.value, __ATOMIC_ACQUIRE);
+        return __atomic_load_n(&area->gpu[c % kStreamSlots].value, __ATOMIC_ACQUIRE) == base + c + 1;
     }
-    // Until the GPU is done with chunk c in its slot.
-    bool Wait(uint32_t c)
+    bool MayTake(uint32_t c) const
     {
-        const StreamArea::Word &word = area->gpu[c % kStreamSlots];
-        const uint64_t wanted = base + c + 1;
-        std::chrono::steady_clock::time_point since{};
-        for (uint32_t spins = 1; Load(word) != wanted; ++spins) {
-            if (spins % 1024 != 0) {
-                CpuRelax();
-                continue;
-            }
-            if (stopped.load(std::memory_order_relaxed)) {
-                return false;
-            }
-            const auto now = std::chrono::steady_clock::now();
-            if (spins == 1024 || !launched.load(std::memory_order_acquire)) {
-                since = now;
-            } else if (now - since > std::chrono::milliseconds(kStreamLookMillis)) {
-                // the words of a launch that is over have all arrived
-                if (mfrt_stream_done(stream) != 0 && Load(word) != wanted) {
-                    stopped.store(true, std::memory_order_relaxed);
-                    return false;
-                }
-                since = now;
-                std::this_thread::yield();
-            }
-        }
-        return true;
+        return toHost ? Done(c) : c < kStreamSlots || Done(c - kStreamSlots);
     }
     void Copy(void *to, const void *from, uint32_t len) const
     {
@@ -253,30 +233,103 @@ struct Streaming {
             std::memcpy(to, from, len);
         }
     }
-    static void Part(void *context)
+    void Move(uint32_t c)
     {
-        Streaming &s = *static_cast<Streaming *>(context);
-        for (;;) {
-            const uint32_t c = s.next.fetch_add(1, std::memory_order_relaxed);
-            if (c >= s.count) {
+        const uint32_t slot = c % kStreamSlots;
+        const StreamChunk &chunk = area->list[c];
+        uint8_t *there = area->ring[slot] + (chunk.at & (kStreamLine - 1));
+        if (toHost) {
+            Copy(const_cast<uint8_t *>(memory[c]), there, chunk.len);
+        } else {
+            Copy(there, memory[c], chunk.len);
+        }
+        __atomic_store_n(&area->host[slot].value, base + c + 1, __ATOMIC_RELEASE);
+    }
+    // Until all chunks are taken, or none can be for a while.
+    void Work()
+    {
+        std::chrono::steady_clock::time_point since{};
+        for (uint32_t idle = 0;;) {
+            uint32_t c = next.load(std::memory_order_relaxed);
+            if (c >= count) {
                 return;
             }
-            const uint32_t slot = c % kStreamSlots;
-            const StreamChunk &chunk = s.area->list[c];
-            uint8_t *there = s.area->ring[slot] + (chunk.at & (kStreamLine - 1));
-            if (s.toHost) {
-                if (!s.Wait(c)) {
-                    return;
+            if (MayTake(c)) {
+                if (next.compare_exchange_weak(c, c + 1, std::memory_order_relaxed)) {
+                    Move(c);
+                    idle = 0;
                 }
-                s.Copy(const_cast<uint8_t *>(s.memory[c]), there, chunk.len);
-            } else {
-                if (c >= kStreamSlots && !s.Wait(c - kStreamSlots)) {
-                    return;
-                }
-                s.Copy(there, s.memory[c], chunk.len);
+                continue;
             }
-            __atomic_store_n(&s.area->host[slot].value, s.base + c + 1, __ATOMIC_RELEASE);
+            CpuRelax();
+            if (++idle % 64 != 0) {
+                continue;
+            }
+            const auto now = std::chrono::steady_clock::now();
+            if (idle == 64) {
+                since = now;
+            } else if (now - since > std::chrono::microseconds(kStreamIdleMicros)) {
+                return;
+            }
         }
+    }
+    static void Part(void *context)
+    {
+        static_cast<Streaming *>(context)->Work();
+    }
+    // The caller's wait for the GPU, with the helpers given back.  What ends it is that done() says so, or that the launch has.
+    template <class F>
+    bool Await(F done)
+    {
+        const auto start = std::chrono::steady_clock::now();
+        auto looked = start;
+        for (uint32_t polls = 1; !done(); ++polls) {
+            if (polls % 64 != 0) {
+                CpuRelax();
+                continue;
+            }
+            const auto now = std::chrono::steady_clock::now();
+            if (now - start < std::chrono::microseconds(kStreamPollMicros)) {
+                continue;
+            }
+            polls = 63;
+            if (toHost ? count <= kStreamSlots : next.load(std::memory_order_relaxed) >= count) {   // it needs nothing more of the CPU
+                stopped = mfrt_stream_sync(stream) != 0 || !done();
+                return !stopped;
+            }
+            std::this_thread::sleep_for(std::chrono::microseconds(kStreamSleepMicros));
+            if (now - looked > std::chrono::milliseconds(kStreamLookMillis)) {
+                looked = now;
+                // the words of a launch that is over have all arrived
+                if (mfrt_stream_done(stream) != 0 && !done()) {
+                    stopped = true;
+                    return false;
+                }
+            }
+        }
+        return true;
+    }
+    // The caller's part behind the launch; `begun`: the helpers are at it.
+    void Run(HostCopyHelper &helper, bool begun)
+    {
+        for (;;) {
+            Work();
+            helper.End(begun);
+            if (next.load(std::memory_order_relaxed) >= count) {
+                break;
+            }
+            if (!Await([&] { return MayTake(next.load(std::memory_order_relaxed)); })) {
+                return;
+            }
+            begun = helper.Begin(&Streaming::Part, this);
+        }
+        uint32_t seen = count <= kStreamSlots ? 0 : count - kStreamSlots;
+        (void)(toHost || Await([&] {
+            while (seen < count && Done(seen)) {
+                ++seen;
+            }
+            return seen == count;
+        }));
     }
 };
 
@@ -338,16 +391,12 @@ int StreamAll(void *const *src, void *const *dst, const uint64_t *len, uint32_t 
         const bool begun = helper.Begin(&Streaming::Part, &job);
         const int err = mfk_stream_chunks(toHost ? 1 : 0, area->ring, area->list, area->host, area->gpu, job.base, count, kStreamSlots,
                                           kStreamLimitMillis, stream);
-        if (err != 0) {
-            job.stopped.store(true, std::memory_order_relaxed);
+        if (err == 0) {
+            job.Run(helper, begun);
         } else {
-            job.launched.store(true, std::memory_order_release);
-            Streaming::Part(&job);
-            for (uint32_t c = toHost || count <= kStreamSlots ? 0 : count - kStreamSlots; !toHost && c < count && job.Wait(c); ++c) {
-            }
+            helper.End(begun);
         }
-        helper.End(begun);
-        if (job.stopped.load(std::memory_order_relaxed)) {
+        if (err != 0 || job.stopped) {
             const int sync = err != 0 ? 0 : mfrt_stream_sync(stream);
             if (sync != 0) {
                 MF_FAIL(BM_ERROR, "copy failed on the GPU: " << mfrt_error_string(sync));

@@ -59,6 +59,7 @@ uint32_t g_streamChunks = 0;              // chunks after which such a launch le
 std::atomic<uint32_t> g_streamsRunning{0};
 std::atomic<uint64_t> g_chunksStreamed{0};
 uint32_t g_streamLaunchMillis = 0;        // what the call that launches one takes
+uint32_t g_streamBusyMillis = 0;          // of other work that is in front of it on its stream
 std::thread g_streamThread;
 void JoinStreamed()
 {
@@ -450,6 +451,7 @@ void fake_rt_stream_chunks(uint32_t most) { g_streamChunks = most; }
 void fake_rt_stream_launch_takes(uint32_t millis) { g_streamLaunchMillis = millis; }
 uint64_t fake_rt_chunks_streamed(void) { return g_chunksStreamed.exchange(0); }
 
+void fake_rt_stream_busy(uint32_t millis) { g_streamBusyMillis = millis; }
 uint32_t g_streamPrelaunches = 0;
 uint32_t fake_rt_stream_prelaunches(void) { return g_streamPrelaunches; }
 int mfk_stream_prelaunch(void *) { ++g_streamPrelaunches; return 0; }
@@ -466,7 +468,9 @@ int mfk_stream_chunks(int toHost, void *ring, const void *chunks, void *hostWord
     ++g_launches;
     ++g_streamsRunning;
     const uint32_t most = g_streamChunks;
+    const uint32_t busy = g_streamBusyMillis;
     g_streamThread = std::thread([=] {
+        std::this_thread::sleep_for(std::chrono::milliseconds(busy));
         auto word = [](void *words, uint32_t slot) {
             return reinterpret_cast<uint64_t *>(static_cast<uint8_t *>(words) + static_cast<uint64_t>(slot) * mf::kStreamWordBytes);
         };

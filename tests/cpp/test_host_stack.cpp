@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <ctime>
 #include <random>
 #include <atomic>
 #include <chrono>
@@ -60,6 +61,7 @@ extern "C" void fake_rt_release_reports(void);
 extern "C" void fake_rt_stream_state(int state);
 extern "C" void fake_rt_stream_chunks(uint32_t most);
 extern "C" void fake_rt_stream_launch_takes(uint32_t millis);
+extern "C" void fake_rt_stream_busy(uint32_t millis);
 extern "C" uint32_t fake_rt_stream_prelaunches(void);
 extern "C" uint64_t fake_rt_chunks_streamed(void);
 
@@ -2589,6 +2591,77 @@ static void TestStreamedCopiesLaunchedLate()
     smem_bm_uninit(0);
 }
 
+// While other work is in front of the launch on its stream, one thread waits, asleep for most of the time, and the helpers are at the
+// disposal of other threads.
+static void TestStreamedCopiesBehindOtherWork()
+{
+    smem_bm_config_t cfg;
+    smem_bm_config_init(&cfg);
+    CHECK(smem_bm_init("tcp://127.0.0.1:1", 1, 0, &cfg) == SM_OK);
+    smem_bm_t bm = smem_bm_create(7, 1, SMEMB_DATA_OP_SDMA, 2u << 20, 80ull << 20, 0);
+    CHECK(bm != nullptr && smem_bm_join(bm, 0) == SM_OK);
+    auto *dev = static_cast<uint8_t *>(smem_bm_ptr_by_mem_type(bm, SMEM_MEM_TYPE_DEVICE, 0));
+    std::mt19937 rng(13);
+    fake_rt_stream_chunks(~0u);
+    constexpr uint32_t kBusyMillis = 400;
+    std::vector<uint64_t> shortOnes(480, 1000);        // with the one behind them more chunks than the ring has slots
+    shortOnes.push_back(7864320);
+    const std::vector<std::vector<uint64_t>> loads = {{70ull << 20}, {5ull << 20}, shortOnes}, saves = {{1ull << 20}, {8ull << 20}, shortOnes};
+    for (const bool toHost : {false, true}) {
+        for (const std::vector<uint64_t> &len : toHost ? saves : loads) {
+            uint64_t bytes = 0;
+            std::vector<void *> here, there;
+            for (uint64_t l : len) {
+                bytes += l;
+            }
+            std::vector<uint8_t> outside(bytes);
+            for (size_t i = 0; i < bytes; i += 7) {
+                outside[i] = static_cast<uint8_t>(rng());
+            }
+            uint64_t at = 0;
+            for (uint64_t l : len) {
+                here.push_back(dev + at);
+                there.push_back(outside.data() + at);
+                at += l;
+            }
+            const std::vector<uint8_t> before = outside;
+            if (toHost) {
+                std::memcpy(dev, before.data(), bytes);
+                std::fill(outside.begin(), outside.end(), 0);
+            } else {
+                std::memset(dev, 0, bytes);
+            }
+            smem_batch_copy_params params{toHost ? here.data() : there.data(), toHost ? there.data() : here.data(), len.data(), static_cast<uint32_t>(len.size())};
+            auto cpuMillis = [&] {
+                const clock_t cpu = clock();
+                CHECK(smem_bm_copy_batch(bm, &params, toHost ? SMEMB_COPY_G2H : SMEMB_COPY_H2G, 0) == SM_OK);
+                return 1000.0 * static_cast<double>(clock() - cpu) / CLOCKS_PER_SEC;
+            };
+            const double idleMillis = cpuMillis();
+            (void)fake_rt_chunks_streamed();
+            fake_rt_stream_busy(kBusyMillis);
+            bool shared = false;
+            std::thread other([&] {
+                std::this_thread::sleep_for(std::chrono::milliseconds(kBusyMillis / 2));
+                const uint64_t copies = HostCopyHelper::Instance().SharedCopies();
+                std::vector<uint8_t> a(1u << 20, 1), b(1u << 20);
+                HostCopyHelper::Instance().Copy(b.data(), a.data(), a.size());
+                shared = HostCopyHelper::Instance().SharedCopies() - copies == 1;
+            });
+            const double busyMillis = cpuMillis();
+            other.join();
+            fake_rt_stream_busy(0);
+            CHECK(outside == before && std::memcmp(dev, before.data(), bytes) == 0);
+            CHECK(fake_rt_chunks_streamed() != 0);
+            CHECK(shared);
+            CHECK(busyMillis - idleMillis < kBusyMillis * 3 / 4);       // four threads that poll take 1600 ms more
+        }
+    }
+    fake_rt_stream_chunks(0);
+    smem_bm_destroy(bm);
+    smem_bm_uninit(0);
+}
+
 int main()
 {
     SetLogLevel(3);
@@ -2599,6 +2672,7 @@ int main()
     TestHostCopy();
     TestStreamedCopies();
     TestStreamedCopiesLaunchedLate();
+    TestStreamedCopiesBehindOtherWork();
     TestSlotRing();
     TestReportsThatDoNotCome();
     TestRecordedCalls();
