@@ -153,7 +153,14 @@ uint64_t RoundBytes(uint64_t wanted, uint64_t left)
 // link has work from the first 64 KiB on, and no round waits for a launch or for its completion word.  What follows the ring stays from
 // copy to copy: the words of both sides, what they count from, and the launch's list.
 constexpr uint32_t kStreamSlots = 512;
-constexpr uint32_t kStreamListChunks = 1u << 13;       // of one launch, 512 MiB: a longer copy is several
+constexpr uint32_t kStreamListChunks = 1u << 13;       // 512 MiB: a longer copy is several
+// Chunks of one launch, 4 MiB.  A launch that waits for the CPU holds its hardware queue, and with it the launches of other streams that the
+// runtime has put there: a small kernel and its wait beside loads of 64 MiB, median and 99 % in us, one launch for the whole copy 1201 and 1243, of 8
+// MiB 157 / 173, of 4 MiB 81 / 98, of 2 MiB 43 / 79 (in rounds 95 to 146 / 470); the load 1252, 1253, 1257 and 1274 (1330 to 1350).  Beside loads of 4 MiB
+// 92 / 102, of 2 MiB 50 / 80 (41 to 54 / 91).
+constexpr uint32_t kStreamLaunchChunks = 64;
+constexpr uint32_t kStreamLead = 24;                    // chunks in front of its end at which the next one goes out: the link takes 28 us for them
+static_assert(kStreamSlots % kStreamLaunchChunks == 0, "a launch's slots lie side by side");
 struct StreamArea {
     uint8_t ring[kStreamSlots][kStreamChunkBytes];
     struct Word {
@@ -202,7 +209,7 @@ StreamArea *AreaOf(XcopyEngine &engine)
     return area;
 }
 
-// One launch's copy.  The caller and the helpers take chunk after chunk, each only when the GPU is done with its slot, so that whoever
+// A copy of up to kStreamListChunks.  The caller and the helpers take chunk after chunk, each only when the GPU is done with its slot, so that whoever
 // finds nothing to do can leave at any time.  The helpers do so after kStreamIdleMicros: a stream that has other work in front of the
 // launch is waited for by the caller alone, which polls as long as it does for a round, and then sleeps.  CPU time of a call behind 30 ms
 // of matrix products, with all of them polling for it / so: 1 MiB to the host 115 ms / 31 (the runtime polls too), 64 MiB to the GPU 127 / 6.
@@ -215,8 +222,27 @@ struct Streaming {
     void *stream;
     const uint8_t *const *memory;       // the caller's, by chunk
     std::atomic<uint32_t> next{0};
-    bool stopped = false;               // the launch has ended, or never began, with chunks left
+    uint32_t launched = 0;              // chunks; the caller launches
+    int error = 0;                      // of a launch
+    bool stopped = false;               // the launches have ended, or never began, with chunks left
 
+    // The next launch goes out when the one before is nearly done, and beside it, so that the link is not left idle in between.
+    bool LaunchMore()
+    {
+        if (launched >= count || error != 0 || (launched != 0 && !Done(launched - kStreamLead))) {
+            return false;
+        }
+        const uint32_t slot = launched % kStreamSlots;
+        const uint32_t some = std::min(count - launched, kStreamLaunchChunks);
+        const auto launch = launched == 0 ? mfk_stream_chunks : mfk_stream_chunks_beside;
+        error = launch(toHost ? 1 : 0, area->ring[slot], area->list + launched, area->host + slot, area->gpu + slot, base + launched, some,
+                       kStreamSlots - slot, kStreamLimitMillis, stream);
+        if (error != 0) {
+            return false;
+        }
+        launched += some;
+        return true;
+    }
     bool Done(uint32_t c) const         // the GPU with chunk c in its slot
     {
         return __atomic_load_n(&area->gpu[c % kStreamSlots].value, __ATOMIC_ACQUIRE) == base + c + 1;
@@ -246,10 +272,13 @@ struct Streaming {
         __atomic_store_n(&area->host[slot].value, base + c + 1, __ATOMIC_RELEASE);
     }
     // Until all chunks are taken, or none can be for a while.
-    void Work()
+    void Work(bool helps)
     {
         std::chrono::steady_clock::time_point since{};
         for (uint32_t idle = 0;;) {
+            if (!helps) {
+                (void)LaunchMore();
+            }
             uint32_t c = next.load(std::memory_order_relaxed);
             if (c >= count) {
                 return;
@@ -275,15 +304,21 @@ struct Streaming {
     }
     static void Part(void *context)
     {
-        static_cast<Streaming *>(context)->Work();
+        static_cast<Streaming *>(context)->Work(true);
     }
-    // The caller's wait for the GPU, with the helpers given back.  What ends it is that done() says so, or that the launch has.
+    // The caller's wait for the GPU, with the helpers given back.  What ends it is that done() says so, or that the launches have.
     template <class F>
     bool Await(F done)
     {
-        const auto start = std::chrono::steady_clock::now();
+        auto start = std::chrono::steady_clock::now();
         auto looked = start;
         for (uint32_t polls = 1; !done(); ++polls) {
+            if (LaunchMore()) {
+                start = looked = std::chrono::steady_clock::now();
+            }
+            if (error != 0) {
+                return false;
+            }
             if (polls % 64 != 0) {
                 CpuRelax();
                 continue;
@@ -293,7 +328,7 @@ struct Streaming {
                 continue;
             }
             polls = 63;
-            if (toHost ? count <= kStreamSlots : next.load(std::memory_order_relaxed) >= count) {   // it needs nothing more of the CPU
+            if (launched >= count && (toHost || next.load(std::memory_order_relaxed) >= count)) {    // they need nothing more of the CPU
                 stopped = mfrt_stream_sync(stream) != 0 || !done();
                 return !stopped;
             }
@@ -301,7 +336,7 @@ struct Streaming {
             if (now - looked > std::chrono::milliseconds(kStreamLookMillis)) {
                 looked = now;
                 // the words of a launch that is over have all arrived
-                if (mfrt_stream_done(stream) != 0 && !done()) {
+                if (mfrt_stream_done(stream) != 0 && !LaunchMore() && !done()) {
                     stopped = true;
                     return false;
                 }
@@ -309,11 +344,11 @@ struct Streaming {
         }
         return true;
     }
-    // The caller's part behind the launch; `begun`: the helpers are at it.
-    void Run(HostCopyHelper &helper, bool begun)
+    void Run(HostCopyHelper &helper)
     {
+        bool begun = helper.Begin(&Streaming::Part, this);
         for (;;) {
-            Work();
+            Work(false);
             helper.End(begun);
             if (next.load(std::memory_order_relaxed) >= count) {
                 break;
@@ -364,7 +399,7 @@ int StreamAll(void *const *src, void *const *dst, const uint64_t *len, uint32_t 
     while (i < n) {
         memory.clear();
         uint32_t count = 0;
-        while (i < n && count < kStreamListChunks) {
+        while (i < n && count < (toHost ? kStreamSlots : kStreamListChunks)) {      // to the host the GPU waits for nothing
             const uint64_t left = len[i] - at;
             if (left == 0) {
                 ++i;
@@ -388,16 +423,9 @@ int StreamAll(void *const *src, void *const *dst, const uint64_t *len, uint32_t 
         }
         Streaming job{area, toHost, total >= kPastCachesBytes, area->base.value, count, stream, memory.data()};
         area->base.value += count;
-        const bool begun = helper.Begin(&Streaming::Part, &job);
-        const int err = mfk_stream_chunks(toHost ? 1 : 0, area->ring, area->list, area->host, area->gpu, job.base, count, kStreamSlots,
-                                          kStreamLimitMillis, stream);
-        if (err == 0) {
-            job.Run(helper, begun);
-        } else {
-            helper.End(begun);
-        }
-        if (err != 0 || job.stopped) {
-            const int sync = err != 0 ? 0 : mfrt_stream_sync(stream);
+        job.Run(helper);
+        if (job.error != 0 || job.stopped) {
+            const int sync = job.launched == 0 ? 0 : mfrt_stream_sync(stream);
             if (sync != 0) {
                 MF_FAIL(BM_ERROR, "copy failed on the GPU: " << mfrt_error_string(sync));
             }

@@ -1,12 +1,13 @@
 // Copies between a ring of slots in pinned host memory and HBM that run while the CPU fills or empties the ring.
 //
-// One launch moves all chunks of a copy.  Workgroup g takes the chunks g, g + groups, ...; chunk c uses slot c % slots.  Each side says
-// in a word per slot, on a line of its own, which chunk it has finished there (base + c + 1), and waits for the other's word: on the way
-// to HBM the GPU for the chunk to be filled, on the way to the host, once the ring has been round, for the chunk before to be emptied.
+// A launch moves the chunks of 4 MiB, the launches of a copy follow one another without a gap.  Workgroup g takes the chunks g, g + groups, ...; chunk
+// c uses slot c % slots.  Each side says in a word per slot, on a line of its own, which chunk it has finished there (base + c + 1).  On the
+// way to HBM the GPU waits for the chunk to be filled; to the host it waits for nothing, the host launches no more chunks than there are slots free.
 // The GPU's waits end after limitTicks of the constant-rate clock: a workgroup then leaves, the host finds that nothing of the
 // launch is left and copies another way.
 // Bound: the host link, 56 to 57 GB/s.  A launch a round of up to 8 MiB instead, filled or emptied by the CPU as a whole, waits for the CPU at one
 // end of the copy, and for a launch and its completion word in every round.
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -97,9 +98,9 @@ __global__ __launch_bounds__(kStreamThreads) void StreamChunksKernel(uint64_t ri
         const uint32_t slot = c % slots;
         const uint64_t at = list[c].at;
         const uint32_t len = list[c].len;
-        if (!kToHost || c >= slots) {
+        if (!kToHost) {
             if (threadIdx.x == 0) {
-                const uint64_t wanted = kToHost ? base + c - slots + 1 : base + c + 1;
+                const uint64_t wanted = base + c + 1;
                 const uint64_t start = wall_clock64();
                 uint64_t seen = ReadWord(hostWords + static_cast<uint64_t>(slot) * kStreamWordBytes);
                 while (seen != wanted && wall_clock64() - start < limitTicks) {
@@ -142,20 +143,38 @@ extern "C" int mfk_stream_prelaunch(void *stream)
     return in != 0 ? in : out;
 }
 
-extern "C" int mfk_stream_chunks(int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count,
-                                 uint32_t slots, uint32_t limitMillis, void *stream)
+static int LaunchChunks(bool beside, int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count,
+                        uint32_t slots, uint32_t limitMillis, void *stream)
 {
     using namespace mf;
     int dev = 0;
     int khz = 0;
     if (ring == nullptr || chunks == nullptr || hostWords == nullptr || gpuWords == nullptr || count == 0 || slots == 0 ||
-        limitMillis == 0 || limitMillis > kStreamMostMillis ||
+        (toHost != 0 && count > slots) || limitMillis == 0 || limitMillis > kStreamMostMillis ||
         hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0 || khz > 1000000) {
         return -1;
     }
     const uint32_t most = toHost != 0 ? kStreamGroupsOut : kStreamGroupsIn;
     const uint32_t groups = count < most ? count : most;
-    return Launch(toHost != 0 ? StreamChunksKernel<true> : StreamChunksKernel<false>, groups, kStreamThreads, 0, static_cast<hipStream_t>(stream),
-                  At(ring), At(chunks), At(hostWords), At(gpuWords), base, count, slots, groups,
-                  static_cast<uint32_t>(khz) * limitMillis);
+    const uint32_t ticks = static_cast<uint32_t>(khz) * limitMillis;
+    const auto kernel = toHost != 0 ? StreamChunksKernel<true> : StreamChunksKernel<false>;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (!beside) {
+        return Launch(kernel, groups, kStreamThreads, 0, s, At(ring), At(chunks), At(hostWords), At(gpuWords), base, count, slots, groups, ticks);
+    }
+    hipExtLaunchKernelGGL(kernel, dim3(groups), dim3(kStreamThreads), 0, s, nullptr, nullptr, hipExtAnyOrderLaunch, At(ring), At(chunks),
+                          At(hostWords), At(gpuWords), base, count, slots, groups, ticks);
+    return static_cast<int>(hipGetLastError());
+}
+
+extern "C" int mfk_stream_chunks(int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count,
+                                 uint32_t slots, uint32_t limitMillis, void *stream)
+{
+    return LaunchChunks(false, toHost, ring, chunks, hostWords, gpuWords, base, count, slots, limitMillis, stream);
+}
+
+extern "C" int mfk_stream_chunks_beside(int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count,
+                                        uint32_t slots, uint32_t limitMillis, void *stream)
+{
+    return LaunchChunks(true, toHost, ring, chunks, hostWords, gpuWords, base, count, slots, limitMillis, stream);
 }

@@ -148,9 +148,12 @@ int mfk_xcopy_table_static(const void *triples, uint32_t nseg, uint32_t units, i
 /* `count` mf::StreamChunk (kernels/staging.h) in pinned host memory, chunk c between HBM and slot c % slots, of kStreamChunkBytes, of a ring
  * in pinned host memory, where it begins `at` % kStreamLine bytes in; the launch runs while the CPU fills (toHost 0) or empties the slots.  hostWords and
  * gpuWords: a 64-bit word per slot, kStreamWordBytes apart, in which the CPU and the GPU say base + c + 1 when they are done with chunk c
- * there.  A workgroup that waits limitMillis for the CPU leaves, and the chunks it has left are not copied. */
+ * there.  A workgroup that waits limitMillis for the CPU leaves, and the chunks it has left are not copied.  To the host it waits for
+ * nothing, and count is at most slots.  The second form does not wait for launches queued before it on `stream` (it carries no barrier). */
 int mfk_stream_chunks(int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count, uint32_t slots,
                       uint32_t limitMillis, void *stream);
+int mfk_stream_chunks_beside(int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count,
+                             uint32_t slots, uint32_t limitMillis, void *stream);
 
 /* Every kernel of theirs once, on nothing. */
 int mfk_stream_prelaunch(void *stream);

@@ -55,17 +55,21 @@ const void *g_lastRestList = nullptr;
 bool g_failAllocations = false;
 
 // Streamed copies run on a thread of their own; off unless a test asks for them, so that the others see copies in rounds.
-uint32_t g_streamChunks = 0;              // chunks after which such a launch leaves; 0: it cannot be launched
+uint32_t g_streamChunks = 0;              // chunks after which the launches of a copy leave; 0: it cannot be launched
 std::atomic<uint32_t> g_streamsRunning{0};
 std::atomic<uint64_t> g_chunksStreamed{0};
 uint32_t g_streamLaunchMillis = 0;        // what the call that launches one takes
 uint32_t g_streamBusyMillis = 0;          // of other work that is in front of it on its stream
-std::thread g_streamThread;
+uint32_t g_mostChunksLaunched = 0;        // of one launch
+uint32_t g_streamLaunches = ~0u;          // after which they fail
+uint64_t g_streamBase = 0;                // what the copy's first launch counts from
+std::vector<std::thread> g_streamThreads;
 void JoinStreamed()
 {
-    if (g_streamThread.joinable()) {
-        g_streamThread.join();
+    for (std::thread &thread : g_streamThreads) {
+        thread.join();
     }
+    g_streamThreads.clear();
 }
 
 void *Track(uint64_t bytes, int kind)
@@ -451,36 +455,48 @@ void fake_rt_stream_chunks(uint32_t most) { g_streamChunks = most; }
 void fake_rt_stream_launch_takes(uint32_t millis) { g_streamLaunchMillis = millis; }
 uint64_t fake_rt_chunks_streamed(void) { return g_chunksStreamed.exchange(0); }
 
+void fake_rt_stream_launches(uint32_t most) { g_streamLaunches = most; }
 void fake_rt_stream_busy(uint32_t millis) { g_streamBusyMillis = millis; }
 uint32_t g_streamPrelaunches = 0;
 uint32_t fake_rt_stream_prelaunches(void) { return g_streamPrelaunches; }
 int mfk_stream_prelaunch(void *) { ++g_streamPrelaunches; return 0; }
 
-// Chunk after chunk, with the words of both sides as the kernel reads and writes them.
-int mfk_stream_chunks(int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count, uint32_t slots,
-                      uint32_t limitMillis, void *)
+uint32_t fake_rt_most_chunks_launched(void)
 {
-    if (g_streamChunks == 0) {
+    const uint32_t most = g_mostChunksLaunched;
+    g_mostChunksLaunched = 0;
+    return most;
+}
+
+// Chunk after chunk, with the words of both sides as the kernel reads and writes them.
+static int RunChunks(bool beside, int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count, uint32_t slots,
+                     uint32_t limitMillis)
+{
+    if (g_streamChunks == 0 || count == 0 || (toHost != 0 && count > slots) || g_streamLaunches == 0) {
         return -1;
     }
-    JoinStreamed();
+    --g_streamLaunches;
+    if (!beside) {
+        JoinStreamed();
+        g_streamBase = base;
+    }
     std::this_thread::sleep_for(std::chrono::milliseconds(g_streamLaunchMillis));
     ++g_launches;
     ++g_streamsRunning;
-    const uint32_t most = g_streamChunks;
-    const uint32_t busy = g_streamBusyMillis;
-    g_streamThread = std::thread([=] {
+    g_mostChunksLaunched = count > g_mostChunksLaunched ? count : g_mostChunksLaunched;
+    const uint64_t most = g_streamBase + g_streamChunks;
+    const uint32_t busy = beside ? 0 : g_streamBusyMillis;
+    g_streamThreads.emplace_back([=] {
         std::this_thread::sleep_for(std::chrono::milliseconds(busy));
         auto word = [](void *words, uint32_t slot) {
             return reinterpret_cast<uint64_t *>(static_cast<uint8_t *>(words) + static_cast<uint64_t>(slot) * mf::kStreamWordBytes);
         };
-        for (uint32_t c = 0; c < count && c < most; ++c) {
+        for (uint32_t c = 0; c < count && base + c < most; ++c) {
             const mf::StreamChunk &chunk = static_cast<const mf::StreamChunk *>(chunks)[c];
             const uint32_t slot = c % slots;
-            if (toHost == 0 || c >= slots) {
-                const uint64_t wanted = toHost != 0 ? base + c - slots + 1 : base + c + 1;
+            if (toHost == 0) {
                 const auto start = std::chrono::steady_clock::now();
-                while (__atomic_load_n(word(hostWords, slot), __ATOMIC_ACQUIRE) != wanted) {
+                while (__atomic_load_n(word(hostWords, slot), __ATOMIC_ACQUIRE) != base + c + 1) {
                     if (std::chrono::steady_clock::now() - start > std::chrono::milliseconds(limitMillis)) {
                         --g_streamsRunning;
                         return;
@@ -501,6 +517,16 @@ int mfk_stream_chunks(int toHost, void *ring, const void *chunks, void *hostWord
         --g_streamsRunning;
     });
     return 0;
+}
+int mfk_stream_chunks(int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count, uint32_t slots,
+                      uint32_t limitMillis, void *)
+{
+    return RunChunks(false, toHost, ring, chunks, hostWords, gpuWords, base, count, slots, limitMillis);
+}
+int mfk_stream_chunks_beside(int toHost, void *ring, const void *chunks, void *hostWords, void *gpuWords, uint64_t base, uint32_t count,
+                             uint32_t slots, uint32_t limitMillis, void *)
+{
+    return RunChunks(true, toHost, ring, chunks, hostWords, gpuWords, base, count, slots, limitMillis);
 }
 
 // The pieces in the order of the kernel's workgroups.  One that is longer than its workgroup or reaches past the end of the list

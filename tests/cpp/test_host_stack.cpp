@@ -62,6 +62,8 @@ extern "C" void fake_rt_stream_state(int state);
 extern "C" void fake_rt_stream_chunks(uint32_t most);
 extern "C" void fake_rt_stream_launch_takes(uint32_t millis);
 extern "C" void fake_rt_stream_busy(uint32_t millis);
+extern "C" void fake_rt_stream_launches(uint32_t most);
+extern "C" uint32_t fake_rt_most_chunks_launched(void);
 extern "C" uint32_t fake_rt_stream_prelaunches(void);
 extern "C" uint64_t fake_rt_chunks_streamed(void);
 
@@ -2502,7 +2504,8 @@ static void TestStreamedCopies()
         std::vector<uint64_t>(60, 16383), std::vector<uint64_t>(60, 16384),
     };
     std::mt19937 rng(5);
-    for (const uint32_t most : {~0u, 1u, 900u, 1500u, 0u}) {
+    constexpr uint32_t kThreeLaunches = 3 * 64;        // and no more of them
+    for (const uint32_t most : {~0u, 1u, 900u, 1500u, kThreeLaunches, 0u}) {
         for (size_t k = 0; k < lists.size(); ++k) {
             std::vector<uint64_t> len = lists[k];
             const uint64_t total = [&] { uint64_t sum = 0; for (uint64_t l : len) { sum += l; } return sum; }();
@@ -2529,17 +2532,21 @@ static void TestStreamedCopies()
                 std::memcpy(expect.data() + (static_cast<uint8_t *>(in[i]) - dev), out[i], len[i]);
             }
             (void)fake_rt_chunks_streamed();
-            fake_rt_stream_chunks(most);
+            fake_rt_stream_chunks(most == kThreeLaunches ? ~0u : most);
+            fake_rt_stream_launches(most == kThreeLaunches ? 3 : ~0u);
             smem_batch_copy_params load{out.data(), in.data(), len.data(), static_cast<uint32_t>(len.size())};
             CHECK(smem_bm_copy_batch(bm, &load, SMEMB_COPY_H2G, 0) == SM_OK);
             CHECK(std::memcmp(dev, expect.data(), room) == 0);
             const bool streams = total > (864u << 10) && total / len.size() >= 16384;
             CHECK((fake_rt_chunks_streamed() != 0) == (streams && most != 0));
+            CHECK(fake_rt_most_chunks_launched() <= 64);    // no launch holds its queue for longer than 4 MiB take
             const std::vector<uint8_t> before = outside;
             std::fill(outside.begin(), outside.end(), 0);
+            fake_rt_stream_launches(most == kThreeLaunches ? 1 : ~0u);
             smem_batch_copy_params save{in.data(), out.data(), len.data(), static_cast<uint32_t>(len.size())};
             CHECK(smem_bm_copy_batch(bm, &save, SMEMB_COPY_G2H, 0) == SM_OK);
             CHECK(outside == before);
+            fake_rt_stream_launches(~0u);
             CHECK((fake_rt_chunks_streamed() != 0) == (streams && total <= (8u << 20) && most != 0));
             fake_rt_stream_chunks(0);
         }
@@ -2574,7 +2581,7 @@ static void TestStreamedCopiesLaunchedLate()
         smem_batch_copy_params load{&there, &here, &len, 1};
         CHECK(smem_bm_copy_batch(bm, &load, SMEMB_COPY_H2G, 0) == SM_OK);
         CHECK(std::memcmp(dev, before.data(), bytes) == 0);
-        CHECK(fake_rt_launches() - launches == 1 && fake_rt_chunks_streamed() == bytes >> 16);
+        CHECK(fake_rt_launches() - launches == ((bytes >> 16) + 63) / 64 && fake_rt_chunks_streamed() == bytes >> 16);
         if (bytes > (8u << 20)) {
             continue;
         }
@@ -2583,7 +2590,7 @@ static void TestStreamedCopiesLaunchedLate()
         smem_batch_copy_params save{&here, &there, &len, 1};
         CHECK(smem_bm_copy_batch(bm, &save, SMEMB_COPY_G2H, 0) == SM_OK);
         CHECK(outside == before);
-        CHECK(fake_rt_launches() - launches == 1 && fake_rt_chunks_streamed() == bytes >> 16);
+        CHECK(fake_rt_launches() - launches == ((bytes >> 16) + 63) / 64 && fake_rt_chunks_streamed() == bytes >> 16);
     }
     fake_rt_stream_launch_takes(0);
     fake_rt_stream_chunks(0);
