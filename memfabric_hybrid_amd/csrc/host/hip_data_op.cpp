@@ -310,11 +310,23 @@ struct Streaming {
     template <class F>
     bool Await(F done)
     {
+        // Behind the launches: others may put work on the stream for as long as this lasts, so that it need not become idle.
+        struct Marker {
+            void *event = nullptr;
+            bool recorded = false;
+            ~Marker()
+            {
+                if (event != nullptr) {
+                    (void)mfrt_event_destroy(event);
+                }
+            }
+        } marker;
         auto start = std::chrono::steady_clock::now();
         auto looked = start;
         for (uint32_t polls = 1; !done(); ++polls) {
             if (LaunchMore()) {
                 start = looked = std::chrono::steady_clock::now();
+                marker.recorded = false;
             }
             if (error != 0) {
                 return false;
@@ -335,8 +347,17 @@ struct Streaming {
             std::this_thread::sleep_for(std::chrono::microseconds(kStreamSleepMicros));
             if (now - looked > std::chrono::milliseconds(kStreamLookMillis)) {
                 looked = now;
+                if (!marker.recorded) {
+                    marker.event = marker.event != nullptr ? marker.event : mfrt_event_create();
+                    marker.recorded = marker.event != nullptr && mfrt_event_record(marker.event, stream) == 0;
+                }
                 // the words of a launch that is over have all arrived
-                if (mfrt_stream_done(stream) != 0 && !LaunchMore() && !done()) {
+                const int over = marker.recorded ? mfrt_event_done(marker.event) : mfrt_stream_done(stream);
+                if (over != 0 && !done()) {
+                    if (LaunchMore()) {
+                        marker.recorded = false;
+                        continue;
+                    }
                     stopped = true;
                     return false;
                 }

@@ -326,7 +326,7 @@ int mfrt_event_sync(void *e) { Retire(*static_cast<uint64_t *>(e)); return 0; }
 static uint64_t g_streamWaits = 0;
 extern "C" uint64_t fake_rt_stream_waits(void) { return g_streamWaits; }
 int mfrt_stream_wait_event(void *, void *) { ++g_streamWaits; return 0; }
-int mfrt_event_done(void *) { return 1; }
+int mfrt_event_done(void *) { return g_streamsRunning.load() != 0 ? 0 : 1; }
 float mfrt_event_elapsed_ms(void *, void *) { return 0.0f; }
 int mfrt_memcpy(void *dst, const void *src, uint64_t bytes) { std::memmove(dst, src, bytes); return 0; }
 int mfrt_memcpy_async(void *dst, const void *src, uint64_t bytes, void *) { std::memmove(dst, src, bytes); return 0; }

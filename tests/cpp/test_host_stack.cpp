@@ -2598,6 +2598,33 @@ static void TestStreamedCopiesLaunchedLate()
     smem_bm_uninit(0);
 }
 
+// Launches that leave are noticed although the stream is never idle, because others put work behind them.
+static void TestStreamedCopiesLeftOnABusyStream()
+{
+    smem_bm_config_t cfg;
+    smem_bm_config_init(&cfg);
+    CHECK(smem_bm_init("tcp://127.0.0.1:1", 1, 0, &cfg) == SM_OK);
+    smem_bm_t bm = smem_bm_create(7, 1, SMEMB_DATA_OP_SDMA, 2u << 20, 80ull << 20, 0);
+    CHECK(bm != nullptr && smem_bm_join(bm, 0) == SM_OK);
+    auto *dev = static_cast<uint8_t *>(smem_bm_ptr_by_mem_type(bm, SMEM_MEM_TYPE_DEVICE, 0));
+    std::mt19937 rng(17);
+    fake_rt_stream_state(0);
+    for (const uint32_t most : {1u, 64u, 600u}) {
+        std::vector<uint8_t> outside(70u << 20);
+        for (size_t i = 0; i < outside.size(); i += 9) {
+            outside[i] = static_cast<uint8_t>(rng());
+        }
+        fake_rt_stream_chunks(most);
+        smem_copy_params load{outside.data(), dev, outside.size()};
+        CHECK(smem_bm_copy(bm, &load, SMEMB_COPY_H2G, 0) == SM_OK);
+        CHECK(std::memcmp(dev, outside.data(), outside.size()) == 0);
+    }
+    fake_rt_stream_chunks(0);
+    fake_rt_stream_state(1);
+    smem_bm_destroy(bm);
+    smem_bm_uninit(0);
+}
+
 // While other work is in front of the launch on its stream, one thread waits, asleep for most of the time, and the helpers are at the
 // disposal of other threads.
 static void TestStreamedCopiesBehindOtherWork()
@@ -2679,6 +2706,7 @@ int main()
     TestHostCopy();
     TestStreamedCopies();
     TestStreamedCopiesLaunchedLate();
+    TestStreamedCopiesLeftOnABusyStream();
     TestStreamedCopiesBehindOtherWork();
     TestSlotRing();
     TestReportsThatDoNotCome();
