@@ -223,6 +223,7 @@ struct Streaming {
     const uint8_t *const *memory;       // the caller's, by chunk
     std::atomic<uint32_t> next{0};
     uint32_t launched = 0;              // chunks; the caller launches
+    uint32_t launches = 0;
     int error = 0;                      // of a launch
     bool stopped = false;               // the launches have ended, or never began, with chunks left
 
@@ -241,6 +242,7 @@ struct Streaming {
             return false;
         }
         launched += some;
+        ++launches;
         return true;
     }
     bool Done(uint32_t c) const         // the GPU with chunk c in its slot
@@ -445,6 +447,7 @@ int StreamAll(void *const *src, void *const *dst, const uint64_t *len, uint32_t 
         Streaming job{area, toHost, total >= kPastCachesBytes, area->base.value, count, stream, memory.data()};
         area->base.value += count;
         job.Run(helper);
+        XcopyEngine::Instance().NoteDone(stream, job.launches);     // waited for here or below
         if (job.error != 0 || job.stopped) {
             const int sync = job.launched == 0 ? 0 : mfrt_stream_sync(stream);
             if (sync != 0) {

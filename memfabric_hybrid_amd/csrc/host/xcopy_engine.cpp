@@ -1680,6 +1680,14 @@ void XcopyEngine::NoteQueued(void *stream, uint64_t bytes)
     NotePending(stream, bytes);
 }
 
+void XcopyEngine::NoteDone(void *stream, uint32_t launches)
+{
+    g_launches.fetch_add(launches, std::memory_order_relaxed);
+    if (t_ctx.HasLiveLease() && stream == t_ctx.lease->stream) {
+        t_ctx.lease->pendingBytes = 0;
+    }
+}
+
 void XcopyEngine::QuiesceSubmitters()
 {
     for (uint32_t w = 0; w < kFanStreams; ++w) {

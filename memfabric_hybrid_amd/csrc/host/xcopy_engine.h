@@ -207,6 +207,8 @@ public:
     // Work that another part of the library has queued on `stream`: if it is the calling thread's own stream, the next
     // DrainThread() takes `bytes` into account when it chooses between polling and sleeping (~0: sleep).
     void NoteQueued(void *stream, uint64_t bytes);
+    // The same for launches that move data and have been waited for, with everything queued on `stream` before them.
+    void NoteDone(void *stream, uint32_t launches);
 
     // Enqueue one batch.  Addresses must be device-accessible.  stream may be
     // NULL (thread stream).  mask/maskValue: plugin completion word or NULL.

@@ -2598,6 +2598,36 @@ static void TestStreamedCopiesLaunchedLate()
     smem_bm_uninit(0);
 }
 
+// A streamed copy's launches are counted as those of the others, and what the thread had queued on its stream before one is not queued any more.
+static void TestStreamedCopiesAreCounted()
+{
+    smem_bm_config_t cfg;
+    smem_bm_config_init(&cfg);
+    CHECK(smem_bm_init("tcp://127.0.0.1:1", 1, 0, &cfg) == SM_OK);
+    smem_bm_t bm = smem_bm_create(7, 1, SMEMB_DATA_OP_SDMA, 2u << 20, 80ull << 20, 0);
+    CHECK(bm != nullptr && smem_bm_join(bm, 0) == SM_OK);
+    auto *dev = static_cast<uint8_t *>(smem_bm_ptr_by_mem_type(bm, SMEM_MEM_TYPE_DEVICE, 0));
+    std::vector<uint8_t> outside(5u << 20, 3);
+    smem_copy_params queued{dev, dev + (40u << 20), 40u << 20}, little{dev, dev + (40u << 20), 4096};
+    smem_copy_params load{outside.data(), dev, outside.size()}, save{dev, outside.data(), outside.size()};
+    fake_rt_stream_chunks(~0u);
+    for (const bool toHost : {false, true}) {
+        for (int i = 0; i < 8; ++i) {       // 320 MiB, more than a wait polls for
+            CHECK(smem_bm_copy(bm, &queued, SMEMB_COPY_G2G, ASYNC_COPY_FLAG) == SM_OK);
+        }
+        const uint64_t launches = mf_xcopy_launch_count();
+        CHECK(smem_bm_copy(bm, toHost ? &save : &load, toHost ? SMEMB_COPY_G2H : SMEMB_COPY_H2G, 0) == SM_OK);
+        CHECK(mf_xcopy_launch_count() - launches == 2);
+        CHECK(smem_bm_copy(bm, &little, SMEMB_COPY_G2G, ASYNC_COPY_FLAG) == SM_OK);
+        const uint64_t signals = fake_rt_signals(), syncs = fake_rt_stream_syncs();
+        CHECK(smem_bm_wait(bm) == SM_OK);
+        CHECK(fake_rt_signals() == signals + 1 && fake_rt_stream_syncs() == syncs);
+    }
+    fake_rt_stream_chunks(0);
+    smem_bm_destroy(bm);
+    smem_bm_uninit(0);
+}
+
 // Launches that leave are noticed although the stream is never idle, because others put work behind them.
 static void TestStreamedCopiesLeftOnABusyStream()
 {
@@ -2706,6 +2736,7 @@ int main()
     TestHostCopy();
     TestStreamedCopies();
     TestStreamedCopiesLaunchedLate();
+    TestStreamedCopiesAreCounted();
     TestStreamedCopiesLeftOnABusyStream();
     TestStreamedCopiesBehindOtherWork();
     TestSlotRing();
