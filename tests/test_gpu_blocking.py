@@ -2,6 +2,7 @@
 
 import ctypes
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -161,6 +162,129 @@ def test_chunks_that_the_host_never_fills(lib, pool):
     finally:
         del view, words
         lib.mfrt_free_host(host)
+
+
+@pytest.mark.parametrize("way, sizes", [
+    ("load", [3 * LEAST_ROUND // 2 + 1]), ("load", [16384] * 55), ("load", [4 << 20]), ("load", [(4 << 20) + 1]), ("load", [50000, 300001, 70000] * 9),
+    ("load", [(40 << 20) + 77]), ("save", [3 * LEAST_ROUND // 2 + 1]), ("save", [16384] * 55), ("save", [(4 << 20) + 1]), ("save", [8 << 20]),
+    ("save", [1000] * 480 + [7864320]),
+], ids=lambda v: v if isinstance(v, str) else f"{len(v)}x{v[0]}")
+def test_copies_are_made_beside_the_cpu(lib, pool, way, sizes):
+    """In launches of 64 chunks and no others: a copy whose launches cannot be made, or leave, has the same bytes and more launches."""
+    room = sum(sizes) + 256 * len(sizes)
+    big = bm.create(2, 0, (room + (2 << 20)) // (2 << 20) * (2 << 20))
+    try:
+        inside = big.peer_rank_ptr(0) + np.cumsum([0] + [(n + 255) // 128 * 128 for n in sizes[:-1]])
+        flat = np.random.default_rng(3).integers(0, 256, sum(sizes), dtype=np.uint8)
+        outside = flat.ctypes.data + np.cumsum([0] + sizes[:-1])
+        expect = flat.copy()
+        load, save = bm.BmCopyType.H2G, bm.BmCopyType.G2H
+        assert big.copy_data_batch(outside.tolist(), inside.tolist(), sizes, len(sizes), load) == 0, native.last_error()
+        chunks = sum((n + 65535) // 65536 for n in sizes)
+        for _ in range(3):
+            if way == "save":
+                flat[:] = 0
+            launches = lib.mf_xcopy_launch_count()
+            source, target = (outside, inside) if way == "load" else (inside, outside)
+            assert big.copy_data_batch(source.tolist(), target.tolist(), sizes, len(sizes), load if way == "load" else save) == 0, native.last_error()
+            most = chunks if way == "load" else 512
+            jobs = [min(most, chunks - at) for at in range(0, chunks, most)]
+            assert lib.mf_xcopy_launch_count() - launches == sum((j + 63) // 64 for j in jobs)
+        if way == "load":
+            flat[:] = 0
+            assert big.copy_data_batch(inside.tolist(), outside.tolist(), sizes, len(sizes), save) == 0, native.last_error()
+        assert np.array_equal(flat, expect)
+    finally:
+        big.destroy()
+
+
+class _Ring:
+    """The area that a launch of chunks and the CPU share, of `slots` slots and `count` chunks at `addresses` of `lengths` bytes."""
+
+    def __init__(self, lib, slots, addresses, lengths, base):
+        self.lib, self.slots, self.count, self.base = lib, slots, len(addresses), base
+        self.listed = slots << 16
+        self.words_at = [self.listed + 16 * self.count + 64, 0]
+        self.words_at[0] = self.words_at[0] // 64 * 64
+        self.words_at[1] = self.words_at[0] + 64 * slots
+        size = self.words_at[1] + 64 * slots
+        self.host = lib.mfrt_alloc_host(size)
+        self.bytes = np.ctypeslib.as_array((ctypes.c_uint8 * size).from_address(self.host))
+        self.bytes[:] = 0
+        pairs = self.bytes[self.listed:self.listed + 16 * self.count].view(np.uint64)
+        pairs[0::2], pairs[1::2] = addresses, lengths
+        self.filled, self.done = (self.bytes[at:at + 64 * slots].view(np.uint64)[::8] for at in self.words_at)
+        self.places = [(c % slots << 16) + addresses[c] % 128 for c in range(self.count)]
+
+    def launch(self, beside, to_host, first, count, limit=1000):
+        slot = first % self.slots
+        call = self.lib.mfk_stream_chunks_beside if beside else self.lib.mfk_stream_chunks
+        return call(int(to_host), ctypes.c_void_p(self.host + (slot << 16)), ctypes.c_void_p(self.host + self.listed + 16 * first),
+                    ctypes.c_void_p(self.host + self.words_at[0] + 64 * slot), ctypes.c_void_p(self.host + self.words_at[1] + 64 * slot),
+                    ctypes.c_uint64(self.base + first), count, self.slots - slot, limit, ctypes.c_void_p(self.lib.mf_xcopy_thread_stream()))
+
+    def wait(self, c):
+        end = time.monotonic() + 5
+        while int(self.done[c % self.slots]) != self.base + c + 1:
+            assert time.monotonic() < end
+
+    def close(self):
+        assert self.lib.mfrt_device_sync() == 0
+        del self.bytes, self.filled, self.done
+        self.lib.mfrt_free_host(self.host)
+
+
+CHUNK_LENGTHS = [1, 15, 16, 17, 127, 128, 4096, 8191, 40000, 65409, 65408, 30001]
+
+
+@pytest.mark.parametrize("base", [0, (1 << 40) - 3])
+def test_chunks_to_the_host(lib, pool, base):
+    """Two launches, the second beside the first: every byte of a chunk lies in its slot as far behind a line as in HBM, and no other is written."""
+    memory = pool.peer_rank_ptr(0)
+    slots = 2 * len(CHUNK_LENGTHS)
+    lengths = CHUNK_LENGTHS + CHUNK_LENGTHS[::-1]
+    starts = [(c << 17) + (127 if n == 65409 else c * 37 % 128) for c, n in enumerate(lengths)]
+    image = np.random.default_rng(5).integers(1, 256, slots << 17, dtype=np.uint8)
+    assert lib.mfrt_memcpy(memory, image.ctypes.data, image.size) == 0
+    ring = _Ring(lib, slots, [memory + a for a in starts], lengths, base)
+    try:
+        half = len(CHUNK_LENGTHS)
+        assert ring.launch(False, True, 0, slots + 1) != 0                 # more chunks than slots: nobody would empty them
+        assert ring.launch(False, True, 0, half) == 0 and ring.launch(True, True, half, half) == 0
+        assert lib.mfrt_device_sync() == 0
+        expect = np.zeros(slots << 16, dtype=np.uint8)
+        for c, (a, n) in enumerate(zip(starts, lengths)):
+            expect[ring.places[c]:ring.places[c] + n] = image[a:a + n]
+            assert int(ring.done[c]) == base + c + 1
+        assert np.array_equal(ring.bytes[:slots << 16], expect)
+    finally:
+        ring.close()
+
+
+def test_chunks_from_the_host_round_the_ring(lib, pool):
+    """Five times as many chunks as slots, in launches beside one another, while the CPU fills what has been emptied."""
+    memory = pool.peer_rank_ptr(0)
+    slots, times = len(CHUNK_LENGTHS), 5
+    lengths = CHUNK_LENGTHS * times
+    starts = [(c << 16) + (127 if n == 65409 else c * 53 % 128) for c, n in enumerate(lengths)]
+    before = _read(lib, memory, len(lengths) << 16)
+    data = np.random.default_rng(6).integers(0, 256, before.size, dtype=np.uint8)
+    ring = _Ring(lib, slots, [memory + a for a in starts], lengths, 77)
+    try:
+        for c, (a, n) in enumerate(zip(starts, lengths)):
+            if c % slots == 0:
+                assert ring.launch(c != 0, False, c, slots) == 0
+            if c >= slots:
+                ring.wait(c - slots)
+            ring.bytes[ring.places[c]:ring.places[c] + n] = data[a:a + n]
+            before[a:a + n] = data[a:a + n]
+            ring.filled[c % slots] = 77 + c + 1
+        for c in range(len(lengths) - slots, len(lengths)):
+            ring.wait(c)
+        assert lib.mfrt_device_sync() == 0
+        assert np.array_equal(_read(lib, memory, before.size), before)
+    finally:
+        ring.close()
 
 
 @pytest.mark.parametrize("count, most, launches", [(513, 131072, 1), (1400, 65536, 2), (1601, 131072, 3)])
