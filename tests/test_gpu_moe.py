@@ -270,8 +270,11 @@ def test_out_of_range_expert_ids_are_flagged_not_followed(gpu, oracle):
 
 
 @pytest.mark.parametrize("T,H,K", [
-    (3600, 7168, 8),   # 25 200 slices: one full period for 4096 waves and a last period of two read parts and a short third
-    (3300, 8000, 8),   # rows of 1000 units in eight slices of 125: ragged slices, a last period of three read parts
+    (3600, 7168, 8),   # 25 200 slices: one period of three read parts for 5120 waves, then one read part and a short second
+    (3300, 8000, 8),   # rows of 1000 units in eight slices of 125: ragged slices, a last period of two read parts and a short third
+    (3200, 8192, 8),   # 25 600 slices: the last period ends with its second read part
+    (3840, 8192, 8),   # 30 720: with its third, two whole periods
+    (991, 31744, 8),   # one slice more: a third period of one wave
     (700, 1024, 8),    # narrow rows: one four-wave workgroup per token
     (60, 7168, 8),     # wide rows, few tokens: one workgroup per slice
     (300, 16384, 3),   # any other topK
@@ -284,7 +287,7 @@ def test_out_of_range_expert_ids_are_flagged_not_followed(gpu, oracle):
 ])
 def test_combine_of_rows_that_differ_within_a_token(gpu, oracle, T, H, K):
     """After a dispatch the rows of a token are copies of one another, so a combine that mixed them up would still pass
-    the dispatch-then-combine tests; here every row is different.  The first two shapes and the top-6 shape of 5400 tokens have enough tokens of wide rows
+    the dispatch-then-combine tests; here every row is different.  The first five shapes and the top-6 shape of 5400 tokens have enough tokens of wide rows
     for the combine whose waves stay and alternate between reading and writing: same bits as the oracle at the
     default pace, at a slow and at an absurdly fast one, with slots without a row, and with the form switched off."""
     rng = np.random.default_rng(T)
@@ -319,12 +322,12 @@ def test_combine_of_rows_that_differ_within_a_token(gpu, oracle, T, H, K):
 
 
 @pytest.mark.parametrize("T,H,K,stays", [
-    (3510, 7168, 8, False),   # one token short of six slices a wave
-    (3511, 7168, 8, True),    # one token more: a full period, two read parts and one slice of a third
-    (2081, 7168, 8, False),   # more than 256 MiB, 3.6 slices a wave
-    (6145, 2048, 8, False),   # the fewest entries beyond the dispatch that counts, three slices a wave
+    (3510, 7168, 8, False),   # one token short of 96 slices a CU
+    (3511, 7168, 8, True),    # one token more: 24 577 slices, one period and two read parts, the second short
+    (2081, 7168, 8, False),   # more than 256 MiB, 57 slices a CU
+    (6145, 2048, 8, False),   # the fewest entries beyond the dispatch that counts, 48 slices a CU
     (3845, 7168, 6, False), (3846, 7168, 6, True),      # where those rows end at top-6
-    (8192, 3072, 6, False), (8193, 3072, 6, True),      # the fewest entries beyond the dispatch that counts, at six slices a wave
+    (8192, 3072, 6, False), (8193, 3072, 6, True),      # the fewest entries beyond the dispatch that counts, at 96 slices a CU
     (8200, 3072, 4, False),
 ])
 def test_combine_where_its_waves_begin_to_stay(gpu, oracle, T, H, K, stays):
