@@ -198,6 +198,64 @@ def test_copies_are_made_beside_the_cpu(lib, pool, way, sizes):
         big.destroy()
 
 
+@pytest.mark.parametrize("way, nbytes", [("load", 1 << 20), ("load", 40 << 20), ("save", 1 << 20), ("save", 8 << 20)])
+def test_copies_behind_other_work(lib, pool, way, nbytes):
+    """Several milliseconds of it on the same stream: the caller has gone over from polling to waiting when the launch begins."""
+    other = 128 << 20
+    big = bm.create(2, 0, 2 * other + (64 << 20))
+    try:
+        dev = big.peer_rank_ptr(0)
+        at = dev + 2 * other + 77
+        flat = np.random.default_rng(nbytes).integers(0, 256, nbytes, dtype=np.uint8)
+        expect = flat.copy()
+        load, save = bm.BmCopyType.H2G, bm.BmCopyType.G2H
+        if way == "save":
+            assert big.copy_data(flat.ctypes.data, at, nbytes, load) == 0, native.last_error()
+            flat[:] = 0
+        for _ in range(100):
+            assert big.copy_data(dev, dev + other, other, bm.BmCopyType.G2G, native.ASYNC_COPY_FLAG) == 0, native.last_error()
+        launches = lib.mf_xcopy_launch_count()
+        source, target = (flat.ctypes.data, at) if way == "load" else (at, flat.ctypes.data)
+        assert big.copy_data(source, target, nbytes, load if way == "load" else save) == 0, native.last_error()
+        assert lib.mf_xcopy_launch_count() - launches == (nbytes // 65536 + 64) // 64          # one chunk more than whole ones: they begin off a line
+        assert np.array_equal(flat if way == "save" else _read(lib, at, nbytes), expect)
+    finally:
+        assert lib.mfrt_device_sync() == 0
+        big.destroy()
+
+
+def test_threads_that_stream_at_once(lib, pool):
+    """One of them has the helpers, the others copy alone."""
+    count, room = 4, 12 << 20
+    big = bm.create(2, 0, count * room + (2 << 20))
+    errors = []
+
+    def run(k):
+        try:
+            rng = np.random.default_rng(k)
+            at = big.peer_rank_ptr(0) + k * room
+            for nbytes in (1 << 20, (9 << 20) + 5, 3000001, 8 << 20):
+                flat = rng.integers(0, 256, nbytes, dtype=np.uint8)
+                back = np.zeros_like(flat)
+                for _ in range(5):
+                    assert big.copy_data(flat.ctypes.data, at + k, nbytes, bm.BmCopyType.H2G) == 0, native.last_error()
+                    assert big.copy_data(at + k, back.ctypes.data, nbytes, bm.BmCopyType.G2H) == 0, native.last_error()
+                    assert np.array_equal(flat, back)
+                    back[:] = 0
+        except BaseException as e:   # noqa: BLE001 - handed to the test's own thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(count)]
+    try:
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not errors, errors[0]
+    finally:
+        big.destroy()
+
+
 class _Ring:
     """The area that a launch of chunks and the CPU share, of `slots` slots and `count` chunks at `addresses` of `lengths` bytes."""
 
