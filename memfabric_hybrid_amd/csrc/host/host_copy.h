@@ -4,7 +4,7 @@
 // by the calling thread alone is bound by that core (reference counterpart: the staging copies of
 // HostDataOpSDMA::CopyLH2GD / CopyGD2LH, src/hybm/csrc/data_operation/host/hybm_data_op_sdma.cpp:
 // 111-221, which run on the calling thread).  Here helper threads take equal shares of every large
-// set of pieces, or one chunk after another of a copy that a launch makes meanwhile (Begin, End).
+// set of pieces, or one chunk after another of a copy that launches make meanwhile (Begin, End).
 #ifndef MF_HOST_COPY_H
 #define MF_HOST_COPY_H
 

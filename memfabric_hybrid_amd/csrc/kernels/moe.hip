@@ -131,8 +131,11 @@ constexpr uint64_t kWarmMaxBytes = 224ull << 20;
 constexpr uint32_t kWarmGroups = 128;
 constexpr uint32_t kWarmPieces = 8;                     // 128-bit loads in flight per lane
 constexpr uint32_t kWarmHistPercent = 30;               // share of the shorter first launch
-// Rows of so many bytes are read by all CUs that rank nothing, as long as those are many: 8192 tokens of 7168 elements, 117 MB, dispatch with 128 groups and 30 % / so, top-8 over 256 experts
-// 181.0 / 177.1 us, over 8 170.0 / 165.6, top-4 115.0 / 109.7, top-2 74.4 / 73.7; but 84 MB, partly in that cache, 98.2 / 100.1.
+// Rows of so many bytes are read by all CUs that rank nothing, as long as those are many.  Dispatch with 128 groups and 30 % / so, us, four processes each in turn on one machine, each
+// within 0.5: 8192 tokens of 7168 elements (117 MB) top-8 over 256 experts 180.6 / 176.5, over 8 169.4 / 164.9, top-6 144.8 / 140.8, top-4 112.2 / 108.0, top-2 73.9 / 73.4; 7168 of 7168 (103 MB)
+// 155.3 / 153.5, 6144 of 10 240 (126 MB) 194.0 / 188.9, 8192 of 8192 and 4096 of 16 384 (134 MB) 204.5 / 202.6, 204.3 / 202.0; at top-4 over 64 8192 of 12 288 (201 MB) 208.5 / 194.1, 3584 of 28 672
+// (206 MB) 213.7 / 211.0; but 84 MB, partly in that cache, 98.2 / 100.1.  Under a tracer, which sets the launches apart, the histograms, ranks and permute of the first take 8.7 + 18.8 + 157 / 9.1 +
+// 14.5 + 162, at top-4 8.3 + 18.6 + 84.7 / 8.7 + 13.7 + 84.7.
 constexpr uint64_t kWarmMoreBytes = 96ull << 20;
 constexpr uint32_t kWarmMoreGroups = 192;
 constexpr uint32_t kWarmMoreBlocks = 64;                // with which they are 256 (16 384 tokens of 4096 elements, 128 blocks, dispatch 208.3 / 210.0)
@@ -1285,8 +1288,9 @@ __global__ __launch_bounds__(kThreads) void MoeCombineKernel(uint64_t rowsIn, ui
 // AgreedStart(); after that every wave goes by the constant-rate clock alone.  8192 tokens of 7168
 // elements at top-8: 162 us against 177-181 us for one workgroup per item.  Read parts are paced at 6.8 TB/s, write parts at 6.5.
 // HBM is the bound.  Results in registers, four an item (116 of them), left room for 4096 waves: 5120 have a quarter more time for loads that come late in as
-// much longer parts.  Dispatch and combine, us, 4096 waves at 6.8 and 6.2 / 5120 at 6.8 and 6.5: 8192 tokens of 7168 elements at top-8 over 256 experts 352 / 344, over 8 331 /
-// 329, at top-6 274 / 271, of 5120 246 / 244, of 4096 191.0 / 191.5; combine alone of 3600 of 7168 74.3 / 72.7.  Reads at 6.85 make the waves fall behind behind a
+// much longer parts.  Combine, and dispatch and combine, us, 4096 waves at 6.8 and 6.2 / 5120 at 6.8 and 6.5: 8192 tokens of 7168 elements at top-8 over 256 experts 165.8 / 161.5, 352.7 / 349.6, over
+// 8 166.1 / 163.1, 336.2 / 334.3, at top-6 129.9 / 126.0, 275.8 / 271.1, of 5120 117.9 / 116.0, 245.3 / 243.9, of 4096, two whole periods before and now an eighth more, 92.9 / 93.6, 190.5 / 190.7;
+// 3600 of 7168 74.5 / 73.2, 155.4 / 154.2 (five processes each in turn, within 0.5).  Reads at 6.85 make the waves fall behind behind a
 // dispatch, whose rows are still on their way out of the last-level cache (350).  Not taken: 6144 waves (80 registers spill), four results (LDS for 18 waves, 346).
 // Arithmetic and the rule for slots without a row are MoeCombineKernel's.
 constexpr uint32_t kCombineItems = 3;                  // of which the results, 2 KiB each, wait in LDS
