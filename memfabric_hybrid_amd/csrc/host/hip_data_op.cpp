@@ -175,10 +175,30 @@ struct StreamArea {
 };
 static_assert(sizeof(StreamArea::ring) == kBounceBytes, "the rounds use it too, and nothing behind it");
 // What is one round stays one: 512 KiB to the host 21.9 us, streamed 24.5, and below kSplitMin a copy of its own would wake the helpers for it (260 KB to the GPU 2 ms
-// behind the last 24 us, streamed 33).  Shorter segments make chunks that are not worth their words.  Before / streamed, us, to the GPU and back: 1 MiB 37.7 / 32.4, 40.8 /
+// behind the last 24 us, streamed 33).  Before / streamed, us, to the GPU and back: 1 MiB 37.7 / 32.4, 40.8 /
 // 36.5, 2 MiB 65.6 / 54.4, 63.4 / 56.0; 2 ms behind the last 53.2 / 45.2, 54.5 / 50.0, 74.4 / 67.7, 73.1 / 68.0.
 constexpr uint64_t kStreamMinBytes = kRoundMinBytes / 2 * 3 + 1;
-constexpr uint64_t kStreamMinSegmentBytes = 16ull << 10;
+// A chunk costs a launch 0.33 us beyond its bytes, so a list that makes many more of them than full ones would be goes in rounds, which gather: at most 16 more, and one for 128 KiB, up
+// to 64.  us, rounds / streamed, one behind the other and 2 ms apart, to the GPU and back:
+//     segments              more chunks, of     to the GPU                        back
+//     32 of 32 768             16      24       37 / 34          58 / 49          42 / 35          60 / 49
+//     20 of 4096 and 61 440    20      26       41 / 44          68 / 60          41 / 43          57 / 57
+//     36 of 28 672             20      24       37 / 36          58 / 52          42 / 36          58 / 51
+//     42 of 24 576             26      24       37 / 39          60 / 56          42 / 37          60 / 51
+//     52 of 20 000             36      24       37 / 42          60 / 58          42 / 39          60 / 54
+//     64 of 16 384             48      24       38 / 46          60 / 62          43 / 41          60 / 56
+//     60 of 1024, 1 MiB        60      24       39 / 66          59 / 75          46 / 52          59 / 67
+//     64 of 32 768             32      32       62 / 63          76 / 75          63 / 57          77 / 72
+//     128 of 32 768            64      48      106 / 112        122 / 123        107 / 101        115 / 116
+//     119 of 70 000           111      64      190 / 198        204 / 210        186 / 178        192 / 193
+//     204 of 40 960            77      64      186 / 192        204 / 205        180 / 180        189 / 193
+//     512 of 16 384           384      64      195 / 301            -            187 / 252            -
+//     292 of 57 344            36      64      339 / 339            -
+//     341 of 49 152            85      64      341 / 348        357 / 356
+//     4096 of 16 384         3072      64     1267 / 2294           -
+constexpr uint64_t kStreamShortLeast = 16;
+constexpr uint64_t kStreamShortBytes = 128ull << 10;
+constexpr uint64_t kStreamShortMost = 64;
 // A segment whose last chunk would be this short is cut into equal ones: full chunks and short ones in turn leave most of the work to a part of the launch's
 // workgroups, which take every eighth or sixteenth.  us, a launch a round / full chunks and a tail / equal ones: 22 segments of 68 181 bytes in 47.8 / 51.6 /
 // 46.9, out 46.4 / 47.6 / 46.1; 32 of 72 022 in 71.0 / 74.3 / 69.8; out 32 of 203 125 145.4 / 147.6 / 139.7, of 100 000 80.6 / 78.5 / 75.1; but 4 of 375 000, a tail of
@@ -187,6 +207,7 @@ constexpr uint64_t kStreamShortTail = kStreamChunkBytes / 8 * 5;
 // To the host rounds are the better from here on: a core empties its share of one, 2 MiB, in one piece, sooner than as many chunks (10 MiB 216 to 229 us, streamed 214 in
 // some processes and 245 in others; 8 MiB in 20 parts 188 / 175).
 constexpr uint64_t kStreamMostBytesOut = kRoundBytes;
+static_assert(2 * (kStreamMostBytesOut / kStreamChunkBytes + kStreamShortMost) <= kStreamSlots, "to the host no slot is used twice, and a segment off a line may make one chunk more");
 // Copies of so many bytes go past the CPU's caches, which they would sweep, ring and all.  us, rounds by memcpy / rounds past the caches / streamed: to the host 4 MiB 103 / 108 / 96, 8 MiB in 20
 // parts 188 / 191 / 172, 12 MiB 265 / 255 / 253, 16 MiB 376 / 338 / 334, 64 MiB 1273 / 1242 / 1352; to the GPU 4 MiB 109 / 114 / 101, 16 MiB 370 / 350 / 340, 64 MiB 1339 / 1286 /
 // 1262, 128 MiB 2559 / 2503 / 2490.  What reads the caller's array next is no slower for it, as the caches that memcpy leaves it in are mostly other cores': a save and a sum over
@@ -396,11 +417,13 @@ struct Streaming {
 bool Streams(const uint64_t *len, uint32_t n, bool toHost, void *stream)
 {
     uint64_t total = 0;
+    uint64_t chunks = 0;
     for (uint32_t i = 0; i < n; ++i) {
         total += len[i];
+        chunks += len[i] / kStreamChunkBytes + (len[i] % kStreamChunkBytes != 0 ? 1 : 0);
     }
-    return total >= kStreamMinBytes && !(toHost && total > kStreamMostBytesOut) && total / n >= kStreamMinSegmentBytes &&
-           mfrt_stream_capturing(stream) == 0;
+    return total >= kStreamMinBytes && !(toHost && total > kStreamMostBytesOut) &&
+           chunks <= total / kStreamChunkBytes + std::min(kStreamShortLeast + total / kStreamShortBytes, kStreamShortMost) && mfrt_stream_capturing(stream) == 0;
 }
 
 constexpr int kNotStreamed = 1;
@@ -424,7 +447,7 @@ int StreamAll(void *const *src, void *const *dst, const uint64_t *len, uint32_t 
     while (i < n) {
         memory.clear();
         uint32_t count = 0;
-        while (i < n && count < (toHost ? kStreamSlots : kStreamListChunks)) {      // to the host the GPU waits for nothing
+        while (i < n && count < kStreamListChunks) {
             const uint64_t left = len[i] - at;
             if (left == 0) {
                 ++i;

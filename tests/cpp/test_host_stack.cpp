@@ -8,6 +8,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <ctime>
+#include <algorithm>
 #include <random>
 #include <atomic>
 #include <chrono>
@@ -2501,7 +2502,8 @@ static void TestStreamedCopies()
     auto *dev = static_cast<uint8_t *>(smem_bm_ptr_by_mem_type(bm, SMEM_MEM_TYPE_DEVICE, 0));
     const std::vector<std::vector<uint64_t>> lists = {
         {256u << 10}, {(256u << 10) - 1}, {(864u << 10) + 1}, {(33u << 20) + 13}, {70u << 20}, {8u << 20}, {(8u << 20) + 1}, {512u << 10}, {(512u << 10) - 1}, {864u << 10}, {40000, 0, 16384, 1, 300000, 16385}, std::vector<uint64_t>(200, 32768), {8u << 20, 5, (25u << 20) + 1, 127},
-        std::vector<uint64_t>(60, 16383), std::vector<uint64_t>(60, 16384),
+        std::vector<uint64_t>(60, 16383), std::vector<uint64_t>(60, 16384), std::vector<uint64_t>(37, 25600), std::vector<uint64_t>(38, 25600),
+        std::vector<uint64_t>(1000, 16384), std::vector<uint64_t>(1024, 32768), [] { std::vector<uint64_t> l(60, 1024); l.push_back(1u << 20); return l; }(),
     };
     std::mt19937 rng(5);
     constexpr uint32_t kThreeLaunches = 3 * 64;        // and no more of them
@@ -2537,7 +2539,11 @@ static void TestStreamedCopies()
             smem_batch_copy_params load{out.data(), in.data(), len.data(), static_cast<uint32_t>(len.size())};
             CHECK(smem_bm_copy_batch(bm, &load, SMEMB_COPY_H2G, 0) == SM_OK);
             CHECK(std::memcmp(dev, expect.data(), room) == 0);
-            const bool streams = total > (864u << 10) && total / len.size() >= 16384;
+            uint64_t chunks = 0;
+            for (uint64_t l : len) {
+                chunks += (l + 65535) / 65536;
+            }
+            const bool streams = total > (864u << 10) && chunks <= total / 65536 + std::min<uint64_t>(16 + total / 131072, 64);    // no more short ones
             CHECK((fake_rt_chunks_streamed() != 0) == (streams && most != 0));
             CHECK(fake_rt_most_chunks_launched() <= 64);    // no launch holds its queue for longer than 4 MiB take
             const std::vector<uint8_t> before = outside;
@@ -2668,8 +2674,7 @@ static void TestStreamedCopiesBehindOtherWork()
     std::mt19937 rng(13);
     fake_rt_stream_chunks(~0u);
     constexpr uint32_t kBusyMillis = 400;
-    std::vector<uint64_t> shortOnes(480, 1000);        // with the one behind them more chunks than the ring has slots
-    shortOnes.push_back(7864320);
+    const std::vector<uint64_t> shortOnes(100, 40000);
     const std::vector<std::vector<uint64_t>> loads = {{70ull << 20}, {5ull << 20}, shortOnes}, saves = {{1ull << 20}, {8ull << 20}, shortOnes};
     for (const bool toHost : {false, true}) {
         for (const std::vector<uint64_t> &len : toHost ? saves : loads) {

