@@ -1781,12 +1781,12 @@ BatchStats StatsOf(const uint64_t *src, const uint64_t *dst, const uint64_t *len
     return st;
 }
 
-bool InOrder(const uint64_t *at, const uint64_t *len, uint32_t n)
+bool InOrder(const uint64_t *at, const uint64_t *len, uint32_t n, uint64_t gap)
 {
     const uint32_t seen = n < 256 ? n : 256;
     uint32_t following = 0;
     for (uint32_t i = 1; i < seen; ++i) {
-        following += at[i - 1] + len[i - 1] == at[i] ? 1 : 0;
+        following += at[i] - (at[i - 1] + len[i - 1]) <= gap ? 1 : 0;
     }
     return following >= seen / 2;
 }
@@ -1892,13 +1892,17 @@ uint32_t XcopyEngine::PieceUnits(const BatchStats &stats, uint32_t n, bool unord
 //     8192 of up to 50 000               85.8   85.5   86.9     -    84.4   86.1   86.7    (73 %: left as it was)
 //     4000 of up to 70 000 (2 held)      53.3   56.6   55.3     -    53.7   53.7   55.9
 //     4000 of up to 131 072 (3 held)     98.5  102.5   99.6     -    98.5   94.7   92.9
-// so only those that are not held.
+// so only those that are not held.  Written in order they are the quicker without windows up to gaps of some 64 KiB, in which a launch still finds rows of HBM open; read in
+// order only without a gap.  us without / in windows, 8700 of up to 70 000 bytes, 290 MB, gaps of 1 to 4096 / 20 000 / 60 000 / 200 000: written in order 107 / 114, 110 / 114, 114 / 114,
+// 119 / 115, read too 100 / 114, 105 / 114, 114 / 114, 117 / 115, read alone 116 / 115, 118 / 114, 120 / 115, 123 / 115; 6700 of up to 131 072, 420 MB, 153 / 160, 155 / 159,
+// 159 / 160, 166 / 160, read too 143 / 159, 148 / 159, 151 / 159, 160 / 162, read alone 167 / 161, 170 / 160, 171 / 162, 173 / 161.
 uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n, uint32_t count, uint32_t units,
                                       bool unordered, uint32_t &reading) const
 {
     constexpr uint64_t kLessFullBytes = 24000;
     constexpr uint32_t kShortReading = 30;
     constexpr uint64_t kOddPercent = 75;
+    constexpr uint64_t kOddGapBytes = 64ull << 10;
     if (unordered || units != kDeepUnits || !WindowsApply(stats.total, MFRT_ROUTE_HBM, kPieceWindowMinBytes)) {
         return 0;
     }
@@ -1910,7 +1914,7 @@ uint32_t XcopyEngine::PieceWindowRate(const BatchStats &stats, const uint64_t *s
     const bool longBlocks = mean >= kWindowLongBlockBytes;
     if (!OnLines(stats)) {
         const bool holds = !equal && mean < kHeldOddBytes && count > 2 * kHeldMaxPieces && percent >= kOddPercent;
-        return holds && !InOrder(dst, len, n) && !InOrder(src, len, n) ? rate * (percent >= 85 ? 58 : 57) : 0;
+        return holds && !InOrder(dst, len, n, kOddGapBytes) && !InOrder(src, len, n) ? rate * (percent >= 85 ? 58 : 57) : 0;
     }
     if (InOrder(dst, len, n)) {
         return onGrid ? rate * 68 : equal || (longBlocks && percent >= 85) ? rate * 66 : 0;

@@ -51,8 +51,8 @@ struct BatchStats {
     uint64_t deepPieces = 0;        // of 16 KiB, at the most
 };
 BatchStats StatsOf(const uint64_t *src, const uint64_t *dst, const uint64_t *len, uint32_t n);
-// Whether most of the first segments of a batch lie one behind the other, in source or destination.
-bool InOrder(const uint64_t *at, const uint64_t *len, uint32_t n);
+// Whether most of the first segments of a batch lie one behind the other, in source or destination, with at most `gap` bytes in between.
+bool InOrder(const uint64_t *at, const uint64_t *len, uint32_t n, uint64_t gap = 0);
 
 // A batch of this much and more is cut into pieces of 8 and 16 KiB.  Shorter ones keep 4 KiB, which more CUs share: 150 pages of 8 KiB
 // 2.8 us, 4.0 in waves of 16 KiB; 200 pages of 32 KiB 4.4 / 4.6.  From there on the longer pieces are as fast and a quarter of the

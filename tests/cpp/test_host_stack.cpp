@@ -2339,6 +2339,31 @@ static void TestWindowRatesOfLists()
         fake_rt_piece_launches(&most, &wait);
         CHECK(fake_rt_last_window() == (more ? randomLong : 0) && (wait != 0) == !more && (most > kHeldMaxPieces) == more);
     }
+    // lists off the lines: in windows where they are written here and there, or with wide gaps
+    struct Odd { uint64_t least, most, gap; bool inOrder; uint32_t rate; };
+    for (const Odd &f : {Odd{1, 70000, 0, false, part * 57}, Odd{90000, 98000, 0, false, part * 58}, Odd{1, 45000, 0, false, 0}, Odd{1, 70000, 0, true, 0},
+                         Odd{1, 70000, 1, true, 0}, Odd{1, 70000, 300, true, 0}, Odd{1, 70000, 4096, true, 0}, Odd{1, 70000, 64 * k, true, 0},
+                         Odd{1, 70000, 200 * k, true, part * 57}, Odd{90000, 98000, 20000, true, 0}}) {
+        constexpr uint32_t n = 8192;
+        std::mt19937 rng(5);
+        std::vector<uint64_t> s(n), d(n), l(n);
+        uint64_t at = (1ull << 42) + 3;
+        for (uint32_t i = 0; i < n; ++i) {
+            l[i] = f.least + rng() % (f.most - f.least + 1);
+            s[i] = (1ull << 40) + (i * 5077ull % n) * 256 * k + 1;
+            d[i] = f.inOrder ? at : (1ull << 42) + (i * 7919ull % n) * 256 * k + 3;
+            at += l[i] + (f.gap > 1 ? f.gap / 2 + rng() % (f.gap / 2 + 1) : f.gap);
+        }
+        (void)fake_rt_last_window();
+        CHECK(XcopyEngine::Instance().Submit(s.data(), d.data(), l.data(), n, MF_ROUTE_HBM, mf_xcopy_thread_stream(), nullptr, 0) == BM_OK);
+        CHECK(XcopyEngine::Instance().DrainThread() == BM_OK);
+        const uint32_t got = fake_rt_last_window();
+        CHECK(got == f.rate);
+        if (got != f.rate) {
+            std::printf("  of %llu to %llu bytes, gaps of up to %llu: rate %u, expected %u\n", static_cast<unsigned long long>(f.least), static_cast<unsigned long long>(f.most),
+                        static_cast<unsigned long long>(f.gap), got, f.rate);
+        }
+    }
     fake_rt_skip_copies(0);
     hybm_uninit();
 }
