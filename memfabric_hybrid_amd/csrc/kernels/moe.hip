@@ -36,6 +36,7 @@
 
 #include "../rt/mf_rt.h"
 #include "launch.h"
+#include "through.h"
 #include "window_clock.h"
 
 namespace mf {
@@ -454,7 +455,7 @@ template <int kMode>
 __device__ __forceinline__ void RowStore(MF_GLOBAL u32x4 *p, u32x4 v)
 {
     if (kMode == 2) {
-        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt" : : "v"(p), "v"(v) : "memory");
+        StoreThrough16(reinterpret_cast<uint64_t>(p), v);
     } else if (kMode == 1) {
         __builtin_nontemporal_store(v, p);
     } else {

@@ -14,6 +14,7 @@
 #include "../rt/mf_rt.h"
 #include "launch.h"
 #include "staging.h"
+#include "through.h"
 
 namespace mf {
 namespace {
@@ -36,15 +37,9 @@ __device__ __forceinline__ uint64_t ReadWord(uint64_t at)
     return __hip_atomic_load(Buffer<uint64_t>(at), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Written through: it has reached its memory, HBM or the host's, when vmcnt says so.
-__device__ __forceinline__ void StoreThrough(uint64_t at, u32x4 v)
-{
-    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt" : : "v"(reinterpret_cast<MF_GLOBAL u32x4 *>(at)), "v"(v) : "memory");
-}
 __device__ __forceinline__ void CopyByteThrough(uint64_t src, uint64_t dst)
 {
-    const uint32_t v = *reinterpret_cast<const MF_GLOBAL uint8_t *>(src);
-    asm volatile("global_store_byte %0, %1, off sc0 sc1 nt" : : "v"(reinterpret_cast<MF_GLOBAL uint8_t *>(dst)), "v"(v) : "memory");
+    StoreThrough1(dst, *reinterpret_cast<const MF_GLOBAL uint8_t *>(src));
 }
 
 // `len` bytes between addresses that agree modulo kStreamLine, in units counted from the line they begin in; with what lies in front of
@@ -71,7 +66,7 @@ __device__ __forceinline__ void CopyChunkThrough(uint64_t src, uint64_t dst, uin
         for (uint32_t j = 0; j < kStreamUnits; ++j) {
             const uint32_t u = j * kStreamThreads + threadIdx.x;
             if (u >= first && u < last) {
-                StoreThrough(d + u * 16, v[j]);
+                StoreThrough16(d + u * 16, v[j]);
             }
         }
     }

@@ -26,6 +26,7 @@
 
 #include "xcopy_plan.h"
 #include "launch.h"
+#include "through.h"
 #include "window_clock.h"
 #include "../rt/mf_rt.h"
 
@@ -75,7 +76,7 @@ __device__ __forceinline__ void StoreUnit(uint64_t addr, u32x4 v)
 {
     GDstUnit p = reinterpret_cast<GDstUnit>(addr);
     if (kStore == kStoreThrough) {
-        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt" : : "v"(p), "v"(v) : "memory");
+        StoreThrough16(addr, v);
     } else if (kStore == kStoreStream) {
         __builtin_nontemporal_store(v, p);
     } else {
@@ -89,7 +90,7 @@ __device__ __forceinline__ void CopyByte(uint64_t src, uint64_t dst)
     GDstByte p = reinterpret_cast<GDstByte>(dst);
     const uint8_t v = *reinterpret_cast<GSrcByte>(src);
     if (kStore == kStoreThrough) {
-        asm volatile("global_store_byte %0, %1, off sc0 sc1 nt" : : "v"(p), "v"(static_cast<uint32_t>(v)) : "memory");
+        StoreThrough1(dst, v);
     } else {
         *p = v;
     }
