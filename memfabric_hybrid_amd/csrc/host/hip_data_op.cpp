@@ -213,7 +213,12 @@ static_assert(2 * (kStreamMostBytesOut / kStreamChunkBytes + kStreamShortMost) <
 // 1262, 128 MiB 2559 / 2503 / 2490.  What reads the caller's array next is no slower for it, as the caches that memcpy leaves it in are mostly other cores': a save and a sum over
 // the array on one core, by memcpy / past the caches, medians on three machines, 12 MiB 629 / 582, 16 MiB 816 / 724, 64 MiB 2834 / 2739; and a copy of it 705 / 706 (on one of them 632 / 721),
 // 918 / 876, 3403 / 3362.
+// Saves of short segments do so from 48 MiB on only.  us, rounds by memcpy / past the caches, two processes each: 16 MiB in segments of 16 KiB 359 / 385, 64 KiB 334 / 348, 512 KiB 329 / 338, 1 MiB, which memcpy
+// itself writes another way, 367 / 337; 24 MiB 516 / 536, 484 / 498, 483 / 487, 508 / 486; 32 MiB of 16 and 512 KiB 676 / 691, 630 / 634; 40 MiB 852 / 848, 782 / 783; 48 MiB 1032 / 1002, 948 / 931; 64 MiB 1354 /
+// 1315, 1267 / 1232.  Loads of short segments gain as the others do: 1024 of 16 KiB 383 / 361.
 constexpr uint64_t kPastCachesBytes = 12ull << 20;
+constexpr uint64_t kPastCachesLongSegment = 1ull << 20;
+constexpr uint64_t kPastCachesShortBytes = 48ull << 20;
 constexpr uint32_t kStreamLimitMillis = 1000;
 constexpr uint32_t kStreamLookMillis = 50;              // without a word from the GPU: then whether it has left
 constexpr uint32_t kStreamIdleMicros = 100;             // a launch on an idle stream says its first word after some 20
@@ -542,7 +547,7 @@ int StageOut(void *const *src, void *const *dst, const uint64_t *len, uint32_t n
         MF_FAIL(BM_MALLOC_FAILED, "pinned staging allocation failed");
     }
     RoundCursor cursor(src, dst, len, n);
-    const bool pastCaches = cursor.Left() >= kPastCachesBytes;
+    const bool pastCaches = cursor.Left() >= (cursor.Left() / n >= kPastCachesLongSegment ? kPastCachesBytes : kPastCachesShortBytes);
     StagedLaunches launches(stream);
     std::vector<uint64_t> a, b, l;
     std::vector<HostCopyHelper::Task> tasks[kSlots];   // the CPU copies of the rounds in flight

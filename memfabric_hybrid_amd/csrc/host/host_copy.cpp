@@ -214,6 +214,7 @@ void HostCopyHelper::CopySet(const Task *tasks, size_t count, bool pastCaches)
         Join(w);
     }
     shared_.fetch_add(1, std::memory_order_relaxed);
+    pastCaches_.fetch_add(pastCaches ? 1 : 0, std::memory_order_relaxed);
 }
 
 }  // namespace mf

@@ -56,6 +56,10 @@ public:
     {
         return shared_.load(std::memory_order_relaxed);
     }
+    uint64_t PastCaches() const     // of them, those that went past the caches
+    {
+        return pastCaches_.load(std::memory_order_relaxed);
+    }
 
 private:
     HostCopyHelper() = default;
@@ -95,6 +99,7 @@ private:
     Worker workers_[kWorkers];
     uint64_t tickets_[kWorkers] = {};  // of the shares posted last; guarded by owner_
     std::atomic<uint64_t> shared_{0};
+    std::atomic<uint64_t> pastCaches_{0};
 };
 
 }  // namespace mf

@@ -2513,6 +2513,43 @@ static void TestHeldLaunches()
     hybm_uninit();
 }
 
+// Which copies in rounds go past the CPU's caches: loads from 12 MiB on, saves of long segments too, of short ones from 48 MiB on.
+static void TestCopiesPastTheCaches()
+{
+    smem_bm_config_t cfg;
+    smem_bm_config_init(&cfg);
+    CHECK(smem_bm_init("tcp://127.0.0.1:1", 1, 0, &cfg) == SM_OK);
+    const uint64_t m = 1u << 20, room = 64 * m;
+    smem_bm_t bm = smem_bm_create(7, 1, SMEMB_DATA_OP_SDMA, 2 * m, room, 0);
+    CHECK(bm != nullptr && smem_bm_join(bm, 0) == SM_OK);
+    auto *dev = static_cast<uint8_t *>(smem_bm_ptr_by_mem_type(bm, SMEM_MEM_TYPE_DEVICE, 0));
+    std::vector<uint8_t> outside(room);
+    struct { uint32_t n; uint64_t len; bool load, save; } lists[] = {
+        {1, 12 * m - 1, false, false}, {1, 12 * m, true, true}, {12, m, true, true}, {13, m - 1, true, false}, {1024, 16384, true, false},
+        {3071, 16384, true, false}, {3072, 16384, true, true}, {48, m - 1, true, false}, {49, m - 1, true, true}, {64, m, true, true},
+    };
+    for (const auto &list : lists) {
+        std::vector<void *> in, out;
+        std::vector<uint64_t> len(list.n, list.len);
+        for (uint32_t i = 0; i < list.n; ++i) {
+            in.push_back(dev + i * list.len);
+            out.push_back(outside.data() + i * list.len);
+        }
+        for (const bool load : {true, false}) {
+            const uint64_t before = HostCopyHelper::Instance().PastCaches();
+            smem_batch_copy_params params{load ? out.data() : in.data(), load ? in.data() : out.data(), len.data(), list.n};
+            CHECK(smem_bm_copy_batch(bm, &params, load ? SMEMB_COPY_H2G : SMEMB_COPY_G2H, 0) == SM_OK);
+            const bool past = HostCopyHelper::Instance().PastCaches() != before;
+            CHECK(past == (load ? list.load : list.save));
+            if (past != (load ? list.load : list.save)) {
+                std::printf("  %u of %llu bytes, %s\n", list.n, static_cast<unsigned long long>(list.len), load ? "load" : "save");
+            }
+        }
+    }
+    smem_bm_destroy(bm);
+    smem_bm_uninit(0);
+}
+
 // Copies between ordinary memory and the pool while one launch runs: chunks at every byte, more than the ring has slots, several
 // segments, and a launch that leaves before it is done or cannot be made, whose copy is made in rounds.
 static void TestStreamedCopies()
@@ -2764,6 +2801,7 @@ int main()
     TestPlanners();
     TestPayloadOfPlannedTables();
     TestHostCopy();
+    TestCopiesPastTheCaches();
     TestStreamedCopies();
     TestStreamedCopiesLaunchedLate();
     TestStreamedCopiesAreCounted();
